@@ -139,6 +139,48 @@ def test_nu_smo_solve(n, ws):
     assert np.array_equal(G.host(ad_d), ad_want)
 
 
+@pytest.mark.parametrize("ws", [2, 63, 64, 65, 128, 129, 256, 257, 512, 513, 1023, 1024])
+@pytest.mark.parametrize("nu", [False, True])
+@pytest.mark.parametrize("start", ["first iteration", "threshold zero"])
+def test_local_solver_at_the_edges_of_its_variants(ws, nu, start):
+    """Working-set sizes on both sides of every variant of the solver (one wavefront of one, two or four elements per
+    thread, four wavefronts of two or four).  "first iteration": alpha = 0, f = -y and repeated instances, so that every
+    extremum is a tie that the lowest index has to win, in both wavefront-wide and workgroup-wide reductions; "threshold
+    zero": eps = 0 from a state without violators by more than that, where an element can violate without being a
+    candidate for the second index.  Everything equals the oracle bit for bit."""
+    n, Cc = ws + 37, 1.0
+    y, alpha, f, ws_ids, _, _ = _solver_inputs(n, 6, ws, 3 * ws, Cc)
+    rng = np.random.default_rng(ws)
+    x = rng.standard_normal((n, 6)).astype(np.float32)
+    x[n // 2:n // 2 + n // 4] = x[:n // 4]          # instances that occur twice: equal kernel rows, a = 0
+    data = from_dense(x)
+    km = O.KernelMatrix(data.ptr, data.col, data.val, O.make_param(kernel_type=O.RBF, gamma=0.5, expf_mode=1))
+    k_rows, diag = km.get_rows(ws_ids), km.diag()
+    eps, max_iter = 1e-3, 300
+    if start == "first iteration":
+        if not nu:
+            alpha, f = np.zeros(n), -y.astype(np.float64)
+        else:
+            f = np.where(rng.random(n) < 0.5, 0.25, -0.5)
+    else:
+        eps, max_iter = 0.0, 40
+        f = np.round(f)
+    solve = O.nu_smo_solve if nu else O.c_smo_solve
+    args = (Cc,) if nu else (Cc, Cc)
+    a_want, ad_want, diff_want = solve(y, f, alpha, ws_ids, *args, k_rows, diag, n, eps, max_iter)
+    y_d, f_d, ws_d, dg_d = G.dev(y), G.dev(f), G.dev(ws_ids), G.dev(diag)
+    wsp = torch.empty(capi.kernel_lib().tsvm_smo_solve_workspace(ws), dtype=torch.uint8, device="cuda")
+    for row_type, rows in ((capi.ROW_F64, k_rows), (capi.ROW_F32, k_rows.astype(np.float32))):
+        a_d, k_d = G.dev(alpha), G.dev(rows)
+        ad_d = torch.zeros(ws, dtype=torch.float64, device="cuda")
+        diff_d = torch.zeros(2, dtype=torch.float64, device="cuda")
+        capi.call("tsvm_nu_smo_solve" if nu else "tsvm_c_smo_solve", G.ptr(y_d), G.ptr(f_d), G.ptr(a_d), G.ptr(ad_d), G.ptr(ws_d), ws,
+                  *args, G.ptr(k_d), row_type, None, n, G.ptr(dg_d), eps, G.ptr(diff_d), max_iter, G.ptr(wsp), G.stream())
+        assert np.array_equal(G.host(diff_d), diff_want) if not nu else G.host(diff_d)[0] == diff_want[0]
+        assert np.array_equal(G.host(a_d), a_want, equal_nan=True)
+        assert np.array_equal(G.host(ad_d), ad_want, equal_nan=True)
+
+
 @pytest.mark.parametrize("nu", [False, True])
 @pytest.mark.parametrize("n,ws", [(300, 16), (2000, 1024), (900, 200)])
 def test_smo_solve_block_on_a_chosen_xcd(n, ws, nu):

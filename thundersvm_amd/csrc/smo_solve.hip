@@ -1,22 +1,27 @@
 // The local SMO solvers: c_smo_solve / nu_smo_solve (src/thundersvm/kernel/smo_kernel.cpp:12-287,
 // USE_CUDA=OFF semantics) as one LDS-resident workgroup on gfx950.
 //
-// Shape of the kernel.  One workgroup of 256 threads (one wavefront per SIMD of the CU) holds the
-// whole working set: element t = tid*E + e lives in register slot e of thread tid (E = ws/256
-// slots, up to 4: a thread's elements are neighbours, so its share of a block row is one load) with its f and diagonal; alpha lives in LDS (only two entries change per
-// iteration) and the I_up / I_low membership of a thread's elements is a bit field in one register.
-// One inner iteration is
-//   1. (i, up) = first argmin of f over I_up and low = max of f over I_low: a per-thread scan of
-//      its E slots, a DPP reduction inside each wavefront, four partial results through LDS;
+// Shape of the kernels.  One workgroup of one or four wavefronts (one per SIMD of the CU) holds the whole working set:
+// element t = tid*E + e lives in register slot e of thread tid (a thread's elements are neighbours, so its share of a
+// block row is one load) with its f and diagonal; alpha lives in LDS (only two entries change per iteration) and the
+// I_up / I_low membership of a thread's elements is a bit field in one register.  One inner iteration is
+//   1. (i, up) = first argmin of f over I_up: a per-thread scan of its E slots, a DPP reduction inside each wavefront,
+//      the wavefronts' candidates through LDS;
 //   2. row K[i, .] of the gathered ws x ws block (coalesced);
 //   3. j2 = first argmin of -b^2/a over I_low with f > up: same reduction shape;
 //   4. the two-variable step, row K[j2, .], f -= l * (K[j2, .] - K[i, .]).
-// Two workgroup barriers per iteration.  With one wavefront per SIMD nothing hides an instruction's
-// issue slot or a taken branch, so the loop body is bound by its instruction count: it is written
-// with selects instead of branches (the same loop with if-blocks measured about 1.3x slower), with
-// v_min_f64 / v_max_f64 for the value reductions, and with everything that concerns only the two
-// chosen elements (their alpha, their set membership) computed once per thread from LDS rather than
-// per element.  Reductions are lexicographic (value, element index) minima, so ties go to the lowest
+//
+// What bounds it: one chain of dependent instructions.  With one wavefront per SIMD an instruction takes four cycles
+// whatever it does, an LDS access fifty, a block row 250 (from the L2), a value that crosses to the scalar unit and
+// comes back about forty, a branch around a few instructions about forty-five, and a write or a broadcast read by all
+// 256 threads takes the LDS four wavefronts' worth of cycles.  Hence: no branches inside the loop; what one lane knows is written by that
+// lane alone (exec set to one bit around the write); every wavefront keeps its own copy of alpha; each thread reads one
+// wavefront's candidate and two DPP steps compare them; the winner's index by ballot instead of a second reduction; the
+// exit test folded into the loop's branch (the last round computes a step that is not taken); and everything that does
+// not need the row on its way pinned in front of the first instruction that does.
+// Measured on a call of 483 iterations with ws = 1024: 1.37 us per iteration before that, 1.08 with it (2,590 cycles).
+//
+// Reductions are lexicographic (value, element index) minima, so ties go to the lowest
 // index exactly as the reference's serial loops resolve them, and all arithmetic is the reference's
 // expression order in IEEE double (the library is compiled with -ffp-contract=off; the one fused
 // operation, f -= l*(kJ - kI), is an explicit fma as gcc -O3 contracts it on an FMA host, and
@@ -32,8 +37,7 @@
 
 #define TSVM_INF __builtin_inf()
 #define MAX_WS 1024
-#define SV_T 256           // threads of the solver workgroup
-#define SV_W (SV_T / 64)   // wavefronts
+#define SV_LD 256          // smallest row stride of the ws x ws block
 
 // kws[r*ldk + t] = K_r[working_set[t]] for t < ws, 0 for ws <= t < ldk: the ws x ws block the solver
 // reads, gathered once per call so that the two row reads per inner iteration
@@ -107,69 +111,184 @@ __global__ __launch_bounds__(RA_T) void row_slots_assign_kernel(const int *__res
     if (tid < ws) slots_ws[tid] = slot_of_id[ids_ws[tid]];
 }
 
-// Cross-wavefront combination of the per-wavefront (value, index) minima held in LDS.
-__device__ __forceinline__ void block_argmin(const double *s_v, const int *s_i, double &v, int &i, int none) {
-    double m = s_v[0];
-#pragma unroll
-    for (int w = 1; w < SV_W; ++w) m = fmin_f64(m, s_v[w]);
-    int r = none;
-#pragma unroll
-    for (int w = 0; w < SV_W; ++w) r = imin_sel(r, s_v[w] == m ? s_i[w] : none);
-    v = m;
-    i = r;
+// What a masked-out element or score is replaced by: larger than any f or score of a problem in range.  Only the
+// high word is replaced (one instruction), so every value from SV_NONE on means "not a candidate".
+#define SV_NONE_HI 0x7fe00000
+#define SV_NONE 0x1p1023
+
+// x when the sign bit of `bit_at_top` is set, otherwise a value >= SV_NONE (SIGN = 0) or <= -SV_NONE (SIGN = 1).
+template <int SIGN>
+__device__ __forceinline__ double keep_or_none(unsigned bit_at_top, double x) {
+    const int m = (int) bit_at_top >> 31;
+    return __hiloint2double((m & __double2hiint(x)) | (~m & (int) (SV_NONE_HI | (SIGN ? 0x80000000u : 0u))), __double2loint(x));
 }
+
+// The scalar test for such a value.
+__device__ __forceinline__ bool is_none(double v) { return __builtin_amdgcn_readfirstlane(__double2hiint(v)) >= SV_NONE_HI; }
+
+// The smallest of a wavefront's E * 64 values (x[e] of a lane is element base + e) and the first element that has it:
+// `value` is the minimum; m and at are every lane's own smallest value and its first element; the lane returned is the
+// lowest one whose m is the minimum, so its `at` is the lowest element among equals.
+// With one wavefront per SIMD an instruction costs its four cycles whatever it does, a DPP operand has to be two wait
+// states old, and a value that crosses to the scalar unit and back costs about forty cycles, as much as a branch around
+// a few instructions (all measured on this part).  Hence one chain of six DPP steps on doubles with the instructions
+// that find the thread's own element in its gaps, and the winner by ballot instead of a second chain over the indices.
+#define SV_PIN __builtin_amdgcn_sched_barrier(0)
+// (the same for memory accesses: a row's load stays in front of the work that is to pass while it is on its way, and
+// in front of the exit test; the block is not declared restrict, or the load could be moved all the same)
+#define SV_PIN_MEMORY asm volatile("" ::: "memory")
+template <int E>
+__device__ __forceinline__ int wave_first_argmin(const double (&x)[E], int base, double &value, double &m, int &at) {
+    m = x[0];
+#pragma unroll
+    for (int e = 1; e < E; ++e) m = fmin_f64(m, x[e]);
+    SV_PIN;
+    uint64_t has[E];   // which lanes' element e is their minimum
+#pragma unroll
+    for (int e = 0; e < E - 1; ++e) asm volatile("v_cmp_eq_f64_e64 %0, %1, %2" : "=s"(has[e]) : "v"(x[e]), "v"(m));
+    SV_PIN;
+    int tl = dpp_i32<TSVM_DPP_XOR1>(__double2loint(m)), th = dpp_i32<TSVM_DPP_XOR1>(__double2hiint(m));
+    double r = fmin_f64(m, __hiloint2double(th, tl));
+    SV_PIN;
+    at = base + E - 1;
+#pragma unroll
+    for (int e = E - 2; e >= 0 && e >= E - 3; --e) asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(at) : "v"(at), "v"(base + e), "s"(has[e]));
+    SV_PIN;
+    tl = dpp_i32<TSVM_DPP_XOR2>(__double2loint(r));
+    th = dpp_i32<TSVM_DPP_XOR2>(__double2hiint(r));
+    r = fmin_f64(r, __hiloint2double(th, tl));
+    SV_PIN;
+#pragma unroll
+    for (int e = E - 4; e >= 0; --e) asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(at) : "v"(at), "v"(base + e), "s"(has[e]));
+    SV_PIN;
+    tl = dpp_i32<TSVM_DPP_HALF_MIRROR>(__double2loint(r));
+    th = dpp_i32<TSVM_DPP_HALF_MIRROR>(__double2hiint(r));
+    r = fmin_f64(r, __hiloint2double(th, tl));
+    tl = dpp_i32<TSVM_DPP_MIRROR>(__double2loint(r));
+    th = dpp_i32<TSVM_DPP_MIRROR>(__double2hiint(r));
+    r = fmin_f64(r, __hiloint2double(th, tl));
+    // (lanes outside the row mask keep what the step before moved there, which is no smaller than their own r)
+    tl = __builtin_amdgcn_update_dpp(tl, __double2loint(r), TSVM_DPP_BCAST15, 0xa, 0xf, false);
+    th = __builtin_amdgcn_update_dpp(th, __double2hiint(r), TSVM_DPP_BCAST15, 0xa, 0xf, false);
+    r = fmin_f64(r, __hiloint2double(th, tl));
+    tl = __builtin_amdgcn_update_dpp(tl, __double2loint(r), TSVM_DPP_BCAST31, 0xc, 0xf, false);
+    th = __builtin_amdgcn_update_dpp(th, __double2hiint(r), TSVM_DPP_BCAST31, 0xc, 0xf, false);
+    r = fmin_f64(r, __hiloint2double(th, tl));
+    value = readlane_f64(r, 63);
+    return __builtin_ctzll(__builtin_amdgcn_ballot_w64(m == value));
+}
+
+// The LDS address of a __shared__ object as the ds instructions take it.
+template <typename T>
+__device__ __forceinline__ unsigned lds_at(const T *p) {
+    return (unsigned) (uintptr_t) (const __attribute__((address_space(3))) T *) p;
+}
+
+// One wavefront's best candidate for the others: the workgroup's minimum is taken over W of these.
+struct __align__(16) SvCand {
+    double v;
+    int at;
+    int flag;
+};
+
+// Writes by one lane, without the branch that an if around them costs (all 64 lanes are active before and after).
+// Four wavefronts share the LDS, so a write or a broadcast read by 64 lanes is paid four times over: what one lane
+// knows is written by that lane alone.
+__device__ __forceinline__ void publish(SvCand *slot, int lane, double m, int at, int flag) {
+    typedef int v4i __attribute__((ext_vector_type(4)));
+    const v4i c = {__double2loint(m), __double2hiint(m), at, flag};
+    asm volatile("s_mov_b64 exec, %2\n\tds_write_b128 %0, %1\n\ts_mov_b64 exec, -1"
+                 :: "v"(lds_at(slot)), "v"(c), "s"(1ull << lane) : "memory");
+}
+// The same with the lane's E values of f and of the block row for the step (the row's values in slots of eight bytes).  (One asm statement each: nothing else may
+// come between the two writes of exec.)
+#define SV_EXEC_ON "s_mov_b64 exec, %0\n\t"
+#define SV_EXEC_OFF "s_mov_b64 exec, -1"
+template <int E, typename TB>
+__device__ __forceinline__ void publish_row(double *f_slot, double *k_slot, int lane, const double (&f)[E], const TB (&k)[E]) {
+    const unsigned fa = lds_at(f_slot), ka = lds_at(k_slot);
+    const uint64_t only = 1ull << lane;
+    static_assert(E == 1 || E == 2 || E == 4, "elements per thread");
+    if constexpr (E == 1 && sizeof(TB) == 4)
+        asm volatile(SV_EXEC_ON "ds_write_b64 %1, %3\n\tds_write_b32 %2, %4\n\t" SV_EXEC_OFF
+                     :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(k[0]) : "memory");
+    else if constexpr (E == 1)
+        asm volatile(SV_EXEC_ON "ds_write_b64 %1, %3\n\tds_write_b64 %2, %4\n\t" SV_EXEC_OFF
+                     :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(k[0]) : "memory");
+    else if constexpr (E == 2 && sizeof(TB) == 4)
+        asm volatile(SV_EXEC_ON "ds_write2_b64 %1, %3, %4 offset1:1\n\tds_write2_b32 %2, %5, %6 offset1:2\n\t" SV_EXEC_OFF
+                     :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(f[1]), "v"(k[0]), "v"(k[1]) : "memory");
+    else if constexpr (E == 2)
+        asm volatile(SV_EXEC_ON "ds_write2_b64 %1, %3, %4 offset1:1\n\tds_write2_b64 %2, %5, %6 offset1:1\n\t" SV_EXEC_OFF
+                     :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(f[1]), "v"(k[0]), "v"(k[1]) : "memory");
+    else if constexpr (sizeof(TB) == 4)
+        asm volatile(SV_EXEC_ON "ds_write2_b64 %1, %3, %4 offset1:1\n\tds_write2_b64 %1, %5, %6 offset0:2 offset1:3\n\t"
+                     "ds_write2_b32 %2, %7, %8 offset1:2\n\tds_write2_b32 %2, %9, %10 offset0:4 offset1:6\n\t" SV_EXEC_OFF
+                     :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "v"(k[0]), "v"(k[1]), "v"(k[2]), "v"(k[3]) : "memory");
+    else
+        asm volatile(SV_EXEC_ON "ds_write2_b64 %1, %3, %4 offset1:1\n\tds_write2_b64 %1, %5, %6 offset0:2 offset1:3\n\t"
+                     "ds_write2_b64 %2, %7, %8 offset1:1\n\tds_write2_b64 %2, %9, %10 offset0:2 offset1:3\n\t" SV_EXEC_OFF
+                     :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "v"(k[0]), "v"(k[1]), "v"(k[2]), "v"(k[3]) : "memory");
+}
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+// (p, then q: if both name one element the second value is the final one; `on` = 0: nothing is written)
+__device__ __forceinline__ void write_by_lane0(int on, double *p, double v, double *q, double w) {
+    asm volatile(SV_EXEC_ON "ds_write_b64 %1, %2\n\tds_write_b64 %3, %4\n\t" SV_EXEC_OFF
+                 :: "s"((uint64_t) (uint32_t) __builtin_amdgcn_readfirstlane(on)), "v"(lds_at(p)), "v"(v), "v"(lds_at(q)), "v"(w) : "memory");
+}
+
+// The workgroup's best candidate: every lane reads one of the W, two DPP steps compare them.  The elements of a
+// wavefront are neighbours and the wavefronts follow one another: among equal values the first wavefront has the
+// lowest element.  `at` and `flags` come back as scalars.
+template <int W>
+__device__ __forceinline__ void block_argmin(const SvCand *slots, int lane, double &v, int &at, int &flags) {
+    static_assert(W == 2 || W == 4, "quad_perm steps");
+    const SvCand c = slots[lane & (W - 1)];
+    double m = fmin_f64(c.v, dpp_f64<TSVM_DPP_XOR1>(c.v));
+    if (W == 4) m = fmin_f64(m, dpp_f64<TSVM_DPP_XOR2>(m));
+    v = m;
+    at = __builtin_amdgcn_readlane(c.at, __builtin_ctzll(__builtin_amdgcn_ballot_w64(c.v == m)));
+    flags = __builtin_amdgcn_ballot_w64(c.flag != 0) != 0;
+}
+template <int W>
 __device__ __forceinline__ double block_max(const double *s_v) {
     double v = s_v[0];
 #pragma unroll
-    for (int w = 1; w < SV_W; ++w) v = fmax_f64(v, s_v[w]);
+    for (int w = 1; w < W; ++w) v = fmax_f64(v, s_v[w]);
     return v;
 }
 
-// The wavefront's lexicographic minimum of the candidates x[e] (element index e*256 + tid):
-// value pass, then the smallest element index among those equal to the minimum.  (Taking the index
-// from ballots of x[e] == minimum on the scalar unit instead measured slightly slower.)
-template <int E>
-__device__ __forceinline__ void wave_first_argmin(const double (&x)[E], int tid, double &v, int &idx) {
-    double m = x[0];
-#pragma unroll
-    for (int e = 1; e < E; ++e) m = fmin_f64(m, x[e]);
-    m = wave_min_f64(m);
-    int r = MAX_WS;
-#pragma unroll
-    for (int e = E - 1; e >= 0; --e) r = x[e] == m ? tid * E + e : r;
-    idx = wave_min_i32(r);
-    v = m;
+// Replaces the WIDTH membership bits of element t (the same in all threads) in the bit field of the thread that owns it.
+template <int E, int WIDTH>
+__device__ __forceinline__ unsigned set_member_bits(unsigned m, int tid, int t, unsigned bits) {
+    const int sh = (t & (E - 1)) * WIDTH;
+    const unsigned field = ((1u << WIDTH) - 1u) << sh;
+    const unsigned changed = (m & ~field) | (bits << sh);
+    return tid == (int) ((unsigned) t / E) ? changed : m;
 }
 
-// Replaces the `width` membership bits of element t in the bit field of the thread that owns it.
-template <int E>
-__device__ __forceinline__ unsigned set_member_bits(unsigned m, int tid, int t, unsigned bits, int width) {
-    const int sh = (t % E) * width;
-    const unsigned field = ((1u << width) - 1u) << sh;
-    return tid == t / E ? ((m & ~field) | (bits << sh)) : m;
+// How far alpha can move along its label y = +-1 (y > 0 ? Cp - a : a; the element is in I_up while this is positive)
+// and against it (y > 0 ? a : Cn - a; in I_low while positive), smo_kernel.h:13-23 and smo_kernel.cpp:94-99: one fma
+// each on the half bounds, which rounds exactly as the selected subtraction does.
+__device__ __forceinline__ double room_up(double a, double y, double half_Cp) {
+    return __builtin_fma(-y, a, __builtin_fma(y, half_Cp, half_Cp));
+}
+__device__ __forceinline__ double room_low(double a, double y, double half_Cn) {
+    return __builtin_fma(y, a, __builtin_fma(-y, half_Cn, half_Cn));
 }
 
-// A thread's E consecutive elements of a block row: one 4E- or 8E-byte load, widened to double.
+// A thread's E consecutive elements of a block row: one 4E- or 8E-byte load.
 template <int E, typename TB>
-__device__ __forceinline__ void load_row_elems(const TB *__restrict__ row, int tid, double (&out)[E]) {
+__device__ __forceinline__ void load_row_elems(const TB *__restrict__ row, int tid, TB (&out)[E]) {
     if constexpr (E == 1) {
-        out[0] = (double) row[tid];
+        out[0] = row[tid];
     } else {
         typedef TB vec_t __attribute__((ext_vector_type(E)));
         const vec_t v = *(const vec_t *) (row + tid * E);
 #pragma unroll
-        for (int e = 0; e < E; ++e) out[e] = (double) v[e];
+        for (int e = 0; e < E; ++e) out[e] = v[e];
     }
 }
-
-// Each wavefront knows its own best candidate a barrier and an LDS round trip before the workgroup
-// knows the winner, and the winner is always one of the four.  One load per lane, 128 bytes apart,
-// touches every cache line of a candidate's row, so the row the workgroup then reads is already
-// on its way into the CU's L1 / the XCD's L2 (the four candidates' rows of a float block, 4 KB each, fit the L1 together).
-// A wavefront without a candidate reports an index
-// that may lie beyond the block's ws rows (an inactive element or MAX_WS): it touches row 0 instead.
-#define TSVM_TOUCH_ROW(kws, t, ws, ldk, lane) \
-    (((const unsigned *) ((kws) + (int64_t) ((t) < (ws) ? (t) : 0) * (ldk)))[(lane) * 32 < (int) ((ldk) * sizeof(*(kws)) / 4) ? (lane) * 32 : 0])
 
 // One solver on a chosen XCD.  A kernel of one workgroup runs on whichever XCD its stream's hardware queue starts
 // dealing at; launched as eight workgroups under a CU mask with one CU per XCD, one workgroup lands on every XCD, and
@@ -198,27 +317,124 @@ __device__ __forceinline__ bool solver_elected(int *gate, int epoch, int target_
     return s_elected != 0;
 }
 
+// What the two solvers keep in LDS, per element of the working set.
+template <int N, int W>
+struct SvShared {
+    double kd[N], y[N];       // diagonal, label (0: inactive element)
+    double a[W][N];           // alpha: every wavefront keeps a copy of its own, which needs no barrier
+};
+
+// The iterations of c_smo_solve.  NONE: the threshold is not positive, so that an element may violate it without being
+// a candidate for j2 (the reference's j2 then stays 0, smo_kernel.cpp:78); otherwise that cannot happen.
+template <int E, int W, int LDK, bool NONE, typename TB>
+__device__ __forceinline__ int c_smo_iterate(SvShared<E * 64 * W, W> &sh, double *s_f, double *s_k, SvCand *s_i, SvCand *s_j, int ws, double Cp,
+                                             double Cn, const TB *kws, const double (&kd)[E], double (&f)[E], unsigned member,
+                                             double local_eps, int max_iter) {
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const double half_Cp = 0.5 * Cp, half_Cn = 0.5 * Cn;
+    int numOfIter = 0;
+    bool go_on;
+    do {
+        // i = first argmin of f over I_up (smo_kernel.cpp:41-59); with an empty I_up any i does, since nothing violates then
+        double fu[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) fu[e] = keep_or_none<0>(member << (31 - 2 * e), f[e]);
+        double up_value, m;
+        int at, i, j2, go;
+        const int win_i = wave_first_argmin<E>(fu, tid * E, up_value, m, at);
+        if constexpr (W > 1) {
+            publish(s_i + wave, win_i, m, at, 0);
+            lds_barrier();
+            block_argmin<W>(s_i, lane, up_value, i, go);
+        } else {
+            i = __builtin_amdgcn_readlane(at, win_i);
+        }
+        i = i < ws ? i : ws - 1;   // (without a candidate the index may be an inactive element's)
+        TB kI[E];
+        load_row_elems<E, TB>(kws + (unsigned) i * (unsigned) LDK, tid, kI);
+        SV_PIN_MEMORY;
+        const double kd_i = sh.kd[i], y_i = sh.y[i], a_i = sh.a[wave][i];
+        double a_part[E], b_low[E], b_max = -TSVM_INF;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            a_part[e] = kd_i + kd[e];
+            b_low[e] = keep_or_none<1>(member << (30 - 2 * e), -up_value + f[e]);
+            b_max = e == 0 ? b_low[e] : fmax_f64(b_max, b_low[e]);
+        }
+        // some I_low element still violates: low - up >= local_eps (smo_kernel.cpp:68)
+        go = __builtin_amdgcn_ballot_w64(!(b_max < local_eps)) != 0;
+        double up_i = room_up(a_i, y_i, half_Cp);
+        asm("" : "+v"(up_i));
+        SV_PIN;   // (all of this while the row is on its way)
+        // j2 = first argmin of -b^2/a over I_low with f > up (smo_kernel.cpp:77-90)
+        double qs[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const double aIJ = __builtin_fma(-2.0, (double) kI[e], a_part[e]);
+            const double q = -b_low[e] * b_low[e] / aIJ;
+            // (-up > -f in the reference: f > up, which is b > 0; outside I_low b is negative and q of no use)
+            qs[e] = __hiloint2double(b_low[e] > 0.0 ? __double2hiint(q) : SV_NONE_HI, __double2loint(q));
+        }
+        double min_t;
+        const int win_j = wave_first_argmin<E>(qs, tid * E, min_t, m, at);
+        publish_row<E, TB>(s_f + tid * E, s_k + tid * E, win_j, f, kI);
+        if constexpr (W > 1) {
+            publish(s_j + wave, win_j, m, at, go);
+            lds_barrier();
+            block_argmin<W>(s_j, lane, min_t, j2, go);
+        } else {
+            j2 = __builtin_amdgcn_readlane(at, win_j);
+        }
+        if (NONE && is_none(min_t)) {
+            j2 = 0;
+            __syncthreads();
+            if (tid == 0) { s_f[0] = f[0]; *(TB *) s_k = kI[0]; }
+            __syncthreads();
+        }
+        j2 = j2 < ws ? j2 : ws - 1;
+        TB kJ[E];
+        load_row_elems<E, TB>(kws + (unsigned) j2 * (unsigned) LDK, tid, kJ);
+        SV_PIN_MEMORY;
+        const double kd_j = sh.kd[j2], y_j = sh.y[j2], a_j = sh.a[wave][j2], f_j = s_f[j2];
+        const double kIj = (double) *(const TB *) (s_k + j2);
+        SV_PIN;   // the row is on its way while the step is computed
+        // two-variable step (smo_kernel.cpp:92-103; the last round computes one that is not taken)
+        go_on = go && !(numOfIter > max_iter);
+        const double q2 = (-up_value + f_j) / __builtin_fma(-2.0, kIj, kd_i + kd_j);
+        const double l = fmin_f64(up_i, fmin_f64(room_low(a_j, y_j, half_Cn), q2));
+        const double na_i = __builtin_fma(l, y_i, a_i), na_j = __builtin_fma(-l, y_j, NONE && j2 == i ? na_i : a_j);
+        member = set_member_bits<E, 2>(member, tid, i, (room_up(na_i, y_i, half_Cp) > 0 ? 1u : 0u) | (room_low(na_i, y_i, half_Cn) > 0 ? 2u : 0u));
+        member = set_member_bits<E, 2>(member, tid, j2, (room_up(na_j, y_j, half_Cp) > 0 ? 1u : 0u) | (room_low(na_j, y_j, half_Cn) > 0 ? 2u : 0u));
+        write_by_lane0(go_on, &sh.a[wave][i], na_i, &sh.a[wave][j2], na_j);
+        SV_PIN;   // (nothing above waits for the row)
+#pragma unroll
+        for (int e = 0; e < E; ++e) f[e] = __builtin_fma(-l, (double) kJ[e] - (double) kI[e], f[e]);
+        numOfIter += go_on;
+    } while (go_on);
+    return numOfIter;
+}
+
 // Elements beyond ws are given y = 0, which puts them in neither I_up nor I_low.
-template <int E, typename TB>
-__global__ __launch_bounds__(SV_T) void c_smo_solve_kernel(
+// E elements per thread, W wavefronts; LDK: row stride of the block (E * 64 * W <= LDK).
+template <int E, int W, int LDK, typename TB>
+__global__ __launch_bounds__(64 * W) void c_smo_solve_kernel(
     const int *__restrict__ label, const double *__restrict__ f_val, double *__restrict__ alpha,
     double *__restrict__ alpha_diff, const int *__restrict__ working_set, int ws, double Cp, double Cn,
-    const TB *__restrict__ kws, const double *__restrict__ k_diag, double eps, double *__restrict__ diff,
+    const TB *kws, const double *__restrict__ k_diag, double eps, double *__restrict__ diff,
     int max_iter, int *__restrict__ gate, int epoch, int target_xcd) {
     if (gate && !solver_elected(gate, epoch, target_xcd)) return;
-    constexpr int LDK = E * SV_T;
-    __shared__ double s_kd[LDK];
-    __shared__ float s_y[LDK];
-    __shared__ double s_a[LDK];
-    __shared__ double s_f[2][LDK];
-    __shared__ double sA_v[SV_W], sA_l[SV_W], sB_v[SV_W];
-    __shared__ int sA_i[SV_W], sB_i[SV_W], sB_go[SV_W];
+    constexpr int N = E * 64 * W;
+    __shared__ SvShared<N, W> sh;
+    __shared__ double s_f[N], s_k[N];   // f and row i at the elements of the wavefronts' candidates for j2 (the others are not written)
+    __shared__ double s_red[2][W];
+    __shared__ SvCand s_i[W], s_j[W];
 
     // This workgroup is a chain of dependent operations; when a chip-wide kernel runs next to it on
     // another stream its wavefronts must not wait behind that kernel's for issue slots.
     __builtin_amdgcn_s_setprio(3);
     const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     double f[E], a_old[E], kd[E];
     unsigned member = 0;   // bit 2e: element e is in I_up; bit 2e+1: in I_low
 #pragma unroll
@@ -230,15 +446,12 @@ __global__ __launch_bounds__(SV_T) void c_smo_solve_kernel(
         a_old[e] = active ? alpha[w] : 0.0;
         const double y = active ? (double) label[w] : 0.0;
         kd[e] = active ? k_diag[w] : 1.0;
-        s_kd[t] = kd[e];
-        s_y[t] = (float) y;
-        s_a[t] = a_old[e];
+        sh.kd[t] = kd[e];
+        sh.y[t] = y;
+#pragma unroll
+        for (int w = 0; w < W; ++w) sh.a[w][t] = a_old[e];
         member |= ((is_I_up(a_old[e], y, Cp, Cn) ? 1u : 0u) | (is_I_low(a_old[e], y, Cp, Cn) ? 2u : 0u)) << (2 * e);
     }
-    // The alpha of the two elements changed by an iteration is written to LDS by thread 0 after the
-    // next iteration's first barrier, when no wavefront can still be reading the old values.
-    int pend_i = 0, pend_j = 0;
-    double pend_ai = a_old[0], pend_aj = a_old[0];   // for thread 0 this is s_a[0]: the first write changes nothing
     // The initial gap fixes the local stopping threshold (smo_kernel.cpp:61-66).  It is the only place
     // where the value of low = max of f over I_low is needed: inside the loop the stopping test
     // low - up < local_eps is evaluated per element, as "no I_low element has f - up >= local_eps"
@@ -254,105 +467,25 @@ __global__ __launch_bounds__(SV_T) void c_smo_solve_kernel(
         }
         mn = wave_min_f64(mn);
         mx = wave_max_f64(mx);
-        if (lane == 0) { sA_v[wave] = mn; sA_l[wave] = mx; }
+        if (lane == 0) { s_red[0][wave] = mn; s_red[1][wave] = mx; }
         __syncthreads();
-        double up0 = sA_v[0];
+        double up0 = s_red[0][0];
 #pragma unroll
-        for (int w = 1; w < SV_W; ++w) up0 = fmin_f64(up0, sA_v[w]);
-        const double local_diff = block_max(sA_l) - up0;
+        for (int w = 1; w < W; ++w) up0 = fmin_f64(up0, s_red[0][w]);
+        const double local_diff = block_max<W>(s_red[1]) - up0;
         const double t = 0.1f * local_diff;   // float literal, as in the reference (smo_kernel.cpp:64)
         local_eps = eps > t ? eps : t;
         if (tid == 0) diff[0] = local_diff;
-        __syncthreads();   // sA_* are written again below
     }
-    int numOfIter = 0;
-    unsigned touched = 0;
-    while (true) {
-        const int par = numOfIter & 1;
-        // i = first argmin of f over I_up (smo_kernel.cpp:41-59)
-        double fu[E];
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            s_f[par][tid * E + e] = f[e];
-            fu[e] = (member >> (2 * e)) & 1u ? f[e] : TSVM_INF;
-        }
-        double v;
-        int vi;
-        wave_first_argmin<E>(fu, tid, v, vi);
-        const unsigned pre_i = TSVM_TOUCH_ROW(kws, vi, ws, LDK, lane);
-        if (lane == 0) { sA_v[wave] = v; sA_i[wave] = vi; }
-        __syncthreads();
-        if (tid == 0) {
-            s_a[pend_i] = pend_ai;
-            s_a[pend_j] = pend_aj;   // after pend_i: if both name one element the second value is the final one
-        }
-        double up_value;
-        int i;
-        block_argmin(sA_v, sA_i, up_value, i, MAX_WS);
-        i = up_value < TSVM_INF ? i : 0;
-        const TB *row_i = kws + (int64_t) i * LDK;
-        double kI[E];
-        load_row_elems<E, TB>(row_i, tid, kI);
-        const double kd_i = s_kd[i];
-        // j2 = first argmin of -b^2/a over I_low with f > up (smo_kernel.cpp:77-90)
-        double qs[E];
-        bool go = false;   // some I_low element still violates: low - up >= local_eps (smo_kernel.cpp:68)
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            const bool low = (member >> (2 * e + 1)) & 1u;
-            const double aIJ = __builtin_fma(-2.0, kI[e], kd_i + kd[e]);
-            const double bIJ = -up_value + f[e];
-            const double q = -bIJ * bIJ / aIJ;
-            qs[e] = low && (-up_value > -f[e]) ? q : TSVM_INF;
-            go |= low && !(f[e] - up_value < local_eps);
-        }
-        double ft;
-        int fi;
-        wave_first_argmin<E>(qs, tid, ft, fi);
-        const unsigned pre_j = TSVM_TOUCH_ROW(kws, fi, ws, LDK, lane);
-        const bool wave_go = __builtin_amdgcn_ballot_w64(go) != 0;
-        if (lane == 0) { sB_v[wave] = ft; sB_i[wave] = fi; sB_go[wave] = wave_go; }
-        __syncthreads();
-        bool any_go = false;
-#pragma unroll
-        for (int w = 0; w < SV_W; ++w) any_go |= sB_go[w] != 0;
-        if (numOfIter > max_iter || !any_go) break;
-        double min_t;
-        int j2;
-        block_argmin(sB_v, sB_i, min_t, j2, MAX_WS);
-        j2 = min_t < TSVM_INF ? j2 : 0;
-        const TB *row_j = kws + (int64_t) j2 * LDK;
-        double kJ[E];
-        load_row_elems<E, TB>(row_j, tid, kJ);
-        const double kIj = (double) row_i[j2];
-        // two-variable step (smo_kernel.cpp:92-103)
-        const double a_i = s_a[i], y_i = (double) s_y[i];
-        const double a_j0 = s_a[j2], y_j = (double) s_y[j2];
-        const double alpha_i_diff = y_i > 0 ? Cp - a_i : a_i;
-        const double q1 = y_j > 0 ? a_j0 : Cn - a_j0;
-        const double q2 = (-up_value + s_f[par][j2]) / (kd_i + s_kd[j2] - 2 * kIj);
-        const double alpha_j_diff = q1 < q2 ? q1 : q2;
-        const double l = alpha_i_diff < alpha_j_diff ? alpha_i_diff : alpha_j_diff;
-        const double na_i = a_i + l * y_i;
-        const double na_j = (j2 == i ? na_i : a_j0) - l * y_j;
-        member = set_member_bits<E>(member, tid, i, (is_I_up(na_i, y_i, Cp, Cn) ? 1u : 0u) | (is_I_low(na_i, y_i, Cp, Cn) ? 2u : 0u), 2);
-        member = set_member_bits<E>(member, tid, j2, (is_I_up(na_j, y_j, Cp, Cn) ? 1u : 0u) | (is_I_low(na_j, y_j, Cp, Cn) ? 2u : 0u), 2);
-        pend_i = i;
-        pend_j = j2;
-        pend_ai = na_i;
-        pend_aj = na_j;
-#pragma unroll
-        for (int e = 0; e < E; ++e) f[e] = __builtin_fma(-l, kJ[e] - kI[e], f[e]);
-        touched ^= pre_i ^ pre_j;
-        ++numOfIter;
-    }
-    __syncthreads();   // the pending alpha writes of the last step were made before the loop's exit test
+    const int numOfIter = __builtin_amdgcn_readfirstlane(local_eps > 0.0 ? 1 : 0)
+                              ? c_smo_iterate<E, W, LDK, false, TB>(sh, s_f, s_k, s_i, s_j, ws, Cp, Cn, kws, kd, f, member, local_eps, max_iter)
+                              : c_smo_iterate<E, W, LDK, true, TB>(sh, s_f, s_k, s_i, s_j, ws, Cp, Cn, kws, kd, f, member, local_eps, max_iter);
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const int t = tid * E + e;
         if (t < ws) {
-            const double a = s_a[t];
-            alpha_diff[t] = -(a - a_old[e]) * (double) s_y[t];
+            const double a = sh.a[wave][t];
+            alpha_diff[t] = -(a - a_old[e]) * sh.y[t];
             alpha[working_set[t]] = a;
         }
     }
@@ -362,35 +495,33 @@ __global__ __launch_bounds__(SV_T) void c_smo_solve_kernel(
         __threadfence_system();
         diff[1] = (double) numOfIter;
     }
-    if (touched == 0x7ff00001u && numOfIter < 0) diff[0] = 0.0;   // keeps the row-touching loads alive; never true
 }
 
 // nu variant (smo_kernel.cpp:127-287): four extrema, two second-order candidates.  Keeps the CPU
 // code's j2n score, which uses kd[ip] and K[ip, .] (smo_kernel.cpp:239), and leaves diff[1] alone.
 // Membership bits per element: 0 = y>0 & a<C (I_up, positive), 1 = y<0 & a>0 (I_up, negative),
 // 2 = y>0 & a>0 (I_low, positive), 3 = y<0 & a<C (I_low, negative).
-__device__ __forceinline__ unsigned nu_member_bits(double a, double y, double C) {
-    return (y > 0 && a < C ? 1u : 0u) | (y < 0 && a > 0 ? 2u : 0u) | (y > 0 && a > 0 ? 4u : 0u) | (y < 0 && a < C ? 8u : 0u);
+__device__ __forceinline__ unsigned nu_member_bits(double a, double y, double half_C) {
+    const unsigned b = (room_up(a, y, half_C) > 0 ? 1u : 0u) | (room_low(a, y, half_C) > 0 ? 4u : 0u);
+    return y > 0 ? b : b << 1;
 }
 
-template <int E, typename TB>
-__global__ __launch_bounds__(SV_T) void nu_smo_solve_kernel(
+template <int E, int W, int LDK, typename TB>
+__global__ __launch_bounds__(64 * W) void nu_smo_solve_kernel(
     const int *__restrict__ label, const double *__restrict__ f_val, double *__restrict__ alpha,
     double *__restrict__ alpha_diff, const int *__restrict__ working_set, int ws, double C,
-    const TB *__restrict__ kws, const double *__restrict__ k_diag, double eps, double *__restrict__ diff,
+    const TB *kws, const double *__restrict__ k_diag, double eps, double *__restrict__ diff,
     int max_iter, int *__restrict__ gate, int epoch, int target_xcd) {
     if (gate && !solver_elected(gate, epoch, target_xcd)) return;
-    constexpr int LDK = E * SV_T;
-    __shared__ double s_kd[LDK];
-    __shared__ float s_y[LDK];
-    __shared__ double s_a[LDK];
-    __shared__ double s_f[2][LDK];
-    __shared__ double sA_vp[SV_W], sA_vn[SV_W], sA_lp[SV_W], sA_ln[SV_W], sB_vp[SV_W], sB_vn[SV_W];
-    __shared__ int sA_ip[SV_W], sA_in[SV_W], sB_ip[SV_W], sB_in[SV_W], sB_go[SV_W];
+    constexpr int N = E * 64 * W;
+    __shared__ SvShared<N, W> sh;
+    __shared__ double s_f[2][N], s_k[2][N];   // f and the rows ip / in at the elements of the wavefronts' candidates for j2
+    __shared__ double s_red[4][W];
+    __shared__ SvCand s_ip[W], s_in[W], s_jp[W], s_jn[W];
 
     __builtin_amdgcn_s_setprio(3);
     const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     double f[E], a_old[E], kd[E];
     unsigned member = 0;
 #pragma unroll
@@ -402,13 +533,12 @@ __global__ __launch_bounds__(SV_T) void nu_smo_solve_kernel(
         a_old[e] = active ? alpha[w] : 0.0;
         const double y = active ? (double) label[w] : 0.0;
         kd[e] = active ? k_diag[w] : 1.0;
-        s_kd[t] = kd[e];
-        s_y[t] = (float) y;
-        s_a[t] = a_old[e];
-        member |= nu_member_bits(a_old[e], y, C) << (4 * e);
+        sh.kd[t] = kd[e];
+        sh.y[t] = y;
+#pragma unroll
+        for (int w = 0; w < W; ++w) sh.a[w][t] = a_old[e];
+        member |= (active ? nu_member_bits(a_old[e], y, 0.5 * C) : 0u) << (4 * e);
     }
-    int pend_i = 0, pend_j = 0;
-    double pend_ai = a_old[0], pend_aj = a_old[0];
     // initial gap -> local stopping threshold (smo_kernel.cpp:176-183); inside the loop the stopping
     // test is evaluated per element, as in the C variant
     double local_eps, first_diff;
@@ -426,118 +556,124 @@ __global__ __launch_bounds__(SV_T) void nu_smo_solve_kernel(
         mnn = wave_min_f64(mnn);
         mxp = wave_max_f64(mxp);
         mxn = wave_max_f64(mxn);
-        if (lane == 0) { sA_vp[wave] = mnp; sA_vn[wave] = mnn; sA_lp[wave] = mxp; sA_ln[wave] = mxn; }
+        if (lane == 0) { s_red[0][wave] = mnp; s_red[1][wave] = mnn; s_red[2][wave] = mxp; s_red[3][wave] = mxn; }
         __syncthreads();
-        double up_p0 = sA_vp[0], up_n0 = sA_vn[0];
+        double up_p0 = s_red[0][0], up_n0 = s_red[1][0];
 #pragma unroll
-        for (int w = 1; w < SV_W; ++w) { up_p0 = fmin_f64(up_p0, sA_vp[w]); up_n0 = fmin_f64(up_n0, sA_vn[w]); }
-        const double dp = block_max(sA_lp) - up_p0, dn = block_max(sA_ln) - up_n0;
+        for (int w = 1; w < W; ++w) { up_p0 = fmin_f64(up_p0, s_red[0][w]); up_n0 = fmin_f64(up_n0, s_red[1][w]); }
+        const double dp = block_max<W>(s_red[2]) - up_p0, dn = block_max<W>(s_red[3]) - up_n0;
         const double local_diff = dp > dn ? dp : dn;
         const double t = 0.1 * local_diff;
         local_eps = eps > t ? eps : t;
         first_diff = local_diff;
-        __syncthreads();
     }
+    __syncthreads();
+    const bool none_possible = __builtin_amdgcn_readfirstlane(local_eps > 0.0 ? 0 : 1) != 0;
+    const double half_C = 0.5 * C;
     int numOfIter = 0;
-    unsigned touched = 0;
     while (true) {
-        const int par = numOfIter & 1;
         double fup[E], fun[E];
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            s_f[par][tid * E + e] = f[e];
-            const unsigned b = member >> (4 * e);
-            fup[e] = b & 1u ? f[e] : TSVM_INF;
-            fun[e] = b & 2u ? f[e] : TSVM_INF;
+            fup[e] = keep_or_none<0>(member << (31 - 4 * e), f[e]);
+            fun[e] = keep_or_none<0>(member << (30 - 4 * e), f[e]);
         }
-        double vp, vn;
-        int ipi, ini;
-        wave_first_argmin<E>(fup, tid, vp, ipi);
-        wave_first_argmin<E>(fun, tid, vn, ini);
-        const unsigned pre_i = TSVM_TOUCH_ROW(kws, ipi, ws, LDK, lane) ^ TSVM_TOUCH_ROW(kws, ini, ws, LDK, lane);
-        if (lane == 0) { sA_vp[wave] = vp; sA_ip[wave] = ipi; sA_vn[wave] = vn; sA_in[wave] = ini; }
-        __syncthreads();
-        if (tid == 0) {
-            s_a[pend_i] = pend_ai;
-            s_a[pend_j] = pend_aj;
+        double up_value_p, up_value_n, m_p, m_n;
+        int ip, in, at_p, at_n, go;
+        const int win_ip = wave_first_argmin<E>(fup, tid * E, up_value_p, m_p, at_p);
+        const int win_in = wave_first_argmin<E>(fun, tid * E, up_value_n, m_n, at_n);
+        if constexpr (W > 1) {
+            publish(s_ip + wave, win_ip, m_p, at_p, 0);
+            publish(s_in + wave, win_in, m_n, at_n, 0);
+            lds_barrier();
+            block_argmin<W>(s_ip, lane, up_value_p, ip, go);
+            block_argmin<W>(s_in, lane, up_value_n, in, go);
+        } else {
+            ip = __builtin_amdgcn_readlane(at_p, win_ip);
+            in = __builtin_amdgcn_readlane(at_n, win_in);
         }
-        double up_value_p, up_value_n;
-        int ip, in;
-        block_argmin(sA_vp, sA_ip, up_value_p, ip, MAX_WS);
-        block_argmin(sA_vn, sA_in, up_value_n, in, MAX_WS);
-        ip = up_value_p < TSVM_INF ? ip : 0;
-        in = up_value_n < TSVM_INF ? in : 0;
-        const TB *row_p = kws + (int64_t) ip * LDK;
-        const TB *row_n = kws + (int64_t) in * LDK;
-        double kIp[E], kIn[E];
-        load_row_elems<E, TB>(row_p, tid, kIp);
-        load_row_elems<E, TB>(row_n, tid, kIn);
-        const double kd_ip = s_kd[ip];
-        double qp[E], qn[E];
-        bool go = false;   // max(low_p - up_p, low_n - up_n) >= local_eps (smo_kernel.cpp:185)
+        // (an empty side's index stays 0: its row enters the other side's scores, smo_kernel.cpp:239)
+        ip = is_none(up_value_p) ? 0 : ip;
+        in = is_none(up_value_n) ? 0 : in;
+        TB kIp[E], kIn[E];
+        load_row_elems<E, TB>(kws + (unsigned) ip * (unsigned) LDK, tid, kIp);
+        load_row_elems<E, TB>(kws + (unsigned) in * (unsigned) LDK, tid, kIn);
+        SV_PIN_MEMORY;
+        const double kd_ip = sh.kd[ip], kd_in = sh.kd[in];
+        double a_part[E], lp[E], ln[E], b_max = -TSVM_INF;
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            const unsigned b = member >> (4 * e);
-            const double aIJ = __builtin_fma(-2.0, kIp[e], kd_ip + kd[e]);
-            const double bp = -up_value_p + f[e], bn = -up_value_n + f[e];
-            qp[e] = (b & 4u) && (-up_value_p > -f[e]) ? -bp * bp / aIJ : TSVM_INF;
-            qn[e] = (b & 8u) && (-up_value_n > -f[e]) ? -bn * bn / aIJ : TSVM_INF;
-            go |= ((b & 4u) && !(f[e] - up_value_p < local_eps)) || ((b & 8u) && !(f[e] - up_value_n < local_eps));
+            a_part[e] = kd_ip + kd[e];
+            lp[e] = keep_or_none<1>(member << (29 - 4 * e), -up_value_p + f[e]);
+            ln[e] = keep_or_none<1>(member << (28 - 4 * e), -up_value_n + f[e]);
+            b_max = fmax_f64(e == 0 ? lp[e] : fmax_f64(b_max, lp[e]), ln[e]);
         }
-        double ftp, ftn;
-        int jpi, jni;
-        wave_first_argmin<E>(qp, tid, ftp, jpi);
-        wave_first_argmin<E>(qn, tid, ftn, jni);
-        const unsigned pre_j = TSVM_TOUCH_ROW(kws, jpi, ws, LDK, lane) ^ TSVM_TOUCH_ROW(kws, jni, ws, LDK, lane);
-        const bool wave_go = __builtin_amdgcn_ballot_w64(go) != 0;
-        if (lane == 0) { sB_vp[wave] = ftp; sB_ip[wave] = jpi; sB_vn[wave] = ftn; sB_in[wave] = jni; sB_go[wave] = wave_go; }
-        __syncthreads();
-        bool any_go = false;
+        // max(low_p - up_p, low_n - up_n) >= local_eps (smo_kernel.cpp:185)
+        go = __builtin_amdgcn_ballot_w64(!(b_max < local_eps)) != 0;
+        SV_PIN;   // (all of this while the rows are on their way)
+        double qp[E], qn[E];
 #pragma unroll
-        for (int w = 0; w < SV_W; ++w) any_go |= sB_go[w] != 0;
-        if (numOfIter > max_iter || !any_go) break;
+        for (int e = 0; e < E; ++e) {
+            const double aIJ = __builtin_fma(-2.0, (double) kIp[e], a_part[e]);
+            const double q_p = -lp[e] * lp[e] / aIJ, q_n = -ln[e] * ln[e] / aIJ;
+            // (-up > -f in the reference: f > up)
+            qp[e] = __hiloint2double(lp[e] > 0.0 ? __double2hiint(q_p) : SV_NONE_HI, __double2loint(q_p));
+            qn[e] = __hiloint2double(ln[e] > 0.0 ? __double2hiint(q_n) : SV_NONE_HI, __double2loint(q_n));
+        }
         double f_val_j2p, f_val_j2n;
         int j2p, j2n;
-        block_argmin(sB_vp, sB_ip, f_val_j2p, j2p, MAX_WS);
-        block_argmin(sB_vn, sB_in, f_val_j2n, j2n, MAX_WS);
-        j2p = f_val_j2p < TSVM_INF ? j2p : 0;
-        j2n = f_val_j2n < TSVM_INF ? j2n : 0;
-        const bool take_p = f_val_j2p < f_val_j2n;
+        const int win_jp = wave_first_argmin<E>(qp, tid * E, f_val_j2p, m_p, at_p);
+        const int win_jn = wave_first_argmin<E>(qn, tid * E, f_val_j2n, m_n, at_n);
+        publish_row<E, TB>(s_f[0] + tid * E, s_k[0] + tid * E, win_jp, f, kIp);
+        publish_row<E, TB>(s_f[1] + tid * E, s_k[1] + tid * E, win_jn, f, kIn);
+        if constexpr (W > 1) {
+            publish(s_jp + wave, win_jp, m_p, at_p, go);
+            publish(s_jn + wave, win_jn, m_n, at_n, go);
+            lds_barrier();
+            block_argmin<W>(s_jp, lane, f_val_j2p, j2p, go);
+            int go_n;
+            block_argmin<W>(s_jn, lane, f_val_j2n, j2n, go_n);
+        } else {
+            j2p = __builtin_amdgcn_readlane(at_p, win_jp);
+            j2n = __builtin_amdgcn_readlane(at_n, win_jn);
+        }
+        // (two sides without a candidate are equal, whatever the low words of their values hold)
+        const bool take_p = __builtin_amdgcn_readfirstlane(f_val_j2p < f_val_j2n && f_val_j2p < SV_NONE ? 1 : 0) != 0;
+        const int side = take_p ? 0 : 1;
         const int i = take_p ? ip : in;
-        const int j2 = take_p ? j2p : j2n;
+        int j2 = take_p ? j2p : j2n;
+        if (none_possible && is_none(take_p ? f_val_j2p : f_val_j2n)) {
+            j2 = 0;
+            __syncthreads();
+            if (tid == 0) { s_f[side][0] = f[0]; *(TB *) s_k[side] = take_p ? kIp[0] : kIn[0]; }
+            __syncthreads();
+        }
+        j2 = j2 < ws ? j2 : ws - 1;
+        TB kJ[E];
+        load_row_elems<E, TB>(kws + (unsigned) j2 * (unsigned) LDK, tid, kJ);
+        SV_PIN_MEMORY;
+        const double kd_j = sh.kd[j2], y_j = sh.y[j2], a_j = sh.a[wave][j2], y_i = sh.y[i], a_i = sh.a[wave][i], f_j = s_f[side][j2];
+        const double kIj = (double) *(const TB *) (s_k[side] + j2);
+        SV_PIN;   // the row is on its way while the exit test and the step are computed
+        if (numOfIter > max_iter || !go) break;
         const double up_value = take_p ? up_value_p : up_value_n;
-        const TB *row_i = take_p ? row_p : row_n;
-        const TB *row_j = kws + (int64_t) j2 * LDK;
-        double kJ[E];
-        load_row_elems<E, TB>(row_j, tid, kJ);
-        const double kIj = (double) row_i[j2];
-        const double a_i = s_a[i], y_i = (double) s_y[i];
-        const double a_j0 = s_a[j2], y_j = (double) s_y[j2];
-        const double alpha_i_diff = y_i > 0 ? C - a_i : a_i;
-        const double q1 = y_j > 0 ? a_j0 : C - a_j0;
-        const double q2 = (-up_value + s_f[par][j2]) / (s_kd[i] + s_kd[j2] - 2 * kIj);
-        const double alpha_j_diff = q1 < q2 ? q1 : q2;
-        const double l = alpha_i_diff < alpha_j_diff ? alpha_i_diff : alpha_j_diff;
-        const double na_i = a_i + l * y_i;
-        const double na_j = (j2 == i ? na_i : a_j0) - l * y_j;
-        member = set_member_bits<E>(member, tid, i, nu_member_bits(na_i, y_i, C), 4);
-        member = set_member_bits<E>(member, tid, j2, nu_member_bits(na_j, y_j, C), 4);
-        pend_i = i;
-        pend_j = j2;
-        pend_ai = na_i;
-        pend_aj = na_j;
+        const double q2 = (-up_value + f_j) / __builtin_fma(-2.0, kIj, (take_p ? kd_ip : kd_in) + kd_j);
+        const double l = fmin_f64(room_up(a_i, y_i, half_C), fmin_f64(room_low(a_j, y_j, half_C), q2));
+        const double na_i = __builtin_fma(l, y_i, a_i), na_j = __builtin_fma(-l, y_j, j2 == i ? na_i : a_j);   // (labels are +-1: exact products)
+        member = set_member_bits<E, 4>(member, tid, i, nu_member_bits(na_i, y_i, half_C));
+        member = set_member_bits<E, 4>(member, tid, j2, nu_member_bits(na_j, y_j, half_C));
+        write_by_lane0(1, &sh.a[wave][i], na_i, &sh.a[wave][j2], na_j);
+        SV_PIN;   // (nothing above waits for the row)
 #pragma unroll
-        for (int e = 0; e < E; ++e) f[e] = __builtin_fma(-l, kJ[e] - (take_p ? kIp[e] : kIn[e]), f[e]);
-        touched ^= pre_i ^ pre_j;
+        for (int e = 0; e < E; ++e) f[e] = __builtin_fma(-l, (double) kJ[e] - (double) (take_p ? kIp[e] : kIn[e]), f[e]);
         ++numOfIter;
     }
-    __syncthreads();
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const int t = tid * E + e;
         if (t < ws) {
-            const double a = s_a[t];
-            alpha_diff[t] = -(a - a_old[e]) * (double) s_y[t];
+            const double a = sh.a[wave][t];
+            alpha_diff[t] = -(a - a_old[e]) * sh.y[t];
             alpha[working_set[t]] = a;
         }
     }
@@ -547,7 +683,6 @@ __global__ __launch_bounds__(SV_T) void nu_smo_solve_kernel(
         __threadfence_system();
         diff[0] = first_diff;
     }
-    if (touched == 0x7ff00001u && numOfIter < 0) diff[0] = 0.0;   // keeps the row-touching loads alive; never true
 }
 
 // The solver workgroup asks for the rest of the CU's 160 KB of LDS as (unused) dynamic shared memory:
@@ -581,7 +716,7 @@ static int solver_dyn_lds(const void *kernel, size_t *dyn) {
 
 extern "C" {
 
-static int solver_ldk(int ws_size) { return ws_size <= SV_T ? SV_T : (ws_size <= 2 * SV_T ? 2 * SV_T : 4 * SV_T); }
+static int solver_ldk(int ws_size) { return ws_size <= SV_LD ? SV_LD : (ws_size <= 2 * SV_LD ? 2 * SV_LD : 4 * SV_LD); }
 
 size_t tsvm_smo_solve_workspace(int ws_size) {
     if (ws_size < 0) return 0;
@@ -610,21 +745,26 @@ static int launch_gather(const void *k_rows, int row_type, const int *slots, int
     return 0;
 }
 
-#define TSVM_LAUNCH_SOLVER(KERNEL, EVAL, TB, ...)                                                   \
-    do {                                                                                            \
-        size_t dyn_ = 0;                                                                            \
-        if (solver_grid_ == 1) {                                                                    \
-            const int rc_ = solver_dyn_lds(reinterpret_cast<const void *>(KERNEL<EVAL, TB>), &dyn_); \
-            if (rc_) return rc_;                                                                    \
-        }                                                                                           \
-        hipLaunchKernelGGL((KERNEL<EVAL, TB>), dim3(solver_grid_), dim3(SV_T), dyn_, s, __VA_ARGS__); \
+#define TSVM_LAUNCH_SOLVER(KERNEL, TB, EVAL, WVAL, LDKVAL, ...)                                                \
+    do {                                                                                                       \
+        size_t dyn_ = 0;                                                                                       \
+        if (solver_grid_ == 1) {                                                                               \
+            const int rc_ = solver_dyn_lds(reinterpret_cast<const void *>(KERNEL<EVAL, WVAL, LDKVAL, TB>), &dyn_); \
+            if (rc_) return rc_;                                                                               \
+        }                                                                                                      \
+        hipLaunchKernelGGL((KERNEL<EVAL, WVAL, LDKVAL, TB>), dim3(solver_grid_), dim3(64 * WVAL), dyn_, s, __VA_ARGS__); \
     } while (0)
 
+// Up to 256 elements one wavefront alone, without a barrier (0.59 / 0.65 / 0.76 us per iteration at 64 / 128 / 256
+// elements; four wavefronts take 0.95 / 0.90 / 0.87); above that four, two or four elements per thread (two wavefronts
+// of four elements at 512: 0.99 us, four of two: 0.95).
 #define TSVM_DISPATCH_E_T(KERNEL, TB, ...)                                                      \
     do {                                                                                        \
-        if (ws_size <= SV_T) TSVM_LAUNCH_SOLVER(KERNEL, 1, TB, __VA_ARGS__);                    \
-        else if (ws_size <= 2 * SV_T) TSVM_LAUNCH_SOLVER(KERNEL, 2, TB, __VA_ARGS__);           \
-        else TSVM_LAUNCH_SOLVER(KERNEL, 4, TB, __VA_ARGS__);                                    \
+        if (ws_size <= 64) TSVM_LAUNCH_SOLVER(KERNEL, TB, 1, 1, SV_LD, __VA_ARGS__);            \
+        else if (ws_size <= 128) TSVM_LAUNCH_SOLVER(KERNEL, TB, 2, 1, SV_LD, __VA_ARGS__);      \
+        else if (ws_size <= SV_LD) TSVM_LAUNCH_SOLVER(KERNEL, TB, 4, 1, SV_LD, __VA_ARGS__);    \
+        else if (ws_size <= 2 * SV_LD) TSVM_LAUNCH_SOLVER(KERNEL, TB, 2, 4, 2 * SV_LD, __VA_ARGS__); \
+        else TSVM_LAUNCH_SOLVER(KERNEL, TB, 4, 4, 4 * SV_LD, __VA_ARGS__);                      \
     } while (0)
 
 // (kws_: the block; block_type_: its element type)
@@ -689,9 +829,12 @@ int tsvm_c_smo_solve_static_init(void) {
     int rc = solver_block_address(&block);
     if (rc) return rc;
     size_t dyn = 0;
-    const void *kernels[] = {reinterpret_cast<const void *>(c_smo_solve_kernel<1, float>), reinterpret_cast<const void *>(c_smo_solve_kernel<2, float>),
-                             reinterpret_cast<const void *>(c_smo_solve_kernel<4, float>), reinterpret_cast<const void *>(c_smo_solve_kernel<1, double>),
-                             reinterpret_cast<const void *>(c_smo_solve_kernel<2, double>), reinterpret_cast<const void *>(c_smo_solve_kernel<4, double>)};
+#define SV_EVERY(TB)                                                                                                         \
+    reinterpret_cast<const void *>(c_smo_solve_kernel<1, 1, SV_LD, TB>), reinterpret_cast<const void *>(c_smo_solve_kernel<2, 1, SV_LD, TB>), \
+        reinterpret_cast<const void *>(c_smo_solve_kernel<4, 1, SV_LD, TB>), reinterpret_cast<const void *>(c_smo_solve_kernel<2, 4, 2 * SV_LD, TB>), \
+        reinterpret_cast<const void *>(c_smo_solve_kernel<4, 4, 4 * SV_LD, TB>)
+    const void *kernels[] = {SV_EVERY(float), SV_EVERY(double)};
+#undef SV_EVERY
     for (const void *k : kernels) {
         rc = solver_dyn_lds(k, &dyn);
         if (rc) return rc;

@@ -398,16 +398,6 @@ __device__ __forceinline__ double wave_max_f64(double v) {
     v = fmax_f64(v, dpp_f64<TSVM_DPP_BCAST31, 0xc>(v));
     return readlane_f64(v, 63);
 }
-__device__ __forceinline__ int wave_min_i32(int v) {
-    v = imin_sel(v, dpp_i32<TSVM_DPP_XOR1>(v));
-    v = imin_sel(v, dpp_i32<TSVM_DPP_XOR2>(v));
-    v = imin_sel(v, dpp_i32<TSVM_DPP_HALF_MIRROR>(v));
-    v = imin_sel(v, dpp_i32<TSVM_DPP_MIRROR>(v));
-    v = imin_sel(v, dpp_i32<TSVM_DPP_BCAST15, 0xa>(v));
-    v = imin_sel(v, dpp_i32<TSVM_DPP_BCAST31, 0xc>(v));
-    return __builtin_amdgcn_readlane(v, 63);
-}
-
 // Maps the launch's linear workgroup id to a logical one so that logical neighbours run on the
 // same XCD (the hardware deals consecutive workgroup ids round-robin over the 8 XCDs, each with
 // its own L2).
