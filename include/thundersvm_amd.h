@@ -279,6 +279,11 @@ int tsvm_nu_smo_solve_block_on_xcd(const int *y, const double *f_val, double *al
                                    int ws_size, double C, const void *kws, int block_type, const double *k_diag, double eps,
                                    double *diff, int max_iter, int *gate, int epoch, int xcd, tsvm_stream stream);
 
+/* No counterpart in the reference: reads a block (laid out as the block solvers take it) on accelerator die `xcd`
+ * (0..7), so that a solver that is then launched onto that die finds its rows in the die's L2.  Blocks that do not fit the L2 (ws_size
+ * above 512 with doubles) are left alone.  sink: one int of device memory, never written in practice. */
+int tsvm_smo_warm_block(const void *kws, int block_type, int ws_size, int xcd, int *sink, tsvm_stream stream);
+
 /* nu_smo_solve (smo_kernel.cpp:127-298), same conventions; diff[1] is left untouched as in the
  * reference's CPU code. */
 int tsvm_nu_smo_solve(const int *y, const double *f_val, double *alpha, double *alpha_diff, const int *working_set,

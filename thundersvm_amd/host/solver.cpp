@@ -687,6 +687,9 @@ struct SolveTask::Impl {
         }
         timer.end(stats.ms_local);
         if (!on_one_stream && !block_on_solver_cus) TSVM_HIP_CHECK(hipEventRecord(block_done, sa));
+        // (beside the solver when it has a stream of its own, in front of it otherwise)
+        if (split && !block_on_solver_cus)
+            abi_check(tsvm_smo_warm_block(d_kws.data(), row_type, ws_size, solver_xcd, d_gate.data() + 3, sa));
     }
 
     void enqueue_solver() {
@@ -700,7 +703,7 @@ struct SolveTask::Impl {
         solver_enqueued = std::chrono::steady_clock::now();
         next_stream_check = solver_enqueued + std::chrono::milliseconds(200);
         if (!on_one_stream && !block_on_solver_cus) TSVM_HIP_CHECK(hipStreamWaitEvent(ss, block_done, 0));
-        if (solver_xcd >= 0 && st == ss) {   // on the masked solver stream: elected onto this lane's XCD
+        if (solver_xcd >= 0) {   // elected onto this lane's XCD, where the block has been read (launches are ordered, whichever stream they are on)
             ++solver_epoch;
             if (nu)
                 abi_check(tsvm_nu_smo_solve_block_on_xcd(d_y.data(), d_f.data(), d_alpha.data(), d_alpha_diff.data(), ws_ids(), ws_size, Cp,
