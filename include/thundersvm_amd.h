@@ -279,6 +279,12 @@ int tsvm_nu_smo_solve_block_on_xcd(const int *y, const double *f_val, double *al
                                    int ws_size, double C, const void *kws, int block_type, const double *k_diag, double eps,
                                    double *diff, int max_iter, int *gate, int epoch, int xcd, tsvm_stream stream);
 
+/* What a solve's device state starts from (CSMOSolver::solve's array constructions, csmosolver.cpp:26-56), in one launch: n_diff
+ * entries of alpha_diff zeroed, the block's columns beyond ws_size zeroed (for ws_size below the block's row stride), slot_of_id[0..n_ids) = -1, two ints of state and
+ * four of gate zeroed (either may be NULL). */
+int tsvm_smo_start(double *alpha_diff, int n_diff, void *kws, int block_type, int ws_size, int *slot_of_id, int n_ids, int *state,
+                   int *gate, tsvm_stream stream);
+
 /* No counterpart in the reference: reads a block (laid out as the block solvers take it) on accelerator die `xcd`
  * (0..7), so that a solver that is then launched onto that die finds its rows in the die's L2.  Blocks that do not fit the L2 (ws_size
  * above 512 with doubles) are left alone.  sink: one int of device memory, never written in practice. */

@@ -60,6 +60,7 @@ SIGNATURES = {
     "tsvm_nu_smo_solve_block": (_int, [_p, _p, _p, _p, _p, _int, _dbl, _p, _int, _p, _dbl, _p, _int, _p]),
     "tsvm_c_smo_solve_block_on_xcd": (_int, [_p, _p, _p, _p, _p, _int, _dbl, _dbl, _p, _int, _p, _dbl, _p, _int, _p, _int, _int, _p]),
     "tsvm_nu_smo_solve_block_on_xcd": (_int, [_p, _p, _p, _p, _p, _int, _dbl, _p, _int, _p, _dbl, _p, _int, _p, _int, _int, _p]),
+    "tsvm_smo_start": (_int, [_p, _int, _p, _int, _int, _p, _int, _p, _p, _p]),
     "tsvm_smo_warm_block": (_int, [_p, _int, _int, _int, _p, _p]),
     "tsvm_select_workspace": (C.c_size_t, [_i64]),
     "tsvm_report_ids": (_int, [_p, _int, _int, _p, _int, _int, _p]),

@@ -31,6 +31,7 @@
 #include "tsvm_device.h"
 #include "tsvm_internal.h"
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -109,6 +110,19 @@ __global__ __launch_bounds__(RA_T) void row_slots_assign_kernel(const int *__res
         info[1] = base + total;
     }
     if (tid < ws) slots_ws[tid] = slot_of_id[ids_ws[tid]];
+}
+
+// What a solve starts from besides its vectors, in one launch: zeroed alpha_diff, the block's columns beyond ws (the
+// solver reads them), no slot for any instance, zeroed counters and gate.
+template <typename TB>
+__global__ void smo_start_kernel(double *alpha_diff, int n_diff, TB *kws, int ws, int ldk, int *slot_of_id, int n_ids, int *state, int *gate) {
+    const int64_t gid = (int64_t) blockIdx.x * blockDim.x + threadIdx.x, stride = (int64_t) gridDim.x * blockDim.x;
+    for (int64_t i = gid; i < n_diff; i += stride) alpha_diff[i] = 0.0;
+    for (int64_t i = gid; i < n_ids; i += stride) slot_of_id[i] = -1;
+    if (ws < ldk)
+        for (int64_t i = gid; i < (int64_t) ws * ldk; i += stride) kws[i] = (TB) 0;
+    if (state && gid < 2) state[gid] = 0;
+    if (gate && gid < 4) gate[gid] = 0;
 }
 
 // What a masked-out element or score is replaced by: larger than any f or score of a problem in range.  Only the
@@ -921,6 +935,23 @@ int tsvm_row_slots_assign(const int *ids_new, int n_new, int *slot_of_id, int *s
                  n_new, ws_size, MAX_WS);
     hipLaunchKernelGGL(row_slots_assign_kernel, dim3(1), dim3(RA_T), 0, tsvm_s(stream), ids_new, n_new, slot_of_id, state, miss_ids,
                        miss_slots, ids_ws, ws_size, slots_ws, info);
+    TSVM_LAUNCH_CHECK();
+    return 0;
+}
+
+int tsvm_smo_start(double *alpha_diff, int n_diff, void *kws, int block_type, int ws_size, int *slot_of_id, int n_ids, int *state,
+                   int *gate, tsvm_stream stream) {
+    TSVM_REQUIRE(alpha_diff && kws && n_diff >= 0 && n_ids >= 0 && (n_ids == 0 || slot_of_id), "tsvm_smo_start: bad arguments");
+    TSVM_REQUIRE(ws_size >= 1 && ws_size <= MAX_WS, "tsvm_smo_start: ws_size %d outside [1, %d]", ws_size, MAX_WS);
+    const int ldk = solver_ldk(ws_size);
+    const int64_t most = std::max<int64_t>(std::max(n_diff, n_ids), ws_size < ldk ? (int64_t) ws_size * ldk : 1);
+    const dim3 grid((unsigned) std::min<int64_t>((most + 255) / 256, 1024));
+    if (block_type == TSVM_ROW_F32)
+        hipLaunchKernelGGL(smo_start_kernel<float>, grid, dim3(256), 0, tsvm_s(stream), alpha_diff, n_diff, (float *) kws, ws_size, ldk, slot_of_id,
+                           n_ids, state, gate);
+    else
+        hipLaunchKernelGGL(smo_start_kernel<double>, grid, dim3(256), 0, tsvm_s(stream), alpha_diff, n_diff, (double *) kws, ws_size, ldk, slot_of_id,
+                           n_ids, state, gate);
     TSVM_LAUNCH_CHECK();
     return 0;
 }

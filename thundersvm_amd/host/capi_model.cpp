@@ -341,7 +341,10 @@ int tsvm_cmdparser_train(int argc, char **argv, tsvm_param *param, int *gamma_se
 }
 
 int tsvm_release_device_cache(void) {
-    TSVM_GUARD({ tsvm::RowArena::instance().release(); })
+    TSVM_GUARD({
+        tsvm::RowArena::instance().release();
+        tsvm::DevicePool::instance().flush();
+    })
 }
 
 int tsvm_model_save(void *model, const char *path) {

@@ -3,6 +3,7 @@
 // an explicit call (the reference's implicit host_data()/device_data() mirroring,
 // src/thundersvm/syncmem.cpp:58-108, is what forces a device-host round trip per solver iteration).
 #pragma once
+#include <functional>
 #include <mutex>
 #include <hip/hip_runtime.h>
 
@@ -28,6 +29,62 @@ inline void abi_check(int rc) {
     if (rc == 2) throw std::bad_alloc();
     throw std::runtime_error(std::string("thundersvm_amd kernel call failed: ") + tsvm_last_error());
 }
+
+// Device blocks that buffers have released, kept for the next buffer of about the same size: hipMalloc and hipFree cost
+// microseconds to milliseconds each (hipFree waits for the device), and a small training run makes some forty of them.
+// Blocks are rounded up to quarter powers of two; blocks above 64 MiB and whatever would take the pool over 512 MiB go
+// back to the driver, everything does when the device runs out of memory, on tsvm_release_device_cache() and when the
+// process ends.  A block is handed out again only after the device has been idle since its release (as hipFree would
+// have waited for), unless whoever released it knows that nothing uses it any more (`idle`).  One list per device; any
+// number of threads.
+class DevicePool {
+public:
+    static DevicePool &instance();
+    void *take(size_t bytes);
+    void give(void *p, size_t bytes, bool idle);
+    void flush();
+
+private:
+    struct Impl;
+    Impl &impl();
+};
+
+// Small page-locked, device-mapped host blocks (PINNED_BLOCK bytes each) and events without timing, kept likewise.
+constexpr size_t PINNED_BLOCK = 32768;
+struct PinnedBlock {
+    char *host = nullptr, *dev = nullptr;
+};
+PinnedBlock take_pinned_block();
+void give_pinned_block(const PinnedBlock &b);
+hipEvent_t take_event();
+void give_event(hipEvent_t e);
+
+// Copies between pageable host memory and the device through a ring of page-locked chunks: the host fills (or empties)
+// one chunk while the others are on their way.  Asynchronous on `stream` as far as the device side goes; when upload()
+// returns the source has been read, when download() returns the destination holds the data.  One ring per process,
+// one user at a time.
+class HostStaging {
+public:
+    static HostStaging &instance();
+    // fill(to, offset, length): writes bytes [offset, offset + length) of what is to be uploaded
+    void upload(void *dst, size_t bytes, const std::function<void(char *, size_t, size_t)> &fill, hipStream_t stream);
+    // what lies at `parts`, one after another
+    struct Part {
+        const void *from;
+        size_t bytes, at;   // at: byte offset in the destination, ascending
+    };
+    void upload(void *dst, const std::vector<Part> &parts, hipStream_t stream);
+    // take(from, offset, length): bytes [offset, offset + length) have arrived
+    void download(const void *src, size_t bytes, const std::function<void(const char *, size_t, size_t)> &take, hipStream_t stream);
+
+    static constexpr size_t CHUNK = (size_t) 4 << 20;
+
+private:
+    struct Impl;
+    Impl &impl();
+};
+// memcpy on as many threads as pay for a block of this size
+void parallel_memcpy(void *to, const void *from, size_t bytes);
 
 size_t &device_bytes_in_use();   // running total of DeviceBuffer allocations (the SyncMem byte counter's role)
 
@@ -74,14 +131,16 @@ public:
         if (count == count_) return;
         release();
         if (count) {
-            TSVM_HIP_CHECK(hipMalloc((void **) &ptr_, count * sizeof(T)));
+            ptr_ = (T *) DevicePool::instance().take(count * sizeof(T));
             device_bytes_in_use() += count * sizeof(T);
         }
         count_ = count;
     }
-    void release() {
+    // idle: nothing enqueued on the device uses the buffer any more (otherwise it is handed out again only after the
+    // device has been idle)
+    void release(bool idle = false) {
         if (ptr_) {
-            (void) hipFree(ptr_);
+            DevicePool::instance().give(ptr_, count_ * sizeof(T), idle);
             device_bytes_in_use() -= count_ * sizeof(T);
         }
         ptr_ = nullptr;

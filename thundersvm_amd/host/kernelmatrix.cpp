@@ -5,10 +5,297 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
+#include <map>
+#include <mutex>
 
 using tsvm::abi_check;
 
 namespace tsvm {
+struct DevicePool::Impl {
+    static constexpr size_t MAX_BLOCK = (size_t) 64 << 20, MAX_TOTAL = (size_t) 512 << 20;
+    std::mutex mu;
+    // [device, block size] -> blocks; `waiting`: released since the device was last known to be idle
+    std::map<std::pair<int, size_t>, std::vector<void *>> ready, waiting;
+    size_t total = 0;
+    // quarter powers of two from 256 bytes on
+    static size_t block_size(size_t bytes) {
+        size_t p = 256;
+        while (p < bytes) p <<= 1;
+        if (p == 256) return p;
+        const size_t q = p / 8;   // between p/2 and p: p/2 + k * p/8
+        return p / 2 + (bytes - p / 2 + q - 1) / q * q;
+    }
+    static int device() {
+        int dev = 0;
+        TSVM_HIP_CHECK(hipGetDevice(&dev));
+        return dev;
+    }
+    void flush_locked() {
+        for (auto *m : {&ready, &waiting}) {
+            for (auto &kv : *m)
+                for (void *p : kv.second) (void) hipFree(p);
+            m->clear();
+        }
+        total = 0;
+    }
+};
+
+DevicePool &DevicePool::instance() {
+    static DevicePool pool;
+    return pool;
+}
+
+DevicePool::Impl &DevicePool::impl() {
+    // (never destroyed; emptied by an atexit handler, which runs before the HIP runtime's tear-down)
+    static Impl *i = [] {
+        Impl *n = new Impl();
+        atexit([] { DevicePool::instance().flush(); });
+        return n;
+    }();
+    return *i;
+}
+
+void *DevicePool::take(size_t bytes) {
+    Impl &I = impl();
+    const int dev = Impl::device();
+    const size_t size = Impl::block_size(bytes);
+    std::lock_guard<std::mutex> lock(I.mu);
+    const auto key = std::make_pair(dev, size);
+    auto it = I.ready.find(key);
+    if (it == I.ready.end() || it->second.empty()) {
+        auto w = I.waiting.find(key);
+        if (w != I.waiting.end() && !w->second.empty()) {
+            TSVM_HIP_CHECK(hipDeviceSynchronize());
+            for (auto k = I.waiting.lower_bound(std::make_pair(dev, (size_t) 0)); k != I.waiting.end() && k->first.first == dev; ++k) {
+                std::vector<void *> &to = I.ready[k->first];
+                to.insert(to.end(), k->second.begin(), k->second.end());
+                k->second.clear();
+            }
+            it = I.ready.find(key);
+        }
+    }
+    if (it != I.ready.end() && !it->second.empty()) {
+        void *p = it->second.back();
+        it->second.pop_back();
+        I.total -= size;
+        return p;
+    }
+    void *p = nullptr;
+    hipError_t e = hipMalloc(&p, size);
+    if (e == hipErrorOutOfMemory && I.total > 0) {
+        (void) hipGetLastError();
+        I.flush_locked();
+        e = hipMalloc(&p, size);
+    }
+    TSVM_HIP_CHECK(e);
+    return p;
+}
+
+void DevicePool::give(void *p, size_t bytes, bool idle) {
+    Impl &I = impl();
+    const size_t size = Impl::block_size(bytes);
+    std::lock_guard<std::mutex> lock(I.mu);
+    int dev = 0;
+    if (size > Impl::MAX_BLOCK || I.total + size > Impl::MAX_TOTAL || hipGetDevice(&dev) != hipSuccess) {
+        (void) hipFree(p);
+        return;
+    }
+    (idle ? I.ready : I.waiting)[std::make_pair(dev, size)].push_back(p);
+    I.total += size;
+}
+
+void DevicePool::flush() {
+    Impl &I = impl();
+    std::lock_guard<std::mutex> lock(I.mu);
+    I.flush_locked();
+}
+
+namespace {
+// (as the pool above: never destroyed, emptied before the HIP runtime's tear-down)
+struct HostPool {
+    std::mutex mu;
+    std::vector<PinnedBlock> pinned;
+    std::map<int, std::vector<hipEvent_t>> events;   // by device
+};
+HostPool &host_pool() {
+    static HostPool *h = [] {
+        HostPool *n = new HostPool();
+        atexit([] {
+            HostPool &p = host_pool();
+            std::lock_guard<std::mutex> lock(p.mu);
+            for (const PinnedBlock &b : p.pinned) (void) hipHostFree(b.host);
+            for (auto &kv : p.events)
+                for (hipEvent_t e : kv.second) (void) hipEventDestroy(e);
+            p.pinned.clear();
+            p.events.clear();
+        });
+        return n;
+    }();
+    return *h;
+}
+constexpr size_t HOST_POOL_MAX = 64;   // blocks, and events per device, kept at most
+}  // namespace
+
+PinnedBlock take_pinned_block() {
+    HostPool &h = host_pool();
+    {
+        std::lock_guard<std::mutex> lock(h.mu);
+        if (!h.pinned.empty()) {
+            const PinnedBlock b = h.pinned.back();
+            h.pinned.pop_back();
+            return b;
+        }
+    }
+    PinnedBlock b;
+    TSVM_HIP_CHECK(hipHostMalloc((void **) &b.host, PINNED_BLOCK, hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable));
+    TSVM_HIP_CHECK(hipHostGetDevicePointer((void **) &b.dev, b.host, 0));
+    return b;
+}
+
+void give_pinned_block(const PinnedBlock &b) {
+    HostPool &h = host_pool();
+    std::lock_guard<std::mutex> lock(h.mu);
+    if (h.pinned.size() < HOST_POOL_MAX) h.pinned.push_back(b);
+    else (void) hipHostFree(b.host);
+}
+
+hipEvent_t take_event() {
+    HostPool &h = host_pool();
+    int dev = 0;
+    TSVM_HIP_CHECK(hipGetDevice(&dev));
+    {
+        std::lock_guard<std::mutex> lock(h.mu);
+        std::vector<hipEvent_t> &v = h.events[dev];
+        if (!v.empty()) {
+            const hipEvent_t e = v.back();
+            v.pop_back();
+            return e;
+        }
+    }
+    hipEvent_t e = nullptr;
+    TSVM_HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    return e;
+}
+
+void give_event(hipEvent_t e) {
+    HostPool &h = host_pool();
+    int dev = 0;
+    if (hipGetDevice(&dev) == hipSuccess) {
+        std::lock_guard<std::mutex> lock(h.mu);
+        std::vector<hipEvent_t> &v = h.events[dev];
+        if (v.size() < HOST_POOL_MAX) {
+            v.push_back(e);
+            return;
+        }
+    }
+    (void) hipEventDestroy(e);
+}
+
+void parallel_memcpy(void *to, const void *from, size_t bytes) {
+    const size_t piece = (size_t) 256 << 10;
+    if (bytes < 4 * piece) {
+        memcpy(to, from, bytes);
+        return;
+    }
+    const long n = (long) ((bytes + piece - 1) / piece);
+#pragma omp parallel for schedule(static)
+    for (long i = 0; i < n; ++i) memcpy((char *) to + i * piece, (const char *) from + i * piece, std::min(piece, bytes - i * piece));
+}
+
+struct HostStaging::Impl {
+    static constexpr int CHUNKS = 4;
+    std::mutex mu;
+    struct Chunk {
+        char *host = nullptr;
+        hipEvent_t event = nullptr;
+        int device = -1;   // the event's device; -1: nothing pending
+    } chunk[CHUNKS];
+    int next = 0;
+    Chunk &take() {
+        Chunk &c = chunk[next];
+        next = (next + 1) % CHUNKS;
+        if (!c.host) TSVM_HIP_CHECK(hipHostMalloc((void **) &c.host, CHUNK, hipHostMallocPortable));
+        wait(c);
+        return c;
+    }
+    void wait(Chunk &c) {
+        if (c.device < 0) return;
+        TSVM_HIP_CHECK(hipEventSynchronize(c.event));
+        give_event(c.event);
+        c.device = -1;
+    }
+    void record(Chunk &c, hipStream_t stream) {
+        c.event = take_event();
+        TSVM_HIP_CHECK(hipEventRecord(c.event, stream));
+        TSVM_HIP_CHECK(hipGetDevice(&c.device));
+    }
+};
+
+HostStaging &HostStaging::instance() {
+    static HostStaging s;
+    return s;
+}
+
+HostStaging::Impl &HostStaging::impl() {
+    static Impl *i = [] {   // (never destroyed; its memory goes back before the HIP runtime's tear-down)
+        Impl *n = new Impl();
+        atexit([] {
+            Impl &I = HostStaging::instance().impl();
+            std::lock_guard<std::mutex> lock(I.mu);
+            for (Impl::Chunk &c : I.chunk) {
+                if (c.host) (void) hipHostFree(c.host);
+                c = Impl::Chunk();
+            }
+        });
+        return n;
+    }();
+    return *i;
+}
+
+void HostStaging::upload(void *dst, size_t bytes, const std::function<void(char *, size_t, size_t)> &fill, hipStream_t stream) {
+    Impl &I = impl();
+    std::lock_guard<std::mutex> lock(I.mu);
+    for (size_t off = 0; off < bytes; off += CHUNK) {
+        const size_t len = std::min(CHUNK, bytes - off);
+        Impl::Chunk &c = I.take();
+        fill(c.host, off, len);
+        TSVM_HIP_CHECK(hipMemcpyAsync((char *) dst + off, c.host, len, hipMemcpyHostToDevice, stream));
+        I.record(c, stream);
+    }
+}
+
+void HostStaging::upload(void *dst, const std::vector<Part> &parts, hipStream_t stream) {
+    if (parts.empty()) return;
+    upload(dst, parts.back().at + parts.back().bytes, [&](char *to, size_t off, size_t len) {
+        for (const Part &p : parts) {
+            const size_t lo = std::max(off, p.at), hi = std::min(off + len, p.at + p.bytes);
+            if (lo < hi) parallel_memcpy(to + (lo - off), (const char *) p.from + (lo - p.at), hi - lo);
+        }
+    }, stream);
+}
+
+void HostStaging::download(const void *src, size_t bytes, const std::function<void(const char *, size_t, size_t)> &take, hipStream_t stream) {
+    Impl &I = impl();
+    std::lock_guard<std::mutex> lock(I.mu);
+    struct Flying { Impl::Chunk *c; size_t off, len; };
+    std::vector<Flying> queue;
+    size_t head = 0, off = 0;
+    while (head < queue.size() || off < bytes) {
+        while (off < bytes && queue.size() - head < Impl::CHUNKS - 1) {
+            const size_t len = std::min(CHUNK, bytes - off);
+            Impl::Chunk &c = I.take();
+            TSVM_HIP_CHECK(hipMemcpyAsync(c.host, (const char *) src + off, len, hipMemcpyDeviceToHost, stream));
+            I.record(c, stream);
+            queue.push_back({&c, off, len});
+            off += len;
+        }
+        const Flying f = queue[head++];
+        I.wait(*f.c);
+        take(f.c->host, f.off, f.len);
+    }
+}
+
 size_t &device_bytes_in_use() {
     static size_t bytes = 0;
     return bytes;
@@ -56,7 +343,13 @@ void *RowArena::acquire(size_t bytes, bool auto_sized) {
         want = take_all ? std::max(bytes, budget) : std::max(bytes * 2, cap_ + cap_ / 2);
     }
     release();
-    TSVM_HIP_CHECK(hipMalloc(&ptr_, want));
+    hipError_t e = hipMalloc(&ptr_, want);
+    if (e == hipErrorOutOfMemory) {   // (what other buffers have left in the pool may be what is missing)
+        (void) hipGetLastError();
+        DevicePool::instance().flush();
+        e = hipMalloc(&ptr_, want);
+    }
+    TSVM_HIP_CHECK(e);
     cap_ = want;
     full_budget_ = take_all;
     static bool registered = false;

@@ -7,6 +7,7 @@
 #include <climits>
 #include <cmath>
 #include <algorithm>
+#include <cstring>
 
 using tsvm::abi_check;
 using tsvm::DeviceBuffer;
@@ -160,8 +161,11 @@ struct SolveTask::Impl {
 
     // d_slots_a holds three tables of ws entries back to back: the slot of every working-set row, then the ids and
     // the slots of the rows to compute; the host fills the same layout in h_slots and sends it with one copy.
-    DeviceBuffer<int> d_y, d_ws, d_slots_a, d_slots_b, d_ws_folded;
-    DeviceBuffer<float_type> d_alpha, d_f, d_alpha_diff;
+    DeviceBuffer<int> d_ws, d_slots_a, d_slots_b, d_ws_folded;
+    DeviceBuffer<char> d_start;                    // alpha, f and y, as they came from the host
+    float_type *d_alpha = nullptr, *d_f = nullptr;
+    int *d_y = nullptr;
+    DeviceBuffer<float_type> d_alpha_diff;
     DeviceBuffer<unsigned char> d_sel_ws;
     DeviceBuffer<kernel_type> d_kws;
     // The working set of iteration t is the window d_ws[ws_off .. ws_off + ws_size): the ids kept from the previous
@@ -213,6 +217,7 @@ struct SolveTask::Impl {
     bool device_cache = false;
     DeviceBuffer<int> d_cache_state;                  // slots in use, rows to compute
     int *h_cache_info = nullptr, *d_cache_info = nullptr;   // the same two numbers in pinned host memory
+    tsvm::PinnedBlock pinned;
     int *h_ids = nullptr, *h_slots = nullptr;
     int *d_ids_host = nullptr;   // h_ids as the device addresses it
     // diff (the solver's 16 bytes for the host, smo_kernel.cpp:87,120) lives in pinned host memory that the device
@@ -334,22 +339,16 @@ struct SolveTask::Impl {
         wall0 = std::chrono::steady_clock::now();
         (void) process_epoch();
         stats.ws_size = ws_size;
-        d_y.resize(n); d_ws.resize((size_t) WS_HALVES * q + ws_size); d_slots_a.resize(3 * (size_t) ws_size); d_slots_b.resize(ws_size);
+        d_ws.resize((size_t) WS_HALVES * q + ws_size); d_slots_a.resize(3 * (size_t) ws_size); d_slots_b.resize(ws_size);
         if (rep > 1) d_ws_folded.resize(d_ws.size());
-        d_alpha.resize(n); d_f.resize(n); d_alpha_diff.resize(ws_size);
+        d_alpha_diff.resize(ws_size);
         d_sel_ws.resize(tsvm_select_workspace(n));
         d_kws.resize((size_t) ws_size * ldk);
-        d_y.upload(y.data(), n);
-        d_alpha.upload(alpha.data(), n);
-        d_f.upload(f_val.data(), n);
-        d_alpha_diff.zero();
-        d_kws.zero();
         alone = n_lanes == 1;
         split = !solver.profile && create_split_streams(lane, n_lanes);
         if (split) {
             solver_xcd = lane;
             d_gate.resize(4);
-            d_gate.zero();
         }
         if (!split) {
             TSVM_HIP_CHECK(hipStreamCreateWithFlags(&sa, hipStreamNonBlocking));
@@ -358,10 +357,10 @@ struct SolveTask::Impl {
         // The read-back of the newly selected ids follows the selection on the same stream: it is enqueued before
         // anything else of the iteration, so it waits for nothing but the selection.
         ids = sa;
-        TSVM_HIP_CHECK(hipEventCreateWithFlags(&selected, hipEventDisableTiming));
-        TSVM_HIP_CHECK(hipEventCreateWithFlags(&diff_ready, hipEventDisableTiming));
-        TSVM_HIP_CHECK(hipEventCreateWithFlags(&block_done, hipEventDisableTiming));
-        TSVM_HIP_CHECK(hipEventCreateWithFlags(&solved, hipEventDisableTiming));
+        selected = tsvm::take_event();
+        diff_ready = tsvm::take_event();
+        block_done = tsvm::take_event();
+        solved = tsvm::take_event();
 
         // Kernel rows live in slots of one pool.  With a cache the pool holds up to pool_rows rows and the
         // host tracks which instance sits in which slot; without one it holds exactly ws rows.
@@ -391,27 +390,40 @@ struct SolveTask::Impl {
             device_cache = d_slot_of.size() == (size_t) n_u && rep == 1 && k_mat.dense_layout();
         }
         if (device_cache) {
-            TSVM_HIP_CHECK(hipMemset(d_slot_of.data(), 0xff, sizeof(int) * (size_t) n_u));
             d_cache_state.resize(2);
-            d_cache_state.zero();
-            TSVM_HIP_CHECK(hipHostMalloc((void **) &h_cache_info, 2 * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
-            TSVM_HIP_CHECK(hipHostGetDevicePointer((void **) &d_cache_info, h_cache_info, 0));
-            h_cache_info[0] = h_cache_info[1] = 0;
         }
         cur_slots.resize(ws_size);
         cur_ids.resize(ws_size);
-        TSVM_HIP_CHECK(hipHostMalloc((void **) &h_diff, 2 * sizeof(double), hipHostMallocMapped | hipHostMallocCoherent));
-        TSVM_HIP_CHECK(hipHostGetDevicePointer((void **) &d_diff, h_diff, 0));
-        TSVM_HIP_CHECK(hipHostMalloc((void **) &h_ids, (ws_size + 16) * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
-        TSVM_HIP_CHECK(hipHostGetDevicePointer((void **) &d_ids_host, h_ids, 0));
+        // one page-locked block: diff, the cache's two numbers, the reported ids, the slot tables
+        pinned = tsvm::take_pinned_block();
+        static_assert(64 + (1024 + 16) * sizeof(int) + 3 * 1024 * sizeof(int) <= tsvm::PINNED_BLOCK, "pinned block");
+        h_diff = (double *) pinned.host;
+        d_diff = (double *) pinned.dev;
+        h_cache_info = (int *) (pinned.host + 32);
+        d_cache_info = (int *) (pinned.dev + 32);
+        h_ids = (int *) (pinned.host + 64);
+        d_ids_host = (int *) (pinned.dev + 64);
+        h_slots = h_ids + ws_size + 16;
+        h_cache_info[0] = h_cache_info[1] = 0;
         h_ids[ws_size] = 0;
-        TSVM_HIP_CHECK(hipHostMalloc((void **) &h_slots, 3 * ws_size * sizeof(int)));
         h_diff[0] = h_diff[1] = 0;
+        // what the device starts from: the three vectors in one copy, the rest by one kernel
+        const size_t f_at = ((size_t) n * sizeof(float_type) + 255) / 256 * 256;
+        d_start.resize(2 * f_at + (size_t) n * sizeof(int));
+        tsvm::HostStaging::instance().upload(d_start.data(), {{alpha.data(), (size_t) n * sizeof(float_type), 0},
+                                                              {f_val.data(), (size_t) n * sizeof(float_type), f_at},
+                                                              {y.data(), (size_t) n * sizeof(int), 2 * f_at}}, nullptr);
+        d_alpha = (float_type *) d_start.data();
+        d_f = (float_type *) (d_start.data() + f_at);
+        d_y = (int *) (d_start.data() + 2 * f_at);
+        abi_check(tsvm_smo_start(d_alpha_diff.data(), ws_size, d_kws.data(), row_type, ws_size, device_cache ? d_slot_of.data() : nullptr,
+                                 device_cache ? n_u : 0, device_cache ? d_cache_state.data() : nullptr, split ? d_gate.data() : nullptr,
+                                 nullptr));
         if (!caching) {
             for (int t = 0; t < ws_size; ++t) cur_slots[t] = t;
             upload_rotation(cur_slots);
         }
-        solver.init_f(alpha, y, k_mat, d_f.data());
+        solver.init_f(alpha, y, k_mat, d_f);
         TSVM_HIP_CHECK(hipDeviceSynchronize());   // uploads, fills and init_f ran on the default stream
 
         max_iter = std::max(100000, ws_size > INT_MAX / 100 ? INT_MAX : 100 * ws_size);
@@ -441,24 +453,24 @@ struct SolveTask::Impl {
 
     ~Impl() {
         if (abandoned) {   // nothing that could wait for the device
-            for (DeviceBuffer<int> *b : {&d_y, &d_ws, &d_slots_a, &d_slots_b, &d_ws_folded, &d_gate, &d_slot_of, &d_cache_state}) b->abandon();
-            for (DeviceBuffer<float_type> *b : {&d_alpha, &d_f, &d_alpha_diff, &d_kws}) b->abandon();
+            for (DeviceBuffer<int> *b : {&d_ws, &d_slots_a, &d_slots_b, &d_ws_folded, &d_gate, &d_slot_of, &d_cache_state}) b->abandon();
+            for (DeviceBuffer<float_type> *b : {&d_alpha_diff, &d_kws}) b->abandon();
+            d_start.abandon();
             d_sel_ws.abandon();
             return;
         }
         if (sa) (void) hipStreamSynchronize(sa);   // a selection enqueued ahead may still be running
         if (ss && ss != sa) (void) hipStreamSynchronize(ss);
-        if (ids && ids != sa) { (void) hipStreamSynchronize(ids); (void) hipStreamDestroy(ids); }
         if (split) release_split_streams();         // masked streams go back to the pool
         else if (sa) (void) hipStreamDestroy(sa);
-        if (block_done) (void) hipEventDestroy(block_done);
-        if (solved) (void) hipEventDestroy(solved);
-        if (selected) (void) hipEventDestroy(selected);
-        if (diff_ready) (void) hipEventDestroy(diff_ready);
-        if (h_diff) (void) hipHostFree(h_diff);
-        if (h_cache_info) (void) hipHostFree(h_cache_info);
-        if (h_ids) (void) hipHostFree(h_ids);
-        if (h_slots) (void) hipHostFree(h_slots);
+        // (both streams are empty: nothing uses the buffers any more)
+        for (DeviceBuffer<int> *b : {&d_ws, &d_slots_a, &d_slots_b, &d_ws_folded, &d_gate, &d_slot_of, &d_cache_state}) b->release(true);
+        for (DeviceBuffer<float_type> *b : {&d_alpha_diff, &d_kws}) b->release(true);
+        d_start.release(true);
+        d_sel_ws.release(true);
+        for (hipEvent_t e : {block_done, solved, selected, diff_ready})
+            if (e) tsvm::give_event(e);
+        if (pinned.host) tsvm::give_pinned_block(pinned);
     }
 
     // Two streams with disjoint CU masks from the pool (make_lane_group above).  Anything unexpected (another CU
@@ -531,14 +543,14 @@ struct SolveTask::Impl {
         const int *kept = it == 0 ? nullptr : d_ws.data() + sel_off;            // the half that stays: no candidates
         int *out = d_ws.data() + sel_off + (it == 0 ? 0 : q);
         if (rep > 1) {
-            abi_check(tsvm_select_working_set_folded(d_f.data(), d_y.data(), d_alpha.data(), n, Cp, Cn, kept, it == 0 ? 0 : q, out,
+            abi_check(tsvm_select_working_set_folded(d_f, d_y, d_alpha, n, Cp, Cn, kept, it == 0 ? 0 : q, out,
                                                      n_sel, nu, d_sel_ws.data(), it > 0, n_u,
                                                      d_ws_folded.data() + sel_off + (it == 0 ? 0 : q), sel));
         } else if (it == 0) {
-            abi_check(tsvm_select_working_set(d_f.data(), d_y.data(), d_alpha.data(), n, Cp, Cn, kept, 0, out, n_sel, nu,
+            abi_check(tsvm_select_working_set(d_f, d_y, d_alpha, n, Cp, Cn, kept, 0, out, n_sel, nu,
                                               d_sel_ws.data(), sel));
         } else {
-            abi_check(tsvm_select_working_set_again(d_f.data(), d_y.data(), d_alpha.data(), n, Cp, Cn, kept, q, out, n_sel, nu,
+            abi_check(tsvm_select_working_set_again(d_f, d_y, d_alpha, n, Cp, Cn, kept, q, out, n_sel, nu,
                                                     d_sel_ws.data(), sel));
         }
     }
@@ -706,18 +718,18 @@ struct SolveTask::Impl {
         if (solver_xcd >= 0) {   // elected onto this lane's XCD, where the block has been read (launches are ordered, whichever stream they are on)
             ++solver_epoch;
             if (nu)
-                abi_check(tsvm_nu_smo_solve_block_on_xcd(d_y.data(), d_f.data(), d_alpha.data(), d_alpha_diff.data(), ws_ids(), ws_size, Cp,
+                abi_check(tsvm_nu_smo_solve_block_on_xcd(d_y, d_f, d_alpha, d_alpha_diff.data(), ws_ids(), ws_size, Cp,
                                                          d_kws.data(), row_type, k_mat.diag(), eps, d_diff, max_iter, d_gate.data(),
                                                          solver_epoch, solver_xcd, st));
             else
-                abi_check(tsvm_c_smo_solve_block_on_xcd(d_y.data(), d_f.data(), d_alpha.data(), d_alpha_diff.data(), ws_ids(), ws_size, Cp,
+                abi_check(tsvm_c_smo_solve_block_on_xcd(d_y, d_f, d_alpha, d_alpha_diff.data(), ws_ids(), ws_size, Cp,
                                                         Cn, d_kws.data(), row_type, k_mat.diag(), eps, d_diff, max_iter, d_gate.data(),
                                                         solver_epoch, solver_xcd, st));
         } else if (nu) {
-            abi_check(tsvm_nu_smo_solve_block(d_y.data(), d_f.data(), d_alpha.data(), d_alpha_diff.data(), ws_ids(), ws_size,
+            abi_check(tsvm_nu_smo_solve_block(d_y, d_f, d_alpha, d_alpha_diff.data(), ws_ids(), ws_size,
                                               Cp, d_kws.data(), row_type, k_mat.diag(), eps, d_diff, max_iter, st));
         } else {
-            abi_check(tsvm_c_smo_solve_block(d_y.data(), d_f.data(), d_alpha.data(), d_alpha_diff.data(), ws_ids(), ws_size,
+            abi_check(tsvm_c_smo_solve_block(d_y, d_f, d_alpha, d_alpha_diff.data(), ws_ids(), ws_size,
                                              Cp, Cn, d_kws.data(), row_type, k_mat.diag(), eps, d_diff, max_iter, st));
         }
         timer.end(stats.ms_local);
@@ -729,14 +741,14 @@ struct SolveTask::Impl {
         if (select_ahead && fuse_select) {
             // the next selection's first pass over the instances rides on update_f's last one
             advance_window();
-            abi_check(tsvm_update_f_select(d_f.data(), d_alpha_diff.data(), ws_size, k_rows, row_type, slots, ld, n_u, rep,
-                                           d_y.data(), d_alpha.data(), Cp, Cn, d_ws.data() + sel_off, q, d_ws.data() + sel_off + q, q,
+            abi_check(tsvm_update_f_select(d_f, d_alpha_diff.data(), ws_size, k_rows, row_type, slots, ld, n_u, rep,
+                                           d_y, d_alpha, Cp, Cn, d_ws.data() + sel_off, q, d_ws.data() + sel_off + q, q,
                                            nu, d_sel_ws.data(), rep > 1 ? d_ws_folded.data() + sel_off + q : nullptr, sa));
             select_enqueued = true;
             return;
         }
         timer.begin();
-        abi_check(tsvm_update_f(d_f.data(), d_alpha_diff.data(), ws_size, k_rows, row_type, slots, ld, n_u, rep, sa));
+        abi_check(tsvm_update_f(d_f, d_alpha_diff.data(), ws_size, k_rows, row_type, slots, ld, n_u, rep, sa));
         timer.end(stats.ms_update_f);
         if (timer.on) {   // (profiling runs every step to completion anyway) how many rows did update_f have to read?
             std::vector<float_type> ad = d_alpha_diff.to_host();
@@ -788,8 +800,14 @@ struct SolveTask::Impl {
                 stats.cache_hits = stats.cache_lookups - h_cache_info[1];
                 stats.rows_computed = h_cache_info[1];
             }
-            d_alpha.download(alpha.data(), n);
-            d_f.download(f_val.data(), n);
+            const size_t vec = (size_t) n * sizeof(float_type), f_at = (size_t) ((char *) d_f - d_start.data());
+            tsvm::HostStaging::instance().download(d_start.data(), f_at + vec, [&](const char *from, size_t off, size_t len) {
+                if (off < vec) tsvm::parallel_memcpy((char *) alpha.data() + off, from, std::min(len, vec - off));
+                if (off + len > f_at) {
+                    const size_t lo = std::max(off, f_at);
+                    tsvm::parallel_memcpy((char *) f_val.data() + (lo - f_at), from + (lo - off), off + len - lo);
+                }
+            }, sa);
             rho = solver.calculate_rho(f_val, y, alpha, Cp, Cn);
             stats.n_iter = iter + 1;
             stats.local_iter = local_iter;
