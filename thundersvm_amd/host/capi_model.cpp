@@ -2,6 +2,7 @@
 #include <chrono>
 #include "../../include/thundersvm_amd_model.h"
 
+#include <algorithm>
 #include <cstring>
 #include <exception>
 #include <stdexcept>
@@ -92,7 +93,7 @@ int tsvm_model_train_csr(void *model, int64_t n, const int64_t *row_ptr, const i
     TSVM_GUARD({
         Handle *h = (Handle *) model;
         DataSet ds;
-        ds.load_from_csr(n, row_ptr, col, val, y);
+        ds.load_from_csr(n, row_ptr, col, val, y, false);   // (the caller's arrays outlive this call)
         configure(h, param, ws_override, keep_binary, trace_cap, profile);
         h->model->train(ds, to_param(*param));
     })
@@ -136,24 +137,18 @@ int64_t tsvm_dataset_info(void *dataset, int64_t *n_features, int *zero_based, i
     if (n_features) *n_features = (int64_t) ds.n_features();
     if (zero_based) *zero_based = ds.is_zero_based();
     if (has_labels) *has_labels = ds.y().size() == ds.n_instances();
-    int64_t nnz = 0;
-    for (const auto &row : ds.instances()) nnz += (int64_t) row.size();
-    return nnz;
+    return (int64_t) ds.rows().nnz();
 }
 
 void tsvm_dataset_get_csr(void *dataset, int64_t *row_ptr, int *col, double *val, double *y) {
     const DataSet &ds = *(DataSet *) dataset;
-    int64_t e = 0;
-    for (size_t r = 0; r < ds.n_instances(); ++r) {
-        if (row_ptr) row_ptr[r] = e;
-        for (const auto &nd : ds.instances()[r]) {
-            if (col) col[e] = nd.index;
-            if (val) val[e] = nd.value;
-            ++e;
-        }
-        if (y && r < ds.y().size()) y[r] = ds.y()[r];
-    }
-    if (row_ptr) row_ptr[ds.n_instances()] = e;
+    const RowStore &R = ds.rows();
+    const size_t nnz = R.nnz();
+    if (row_ptr)
+        for (size_t r = 0; r <= R.size(); ++r) row_ptr[r] = R.ptr()[r] - R.ptr()[0];
+    if (col) memcpy(col, R.col() + R.ptr()[0], nnz * sizeof(int));
+    if (val) memcpy(val, R.val() + R.ptr()[0], nnz * sizeof(double));
+    if (y) memcpy(y, ds.y().data(), std::min(ds.y().size(), R.size()) * sizeof(double));
 }
 
 int tsvm_rule_choose_dense(int64_t n, int64_t n_features, int64_t nnz) {
@@ -222,12 +217,8 @@ int tsvm_model_info(void *model, int *n_classes, int *n_binary_models, int *tota
         SvmModel &m = *((Handle *) model)->model;
         if (n_classes) *n_classes = m.get_n_classes();
         if (n_binary_models) *n_binary_models = m.get_n_binary_models();
-        if (total_sv) *total_sv = (int) m.svs().size();
-        if (sv_nnz) {
-            int64_t t = 0;
-            for (const auto &r : m.svs()) t += (int64_t) r.size();
-            *sv_nnz = t;
-        }
+        if (total_sv) *total_sv = (int) m.sv_rows().size();
+        if (sv_nnz) *sv_nnz = (int64_t) m.sv_rows().nnz();
     })
 }
 
@@ -240,16 +231,11 @@ int tsvm_model_get(void *model, int *label, int *n_sv, double *rho, double *coef
         if (rho) memcpy(rho, m.get_rho().data(), sizeof(double) * m.get_rho().size());
         if (coef && !m.get_coef().empty()) memcpy(coef, m.get_coef().data(), sizeof(double) * m.get_coef().size());
         if (sv_indices && !m.get_sv_ind().empty()) memcpy(sv_indices, m.get_sv_ind().data(), sizeof(int) * m.get_sv_ind().size());
-        int64_t e = 0;
-        if (sv_ptr) sv_ptr[0] = 0;
-        for (size_t r = 0; (sv_ptr || sv_col || sv_val) && r < m.svs().size(); ++r) {
-            for (const auto &nd : m.svs()[r]) {
-                if (sv_col) sv_col[e] = nd.index;
-                if (sv_val) sv_val[e] = nd.value;
-                ++e;
-            }
-            if (sv_ptr) sv_ptr[r + 1] = e;
-        }
+        const RowStore &R = m.sv_rows();
+        if (sv_ptr)
+            for (size_t r = 0; r <= R.size(); ++r) sv_ptr[r] = R.ptr()[r] - R.ptr()[0];
+        if (sv_col) memcpy(sv_col, R.col() + R.ptr()[0], R.nnz() * sizeof(int));
+        if (sv_val) memcpy(sv_val, R.val() + R.ptr()[0], R.nnz() * sizeof(double));
     })
 }
 
@@ -307,8 +293,8 @@ int tsvm_model_predict_csr(void *model, int64_t nrows, const int64_t *row_ptr, c
     TSVM_GUARD({
         SvmModel &m = *((Handle *) model)->model;
         DataSet ds;
-        ds.load_from_csr(nrows, row_ptr, col, val, nullptr);
-        std::vector<float_type> out = m.predict(ds.instances(), batch_size);
+        ds.load_from_csr(nrows, row_ptr, col, val, nullptr, false);
+        std::vector<float_type> out = m.predict(ds, batch_size);
         if (labels) memcpy(labels, out.data(), sizeof(double) * (size_t) nrows);
         if (dec_values) memcpy(dec_values, m.get_dec_value().data(), sizeof(double) * m.get_dec_value().size());
     })

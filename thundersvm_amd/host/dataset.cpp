@@ -17,7 +17,19 @@
 #include <stdexcept>
 
 DataSet::DataSet(const node2d &instances, int n_features, const std::vector<float_type> &y)
-    : y_(y), instances_(instances), n_features_(n_features) {}
+    : y_(y), rows_(RowStore::from_nodes(instances)), n_features_(n_features) {}
+
+DataSet::DataSet(std::shared_ptr<const RowStore> rows, int n_features, const std::vector<float_type> &y)
+    : y_(y), rows_(std::move(rows)), n_features_(n_features) {}
+
+void DataSet::set_rows(std::shared_ptr<const RowStore> rows) {
+    device_slot_ = std::make_shared<std::shared_ptr<void>>();   // new instances: any device copy is stale
+    rows_ = std::move(rows);
+    start_.clear();
+    count_.clear();
+    label_.clear();
+    perm_.clear();
+}
 
 // ------------------------------------------------------------------------------------------------
 // LibSVM text loader.  The reference reads 16 MB at a time and lets every OpenMP thread parse a run of whole lines
@@ -36,14 +48,16 @@ using tsvm::parse_float;
 
 struct LoadedRun {
     std::vector<float_type> y;
-    DataSet::node2d rows;
+    std::vector<int> len, col;       // entries per row, then the entries
+    std::vector<float> val;
     size_t max_index = 0;
     bool zero_based = false;
     bool bad = false;
 };
 
 void parse_run(const char *p, const char *end, LoadedRun &out) {
-    std::vector<DataSet::node> row;   // assembled here, copied out at its final size: one allocation per instance
+    out.col.reserve((size_t) (end - p) / 8);
+    out.val.reserve((size_t) (end - p) / 8);
     while (p < end) {
         const char *eol = (const char *) memchr(p, '\n', end - p);
         if (!eol) eol = end;
@@ -53,7 +67,7 @@ void parse_run(const char *p, const char *end, LoadedRun &out) {
             out.y.push_back(parse_double(p, eol, &q));
             if (q == p) { out.bad = true; return; }
             p = q;
-            row.clear();
+            const size_t first = out.col.size();
             while (p < eol) {
                 while (p < eol && is_blank(*p)) ++p;
                 if (p >= eol) break;
@@ -70,11 +84,12 @@ void parse_run(const char *p, const char *end, LoadedRun &out) {
                 const float v = parse_float(p, eol, &q);
                 if (q == p) { out.bad = true; return; }
                 p = q;
-                row.emplace_back((int) idx, (kernel_type) v);
+                out.col.push_back((int) idx);
+                out.val.push_back(v);
                 if (idx == 0) out.zero_based = true;
                 if (idx > 0 && (size_t) idx > out.max_index) out.max_index = (size_t) idx;
             }
-            out.rows.emplace_back(row.begin(), row.end());
+            out.len.push_back((int) (out.col.size() - first));
         }
         p = eol + 1;
     }
@@ -83,9 +98,8 @@ void parse_run(const char *p, const char *end, LoadedRun &out) {
 }  // namespace
 
 void DataSet::load_from_file(std::string file_name, int n_threads) {
-    device_slot_ = std::make_shared<std::shared_ptr<void>>();   // new instances: any device copy is stale
     y_.clear();
-    instances_.clear();
+    set_rows(std::make_shared<RowStore>(0, 0));
     n_features_ = 0;
     zero_based_ = false;
     const int fd = open(file_name.c_str(), O_RDONLY);
@@ -156,87 +170,101 @@ void DataSet::load_from_file(std::string file_name, int n_threads) {
         if (r < n_body_runs) parse_run(text + cut[r], text + cut[r + 1], runs[r]);
         else parse_run(tail.c_str(), tail.c_str() + tail.size(), runs[r]);
     }
-    std::vector<size_t> first(n_runs + 1, 0);
+    std::vector<size_t> first(n_runs + 1, 0), first_entry(n_runs + 1, 0);
     for (int r = 0; r < n_runs; ++r) {
         if (runs[r].bad) throw std::runtime_error("read error, using [index]:[value] format");
-        first[r + 1] = first[r] + runs[r].rows.size();
+        first[r + 1] = first[r] + runs[r].len.size();
+        first_entry[r + 1] = first_entry[r] + runs[r].col.size();
         if (runs[r].max_index > n_features_) n_features_ = runs[r].max_index;
         zero_based_ = zero_based_ || runs[r].zero_based;
     }
     y_.resize(first[n_runs]);
-    instances_.resize(first[n_runs]);
+    auto rows = std::make_shared<RowStore>(first[n_runs], first_entry[n_runs]);
 #pragma omp parallel for num_threads(n_threads) schedule(dynamic, 1)
     for (int r = 0; r < n_runs; ++r) {
         LoadedRun &run = runs[r];
         std::copy(run.y.begin(), run.y.end(), y_.begin() + first[r]);
-        std::move(run.rows.begin(), run.rows.end(), instances_.begin() + first[r]);
+        int64_t e = (int64_t) first_entry[r];
+        for (size_t i = 0; i < run.len.size(); ++i) rows->ptr_mut()[first[r] + i + 1] = e += run.len[i];
+        std::copy(run.col.begin(), run.col.end(), rows->col_mut() + first_entry[r]);
+        std::copy(run.val.begin(), run.val.end(), rows->val_mut() + first_entry[r]);
         run = LoadedRun();      // the run's own arrays are released by the thread that moved it
     }
+    set_rows(rows);
     TSVM_LOG << "#instances = " << n_instances() << ", #features = " << n_features();
 }
 
 void DataSet::load_from_python(float *y, char **x, int len) {
-    device_slot_ = std::make_shared<std::shared_ptr<void>>();   // new instances: any device copy is stale
     y_.clear();
-    instances_.clear();
+    node2d nodes;
     n_features_ = 0;
     for (int i = 0; i < len; ++i) {
         y_.push_back(y[i]);
-        instances_.emplace_back();
+        nodes.emplace_back();
         std::stringstream ss(x[i]);
         std::string tuple;
         while (ss >> tuple) {
             int ind;
             float v;
             if (sscanf(tuple.c_str(), "%d:%f", &ind, &v) != 2) throw std::runtime_error("read error, using [index]:[value] format");
-            instances_.back().emplace_back(ind, v);
+            nodes.back().emplace_back(ind, v);
             if ((size_t) ind > n_features_) n_features_ = ind;
         }
     }
+    set_rows(RowStore::from_nodes(nodes));
 }
 
 void DataSet::load_from_sparse(int row_size, float *val, int *row_ptr, int *col_ptr, float *label) {
-    device_slot_ = std::make_shared<std::shared_ptr<void>>();   // new instances: any device copy is stale
-    y_.clear();
-    instances_.assign(row_size, {});
+    y_.assign(label, label + (label ? row_size : 0));
     n_features_ = 0;
+    const size_t nnz = (size_t) std::max(row_ptr[row_size] - row_ptr[0], 0);
+    auto rows = std::make_shared<RowStore>((size_t) row_size, nnz);
+    int max_index = 0;
+#pragma omp parallel for schedule(static) reduction(max : max_index) num_threads(threads_for(nnz))
     for (int r = 0; r < row_size; ++r) {
-        if (label) y_.push_back(label[r]);
+        rows->ptr_mut()[r + 1] = row_ptr[r + 1] - row_ptr[0];
         for (int e = row_ptr[r]; e < row_ptr[r + 1]; ++e) {
-            int ind = col_ptr[e] + 1;  // to one-based
-            instances_[r].emplace_back(ind, val[e]);
-            if ((size_t) ind > n_features_) n_features_ = ind;
+            const int ind = col_ptr[e] + 1;  // to one-based
+            rows->col_mut()[e - row_ptr[0]] = ind;
+            rows->val_mut()[e - row_ptr[0]] = val[e];
+            max_index = std::max(max_index, ind);
         }
     }
+    n_features_ = (size_t) max_index;
+    set_rows(rows);
 }
 
 void DataSet::load_from_dense(int row_size, int features, float *data, float *label) {
-    device_slot_ = std::make_shared<std::shared_ptr<void>>();   // new instances: any device copy is stale
-    y_.clear();
-    instances_.assign(row_size, {});
+    y_.assign(label, label + (label ? row_size : 0));
+    const size_t nnz = (size_t) row_size * features;
+    auto rows = std::make_shared<RowStore>((size_t) row_size, nnz);
+#pragma omp parallel for schedule(static) num_threads(threads_for(nnz))
     for (int r = 0; r < row_size; ++r) {
-        if (label) y_.push_back(label[r]);
-        instances_[r].reserve(features);
-        for (int j = 1; j <= features; ++j) instances_[r].emplace_back(j, data[(size_t) r * features + j - 1]);
-    }
-    n_features_ = features;
-}
-
-void DataSet::load_from_csr(int64_t n, const int64_t *row_ptr, const int *col, const double *val, const double *y) {
-    device_slot_ = std::make_shared<std::shared_ptr<void>>();   // new instances: any device copy is stale
-    y_.clear();
-    instances_.assign(n, {});
-    n_features_ = 0;
-    zero_based_ = false;
-    for (int64_t r = 0; r < n; ++r) {
-        if (y) y_.push_back(y[r]);
-        instances_[r].reserve(row_ptr[r + 1] - row_ptr[r]);
-        for (int64_t e = row_ptr[r]; e < row_ptr[r + 1]; ++e) {
-            instances_[r].emplace_back(col[e], val[e]);
-            if (col[e] == 0) zero_based_ = true;
-            if ((size_t) col[e] > n_features_) n_features_ = col[e];
+        const size_t e = (size_t) r * features;
+        rows->ptr_mut()[r + 1] = (int64_t) (e + features);
+        for (int j = 0; j < features; ++j) {
+            rows->col_mut()[e + j] = j + 1;
+            rows->val_mut()[e + j] = data[e + j];
         }
     }
+    n_features_ = features;
+    set_rows(rows);
+}
+
+void DataSet::load_from_csr(int64_t n, const int64_t *row_ptr, const int *col, const double *val, const double *y, bool keep) {
+    y_.assign(y, y + (y ? n : 0));
+    std::shared_ptr<const RowStore> rows = keep ? RowStore::copy_of((size_t) n, row_ptr, col, val)
+                                                : std::make_shared<RowStore>((size_t) n, row_ptr, col, val);
+    int max_index = 0, zero = 0;
+    const int64_t lo = row_ptr[0], hi = row_ptr[n];
+#pragma omp parallel for schedule(static) reduction(max : max_index, zero) num_threads(threads_for((size_t) (hi - lo)))
+    for (int64_t e = lo; e < hi; ++e) {
+        max_index = std::max(max_index, col[e]);
+        zero |= col[e] == 0;
+    }
+    n_features_ = (size_t) max_index;
+    zero_based_ = zero != 0;
+    set_rows(std::move(rows));
 }
 
 // Classes are numbered in order of first appearance; perm_ lists the instance ids class by class
@@ -246,7 +274,7 @@ void DataSet::group_classes(bool classification) {
     count_.clear();
     label_.clear();
     perm_.clear();
-    const size_t n = instances().size();
+    const size_t n = n_instances();
     if (!classification) {
         perm_.resize(n);
         for (size_t i = 0; i < n; ++i) perm_[i] = (int) i;
@@ -277,7 +305,7 @@ DataSet DataSet::grouped_view() const {
     v.y_ = y_;
     v.n_features_ = n_features_;
     v.zero_based_ = zero_based_;
-    v.base_ = base_ ? base_ : &instances_;
+    v.rows_ = rows_;
     v.device_slot_ = device_slot_;   // same instances, same device copy
     v.group_classes(true);
     return v;

@@ -4,19 +4,17 @@
 #pragma once
 #include <memory>
 
+#include "rows.h"
 #include "thundersvm.h"
 
 class DataSet {
 public:
-    struct node {
-        node(int index, kernel_type value) : index(index), value(value) {}
-        int index;
-        kernel_type value;
-    };
-    typedef std::vector<std::vector<node>> node2d;
+    typedef RowNode node;
+    typedef RowStore::node2d node2d;
 
     DataSet() = default;
     DataSet(const node2d &instances, int n_features, const std::vector<float_type> &y);
+    DataSet(std::shared_ptr<const RowStore> rows, int n_features, const std::vector<float_type> &y);
 
     // n_threads: threads that read and parse (0: as many as OpenMP would start, which the `-o` option sets, as in
     // the reference)
@@ -24,20 +22,22 @@ public:
     void load_from_python(float *y, char **x, int len);
     void load_from_sparse(int row_size, float *val, int *row_ptr, int *col_ptr, float *label);
     void load_from_dense(int row_size, int features, float *data, float *label);
-    // CSR with the caller's (1-based) feature ids and double values (already float32-exact)
-    void load_from_csr(int64_t n, const int64_t *row_ptr, const int *col, const double *val, const double *y);
+    // CSR with the caller's (1-based) feature ids and double values (already float32-exact).  keep: whether the DataSet
+    // is to own its rows; otherwise it refers to the caller's arrays, which have to outlive it.
+    void load_from_csr(int64_t n, const int64_t *row_ptr, const int *col, const double *val, const double *y, bool keep = true);
 
     void group_classes(bool classification = true);
     // A grouped DataSet that refers to this one's instances instead of copying them.
     DataSet grouped_view() const;
-    size_t n_instances() const { return instances().size(); }
+    size_t n_instances() const { return rows_->size(); }
     size_t n_features() const { return n_features_; }
     size_t n_classes() const { return start_.size(); }
     const std::vector<int> &count() const { return count_; }
     const std::vector<int> &start() const { return start_; }
     const std::vector<int> &label() const { return label_; }
     const std::vector<float_type> &y() const { return y_; }
-    const node2d &instances() const { return base_ ? *base_ : instances_; }
+    const RowStore &rows() const { return *rows_; }
+    const node2d &instances() const { return rows_->nodes(); }
     const node2d instances(int y_i) const;
     const node2d instances(int y_i, int y_j) const;
     const std::vector<int> original_index() const { return perm_; }
@@ -51,8 +51,8 @@ public:
 
 private:
     std::vector<float_type> y_;
-    node2d instances_;
-    const node2d *base_ = nullptr;   // set by grouped_view(): instances live in another DataSet
+    void set_rows(std::shared_ptr<const RowStore> rows);
+    std::shared_ptr<const RowStore> rows_ = std::make_shared<RowStore>(0, 0);   // shared with grouped views
     size_t n_features_ = 0;
     std::vector<int> start_, count_, label_, perm_;
     bool zero_based_ = false;

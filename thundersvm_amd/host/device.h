@@ -30,6 +30,11 @@ inline void abi_check(int rc) {
     throw std::runtime_error(std::string("thundersvm_amd kernel call failed: ") + tsvm_last_error());
 }
 
+// The stream that everything outside a solve's own streams is enqueued on: uploads, row layouts, prediction.  One per
+// device and process, independent of the default stream (whose work would wait for, and hold up, every class pair that
+// is being solved).
+hipStream_t work_stream();
+
 // Device blocks that buffers have released, kept for the next buffer of about the same size: hipMalloc and hipFree cost
 // microseconds to milliseconds each (hipFree waits for the device), and a small training run makes some forty of them.
 // Blocks are rounded up to quarter powers of two; blocks above 64 MiB and whatever would take the pool over 512 MiB go
@@ -43,6 +48,12 @@ public:
     void *take(size_t bytes);
     void give(void *p, size_t bytes, bool idle);
     void flush();
+    // While one exists on a thread, what the thread releases counts as idle.
+    struct Idle {
+        Idle() { ++depth(); }
+        ~Idle() { --depth(); }
+        static int &depth() { static thread_local int d = 0; return d; }
+    };
 
 private:
     struct Impl;
@@ -152,15 +163,19 @@ public:
     // Gives the memory up without freeing it: for a device that has stopped answering, where hipFree would not return.
     void abandon() { ptr_ = nullptr; count_ = 0; }
 
+    // (on work_stream(), as everything here; when upload returns the source has been read)
     void upload(const T *host, size_t count, size_t offset = 0) {
-        if (count) TSVM_HIP_CHECK(hipMemcpy(ptr_ + offset, host, count * sizeof(T), hipMemcpyHostToDevice));
+        if (count) HostStaging::instance().upload(ptr_ + offset, {{host, count * sizeof(T), 0}}, work_stream());
     }
     void upload(const std::vector<T> &v) { resize(v.size()); upload(v.data(), v.size()); }
     void download(T *host, size_t count, size_t offset = 0) const {
-        if (count) TSVM_HIP_CHECK(hipMemcpy(host, ptr_ + offset, count * sizeof(T), hipMemcpyDeviceToHost));
+        if (count)
+            HostStaging::instance().download(ptr_ + offset, count * sizeof(T), [host](const char *from, size_t off, size_t len) {
+                parallel_memcpy((char *) host + off, from, len);
+            }, work_stream());
     }
     std::vector<T> to_host() const { std::vector<T> v(count_); download(v.data(), count_); return v; }
-    void zero() { if (count_) TSVM_HIP_CHECK(hipMemset(ptr_, 0, count_ * sizeof(T))); }
+    void zero() { if (count_) TSVM_HIP_CHECK(hipMemsetAsync(ptr_, 0, count_ * sizeof(T), work_stream())); }
 
 private:
     T *ptr_ = nullptr;

@@ -41,6 +41,29 @@ struct DevicePool::Impl {
     }
 };
 
+hipStream_t work_stream() {
+    static std::mutex mu;
+    static std::map<int, hipStream_t> streams;
+    int dev = 0;
+    TSVM_HIP_CHECK(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lock(mu);
+    auto it = streams.find(dev);
+    if (it == streams.end()) {
+        hipStream_t s = nullptr;
+        TSVM_HIP_CHECK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+        it = streams.emplace(dev, s).first;
+        static bool registered = false;
+        if (!registered) {
+            registered = true;
+            atexit([] {
+                for (auto &kv : streams) (void) hipStreamDestroy(kv.second);
+                streams.clear();
+            });
+        }
+    }
+    return it->second;
+}
+
 DevicePool &DevicePool::instance() {
     static DevicePool pool;
     return pool;
@@ -101,7 +124,7 @@ void DevicePool::give(void *p, size_t bytes, bool idle) {
         (void) hipFree(p);
         return;
     }
-    (idle ? I.ready : I.waiting)[std::make_pair(dev, size)].push_back(p);
+    (idle || Idle::depth() > 0 ? I.ready : I.waiting)[std::make_pair(dev, size)].push_back(p);
     I.total += size;
 }
 
@@ -379,57 +402,56 @@ bool KernelMatrix::choose_dense(size_t n, size_t n_features, size_t nnz) {
     return (double) ld <= 32.0 * std::max(avg, 1.0);
 }
 
-// CSR assembly on the host (kernelmatrix.cpp:183-207): n_features = largest feature id + 1, ids kept
-// as given; self dot products from the CSR values in stored order; then the layout is chosen.
-std::shared_ptr<DeviceRows> DeviceRows::from_host(const DataSet::node2d &all, const int *rows, size_t n_rows) {
+// The reference's CSR arrays (kernelmatrix.cpp:183-207): n_features = largest feature id + 1, ids kept as given; self dot
+// products from the CSR values in stored order; then the layout is chosen.
+std::shared_ptr<DeviceRows> DeviceRows::from_host(const RowStore &rows) {
     auto out = std::make_shared<DeviceRows>();
     DeviceRows &r = *out;
-    r.n = n_rows;
-    std::vector<int64_t> ptr(n_rows + 1, 0);
-    int max_index = 0;
-#pragma omp parallel for reduction(max : max_index) schedule(static)
-    for (size_t i = 0; i < n_rows; ++i) {
-        const auto &row = all[rows ? rows[i] : i];
-        ptr[i + 1] = (int64_t) row.size();
-        for (const auto &nd : row) max_index = std::max(max_index, nd.index);
+    r.n = rows.size();
+    r.nnz = rows.nnz();
+    const int64_t first = rows.ptr()[0];
+    const int *const col = rows.col() + first;
+    const kernel_type *const val = rows.val() + first;
+    int max_index = 0, all_float = 1;
+#pragma omp parallel for schedule(static) reduction(max : max_index) reduction(min : all_float) num_threads(threads_for(r.nnz))
+    for (size_t e = 0; e < r.nnz; ++e) {
+        max_index = std::max(max_index, col[e]);
+        all_float = (double) (float) val[e] != (double) val[e] ? 0 : all_float;
     }
-    for (size_t i = 0; i < n_rows; ++i) ptr[i + 1] += ptr[i];
-    r.nnz = (size_t) ptr[n_rows];
     r.n_features = (size_t) max_index + 1;
-    // (not value-initialised: a std::vector would be zero-filled by one thread, 12 bytes per non-zero, before the
-    // threads below write every element anyway)
-    std::unique_ptr<kernel_type[]> val(new kernel_type[r.nnz]);
-    std::unique_ptr<int[]> col(new int[r.nnz]);
-    int all_float = 1;
-#pragma omp parallel for schedule(static) reduction(min : all_float)
-    for (size_t i = 0; i < n_rows; ++i) {
-        const auto &row = all[rows ? rows[i] : i];
-        size_t e = (size_t) ptr[i];
-        for (const auto &nd : row) {
-            val[e] = nd.value;
-            col[e] = nd.index;
-            if ((double) (float) nd.value != (double) nd.value) all_float = 0;
-            ++e;
-        }
-    }
     r.values_fit_float = all_float != 0;
-    r.val.resize(r.nnz);
-    r.val.upload(val.get(), r.nnz);
-    r.col.resize(r.nnz);
-    r.col.upload(col.get(), r.nnz);
-    r.row_ptr.upload(ptr);
-    r.self_dot.resize(r.n);
-    abi_check(tsvm_csr_self_dot(r.val.data(), r.row_ptr.data(), (int64_t) r.n, r.self_dot.data(), nullptr));
     r.dense = KernelMatrix::choose_dense(r.n, r.n_features, r.nnz);
+    r.val.resize(r.nnz);
+    r.col.resize(r.nnz);
+    r.row_ptr.resize(r.n + 1);
+    tsvm::HostStaging &staging = tsvm::HostStaging::instance();
+    if (r.nnz) {
+        staging.upload(r.val.data(), {{val, r.nnz * sizeof(kernel_type), 0}}, tsvm::work_stream());
+        staging.upload(r.col.data(), {{col, r.nnz * sizeof(int), 0}}, tsvm::work_stream());
+    }
+    std::vector<int64_t> ptr;
+    const int64_t *host_ptr = rows.ptr();
+    if (first != 0 || !r.dense) {
+        ptr.assign(rows.ptr(), rows.ptr() + r.n + 1);
+        for (int64_t &p : ptr) p -= first;
+        host_ptr = ptr.data();
+    }
+    staging.upload(r.row_ptr.data(), {{host_ptr, (r.n + 1) * sizeof(int64_t), 0}}, tsvm::work_stream());
+    r.self_dot.resize(r.n);
+    abi_check(tsvm_csr_self_dot(r.val.data(), r.row_ptr.data(), (int64_t) r.n, r.self_dot.data(), tsvm::work_stream()));
     if (r.dense) {
         r.ld = (int64_t) ((r.n_features + 7) / 8 * 8);
         r.x.resize(r.n * (size_t) r.ld);
-        abi_check(tsvm_csr_to_dense(r.val.data(), r.col.data(), r.row_ptr.data(), (int64_t) r.n, r.x.data(), r.ld, nullptr));
-        TSVM_HIP_CHECK(hipDeviceSynchronize());
+        abi_check(tsvm_csr_to_dense(r.val.data(), r.col.data(), r.row_ptr.data(), (int64_t) r.n, r.x.data(), r.ld, tsvm::work_stream()));
         r.val.release();
         r.col.release();
         r.row_ptr.release();
-        r.find_indicator_columns();
+        // indicator columns are a run that ends with the last column: one other value there, in most data sets the
+        // first, and there are none
+        bool last_is_indicator = true;
+        for (size_t e = 0; e < r.nnz && last_is_indicator; ++e)
+            if (col[e] == max_index && val[e] != 0.0 && val[e] != 1.0) last_is_indicator = false;
+        if (last_is_indicator) r.find_indicator_columns();
     } else {
         r.host_row_ptr = std::move(ptr);
         r.build_sliced();
@@ -460,8 +482,7 @@ void DeviceRows::build_sliced() {
     ell_col.resize((size_t) sp[n_slices]);
     ell_val.resize((size_t) sp[n_slices] * (values_fit_float ? sizeof(float) : sizeof(double)));
     abi_check(tsvm_csr_to_sliced(val.data(), col.data(), row_ptr.data(), (int64_t) n, slice_ptr.data(), (int) n_features, ell_col.data(),
-                                 ell_val.data(), vt, nullptr));
-    TSVM_HIP_CHECK(hipDeviceSynchronize());
+                                 ell_val.data(), vt, tsvm::work_stream()));
     sliced_lds = need;
 }
 
@@ -476,17 +497,17 @@ std::shared_ptr<DeviceRows> DeviceRows::subset(const DeviceRows &base, const int
     tsvm::DeviceBuffer<int> d_rows(n_rows);
     d_rows.upload(rows, n_rows);
     r.self_dot.resize(n_rows);
-    abi_check(tsvm_gather_f64(base.self_dot.data(), d_rows.data(), (int) n_rows, r.self_dot.data(), nullptr));
+    abi_check(tsvm_gather_f64(base.self_dot.data(), d_rows.data(), (int) n_rows, r.self_dot.data(), tsvm::work_stream()));
     if (base.dense) {
         r.x.resize(n_rows * (size_t) r.ld);
-        abi_check(tsvm_gather_rows_f64(base.x.data(), base.ld, d_rows.data(), (int64_t) n_rows, r.x.data(), nullptr));
+        abi_check(tsvm_gather_rows_f64(base.x.data(), base.ld, d_rows.data(), (int64_t) n_rows, r.x.data(), tsvm::work_stream()));
         r.nnz = n_rows ? base.nnz / std::max<size_t>(base.n, 1) * n_rows : 0;   // estimate, informational only
         if (base.ind_first >= 0) {   // indicator columns of all rows are indicator columns of a subset (masks move as 8-byte words)
             r.ind_first = base.ind_first;
             r.ind_max_ones = base.ind_max_ones;
             r.ind_mask.resize(n_rows);
             abi_check(tsvm_gather_f64(reinterpret_cast<const double *>(base.ind_mask.data()), d_rows.data(), (int) n_rows,
-                                      reinterpret_cast<double *>(r.ind_mask.data()), nullptr));
+                                      reinterpret_cast<double *>(r.ind_mask.data()), tsvm::work_stream()));
         }
     } else {
         r.host_row_ptr.assign(n_rows + 1, 0);
@@ -497,18 +518,17 @@ std::shared_ptr<DeviceRows> DeviceRows::subset(const DeviceRows &base, const int
         r.val.resize(r.nnz);
         r.col.resize(r.nnz);
         abi_check(tsvm_csr_gather_rows(base.val.data(), base.col.data(), base.row_ptr.data(), d_rows.data(), (int64_t) n_rows,
-                                       r.row_ptr.data(), r.val.data(), r.col.data(), nullptr));
+                                       r.row_ptr.data(), r.val.data(), r.col.data(), tsvm::work_stream()));
         r.build_sliced();
     }
-    TSVM_HIP_CHECK(hipDeviceSynchronize());   // d_rows is released on return
     return out;
 }
 
 const std::vector<int> &DeviceRows::column_stats() const {
     if (column_stats_.size() != 2 * n_features) {
         tsvm::DeviceBuffer<int> d_counts(2 * n_features);
-        if (dense) abi_check(tsvm_column_stats_dense(x.data(), ld, (int64_t) n, (int) n_features, d_counts.data(), nullptr));
-        else abi_check(tsvm_column_stats_csr(val.data(), col.data(), (int64_t) nnz, (int) n_features, d_counts.data(), nullptr));
+        if (dense) abi_check(tsvm_column_stats_dense(x.data(), ld, (int64_t) n, (int) n_features, d_counts.data(), tsvm::work_stream()));
+        else abi_check(tsvm_column_stats_csr(val.data(), col.data(), (int64_t) nnz, (int) n_features, d_counts.data(), tsvm::work_stream()));
         column_stats_ = d_counts.to_host();
     }
     return column_stats_;
@@ -537,7 +557,7 @@ void DeviceRows::find_indicator_columns() {
     if (first == (int) n_features) return;
     tsvm::DeviceBuffer<uint64_t> masks(n);
     tsvm::DeviceBuffer<int> d_max(1);
-    abi_check(tsvm_indicator_masks(x.data(), ld, (int64_t) n, first, (int) n_features - first, masks.data(), d_max.data(), nullptr));
+    abi_check(tsvm_indicator_masks(x.data(), ld, (int64_t) n, first, (int) n_features - first, masks.data(), d_max.data(), tsvm::work_stream()));
     const int max_ones = d_max.to_host()[0];
     if (!indicator_run_pays((int) n_features, first, max_ones)) return;
     ind_first = first;
@@ -547,19 +567,13 @@ void DeviceRows::find_indicator_columns() {
 
 std::shared_ptr<DeviceRows> DeviceRows::of(const DataSet &dataset) {
     std::shared_ptr<void> &slot = dataset.device_cache();
-    if (!slot) slot = from_host(dataset.instances(), nullptr, dataset.instances().size());
+    if (!slot) slot = from_host(dataset.rows());
     return std::static_pointer_cast<DeviceRows>(slot);
 }
 
-KernelMatrix::KernelMatrix(const DataSet::node2d &instances, SvmParam param) : param(param) {
-    rows_ = DeviceRows::from_host(instances, nullptr, instances.size());
+KernelMatrix::KernelMatrix(const RowStore &rows, SvmParam param) : param(param) {
+    rows_ = DeviceRows::from_host(rows);
     finish(1);
-}
-
-KernelMatrix::KernelMatrix(const DataSet::node2d &all, const int *rows, size_t n_rows, SvmParam param, int repeat)
-    : param(param) {
-    rows_ = DeviceRows::from_host(all, rows, n_rows);
-    finish(repeat);
 }
 
 KernelMatrix::KernelMatrix(const DataSet &dataset, const int *rows, size_t n_rows, SvmParam param, int repeat)
@@ -577,11 +591,10 @@ void KernelMatrix::finish(int repeat) {
     repeat_ = repeat;
     diag_.resize(n_unique_ * repeat_);
     abi_check(tsvm_kernel_diag(rows_->self_dot.data(), (int64_t) n_unique_, (int) param.kernel_type, param.gamma, param.coef0,
-                               param.degree, diag_.data(), nullptr));
+                               param.degree, diag_.data(), tsvm::work_stream()));
     for (int rep = 1; rep < repeat_; ++rep)
         TSVM_HIP_CHECK(hipMemcpyAsync(diag_.data() + rep * n_unique_, diag_.data(), n_unique_ * sizeof(kernel_type),
-                                      hipMemcpyDeviceToDevice, nullptr));
-    TSVM_HIP_CHECK(hipDeviceSynchronize());
+                                      hipMemcpyDeviceToDevice, tsvm::work_stream()));
 }
 
 size_t KernelMatrix::reference_syncmem_bytes() const {
@@ -616,6 +629,13 @@ size_t KernelMatrix::reference_syncmem_bytes() const {
     if (dense_cols < nf && nnz_sparse != 0)   // some entry lies outside the dense part (kernelmatrix.cpp:151-176)
         bytes += (size_t) nnz_sparse * (sizeof(kernel_type) + sizeof(int)) + (size_t) (m + 1) * sizeof(int);
     return bytes;
+}
+
+size_t KernelMatrix::reference_syncmem_bytes_at_most() const {
+    // every stored entry counted twice (in the CSR arrays and in the sparse part), every column in the dense part
+    // (a gathered subset's entry count is an estimate: every cell then)
+    const size_t m = n_instances(), cells = m * n_features(), entries = rows_->dense ? cells : rows_->nnz * repeat_;
+    return 2 * entries * (sizeof(kernel_type) + sizeof(int)) + 2 * (m + 1) * sizeof(int) + 2 * m * sizeof(kernel_type) + cells * sizeof(kernel_type);
 }
 
 // A staging buffer that is all-zero whenever it is not in use: grown (and cleared) only when a call needs more.
@@ -704,78 +724,71 @@ void KernelMatrix::get_block(const int *d_idx, int m, void *d_out, int64_t ld, h
                                     stage_blk_.data(), wt, 1, stream));
 }
 
-// External batch (kernelmatrix.cpp:281-312, 385-406): features with id >= R.n_features are left out of
-// the dot product but stay in the batch row's self dot.
-void KernelMatrix::get_rows(const DataSet::node2d &instances, void *d_out, int64_t ld) const {
-    get_rows(instances.data(), instances.size(), d_out, ld);
-}
-
 // The batch goes to the device as CSR (flattened by all cores into pinned memory, copied asynchronously) together
 // with its rows' self dot products; with dense stored rows it is also laid out as a dense matrix of the stored rows'
 // width (columns >= n_features are dropped from the products, kernelmatrix.cpp:392, but stay in the self dot).
-KernelMatrix::StagedBatch KernelMatrix::stage_batch(const std::vector<DataSet::node> *instances, size_t n_rows) const {
+KernelMatrix::StagedBatch KernelMatrix::stage_batch(const RowStore &batch, size_t first, size_t n_rows) const {
     const DeviceRows &R = *rows_;
     const int m = (int) n_rows;
-    TSVM_HIP_CHECK(hipStreamSynchronize(nullptr));   // a previous batch's copies have left the staging memory
+    TSVM_HIP_CHECK(hipStreamSynchronize(tsvm::work_stream()));   // a previous batch's copies have left the staging memory
     h_ptr_.reserve((size_t) m + 1);
     int64_t *ptr = h_ptr_.data();
-    ptr[0] = 0;
-    for (int r = 0; r < m; ++r) ptr[r + 1] = ptr[r] + (int64_t) instances[r].size();
+    const int64_t e0 = batch.ptr()[first];
+    for (int r = 0; r <= m; ++r) ptr[r] = batch.ptr()[first + r] - e0;
     const size_t total = (size_t) ptr[m];
     h_val_.reserve(total);
     h_col_.reserve(total);
     kernel_type *val = h_val_.data();
     int *col = h_col_.data();
+    const kernel_type *const from_val = batch.val() + e0;
+    const int *const from_col = batch.col() + e0;
     // (indicator columns of the stored rows: the batch can use them when its own values there are zeros and ones)
     const int ind_lo = R.ind_first >= 0 ? R.ind_first : 0x7fffffff, ind_hi = (int) R.n_features;
     int not_indicator = 0;
-#pragma omp parallel for schedule(static) reduction(max : not_indicator)
-    for (int r = 0; r < m; ++r) {
-        size_t e = (size_t) ptr[r];
-        for (const auto &nd : instances[r]) {
-            val[e] = nd.value;
-            col[e] = nd.index;
-            if (nd.index >= ind_lo && nd.index < ind_hi && nd.value != 0.0 && nd.value != 1.0) not_indicator = 1;
-            ++e;
-        }
+#pragma omp parallel for schedule(static) reduction(max : not_indicator) num_threads(threads_for(total))
+    for (size_t e = 0; e < total; ++e) {
+        val[e] = from_val[e];
+        col[e] = from_col[e];
+        if (col[e] >= ind_lo && col[e] < ind_hi && val[e] != 0.0 && val[e] != 1.0) not_indicator = 1;
     }
     if (b_val_.size() < total) { b_val_.resize(total); b_col_.resize(total); }
     if (b_ptr_.size() < (size_t) m + 1) b_ptr_.resize(m + 1);
     if (total) {
-        TSVM_HIP_CHECK(hipMemcpyAsync(b_val_.data(), val, total * sizeof(kernel_type), hipMemcpyHostToDevice, nullptr));
-        TSVM_HIP_CHECK(hipMemcpyAsync(b_col_.data(), col, total * sizeof(int), hipMemcpyHostToDevice, nullptr));
+        TSVM_HIP_CHECK(hipMemcpyAsync(b_val_.data(), val, total * sizeof(kernel_type), hipMemcpyHostToDevice, tsvm::work_stream()));
+        TSVM_HIP_CHECK(hipMemcpyAsync(b_col_.data(), col, total * sizeof(int), hipMemcpyHostToDevice, tsvm::work_stream()));
     }
-    TSVM_HIP_CHECK(hipMemcpyAsync(b_ptr_.data(), ptr, ((size_t) m + 1) * sizeof(int64_t), hipMemcpyHostToDevice, nullptr));
+    TSVM_HIP_CHECK(hipMemcpyAsync(b_ptr_.data(), ptr, ((size_t) m + 1) * sizeof(int64_t), hipMemcpyHostToDevice, tsvm::work_stream()));
     if (stage_sd_.size() < (size_t) m) stage_sd_.resize(m);
-    abi_check(tsvm_csr_self_dot(b_val_.data(), b_ptr_.data(), m, stage_sd_.data(), nullptr));
+    abi_check(tsvm_csr_self_dot(b_val_.data(), b_ptr_.data(), m, stage_sd_.data(), tsvm::work_stream()));
     StagedBatch out;
     out.sd = stage_sd_.data();
     out.indicator_values = R.ind_first >= 0 && !not_indicator;
     if (R.dense) {
         if (stage_.size() < (size_t) m * R.ld) stage_.resize((size_t) m * R.ld);
-        abi_check(tsvm_csr_to_dense(b_val_.data(), b_col_.data(), b_ptr_.data(), m, stage_.data(), R.ld, nullptr));
+        abi_check(tsvm_csr_to_dense(b_val_.data(), b_col_.data(), b_ptr_.data(), m, stage_.data(), R.ld, tsvm::work_stream()));
         out.a = stage_.data();
         out.lda = R.ld;
     }
     return out;
 }
 
-void KernelMatrix::get_rows(const std::vector<DataSet::node> *instances, size_t n_rows, void *d_out, int64_t ld) const {
+// External batch (kernelmatrix.cpp:281-312, 385-406).
+void KernelMatrix::get_rows(const RowStore &batch, size_t first, size_t n_rows, void *d_out, int64_t ld) const {
     const DeviceRows &R = *rows_;
     const int m = (int) n_rows;
     if (m == 0) return;
-    const StagedBatch b = stage_batch(instances, n_rows);
+    const StagedBatch b = stage_batch(batch, first, n_rows);
     const int n = (int) n_unique_;
     if (R.dense) {
         abi_check(tsvm_get_rows_dense(R.x.data(), R.ld, nullptr, n, (int) R.n_features, R.self_dot.data(), b.a, b.lda, nullptr, m,
                                       b.sd, (int) param.kernel_type, param.gamma, param.coef0, param.degree,
-                                      d_out, row_type(), nullptr, ld, nullptr));
+                                      d_out, row_type(), nullptr, ld, tsvm::work_stream()));
     } else {
         if (stage_.size() < (size_t) m * R.n_features) stage_.resize((size_t) m * R.n_features);
         abi_check(tsvm_csr_stage_rows(b_val_.data(), b_col_.data(), b_ptr_.data(), nullptr, m, (int) R.n_features,
-                                      stage_.data(), nullptr));
+                                      stage_.data(), tsvm::work_stream()));
         abi_check(tsvm_get_rows_csr(R.val.data(), R.col.data(), R.row_ptr.data(), nullptr, n, R.self_dot.data(), stage_.data(), m,
                                     b.sd, (int) param.kernel_type, param.gamma, param.coef0, param.degree,
-                                    d_out, row_type(), nullptr, ld, nullptr));
+                                    d_out, row_type(), nullptr, ld, tsvm::work_stream()));
     }
 }

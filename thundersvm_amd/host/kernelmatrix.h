@@ -54,8 +54,8 @@ struct DeviceRows {
     static int indicator_run_start(const int *stats, int n_features);
     static bool indicator_run_pays(int n_features, int first, int max_ones);
 
-    // rows[0..n_rows) of `all` (rows == nullptr: the first n_rows), assembled on the host and uploaded
-    static std::shared_ptr<DeviceRows> from_host(const DataSet::node2d &all, const int *rows, size_t n_rows);
+    // all rows of `rows`, uploaded
+    static std::shared_ptr<DeviceRows> from_host(const RowStore &rows);
     // rows[0..n_rows) of `base`, gathered on the device; keeps base's layout and feature count
     static std::shared_ptr<DeviceRows> subset(const DeviceRows &base, const int *rows, size_t n_rows);
     // the device copy of all instances of a DataSet, built on first use and kept with the DataSet
@@ -64,9 +64,7 @@ struct DeviceRows {
 
 class KernelMatrix {
 public:
-    KernelMatrix(const DataSet::node2d &instances, SvmParam param);
-    // Rows `rows[0..n_rows)` of `all`, without materialising a node2d copy.
-    KernelMatrix(const DataSet::node2d &all, const int *rows, size_t n_rows, SvmParam param, int repeat = 1);
+    KernelMatrix(const RowStore &rows, SvmParam param);
     // Rows `rows[0..n_rows)` of the DataSet's device-resident instances (rows == nullptr: all of them, shared
     // in place).  The feature count is the whole DataSet's, not the subset's: extra all-zero columns add
     // exact zeros to every dot product.
@@ -82,8 +80,7 @@ public:
     // the m x m block K(x_idx[r], x_idx[t]) -> d_out[r*ld + t] (what the local solver reads; row_type() elements)
     void get_block(const int *d_idx, int m, void *d_out, int64_t ld, hipStream_t stream = nullptr) const;
     // kernel rows of an external batch -> element i*ld + j of d_out (row_type() elements)
-    void get_rows(const DataSet::node2d &instances, void *d_out, int64_t ld) const;
-    void get_rows(const std::vector<DataSet::node> *instances, size_t m, void *d_out, int64_t ld) const;   // the same for a slice
+    void get_rows(const RowStore &batch, size_t first, size_t m, void *d_out, int64_t ld) const;
 
     // An external batch on the device: dense [m][lda] in the stored rows' column layout (dense stored rows only) and
     // the rows' self dot products; valid until the next call that stages a batch.  indicator_values: the stored rows
@@ -94,7 +91,7 @@ public:
         const kernel_type *sd = nullptr;
         bool indicator_values = false;
     };
-    StagedBatch stage_batch(const std::vector<DataSet::node> *instances, size_t m) const;
+    StagedBatch stage_batch(const RowStore &batch, size_t first, size_t m) const;   // rows first .. first + m - 1 of `batch`
     const DeviceRows &rows() const { return *rows_; }
 
     const kernel_type *diag() const { return diag_.data(); }          // device, n_instances() entries
@@ -117,6 +114,7 @@ public:
     // what SvmModel::get_working_set_size subtracts from the memory budget (svmmodel.cpp:437-451).  An entry
     // stored with the value 0 counts as absent in the dense layout and as a non-zero entry in the CSR layout.
     size_t reference_syncmem_bytes() const;
+    size_t reference_syncmem_bytes_at_most() const;   // no less than that, from the shape alone
 
 private:
     void finish(int repeat);

@@ -42,7 +42,7 @@ int main(int argc, char **argv) {
         test.load_from_file(parser.svmpredict_input_file);
         TSVM_LOG << "data loading time = " << since(t0);
         t0 = now();
-        std::vector<float_type> predict_y = model->predict(test.instances(), -1);
+        std::vector<float_type> predict_y = model->predict(test, -1);
         TSVM_LOG << "prediction time = " << since(t0);
         std::ofstream out(parser.svmpredict_output_file);
         for (float_type v : predict_y) out << v << '\n';   // (the reference ends each line with std::endl: the same bytes)

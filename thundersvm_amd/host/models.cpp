@@ -36,7 +36,7 @@ void SvmModel::model_setup(const DataSet &, SvmParam &p) {   // svmmodel.cpp:22-
     n_binary_models = n_classes * (n_classes - 1) / 2;
     rho.assign(n_binary_models, 0);
     n_sv.assign(n_classes, 0);
-    sv.clear();
+    sv = std::make_shared<RowStore>(0, 0);
     sv_k_mat.reset();
     predict_plan_.reset();
     sv_indices.clear();
@@ -74,23 +74,27 @@ int SvmModel::get_working_set_size(const KernelMatrix &k_mat, size_t held_bytes)
                                         std::to_string(n_instances) + " instances");
         return ws_override;
     }
-    const size_t used = k_mat.reference_syncmem_bytes() + n_instances * (sizeof(int) + 2 * sizeof(float_type)) + held_bytes;
-    if (param.max_mem_size < used) throw std::bad_alloc();
-    const size_t free_mem = param.max_mem_size - used;
-    const size_t by_mem = (size_t) max2power((double) (free_mem / sizeof(kernel_type) / (n_instances + n_features)));
-    const int ws = std::min(max2power((double) n_instances), (int) std::min(by_mem, (size_t) 1024));
+    const size_t others = n_instances * (sizeof(int) + 2 * sizeof(float_type)) + held_bytes;
+    const auto size_for = [&](size_t used) {
+        const size_t free_mem = param.max_mem_size - used;
+        const size_t by_mem = (size_t) max2power((double) (free_mem / sizeof(kernel_type) / (n_instances + n_features)));
+        return std::min(max2power((double) n_instances), (int) std::min(by_mem, (size_t) 1024));
+    };
+    // (counting the reference's column split takes a pass over the columns; where even the most that it can come to
+    // leaves room for the largest working set, the count changes nothing)
+    const size_t at_most = k_mat.reference_syncmem_bytes_at_most() + others;
+    int ws = param.max_mem_size > at_most ? size_for(at_most) : 0;
+    if (ws < std::min(max2power((double) n_instances), 1024)) {
+        const size_t used = k_mat.reference_syncmem_bytes() + others;
+        if (param.max_mem_size < used) throw std::bad_alloc();
+        ws = size_for(used);
+    }
     TSVM_LOG << "working set size = " << ws;
     return ws;
 }
 
-// sv[s] = instances[sv_indices[s]]: the model owns copies of its support vectors (svc.cpp:86-108).  With
-// hundreds of thousands of support vectors the copy is tens of milliseconds of memory traffic, so it is
-// spread over the host cores.
-void SvmModel::copy_support_vectors(const DataSet::node2d &instances) {
-    sv.resize(sv_indices.size());
-#pragma omp parallel for schedule(static)
-    for (size_t s = 0; s < sv_indices.size(); ++s) sv[s] = instances[sv_indices[s]];
-}
+// The model owns copies of its support vectors (svc.cpp:86-108).
+void SvmModel::copy_support_vectors(const RowStore &rows) { sv = rows.gather(sv_indices.data(), sv_indices.size()); }
 
 void SvmModel::run_solver(CSMOSolver &solver, const KernelMatrix &k_mat, const std::vector<int> &y,
                           std::vector<float_type> &alpha, float_type &rho_out, std::vector<float_type> &f_val,
@@ -109,9 +113,8 @@ std::vector<float_type> SvmModel::cross_validation(DataSet dataset, SvmParam p, 
     dataset.group_classes(this->param.svm_type == SvmParam::C_SVC);
     std::vector<float_type> y_predict_all(dataset.n_instances());
     for (int k = 0; k < n_fold; ++k) {
-        DataSet::node2d x_train, x_test;
         std::vector<float_type> y_train;
-        std::vector<int> test_idx;
+        std::vector<int> train_idx, test_idx;
         for (size_t c = 0; c < dataset.n_classes(); ++c) {
             const int fold = dataset.count()[c] / n_fold;
             const std::vector<int> ids = dataset.original_index((int) c);
@@ -119,17 +122,17 @@ std::vector<float_type> SvmModel::cross_validation(DataSet dataset, SvmParam p, 
             const size_t hi = (k == n_fold - 1) ? ids.size() : std::min(ids.size(), lo + fold);
             for (size_t t = 0; t < ids.size(); ++t) {
                 if (t >= lo && t < hi) {
-                    x_test.push_back(dataset.instances()[ids[t]]);
                     test_idx.push_back(ids[t]);
                 } else {
-                    x_train.push_back(dataset.instances()[ids[t]]);
+                    train_idx.push_back(ids[t]);
                     y_train.push_back(dataset.y()[ids[t]]);
                 }
             }
         }
-        DataSet train_set(x_train, (int) dataset.n_features(), y_train);
+        DataSet train_set(dataset.rows().gather(train_idx.data(), train_idx.size()), (int) dataset.n_features(), y_train);
         this->train(train_set, p);
-        std::vector<float_type> y_predict = this->predict(x_test, 1000);
+        predict_dec_values(*dataset.rows().gather(test_idx.data(), test_idx.size()), dec_values, 1000);
+        std::vector<float_type> y_predict = finish_predict((int) test_idx.size());
         for (size_t i = 0; i < y_predict.size(); ++i) y_predict_all[test_idx[i]] = y_predict[i];
     }
     return y_predict_all;
@@ -137,8 +140,8 @@ std::vector<float_type> SvmModel::cross_validation(DataSet dataset, SvmParam p, 
 
 void SvmModel::compute_linear_coef_single_model(size_t n_feature, bool zero_based) {
     linear_coef.assign(zero_based ? n_feature + 1 : n_feature, 0);
-    for (size_t i = 0; i < sv.size(); ++i)
-        for (const auto &nd : sv[i]) linear_coef[zero_based ? nd.index : nd.index - 1] += coef[i] * nd.value;
+    for (size_t i = 0; i < sv->size(); ++i)
+        for (int64_t e = sv->ptr()[i]; e < sv->ptr()[i + 1]; ++e) linear_coef[zero_based ? sv->col()[e] : sv->col()[e] - 1] += coef[i] * sv->val()[e];
 }
 
 // LibSVM text model (svmmodel.cpp:193-264): rho/gamma at stream default precision, coefficients with
@@ -153,7 +156,7 @@ std::string SvmModel::save_to_string() {
     if (param.kernel_type == SvmParam::POLY || param.kernel_type == SvmParam::SIGMOID)
         s << "coef0 " << param.coef0 << std::endl;
     s << "nr_class " << n_classes << std::endl;
-    s << "total_sv " << sv.size() << std::endl;
+    s << "total_sv " << sv->size() << std::endl;
     s << "rho ";
     for (int i = 0; i < n_binary_models; ++i) s << rho[i] << " ";
     s << std::endl;
@@ -181,7 +184,7 @@ std::string SvmModel::save_to_string() {
     // side by side into strings of their own and joined in order.  "%.16g" / "%.8g" are what the stream writes for
     // setprecision(16) / setprecision(8) (its num_put goes through the same printf conversion in the C locale).
     const int rows = (param.svm_type == SvmParam::NU_SVC || param.svm_type == SvmParam::C_SVC) ? n_classes - 1 : 1;
-    const size_t n = sv.size();
+    const size_t n = sv->size();
     const int n_runs = (int) std::max<size_t>(1, std::min<size_t>((size_t) omp_get_max_threads() * 4, n / 256));
     std::vector<std::string> run_text(n_runs);
 #pragma omp parallel for schedule(dynamic, 1)
@@ -190,7 +193,8 @@ std::string SvmModel::save_to_string() {
         char buf[64];
         for (size_t i = n * r / n_runs; i < n * (r + 1) / n_runs; ++i) {
             for (int j = 0; j < rows; ++j) o.append(buf, snprintf(buf, sizeof buf, "%.16g ", (double) coef[j * n + i]));
-            for (const auto &nd : sv[i]) o.append(buf, snprintf(buf, sizeof buf, "%d:%.8g ", nd.index, (double) nd.value));
+            for (int64_t e = sv->ptr()[i]; e < sv->ptr()[i + 1]; ++e)
+                o.append(buf, snprintf(buf, sizeof buf, "%d:%.8g ", sv->col()[e], (double) sv->val()[e]));
             o.push_back('\n');
         }
     }
@@ -273,7 +277,7 @@ void SvmModel::load_from_string(std::string data) {
             // reference give.  Exactly total_sv lines are read; missing ones leave empty vectors with zero coefficients.
             const bool cls = param.svm_type == SvmParam::C_SVC || param.svm_type == SvmParam::NU_SVC;
             const int rows = cls ? n_classes - 1 : 1;
-            sv.assign(n_total_sv, {});
+            DataSet::node2d nodes(n_total_sv);
             coef.assign((size_t) rows * n_total_sv, 0);
             const char *text = data.c_str();
             const size_t size = data.size();
@@ -333,7 +337,7 @@ void SvmModel::load_from_string(std::string data) {
                         run_max[r] = std::max(run_max[r], (int) idx);
                     }
                     if (run_bad[r]) break;
-                    sv[i].assign(row.begin(), row.end());
+                    nodes[i].assign(row.begin(), row.end());
                     q = eol + 1;
                 }
             }
@@ -341,6 +345,7 @@ void SvmModel::load_from_string(std::string data) {
                 if (run_bad[r]) throw std::runtime_error("error when loading model file");
                 sv_max_index = std::max(sv_max_index, run_max[r]);
             }
+            sv = RowStore::from_nodes(nodes);
             break;                                                        // nothing follows the support vectors
         }
     }
@@ -412,8 +417,8 @@ void SVC::train(const DataSet &dataset, SvmParam p) {   // svc.cpp:41-145
                 n_sv[c]++;
                 sv_indices.push_back(id);
             }
-    copy_support_vectors(grouped.instances());
-    n_total_sv = (int) sv.size();
+    copy_support_vectors(grouped.rows());
+    n_total_sv = (int) sv->size();
     TSVM_LOG << "#total unique sv = " << n_total_sv;
     // LibSVM coefficient layout: pair (i<j) stores class i's SVs in row j-1 and class j's SVs in row i
     coef.assign((size_t) (n_classes - 1) * n_total_sv, 0);
@@ -440,8 +445,9 @@ void SVC::train(const DataSet &dataset, SvmParam p) {   // svc.cpp:41-145
                 const std::vector<int> ids = grouped.original_index(i, j);
                 for (size_t l = 0; l < ids.size(); ++l) {
                     if (alpha[k][l] == 0) continue;
-                    for (const auto &nd : grouped.instances()[ids[l]])
-                        linear_coef[k * nf + (grouped.is_zero_based() ? nd.index : nd.index - 1)] += alpha[k][l] * nd.value;
+                    const RowStore &R = grouped.rows();
+                    for (int64_t e = R.ptr()[ids[l]]; e < R.ptr()[ids[l] + 1]; ++e)
+                        linear_coef[k * nf + (grouped.is_zero_based() ? R.col()[e] : R.col()[e] - 1)] += alpha[k][l] * R.val()[e];
                 }
             }
     }
@@ -608,7 +614,11 @@ void SVC::train_pairs_in_lockstep(const DataSet &grouped, int lanes, std::vector
         BinaryProblem &p = *active[a];
         solver_stats[p.k] = p.task->stats();
         if (keep_binary) binary_f[p.k] = p.f_val;
-        p.task.reset();   // synchronises and releases the pair's stream before its lane is reused
+        {
+            p.task.reset();   // synchronises and releases the pair's stream before its lane is reused
+            tsvm::DevicePool::Idle idle;
+            p.k_mat.reset();
+        }
         (void) hipEventDestroy(p.rows_done);
         (void) hipEventDestroy(p.solved);
         finish_binary(p, alpha[p.k]);
@@ -823,9 +833,8 @@ void SVC::probability_train(const DataSet &grouped) {
     const int n_fold = 5;
     std::vector<float_type> dec_all(grouped.n_instances() * (size_t) n_binary_models);
     for (int fold = 0; fold < n_fold; ++fold) {
-        DataSet::node2d x_train, x_test;
         std::vector<float_type> y_train;
-        std::vector<int> test_idx;
+        std::vector<int> train_idx, test_idx;
         for (size_t c = 0; c < grouped.n_classes(); ++c) {
             const std::vector<int> ids = grouped.original_index((int) c);
             const size_t per_fold = ids.size() / n_fold;
@@ -833,10 +842,9 @@ void SVC::probability_train(const DataSet &grouped) {
             const size_t end = fold == n_fold - 1 ? ids.size() : std::min(ids.size(), begin + per_fold);
             for (size_t l = 0; l < ids.size(); ++l) {
                 if (l >= begin && l < end) {
-                    x_test.push_back(grouped.instances()[ids[l]]);
                     test_idx.push_back(ids[l]);
                 } else {
-                    x_train.push_back(grouped.instances()[ids[l]]);
+                    train_idx.push_back(ids[l]);
                     y_train.push_back(grouped.y()[ids[l]]);
                 }
             }
@@ -845,10 +853,10 @@ void SVC::probability_train(const DataSet &grouped) {
         fold_model.set_max_iter(max_iter);
         fold_model.cache_bytes = cache_bytes;
         fold_model.pair_lanes = pair_lanes;
-        fold_model.train(DataSet(x_train, (int) grouped.n_features(), y_train), param_no_prob);
+        fold_model.train(DataSet(grouped.rows().gather(train_idx.data(), train_idx.size()), (int) grouped.n_features(), y_train), param_no_prob);
         std::vector<float_type> dec;
-        fold_model.predict_dec_values(x_test, dec, 1000);
-        for (size_t t = 0; t < x_test.size(); ++t)
+        fold_model.predict_dec_values(*grouped.rows().gather(test_idx.data(), test_idx.size()), dec, 1000);
+        for (size_t t = 0; t < test_idx.size(); ++t)
             std::copy(dec.begin() + t * n_binary_models, dec.begin() + (t + 1) * n_binary_models,
                       dec_all.begin() + (size_t) test_idx[t] * n_binary_models);
     }
@@ -959,11 +967,11 @@ void SVR::train(const DataSet &dataset, SvmParam p) {
     CSMOSolver solver;
     run_solver(solver, k_mat, y, alpha_2, rho[0], f_val, param.C, param.C);
     if (keep_binary) binary_alpha.push_back(alpha_2);
-    save_svr_coef(alpha_2, dataset.instances());
+    save_svr_coef(alpha_2, dataset.rows());
     if (param.kernel_type == SvmParam::LINEAR) compute_linear_coef_single_model(dataset.n_features(), dataset.is_zero_based());
 }
 
-void SVR::save_svr_coef(const std::vector<float_type> &alpha_2, const DataSet::node2d &instances) {   // svr.cpp:43-62
+void SVR::save_svr_coef(const std::vector<float_type> &alpha_2, const RowStore &rows) {   // svr.cpp:43-62
     const size_t n = alpha_2.size() / 2;
     for (size_t i = 0; i < n; ++i) {
         const float_type a = alpha_2[i] - alpha_2[i + n];
@@ -972,11 +980,11 @@ void SVR::save_svr_coef(const std::vector<float_type> &alpha_2, const DataSet::n
             coef.push_back(a);
         }
     }
-    copy_support_vectors(instances);
-    n_sv[0] = (int) sv.size();
+    copy_support_vectors(rows);
+    n_sv[0] = (int) sv->size();
     n_sv[1] = 0;
-    n_total_sv = (int) sv.size();
-    TSVM_LOG << "rho = " << rho[0] << ", #sv = " << sv.size();
+    n_total_sv = (int) sv->size();
+    TSVM_LOG << "rho = " << rho[0] << ", #sv = " << sv->size();
 }
 
 void NuSVR::model_setup(const DataSet &dataset, SvmParam &p) {
@@ -1001,7 +1009,7 @@ void NuSVR::train(const DataSet &dataset, SvmParam p) {   // nusvr.cpp:7-41
     NuSMOSolver solver(true);
     run_solver(solver, k_mat, y, alpha_2, rho[0], f_val, param.C, param.C);
     if (keep_binary) binary_alpha.push_back(alpha_2);
-    save_svr_coef(alpha_2, dataset.instances());
+    save_svr_coef(alpha_2, dataset.rows());
     if (param.kernel_type == SvmParam::LINEAR) compute_linear_coef_single_model(dataset.n_features(), dataset.is_zero_based());
 }
 
@@ -1031,10 +1039,10 @@ void OneClassSVC::train(const DataSet &dataset, SvmParam p) {
             sv_indices.push_back(i);
             coef.push_back(alpha[i]);
         }
-    copy_support_vectors(dataset.instances());
-    n_sv[0] = (int) sv.size();
+    copy_support_vectors(dataset.rows());
+    n_sv[0] = (int) sv->size();
     n_sv[1] = 0;
-    n_total_sv = (int) sv.size();
+    n_total_sv = (int) sv->size();
     if (param.kernel_type == SvmParam::LINEAR) compute_linear_coef_single_model(dataset.n_features(), dataset.is_zero_based());
 }
 

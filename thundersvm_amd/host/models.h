@@ -15,7 +15,7 @@ public:
     virtual ~SvmModel() = default;
     virtual void train(const DataSet &dataset, SvmParam param) = 0;
     std::vector<float_type> predict(const DataSet::node2d &instances, int batch_size = -1);
-    void predict_dec_values(const DataSet::node2d &instances, std::vector<float_type> &dec_values, int batch_size) const;
+    void predict_dec_values(const RowStore &rows, std::vector<float_type> &dec_values, int batch_size) const;
     // The same for the instances of a DataSet; when the DataSet has a device-resident copy of its rows in the dense
     // layout (DeviceRows::of), the kernels read the rows where they lie: nothing is assembled on the host or uploaded.
     std::vector<float_type> predict(const DataSet &dataset, int batch_size = -1);
@@ -28,7 +28,8 @@ public:
     virtual void load_from_string(std::string data);
 
     int total_sv() const { return n_total_sv; }
-    const DataSet::node2d &svs() const { return sv; }
+    const DataSet::node2d &svs() const { return sv->nodes(); }
+    const RowStore &sv_rows() const { return *sv; }
     const std::vector<int> &get_n_sv() const { return n_sv; }
     const std::vector<float_type> &get_coef() const { return coef; }
     const std::vector<float_type> &get_linear_coef() const { return linear_coef; }
@@ -69,7 +70,7 @@ protected:
     // one batch, rows already on the device as a dense matrix; false when the kernels do not take this model's shape
     bool predict_batch_fused(const PredictPlan &plan, const kernel_type *a, int64_t lda, const kernel_type *sd_a, size_t m,
                              bool indicator_values, float_type *dec_out) const;
-    void copy_support_vectors(const DataSet::node2d &instances);
+    void copy_support_vectors(const RowStore &rows);
     void run_solver(CSMOSolver &solver, const KernelMatrix &k_mat, const std::vector<int> &y, std::vector<float_type> &alpha,
                     float_type &rho, std::vector<float_type> &f_val, float_type Cp, float_type Cn, size_t held_bytes = 0);
     void compute_linear_coef_single_model(size_t n_feature, bool zero_based);
@@ -79,7 +80,7 @@ protected:
     std::vector<float_type> own_weight;
     std::vector<float_type> coef;
     std::vector<float_type> linear_coef;
-    DataSet::node2d sv;
+    std::shared_ptr<const RowStore> sv = std::make_shared<RowStore>(0, 0);
     mutable std::shared_ptr<KernelMatrix> sv_k_mat;   // device copy of sv, built by the first predict call
     mutable std::shared_ptr<PredictPlan> predict_plan_;
     std::vector<int> sv_indices;
@@ -138,7 +139,7 @@ public:
 
 protected:
     void model_setup(const DataSet &dataset, SvmParam &param) override;
-    void save_svr_coef(const std::vector<float_type> &alpha_2, const DataSet::node2d &instances);
+    void save_svr_coef(const std::vector<float_type> &alpha_2, const RowStore &rows);
 };
 
 class NuSVR : public SVR {

@@ -36,11 +36,11 @@ const SvmModel::PredictPlan &SvmModel::predict_plan() const {
     if (predict_plan_) return *predict_plan_;
     // the support vectors' device copy is built by the first predict call and kept for the next ones (the
     // reference rebuilds it per call, svmmodel.cpp:84)
-    if (!sv_k_mat) sv_k_mat.reset(new KernelMatrix(sv, param));
+    if (!sv_k_mat) sv_k_mat.reset(new KernelMatrix(*sv, param));
     auto plan = std::make_shared<PredictPlan>();
     PredictPlan &P = *plan;
     const DeviceRows &R = sv_k_mat->rows();
-    const size_t T = sv.size();
+    const size_t T = sv->size();
     std::vector<int> sv_start(n_classes, 0);
     for (int c = 1; c < n_classes; ++c) sv_start[c] = sv_start[c - 1] + n_sv[c - 1];
     P.rho.upload(rho);
@@ -119,7 +119,7 @@ bool SvmModel::predict_batch_fused(const PredictPlan &P, const kernel_type *a, i
         if (P.mask_a.size() < m) P.mask_a.resize(m);
         if (P.mask_max.size() < 1) P.mask_max.resize(1);
         abi_check(tsvm_indicator_masks(a, lda, (int64_t) m, R.ind_first, (int) R.n_features - R.ind_first, P.mask_a.data(),
-                                       P.mask_max.data(), nullptr));
+                                       P.mask_max.data(), tsvm::work_stream()));
     }
     const int km1 = n_classes - 1;
     // partial sums and decision values: from the persistent row arena (no allocation per call)
@@ -132,17 +132,20 @@ bool SvmModel::predict_batch_fused(const PredictPlan &P, const kernel_type *a, i
                                             P.col_map.data(), P.n_pad, P.coef_t.data(), P.chunks.data(), P.n_chunks,
                                             P.class_chunk_start.data(), P.rho.data(), n_classes, a, lda, (int64_t) m, sd_a,
                                             plan_masks ? P.mask_a.data() : nullptr, R.ind_max_ones, (int) param.kernel_type,
-                                            param.gamma, param.coef0, param.degree, d_part, d_dec, nullptr));
-    TSVM_HIP_CHECK(hipMemcpy(dec_out, d_dec, dec_doubles * sizeof(float_type), hipMemcpyDeviceToHost));
+                                            param.gamma, param.coef0, param.degree, d_part, d_dec, tsvm::work_stream()));
+    tsvm::HostStaging::instance().download(d_dec, dec_doubles * sizeof(float_type), [dec_out](const char *from, size_t off, size_t len) {
+        tsvm::parallel_memcpy((char *) dec_out + off, from, len);
+    }, tsvm::work_stream());
     return true;
 }
 
-void SvmModel::predict_dec_values(const DataSet::node2d &instances, std::vector<float_type> &dec, int batch_size) const {
-    dec.assign(instances.size() * (size_t) n_binary_models, 0);
-    if (instances.empty()) return;
-    const size_t T = sv.size();
+void SvmModel::predict_dec_values(const RowStore &rows, std::vector<float_type> &dec, int batch_size) const {
+    const size_t n_rows = rows.size();
+    dec.assign(n_rows * (size_t) n_binary_models, 0);
+    if (n_rows == 0) return;
+    const size_t T = sv->size();
     if (T == 0) {
-        for (size_t r = 0; r < instances.size(); ++r)
+        for (size_t r = 0; r < n_rows; ++r)
             for (int p = 0; p < n_binary_models; ++p) dec[r * n_binary_models + p] = -rho[p];
         return;
     }
@@ -160,14 +163,14 @@ void SvmModel::predict_dec_values(const DataSet::node2d &instances, std::vector<
         }
         if (batch_size < 1) batch_size = 1;
     }
-    const size_t bmax = std::min((size_t) batch_size, instances.size());
+    const size_t bmax = std::min((size_t) batch_size, n_rows);
     void *d_k = nullptr;
     const int64_t ldk = ((int64_t) T + 15) / 16 * 16;   // (rows padded to 16 elements: get_rows writes whole aligned vectors)
     DeviceBuffer<float_type> d_dec;
-    for (size_t b0 = 0; b0 < instances.size(); b0 += batch_size) {
-        const size_t bm = std::min((size_t) batch_size, instances.size() - b0);
+    for (size_t b0 = 0; b0 < n_rows; b0 += batch_size) {
+        const size_t bm = std::min((size_t) batch_size, n_rows - b0);
         if (fused) {
-            const KernelMatrix::StagedBatch b = k_mat.stage_batch(instances.data() + b0, bm);
+            const KernelMatrix::StagedBatch b = k_mat.stage_batch(rows, b0, bm);
             if (predict_batch_fused(P, b.a, b.lda, b.sd, bm, b.indicator_values, dec.data() + b0 * n_binary_models)) continue;
         }
         // kernel values of one batch (taken from the persistent row arena), then the reduction
@@ -175,16 +178,16 @@ void SvmModel::predict_dec_values(const DataSet::node2d &instances, std::vector<
             d_k = tsvm::RowArena::instance().acquire(bmax * (size_t) ldk * k_mat.row_elem_size(), false);
             d_dec.resize(bmax * n_binary_models);
         }
-        k_mat.get_rows(instances.data() + b0, bm, d_k, ldk);
+        k_mat.get_rows(rows, b0, bm, d_k, ldk);
         abi_check(tsvm_sum_kernel_values(P.coef.data(), (int) T, P.sv_start.data(), P.sv_count.data(), P.rho.data(), d_k,
-                                         k_mat.row_type(), ldk, d_dec.data(), n_classes, (int64_t) bm, nullptr));
+                                         k_mat.row_type(), ldk, d_dec.data(), n_classes, (int64_t) bm, tsvm::work_stream()));
         d_dec.download(dec.data() + b0 * n_binary_models, bm * n_binary_models);
     }
 }
 
 void SvmModel::predict_dec_values(const DataSet &dataset, std::vector<float_type> &dec, int batch_size) const {
     const std::shared_ptr<void> &slot = dataset.device_cache();
-    if (slot && !sv.empty() && dataset.n_instances() > 0) {
+    if (slot && sv->size() > 0 && dataset.n_instances() > 0) {
         const DeviceRows &A = *std::static_pointer_cast<DeviceRows>(slot);
         const PredictPlan &P = predict_plan();
         const DeviceRows &R = sv_k_mat->rows();
@@ -208,11 +211,11 @@ void SvmModel::predict_dec_values(const DataSet &dataset, std::vector<float_type
             if (ok) return;
         }
     }
-    predict_dec_values(dataset.instances(), dec, batch_size);
+    predict_dec_values(dataset.rows(), dec, batch_size);
 }
 
 std::vector<float_type> SvmModel::predict(const DataSet::node2d &instances, int batch_size) {   // svmmodel.cpp:157-171
-    predict_dec_values(instances, dec_values, batch_size);
+    predict_dec_values(*RowStore::from_nodes(instances), dec_values, batch_size);
     return finish_predict((int) instances.size());
 }
 

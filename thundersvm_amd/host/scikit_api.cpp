@@ -91,7 +91,7 @@ void train_on(DataSet &train, int svm_type, int kernel_type, int degree, float g
 int predict_on(DataSet &data, SvmModel *model, float *predict_label, int verbose) {
     tsvm::Log::enabled() = verbose != 0;
     const bool ok = guarded("prediction", [&] {
-        const std::vector<float_type> y = model->predict(data.instances(), -1);
+        const std::vector<float_type> y = model->predict(data, -1);
         for (size_t i = 0; i < y.size(); ++i) predict_label[i] = (float) y[i];
     });
     if (!ok) std::fill(predict_label, predict_label + data.n_instances(), std::nanf(""));
@@ -100,7 +100,7 @@ int predict_on(DataSet &data, SvmModel *model, float *predict_label, int verbose
 
 void decision_on(DataSet &data, SvmModel *model, int value_size, float *dec_value) {
     const bool ok = guarded("decision values", [&] {
-        model->predict(data.instances(), -1);
+        model->predict(data, -1);
         copy_out(model->get_dec_value(), dec_value, (size_t) (value_size > 0 ? value_size : 0));
     });
     if (!ok) std::fill(dec_value, dec_value + (value_size > 0 ? value_size : 0), std::nanf(""));

@@ -412,19 +412,21 @@ struct SolveTask::Impl {
         d_start.resize(2 * f_at + (size_t) n * sizeof(int));
         tsvm::HostStaging::instance().upload(d_start.data(), {{alpha.data(), (size_t) n * sizeof(float_type), 0},
                                                               {f_val.data(), (size_t) n * sizeof(float_type), f_at},
-                                                              {y.data(), (size_t) n * sizeof(int), 2 * f_at}}, nullptr);
+                                                              {y.data(), (size_t) n * sizeof(int), 2 * f_at}}, tsvm::work_stream());
         d_alpha = (float_type *) d_start.data();
         d_f = (float_type *) (d_start.data() + f_at);
         d_y = (int *) (d_start.data() + 2 * f_at);
         abi_check(tsvm_smo_start(d_alpha_diff.data(), ws_size, d_kws.data(), row_type, ws_size, device_cache ? d_slot_of.data() : nullptr,
                                  device_cache ? n_u : 0, device_cache ? d_cache_state.data() : nullptr, split ? d_gate.data() : nullptr,
-                                 nullptr));
+                                 tsvm::work_stream()));
         if (!caching) {
             for (int t = 0; t < ws_size; ++t) cur_slots[t] = t;
             upload_rotation(cur_slots);
         }
         solver.init_f(alpha, y, k_mat, d_f);
-        TSVM_HIP_CHECK(hipDeviceSynchronize());   // uploads, fills and init_f ran on the default stream
+        TSVM_HIP_CHECK(hipEventRecord(solved, tsvm::work_stream()));   // the rows, the uploads and init_f
+        TSVM_HIP_CHECK(hipStreamWaitEvent(sa, solved, 0));
+        if (ss != sa) TSVM_HIP_CHECK(hipStreamWaitEvent(ss, solved, 0));
 
         max_iter = std::max(100000, ws_size > INT_MAX / 100 ? INT_MAX : 100 * ws_size);
         timer.stream = sa;
@@ -517,6 +519,7 @@ struct SolveTask::Impl {
         for (int t = 0; t < ws_size; ++t) other[t] = slots_now[(t + q) % ws_size];
         d_slots_a.upload(slots_now.data(), ws_size);
         d_slots_b.upload(other.data(), ws_size);
+        TSVM_HIP_CHECK(hipStreamSynchronize(tsvm::work_stream()));   // (the readers are on another stream)
     }
 
     // Working-set selection of iteration `it`: the first one picks ws_size ids, later ones keep the last
@@ -894,9 +897,8 @@ void CSMOSolver::init_f(const std::vector<float_type> &alpha, const std::vector<
             }
             d_idx.upload(idx_vec.data(), m);
             d_ad.upload(alpha_diff_vec.data(), m);
-            k_mat.get_rows(d_idx.data(), m, d_rows.data(), ld);
-            abi_check(tsvm_update_f(d_f, d_ad.data(), m, d_rows.data(), k_mat.row_type(), nullptr, ld, n_u, k_mat.repeat(), nullptr));
-            TSVM_HIP_CHECK(hipStreamSynchronize(nullptr));
+            k_mat.get_rows(d_idx.data(), m, d_rows.data(), ld, nullptr, tsvm::work_stream());
+            abi_check(tsvm_update_f(d_f, d_ad.data(), m, d_rows.data(), k_mat.row_type(), nullptr, ld, n_u, k_mat.repeat(), tsvm::work_stream()));
             idx_vec.clear();
             alpha_diff_vec.clear();
         }
