@@ -1,0 +1,59 @@
+"""Whole solves of small problems in one kernel (csrc/smo_small.hip) against the CPU oracle, at the edges of its variants:
+256, 512 and 1,024 slots (a class takes its instances rounded up to four), one instance, the first size that goes the other way,
+repeated instances (ties decided by the working-set position), both element types, and several class pairs from one
+kernel matrix.  Same trajectory, hence the tolerances of the model tests."""
+import numpy as np
+import pytest
+
+from thundersvm_amd import data as D
+from thundersvm_amd.model import Model, make_param
+
+import test_gpu_models as T
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows(n, seed, ties):
+    rng = np.random.default_rng(seed)
+    x = rng.standard_normal((n, 6)).astype(np.float32)
+    if ties:
+        x[n // 2:] = x[:n - n // 2]
+        x = np.round(x)
+    return x, rng
+
+
+@pytest.mark.parametrize("ties", [False, True])
+@pytest.mark.parametrize("svm_type,kernel_type", [(0, 2), (0, 0), (1, 2)])
+@pytest.mark.parametrize("n_pos,n_neg", [(1, 1), (3, 5), (1, 252), (4, 252), (5, 249), (256, 256), (253, 257), (510, 511), (509, 512), (511, 513)])
+def test_two_classes(n_pos, n_neg, svm_type, kernel_type, ties):
+    n = n_pos + n_neg
+    x, rng = _rows(n, n, ties)
+    y = np.array([1.0] * n_pos + [0.0] * n_neg)
+    order = rng.permutation(n)
+    x[:, 0] += y - 0.5
+    d = D.from_dense(x[order], y[order])
+    nu = 0.5 * min(n_pos, n_neg) / n
+    T._compare(d, d, make_param(svm_type=svm_type, kernel_type=kernel_type, gamma=0.2, C=3.0, nu=nu, max_iter=40), trace=0)
+
+
+@pytest.mark.parametrize("ties", [False, True])
+@pytest.mark.parametrize("svm_type,kernel_type", [(2, 2), (3, 2), (3, 0), (4, 2)])
+@pytest.mark.parametrize("n", [1, 2, 63, 128, 129, 256, 257, 510, 512, 513])
+def test_one_class_and_regression(n, svm_type, kernel_type, ties):
+    x, rng = _rows(n, 1000 + n, ties)
+    d = D.from_dense(x, np.sin(x[:, 0]))
+    T._compare(d, d, make_param(svm_type=svm_type, kernel_type=kernel_type, gamma=0.2, C=3.0, nu=0.3, p=0.05, max_iter=40), trace=0)
+
+
+@pytest.mark.parametrize("sizes", [(5, 40, 90), (300, 200, 700, 900), (8, 8, 1100)])
+def test_class_pairs_from_one_matrix(sizes):
+    """Small pairs side by side, in the second and third case next to pairs that are too large; the same pairs one at a time."""
+    x, rng = _rows(sum(sizes), sum(sizes), False)
+    y = np.repeat(np.arange(len(sizes)), sizes).astype(np.float64)
+    x[:, 0] += y
+    order = rng.permutation(len(y))
+    d = D.from_dense(x[order], y[order])
+    T._compare(d, d, make_param(gamma=0.2, C=3.0), trace=0)
+    a = Model(0).train(d, make_param(gamma=0.2, C=3.0, kernel_type=0))
+    b = Model(0).train(d, make_param(gamma=0.2, C=3.0, kernel_type=0, pair_lanes=1, cache_bytes=0))   # (asks for the other path)
+    assert np.array_equal(a.coef, b.coef) and np.array_equal(a.rho, b.rho) and np.array_equal(a.sv_indices, b.sv_indices)

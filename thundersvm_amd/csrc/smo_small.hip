@@ -1,0 +1,690 @@
+// Whole SMO solves of small problems: CSMOSolver::solve / NuSMOSolver::solve (src/thundersvm/solver/csmosolver.cpp:10-121,
+// nusmosolver.cpp) with everything between the kernel matrix and the solution in one kernel, one workgroup per problem
+// and as many problems as there are in one launch (the class pairs of a one-vs-one run).
+//
+// Why.  A problem of a few hundred instances needs some ten outer iterations of some fifty steps.  As a chain of launches
+// (selection, rows, block, solver, update) an outer iteration took 150 us of which the solver's steps were 50, each
+// problem another 600 us of set-up, and one host thread fed all pairs.  Here an outer iteration's selection is a sort in LDS
+// of some microseconds, the kernel matrix is computed once for all pairs (it holds every pair's rows and columns), the host
+// takes no part between the upload and the result, and the pairs run side by side.  Whole
+// training calls: 45 pairs of 360 instances in 64 columns 31 -> 1.95 ms, 3 pairs of 100 in 4 columns 2.4 -> 0.70 ms.
+//
+// Shape.  At most 1,024 instances (above that a workgroup's share of update_f and of the selection outlasts what the
+// chip-wide kernels take, and their launches no longer matter): W wavefronts of four neighbouring instances per thread.
+// f, the local solver's f and the sets' membership live in registers, alpha in LDS.  The local solver runs on the
+// instances where they are, not on a gathered working set: an instance outside the working set is in neither I_up nor I_low, a row is
+// read from the kernel matrix in one piece, and ties go to the instance that comes first in the working set (its position
+// there is the upper half of the key that is compared among equals).
+#include "../../include/thundersvm_amd.h"
+#include "smo_local.h"
+#include "tsvm_internal.h"
+
+#define SS_MAX 1024            // instances of a problem (padded) at most
+#define SS_MAX_ITER 256        // outer iterations per launch: the host launches again what is not finished
+#define SS_MAX_INNER 300000    // and local steps per launch after which no outer iteration is begun
+
+__device__ __forceinline__ int wave_min_i32(int v) {
+    v = imin_sel(v, dpp_i32<TSVM_DPP_XOR1>(v));
+    v = imin_sel(v, dpp_i32<TSVM_DPP_XOR2>(v));
+    v = imin_sel(v, dpp_i32<TSVM_DPP_HALF_MIRROR>(v));
+    v = imin_sel(v, dpp_i32<TSVM_DPP_MIRROR>(v));
+    v = imin_sel(v, dpp_i32<TSVM_DPP_BCAST15, 0xa>(v));
+    v = imin_sel(v, dpp_i32<TSVM_DPP_BCAST31, 0xc>(v));
+    return __builtin_amdgcn_readlane(v, 63);
+}
+
+// As wave_first_argmin (smo_local.h), with a key per element in place of its position: among equal values the lowest
+// key wins.
+template <int E>
+__device__ __forceinline__ int wave_argmin_by_key(const double (&x)[E], const int (&key)[E], double &value, double &m, int &at) {
+    m = x[0];
+#pragma unroll
+    for (int e = 1; e < E; ++e) m = fmin_f64(m, x[e]);
+    at = 0x7fffffff;
+#pragma unroll
+    for (int e = 0; e < E; ++e) at = x[e] == m ? imin_sel(at, key[e]) : at;
+    value = wave_min_f64(m);
+    uint64_t who = __builtin_amdgcn_ballot_w64(m == value);
+    if (__popcll(who) != 1) {
+        const int k = wave_min_i32(m == value ? at : 0x7fffffff);
+        who &= __builtin_amdgcn_ballot_w64(at == k);
+    }
+    return __builtin_ctzll(who);
+}
+
+template <int W>
+__device__ __forceinline__ void block_argmin_by_key(const SvCand *slots, int lane, double &v, int &at, int &flags) {
+    static_assert(W == 2 || W == 4, "quad_perm steps");
+    const SvCand c = slots[lane & (W - 1)];
+    double m = fmin_f64(c.v, dpp_f64<TSVM_DPP_XOR1>(c.v));
+    if (W == 4) m = fmin_f64(m, dpp_f64<TSVM_DPP_XOR2>(m));
+    int k = c.v == m ? c.at : 0x7fffffff;
+    k = imin_sel(k, dpp_i32<TSVM_DPP_XOR1>(k));
+    if (W == 4) k = imin_sel(k, dpp_i32<TSVM_DPP_XOR2>(k));
+    v = m;
+    at = __builtin_amdgcn_readfirstlane(k);
+    flags = __builtin_amdgcn_ballot_w64(c.flag != 0) != 0;
+}
+
+__device__ __forceinline__ uint64_t ss_key(double f) {   // order-preserving; -0 and +0 compare equal in the reference's sort
+    if (f == 0.0) f = 0.0;
+    const uint64_t u = (uint64_t) __double_as_longlong(f);
+    return (u >> 63) ? ~u : (u | 0x8000000000000000ull);
+}
+
+template <int W>
+struct SmallShared {
+    static constexpr int N = 256 * W;
+    double kd[N];
+    double a[W][N];                     // alpha: one copy per wavefront (smo_solve.hip)
+    double f[N], k[N];                  // local solver: f and the row at the candidates; selection: sort keys and slots; update: coefficients and rows
+    unsigned short pos[N];              // position of a slot in the working set, 0xffff outside it
+    unsigned short ws[SS_MAX < N ? SS_MAX : N];
+    unsigned char flags[N];             // selection: the sides an instance is a candidate of
+    uint64_t total[2][W];               // per-wavefront counts of a scan
+    double red[4][W];
+    int event[2], first_x[2], first_y[2], n_list;
+    SvCand ci[W], cj[W], ci2[W], cj2[W];
+};
+
+// sort_f + select_working_set (smo_kernel.cpp:321-332, csmosolver.cpp:123-165, nusmosolver.cpp:48-118): writes k picks to
+// sh.ws[base ...]; false when there are fewer candidates.
+//
+// After the sort the alternating scan has a closed form.  Take one pair of sides, `up` reading the order from the low
+// end and `low` from the high end, one pick per round each (up first).  Nothing is skipped until the first event: a side
+// whose next candidate the other has already taken, or a side that is used up.  At that moment every instance that is
+// a candidate of both sides has been taken by one of them (the two ends have met), so from then on each side goes on with
+// the candidates that are its own alone.  The event is the minimum of a round number over the instances, and what remains are
+// prefix counts.
+template <int W, bool NU>
+__device__ bool ss_select(SmallShared<W> &sh, int k, int base) {
+    constexpr int N = 256 * W, T = 64 * W, NP = NU ? 2 : 1;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    uint64_t *skey = (uint64_t *) sh.f;
+    unsigned short *sidx = (unsigned short *) sh.k;
+    // bitonic sort of (key, slot), ascending; two pairs per thread and stage.  Strides below 128 stay inside a wavefront's
+    // 256 entries, which need no barrier with one another.
+    for (int size = 2; size <= N; size <<= 1) {
+        for (int strd = size >> 1; strd > 0; strd >>= 1) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int pr = wave * 128 + h * 64 + lane;   // a wavefront's pairs lie in its own 256 entries while strd < 256
+                const int lo = ((pr & ~(strd - 1)) << 1) | (pr & (strd - 1)), hi = lo | strd;
+                const uint64_t ka = skey[lo], kb = skey[hi];
+                const unsigned short ia = sidx[lo], ib = sidx[hi];
+                const bool asc = (lo & size) == 0, less_ba = kb < ka || (kb == ka && ib < ia);
+                if (asc == less_ba) { skey[lo] = kb; skey[hi] = ka; sidx[lo] = ib; sidx[hi] = ia; }
+            }
+            const int next = strd > 1 ? strd >> 1 : size;
+            if (strd > 128 || next > 128) __syncthreads();
+            else {
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+                __builtin_amdgcn_wave_barrier();
+            }
+        }
+    }
+    __syncthreads();
+    int slot[4];
+    unsigned fl[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        slot[j] = sidx[tid * 4 + j];
+        fl[j] = sh.flags[slot[j]];
+    }
+    // counts of up, low, up alone, low alone in 16-bit fields; inclusive scan over the sorted order
+    uint64_t incl[NP][4], total[NP];
+#pragma unroll
+    for (int q = 0; q < NP; ++q) {
+        uint64_t run = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const unsigned u = (fl[j] >> q) & 1u, l = (fl[j] >> (q + NP)) & 1u;
+            run += (uint64_t) u | (uint64_t) l << 16 | (uint64_t) (u & ~l & 1u) << 32 | (uint64_t) (l & ~u & 1u) << 48;
+            incl[q][j] = run;
+        }
+        uint64_t scan = run;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint64_t o = __shfl_up((unsigned long long) scan, d, 64);
+            if (lane >= d) scan += o;
+        }
+        if (lane == 63) sh.total[q][wave] = scan;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) incl[q][j] += scan - run;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NP; ++q) {
+        uint64_t before = 0;
+        total[q] = 0;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            const uint64_t t = sh.total[q][w];
+            if (w < wave) before += t;
+            total[q] += t;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) incl[q][j] += before;
+        if (tid == 0) {
+            const int n_up = (int) (total[q] & 0xffff), n_low = (int) (total[q] >> 16 & 0xffff);
+            const int dry_up = 2 * n_up, dry_low = 2 * n_low + 1;
+            sh.event[q] = dry_up < dry_low ? dry_up : dry_low;
+            sh.first_x[q] = (int) (total[q] >> 32 & 0xffff);
+            sh.first_y[q] = (int) (total[q] >> 48);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NP; ++q)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (!((fl[j] >> q) & (fl[j] >> (q + NP)) & 1u)) continue;
+            const int ru = (int) (incl[q][j] & 0xffff) - 1, rl = (int) (total[q] >> 16 & 0xffff) - (int) (incl[q][j] >> 16 & 0xffff);
+            atomicMin(&sh.event[q], ru <= rl ? 2 * rl + 1 : 2 * ru);   // the round in which the other side finds it taken
+        }
+    __syncthreads();
+    int a0[NP], b0[NP];
+#pragma unroll
+    for (int q = 0; q < NP; ++q) {
+        b0[q] = sh.event[q] >> 1;
+        a0[q] = b0[q] + (sh.event[q] & 1);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const unsigned u = (fl[j] >> q) & 1u, l = (fl[j] >> (q + NP)) & 1u;
+            const int ru = (int) (incl[q][j] & 0xffff) - 1, rl = (int) (total[q] >> 16 & 0xffff) - (int) (incl[q][j] >> 16 & 0xffff);
+            if (u && ru == a0[q]) sh.first_x[q] = (int) (incl[q][j] >> 32 & 0xffff) - (int) (u & ~l & 1u);
+            if (l && rl == b0[q]) sh.first_y[q] = (int) (total[q] >> 48) - (int) (incl[q][j] >> 48);
+        }
+    }
+    __syncthreads();
+    int len[2 * NP], sum = 0;
+#pragma unroll
+    for (int q = 0; q < NP; ++q) {
+        len[q] = a0[q] + (int) (total[q] >> 32 & 0xffff) - sh.first_x[q];
+        len[q + NP] = b0[q] + (int) (total[q] >> 48) - sh.first_y[q];
+        sum += len[q] + len[q + NP];
+    }
+    auto place = [&](int side, int nth, int s) {   // the nth pick of a side: one pick per side and round while the sides last
+        int at = 0;
+#pragma unroll
+        for (int o = 0; o < 2 * NP; ++o) at += (len[o] < nth ? len[o] : nth) + (o < side && len[o] > nth ? 1 : 0);
+        if (at < k) sh.ws[base + at] = (unsigned short) s;
+    };
+#pragma unroll
+    for (int q = 0; q < NP; ++q)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const unsigned u = (fl[j] >> q) & 1u, l = (fl[j] >> (q + NP)) & 1u;
+            const int ru = (int) (incl[q][j] & 0xffff) - 1, rl = (int) (total[q] >> 16 & 0xffff) - (int) (incl[q][j] >> 16 & 0xffff);
+            if (u) {
+                if (ru < a0[q]) place(q, ru, slot[j]);
+                else if (!l) place(q, a0[q] + (int) (incl[q][j] >> 32 & 0xffff) - 1 - sh.first_x[q], slot[j]);
+            }
+            if (l) {
+                if (rl < b0[q]) place(q + NP, rl, slot[j]);
+                else if (!u) place(q + NP, b0[q] + (int) (total[q] >> 48) - (int) (incl[q][j] >> 48) - sh.first_y[q], slot[j]);
+            }
+        }
+    __syncthreads();
+    return sum >= k;
+}
+
+// Slot s of a problem: its y > 0 instances first, then from a multiple of four on the others, so that a thread's four
+// slots have one label.  In the kernel matrix either group is a run of rows and (the same) columns.
+struct SmallMap {
+    int n0, n1, n0p, col0, col1, n_rows;
+    __device__ __forceinline__ int row(int s) const {
+        const int r = s < n0p ? col0 + s : col1 + (s - n0p);
+        return r < n_rows ? r : n_rows - 1;   // (an inactive slot's: in range, never used)
+    }
+    __device__ __forceinline__ bool active(int s) const { return s < n0p ? s < n0 : s - n0p < n1; }
+    __device__ __forceinline__ int index(int s) const { return s < n0p ? s : n0 + (s - n0p); }
+    __device__ __forceinline__ double label(int s) const { return s < n0p ? 1.0 : -1.0; }
+};
+
+template <typename TB>
+__device__ __forceinline__ void ss_load(const TB *row, TB (&out)[4]) {
+    typedef TB vec_t __attribute__((ext_vector_type(4), aligned(sizeof(TB))));   // (a class's columns start anywhere)
+    const vec_t v = *(const vec_t *) row;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[e] = v[e];
+}
+
+// The local solver: c_smo_iterate of smo_solve.hip (and nu_smo_solve_kernel) with the instances in place of a gathered
+// working set.  Returns the steps taken; the new alpha is in sh.a.
+template <int W, bool NU, typename TB>
+__device__ int ss_local(SmallShared<W> &sh, const SmallMap &map, const TB *K, int64_t ld, int col, const double (&kd)[4], double (&f)[4],
+                        unsigned member, const int (&key)[4], double Cp, double Cn, double local_eps, int max_iter) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const double half_Cp = 0.5 * Cp, half_Cn = NU ? half_Cp : 0.5 * Cn;
+    constexpr int NP = NU ? 2 : 1;   // pairs of sides
+    SvCand *const ci[2] = {sh.ci, sh.ci2}, *const cj[2] = {sh.cj, sh.cj2};
+    const bool none_possible = __builtin_amdgcn_readfirstlane(local_eps > 0.0 ? 0 : 1) != 0;
+    const int first_slot = sh.ws[0];
+    int n_iter = 0;
+    bool go_on;
+    do {
+        double up[NP], m[NP], v;
+        int at[NP], is[NP], go;
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+            double fu[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) fu[e] = keep_or_none<0>(member << (31 - 2 * NP * e - q), f[e]);
+            const int win = wave_argmin_by_key<4>(fu, key, up[q], m[q], at[q]);
+            if constexpr (W > 1) publish(ci[q] + wave, win, m[q], at[q], 0);
+            else is[q] = __builtin_amdgcn_readlane(at[q], win);
+        }
+        if constexpr (W > 1) {
+            lds_barrier();
+#pragma unroll
+            for (int q = 0; q < NP; ++q) block_argmin_by_key<W>(ci[q], lane, up[q], is[q], go);
+        }
+        TB kI[NP][4];
+        double kd_i[NP];
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+            is[q] &= 256 * W - 1;   // (with only NaN left there is no candidate at all)
+            if (NU) is[q] = is_none(up[q]) ? first_slot : is[q];   // (its row enters the other side's scores, smo_kernel.cpp:239)
+            ss_load<TB>(K + (int64_t) map.row(is[q]) * ld + col, kI[q]);
+            kd_i[q] = sh.kd[is[q]];
+        }
+        SV_PIN_MEMORY;
+        double part[4], b[NP][4], b_max = -__builtin_inf();
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            part[e] = kd_i[0] + kd[e];
+#pragma unroll
+            for (int q = 0; q < NP; ++q) {
+                b[q][e] = keep_or_none<1>(member << (31 - 2 * NP * e - NP - q), -up[q] + f[e]);
+                b_max = fmax_f64(b_max, b[q][e]);
+            }
+        }
+        go = __builtin_amdgcn_ballot_w64(!(b_max < local_eps)) != 0;
+        SV_PIN;
+        double best[NP];
+        int js[NP];
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+            double qs[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const double aIJ = __builtin_fma(-2.0, (double) kI[0][e], part[e]);
+                const double s = -b[q][e] * b[q][e] / aIJ;
+                qs[e] = __hiloint2double(b[q][e] > 0.0 ? __double2hiint(s) : SV_NONE_HI, __double2loint(s));
+            }
+            const int win = wave_argmin_by_key<4>(qs, key, best[q], v, at[q]);
+            publish_row<4, TB>(sh.f + tid * 4, sh.k + tid * 4, win, f, kI[q]);
+            if constexpr (W > 1) publish(cj[q] + wave, win, v, at[q], go);
+            else js[q] = __builtin_amdgcn_readlane(at[q], win);
+        }
+        if constexpr (W > 1) {
+            lds_barrier();
+#pragma unroll
+            for (int q = 0; q < NP; ++q) {
+                int g;
+                block_argmin_by_key<W>(cj[q], lane, best[q], js[q], g);
+                if (q == 0) go = g;
+            }
+        }
+        const bool second = NU && !__builtin_amdgcn_readfirstlane(best[0] < best[NP - 1] && best[0] < SV_NONE ? 1 : 0);
+        const int i = second ? is[NP - 1] : is[0];
+        int j2 = (second ? js[NP - 1] : js[0]) & (256 * W - 1);
+        const double up_value = second ? up[NP - 1] : up[0], kd_i2 = second ? kd_i[NP - 1] : kd_i[0];
+        // (two sides' winners may write different rows into one lane's slots when one of them has no candidate, so with
+        // two sides K[i, j2] is read from the matrix)
+        if (none_possible && is_none(second ? best[NP - 1] : best[0])) {
+            j2 = first_slot;
+            __syncthreads();
+            if (tid == first_slot / 4) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    sh.f[tid * 4 + e] = f[e];
+                    *(TB *) (sh.k + tid * 4 + e) = second ? kI[NP - 1][e] : kI[0][e];
+                }
+            }
+            __syncthreads();
+        }
+        TB kJ[4];
+        ss_load<TB>(K + (int64_t) map.row(j2) * ld + col, kJ);
+        const TB k_ij = NU ? K[(int64_t) map.row(i) * ld + map.row(j2)] : *(const TB *) (sh.k + j2);
+        SV_PIN_MEMORY;
+        const double kd_j = sh.kd[j2], a_j = sh.a[wave][j2], a_i = sh.a[wave][i], f_j = sh.f[j2], y_i = map.label(i), y_j = map.label(j2);
+        SV_PIN;
+        go_on = go && !(n_iter > max_iter);
+        const double q2 = (-up_value + f_j) / __builtin_fma(-2.0, (double) k_ij, kd_i2 + kd_j);
+        const double l = fmin_f64(room_up(a_i, y_i, half_Cp), fmin_f64(room_low(a_j, y_j, half_Cn), q2));
+        const double na_i = __builtin_fma(l, y_i, a_i), na_j = __builtin_fma(-l, y_j, j2 == i ? na_i : a_j);
+        auto bits = [&](double a, double y) {
+            const unsigned u = room_up(a, y, half_Cp) > 0 ? 1u : 0u, w = room_low(a, y, half_Cn) > 0 ? (1u << NP) : 0u;
+            return (u | w) << (NU && y < 0 ? 1 : 0);
+        };
+        member = set_member_bits<4, 2 * NP>(member, tid, i, bits(na_i, y_i));
+        member = set_member_bits<4, 2 * NP>(member, tid, j2, bits(na_j, y_j));
+        write_by_lane0(go_on, &sh.a[wave][i], na_i, &sh.a[wave][j2], na_j);
+        SV_PIN;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f[e] = __builtin_fma(-l, (double) kJ[e] - (double) (second ? kI[NP - 1][e] : kI[0][e]), f[e]);
+        n_iter += go_on;
+    } while (go_on);
+    return n_iter;
+}
+
+// f[j] -= sum over the n_list listed rows (coefficients sh.f, rows in sh.k) in order (smo_kernel.cpp:300-319)
+template <int W, typename TB>
+__device__ __forceinline__ void ss_update_f(const SmallShared<W> &sh, const TB *K, int64_t ld, int col, int first, int last, double (&f)[4]) {
+    const int *rows = (const int *) sh.k;
+    double sum[4] = {0.0, 0.0, 0.0, 0.0};
+    int t = first;
+    constexpr int U = 8;
+    for (; t + U <= last; t += U) {
+        TB k[U][4];
+#pragma unroll
+        for (int u = 0; u < U; ++u) ss_load<TB>(K + (int64_t) rows[t + u] * ld + col, k[u]);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum[e] = __builtin_fma(sh.f[t + u], (double) k[u][e], sum[e]);
+    }
+    for (; t < last; ++t) {
+        TB k[4];
+        ss_load<TB>(K + (int64_t) rows[t] * ld + col, k);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[e] = __builtin_fma(sh.f[t], (double) k[e], sum[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) f[e] -= sum[e];
+}
+
+template <int W, bool NU, typename TB>
+__global__ __launch_bounds__(64 * W) void smo_small_kernel(const TB *K, int64_t ld, int n_rows, const double *__restrict__ k_diag,
+                                                           const tsvm_small_problem *__restrict__ problems,
+                                                           tsvm_small_state *states, int *ws_all, double *alpha_all, double *f_all, double eps, int out_max_iter, int start) {
+    constexpr int N = 256 * W;
+    __shared__ SmallShared<W> sh;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const tsvm_small_problem P = problems[blockIdx.x];
+    tsvm_small_state *const S = states + blockIdx.x;
+    int *const ws_kept = ws_all + (int64_t) blockIdx.x * SS_MAX;
+    if (!start && S->status != 0) return;
+    SmallMap map;
+    map.n0 = P.n_pos;
+    map.n1 = P.n_neg;
+    map.n0p = (P.n_pos + 3) & ~3;   // (both fit: n0p + n_neg <= N is checked on the host)
+    map.col0 = P.row_pos;
+    map.col1 = P.row_neg;
+    map.n_rows = n_rows;
+    double *const alpha = alpha_all + P.at, *const f_out = f_all + P.at;
+    const int ws = P.ws, q = ws / 2;
+    double f[4], kd[4];
+    bool act[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int s = tid * 4 + e;
+        act[e] = map.active(s);
+        const double a = act[e] ? alpha[map.index(s)] : 0.0;
+        f[e] = act[e] ? f_out[map.index(s)] : 0.0;
+        kd[e] = act[e] ? k_diag[map.row(s)] : 1.0;
+        sh.kd[s] = kd[e];
+#pragma unroll
+        for (int w = 0; w < W; ++w) sh.a[w][s] = a;
+    }
+    const double y = map.label(tid * 4);   // (a thread's four slots are of one group)
+    // (a vector that starts at an active slot may end in the columns behind the group's, which nothing uses, or up to
+    // three elements behind the matrix)
+    const int col = act[0] ? map.row(tid * 4) : 0;
+    double previous_diff = __builtin_inf(), last_diff = __builtin_inf(), second_last_diff = __builtin_inf(), diff = 0.0;
+    int same_count = 0, swap_count = 0, iter = 0, status = 0;
+    long long local_iter = 0;
+    if (!start) {
+        previous_diff = S->previous_diff;
+        last_diff = S->last_diff;
+        second_last_diff = S->second_last_diff;
+        same_count = S->same_count;
+        swap_count = S->swap_count;
+        iter = S->iter;
+        local_iter = S->local_iter;
+        for (int t = tid; t < ws; t += 64 * W) sh.ws[t] = (unsigned short) ws_kept[t];
+    }
+    __syncthreads();
+    // the list of the instances with `coef` != 0 in slot order, or of the working set's in its order, for ss_update_f
+    auto make_list = [&](int count, auto coefficient, auto row_of) {   // entry t < count
+        int *rows = (int *) sh.k;
+        __syncthreads();
+        int filled = 0;
+        for (int t0 = 0; t0 < count; t0 += 64 * W) {
+            const int t = t0 + tid;
+            const double c = t < count ? coefficient(t) : 0.0;
+            const uint64_t b = __builtin_amdgcn_ballot_w64(c != 0.0);
+            if (lane == 0) sh.red[0][wave] = (double) __popcll(b);
+            __syncthreads();
+            int before = filled;
+            for (int w = 0; w < W; ++w) {
+                const int cnt = (int) sh.red[0][w];
+                if (w < wave) before += cnt;
+                filled += cnt;
+            }
+            if (c != 0.0) {
+                const int at = before + __popcll(b & ((1ull << lane) - 1ull));
+                sh.f[at] = c;
+                rows[at] = row_of(t);
+            }
+            __syncthreads();
+        }
+        return filled;
+    };
+    if (start) {   // f from a non-zero alpha, in batches of 101 rows (csmosolver.cpp:189-214)
+        const int n = make_list(N, [&](int s) { return map.active(s) ? -sh.a[wave][s] * map.label(s) : 0.0; }, [&](int s) { return map.row(s); });
+        for (int t = 0; t < n; t += 101) ss_update_f<W, TB>(sh, K, ld, col, t, t + 101 < n ? t + 101 : n, f);
+        __syncthreads();
+    }
+    const int iter_end = iter + SS_MAX_ITER;
+    long long inner_here = 0;
+    while (status == 0 && iter < iter_end && inner_here < SS_MAX_INNER) {
+        // the working set: its second half moves to the front, q new ones follow (csmosolver.cpp:63-77)
+        const int n_new = iter == 0 ? ws : q, first_new = iter == 0 ? 0 : ws - n_new;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sh.pos[tid * 4 + e] = 0xffff;
+        unsigned short kept[4];
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            const int t = h * 64 * W + tid;
+            kept[h] = iter > 0 && t < q ? sh.ws[t + q] : 0;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            const int t = h * 64 * W + tid;
+            if (iter > 0 && t < q) {
+                sh.ws[t] = kept[h];
+                sh.pos[kept[h]] = (unsigned short) t;
+            }
+        }
+        __syncthreads();
+        uint64_t *skey = (uint64_t *) sh.f;
+        unsigned short *sidx = (unsigned short *) sh.k;
+        unsigned member_all = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int s = tid * 4 + e;
+            const double a = sh.a[wave][s];
+            unsigned b = 0;
+            if (act[e]) {
+                const unsigned u = is_I_up(a, y, P.Cp, P.Cn) ? 1u : 0u, l = is_I_low(a, y, P.Cp, P.Cn) ? 1u : 0u;
+                b = NU ? (u | l << 2) << (y > 0 ? 0 : 1) : (u | l << 1);
+            }
+            member_all |= b << ((NU ? 4 : 2) * e);
+            sh.flags[s] = (unsigned char) (sh.pos[s] == 0xffff ? b : 0u);
+            skey[s] = act[e] ? ss_key(f[e]) : ~0ull;
+            sidx[s] = (unsigned short) s;
+        }
+        __syncthreads();
+        if (!ss_select<W, NU>(sh, n_new, first_new)) {
+            status = 2;
+            break;
+        }
+        for (int t = tid; t < ws; t += 64 * W) sh.pos[sh.ws[t]] = (unsigned short) t;
+        __syncthreads();
+        unsigned member = 0;
+        int key[4];
+        double fl[4], a_old[4], mn[2] = {__builtin_inf(), __builtin_inf()}, mx[2] = {-__builtin_inf(), -__builtin_inf()};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int s = tid * 4 + e, p = sh.pos[s];
+            const unsigned b = p != 0xffff ? (member_all >> ((NU ? 4 : 2) * e)) & (NU ? 15u : 3u) : 0u;
+            member |= b << ((NU ? 4 : 2) * e);
+            key[e] = (p << 10 | s) & 0x7fffffff;
+            fl[e] = f[e];
+            a_old[e] = sh.a[wave][s];
+#pragma unroll
+            for (int r = 0; r < (NU ? 2 : 1); ++r) {
+                mn[r] = fmin_f64(mn[r], (b >> r) & 1u ? f[e] : __builtin_inf());
+                mx[r] = fmax_f64(mx[r], (b >> (r + (NU ? 2 : 1))) & 1u ? f[e] : -__builtin_inf());
+            }
+        }
+        // the initial gap, and with it the local threshold (smo_kernel.cpp:61-66, 176-183)
+#pragma unroll
+        for (int r = 0; r < (NU ? 2 : 1); ++r) {
+            const double lo = wave_min_f64(mn[r]), hi = wave_max_f64(mx[r]);
+            if (lane == 0) { sh.red[2 * r][wave] = lo; sh.red[2 * r + 1][wave] = hi; }
+        }
+        __syncthreads();
+        double gap[2];
+#pragma unroll
+        for (int r = 0; r < (NU ? 2 : 1); ++r) {
+            double lo = sh.red[2 * r][0];
+#pragma unroll
+            for (int w = 1; w < W; ++w) lo = fmin_f64(lo, sh.red[2 * r][w]);
+            gap[r] = block_max<W>(sh.red[2 * r + 1]) - lo;
+        }
+        diff = NU ? (gap[0] > gap[1] ? gap[0] : gap[1]) : gap[0];
+        const double tenth = NU ? 0.1 * diff : 0.1f * diff;   // (a float literal in the C variant, a double in the nu one)
+        const double local_eps = eps > tenth ? eps : tenth;
+        __syncthreads();
+        const int steps = ss_local<W, NU, TB>(sh, map, K, ld, col, kd, fl, member, key, P.Cp, P.Cn, local_eps, P.max_iter);
+        inner_here += steps;
+        if (!NU) local_iter += steps;   // (the nu variant reports none, smo_kernel.cpp:283)
+        // alpha_diff of the working set, in its order: -(new - old) * y
+        __syncthreads();
+        double *const old = sh.k;   // (free between the local solver and the list)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) old[tid * 4 + e] = a_old[e];
+        __syncthreads();
+        double ad[4];
+        int rr[4], cnt = 0;
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {   // thread t owns entries 4t .. 4t + 3
+            const int t = tid * 4 + h;
+            const int s = t < ws ? sh.ws[t] : 0;
+            ad[h] = t < ws ? -(sh.a[wave][s] - old[s]) * map.label(s) : 0.0;
+            rr[h] = map.row(s);
+            cnt += ad[h] != 0.0;
+        }
+        int incl = cnt;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(incl, d, 64);
+            if (lane >= d) incl += o;
+        }
+        if (lane == 63) sh.red[0][wave] = (double) incl;
+        __syncthreads();
+        int at = incl - cnt, n_list = 0;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            const int c = (int) sh.red[0][w];
+            if (w < wave) at += c;
+            n_list += c;
+        }
+        int *const rows = (int *) sh.k;
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+            if (ad[h] != 0.0) {
+                sh.f[at] = ad[h];
+                rows[at] = rr[h];
+                ++at;
+            }
+        __syncthreads();
+        ss_update_f<W, TB>(sh, K, ld, col, 0, n_list, f);
+        __syncthreads();
+        // stall guards and stopping rule (csmosolver.cpp:86-111)
+        if (__builtin_fabs(diff - previous_diff) < eps * 0.001) {
+            same_count++;
+        } else {
+            same_count = 0;
+            previous_diff = diff;
+        }
+        if (__builtin_fabs(diff - second_last_diff) < eps * 0.001) swap_count++;
+        else swap_count = 0;
+        second_last_diff = last_diff;
+        last_diff = diff;
+        const bool stalled = (same_count >= 10 || swap_count >= 10) && __builtin_fabs(diff - 2.0) > eps;
+        if (stalled || diff < eps || (out_max_iter != -1 && iter == out_max_iter)) status = 1;
+        ++iter;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int s = tid * 4 + e;
+        if (act[e]) {
+            alpha[map.index(s)] = sh.a[wave][s];
+            f_out[map.index(s)] = f[e];
+        }
+    }
+    for (int t = tid; t < ws; t += 64 * W) ws_kept[t] = sh.ws[t];
+    if (tid == 0) {
+        S->previous_diff = previous_diff;
+        S->last_diff = last_diff;
+        S->second_last_diff = second_last_diff;
+        S->same_count = same_count;
+        S->swap_count = swap_count;
+        S->iter = iter;
+        S->local_iter = local_iter;
+        S->diff = diff;
+        S->status = status;
+        S->xcd = (int) __builtin_amdgcn_s_getreg(20 | (0 << 6) | (3 << 11));   // XCC_ID
+    }
+}
+
+template <int W, typename TB>
+static void launch_small(bool nu, const void *k, int64_t ld, int n_rows, const double *k_diag, const tsvm_small_problem *problems, int n_problems,
+                         tsvm_small_state *states, int *ws, double *alpha, double *f, double eps, int out_max_iter, int start,
+                         hipStream_t stream) {
+    if (nu)
+        smo_small_kernel<W, true, TB><<<n_problems, 64 * W, 0, stream>>>((const TB *) k, ld, n_rows, k_diag, problems, states, ws, alpha, f, eps,
+                                                                        out_max_iter, start);
+    else
+        smo_small_kernel<W, false, TB><<<n_problems, 64 * W, 0, stream>>>((const TB *) k, ld, n_rows, k_diag, problems, states, ws, alpha, f, eps,
+                                                                         out_max_iter, start);
+}
+
+extern "C" {
+
+int tsvm_smo_small_max(void) { return SS_MAX; }
+
+int tsvm_smo_solve_small(const void *k, int row_type, int64_t ld, int n_rows, const double *k_diag, const tsvm_small_problem *problems,
+                         int n_problems, int max_slots, tsvm_small_state *states, int *ws, double *alpha, double *f, int nu, double eps,
+                         int out_max_iter, int start, tsvm_stream stream) {
+    TSVM_REQUIRE(row_type == TSVM_ROW_F32 || row_type == TSVM_ROW_F64, "tsvm_smo_solve_small: row type %d", row_type);
+    TSVM_REQUIRE(n_problems >= 0 && n_rows >= 0 && ld >= n_rows, "tsvm_smo_solve_small: %d problems, %d rows, stride %lld", n_problems, n_rows,
+                 (long long) ld);
+    TSVM_REQUIRE(max_slots >= 1 && max_slots <= SS_MAX, "tsvm_smo_solve_small: %d slots (1 .. %d)", max_slots, SS_MAX);
+    if (n_problems == 0) return 0;
+    TSVM_REQUIRE(n_rows > 0 && k && k_diag && problems && states && ws && alpha && f, "tsvm_smo_solve_small: null argument");
+    hipStream_t st = tsvm_s(stream);
+#define TSVM_SMALL(W, TB) \
+    launch_small<W, TB>(nu != 0, k, ld, n_rows, k_diag, problems, n_problems, states, ws, alpha, f, eps, out_max_iter, start, st)
+    // (as few wavefronts as hold the largest problem at four instances per thread: their barriers are what a step pays for)
+    if (row_type == TSVM_ROW_F32) {
+        if (max_slots <= 256) TSVM_SMALL(1, float);
+        else if (max_slots <= 512) TSVM_SMALL(2, float);
+        else TSVM_SMALL(4, float);
+    } else {
+        if (max_slots <= 256) TSVM_SMALL(1, double);
+        else if (max_slots <= 512) TSVM_SMALL(2, double);
+        else TSVM_SMALL(4, double);
+    }
+#undef TSVM_SMALL
+    TSVM_LAUNCH_CHECK();
+    return 0;
+}
+
+}  // extern "C"

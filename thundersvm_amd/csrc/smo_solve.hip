@@ -29,6 +29,7 @@
 // the product by 2 is exact).
 #include "../../include/thundersvm_amd.h"
 #include "tsvm_device.h"
+#include "smo_local.h"
 #include "tsvm_internal.h"
 
 #include <algorithm>
@@ -123,172 +124,6 @@ __global__ void smo_start_kernel(double *alpha_diff, int n_diff, TB *kws, int ws
         for (int64_t i = gid; i < (int64_t) ws * ldk; i += stride) kws[i] = (TB) 0;
     if (state && gid < 2) state[gid] = 0;
     if (gate && gid < 4) gate[gid] = 0;
-}
-
-// What a masked-out element or score is replaced by: larger than any f or score of a problem in range.  Only the
-// high word is replaced (one instruction), so every value from SV_NONE on means "not a candidate".
-#define SV_NONE_HI 0x7fe00000
-#define SV_NONE 0x1p1023
-
-// x when the sign bit of `bit_at_top` is set, otherwise a value >= SV_NONE (SIGN = 0) or <= -SV_NONE (SIGN = 1).
-template <int SIGN>
-__device__ __forceinline__ double keep_or_none(unsigned bit_at_top, double x) {
-    const int m = (int) bit_at_top >> 31;
-    return __hiloint2double((m & __double2hiint(x)) | (~m & (int) (SV_NONE_HI | (SIGN ? 0x80000000u : 0u))), __double2loint(x));
-}
-
-// The scalar test for such a value.
-__device__ __forceinline__ bool is_none(double v) { return __builtin_amdgcn_readfirstlane(__double2hiint(v)) >= SV_NONE_HI; }
-
-// The smallest of a wavefront's E * 64 values (x[e] of a lane is element base + e) and the first element that has it:
-// `value` is the minimum; m and at are every lane's own smallest value and its first element; the lane returned is the
-// lowest one whose m is the minimum, so its `at` is the lowest element among equals.
-// With one wavefront per SIMD an instruction costs its four cycles whatever it does, a DPP operand has to be two wait
-// states old, and a value that crosses to the scalar unit and back costs about forty cycles, as much as a branch around
-// a few instructions (all measured on this part).  Hence one chain of six DPP steps on doubles with the instructions
-// that find the thread's own element in its gaps, and the winner by ballot instead of a second chain over the indices.
-#define SV_PIN __builtin_amdgcn_sched_barrier(0)
-// (the same for memory accesses: a row's load stays in front of the work that is to pass while it is on its way, and
-// in front of the exit test; the block is not declared restrict, or the load could be moved all the same)
-#define SV_PIN_MEMORY asm volatile("" ::: "memory")
-template <int E>
-__device__ __forceinline__ int wave_first_argmin(const double (&x)[E], int base, double &value, double &m, int &at) {
-    m = x[0];
-#pragma unroll
-    for (int e = 1; e < E; ++e) m = fmin_f64(m, x[e]);
-    SV_PIN;
-    uint64_t has[E];   // which lanes' element e is their minimum
-#pragma unroll
-    for (int e = 0; e < E - 1; ++e) asm volatile("v_cmp_eq_f64_e64 %0, %1, %2" : "=s"(has[e]) : "v"(x[e]), "v"(m));
-    SV_PIN;
-    int tl = dpp_i32<TSVM_DPP_XOR1>(__double2loint(m)), th = dpp_i32<TSVM_DPP_XOR1>(__double2hiint(m));
-    double r = fmin_f64(m, __hiloint2double(th, tl));
-    SV_PIN;
-    at = base + E - 1;
-#pragma unroll
-    for (int e = E - 2; e >= 0 && e >= E - 3; --e) asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(at) : "v"(at), "v"(base + e), "s"(has[e]));
-    SV_PIN;
-    tl = dpp_i32<TSVM_DPP_XOR2>(__double2loint(r));
-    th = dpp_i32<TSVM_DPP_XOR2>(__double2hiint(r));
-    r = fmin_f64(r, __hiloint2double(th, tl));
-    SV_PIN;
-#pragma unroll
-    for (int e = E - 4; e >= 0; --e) asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(at) : "v"(at), "v"(base + e), "s"(has[e]));
-    SV_PIN;
-    tl = dpp_i32<TSVM_DPP_HALF_MIRROR>(__double2loint(r));
-    th = dpp_i32<TSVM_DPP_HALF_MIRROR>(__double2hiint(r));
-    r = fmin_f64(r, __hiloint2double(th, tl));
-    tl = dpp_i32<TSVM_DPP_MIRROR>(__double2loint(r));
-    th = dpp_i32<TSVM_DPP_MIRROR>(__double2hiint(r));
-    r = fmin_f64(r, __hiloint2double(th, tl));
-    // (lanes outside the row mask keep what the step before moved there, which is no smaller than their own r)
-    tl = __builtin_amdgcn_update_dpp(tl, __double2loint(r), TSVM_DPP_BCAST15, 0xa, 0xf, false);
-    th = __builtin_amdgcn_update_dpp(th, __double2hiint(r), TSVM_DPP_BCAST15, 0xa, 0xf, false);
-    r = fmin_f64(r, __hiloint2double(th, tl));
-    tl = __builtin_amdgcn_update_dpp(tl, __double2loint(r), TSVM_DPP_BCAST31, 0xc, 0xf, false);
-    th = __builtin_amdgcn_update_dpp(th, __double2hiint(r), TSVM_DPP_BCAST31, 0xc, 0xf, false);
-    r = fmin_f64(r, __hiloint2double(th, tl));
-    value = readlane_f64(r, 63);
-    return __builtin_ctzll(__builtin_amdgcn_ballot_w64(m == value));
-}
-
-// The LDS address of a __shared__ object as the ds instructions take it.
-template <typename T>
-__device__ __forceinline__ unsigned lds_at(const T *p) {
-    return (unsigned) (uintptr_t) (const __attribute__((address_space(3))) T *) p;
-}
-
-// One wavefront's best candidate for the others: the workgroup's minimum is taken over W of these.
-struct __align__(16) SvCand {
-    double v;
-    int at;
-    int flag;
-};
-
-// Writes by one lane, without the branch that an if around them costs (all 64 lanes are active before and after).
-// Four wavefronts share the LDS, so a write or a broadcast read by 64 lanes is paid four times over: what one lane
-// knows is written by that lane alone.
-__device__ __forceinline__ void publish(SvCand *slot, int lane, double m, int at, int flag) {
-    typedef int v4i __attribute__((ext_vector_type(4)));
-    const v4i c = {__double2loint(m), __double2hiint(m), at, flag};
-    asm volatile("s_mov_b64 exec, %2\n\tds_write_b128 %0, %1\n\ts_mov_b64 exec, -1"
-                 :: "v"(lds_at(slot)), "v"(c), "s"(1ull << lane) : "memory");
-}
-// The same with the lane's E values of f and of the block row for the step (the row's values in slots of eight bytes).  (One asm statement each: nothing else may
-// come between the two writes of exec.)
-#define SV_EXEC_ON "s_mov_b64 exec, %0\n\t"
-#define SV_EXEC_OFF "s_mov_b64 exec, -1"
-template <int E, typename TB>
-__device__ __forceinline__ void publish_row(double *f_slot, double *k_slot, int lane, const double (&f)[E], const TB (&k)[E]) {
-    const unsigned fa = lds_at(f_slot), ka = lds_at(k_slot);
-    const uint64_t only = 1ull << lane;
-    static_assert(E == 1 || E == 2 || E == 4, "elements per thread");
-    if constexpr (E == 1 && sizeof(TB) == 4)
-        asm volatile(SV_EXEC_ON "ds_write_b64 %1, %3\n\tds_write_b32 %2, %4\n\t" SV_EXEC_OFF
-                     :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(k[0]) : "memory");
-    else if constexpr (E == 1)
-        asm volatile(SV_EXEC_ON "ds_write_b64 %1, %3\n\tds_write_b64 %2, %4\n\t" SV_EXEC_OFF
-                     :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(k[0]) : "memory");
-    else if constexpr (E == 2 && sizeof(TB) == 4)
-        asm volatile(SV_EXEC_ON "ds_write2_b64 %1, %3, %4 offset1:1\n\tds_write2_b32 %2, %5, %6 offset1:2\n\t" SV_EXEC_OFF
-                     :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(f[1]), "v"(k[0]), "v"(k[1]) : "memory");
-    else if constexpr (E == 2)
-        asm volatile(SV_EXEC_ON "ds_write2_b64 %1, %3, %4 offset1:1\n\tds_write2_b64 %2, %5, %6 offset1:1\n\t" SV_EXEC_OFF
-                     :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(f[1]), "v"(k[0]), "v"(k[1]) : "memory");
-    else if constexpr (sizeof(TB) == 4)
-        asm volatile(SV_EXEC_ON "ds_write2_b64 %1, %3, %4 offset1:1\n\tds_write2_b64 %1, %5, %6 offset0:2 offset1:3\n\t"
-                     "ds_write2_b32 %2, %7, %8 offset1:2\n\tds_write2_b32 %2, %9, %10 offset0:4 offset1:6\n\t" SV_EXEC_OFF
-                     :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "v"(k[0]), "v"(k[1]), "v"(k[2]), "v"(k[3]) : "memory");
-    else
-        asm volatile(SV_EXEC_ON "ds_write2_b64 %1, %3, %4 offset1:1\n\tds_write2_b64 %1, %5, %6 offset0:2 offset1:3\n\t"
-                     "ds_write2_b64 %2, %7, %8 offset1:1\n\tds_write2_b64 %2, %9, %10 offset0:2 offset1:3\n\t" SV_EXEC_OFF
-                     :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "v"(k[0]), "v"(k[1]), "v"(k[2]), "v"(k[3]) : "memory");
-}
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-// (p, then q: if both name one element the second value is the final one; `on` = 0: nothing is written)
-__device__ __forceinline__ void write_by_lane0(int on, double *p, double v, double *q, double w) {
-    asm volatile(SV_EXEC_ON "ds_write_b64 %1, %2\n\tds_write_b64 %3, %4\n\t" SV_EXEC_OFF
-                 :: "s"((uint64_t) (uint32_t) __builtin_amdgcn_readfirstlane(on)), "v"(lds_at(p)), "v"(v), "v"(lds_at(q)), "v"(w) : "memory");
-}
-
-// The workgroup's best candidate: every lane reads one of the W, two DPP steps compare them.  The elements of a
-// wavefront are neighbours and the wavefronts follow one another: among equal values the first wavefront has the
-// lowest element.  `at` and `flags` come back as scalars.
-template <int W>
-__device__ __forceinline__ void block_argmin(const SvCand *slots, int lane, double &v, int &at, int &flags) {
-    static_assert(W == 2 || W == 4, "quad_perm steps");
-    const SvCand c = slots[lane & (W - 1)];
-    double m = fmin_f64(c.v, dpp_f64<TSVM_DPP_XOR1>(c.v));
-    if (W == 4) m = fmin_f64(m, dpp_f64<TSVM_DPP_XOR2>(m));
-    v = m;
-    at = __builtin_amdgcn_readlane(c.at, __builtin_ctzll(__builtin_amdgcn_ballot_w64(c.v == m)));
-    flags = __builtin_amdgcn_ballot_w64(c.flag != 0) != 0;
-}
-template <int W>
-__device__ __forceinline__ double block_max(const double *s_v) {
-    double v = s_v[0];
-#pragma unroll
-    for (int w = 1; w < W; ++w) v = fmax_f64(v, s_v[w]);
-    return v;
-}
-
-// Replaces the WIDTH membership bits of element t (the same in all threads) in the bit field of the thread that owns it.
-template <int E, int WIDTH>
-__device__ __forceinline__ unsigned set_member_bits(unsigned m, int tid, int t, unsigned bits) {
-    const int sh = (t & (E - 1)) * WIDTH;
-    const unsigned field = ((1u << WIDTH) - 1u) << sh;
-    const unsigned changed = (m & ~field) | (bits << sh);
-    return tid == (int) ((unsigned) t / E) ? changed : m;
-}
-
-// How far alpha can move along its label y = +-1 (y > 0 ? Cp - a : a; the element is in I_up while this is positive)
-// and against it (y > 0 ? a : Cn - a; in I_low while positive), smo_kernel.h:13-23 and smo_kernel.cpp:94-99: one fma
-// each on the half bounds, which rounds exactly as the selected subtraction does.
-__device__ __forceinline__ double room_up(double a, double y, double half_Cp) {
-    return __builtin_fma(-y, a, __builtin_fma(y, half_Cp, half_Cp));
-}
-__device__ __forceinline__ double room_low(double a, double y, double half_Cn) {
-    return __builtin_fma(y, a, __builtin_fma(-y, half_Cn, half_Cn));
 }
 
 // Reads the block on one XCD, so that the rows a solver on that XCD asks for are in its L2 (written by kernels on all

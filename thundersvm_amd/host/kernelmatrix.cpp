@@ -631,11 +631,14 @@ size_t KernelMatrix::reference_syncmem_bytes() const {
     return bytes;
 }
 
-size_t KernelMatrix::reference_syncmem_bytes_at_most() const {
+size_t KernelMatrix::reference_syncmem_bytes_at_most(size_t m, size_t n_features, size_t entries) {
     // every stored entry counted twice (in the CSR arrays and in the sparse part), every column in the dense part
-    // (a gathered subset's entry count is an estimate: every cell then)
-    const size_t m = n_instances(), cells = m * n_features(), entries = rows_->dense ? cells : rows_->nnz * repeat_;
-    return 2 * entries * (sizeof(kernel_type) + sizeof(int)) + 2 * (m + 1) * sizeof(int) + 2 * m * sizeof(kernel_type) + cells * sizeof(kernel_type);
+    return 2 * entries * (sizeof(kernel_type) + sizeof(int)) + 2 * (m + 1) * sizeof(int) + 2 * m * sizeof(kernel_type) +
+           m * n_features * sizeof(kernel_type);
+}
+
+size_t KernelMatrix::entries_at_most() const {   // (a gathered dense subset's entry count is an estimate: every cell then)
+    return rows_->dense ? n_instances() * n_features() : rows_->nnz * repeat_;
 }
 
 // A staging buffer that is all-zero whenever it is not in use: grown (and cleared) only when a call needs more.

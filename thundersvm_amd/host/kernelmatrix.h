@@ -114,7 +114,9 @@ public:
     // what SvmModel::get_working_set_size subtracts from the memory budget (svmmodel.cpp:437-451).  An entry
     // stored with the value 0 counts as absent in the dense layout and as a non-zero entry in the CSR layout.
     size_t reference_syncmem_bytes() const;
-    size_t reference_syncmem_bytes_at_most() const;   // no less than that, from the shape alone
+    // no less than that, from the shape alone
+    static size_t reference_syncmem_bytes_at_most(size_t n_instances, size_t n_features, size_t entries);
+    size_t entries_at_most() const;   // stored entries, or more
 
 private:
     void finish(int repeat);

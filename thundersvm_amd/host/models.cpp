@@ -58,6 +58,19 @@ void SvmModel::model_setup(const DataSet &, SvmParam &p) {   // svmmodel.cpp:22-
 
 static int max2power(double n) { return (int) pow(2, floor(log2f(float(n)))); }   // util/common.h:20-23
 
+static int size_for_memory(size_t free_mem, size_t n_instances, size_t n_features) {
+    const size_t by_mem = (size_t) max2power((double) (free_mem / sizeof(kernel_type) / (n_instances + n_features)));
+    return std::min(max2power((double) n_instances), (int) std::min(by_mem, (size_t) 1024));
+}
+
+int SvmModel::working_set_size_of_shape(size_t n_instances, size_t n_features, size_t entries, size_t held_bytes) const {
+    if (ws_override > 0) return (size_t) ws_override <= n_instances ? ws_override : 0;
+    const size_t used = KernelMatrix::reference_syncmem_bytes_at_most(n_instances, n_features, entries) +
+                        n_instances * (sizeof(int) + 2 * sizeof(float_type)) + held_bytes;
+    const int ws = param.max_mem_size > used ? size_for_memory(param.max_mem_size - used, n_instances, n_features) : 0;
+    return ws < std::min(max2power((double) n_instances), 1024) ? 0 : ws;
+}
+
 // svmmodel.cpp:437-451.  The reference subtracts the bytes its SyncMem counter holds at this point of
 // train_binary (svc.cpp:147-166; svr.cpp:9-35 and the other models alike): its KernelMatrix of the problem, the
 // problem's y (int), alpha and f (float_type), and `held_bytes`, what the model has kept from earlier problems
@@ -75,19 +88,13 @@ int SvmModel::get_working_set_size(const KernelMatrix &k_mat, size_t held_bytes)
         return ws_override;
     }
     const size_t others = n_instances * (sizeof(int) + 2 * sizeof(float_type)) + held_bytes;
-    const auto size_for = [&](size_t used) {
-        const size_t free_mem = param.max_mem_size - used;
-        const size_t by_mem = (size_t) max2power((double) (free_mem / sizeof(kernel_type) / (n_instances + n_features)));
-        return std::min(max2power((double) n_instances), (int) std::min(by_mem, (size_t) 1024));
-    };
     // (counting the reference's column split takes a pass over the columns; where even the most that it can come to
     // leaves room for the largest working set, the count changes nothing)
-    const size_t at_most = k_mat.reference_syncmem_bytes_at_most() + others;
-    int ws = param.max_mem_size > at_most ? size_for(at_most) : 0;
-    if (ws < std::min(max2power((double) n_instances), 1024)) {
+    int ws = working_set_size_of_shape(n_instances, n_features, k_mat.entries_at_most(), held_bytes);
+    if (ws == 0) {
         const size_t used = k_mat.reference_syncmem_bytes() + others;
         if (param.max_mem_size < used) throw std::bad_alloc();
-        ws = size_for(used);
+        ws = size_for_memory(param.max_mem_size - used, n_instances, n_features);
     }
     TSVM_LOG << "working set size = " << ws;
     return ws;
@@ -100,6 +107,18 @@ void SvmModel::run_solver(CSMOSolver &solver, const KernelMatrix &k_mat, const s
                           std::vector<float_type> &alpha, float_type &rho_out, std::vector<float_type> &f_val,
                           float_type Cp, float_type Cn, size_t held_bytes) {
     const int ws = get_working_set_size(k_mat, held_bytes);
+    const size_t n_pos = std::find(y.begin(), y.end(), -1) - y.begin();
+    if (small_path_allowed() && SmallSolve::takes(n_pos, y.size() - n_pos, ws) &&
+        SmallSolve::takes_rows(k_mat.n_columns(), k_mat.row_elem_size())) {
+        std::vector<SmallSolve> one(1);
+        one[0] = {&solver, 0, (int) n_pos, k_mat.repeat() > 1 ? 0 : (int) n_pos, (int) (y.size() - n_pos), ws, Cp, Cn, &y, &alpha, &f_val, &rho_out};
+        SmallSolve::run(k_mat, one, param.epsilon, max_iter);
+        if (one[0].solved) {
+            solver_stats.push_back(one[0].stats);
+            if (keep_binary) binary_f.push_back(f_val);
+            return;
+        }
+    }
     solver.profile = profile;
     solver.cache_bytes = cache_bytes;
     solver.trace = solver_stats.empty() ? trace_first : nullptr;
@@ -385,7 +404,9 @@ void SVC::train(const DataSet &dataset, SvmParam p) {   // svc.cpp:41-145
     // (train_pairs_in_lockstep), three when the pairs alternate between a solver phase and a chip-wide phase
     const int lanes = std::min(pair_lanes > 0 ? pair_lanes : SolveTask::cu_split_available() ? 8 : 3, n_binary_models);
     if (lanes > 1 && !profile && !trace_first) {
-        train_pairs_in_lockstep(grouped, lanes, alpha);
+        solver_stats.assign(n_binary_models, SolverStats());
+        if (keep_binary) binary_f.assign(n_binary_models, std::vector<float_type>());
+        train_pairs_in_lockstep(grouped, lanes, alpha, train_small_pairs(grouped, alpha));
     } else {
         size_t held = 0;   // alpha arrays of the pairs already trained (svc.cpp:50-61 keeps them to the end)
         for (int i = 0; i < n_classes; ++i)
@@ -393,6 +414,7 @@ void SVC::train(const DataSet &dataset, SvmParam p) {   // svc.cpp:41-145
                 BinaryProblem p;
                 p.k = k;
                 setup_binary(grouped, i, j, p);
+                take_rows(grouped, p);
                 run_solver(*p.solver, *p.k_mat, p.y, p.alpha, rho[k], p.f_val, p.Cp, p.Cn, held);
                 held += p.y.size() * sizeof(float_type);
                 finish_binary(p, alpha[k]);
@@ -460,8 +482,7 @@ void SVC::train(const DataSet &dataset, SvmParam p) {   // svc.cpp:41-145
 }
 
 void SVC::setup_binary(const DataSet &dataset, int i, int j, BinaryProblem &p) {   // svc.cpp:147-170
-    const std::vector<int> ids = dataset.original_index(i, j);
-    const int ci = dataset.count()[i], n = (int) ids.size();
+    const int ci = dataset.count()[i], n = ci + dataset.count()[j];
     p.i = i;
     p.j = j;
     p.y.resize(n);
@@ -471,10 +492,14 @@ void SVC::setup_binary(const DataSet &dataset, int i, int j, BinaryProblem &p) {
         p.y[l] = l < ci ? +1 : -1;
         p.f_val[l] = l < ci ? -1 : +1;
     }
-    p.k_mat.reset(new KernelMatrix(dataset, ids.data(), ids.size(), param));
     p.solver.reset(new CSMOSolver());
     p.Cp = param.C * c_weight[i];
     p.Cn = param.C * c_weight[j];
+}
+
+void SVC::take_rows(const DataSet &dataset, BinaryProblem &p) {
+    const std::vector<int> ids = dataset.original_index(p.i, p.j);
+    p.k_mat.reset(new KernelMatrix(dataset, ids.data(), ids.size(), param));
 }
 
 void SVC::finish_binary(BinaryProblem &p, std::vector<float_type> &alpha_out) {   // svc.cpp:171-177
@@ -485,6 +510,53 @@ void SVC::finish_binary(BinaryProblem &p, std::vector<float_type> &alpha_out) { 
     }
     TSVM_LOG << "rho = " << rho[p.k] << ", #sv = " << count;
     alpha_out = std::move(p.alpha);
+}
+
+// Pairs that fit one workgroup each (smo_small.hip) are solved side by side from one kernel matrix of their classes' rows.
+std::vector<char> SVC::train_small_pairs(const DataSet &grouped, std::vector<std::vector<float_type>> &alpha) {
+    std::vector<char> done(n_binary_models, 0);
+    if (!small_path_allowed() || pair_lanes > 0) return done;
+    struct Pair { int i, j, k, ws; };
+    std::vector<Pair> small;
+    std::vector<char> needed(n_classes, 0);
+    size_t held = 0;   // (as in train())
+    for (int i = 0, k = 0; i < n_classes; ++i)
+        for (int j = i + 1; j < n_classes; ++j, ++k) {
+            const size_t ci = grouped.count()[i], cj = grouped.count()[j];
+            const int ws = working_set_size_of_shape(ci + cj, grouped.n_features() + 1, std::min(grouped.rows().nnz(), (ci + cj) * (grouped.n_features() + 1)), held);
+            held += (ci + cj) * sizeof(float_type);
+            if (!SmallSolve::takes(ci, cj, ws)) continue;
+            small.push_back({i, j, k, ws});
+            needed[i] = needed[j] = 1;
+        }
+    std::vector<int> first_row(n_classes, 0), ids;
+    for (int c = 0; c < n_classes; ++c) {
+        if (!needed[c]) continue;
+        first_row[c] = (int) ids.size();
+        const std::vector<int> of_class = grouped.original_index(c);
+        ids.insert(ids.end(), of_class.begin(), of_class.end());
+    }
+    if (small.empty() || !SmallSolve::takes_rows(ids.size(), param.kernel_type == SvmParam::LINEAR ? sizeof(double) : sizeof(float))) return done;
+    const KernelMatrix k_mat(grouped, ids.data(), ids.size(), param);
+    std::vector<BinaryProblem> problems(small.size());
+    std::vector<SmallSolve> solves(small.size());
+    for (size_t s = 0; s < small.size(); ++s) {
+        const Pair &q = small[s];
+        BinaryProblem &p = problems[s];
+        p.k = q.k;
+        setup_binary(grouped, q.i, q.j, p);
+        solves[s] = {p.solver.get(), first_row[q.i], grouped.count()[q.i], first_row[q.j], grouped.count()[q.j], q.ws, p.Cp, p.Cn, &p.y, &p.alpha, &p.f_val, &rho[q.k]};
+    }
+    SmallSolve::run(k_mat, solves, param.epsilon, max_iter);
+    for (size_t s = 0; s < small.size(); ++s) {
+        if (!solves[s].solved) continue;
+        const int k = small[s].k;
+        done[k] = 1;
+        solver_stats[k] = solves[s].stats;
+        if (keep_binary) binary_f[k] = problems[s].f_val;
+        finish_binary(problems[s], alpha[k]);
+    }
+    return done;
 }
 
 // The class pairs are independent problems.  Up to `lanes` of them are in flight, each a SolveTask with its own
@@ -505,23 +577,24 @@ void SVC::finish_binary(BinaryProblem &p, std::vector<float_type> &alpha_out) { 
 // eight lanes: 1.87 s; with equal slices in the reference's order 1.93 s; with three large lanes and five small
 // ones 2.35 s: the large pairs are what the time goes into, and they advance at a rate that hardly depends on
 // how many of them share the chip, so long as there are at least five.)
-void SVC::train_pairs_in_lockstep(const DataSet &grouped, int lanes, std::vector<std::vector<float_type>> &alpha) {
+void SVC::train_pairs_in_lockstep(const DataSet &grouped, int lanes, std::vector<std::vector<float_type>> &alpha, const std::vector<char> &done) {
     struct PairId { int i, j; };
     std::vector<PairId> pairs;
     for (int i = 0; i < n_classes; ++i)
         for (int j = i + 1; j < n_classes; ++j) pairs.push_back({i, j});
+    if (std::all_of(done.begin(), done.end(), [](char d) { return d != 0; })) return;
     const size_t esz = param.kernel_type == SvmParam::LINEAR ? sizeof(double) : sizeof(float);
     tsvm::RowArena &arena = tsvm::RowArena::instance();
     const size_t budget = cache_bytes > 0 ? (size_t) cache_bytes : cache_bytes < 0 ? arena.auto_budget() : 0;
     // per pair: bytes of its working-set rows (the least a slice must hold) and of its whole kernel matrix
     std::vector<size_t> ws_bytes(pairs.size()), full_bytes(pairs.size());
-    std::vector<int> by_size(pairs.size());
+    std::vector<int> by_size;   // the pairs that are left to solve
     for (size_t k = 0; k < pairs.size(); ++k) {
         const size_t cols = (size_t) grouped.count()[pairs[k].i] + grouped.count()[pairs[k].j];
         const size_t ld = (cols + 7) / 8 * 8;
         ws_bytes[k] = (size_t) 1024 * ld * esz;
         full_bytes[k] = std::max(cols * ld * esz, ws_bytes[k]);
-        by_size[k] = (int) k;
+        if (!done[k]) by_size.push_back((int) k);
     }
     std::stable_sort(by_size.begin(), by_size.end(), [&](int a, int b) { return full_bytes[a] > full_bytes[b]; });
     const bool two_kinds = SolveTask::cu_split_available();   // (the lockstep schedule keeps equal lanes and the reference's order)
@@ -538,8 +611,8 @@ void SVC::train_pairs_in_lockstep(const DataSet &grouped, int lanes, std::vector
     }
     int n_large_lanes, n_small_lanes;
     if (!two_kinds) {
-        large_q.assign(by_size.size(), 0);
-        for (size_t k = 0; k < pairs.size(); ++k) large_q[k] = (int) k;
+        large_q.assign(by_size.begin(), by_size.end());
+        std::sort(large_q.begin(), large_q.end());
         n_large_lanes = lanes;
         n_small_lanes = 0;
     } else if (small_q.empty()) {
@@ -570,8 +643,6 @@ void SVC::train_pairs_in_lockstep(const DataSet &grouped, int lanes, std::vector
     for (size_t k = 0; k < pairs.size(); ++k)
         alpha_bytes_before[k + 1] = alpha_bytes_before[k] +
                                     ((size_t) grouped.count()[pairs[k].i] + grouped.count()[pairs[k].j]) * sizeof(float_type);
-    solver_stats.assign(pairs.size(), SolverStats());
-    if (keep_binary) binary_f.assign(pairs.size(), std::vector<float_type>());
     std::vector<std::unique_ptr<BinaryProblem>> active;
     std::vector<int> free_lanes;
     for (int l = 0; l < lanes; ++l) free_lanes.push_back(l);
@@ -588,6 +659,7 @@ void SVC::train_pairs_in_lockstep(const DataSet &grouped, int lanes, std::vector
         std::unique_ptr<BinaryProblem> p(new BinaryProblem());
         p->k = k;
         setup_binary(grouped, pairs[k].i, pairs[k].j, *p);
+        take_rows(grouped, *p);
         p->lane = lane;
         const int ws = get_working_set_size(*p->k_mat, alpha_bytes_before[p->k]);
         p->solver->cache_bytes = cache_bytes;
@@ -922,8 +994,7 @@ void NuSVC::model_setup(const DataSet &dataset, SvmParam &p) {
 }
 
 void NuSVC::setup_binary(const DataSet &dataset, int i, int j, BinaryProblem &p) {   // nusvc.cpp:17-50
-    const std::vector<int> ids = dataset.original_index(i, j);
-    const int n_pos = dataset.count()[i], n = (int) ids.size();
+    const int n_pos = dataset.count()[i], n = n_pos + dataset.count()[j];
     p.i = i;
     p.j = j;
     p.y.resize(n);
@@ -937,7 +1008,6 @@ void NuSVC::setup_binary(const DataSet &dataset, int i, int j, BinaryProblem &p)
         p.alpha[l] = std::min(1., budget);
         budget -= p.alpha[l];
     }
-    p.k_mat.reset(new KernelMatrix(dataset, ids.data(), ids.size(), param));
     p.solver.reset(new NuSMOSolver(false));
     p.Cp = 1;
     p.Cn = 1;

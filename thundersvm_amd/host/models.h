@@ -71,6 +71,10 @@ protected:
     bool predict_batch_fused(const PredictPlan &plan, const kernel_type *a, int64_t lda, const kernel_type *sd_a, size_t m,
                              bool indicator_values, float_type *dec_out) const;
     void copy_support_vectors(const RowStore &rows);
+    // whether problems may take the path for small ones: the caller has asked for nothing that only the other path does
+    bool small_path_allowed() const { return !profile && !(trace_first && solver_stats.empty()) && cache_bytes < 0; }
+    // the working-set size where it can be told from the problem's shape alone, 0 otherwise
+    int working_set_size_of_shape(size_t n_instances, size_t n_features, size_t entries, size_t held_bytes) const;
     void run_solver(CSMOSolver &solver, const KernelMatrix &k_mat, const std::vector<int> &y, std::vector<float_type> &alpha,
                     float_type &rho, std::vector<float_type> &f_val, float_type Cp, float_type Cn, size_t held_bytes = 0);
     void compute_linear_coef_single_model(size_t n_feature, bool zero_based);
@@ -118,9 +122,12 @@ protected:
         int lane = 0;
         bool rows_pending = false;   // independent lanes: the iteration's rows and update_f are still to be enqueued
     };
-    virtual void setup_binary(const DataSet &dataset, int i, int j, BinaryProblem &p);   // svc.cpp:147-170
+    virtual void setup_binary(const DataSet &dataset, int i, int j, BinaryProblem &p);   // svc.cpp:147-170 (without the rows)
+    void take_rows(const DataSet &dataset, BinaryProblem &p);
+    // solves the small pairs side by side; which ones were (each then has its stats, alpha and rho)
+    std::vector<char> train_small_pairs(const DataSet &grouped, std::vector<std::vector<float_type>> &alpha);
     void finish_binary(BinaryProblem &p, std::vector<float_type> &alpha_out);            // svc.cpp:171-177
-    void train_pairs_in_lockstep(const DataSet &grouped, int lanes, std::vector<std::vector<float_type>> &alpha);
+    void train_pairs_in_lockstep(const DataSet &grouped, int lanes, std::vector<std::vector<float_type>> &alpha, const std::vector<char> &done);
     std::vector<float_type> predict_label(const std::vector<float_type> &dec_values, int n_instances);
     void probability_train(const DataSet &grouped);                                            // svc.cpp:432-491
     void multiclass_probability(const std::vector<std::vector<float_type>> &r, std::vector<float_type> &p) const;   // svc.cpp:206-263

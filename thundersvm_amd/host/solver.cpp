@@ -138,6 +138,10 @@ void wait_while_pending(const volatile uint64_t *word, uint64_t pending, long lo
 
 }  // namespace tsvm
 
+double ms_since_first_solve() {
+    return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - process_epoch()).count();
+}
+
 struct SolveTask::Impl {
     const CSMOSolver &solver;
     const KernelMatrix &k_mat;

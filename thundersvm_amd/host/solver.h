@@ -58,6 +58,7 @@ public:
 
 protected:
     friend class SolveTask;
+    friend struct SmallSolve;
     virtual bool is_nu() const { return false; }
     virtual float_type calculate_rho(const std::vector<float_type> &f_val, const std::vector<int> &y,
                                      std::vector<float_type> &alpha, float_type Cp, float_type Cn) const;
@@ -124,3 +125,22 @@ private:
     struct Impl;
     Impl *impl_;
 };
+
+// One of several small problems that are solved by one kernel launch from one kernel matrix (smo_small.hip): its y = +1
+// instances are n_pos rows of the matrix from row_pos on, its y = -1 instances n_neg rows from row_neg on.
+struct SmallSolve {
+    const CSMOSolver *solver;   // (all problems of a run: the same kind)
+    int row_pos, n_pos, row_neg, n_neg, ws_size;
+    float_type Cp, Cn;
+    const std::vector<int> *y;
+    std::vector<float_type> *alpha, *f_val;
+    float_type *rho;
+    bool solved = false;        // false after run(): alpha and f_val are untouched, the problem is for a SolveTask
+    SolverStats stats;
+
+    static size_t slots(size_t n_pos, size_t n_neg);
+    static bool takes(size_t n_pos, size_t n_neg, int ws_size);
+    static bool takes_rows(size_t n_rows, size_t elem_size);
+    static void run(const KernelMatrix &k_mat, std::vector<SmallSolve> &problems, float_type eps, int out_max_iter);
+};
+double ms_since_first_solve();   // the clock that SolverStats::ms_start and ms_end are read on
