@@ -290,19 +290,21 @@ int tsvm_smo_start(double *alpha_diff, int n_diff, void *kws, int block_type, in
  * above 512 with doubles) are left alone.  sink: one int of device memory, never written in practice. */
 int tsvm_smo_warm_block(const void *kws, int block_type, int ws_size, int xcd, int *sink, tsvm_stream stream);
 
-/* Whole solves of small problems (csmosolver.cpp:10-121, nusmosolver.cpp), one workgroup each: k is the kernel matrix of
- * n_rows rows (element r*ld + c; three more elements behind the last one are read, not used), k_diag its diagonal.  Problem p has
- * the n_pos rows (and columns) from row_pos on with y = +1 and the n_neg from row_neg on with y = -1; its alpha and f
- * are the n_pos + n_neg entries from `at` on.  max_slots: the most that n_pos rounded up to four plus n_neg comes to
- * (1 .. tsvm_smo_small_max()).  ws: 2 .. n_pos + n_neg, even.  start != 0: a first call (alpha and f hold the start values, f
- * without the terms of a non-zero alpha); 0: goes on with the problems whose state says 0.
- * states[p].status: 0 more to do (a call ends after a bounded number of steps), 1 solved, 2 given up because a working
- * set could not be filled (alpha and f are no longer the start values).  ws_store: n_problems * tsvm_smo_small_max() ints, kept between
- * the calls.  nu: the Cp of each problem is its C. */
+/* Whole solves of small problems (csmosolver.cpp:10-121, nusmosolver.cpp), one workgroup each.  Of problem p, k is the
+ * kernel matrix of n_rows rows (elements row_type wide, r*ld + c; three more behind the last one are read, not used; n_rows *
+ * ld < 2^31), k_diag its diagonal; the n_pos rows (and columns) from row_pos on have y = +1, the n_neg from row_neg on y = -1;
+ * its alpha and f are the n_pos + n_neg entries from `at` on; ws: working-set size, 2 .. n_pos + n_neg, even; max_iter: steps of one
+ * local solve at most; nu: Cp is the problem's C.  max_slots: the most that n_pos rounded up to four plus n_neg comes to
+ * (1 .. tsvm_smo_small_max()).  start != 0: a first call (alpha and f hold the start values, f without the terms of
+ * a non-zero alpha); 0: goes on with the problems whose state says 0.
+ * states[p].status: 0 more to do (a call ends after a bounded number of steps), 1 solved, 2 given up because a working set
+ * could not be filled (alpha and f are no longer the start values).  ws_store: n_problems * tsvm_smo_small_max() ints, kept between the calls. */
 typedef struct {
-    int row_pos, n_pos, row_neg, n_neg, ws, max_iter;   /* max_iter: steps of one local solve at most */
+    const void *k;
+    const double *k_diag;
+    int64_t ld, at;
+    int n_rows, row_pos, n_pos, row_neg, n_neg, ws, max_iter, reserved;
     double Cp, Cn;
-    int64_t at;
 } tsvm_small_problem;
 typedef struct {
     double previous_diff, last_diff, second_last_diff, diff;
@@ -310,9 +312,8 @@ typedef struct {
     int same_count, swap_count, iter, status, xcd, reserved;
 } tsvm_small_state;
 int tsvm_smo_small_max(void);
-int tsvm_smo_solve_small(const void *k, int row_type, int64_t ld, int n_rows, const double *k_diag, const tsvm_small_problem *problems,
-                         int n_problems, int max_slots, tsvm_small_state *states, int *ws_store, double *alpha, double *f, int nu, double eps,
-                         int out_max_iter, int start, tsvm_stream stream);
+int tsvm_smo_solve_small(int row_type, const tsvm_small_problem *problems, int n_problems, int max_slots, tsvm_small_state *states,
+                         int *ws_store, double *alpha, double *f, int nu, double eps, int out_max_iter, int start, tsvm_stream stream);
 
 /* nu_smo_solve (smo_kernel.cpp:127-298), same conventions; diff[1] is left untouched as in the
  * reference's CPU code. */

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from thundersvm_amd import data as D
-from thundersvm_amd.model import Model, make_param
+from thundersvm_amd.model import Dataset, Model, make_param
 
 import test_gpu_models as T
 
@@ -57,3 +57,14 @@ def test_class_pairs_from_one_matrix(sizes):
     a = Model(0).train(d, make_param(gamma=0.2, C=3.0, kernel_type=0))
     b = Model(0).train(d, make_param(gamma=0.2, C=3.0, kernel_type=0, pair_lanes=1, cache_bytes=0))   # (asks for the other path)
     assert np.array_equal(a.coef, b.coef) and np.array_equal(a.rho, b.rho) and np.array_equal(a.sv_indices, b.sv_indices)
+
+
+@pytest.mark.parametrize("svm_type,n,folds", [(0, 203, 5), (1, 120, 3), (2, 61, 4), (3, 90, 3), (4, 90, 3), (0, 1500, 3), (0, 12, 6)])
+def test_folds_side_by_side(svm_type, n, folds):
+    """Cross-validation with its folds solved together, and one fold after the other (a row budget asks for that path)."""
+    x, rng = _rows(n, n + 7, False)
+    y = np.sin(x[:, 0]) if svm_type >= 3 else (x[:, 0] + 0.3 * rng.standard_normal(n) > 0).astype(np.float64) * (svm_type != 2)
+    d = Dataset(D.from_dense(x, y))
+    got = [Model(svm_type).cross_validation(d, make_param(svm_type=svm_type, gamma=0.2, C=3.0, nu=0.2, p=0.05, cache_bytes=c), folds)
+           for c in (-1, 64 << 20)]
+    assert np.array_equal(got[0], got[1])

@@ -63,7 +63,7 @@ SIGNATURES = {
     "tsvm_smo_start": (_int, [_p, _int, _p, _int, _int, _p, _int, _p, _p, _p]),
     "tsvm_smo_warm_block": (_int, [_p, _int, _int, _int, _p, _p]),
     "tsvm_smo_small_max": (_int, []),
-    "tsvm_smo_solve_small": (_int, [_p, _int, _i64, _int, _p, _p, _int, _int, _p, _p, _p, _p, _int, _dbl, _int, _int, _p]),
+    "tsvm_smo_solve_small": (_int, [_int, _p, _int, _int, _p, _p, _p, _p, _int, _dbl, _int, _int, _p]),
     "tsvm_select_workspace": (C.c_size_t, [_i64]),
     "tsvm_report_ids": (_int, [_p, _int, _int, _p, _int, _int, _p]),
     "tsvm_select_working_set": (_int, [_p, _p, _p, _i64, _dbl, _dbl, _p, _int, _p, _int, _int, _p, _p]),

@@ -30,15 +30,16 @@ __device__ __forceinline__ bool is_none(double v) { return __builtin_amdgcn_read
 // (the same for memory accesses: a row's load stays in front of the work that is to pass while it is on its way, and
 // in front of the exit test; the block is not declared restrict, or the load could be moved all the same)
 #define SV_PIN_MEMORY asm volatile("" ::: "memory")
-template <int E>
-__device__ __forceinline__ int wave_first_argmin(const double (&x)[E], int base, double &value, double &m, int &at) {
+// TWICE: `twice` is the lanes of which several elements hold the lane's smallest value.
+template <int E, bool TWICE>
+__device__ __forceinline__ int wave_argmin(const double (&x)[E], int base, double &value, double &m, int &at, uint64_t &twice) {
     m = x[0];
 #pragma unroll
     for (int e = 1; e < E; ++e) m = fmin_f64(m, x[e]);
     SV_PIN;
     uint64_t has[E];   // which lanes' element e is their minimum
 #pragma unroll
-    for (int e = 0; e < E - 1; ++e) asm volatile("v_cmp_eq_f64_e64 %0, %1, %2" : "=s"(has[e]) : "v"(x[e]), "v"(m));
+    for (int e = 0; e < (TWICE ? E : E - 1); ++e) asm volatile("v_cmp_eq_f64_e64 %0, %1, %2" : "=s"(has[e]) : "v"(x[e]), "v"(m));
     SV_PIN;
     int tl = dpp_i32<TSVM_DPP_XOR1>(__double2loint(m)), th = dpp_i32<TSVM_DPP_XOR1>(__double2hiint(m));
     double r = fmin_f64(m, __hiloint2double(th, tl));
@@ -54,6 +55,15 @@ __device__ __forceinline__ int wave_first_argmin(const double (&x)[E], int base,
 #pragma unroll
     for (int e = E - 4; e >= 0; --e) asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(at) : "v"(at), "v"(base + e), "s"(has[e]));
     SV_PIN;
+    if constexpr (TWICE) {   // (scalar work in the gaps of the chain)
+        twice = 0;
+        uint64_t one = E > 1 ? has[0] : 0;
+#pragma unroll
+        for (int e = 1; e < E; ++e) {
+            twice |= one & has[e];
+            one |= has[e];
+        }
+    }
     tl = dpp_i32<TSVM_DPP_HALF_MIRROR>(__double2loint(r));
     th = dpp_i32<TSVM_DPP_HALF_MIRROR>(__double2hiint(r));
     r = fmin_f64(r, __hiloint2double(th, tl));
@@ -69,6 +79,11 @@ __device__ __forceinline__ int wave_first_argmin(const double (&x)[E], int base,
     r = fmin_f64(r, __hiloint2double(th, tl));
     value = readlane_f64(r, 63);
     return __builtin_ctzll(__builtin_amdgcn_ballot_w64(m == value));
+}
+template <int E>
+__device__ __forceinline__ int wave_first_argmin(const double (&x)[E], int base, double &value, double &m, int &at) {
+    uint64_t twice;
+    return wave_argmin<E, false>(x, base, value, m, at, twice);
 }
 
 // The LDS address of a __shared__ object as the ds instructions take it.

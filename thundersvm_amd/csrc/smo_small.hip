@@ -10,11 +10,10 @@
 // training calls: 45 pairs of 360 instances in 64 columns 31 -> 1.95 ms, 3 pairs of 100 in 4 columns 2.4 -> 0.70 ms.
 //
 // Shape.  At most 1,024 instances (above that a workgroup's share of update_f and of the selection outlasts what the
-// chip-wide kernels take, and their launches no longer matter): W wavefronts of four neighbouring instances per thread.
+// chip-wide kernels take, and their launches no longer matter): W wavefronts of E neighbouring instances per thread.
 // f, the local solver's f and the sets' membership live in registers, alpha in LDS.  The local solver runs on the
 // instances where they are, not on a gathered working set: an instance outside the working set is in neither I_up nor I_low, a row is
-// read from the kernel matrix in one piece, and ties go to the instance that comes first in the working set (its position
-// there is the upper half of the key that is compared among equals).
+// read from the kernel matrix in one piece, and ties go to the instance that comes first in the working set.
 #include "../../include/thundersvm_amd.h"
 #include "smo_local.h"
 #include "tsvm_internal.h"
@@ -33,36 +32,45 @@ __device__ __forceinline__ int wave_min_i32(int v) {
     return __builtin_amdgcn_readlane(v, 63);
 }
 
-// As wave_first_argmin (smo_local.h), with a key per element in place of its position: among equal values the lowest
-// key wins.
+// As wave_first_argmin (smo_local.h), but among equal values the element that comes first in the working set wins.
+// Equal values are rare once the first steps have told the instances apart: they are looked for (scalar work beside the
+// reduction) and only then are the positions read.
 template <int E>
-__device__ __forceinline__ int wave_argmin_by_key(const double (&x)[E], const int (&key)[E], double &value, double &m, int &at) {
-    m = x[0];
-#pragma unroll
-    for (int e = 1; e < E; ++e) m = fmin_f64(m, x[e]);
-    at = 0x7fffffff;
-#pragma unroll
-    for (int e = 0; e < E; ++e) at = x[e] == m ? imin_sel(at, key[e]) : at;
-    value = wave_min_f64(m);
+__device__ __forceinline__ int wave_argmin_by_pos(const double (&x)[E], const unsigned short *pos, int tid, double &value, double &m, int &at) {
+    uint64_t twice;
+    int win = wave_argmin<E, true>(x, tid * E, value, m, at, twice);
     uint64_t who = __builtin_amdgcn_ballot_w64(m == value);
-    if (__popcll(who) != 1) {
-        const int k = wave_min_i32(m == value ? at : 0x7fffffff);
-        who &= __builtin_amdgcn_ballot_w64(at == k);
+    if (__builtin_expect(((who & (who - 1)) | (who & twice)) != 0, 0)) {
+        int key = 0x7fffffff;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const int k = (int) pos[tid * E + e] << 10 | e;
+            key = x[e] == value ? imin_sel(key, k) : key;
+        }
+        const int first = wave_min_i32(key);
+        who = __builtin_amdgcn_ballot_w64(key == first && m == value);
+        win = __builtin_ctzll(who);
+        at = tid * E + (key & (E - 1));
     }
-    return __builtin_ctzll(who);
+    return win;
 }
 
 template <int W>
-__device__ __forceinline__ void block_argmin_by_key(const SvCand *slots, int lane, double &v, int &at, int &flags) {
+__device__ __forceinline__ void block_argmin_by_pos(const SvCand *slots, const unsigned short *pos, int lane, double &v, int &at, int &flags) {
     static_assert(W == 2 || W == 4, "quad_perm steps");
     const SvCand c = slots[lane & (W - 1)];
     double m = fmin_f64(c.v, dpp_f64<TSVM_DPP_XOR1>(c.v));
     if (W == 4) m = fmin_f64(m, dpp_f64<TSVM_DPP_XOR2>(m));
-    int k = c.v == m ? c.at : 0x7fffffff;
-    k = imin_sel(k, dpp_i32<TSVM_DPP_XOR1>(k));
-    if (W == 4) k = imin_sel(k, dpp_i32<TSVM_DPP_XOR2>(k));
     v = m;
-    at = __builtin_amdgcn_readfirstlane(k);
+    uint64_t who = __builtin_amdgcn_ballot_w64(c.v == m);
+    if (__builtin_expect((who & (who - 1) & ((1 << W) - 1)) != 0, 0)) {   // (every quad holds the same W)
+        int k = c.v == m ? (int) pos[c.at] : 0x7fffffff;
+        const int mine = k;
+        k = imin_sel(k, dpp_i32<TSVM_DPP_XOR1>(k));
+        k = imin_sel(k, dpp_i32<TSVM_DPP_XOR2>(k));
+        who = __builtin_amdgcn_ballot_w64(mine == k && c.v == m);
+    }
+    at = __builtin_amdgcn_readlane(c.at, __builtin_ctzll(who));
     flags = __builtin_amdgcn_ballot_w64(c.flag != 0) != 0;
 }
 
@@ -72,14 +80,14 @@ __device__ __forceinline__ uint64_t ss_key(double f) {   // order-preserving; -0
     return (u >> 63) ? ~u : (u | 0x8000000000000000ull);
 }
 
-template <int W>
+template <int E, int W>
 struct SmallShared {
-    static constexpr int N = 256 * W;
+    static constexpr int N = 64 * E * W;
     double kd[N];
     double a[W][N];                     // alpha: one copy per wavefront (smo_solve.hip)
-    double f[N], k[N];                  // local solver: f and the row at the candidates; selection: sort keys and slots; update: coefficients and rows
+    double f[N], k[N];                  // local solver: f and the row at the candidates; selection: keys and slots on their way between wavefronts; update: coefficients and rows
     unsigned short pos[N];              // position of a slot in the working set, 0xffff outside it
-    unsigned short ws[SS_MAX < N ? SS_MAX : N];
+    unsigned short ws[N];
     unsigned char flags[N];             // selection: the sides an instance is a candidate of
     uint64_t total[2][W];               // per-wavefront counts of a scan
     double red[4][W];
@@ -96,48 +104,98 @@ struct SmallShared {
 // a candidate of both sides has been taken by one of them (the two ends have met), so from then on each side goes on with
 // the candidates that are its own alone.  The event is the minimum of a round number over the instances, and what remains are
 // prefix counts.
-template <int W, bool NU>
-__device__ bool ss_select(SmallShared<W> &sh, int k, int base) {
-    constexpr int N = 256 * W, T = 64 * W, NP = NU ? 2 : 1;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    uint64_t *skey = (uint64_t *) sh.f;
-    unsigned short *sidx = (unsigned short *) sh.k;
-    // bitonic sort of (key, slot), ascending; two pairs per thread and stage.  Strides below 128 stay inside a wavefront's
-    // 256 entries, which need no barrier with one another.
-    for (int size = 2; size <= N; size <<= 1) {
-        for (int strd = size >> 1; strd > 0; strd >>= 1) {
+// The value of lane ^ D.
+template <int D>
+__device__ __forceinline__ int lane_xor(int v, int lane) {
+    if constexpr (D == 1) return dpp_i32<TSVM_DPP_XOR1>(v);
+    else if constexpr (D == 2) return dpp_i32<TSVM_DPP_XOR2>(v);
+    else if constexpr (D == 4) return dpp_i32<TSVM_DPP_HALF_MIRROR>(dpp_i32<0x1B>(v));   // quad_perm [3,2,1,0]: ^ 3, then ^ 7
+    else if constexpr (D == 8) return dpp_i32<0x128>(v);                                 // row_ror:8
+    else return __builtin_amdgcn_ds_bpermute((lane ^ D) << 2, v);
+}
+
+// One step of the sort at a fixed stride: entry i against entry i ^ STRD, ascending where i & size is zero.
+template <int E, int W, int STRD>
+__device__ __forceinline__ void ss_sort_step(SmallShared<E, W> &sh, uint64_t (&key)[E], int (&slot)[E], int size) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    auto less = [](uint64_t ka, int ia, uint64_t kb, int ib) { return (ka < kb) | ((ka == kb) & (ia < ib)); };
+    if constexpr (STRD < E) {
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int pr = wave * 128 + h * 64 + lane;   // a wavefront's pairs lie in its own 256 entries while strd < 256
-                const int lo = ((pr & ~(strd - 1)) << 1) | (pr & (strd - 1)), hi = lo | strd;
-                const uint64_t ka = skey[lo], kb = skey[hi];
-                const unsigned short ia = sidx[lo], ib = sidx[hi];
-                const bool asc = (lo & size) == 0, less_ba = kb < ka || (kb == ka && ib < ia);
-                if (asc == less_ba) { skey[lo] = kb; skey[hi] = ka; sidx[lo] = ib; sidx[hi] = ia; }
-            }
-            const int next = strd > 1 ? strd >> 1 : size;
-            if (strd > 128 || next > 128) __syncthreads();
-            else {
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-                __builtin_amdgcn_wave_barrier();
+        for (int e = 0; e < E; ++e) {
+            if (e & STRD) continue;
+            const int o = e | STRD;
+            const bool asc = ((tid * E + e) & size) == 0;
+            const bool swap = less(key[o], slot[o], key[e], slot[e]) == asc;
+            const uint64_t ke = swap ? key[o] : key[e], ko = swap ? key[e] : key[o];
+            const int se = swap ? slot[o] : slot[e], so = swap ? slot[e] : slot[o];
+            key[e] = ke; key[o] = ko;
+            slot[e] = se; slot[o] = so;
+        }
+    } else {
+        const bool want_less = ((tid * E & STRD) == 0) == ((tid * E & size) == 0);
+        uint64_t ok[E];
+        int os[E];
+        if constexpr (STRD >= 64 * E) {
+            uint64_t *const xk = (uint64_t *) sh.f;
+            int *const xs = (int *) sh.k;
+#pragma unroll
+            for (int e = 0; e < E; ++e) { xk[e * 64 * W + tid] = key[e]; xs[e * 64 * W + tid] = slot[e]; }
+            __syncthreads();
+            const int other = tid ^ (STRD / E);
+#pragma unroll
+            for (int e = 0; e < E; ++e) { ok[e] = xk[e * 64 * W + other]; os[e] = xs[e * 64 * W + other]; }
+            __syncthreads();
+        } else {
+            constexpr int D = STRD / E;
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const unsigned lo = (unsigned) lane_xor<D>((int) (uint32_t) key[e], lane), hi = (unsigned) lane_xor<D>((int) (uint32_t) (key[e] >> 32), lane);
+                ok[e] = (uint64_t) hi << 32 | lo;
+                os[e] = lane_xor<D>(slot[e], lane);
             }
         }
-    }
-    __syncthreads();
-    int slot[4];
-    unsigned fl[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        slot[j] = sidx[tid * 4 + j];
-        fl[j] = sh.flags[slot[j]];
+        for (int e = 0; e < E; ++e) {
+            const bool take = less(ok[e], os[e], key[e], slot[e]) == want_less;
+            key[e] = take ? ok[e] : key[e];
+            slot[e] = take ? os[e] : slot[e];
+        }
     }
+}
+
+// A bitonic sort of E neighbouring entries per thread in registers: strides below E inside a thread, below 64 * E between
+// the lanes of a wavefront (below 16 * E without the LDS's crossbar, which four wavefronts would queue for), the others through LDS.
+template <int E, int W, int STRD>
+__device__ __forceinline__ void ss_merge(SmallShared<E, W> &sh, uint64_t (&key)[E], int (&slot)[E], int size) {
+    if constexpr (STRD > 0) {
+        if (STRD < size) ss_sort_step<E, W, STRD>(sh, key, slot, size);
+        ss_merge<E, W, STRD / 2>(sh, key, slot, size);
+    }
+}
+
+template <int E, int W, bool NU>
+__device__ bool ss_select(SmallShared<E, W> &sh, const double (&f)[E], const bool (&act)[E], int k, int base) {
+    constexpr int NP = NU ? 2 : 1;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    uint64_t key[E];
+    int slot[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        key[e] = act[e] ? ss_key(f[e]) : ~0ull;
+        slot[e] = tid * E + e;
+    }
+#pragma unroll 1
+    for (int size = 2; size <= 64 * E * W; size <<= 1) ss_merge<E, W, 32 * E * W>(sh, key, slot, size);
+    unsigned fl[E];
+#pragma unroll
+    for (int j = 0; j < E; ++j) fl[j] = sh.flags[slot[j]];
     // counts of up, low, up alone, low alone in 16-bit fields; inclusive scan over the sorted order
-    uint64_t incl[NP][4], total[NP];
+    uint64_t incl[NP][E], total[NP];
 #pragma unroll
     for (int q = 0; q < NP; ++q) {
         uint64_t run = 0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < E; ++j) {
             const unsigned u = (fl[j] >> q) & 1u, l = (fl[j] >> (q + NP)) & 1u;
             run += (uint64_t) u | (uint64_t) l << 16 | (uint64_t) (u & ~l & 1u) << 32 | (uint64_t) (l & ~u & 1u) << 48;
             incl[q][j] = run;
@@ -150,7 +208,7 @@ __device__ bool ss_select(SmallShared<W> &sh, int k, int base) {
         }
         if (lane == 63) sh.total[q][wave] = scan;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) incl[q][j] += scan - run;
+        for (int j = 0; j < E; ++j) incl[q][j] += scan - run;
     }
     __syncthreads();
 #pragma unroll
@@ -164,7 +222,7 @@ __device__ bool ss_select(SmallShared<W> &sh, int k, int base) {
             total[q] += t;
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) incl[q][j] += before;
+        for (int j = 0; j < E; ++j) incl[q][j] += before;
         if (tid == 0) {
             const int n_up = (int) (total[q] & 0xffff), n_low = (int) (total[q] >> 16 & 0xffff);
             const int dry_up = 2 * n_up, dry_low = 2 * n_low + 1;
@@ -177,7 +235,7 @@ __device__ bool ss_select(SmallShared<W> &sh, int k, int base) {
 #pragma unroll
     for (int q = 0; q < NP; ++q)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < E; ++j) {
             if (!((fl[j] >> q) & (fl[j] >> (q + NP)) & 1u)) continue;
             const int ru = (int) (incl[q][j] & 0xffff) - 1, rl = (int) (total[q] >> 16 & 0xffff) - (int) (incl[q][j] >> 16 & 0xffff);
             atomicMin(&sh.event[q], ru <= rl ? 2 * rl + 1 : 2 * ru);   // the round in which the other side finds it taken
@@ -189,7 +247,7 @@ __device__ bool ss_select(SmallShared<W> &sh, int k, int base) {
         b0[q] = sh.event[q] >> 1;
         a0[q] = b0[q] + (sh.event[q] & 1);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < E; ++j) {
             const unsigned u = (fl[j] >> q) & 1u, l = (fl[j] >> (q + NP)) & 1u;
             const int ru = (int) (incl[q][j] & 0xffff) - 1, rl = (int) (total[q] >> 16 & 0xffff) - (int) (incl[q][j] >> 16 & 0xffff);
             if (u && ru == a0[q]) sh.first_x[q] = (int) (incl[q][j] >> 32 & 0xffff) - (int) (u & ~l & 1u);
@@ -213,7 +271,7 @@ __device__ bool ss_select(SmallShared<W> &sh, int k, int base) {
 #pragma unroll
     for (int q = 0; q < NP; ++q)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < E; ++j) {
             const unsigned u = (fl[j] >> q) & 1u, l = (fl[j] >> (q + NP)) & 1u;
             const int ru = (int) (incl[q][j] & 0xffff) - 1, rl = (int) (total[q] >> 16 & 0xffff) - (int) (incl[q][j] >> 16 & 0xffff);
             if (u) {
@@ -242,24 +300,27 @@ struct SmallMap {
     __device__ __forceinline__ double label(int s) const { return s < n0p ? 1.0 : -1.0; }
 };
 
-template <typename TB>
-__device__ __forceinline__ void ss_load(const TB *row, TB (&out)[4]) {
-    typedef TB vec_t __attribute__((ext_vector_type(4), aligned(sizeof(TB))));   // (a class's columns start anywhere)
-    const vec_t v = *(const vec_t *) row;
+template <int E, typename TB>
+__device__ __forceinline__ void ss_load(const TB *row, TB (&out)[E]) {
+    if constexpr (E == 1) {
+        out[0] = *row;
+    } else {
+        typedef TB vec_t __attribute__((ext_vector_type(E), aligned(sizeof(TB))));   // (a class's columns start anywhere)
+        const vec_t v = *(const vec_t *) row;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) out[e] = v[e];
+        for (int e = 0; e < E; ++e) out[e] = v[e];
+    }
 }
 
 // The local solver: c_smo_iterate of smo_solve.hip (and nu_smo_solve_kernel) with the instances in place of a gathered
-// working set.  Returns the steps taken; the new alpha is in sh.a.
-template <int W, bool NU, typename TB>
-__device__ int ss_local(SmallShared<W> &sh, const SmallMap &map, const TB *K, int64_t ld, int col, const double (&kd)[4], double (&f)[4],
-                        unsigned member, const int (&key)[4], double Cp, double Cn, double local_eps, int max_iter) {
+// working set.  Returns the steps taken; the new alpha is in sh.a.  NONE: the threshold is not positive (see there).
+template <int E, int W, bool NU, bool NONE, typename TB>
+__device__ __forceinline__ int ss_local(SmallShared<E, W> &sh, const SmallMap &map, const TB *K, int64_t ld, int col, const double (&kd)[E], double (&f)[E],
+                        unsigned member, double Cp, double Cn, double local_eps, int max_iter) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const double half_Cp = 0.5 * Cp, half_Cn = NU ? half_Cp : 0.5 * Cn;
     constexpr int NP = NU ? 2 : 1;   // pairs of sides
     SvCand *const ci[2] = {sh.ci, sh.ci2}, *const cj[2] = {sh.cj, sh.cj2};
-    const bool none_possible = __builtin_amdgcn_readfirstlane(local_eps > 0.0 ? 0 : 1) != 0;
     const int first_slot = sh.ws[0];
     int n_iter = 0;
     bool go_on;
@@ -268,31 +329,31 @@ __device__ int ss_local(SmallShared<W> &sh, const SmallMap &map, const TB *K, in
         int at[NP], is[NP], go;
 #pragma unroll
         for (int q = 0; q < NP; ++q) {
-            double fu[4];
+            double fu[E];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) fu[e] = keep_or_none<0>(member << (31 - 2 * NP * e - q), f[e]);
-            const int win = wave_argmin_by_key<4>(fu, key, up[q], m[q], at[q]);
+            for (int e = 0; e < E; ++e) fu[e] = keep_or_none<0>(member << (31 - 2 * NP * e - q), f[e]);
+            const int win = wave_argmin_by_pos<E>(fu, sh.pos, tid, up[q], m[q], at[q]);
             if constexpr (W > 1) publish(ci[q] + wave, win, m[q], at[q], 0);
             else is[q] = __builtin_amdgcn_readlane(at[q], win);
         }
         if constexpr (W > 1) {
             lds_barrier();
 #pragma unroll
-            for (int q = 0; q < NP; ++q) block_argmin_by_key<W>(ci[q], lane, up[q], is[q], go);
+            for (int q = 0; q < NP; ++q) block_argmin_by_pos<W>(ci[q], sh.pos, lane, up[q], is[q], go);
         }
-        TB kI[NP][4];
+        TB kI[NP][E];
         double kd_i[NP];
 #pragma unroll
         for (int q = 0; q < NP; ++q) {
-            is[q] &= 256 * W - 1;   // (with only NaN left there is no candidate at all)
+            is[q] &= 64 * E * W - 1;   // (with only NaN left there is no candidate at all)
             if (NU) is[q] = is_none(up[q]) ? first_slot : is[q];   // (its row enters the other side's scores, smo_kernel.cpp:239)
-            ss_load<TB>(K + (int64_t) map.row(is[q]) * ld + col, kI[q]);
+            ss_load<E, TB>(K + (unsigned) map.row(is[q]) * (unsigned) ld + col, kI[q]);
             kd_i[q] = sh.kd[is[q]];
         }
         SV_PIN_MEMORY;
-        double part[4], b[NP][4], b_max = -__builtin_inf();
+        double part[E], b[NP][E], b_max = -__builtin_inf();
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
+        for (int e = 0; e < E; ++e) {
             part[e] = kd_i[0] + kd[e];
 #pragma unroll
             for (int q = 0; q < NP; ++q) {
@@ -306,15 +367,15 @@ __device__ int ss_local(SmallShared<W> &sh, const SmallMap &map, const TB *K, in
         int js[NP];
 #pragma unroll
         for (int q = 0; q < NP; ++q) {
-            double qs[4];
+            double qs[E];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
+            for (int e = 0; e < E; ++e) {
                 const double aIJ = __builtin_fma(-2.0, (double) kI[0][e], part[e]);
                 const double s = -b[q][e] * b[q][e] / aIJ;
                 qs[e] = __hiloint2double(b[q][e] > 0.0 ? __double2hiint(s) : SV_NONE_HI, __double2loint(s));
             }
-            const int win = wave_argmin_by_key<4>(qs, key, best[q], v, at[q]);
-            publish_row<4, TB>(sh.f + tid * 4, sh.k + tid * 4, win, f, kI[q]);
+            const int win = wave_argmin_by_pos<E>(qs, sh.pos, tid, best[q], v, at[q]);
+            publish_row<E, TB>(sh.f + tid * E, sh.k + tid * E, win, f, kI[q]);
             if constexpr (W > 1) publish(cj[q] + wave, win, v, at[q], go);
             else js[q] = __builtin_amdgcn_readlane(at[q], win);
         }
@@ -323,31 +384,31 @@ __device__ int ss_local(SmallShared<W> &sh, const SmallMap &map, const TB *K, in
 #pragma unroll
             for (int q = 0; q < NP; ++q) {
                 int g;
-                block_argmin_by_key<W>(cj[q], lane, best[q], js[q], g);
+                block_argmin_by_pos<W>(cj[q], sh.pos, lane, best[q], js[q], g);
                 if (q == 0) go = g;
             }
         }
         const bool second = NU && !__builtin_amdgcn_readfirstlane(best[0] < best[NP - 1] && best[0] < SV_NONE ? 1 : 0);
         const int i = second ? is[NP - 1] : is[0];
-        int j2 = (second ? js[NP - 1] : js[0]) & (256 * W - 1);
+        int j2 = (second ? js[NP - 1] : js[0]) & (64 * E * W - 1);
         const double up_value = second ? up[NP - 1] : up[0], kd_i2 = second ? kd_i[NP - 1] : kd_i[0];
         // (two sides' winners may write different rows into one lane's slots when one of them has no candidate, so with
         // two sides K[i, j2] is read from the matrix)
-        if (none_possible && is_none(second ? best[NP - 1] : best[0])) {
+        if (NONE && is_none(second ? best[NP - 1] : best[0])) {
             j2 = first_slot;
             __syncthreads();
-            if (tid == first_slot / 4) {
+            if (tid == first_slot / E) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    sh.f[tid * 4 + e] = f[e];
-                    *(TB *) (sh.k + tid * 4 + e) = second ? kI[NP - 1][e] : kI[0][e];
+                for (int e = 0; e < E; ++e) {
+                    sh.f[tid * E + e] = f[e];
+                    *(TB *) (sh.k + tid * E + e) = second ? kI[NP - 1][e] : kI[0][e];
                 }
             }
             __syncthreads();
         }
-        TB kJ[4];
-        ss_load<TB>(K + (int64_t) map.row(j2) * ld + col, kJ);
-        const TB k_ij = NU ? K[(int64_t) map.row(i) * ld + map.row(j2)] : *(const TB *) (sh.k + j2);
+        TB kJ[E];
+        ss_load<E, TB>(K + (unsigned) map.row(j2) * (unsigned) ld + col, kJ);
+        const TB k_ij = NU ? K[(unsigned) map.row(i) * (unsigned) ld + map.row(j2)] : *(const TB *) (sh.k + j2);
         SV_PIN_MEMORY;
         const double kd_j = sh.kd[j2], a_j = sh.a[wave][j2], a_i = sh.a[wave][i], f_j = sh.f[j2], y_i = map.label(i), y_j = map.label(j2);
         SV_PIN;
@@ -359,51 +420,88 @@ __device__ int ss_local(SmallShared<W> &sh, const SmallMap &map, const TB *K, in
             const unsigned u = room_up(a, y, half_Cp) > 0 ? 1u : 0u, w = room_low(a, y, half_Cn) > 0 ? (1u << NP) : 0u;
             return (u | w) << (NU && y < 0 ? 1 : 0);
         };
-        member = set_member_bits<4, 2 * NP>(member, tid, i, bits(na_i, y_i));
-        member = set_member_bits<4, 2 * NP>(member, tid, j2, bits(na_j, y_j));
+        member = set_member_bits<E, 2 * NP>(member, tid, i, bits(na_i, y_i));
+        member = set_member_bits<E, 2 * NP>(member, tid, j2, bits(na_j, y_j));
         write_by_lane0(go_on, &sh.a[wave][i], na_i, &sh.a[wave][j2], na_j);
         SV_PIN;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) f[e] = __builtin_fma(-l, (double) kJ[e] - (double) (second ? kI[NP - 1][e] : kI[0][e]), f[e]);
+        for (int e = 0; e < E; ++e) f[e] = __builtin_fma(-l, (double) kJ[e] - (double) (second ? kI[NP - 1][e] : kI[0][e]), f[e]);
         n_iter += go_on;
     } while (go_on);
     return n_iter;
 }
 
 // f[j] -= sum over the n_list listed rows (coefficients sh.f, rows in sh.k) in order (smo_kernel.cpp:300-319)
-template <int W, typename TB>
-__device__ __forceinline__ void ss_update_f(const SmallShared<W> &sh, const TB *K, int64_t ld, int col, int first, int last, double (&f)[4]) {
+template <int E, int W, typename TB>
+__device__ __forceinline__ void ss_update_f(const SmallShared<E, W> &sh, const TB *K, int64_t ld, int col, int first, int last, double (&f)[E]) {
     const int *rows = (const int *) sh.k;
-    double sum[4] = {0.0, 0.0, 0.0, 0.0};
+    double sum[E] = {};
     int t = first;
     constexpr int U = 8;
     for (; t + U <= last; t += U) {
-        TB k[U][4];
+        TB k[U][E];
 #pragma unroll
-        for (int u = 0; u < U; ++u) ss_load<TB>(K + (int64_t) rows[t + u] * ld + col, k[u]);
+        for (int u = 0; u < U; ++u) ss_load<E, TB>(K + (int64_t) rows[t + u] * ld + col, k[u]);
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) sum[e] = __builtin_fma(sh.f[t + u], (double) k[u][e], sum[e]);
+            for (int e = 0; e < E; ++e) sum[e] = __builtin_fma(sh.f[t + u], (double) k[u][e], sum[e]);
     }
     for (; t < last; ++t) {
-        TB k[4];
-        ss_load<TB>(K + (int64_t) rows[t] * ld + col, k);
+        TB k[E];
+        ss_load<E, TB>(K + (int64_t) rows[t] * ld + col, k);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sum[e] = __builtin_fma(sh.f[t], (double) k[e], sum[e]);
+        for (int e = 0; e < E; ++e) sum[e] = __builtin_fma(sh.f[t], (double) k[e], sum[e]);
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) f[e] -= sum[e];
+    for (int e = 0; e < E; ++e) f[e] -= sum[e];
 }
 
-template <int W, bool NU, typename TB>
-__global__ __launch_bounds__(64 * W) void smo_small_kernel(const TB *K, int64_t ld, int n_rows, const double *__restrict__ k_diag,
-                                                           const tsvm_small_problem *__restrict__ problems,
-                                                           tsvm_small_state *states, int *ws_all, double *alpha_all, double *f_all, double eps, int out_max_iter, int start) {
-    constexpr int N = 256 * W;
-    __shared__ SmallShared<W> sh;
+// Reads the kernel matrices of the problems whose workgroups run on this die into its L2, so that a step finds its rows
+// there (250 cycles instead of 700 and more; a lone workgroup would need 330,000 cycles for 960 instances).  Workgroups are
+// dealt to the eight dies in turn: number x of every eight reads for the problems x, x + 8, ..., up to SS_WARM_BYTES.
+// 963 instances, 1,080 steps: 3.74 -> 3.48 million cycles; 360 instances, 348 steps: 1.25 -> 1.18.
+#define SS_WARM_GROUPS 32
+#define SS_WARM_BYTES (3 << 20)
+template <typename TB>
+__device__ __forceinline__ void ss_warm(const tsvm_small_problem *__restrict__ problems, int n_problems, int x, int group) {
+    typedef uint32_t vec_t __attribute__((ext_vector_type(4), aligned(4)));
+    constexpr int V = 16 / (int) sizeof(TB);
+    int64_t left = SS_WARM_BYTES;
+    for (int p = x; p < n_problems && left > 0; p += 8) {
+        const tsvm_small_problem P = problems[p];
+        const int n = P.n_pos + P.n_neg;
+        left -= (int64_t) n * n * sizeof(TB);
+        for (int r = group; r < n; r += SS_WARM_GROUPS) {
+            const TB *const row = (const TB *) P.k + (int64_t) (r < P.n_pos ? P.row_pos + r : P.row_neg + (r - P.n_pos)) * P.ld;
+#pragma unroll
+            for (int side = 0; side < 2; ++side) {
+                const int from = side ? P.row_neg : P.row_pos, count = side ? P.n_neg : P.n_pos;
+                for (int c = threadIdx.x * V; c < count; c += blockDim.x * V) {
+                    const vec_t v = *(const vec_t *) (row + from + c);
+                    asm volatile("" ::"v"(v));
+                }
+            }
+        }
+    }
+}
+
+template <int E, int W, bool NU, typename TB>
+__global__ __launch_bounds__(64 * W) void smo_small_kernel(const tsvm_small_problem *__restrict__ problems, int n_problems,
+                                                           tsvm_small_state *states, int *ws_all, double *alpha_all, double *f_all, double eps,
+                                                           int out_max_iter, int start) {
+    constexpr int N = 64 * E * W;
+    __shared__ SmallShared<E, W> sh;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if ((int) blockIdx.x >= n_problems) {
+        const int warm = (int) blockIdx.x - (n_problems + 7) / 8 * 8;
+        if (warm >= 0) ss_warm<TB>(problems, n_problems, warm % 8, warm / 8);
+        return;
+    }
+    __builtin_amdgcn_s_setprio(3);   // (a chain of dependent steps: not to wait behind other kernels' wavefronts)
     const tsvm_small_problem P = problems[blockIdx.x];
+    const TB *const K = (const TB *) P.k;
+    const int64_t ld = P.ld;
     tsvm_small_state *const S = states + blockIdx.x;
     int *const ws_kept = ws_all + (int64_t) blockIdx.x * SS_MAX;
     if (!start && S->status != 0) return;
@@ -413,26 +511,26 @@ __global__ __launch_bounds__(64 * W) void smo_small_kernel(const TB *K, int64_t 
     map.n0p = (P.n_pos + 3) & ~3;   // (both fit: n0p + n_neg <= N is checked on the host)
     map.col0 = P.row_pos;
     map.col1 = P.row_neg;
-    map.n_rows = n_rows;
+    map.n_rows = P.n_rows;
     double *const alpha = alpha_all + P.at, *const f_out = f_all + P.at;
     const int ws = P.ws, q = ws / 2;
-    double f[4], kd[4];
-    bool act[4];
+    double f[E], kd[E];
+    bool act[E];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int s = tid * 4 + e;
+    for (int e = 0; e < E; ++e) {
+        const int s = tid * E + e;
         act[e] = map.active(s);
         const double a = act[e] ? alpha[map.index(s)] : 0.0;
         f[e] = act[e] ? f_out[map.index(s)] : 0.0;
-        kd[e] = act[e] ? k_diag[map.row(s)] : 1.0;
+        kd[e] = act[e] ? P.k_diag[map.row(s)] : 1.0;
         sh.kd[s] = kd[e];
 #pragma unroll
         for (int w = 0; w < W; ++w) sh.a[w][s] = a;
     }
-    const double y = map.label(tid * 4);   // (a thread's four slots are of one group)
+    const double y = map.label(tid * E);   // (a thread's four slots are of one group)
     // (a vector that starts at an active slot may end in the columns behind the group's, which nothing uses, or up to
     // three elements behind the matrix)
-    const int col = act[0] ? map.row(tid * 4) : 0;
+    const int col = act[0] ? map.row(tid * E) : 0;
     double previous_diff = __builtin_inf(), last_diff = __builtin_inf(), second_last_diff = __builtin_inf(), diff = 0.0;
     int same_count = 0, swap_count = 0, iter = 0, status = 0;
     long long local_iter = 0;
@@ -475,7 +573,7 @@ __global__ __launch_bounds__(64 * W) void smo_small_kernel(const TB *K, int64_t 
     };
     if (start) {   // f from a non-zero alpha, in batches of 101 rows (csmosolver.cpp:189-214)
         const int n = make_list(N, [&](int s) { return map.active(s) ? -sh.a[wave][s] * map.label(s) : 0.0; }, [&](int s) { return map.row(s); });
-        for (int t = 0; t < n; t += 101) ss_update_f<W, TB>(sh, K, ld, col, t, t + 101 < n ? t + 101 : n, f);
+        for (int t = 0; t < n; t += 101) ss_update_f<E, W, TB>(sh, K, ld, col, t, t + 101 < n ? t + 101 : n, f);
         __syncthreads();
     }
     const int iter_end = iter + SS_MAX_ITER;
@@ -484,16 +582,16 @@ __global__ __launch_bounds__(64 * W) void smo_small_kernel(const TB *K, int64_t 
         // the working set: its second half moves to the front, q new ones follow (csmosolver.cpp:63-77)
         const int n_new = iter == 0 ? ws : q, first_new = iter == 0 ? 0 : ws - n_new;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sh.pos[tid * 4 + e] = 0xffff;
-        unsigned short kept[4];
+        for (int e = 0; e < E; ++e) sh.pos[tid * E + e] = 0xffff;
+        unsigned short kept[E];
 #pragma unroll
-        for (int h = 0; h < 4; ++h) {
+        for (int h = 0; h < E; ++h) {
             const int t = h * 64 * W + tid;
             kept[h] = iter > 0 && t < q ? sh.ws[t + q] : 0;
         }
         __syncthreads();
 #pragma unroll
-        for (int h = 0; h < 4; ++h) {
+        for (int h = 0; h < E; ++h) {
             const int t = h * 64 * W + tid;
             if (iter > 0 && t < q) {
                 sh.ws[t] = kept[h];
@@ -501,12 +599,10 @@ __global__ __launch_bounds__(64 * W) void smo_small_kernel(const TB *K, int64_t 
             }
         }
         __syncthreads();
-        uint64_t *skey = (uint64_t *) sh.f;
-        unsigned short *sidx = (unsigned short *) sh.k;
         unsigned member_all = 0;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int s = tid * 4 + e;
+        for (int e = 0; e < E; ++e) {
+            const int s = tid * E + e;
             const double a = sh.a[wave][s];
             unsigned b = 0;
             if (act[e]) {
@@ -515,25 +611,21 @@ __global__ __launch_bounds__(64 * W) void smo_small_kernel(const TB *K, int64_t 
             }
             member_all |= b << ((NU ? 4 : 2) * e);
             sh.flags[s] = (unsigned char) (sh.pos[s] == 0xffff ? b : 0u);
-            skey[s] = act[e] ? ss_key(f[e]) : ~0ull;
-            sidx[s] = (unsigned short) s;
         }
         __syncthreads();
-        if (!ss_select<W, NU>(sh, n_new, first_new)) {
+        if (!ss_select<E, W, NU>(sh, f, act, n_new, first_new)) {
             status = 2;
             break;
         }
         for (int t = tid; t < ws; t += 64 * W) sh.pos[sh.ws[t]] = (unsigned short) t;
         __syncthreads();
         unsigned member = 0;
-        int key[4];
-        double fl[4], a_old[4], mn[2] = {__builtin_inf(), __builtin_inf()}, mx[2] = {-__builtin_inf(), -__builtin_inf()};
+        double fl[E], a_old[E], mn[2] = {__builtin_inf(), __builtin_inf()}, mx[2] = {-__builtin_inf(), -__builtin_inf()};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int s = tid * 4 + e, p = sh.pos[s];
+        for (int e = 0; e < E; ++e) {
+            const int s = tid * E + e, p = sh.pos[s];
             const unsigned b = p != 0xffff ? (member_all >> ((NU ? 4 : 2) * e)) & (NU ? 15u : 3u) : 0u;
             member |= b << ((NU ? 4 : 2) * e);
-            key[e] = (p << 10 | s) & 0x7fffffff;
             fl[e] = f[e];
             a_old[e] = sh.a[wave][s];
 #pragma unroll
@@ -561,20 +653,22 @@ __global__ __launch_bounds__(64 * W) void smo_small_kernel(const TB *K, int64_t 
         const double tenth = NU ? 0.1 * diff : 0.1f * diff;   // (a float literal in the C variant, a double in the nu one)
         const double local_eps = eps > tenth ? eps : tenth;
         __syncthreads();
-        const int steps = ss_local<W, NU, TB>(sh, map, K, ld, col, kd, fl, member, key, P.Cp, P.Cn, local_eps, P.max_iter);
+        const int steps = __builtin_amdgcn_readfirstlane(local_eps > 0.0 ? 1 : 0)
+                              ? ss_local<E, W, NU, false, TB>(sh, map, K, ld, col, kd, fl, member, P.Cp, P.Cn, local_eps, P.max_iter)
+                              : ss_local<E, W, NU, true, TB>(sh, map, K, ld, col, kd, fl, member, P.Cp, P.Cn, local_eps, P.max_iter);
         inner_here += steps;
         if (!NU) local_iter += steps;   // (the nu variant reports none, smo_kernel.cpp:283)
         // alpha_diff of the working set, in its order: -(new - old) * y
         __syncthreads();
         double *const old = sh.k;   // (free between the local solver and the list)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) old[tid * 4 + e] = a_old[e];
+        for (int e = 0; e < E; ++e) old[tid * E + e] = a_old[e];
         __syncthreads();
-        double ad[4];
-        int rr[4], cnt = 0;
+        double ad[E];
+        int rr[E], cnt = 0;
 #pragma unroll
-        for (int h = 0; h < 4; ++h) {   // thread t owns entries 4t .. 4t + 3
-            const int t = tid * 4 + h;
+        for (int h = 0; h < E; ++h) {   // thread t owns entries E t .. E t + E - 1
+            const int t = tid * E + h;
             const int s = t < ws ? sh.ws[t] : 0;
             ad[h] = t < ws ? -(sh.a[wave][s] - old[s]) * map.label(s) : 0.0;
             rr[h] = map.row(s);
@@ -597,14 +691,14 @@ __global__ __launch_bounds__(64 * W) void smo_small_kernel(const TB *K, int64_t 
         }
         int *const rows = (int *) sh.k;
 #pragma unroll
-        for (int h = 0; h < 4; ++h)
+        for (int h = 0; h < E; ++h)
             if (ad[h] != 0.0) {
                 sh.f[at] = ad[h];
                 rows[at] = rr[h];
                 ++at;
             }
         __syncthreads();
-        ss_update_f<W, TB>(sh, K, ld, col, 0, n_list, f);
+        ss_update_f<E, W, TB>(sh, K, ld, col, 0, n_list, f);
         __syncthreads();
         // stall guards and stopping rule (csmosolver.cpp:86-111)
         if (__builtin_fabs(diff - previous_diff) < eps * 0.001) {
@@ -622,8 +716,8 @@ __global__ __launch_bounds__(64 * W) void smo_small_kernel(const TB *K, int64_t 
         ++iter;
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int s = tid * 4 + e;
+    for (int e = 0; e < E; ++e) {
+        const int s = tid * E + e;
         if (act[e]) {
             alpha[map.index(s)] = sh.a[wave][s];
             f_out[map.index(s)] = f[e];
@@ -644,44 +738,40 @@ __global__ __launch_bounds__(64 * W) void smo_small_kernel(const TB *K, int64_t 
     }
 }
 
-template <int W, typename TB>
-static void launch_small(bool nu, const void *k, int64_t ld, int n_rows, const double *k_diag, const tsvm_small_problem *problems, int n_problems,
-                         tsvm_small_state *states, int *ws, double *alpha, double *f, double eps, int out_max_iter, int start,
-                         hipStream_t stream) {
+template <int E, int W, typename TB>
+static void launch_small(const tsvm_small_problem *problems, int n_problems, tsvm_small_state *states, int *ws, double *alpha, double *f, int nu,
+                         double eps, int out_max_iter, int start, hipStream_t stream) {
+    const int grid = start ? (n_problems + 7) / 8 * 8 + 8 * SS_WARM_GROUPS : n_problems;
     if (nu)
-        smo_small_kernel<W, true, TB><<<n_problems, 64 * W, 0, stream>>>((const TB *) k, ld, n_rows, k_diag, problems, states, ws, alpha, f, eps,
-                                                                        out_max_iter, start);
+        smo_small_kernel<E, W, true, TB><<<grid, 64 * W, 0, stream>>>(problems, n_problems, states, ws, alpha, f, eps, out_max_iter, start);
     else
-        smo_small_kernel<W, false, TB><<<n_problems, 64 * W, 0, stream>>>((const TB *) k, ld, n_rows, k_diag, problems, states, ws, alpha, f, eps,
-                                                                         out_max_iter, start);
+        smo_small_kernel<E, W, false, TB><<<grid, 64 * W, 0, stream>>>(problems, n_problems, states, ws, alpha, f, eps, out_max_iter, start);
 }
 
 extern "C" {
 
 int tsvm_smo_small_max(void) { return SS_MAX; }
 
-int tsvm_smo_solve_small(const void *k, int row_type, int64_t ld, int n_rows, const double *k_diag, const tsvm_small_problem *problems,
-                         int n_problems, int max_slots, tsvm_small_state *states, int *ws, double *alpha, double *f, int nu, double eps,
-                         int out_max_iter, int start, tsvm_stream stream) {
+int tsvm_smo_solve_small(int row_type, const tsvm_small_problem *problems, int n_problems, int max_slots, tsvm_small_state *states, int *ws,
+                         double *alpha, double *f, int nu, double eps, int out_max_iter, int start, tsvm_stream stream) {
     TSVM_REQUIRE(row_type == TSVM_ROW_F32 || row_type == TSVM_ROW_F64, "tsvm_smo_solve_small: row type %d", row_type);
-    TSVM_REQUIRE(n_problems >= 0 && n_rows >= 0 && ld >= n_rows, "tsvm_smo_solve_small: %d problems, %d rows, stride %lld", n_problems, n_rows,
-                 (long long) ld);
+    TSVM_REQUIRE(n_problems >= 0, "tsvm_smo_solve_small: %d problems", n_problems);
     TSVM_REQUIRE(max_slots >= 1 && max_slots <= SS_MAX, "tsvm_smo_solve_small: %d slots (1 .. %d)", max_slots, SS_MAX);
     if (n_problems == 0) return 0;
-    TSVM_REQUIRE(n_rows > 0 && k && k_diag && problems && states && ws && alpha && f, "tsvm_smo_solve_small: null argument");
-    hipStream_t st = tsvm_s(stream);
-#define TSVM_SMALL(W, TB) \
-    launch_small<W, TB>(nu != 0, k, ld, n_rows, k_diag, problems, n_problems, states, ws, alpha, f, eps, out_max_iter, start, st)
-    // (as few wavefronts as hold the largest problem at four instances per thread: their barriers are what a step pays for)
-    if (row_type == TSVM_ROW_F32) {
-        if (max_slots <= 256) TSVM_SMALL(1, float);
-        else if (max_slots <= 512) TSVM_SMALL(2, float);
-        else TSVM_SMALL(4, float);
-    } else {
-        if (max_slots <= 256) TSVM_SMALL(1, double);
-        else if (max_slots <= 512) TSVM_SMALL(2, double);
-        else TSVM_SMALL(4, double);
-    }
+    TSVM_REQUIRE(problems && states && ws && alpha && f, "tsvm_smo_solve_small: null argument");
+#define TSVM_SMALL(E, W, TB) launch_small<E, W, TB>(problems, n_problems, states, ws, alpha, f, nu, eps, out_max_iter, start, tsvm_s(stream))
+    // (the shapes of the local solvers, smo_solve.hip, for the same reasons)
+#define TSVM_SMALL_T(TB)                                  \
+    do {                                                  \
+        if (max_slots <= 64) TSVM_SMALL(1, 1, TB);        \
+        else if (max_slots <= 128) TSVM_SMALL(2, 1, TB);  \
+        else if (max_slots <= 256) TSVM_SMALL(4, 1, TB);  \
+        else if (max_slots <= 512) TSVM_SMALL(4, 2, TB);  \
+        else TSVM_SMALL(4, 4, TB);                        \
+    } while (0)
+    if (row_type == TSVM_ROW_F32) TSVM_SMALL_T(float);
+    else TSVM_SMALL_T(double);
+#undef TSVM_SMALL_T
 #undef TSVM_SMALL
     TSVM_LAUNCH_CHECK();
     return 0;

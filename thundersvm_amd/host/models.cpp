@@ -107,18 +107,6 @@ void SvmModel::run_solver(CSMOSolver &solver, const KernelMatrix &k_mat, const s
                           std::vector<float_type> &alpha, float_type &rho_out, std::vector<float_type> &f_val,
                           float_type Cp, float_type Cn, size_t held_bytes) {
     const int ws = get_working_set_size(k_mat, held_bytes);
-    const size_t n_pos = std::find(y.begin(), y.end(), -1) - y.begin();
-    if (small_path_allowed() && SmallSolve::takes(n_pos, y.size() - n_pos, ws) &&
-        SmallSolve::takes_rows(k_mat.n_columns(), k_mat.row_elem_size())) {
-        std::vector<SmallSolve> one(1);
-        one[0] = {&solver, 0, (int) n_pos, k_mat.repeat() > 1 ? 0 : (int) n_pos, (int) (y.size() - n_pos), ws, Cp, Cn, &y, &alpha, &f_val, &rho_out};
-        SmallSolve::run(k_mat, one, param.epsilon, max_iter);
-        if (one[0].solved) {
-            solver_stats.push_back(one[0].stats);
-            if (keep_binary) binary_f.push_back(f_val);
-            return;
-        }
-    }
     solver.profile = profile;
     solver.cache_bytes = cache_bytes;
     solver.trace = solver_stats.empty() ? trace_first : nullptr;
@@ -127,13 +115,94 @@ void SvmModel::run_solver(CSMOSolver &solver, const KernelMatrix &k_mat, const s
     if (keep_binary) binary_f.push_back(f_val);
 }
 
+void SvmModel::train(const DataSet &dataset, SvmParam p) {
+    Training t = begin_training(dataset, p);
+    SmallBatch::run({&t.small}, param.epsilon, max_iter);
+    t.finish(t.small);
+}
+
+SvmModel::Training SvmModel::begin_single(std::shared_ptr<SingleProblem> s, std::function<void()> after) {
+    Training t;
+    const size_t n_pos = std::find(s->y.begin(), s->y.end(), -1) - s->y.begin();
+    if (small_path_allowed()) {
+        const int ws = get_working_set_size(*s->k_mat);
+        if (SmallSolve::takes(n_pos, s->y.size() - n_pos, ws) && SmallSolve::takes_rows(s->k_mat->n_columns(), s->k_mat->row_elem_size())) {
+            t.small.k_mat = s->k_mat;
+            t.small.solves.push_back({s->solver.get(), 0, (int) n_pos, s->k_mat->repeat() > 1 ? 0 : (int) n_pos, (int) (s->y.size() - n_pos), ws, s->Cp,
+                                      s->Cn, &s->y, &s->alpha, &s->f_val, &rho[0]});
+        }
+    }
+    t.finish = [this, s, after](SmallBatch &small) {
+        if (!small.solves.empty() && small.solves[0].solved) {
+            solver_stats.push_back(small.solves[0].stats);
+            if (keep_binary) binary_f.push_back(s->f_val);
+        } else {
+            run_solver(*s->solver, *s->k_mat, s->y, s->alpha, rho[0], s->f_val, s->Cp, s->Cn);
+        }
+        after();
+    };
+    return t;
+}
+
+void SvmModel::copy_settings(const SvmModel &other) {
+    ws_override = other.ws_override;
+    profile = other.profile;
+    cache_bytes = other.cache_bytes;
+    pair_lanes = other.pair_lanes;
+    max_iter = other.max_iter;
+}
+
+// The dataset's rows go to the device once; every fold takes its rows, its support vectors and the rows it is applied to
+// from there.  Folds whose problems are small (SmallBatch) are set up first and solved together.
+void SvmModel::train_folds(const DataSet &dataset, const std::vector<Fold> &folds, const SvmParam &p, const std::function<SvmModel &(size_t)> &model_of,
+                           const std::function<void(size_t, SvmModel &, std::vector<float_type> &)> &take) {
+    const std::shared_ptr<DeviceRows> all = dataset.device_cache() ? std::static_pointer_cast<DeviceRows>(dataset.device_cache())
+                                                                   : DeviceRows::from_host(dataset.rows());
+    const auto rows_of = [&](const std::vector<int> &ids, const std::vector<float_type> &y) {
+        std::unique_ptr<DataSet> d(new DataSet(dataset.rows().gather(ids.data(), ids.size()), (int) dataset.n_features(), y));
+        d->device_cache() = DeviceRows::subset(*all, ids.data(), ids.size());
+        return d;
+    };
+    struct Begun {
+        size_t k;
+        SvmModel *model;
+        std::unique_ptr<DataSet> rows;
+        Training training;
+    };
+    constexpr size_t ROWS_AT_ONCE = 65536;   // (what the folds in flight hold on the host and the device grows with their rows)
+    for (size_t k = 0; k < folds.size();) {
+        std::vector<Begun> begun;
+        size_t rows = 0;
+        do {
+            begun.push_back({k, &model_of(k), rows_of(folds[k].train_idx, folds[k].y_train), {}});
+            begun.back().training = begun.back().model->begin_training(*begun.back().rows, p);
+            rows += folds[k].train_idx.size();
+            ++k;
+        } while (k < folds.size() && rows < ROWS_AT_ONCE && !begun.back().training.small.solves.empty());
+        std::vector<SmallBatch *> batches;
+        for (Begun &b : begun) batches.push_back(&b.training.small);
+        SmallBatch::run(batches, begun[0].model->param.epsilon, begun[0].model->max_iter);
+        for (Begun &b : begun) {
+            SvmModel &m = *b.model;
+            b.training.finish(b.training.small);
+            if (!m.sv_indices.empty()) m.sv_k_mat.reset(new KernelMatrix(*b.rows, m.sv_indices.data(), m.sv_indices.size(), m.param));
+            const std::unique_ptr<DataSet> test = rows_of(folds[b.k].test_idx, {});
+            std::vector<float_type> dec;
+            m.predict_dec_values(*test, dec, 1000);
+            take(b.k, m, dec);
+            b.training = Training();
+            b.rows.reset();
+        }
+    }
+}
+
 // Stratified folds in class order (svmmodel.cpp:31-71).
 std::vector<float_type> SvmModel::cross_validation(DataSet dataset, SvmParam p, int n_fold) {
     dataset.group_classes(this->param.svm_type == SvmParam::C_SVC);
     std::vector<float_type> y_predict_all(dataset.n_instances());
+    std::vector<Fold> folds(std::max(n_fold, 0));
     for (int k = 0; k < n_fold; ++k) {
-        std::vector<float_type> y_train;
-        std::vector<int> train_idx, test_idx;
+        Fold &f = folds[k];
         for (size_t c = 0; c < dataset.n_classes(); ++c) {
             const int fold = dataset.count()[c] / n_fold;
             const std::vector<int> ids = dataset.original_index((int) c);
@@ -141,19 +210,28 @@ std::vector<float_type> SvmModel::cross_validation(DataSet dataset, SvmParam p, 
             const size_t hi = (k == n_fold - 1) ? ids.size() : std::min(ids.size(), lo + fold);
             for (size_t t = 0; t < ids.size(); ++t) {
                 if (t >= lo && t < hi) {
-                    test_idx.push_back(ids[t]);
+                    f.test_idx.push_back(ids[t]);
                 } else {
-                    train_idx.push_back(ids[t]);
-                    y_train.push_back(dataset.y()[ids[t]]);
+                    f.train_idx.push_back(ids[t]);
+                    f.y_train.push_back(dataset.y()[ids[t]]);
                 }
             }
         }
-        DataSet train_set(dataset.rows().gather(train_idx.data(), train_idx.size()), (int) dataset.n_features(), y_train);
-        this->train(train_set, p);
-        predict_dec_values(*dataset.rows().gather(test_idx.data(), test_idx.size()), dec_values, 1000);
-        std::vector<float_type> y_predict = finish_predict((int) test_idx.size());
-        for (size_t i = 0; i < y_predict.size(); ++i) y_predict_all[test_idx[i]] = y_predict[i];
     }
+    // (this model is the last fold's afterwards, as after training them one by one)
+    std::vector<std::unique_ptr<SvmModel>> others(folds.size());
+    const auto model_of = [&](size_t k) -> SvmModel & {
+        if (k + 1 == folds.size()) return *this;
+        others[k] = make_model(this->svm_type());
+        others[k]->copy_settings(*this);
+        return *others[k];
+    };
+    train_folds(dataset, folds, p, model_of, [&](size_t k, SvmModel &m, std::vector<float_type> &dec) {
+        m.dec_values.swap(dec);
+        const std::vector<float_type> y_predict = m.finish_predict((int) folds[k].test_idx.size());
+        for (size_t i = 0; i < y_predict.size(); ++i) y_predict_all[folds[k].test_idx[i]] = y_predict[i];
+        others[k].reset();
+    });
     return y_predict_all;
 }
 
@@ -391,24 +469,44 @@ void SVC::model_setup(const DataSet &dataset, SvmParam &p) {   // svc.cpp:16-39
     }
 }
 
-void SVC::train(const DataSet &dataset, SvmParam p) {   // svc.cpp:41-145
+SvmModel::Training SVC::begin_training(const DataSet &dataset, SvmParam p) {   // svc.cpp:41-145
     // the reference groups a copy of the data set (svc.cpp:42-43); grouping only reads y, so the copy
     // here shares nothing but the labels and the instances are referenced in place
-    DataSet grouped = dataset.grouped_view();
-    model_setup(grouped, p);
+    auto grouped = std::make_shared<DataSet>(dataset.grouped_view());
+    model_setup(*grouped, p);
+    Training t;
+    auto small = std::make_shared<std::vector<BinaryProblem>>(small_pairs(*grouped, t.small));
+    t.finish = [this, grouped, small](SmallBatch &batch) { finish_training(*grouped, *small, batch); };
+    return t;
+}
+
+void SVC::finish_training(const DataSet &grouped, std::vector<BinaryProblem> &small, SmallBatch &batch) {
     const int n = (int) grouped.n_instances();
     std::vector<std::vector<float_type>> alpha(n_binary_models);
-    std::vector<char> is_sv(n, 0);
-    int k = 0;
+    std::vector<char> is_sv(n, 0), done(n_binary_models, 0);
+    for (size_t s = 0; s < small.size(); ++s) {
+        if (!batch.solves[s].solved) continue;
+        const int k = small[s].k;
+        solver_stats.resize(n_binary_models);
+        if (keep_binary) binary_f.resize(n_binary_models);
+        done[k] = 1;
+        solver_stats[k] = batch.solves[s].stats;
+        if (keep_binary) binary_f[k] = small[s].f_val;
+        finish_binary(small[s], alpha[k]);
+    }
+    batch.k_mat.reset();
+    const bool all_done = std::all_of(done.begin(), done.end(), [](char d) { return d != 0; });
     // pairs in flight: up to eight when every pair's solver gets a CU of its own and the pairs advance independently
     // (train_pairs_in_lockstep), three when the pairs alternate between a solver phase and a chip-wide phase
     const int lanes = std::min(pair_lanes > 0 ? pair_lanes : SolveTask::cu_split_available() ? 8 : 3, n_binary_models);
-    if (lanes > 1 && !profile && !trace_first) {
-        solver_stats.assign(n_binary_models, SolverStats());
-        if (keep_binary) binary_f.assign(n_binary_models, std::vector<float_type>());
-        train_pairs_in_lockstep(grouped, lanes, alpha, train_small_pairs(grouped, alpha));
-    } else {
+    if (all_done) {
+    } else if (lanes > 1 && !profile && !trace_first) {
+        solver_stats.resize(n_binary_models);
+        if (keep_binary) binary_f.resize(n_binary_models);
+        train_pairs_in_lockstep(grouped, lanes, alpha, done);
+    } else {   // (small pairs are left to this path only together)
         size_t held = 0;   // alpha arrays of the pairs already trained (svc.cpp:50-61 keeps them to the end)
+        int k = 0;
         for (int i = 0; i < n_classes; ++i)
             for (int j = i + 1; j < n_classes; ++j, ++k) {
                 BinaryProblem p;
@@ -424,7 +522,8 @@ void SVC::train(const DataSet &dataset, SvmParam p) {   // svc.cpp:41-145
     std::vector<std::pair<int, int>> pair_of;
     for (int i = 0; i < n_classes; ++i)
         for (int j = i + 1; j < n_classes; ++j) pair_of.push_back({i, j});
-#pragma omp parallel for schedule(dynamic, 1)
+    const int threads = threads_for((size_t) n * (n_classes - 1));
+#pragma omp parallel for schedule(dynamic, 1) num_threads(threads)
     for (int kk = 0; kk < n_binary_models; ++kk) {
         const std::vector<int> ids = grouped.original_index(pair_of[kk].first, pair_of[kk].second);
         for (size_t l = 0; l < ids.size(); ++l)
@@ -446,7 +545,7 @@ void SVC::train(const DataSet &dataset, SvmParam p) {   // svc.cpp:41-145
     coef.assign((size_t) (n_classes - 1) * n_total_sv, 0);
     std::vector<int> sv_start(n_classes, 0);
     for (int c = 1; c < n_classes; ++c) sv_start[c] = sv_start[c - 1] + n_sv[c - 1];
-#pragma omp parallel for schedule(dynamic, 1)
+#pragma omp parallel for schedule(dynamic, 1) num_threads(threads)
     for (int kk = 0; kk < n_binary_models; ++kk) {   // (every pair writes two segments of coef that no other pair writes)
         const int i = pair_of[kk].first, j = pair_of[kk].second;
         const std::vector<int> ids = grouped.original_index(i, j);
@@ -461,7 +560,7 @@ void SVC::train(const DataSet &dataset, SvmParam p) {   // svc.cpp:41-145
     if (param.kernel_type == SvmParam::LINEAR) {   // explicit w per pair (svc.cpp:111-135)
         const size_t nf = grouped.n_features();
         linear_coef.assign((size_t) n_binary_models * (grouped.is_zero_based() ? nf + 1 : nf), 0);
-        k = 0;
+        int k = 0;
         for (int i = 0; i < n_classes; ++i)
             for (int j = i + 1; j < n_classes; ++j, ++k) {
                 const std::vector<int> ids = grouped.original_index(i, j);
@@ -512,18 +611,19 @@ void SVC::finish_binary(BinaryProblem &p, std::vector<float_type> &alpha_out) { 
     alpha_out = std::move(p.alpha);
 }
 
-// Pairs that fit one workgroup each (smo_small.hip) are solved side by side from one kernel matrix of their classes' rows.
-std::vector<char> SVC::train_small_pairs(const DataSet &grouped, std::vector<std::vector<float_type>> &alpha) {
-    std::vector<char> done(n_binary_models, 0);
-    if (!small_path_allowed() || pair_lanes > 0) return done;
+// Pairs that fit one workgroup each (smo_small.hip), with one kernel matrix of their classes' rows.
+std::vector<SVC::BinaryProblem> SVC::small_pairs(const DataSet &grouped, SmallBatch &batch) {
+    std::vector<BinaryProblem> problems;
+    if (!small_path_allowed() || pair_lanes > 0) return problems;
     struct Pair { int i, j, k, ws; };
     std::vector<Pair> small;
     std::vector<char> needed(n_classes, 0);
-    size_t held = 0;   // (as in train())
+    size_t held = 0;   // alpha arrays of the pairs before (svc.cpp:50-61 keeps them to the end)
     for (int i = 0, k = 0; i < n_classes; ++i)
         for (int j = i + 1; j < n_classes; ++j, ++k) {
             const size_t ci = grouped.count()[i], cj = grouped.count()[j];
-            const int ws = working_set_size_of_shape(ci + cj, grouped.n_features() + 1, std::min(grouped.rows().nnz(), (ci + cj) * (grouped.n_features() + 1)), held);
+            const size_t nf = grouped.n_features() + 1, entries = std::min(grouped.rows().nnz(), (ci + cj) * nf);
+            const int ws = working_set_size_of_shape(ci + cj, nf, entries, held);
             held += (ci + cj) * sizeof(float_type);
             if (!SmallSolve::takes(ci, cj, ws)) continue;
             small.push_back({i, j, k, ws});
@@ -536,27 +636,18 @@ std::vector<char> SVC::train_small_pairs(const DataSet &grouped, std::vector<std
         const std::vector<int> of_class = grouped.original_index(c);
         ids.insert(ids.end(), of_class.begin(), of_class.end());
     }
-    if (small.empty() || !SmallSolve::takes_rows(ids.size(), param.kernel_type == SvmParam::LINEAR ? sizeof(double) : sizeof(float))) return done;
-    const KernelMatrix k_mat(grouped, ids.data(), ids.size(), param);
-    std::vector<BinaryProblem> problems(small.size());
-    std::vector<SmallSolve> solves(small.size());
+    if (small.empty() || !SmallSolve::takes_rows(ids.size(), param.kernel_type == SvmParam::LINEAR ? sizeof(double) : sizeof(float))) return problems;
+    batch.k_mat = std::make_shared<KernelMatrix>(grouped, ids.data(), ids.size(), param);
+    problems.resize(small.size());
     for (size_t s = 0; s < small.size(); ++s) {
         const Pair &q = small[s];
         BinaryProblem &p = problems[s];
         p.k = q.k;
         setup_binary(grouped, q.i, q.j, p);
-        solves[s] = {p.solver.get(), first_row[q.i], grouped.count()[q.i], first_row[q.j], grouped.count()[q.j], q.ws, p.Cp, p.Cn, &p.y, &p.alpha, &p.f_val, &rho[q.k]};
+        batch.solves.push_back({p.solver.get(), first_row[q.i], grouped.count()[q.i], first_row[q.j], grouped.count()[q.j], q.ws, p.Cp, p.Cn, &p.y,
+                                &p.alpha, &p.f_val, &rho[q.k]});
     }
-    SmallSolve::run(k_mat, solves, param.epsilon, max_iter);
-    for (size_t s = 0; s < small.size(); ++s) {
-        if (!solves[s].solved) continue;
-        const int k = small[s].k;
-        done[k] = 1;
-        solver_stats[k] = solves[s].stats;
-        if (keep_binary) binary_f[k] = problems[s].f_val;
-        finish_binary(problems[s], alpha[k]);
-    }
-    return done;
+    return problems;
 }
 
 // The class pairs are independent problems.  Up to `lanes` of them are in flight, each a SolveTask with its own
@@ -582,7 +673,6 @@ void SVC::train_pairs_in_lockstep(const DataSet &grouped, int lanes, std::vector
     std::vector<PairId> pairs;
     for (int i = 0; i < n_classes; ++i)
         for (int j = i + 1; j < n_classes; ++j) pairs.push_back({i, j});
-    if (std::all_of(done.begin(), done.end(), [](char d) { return d != 0; })) return;
     const size_t esz = param.kernel_type == SvmParam::LINEAR ? sizeof(double) : sizeof(float);
     tsvm::RowArena &arena = tsvm::RowArena::instance();
     const size_t budget = cache_bytes > 0 ? (size_t) cache_bytes : cache_bytes < 0 ? arena.auto_budget() : 0;
@@ -904,9 +994,9 @@ void SVC::probability_train(const DataSet &grouped) {
     param_no_prob.probability = 0;
     const int n_fold = 5;
     std::vector<float_type> dec_all(grouped.n_instances() * (size_t) n_binary_models);
+    std::vector<Fold> folds(n_fold);
     for (int fold = 0; fold < n_fold; ++fold) {
-        std::vector<float_type> y_train;
-        std::vector<int> train_idx, test_idx;
+        Fold &f = folds[fold];
         for (size_t c = 0; c < grouped.n_classes(); ++c) {
             const std::vector<int> ids = grouped.original_index((int) c);
             const size_t per_fold = ids.size() / n_fold;
@@ -914,24 +1004,29 @@ void SVC::probability_train(const DataSet &grouped) {
             const size_t end = fold == n_fold - 1 ? ids.size() : std::min(ids.size(), begin + per_fold);
             for (size_t l = 0; l < ids.size(); ++l) {
                 if (l >= begin && l < end) {
-                    test_idx.push_back(ids[l]);
+                    f.test_idx.push_back(ids[l]);
                 } else {
-                    train_idx.push_back(ids[l]);
-                    y_train.push_back(grouped.y()[ids[l]]);
+                    f.train_idx.push_back(ids[l]);
+                    f.y_train.push_back(grouped.y()[ids[l]]);
                 }
             }
         }
-        SVC fold_model;
-        fold_model.set_max_iter(max_iter);
-        fold_model.cache_bytes = cache_bytes;
-        fold_model.pair_lanes = pair_lanes;
-        fold_model.train(DataSet(grouped.rows().gather(train_idx.data(), train_idx.size()), (int) grouped.n_features(), y_train), param_no_prob);
-        std::vector<float_type> dec;
-        fold_model.predict_dec_values(*grouped.rows().gather(test_idx.data(), test_idx.size()), dec, 1000);
+    }
+    std::vector<std::unique_ptr<SVC>> models(n_fold);
+    const auto model_of = [&](size_t fold) -> SvmModel & {
+        models[fold].reset(new SVC());
+        models[fold]->set_max_iter(max_iter);
+        models[fold]->cache_bytes = cache_bytes;
+        models[fold]->pair_lanes = pair_lanes;
+        return *models[fold];
+    };
+    train_folds(grouped, folds, param_no_prob, model_of, [&](size_t fold, SvmModel &, std::vector<float_type> &dec) {
+        const std::vector<int> &test_idx = folds[fold].test_idx;
         for (size_t t = 0; t < test_idx.size(); ++t)
             std::copy(dec.begin() + t * n_binary_models, dec.begin() + (t + 1) * n_binary_models,
                       dec_all.begin() + (size_t) test_idx[t] * n_binary_models);
-    }
+        models[fold].reset();
+    });
     int k = 0;
     for (int i = 0; i < n_classes; ++i)
         for (int j = i + 1; j < n_classes; ++j, ++k) {
@@ -1022,20 +1117,26 @@ void SVR::model_setup(const DataSet &dataset, SvmParam &p) {
     param.svm_type = SvmParam::EPSILON_SVR;
 }
 
-void SVR::train(const DataSet &dataset, SvmParam p) {
+SvmModel::Training SVR::begin_training(const DataSet &dataset, SvmParam p) {   // svr.cpp:9-41
     model_setup(dataset, p);
     const int n = (int) dataset.n_instances();
-    KernelMatrix k_mat(dataset, nullptr, n, param, 2);
-    std::vector<float_type> f_val(2 * (size_t) n), alpha_2(2 * (size_t) n, 0);
-    std::vector<int> y(2 * (size_t) n);
+    auto s = std::make_shared<SingleProblem>();
+    s->k_mat = std::make_shared<KernelMatrix>(dataset, nullptr, n, param, 2);
+    s->solver.reset(new CSMOSolver());
+    s->f_val.resize(2 * (size_t) n);
+    s->alpha.assign(2 * (size_t) n, 0);
+    s->y.resize(2 * (size_t) n);
     for (int i = 0; i < n; ++i) {
-        f_val[i] = param.p - dataset.y()[i];
-        y[i] = +1;
-        f_val[i + n] = -param.p - dataset.y()[i];
-        y[i + n] = -1;
+        s->f_val[i] = param.p - dataset.y()[i];
+        s->y[i] = +1;
+        s->f_val[i + n] = -param.p - dataset.y()[i];
+        s->y[i + n] = -1;
     }
-    CSMOSolver solver;
-    run_solver(solver, k_mat, y, alpha_2, rho[0], f_val, param.C, param.C);
+    s->Cp = s->Cn = param.C;
+    return begin_single(s, [this, s, &dataset] { finish_svr(s->alpha, dataset); });
+}
+
+void SVR::finish_svr(const std::vector<float_type> &alpha_2, const DataSet &dataset) {
     if (keep_binary) binary_alpha.push_back(alpha_2);
     save_svr_coef(alpha_2, dataset.rows());
     if (param.kernel_type == SvmParam::LINEAR) compute_linear_coef_single_model(dataset.n_features(), dataset.is_zero_based());
@@ -1062,25 +1163,25 @@ void NuSVR::model_setup(const DataSet &dataset, SvmParam &p) {
     param.svm_type = SvmParam::NU_SVR;
 }
 
-void NuSVR::train(const DataSet &dataset, SvmParam p) {   // nusvr.cpp:7-41
+SvmModel::Training NuSVR::begin_training(const DataSet &dataset, SvmParam p) {   // nusvr.cpp:7-41
     model_setup(dataset, p);
     const int n = (int) dataset.n_instances();
-    KernelMatrix k_mat(dataset, nullptr, n, param, 2);
-    std::vector<float_type> f_val(2 * (size_t) n), alpha_2(2 * (size_t) n);
-    std::vector<int> y(2 * (size_t) n);
+    auto s = std::make_shared<SingleProblem>();
+    s->k_mat = std::make_shared<KernelMatrix>(dataset, nullptr, n, param, 2);
+    s->solver.reset(new NuSMOSolver(true));
+    s->f_val.resize(2 * (size_t) n);
+    s->alpha.resize(2 * (size_t) n);
+    s->y.resize(2 * (size_t) n);
     float_type sum = param.C * param.nu * n / 2;
     for (int i = 0; i < n; ++i) {
-        alpha_2[i] = alpha_2[i + n] = std::min(sum, param.C);
-        sum -= alpha_2[i];
-        f_val[i] = f_val[i + n] = -dataset.y()[i];
-        y[i] = +1;
-        y[i + n] = -1;
+        s->alpha[i] = s->alpha[i + n] = std::min(sum, param.C);
+        sum -= s->alpha[i];
+        s->f_val[i] = s->f_val[i + n] = -dataset.y()[i];
+        s->y[i] = +1;
+        s->y[i + n] = -1;
     }
-    NuSMOSolver solver(true);
-    run_solver(solver, k_mat, y, alpha_2, rho[0], f_val, param.C, param.C);
-    if (keep_binary) binary_alpha.push_back(alpha_2);
-    save_svr_coef(alpha_2, dataset.rows());
-    if (param.kernel_type == SvmParam::LINEAR) compute_linear_coef_single_model(dataset.n_features(), dataset.is_zero_based());
+    s->Cp = s->Cn = param.C;
+    return begin_single(s, [this, s, &dataset] { finish_svr(s->alpha, dataset); });
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1092,17 +1193,23 @@ void OneClassSVC::model_setup(const DataSet &dataset, SvmParam &p) {
     param.svm_type = SvmParam::ONE_CLASS;
 }
 
-void OneClassSVC::train(const DataSet &dataset, SvmParam p) {
+SvmModel::Training OneClassSVC::begin_training(const DataSet &dataset, SvmParam p) {   // oneclass_svc.cpp:12-52
     model_setup(dataset, p);
     const int n = (int) dataset.n_instances();
-    KernelMatrix k_mat(dataset, nullptr, n, param);
-    std::vector<float_type> alpha(n, 0), f_val(n, 0);
-    std::vector<int> y(n, 1);
+    auto s = std::make_shared<SingleProblem>();
+    s->k_mat = std::make_shared<KernelMatrix>(dataset, nullptr, n, param);
+    s->solver.reset(new CSMOSolver());
+    s->alpha.assign(n, 0);
+    s->f_val.assign(n, 0);
+    s->y.assign(n, 1);
     const int full = static_cast<int>(param.nu * n);
-    for (int i = 0; i < full; ++i) alpha[i] = 1;
-    if (full < n) alpha[full] = param.nu * n - full;
-    CSMOSolver solver;
-    run_solver(solver, k_mat, y, alpha, rho[0], f_val, 1, 1);
+    for (int i = 0; i < full; ++i) s->alpha[i] = 1;
+    if (full < n) s->alpha[full] = param.nu * n - full;
+    return begin_single(s, [this, s, &dataset] { finish_one_class(s->alpha, dataset); });
+}
+
+void OneClassSVC::finish_one_class(const std::vector<float_type> &alpha, const DataSet &dataset) {
+    const int n = (int) dataset.n_instances();
     if (keep_binary) binary_alpha.push_back(alpha);
     for (int i = 0; i < n; ++i)
         if (alpha[i] != 0) {

@@ -3,6 +3,7 @@
 // file.  Public surface of include/thundersvm/model/{svmmodel,svc,nusvc,oneclass_svc,svr,nusvr}.h;
 // kernel evaluation and the SMO solve run on the GPU through KernelMatrix / CSMOSolver.
 #pragma once
+#include <functional>
 #include <memory>
 
 #include "dataset.h"
@@ -13,7 +14,7 @@
 class SvmModel {
 public:
     virtual ~SvmModel() = default;
-    virtual void train(const DataSet &dataset, SvmParam param) = 0;
+    void train(const DataSet &dataset, SvmParam param);
     std::vector<float_type> predict(const DataSet::node2d &instances, int batch_size = -1);
     void predict_dec_values(const RowStore &rows, std::vector<float_type> &dec_values, int batch_size) const;
     // The same for the instances of a DataSet; when the DataSet has a device-resident copy of its rows in the dense
@@ -61,6 +62,33 @@ public:
 
 protected:
     virtual void model_setup(const DataSet &dataset, SvmParam &param);
+    // A training call in two halves, so that the small problems of several calls can be solved side by side: begin_training
+    // sets up the model and leaves in `small` what SmallBatch::run can solve, finish() solves the rest and makes the
+    // model of the solutions.  (`dataset` has to live until then.)
+    struct Training {
+        SmallBatch small;
+        std::function<void(SmallBatch &)> finish;
+    };
+    virtual Training begin_training(const DataSet &dataset, SvmParam param) = 0;
+    virtual SvmParam::SVM_TYPE svm_type() const = 0;
+    // The folds of a cross-validation: the instances trained on, in this order, with their labels, and the others.
+    struct Fold {
+        std::vector<int> train_idx, test_idx;
+        std::vector<float_type> y_train;
+    };
+    // trains model_of(k) on fold k of the dataset's instances and hands it over with the decision values of the others
+    static void train_folds(const DataSet &dataset, const std::vector<Fold> &folds, const SvmParam &param, const std::function<SvmModel &(size_t)> &model_of,
+                            const std::function<void(size_t, SvmModel &, std::vector<float_type> &)> &take);
+    void copy_settings(const SvmModel &other);
+    // the two halves for a model of one binary problem
+    struct SingleProblem {
+        std::shared_ptr<KernelMatrix> k_mat;
+        std::unique_ptr<CSMOSolver> solver;
+        std::vector<int> y;
+        std::vector<float_type> alpha, f_val;
+        float_type Cp = 1, Cn = 1;
+    };
+    Training begin_single(std::shared_ptr<SingleProblem> problem, std::function<void()> after);
     // what predict returns once dec_values holds the decision values of n_instances rows: the values themselves,
     // class labels (SVC) or the side of the boundary (OneClassSVC)
     virtual std::vector<float_type> finish_predict(int n_instances) { return dec_values; }
@@ -102,10 +130,9 @@ protected:
 };
 
 class SVC : public SvmModel {
-public:
-    void train(const DataSet &dataset, SvmParam param) override;
-
 protected:
+    Training begin_training(const DataSet &dataset, SvmParam param) override;
+    SvmParam::SVM_TYPE svm_type() const override { return SvmParam::C_SVC; }
     void model_setup(const DataSet &dataset, SvmParam &param) override;
     std::vector<float_type> finish_predict(int n_instances) override;
     // One class pair (i, j) of the one-vs-one decomposition: its rows, labels, starting point and solver.
@@ -124,8 +151,9 @@ protected:
     };
     virtual void setup_binary(const DataSet &dataset, int i, int j, BinaryProblem &p);   // svc.cpp:147-170 (without the rows)
     void take_rows(const DataSet &dataset, BinaryProblem &p);
-    // solves the small pairs side by side; which ones were (each then has its stats, alpha and rho)
-    std::vector<char> train_small_pairs(const DataSet &grouped, std::vector<std::vector<float_type>> &alpha);
+    // the pairs that SmallBatch::run takes: their problems and, in the batch, their kernel matrix and solves
+    std::vector<BinaryProblem> small_pairs(const DataSet &grouped, SmallBatch &batch);
+    void finish_training(const DataSet &grouped, std::vector<BinaryProblem> &small, SmallBatch &batch);
     void finish_binary(BinaryProblem &p, std::vector<float_type> &alpha_out);            // svc.cpp:171-177
     void train_pairs_in_lockstep(const DataSet &grouped, int lanes, std::vector<std::vector<float_type>> &alpha, const std::vector<char> &done);
     std::vector<float_type> predict_label(const std::vector<float_type> &dec_values, int n_instances);
@@ -136,33 +164,33 @@ protected:
 
 class NuSVC : public SVC {
 protected:
+    SvmParam::SVM_TYPE svm_type() const override { return SvmParam::NU_SVC; }
     void model_setup(const DataSet &dataset, SvmParam &param) override;
     void setup_binary(const DataSet &dataset, int i, int j, BinaryProblem &p) override;
 };
 
 class SVR : public SvmModel {
-public:
-    void train(const DataSet &dataset, SvmParam param) override;
-
 protected:
+    Training begin_training(const DataSet &dataset, SvmParam param) override;
+    SvmParam::SVM_TYPE svm_type() const override { return SvmParam::EPSILON_SVR; }
     void model_setup(const DataSet &dataset, SvmParam &param) override;
+    void finish_svr(const std::vector<float_type> &alpha_2, const DataSet &dataset);
     void save_svr_coef(const std::vector<float_type> &alpha_2, const RowStore &rows);
 };
 
 class NuSVR : public SVR {
-public:
-    void train(const DataSet &dataset, SvmParam param) override;
-
 protected:
+    Training begin_training(const DataSet &dataset, SvmParam param) override;
+    SvmParam::SVM_TYPE svm_type() const override { return SvmParam::NU_SVR; }
     void model_setup(const DataSet &dataset, SvmParam &param) override;
 };
 
 class OneClassSVC : public SvmModel {
-public:
-    void train(const DataSet &dataset, SvmParam param) override;
-
 protected:
+    Training begin_training(const DataSet &dataset, SvmParam param) override;
+    SvmParam::SVM_TYPE svm_type() const override { return SvmParam::ONE_CLASS; }
     void model_setup(const DataSet &dataset, SvmParam &param) override;
+    void finish_one_class(const std::vector<float_type> &alpha, const DataSet &dataset);
     std::vector<float_type> finish_predict(int n_instances) override;
 };
 

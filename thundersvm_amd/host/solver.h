@@ -2,6 +2,7 @@
 // nusmosolver.cpp) driving the gfx950 kernels.  f, alpha, y, the working set and the ws x n kernel
 // rows stay in HBM for the whole solve; per outer iteration the host reads back 16 bytes (diff).
 #pragma once
+#include <memory>
 #include <string>
 #include "kernelmatrix.h"
 
@@ -58,7 +59,7 @@ public:
 
 protected:
     friend class SolveTask;
-    friend struct SmallSolve;
+    friend struct SmallBatch;
     virtual bool is_nu() const { return false; }
     virtual float_type calculate_rho(const std::vector<float_type> &f_val, const std::vector<int> &y,
                                      std::vector<float_type> &alpha, float_type Cp, float_type Cn) const;
@@ -126,10 +127,10 @@ private:
     Impl *impl_;
 };
 
-// One of several small problems that are solved by one kernel launch from one kernel matrix (smo_small.hip): its y = +1
-// instances are n_pos rows of the matrix from row_pos on, its y = -1 instances n_neg rows from row_neg on.
+// One of several small problems that are solved by one kernel launch (smo_small.hip): its y = +1 instances are n_pos rows
+// of the batch's kernel matrix from row_pos on, its y = -1 instances n_neg rows from row_neg on.
 struct SmallSolve {
-    const CSMOSolver *solver;   // (all problems of a run: the same kind)
+    const CSMOSolver *solver;
     int row_pos, n_pos, row_neg, n_neg, ws_size;
     float_type Cp, Cn;
     const std::vector<int> *y;
@@ -141,6 +142,14 @@ struct SmallSolve {
     static size_t slots(size_t n_pos, size_t n_neg);
     static bool takes(size_t n_pos, size_t n_neg, int ws_size);
     static bool takes_rows(size_t n_rows, size_t elem_size);
-    static void run(const KernelMatrix &k_mat, std::vector<SmallSolve> &problems, float_type eps, int out_max_iter);
+};
+struct SmallBatch {             // problems with rows in one kernel matrix
+    std::shared_ptr<const KernelMatrix> k_mat;
+    std::vector<SmallSolve> solves;
+    // Solves every problem of all batches, side by side as far as the row arena holds their matrices.  (All of one kind: C or
+    // nu, and the same type of kernel row.)
+    static void run(const std::vector<SmallBatch *> &batches, float_type eps, int out_max_iter);
+    static bool is_nu(const SmallSolve &s) { return s.solver->is_nu(); }
+    static void set_results(SmallSolve &s, long long n_iter, long long local_iter);   // rho and the statistics, once alpha and f are there
 };
 double ms_since_first_solve();   // the clock that SolverStats::ms_start and ms_end are read on

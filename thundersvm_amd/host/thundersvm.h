@@ -20,4 +20,5 @@ struct Log {
     ~Log() { if (enabled()) std::cerr << os.str() << std::endl; }
 };
 }  // namespace tsvm
-#define TSVM_LOG ::tsvm::Log().os
+// (a stream that nobody reads costs a microsecond to make)
+#define TSVM_LOG if (!::tsvm::Log::enabled()) {} else ::tsvm::Log().os
