@@ -160,7 +160,7 @@ void SvmModel::train_folds(const DataSet &dataset, const std::vector<Fold> &fold
                                                                    : DeviceRows::from_host(dataset.rows());
     const auto rows_of = [&](const std::vector<int> &ids, const std::vector<float_type> &y) {
         std::unique_ptr<DataSet> d(new DataSet(dataset.rows().gather(ids.data(), ids.size()), (int) dataset.n_features(), y));
-        d->device_cache() = DeviceRows::subset(*all, ids.data(), ids.size());
+        if (!ids.empty()) d->device_cache() = DeviceRows::subset(*all, ids.data(), ids.size());
         return d;
     };
     struct Begun {
