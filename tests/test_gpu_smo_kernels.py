@@ -181,6 +181,49 @@ def test_local_solver_at_the_edges_of_its_variants(ws, nu, start):
         assert np.array_equal(G.host(ad_d), ad_want, equal_nan=True)
 
 
+@pytest.mark.parametrize("ws", [257, 512, 513, 1024])
+@pytest.mark.parametrize("scores", ["apart by 1e-9", "apart by 1e-6", "pairs of equals", "negative a", "f times 1e-25", "f times 1e15", "some a are 0"])
+def test_c_smo_solve_with_scores_that_a_float_cannot_tell_apart(ws, scores):
+    """The four-wavefront solver ranks b^2/a in float and falls back to doubles where that does not decide: scores closer
+    together than a float resolves, equal ones, none that is positive, out of a float's range, infinite.  The same steps as
+    the oracle's, bit for bit."""
+    rng = np.random.default_rng(ws + len(scores))
+    n, Cc, eps, max_iter = ws + 5, 2.0, 1e-3, 60
+    y = np.where(rng.random(n) < 0.5, 1, -1).astype(np.int32)
+    b = rng.random((n, n))
+    k = 0.2 * (b + b.T)
+    f = -y + 0.01 * rng.standard_normal(n)
+    alpha = np.zeros(n)
+    if scores.startswith("apart by"):
+        small = float(scores.split()[-1])
+        k, f = small * k, -y * (1 + small * rng.random(n))
+    elif scores == "pairs of equals":
+        k[1::2][: n // 2] = k[0::2][: n // 2]
+        k[:, 1::2][:, : n // 2] = k[:, 0::2][:, : n // 2]
+        f[1::2], y[1::2] = f[0::2][: n // 2], y[0::2][: n // 2]
+    elif scores == "negative a":
+        k = 4.0 * k
+    elif scores.startswith("f times"):
+        f = f * float(scores.split()[-1])
+        eps = 1e-30 if scores.endswith("-25") else eps
+    else:
+        same = rng.random((n, n)) < 0.05
+        k[same | same.T] = 1.0
+    np.fill_diagonal(k, 1.0)
+    ws_ids = rng.permutation(n)[:ws].astype(np.int32)
+    k_rows, diag = np.ascontiguousarray(k[ws_ids]), np.ones(n)
+    a_want, ad_want, diff_want = O.c_smo_solve(y, f, alpha, ws_ids, Cc, Cc, k_rows, diag, n, eps, max_iter)
+    y_d, f_d, ws_d, dg_d, a_d, k_d = G.dev(y), G.dev(f), G.dev(ws_ids), G.dev(diag), G.dev(alpha), G.dev(k_rows)
+    ad_d = torch.zeros(ws, dtype=torch.float64, device="cuda")
+    diff_d = torch.zeros(2, dtype=torch.float64, device="cuda")
+    wsp = torch.empty(capi.kernel_lib().tsvm_smo_solve_workspace(ws), dtype=torch.uint8, device="cuda")
+    capi.call("tsvm_c_smo_solve", G.ptr(y_d), G.ptr(f_d), G.ptr(a_d), G.ptr(ad_d), G.ptr(ws_d), ws, Cc, Cc, G.ptr(k_d), capi.ROW_F64, None,
+              n, G.ptr(dg_d), eps, G.ptr(diff_d), max_iter, G.ptr(wsp), G.stream())
+    assert np.array_equal(G.host(diff_d), diff_want)
+    assert np.array_equal(G.host(a_d), a_want, equal_nan=True)
+    assert np.array_equal(G.host(ad_d), ad_want, equal_nan=True)
+
+
 @pytest.mark.parametrize("nu", [False, True])
 @pytest.mark.parametrize("n,ws", [(300, 16), (2000, 1024), (900, 200)])
 def test_smo_solve_block_on_a_chosen_xcd(n, ws, nu):

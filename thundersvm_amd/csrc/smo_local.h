@@ -99,19 +99,30 @@ struct __align__(16) SvCand {
     int flag;
 };
 
-// Writes by one lane, without the branch that an if around them costs (all 64 lanes are active before and after).
-// Four wavefronts share the LDS, so a write or a broadcast read by 64 lanes is paid four times over: what one lane
-// knows is written by that lane alone.
-__device__ __forceinline__ void publish(SvCand *slot, int lane, double m, int at, int flag) {
+// Writes by one lane (or by one of each row), without the branch that an if around them costs (all 64 lanes are active
+// before and after).  Four wavefronts share the LDS, so a write or a broadcast read by 64 lanes is paid four times over:
+// what one lane knows is written by that lane alone.
+#define SV_EXEC_ON "s_mov_b64 exec, %0\n\t"
+#define SV_EXEC_OFF "s_mov_b64 exec, -1"
+__device__ __forceinline__ void publish_words(unsigned slot, uint64_t lanes, int a, int b, int c, int d) {
     typedef int v4i __attribute__((ext_vector_type(4)));
-    const v4i c = {__double2loint(m), __double2hiint(m), at, flag};
-    asm volatile("s_mov_b64 exec, %2\n\tds_write_b128 %0, %1\n\ts_mov_b64 exec, -1"
-                 :: "v"(lds_at(slot)), "v"(c), "s"(1ull << lane) : "memory");
+    const v4i v = {a, b, c, d};
+    asm volatile(SV_EXEC_ON "ds_write_b128 %1, %2\n\t" SV_EXEC_OFF :: "s"(lanes), "v"(slot), "v"(v) : "memory");
+}
+__device__ __forceinline__ void publish(SvCand *slot, uint64_t lanes, double m, int at, int flag) {
+    publish_words(lds_at(slot), lanes, __double2loint(m), __double2hiint(m), at, flag);
+}
+template <typename S>
+__device__ __forceinline__ void publish(S *slot, uint64_t lanes, float best, float second, int at, int go) {
+    publish_words(lds_at(slot), lanes, __float_as_int(best), __float_as_int(second), at, go);
+}
+template <typename S>
+__device__ __forceinline__ void publish(S *slot, uint64_t lanes, double x, double y) {
+    static_assert(sizeof(S) == 16, "two doubles");
+    asm volatile(SV_EXEC_ON "ds_write2_b64 %1, %2, %3 offset1:1\n\t" SV_EXEC_OFF :: "s"(lanes), "v"(lds_at(slot)), "v"(x), "v"(y) : "memory");
 }
 // The same with the lane's E values of f and of the block row for the step (the row's values in slots of eight bytes).
 // (One asm statement each: nothing else may come between the two writes of exec.)
-#define SV_EXEC_ON "s_mov_b64 exec, %0\n\t"
-#define SV_EXEC_OFF "s_mov_b64 exec, -1"
 template <int E, typename TB>
 __device__ __forceinline__ void publish_row(double *f_slot, double *k_slot, int lane, const double (&f)[E], const TB (&k)[E]) {
     const unsigned fa = lds_at(f_slot), ka = lds_at(k_slot);

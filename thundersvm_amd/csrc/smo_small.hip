@@ -333,7 +333,7 @@ __device__ __forceinline__ int ss_local(SmallShared<E, W> &sh, const SmallMap &m
 #pragma unroll
             for (int e = 0; e < E; ++e) fu[e] = keep_or_none<0>(member << (31 - 2 * NP * e - q), f[e]);
             const int win = wave_argmin_by_pos<E>(fu, sh.pos, tid, up[q], m[q], at[q]);
-            if constexpr (W > 1) publish(ci[q] + wave, win, m[q], at[q], 0);
+            if constexpr (W > 1) publish(ci[q] + wave, 1ull << win, m[q], at[q], 0);
             else is[q] = __builtin_amdgcn_readlane(at[q], win);
         }
         if constexpr (W > 1) {
@@ -376,7 +376,7 @@ __device__ __forceinline__ int ss_local(SmallShared<E, W> &sh, const SmallMap &m
             }
             const int win = wave_argmin_by_pos<E>(qs, sh.pos, tid, best[q], v, at[q]);
             publish_row<E, TB>(sh.f + tid * E, sh.k + tid * E, win, f, kI[q]);
-            if constexpr (W > 1) publish(cj[q] + wave, win, v, at[q], go);
+            if constexpr (W > 1) publish(cj[q] + wave, 1ull << win, v, at[q], go);
             else js[q] = __builtin_amdgcn_readlane(at[q], win);
         }
         if constexpr (W > 1) {

@@ -4,7 +4,7 @@
 // Shape of the kernels.  One workgroup of one or four wavefronts (one per SIMD of the CU) holds the whole working set:
 // element t = tid*E + e lives in register slot e of thread tid (a thread's elements are neighbours, so its share of a
 // block row is one load) with its f and diagonal; alpha lives in LDS (only two entries change per iteration) and the
-// I_up / I_low membership of a thread's elements is a bit field in one register.  One inner iteration is
+// I_up / I_low membership of a thread's elements is a bit field in a register.  One inner iteration is
 //   1. (i, up) = first argmin of f over I_up: a per-thread scan of its E slots, a DPP reduction inside each wavefront,
 //      the wavefronts' candidates through LDS;
 //   2. row K[i, .] of the gathered ws x ws block (coalesced);
@@ -19,7 +19,8 @@
 // wavefront's candidate and two DPP steps compare them; the winner's index by ballot instead of a second reduction; the
 // exit test folded into the loop's branch (the last round computes a step that is not taken); and everything that does
 // not need the row on its way pinned in front of the first instruction that does.
-// Measured on a call of 483 iterations with ws = 1024: 1.37 us per iteration before that, 1.08 with it (2,590 cycles).
+// Measured on a call of 483 iterations with ws = 1024: 1.37 us per iteration before that, 1.08 with it (2,590 cycles);
+// 0.97 with the scores ranked in float where that decides (c_smo_iterate_rounded).
 //
 // Reductions are lexicographic (value, element index) minima, so ties go to the lowest
 // index exactly as the reference's serial loops resolve them, and all arithmetic is the reference's
@@ -183,34 +184,50 @@ __device__ __forceinline__ bool solver_elected(int *gate, int epoch, int target_
     return s_elected != 0;
 }
 
-// What the two solvers keep in LDS, per element of the working set.
+// What the nu solver keeps in LDS, per element of the working set.
 template <int N, int W>
 struct SvShared {
     double kd[N], y[N];       // diagonal, label (0: inactive element)
     double a[W][N];           // alpha: every wavefront keeps a copy of its own, which needs no barrier
 };
 
+// What c_smo_solve keeps.  alpha is held times its label, z = y * alpha in [lo, hi] with lo = 0, hi = Cp for y > 0 and
+// lo = -Cn, hi = 0 for y < 0: an element is in I_up while z < hi and in I_low while z > lo, and a step moves z_i up and z_j
+// down by the same l.  All of it rounds as the reference's expressions in alpha do (they differ in the sign of both operands).
+struct __align__(16) SvBound {
+    double hi, lo;
+};
+struct __align__(16) SvStep {   // f_t - up and K_ii + K_tt - 2 K_it of a candidate for j2
+    double b, a;
+};
+template <int N, int W>
+struct SvState {
+    double kd[N];
+    SvBound bound[N];
+    double z[W][N];           // every wavefront keeps a copy of its own, which needs no barrier
+    double f[N], k[N];        // f and row i at the elements of the wavefronts' candidates for j2 (the others are not written)
+};
+
 // The iterations of c_smo_solve.  NONE: the threshold is not positive, so that an element may violate it without being
 // a candidate for j2 (the reference's j2 then stays 0, smo_kernel.cpp:78); otherwise that cannot happen.
+// Takes up to `left` steps, counted in n_iter; returns whether the solve has ended (nothing violates, or max_iter).
 template <int E, int W, int LDK, bool NONE, typename TB>
-__device__ __forceinline__ int c_smo_iterate(SvShared<E * 64 * W, W> &sh, double *s_f, double *s_k, SvCand *s_i, SvCand *s_j, int ws, double Cp,
-                                             double Cn, const TB *kws, const double (&kd)[E], double (&f)[E], unsigned member,
-                                             double local_eps, int max_iter) {
+__device__ __forceinline__ bool c_smo_iterate(SvState<E * 64 * W, W> &sh, SvCand *s_i, SvCand *s_j, int ws, const TB *kws,
+                                              const double (&kd)[E], double (&f)[E], unsigned &in_up, unsigned &in_low, double local_eps,
+                                              int max_iter, int &n_iter, int left) {
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const double half_Cp = 0.5 * Cp, half_Cn = 0.5 * Cn;
-    int numOfIter = 0;
     bool go_on;
     do {
         // i = first argmin of f over I_up (smo_kernel.cpp:41-59); with an empty I_up any i does, since nothing violates then
         double fu[E];
 #pragma unroll
-        for (int e = 0; e < E; ++e) fu[e] = keep_or_none<0>(member << (31 - 2 * e), f[e]);
+        for (int e = 0; e < E; ++e) fu[e] = keep_or_none<0>(in_up << (31 - e), f[e]);
         double up_value, m;
         int at, i, j2, go;
         const int win_i = wave_first_argmin<E>(fu, tid * E, up_value, m, at);
         if constexpr (W > 1) {
-            publish(s_i + wave, win_i, m, at, 0);
+            publish(s_i + wave, 1ull << win_i, m, at, 0);
             lds_barrier();
             block_argmin<W>(s_i, lane, up_value, i, go);
         } else {
@@ -220,17 +237,18 @@ __device__ __forceinline__ int c_smo_iterate(SvShared<E * 64 * W, W> &sh, double
         TB kI[E];
         load_row_elems<E, TB>(kws + (unsigned) i * (unsigned) LDK, tid, kI);
         SV_PIN_MEMORY;
-        const double kd_i = sh.kd[i], y_i = sh.y[i], a_i = sh.a[wave][i];
+        const double kd_i = sh.kd[i], z_i = sh.z[wave][i];
+        const SvBound bound_i = sh.bound[i];
         double a_part[E], b_low[E], b_max = -TSVM_INF;
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             a_part[e] = kd_i + kd[e];
-            b_low[e] = keep_or_none<1>(member << (30 - 2 * e), -up_value + f[e]);
+            b_low[e] = keep_or_none<1>(in_low << (31 - e), -up_value + f[e]);
             b_max = e == 0 ? b_low[e] : fmax_f64(b_max, b_low[e]);
         }
         // some I_low element still violates: low - up >= local_eps (smo_kernel.cpp:68)
         go = __builtin_amdgcn_ballot_w64(!(b_max < local_eps)) != 0;
-        double up_i = room_up(a_i, y_i, half_Cp);
+        double up_i = bound_i.hi - z_i;
         asm("" : "+v"(up_i));
         SV_PIN;   // (all of this while the row is on its way)
         // j2 = first argmin of -b^2/a over I_low with f > up (smo_kernel.cpp:77-90)
@@ -244,9 +262,9 @@ __device__ __forceinline__ int c_smo_iterate(SvShared<E * 64 * W, W> &sh, double
         }
         double min_t;
         const int win_j = wave_first_argmin<E>(qs, tid * E, min_t, m, at);
-        publish_row<E, TB>(s_f + tid * E, s_k + tid * E, win_j, f, kI);
+        publish_row<E, TB>(sh.f + tid * E, sh.k + tid * E, win_j, f, kI);
         if constexpr (W > 1) {
-            publish(s_j + wave, win_j, m, at, go);
+            publish(s_j + wave, 1ull << win_j, m, at, go);
             lds_barrier();
             block_argmin<W>(s_j, lane, min_t, j2, go);
         } else {
@@ -255,30 +273,216 @@ __device__ __forceinline__ int c_smo_iterate(SvShared<E * 64 * W, W> &sh, double
         if (NONE && is_none(min_t)) {
             j2 = 0;
             __syncthreads();
-            if (tid == 0) { s_f[0] = f[0]; *(TB *) s_k = kI[0]; }
+            if (tid == 0) { sh.f[0] = f[0]; *(TB *) sh.k = kI[0]; }
             __syncthreads();
         }
         j2 = j2 < ws ? j2 : ws - 1;
         TB kJ[E];
         load_row_elems<E, TB>(kws + (unsigned) j2 * (unsigned) LDK, tid, kJ);
         SV_PIN_MEMORY;
-        const double kd_j = sh.kd[j2], y_j = sh.y[j2], a_j = sh.a[wave][j2], f_j = s_f[j2];
-        const double kIj = (double) *(const TB *) (s_k + j2);
+        const SvBound bound_j = sh.bound[j2];
+        const double kd_j = sh.kd[j2], z_j = sh.z[wave][j2], f_j = sh.f[j2];
+        const double kIj = (double) *(const TB *) (sh.k + j2);
         SV_PIN;   // the row is on its way while the step is computed
         // two-variable step (smo_kernel.cpp:92-103; the last round computes one that is not taken)
-        go_on = go && !(numOfIter > max_iter);
+        go_on = go && !(n_iter > max_iter);
         const double q2 = (-up_value + f_j) / __builtin_fma(-2.0, kIj, kd_i + kd_j);
-        const double l = fmin_f64(up_i, fmin_f64(room_low(a_j, y_j, half_Cn), q2));
-        const double na_i = __builtin_fma(l, y_i, a_i), na_j = __builtin_fma(-l, y_j, NONE && j2 == i ? na_i : a_j);
-        member = set_member_bits<E, 2>(member, tid, i, (room_up(na_i, y_i, half_Cp) > 0 ? 1u : 0u) | (room_low(na_i, y_i, half_Cn) > 0 ? 2u : 0u));
-        member = set_member_bits<E, 2>(member, tid, j2, (room_up(na_j, y_j, half_Cp) > 0 ? 1u : 0u) | (room_low(na_j, y_j, half_Cn) > 0 ? 2u : 0u));
-        write_by_lane0(go_on, &sh.a[wave][i], na_i, &sh.a[wave][j2], na_j);
+        const double l = fmin_f64(up_i, fmin_f64(z_j - bound_j.lo, q2));
+        const double nz_i = z_i + l, nz_j = (NONE && j2 == i ? nz_i : z_j) - l;
+        in_up = set_member_bits<E, 1>(in_up, tid, i, nz_i < bound_i.hi ? 1u : 0u);
+        in_low = set_member_bits<E, 1>(in_low, tid, i, nz_i > bound_i.lo ? 1u : 0u);
+        in_up = set_member_bits<E, 1>(in_up, tid, j2, nz_j < bound_j.hi ? 1u : 0u);
+        in_low = set_member_bits<E, 1>(in_low, tid, j2, nz_j > bound_j.lo ? 1u : 0u);
+        write_by_lane0(go_on, &sh.z[wave][i], nz_i, &sh.z[wave][j2], nz_j);
         SV_PIN;   // (nothing above waits for the row)
 #pragma unroll
         for (int e = 0; e < E; ++e) f[e] = __builtin_fma(-l, (double) kJ[e] - (double) kI[e], f[e]);
-        numOfIter += go_on;
-    } while (go_on);
-    return numOfIter;
+        n_iter += go_on;
+    } while (go_on && --left > 0);
+    return !go_on;
+}
+
+// One row's (sixteen lanes') best and second-best score, rounded to float.
+struct __align__(16) SvScore {
+    float best, second;
+    int at, go;
+};
+// best and second of a row in all its lanes.  Four instructions per step, ordered so that none of the DPP operands is
+// younger than two instructions: no wait states between the steps, so the second-best costs hardly more than the waits would.
+__device__ __forceinline__ void row_best_two(float &best, float &second) {
+    float t;
+#define SV_BEST_STEP(CTRL)                                          \
+    "v_min_f32_dpp %2, %0, %0 " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_max_f32_dpp %0, %0, %0 " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_max_f32_dpp %1, %1, %1 " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_max_f32 %1, %1, %2\n\t"
+    asm("s_nop 1\n\t" SV_BEST_STEP("quad_perm:[1,0,3,2]") SV_BEST_STEP("quad_perm:[2,3,0,1]") SV_BEST_STEP("row_half_mirror")
+            SV_BEST_STEP("row_mirror")
+        : "+v"(best), "+v"(second), "=&v"(t));
+#undef SV_BEST_STEP
+}
+// The smallest of a row's x, in all its lanes.
+__device__ __forceinline__ double row_min(double x) {
+    x = fmin_f64(x, dpp_f64<TSVM_DPP_XOR1>(x));
+    x = fmin_f64(x, dpp_f64<TSVM_DPP_XOR2>(x));
+    x = fmin_f64(x, dpp_f64<TSVM_DPP_HALF_MIRROR>(x));
+    return fmin_f64(x, dpp_f64<TSVM_DPP_MIRROR>(x));
+}
+
+// The smallest of a row's E * 16 values; m and at are every lane's own smallest and its first element (as wave_argmin in
+// smo_local.h, whose first four steps these are).
+template <int E>
+__device__ __forceinline__ double row_first_min(const double (&x)[E], int base, double &m, int &at) {
+    m = x[0];
+#pragma unroll
+    for (int e = 1; e < E; ++e) m = fmin_f64(m, x[e]);
+    SV_PIN;
+    uint64_t has[E];
+#pragma unroll
+    for (int e = 0; e < E - 1; ++e) asm volatile("v_cmp_eq_f64_e64 %0, %1, %2" : "=s"(has[e]) : "v"(x[e]), "v"(m));
+    SV_PIN;
+    double r = fmin_f64(m, dpp_f64<TSVM_DPP_XOR1>(m));
+    SV_PIN;
+    at = base + E - 1;
+    if constexpr (E > 2) asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(at) : "v"(at), "v"(base + E - 2), "s"(has[E - 2]));
+    if constexpr (E > 3) asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(at) : "v"(at), "v"(base + E - 3), "s"(has[E - 3]));
+    SV_PIN;
+    r = fmin_f64(r, dpp_f64<TSVM_DPP_XOR2>(r));
+    SV_PIN;
+    asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(at) : "v"(at), "v"(base), "s"(has[0]));
+    SV_PIN;
+    r = fmin_f64(r, dpp_f64<TSVM_DPP_HALF_MIRROR>(r));
+    return fmin_f64(r, dpp_f64<TSVM_DPP_MIRROR>(r));
+}
+
+// The same iterations for four wavefronts with j2 chosen by b^2/a rounded to float, as long as that decides: the largest
+// score has to beat the second by more than both can be off, and to be in float's range.  A score is off by at most
+// 4.2e-7 (b, a, the two products 2^-24 each, b twice; the reciprocal 2^-23), so a lead of 2^-19 = 1.9e-6 is proof, and the
+// winner is then the reference's j2.  Otherwise the function returns false before the step, which c_smo_iterate then takes.
+// (Scores are floored at 2^-80, which makes smaller ones ties; a score without a lead includes every tie, no candidate at
+// all, negative a, and NaN.  One case is not caught: a below 2^-126 with b below 2^-149.)  That replaces E divisions of some
+// fourteen instructions by six each, and the reduction over doubles by one over floats.
+// Rows of sixteen lanes are reduced by DPP and publish themselves, and after the barrier every lane reads one of the
+// sixteen rows and four more steps compare them: the same eight steps as over a wavefront and then over four of them, without
+// the way through the scalar unit in between.
+template <int E, int LDK, typename TB>
+__device__ __forceinline__ bool c_smo_iterate_rounded(SvState<E * 256, 4> &sh, SvCand *s_i, SvScore *s_j, SvStep *s_step, int ws, const TB *kws,
+                                                      const double (&kd)[E], double (&f)[E], unsigned &in_up, unsigned &in_low,
+                                                      double local_eps, int max_iter, int &n_iter) {
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    SvCand *const my_i = s_i + (tid >> 4);
+    SvScore *const my_j = s_j + (tid >> 4);
+    uint64_t go;
+    // the last step's changes to in_low, which are made while the next row is on its way
+    unsigned bit_i = 0, bit_j = 0, low_i = 0, low_j = 0;
+    int owner_i = -1, owner_j = -1;
+    for (;;) {
+        double fu[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) fu[e] = keep_or_none<0>(in_up << (31 - e), f[e]);
+        double m;
+        int at;
+        const double r = row_first_min<E>(fu, tid * E, m, at);
+        // the lowest lane of every row that has it (every field of sixteen bits has one set, whatever is NaN)
+        const uint64_t has = __builtin_amdgcn_ballot_w64(m == r) | 0x8000800080008000ull;
+        publish(my_i, has & ~(has - 0x0001000100010001ull), m, at, 0);
+        lds_barrier();
+        const SvCand ci = s_i[lane & 15];
+        const double up_value = row_min(ci.v);
+        int i = __builtin_amdgcn_readlane(ci.at, __builtin_ctzll(__builtin_amdgcn_ballot_w64(ci.v == up_value)));
+        i = i < ws ? i : ws - 1;
+        TB kI[E];
+        load_row_elems<E, TB>(kws + (unsigned) i * (unsigned) LDK, tid, kI);
+        SV_PIN_MEMORY;
+        const double kd_i = sh.kd[i], z_i = sh.z[wave][i];
+        const SvBound bound_i = sh.bound[i];
+        in_low = tid == owner_i ? (in_low & ~bit_i) | low_i : in_low;
+        in_low = tid == owner_j ? (in_low & ~bit_j) | low_j : in_low;
+        double a_part[E], b_low[E], b_max = -TSVM_INF;
+        float b32[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            b_low[e] = keep_or_none<1>(in_low << (31 - e), -up_value + f[e]);
+            b_max = e == 0 ? b_low[e] : fmax_f64(b_max, b_low[e]);
+            b32[e] = __builtin_fmaxf((float) b_low[e], 0.0f);
+            a_part[e] = kd_i + kd[e];
+        }
+        const int violates = __builtin_amdgcn_ballot_w64(!(b_max < local_eps)) != 0;
+        double up_i = bound_i.hi - z_i;
+        asm("" : "+v"(up_i));
+        SV_PIN;
+        double aIJ[E];
+        float q[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            aIJ[e] = __builtin_fma(-2.0, (double) kI[e], a_part[e]);
+            q[e] = __builtin_fmaxf(b32[e] * (b32[e] * __builtin_amdgcn_rcpf((float) aIJ[e])), 0x1p-80f);
+        }
+        float best, second;
+        if constexpr (E == 4) {
+            const float h0 = __builtin_fmaxf(q[0], q[1]), h1 = __builtin_fmaxf(q[2], q[3]);
+            best = __builtin_fmaxf(h0, h1);
+            second = __builtin_fmaxf(__builtin_fmaxf(__builtin_fminf(h0, h1), __builtin_fminf(q[0], q[1])), __builtin_fminf(q[2], q[3]));
+        } else {
+            static_assert(E == 2, "elements per thread");
+            best = __builtin_fmaxf(q[0], q[1]);
+            second = __builtin_fminf(q[0], q[1]);
+        }
+        at = tid * E + E - 1;
+        double b_at = b_low[E - 1], a_at = aIJ[E - 1];
+#pragma unroll
+        for (int e = E - 2; e >= 0; --e) {
+            const bool is = q[e] == best;
+            at = is ? tid * E + e : at;
+            b_at = is ? b_low[e] : b_at;
+            a_at = is ? aIJ[e] : a_at;
+        }
+        const float mine = best;
+        row_best_two(best, second);
+        const uint64_t who = __builtin_amdgcn_ballot_w64(mine == best);   // (several only if nothing will be decided)
+        publish(my_j, who, best, second, at, violates);
+        publish(s_step + (tid >> 4), who, b_at, a_at);
+        lds_barrier();
+        const SvScore cj = s_j[lane & 15];
+        const SvStep step = s_step[lane & 15];
+        best = cj.best;
+        second = cj.second;
+        row_best_two(best, second);
+        const int row = __builtin_ctzll(__builtin_amdgcn_ballot_w64(cj.best == best));
+        int j2 = __builtin_amdgcn_readlane(cj.at, row);
+        j2 = j2 < ws ? j2 : ws - 1;
+        TB kJ[E];
+        load_row_elems<E, TB>(kws + (unsigned) j2 * (unsigned) LDK, tid, kJ);
+        SV_PIN_MEMORY;
+        const SvBound bound_j = sh.bound[j2];
+        const double z_j = sh.z[wave][j2];
+        SV_PIN;
+        const double steps = step.b / step.a;   // (every row's, while the bounds are read)
+        const double q2 = readlane_f64(steps, row);
+        SV_PIN;
+        // (the two comparisons come out the same in every lane)
+        go = __builtin_amdgcn_ballot_w64(cj.go != 0);
+        const uint64_t sure = __builtin_amdgcn_ballot_w64(second < best * (1.0f - 0x1p-19f)) & __builtin_amdgcn_ballot_w64(best < 0x1p80f);
+        const uint64_t on = n_iter > max_iter ? 0 : go & sure;
+        if (on == 0) break;
+        const double l = fmin_f64(up_i, fmin_f64(z_j - bound_j.lo, q2));
+        const double nz_i = z_i + l, nz_j = z_j - l;
+        owner_i = i / E;
+        owner_j = j2 / E;
+        bit_i = 1u << (i & (E - 1));
+        bit_j = 1u << (j2 & (E - 1));
+        low_i = nz_i > bound_i.lo ? bit_i : 0;
+        low_j = nz_j > bound_j.lo ? bit_j : 0;
+        in_up = tid == owner_i ? (in_up & ~bit_i) | (nz_i < bound_i.hi ? bit_i : 0) : in_up;
+        in_up = tid == owner_j ? (in_up & ~bit_j) | (nz_j < bound_j.hi ? bit_j : 0) : in_up;
+        write_by_lane0(1, &sh.z[wave][i], nz_i, &sh.z[wave][j2], nz_j);
+        SV_PIN;
+#pragma unroll
+        for (int e = 0; e < E; ++e) f[e] = __builtin_fma(-l, (double) kJ[e] - (double) kI[e], f[e]);
+        ++n_iter;
+    }
+    return go == 0 || n_iter > max_iter;
 }
 
 // Elements beyond ws are given y = 0, which puts them in neither I_up nor I_low.
@@ -291,10 +495,10 @@ __global__ __launch_bounds__(64 * W) void c_smo_solve_kernel(
     int max_iter, int *__restrict__ gate, int epoch, int target_xcd) {
     if (gate && !solver_elected(gate, epoch, target_xcd)) return;
     constexpr int N = E * 64 * W;
-    __shared__ SvShared<N, W> sh;
-    __shared__ double s_f[N], s_k[N];   // f and row i at the elements of the wavefronts' candidates for j2 (the others are not written)
+    __shared__ SvState<N, W> sh;
     __shared__ double s_red[2][W];
-    __shared__ SvCand s_i[W], s_j[W];
+    __shared__ SvCand s_i[4 * W], s_j[4 * W];   // (SvScore has SvCand's size)
+    __shared__ SvStep s_step[4 * W];
 
     // This workgroup is a chain of dependent operations; when a chip-wide kernel runs next to it on
     // another stream its wavefronts must not wait behind that kernel's for issue slots.
@@ -302,7 +506,7 @@ __global__ __launch_bounds__(64 * W) void c_smo_solve_kernel(
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     double f[E], a_old[E], kd[E];
-    unsigned member = 0;   // bit 2e: element e is in I_up; bit 2e+1: in I_low
+    unsigned in_up = 0, in_low = 0, plus = 0;   // bit e: element e is in I_up, in I_low, has a label > 0
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const int t = tid * E + e;
@@ -313,10 +517,13 @@ __global__ __launch_bounds__(64 * W) void c_smo_solve_kernel(
         const double y = active ? (double) label[w] : 0.0;
         kd[e] = active ? k_diag[w] : 1.0;
         sh.kd[t] = kd[e];
-        sh.y[t] = y;
+        sh.bound[t].hi = y > 0 ? Cp : 0.0;
+        sh.bound[t].lo = y < 0 ? -Cn : 0.0;
+        plus |= (y > 0 ? 1u : 0u) << e;
 #pragma unroll
-        for (int w = 0; w < W; ++w) sh.a[w][t] = a_old[e];
-        member |= ((is_I_up(a_old[e], y, Cp, Cn) ? 1u : 0u) | (is_I_low(a_old[e], y, Cp, Cn) ? 2u : 0u)) << (2 * e);
+        for (int w = 0; w < W; ++w) sh.z[w][t] = a_old[e] * y;
+        in_up |= (is_I_up(a_old[e], y, Cp, Cn) ? 1u : 0u) << e;
+        in_low |= (is_I_low(a_old[e], y, Cp, Cn) ? 1u : 0u) << e;
     }
     // The initial gap fixes the local stopping threshold (smo_kernel.cpp:61-66).  It is the only place
     // where the value of low = max of f over I_low is needed: inside the loop the stopping test
@@ -328,8 +535,8 @@ __global__ __launch_bounds__(64 * W) void c_smo_solve_kernel(
         double mn = TSVM_INF, mx = -TSVM_INF;
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            mn = fmin_f64(mn, (member >> (2 * e)) & 1u ? f[e] : TSVM_INF);
-            mx = fmax_f64(mx, (member >> (2 * e + 1)) & 1u ? f[e] : -TSVM_INF);
+            mn = fmin_f64(mn, (in_up >> e) & 1u ? f[e] : TSVM_INF);
+            mx = fmax_f64(mx, (in_low >> e) & 1u ? f[e] : -TSVM_INF);
         }
         mn = wave_min_f64(mn);
         mx = wave_max_f64(mx);
@@ -343,15 +550,31 @@ __global__ __launch_bounds__(64 * W) void c_smo_solve_kernel(
         local_eps = eps > t ? eps : t;
         if (tid == 0) diff[0] = local_diff;
     }
-    const int numOfIter = __builtin_amdgcn_readfirstlane(local_eps > 0.0 ? 1 : 0)
-                              ? c_smo_iterate<E, W, LDK, false, TB>(sh, s_f, s_k, s_i, s_j, ws, Cp, Cn, kws, kd, f, member, local_eps, max_iter)
-                              : c_smo_iterate<E, W, LDK, true, TB>(sh, s_f, s_k, s_i, s_j, ws, Cp, Cn, kws, kd, f, member, local_eps, max_iter);
+    int n_iter = 0;
+    if (!__builtin_amdgcn_readfirstlane(local_eps > 0.0 ? 1 : 0)) {
+        c_smo_iterate<E, W, LDK, true, TB>(sh, s_i, s_j, ws, kws, kd, f, in_up, in_low, local_eps, max_iter, n_iter, 0x7fffffff);
+    } else if constexpr (W == 4) {
+        // Where rounded scores do not decide they often go on not deciding (far apart points of equal f): the
+        // exact stretch doubles each time the rounded one has been the shorter of the two.
+        bool done;
+        int stretch = 64;
+        do {
+            const int before = n_iter;
+            done = c_smo_iterate_rounded<E, LDK, TB>(sh, s_i, (SvScore *) s_j, s_step, ws, kws, kd, f, in_up, in_low, local_eps, max_iter, n_iter);
+            if (done) break;
+            stretch = n_iter - before > stretch ? 64 : stretch < 1024 ? 2 * stretch : stretch;
+            done = c_smo_iterate<E, W, LDK, false, TB>(sh, s_i, s_j, ws, kws, kd, f, in_up, in_low, local_eps, max_iter, n_iter, stretch);
+        } while (!done);
+    } else {
+        c_smo_iterate<E, W, LDK, false, TB>(sh, s_i, s_j, ws, kws, kd, f, in_up, in_low, local_eps, max_iter, n_iter, 0x7fffffff);
+    }
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const int t = tid * E + e;
         if (t < ws) {
-            const double a = sh.a[wave][t];
-            alpha_diff[t] = -(a - a_old[e]) * sh.y[t];
+            const double y = (plus >> e) & 1u ? 1.0 : -1.0;
+            const double a = sh.z[wave][t] * y + 0.0;   // (+ 0.0: a zero comes out as +0, as from alpha +- l)
+            alpha_diff[t] = -(a - a_old[e]) * y;
             alpha[working_set[t]] = a;
         }
     }
@@ -359,7 +582,7 @@ __global__ __launch_bounds__(64 * W) void c_smo_solve_kernel(
     // written before it (diff[0] in particular) has to be visible system-wide first
     if (tid == 0) {
         __threadfence_system();
-        diff[1] = (double) numOfIter;
+        diff[1] = (double) n_iter;
     }
 }
 
@@ -449,8 +672,8 @@ __global__ __launch_bounds__(64 * W) void nu_smo_solve_kernel(
         const int win_ip = wave_first_argmin<E>(fup, tid * E, up_value_p, m_p, at_p);
         const int win_in = wave_first_argmin<E>(fun, tid * E, up_value_n, m_n, at_n);
         if constexpr (W > 1) {
-            publish(s_ip + wave, win_ip, m_p, at_p, 0);
-            publish(s_in + wave, win_in, m_n, at_n, 0);
+            publish(s_ip + wave, 1ull << win_ip, m_p, at_p, 0);
+            publish(s_in + wave, 1ull << win_in, m_n, at_n, 0);
             lds_barrier();
             block_argmin<W>(s_ip, lane, up_value_p, ip, go);
             block_argmin<W>(s_in, lane, up_value_n, in, go);
@@ -493,8 +716,8 @@ __global__ __launch_bounds__(64 * W) void nu_smo_solve_kernel(
         publish_row<E, TB>(s_f[0] + tid * E, s_k[0] + tid * E, win_jp, f, kIp);
         publish_row<E, TB>(s_f[1] + tid * E, s_k[1] + tid * E, win_jn, f, kIn);
         if constexpr (W > 1) {
-            publish(s_jp + wave, win_jp, m_p, at_p, go);
-            publish(s_jn + wave, win_jn, m_n, at_n, go);
+            publish(s_jp + wave, 1ull << win_jp, m_p, at_p, go);
+            publish(s_jn + wave, 1ull << win_jn, m_n, at_n, go);
             lds_barrier();
             block_argmin<W>(s_jp, lane, f_val_j2p, j2p, go);
             int go_n;
