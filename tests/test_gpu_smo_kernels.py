@@ -311,6 +311,30 @@ def test_select_working_set(n, n_select, n_marked, tie_mode, nu):
 
 
 @pytest.mark.parametrize("nu", [0, 1])
+@pytest.mark.parametrize("tie_mode", [0, 2])
+@pytest.mark.parametrize("state", ["all free", "few above 0", "few below C"])
+@pytest.mark.parametrize("n", [9, 65, 129, 513, 1025, 4001])
+def test_selection_whose_sides_meet_or_run_dry(n, state, tie_mode, nu):
+    """Almost every candidate is wanted: the two ends of a pair of sides meet ("all free"), or one side has a few entries
+    and the other goes on alone, with those that the first has not taken."""
+    rng = np.random.default_rng(n + tie_mode)
+    f, y, _, C, _ = _select_case(n, 1, 0, n, tie_mode, nu)
+    few = rng.random(n) < 8.0 / n
+    alpha = {"all free": 0.25 + rng.random(n), "few above 0": np.where(few, 0.5 + rng.random(n), 0.0),
+             "few below C": np.where(few, 0.5 + rng.random(n), C)}[state]
+    alpha = np.where(few & (rng.random(n) < 0.5), C - alpha, alpha)
+    n_select = min(1024, n * 3 // 4 // 4 * 4)
+    want = O.select_working_set(f, y, alpha, C, C, np.zeros(0, dtype=np.int32), n_select, nu=bool(nu))
+    f_d, y_d, a_d = G.dev(f), G.dev(y), G.dev(alpha)
+    out_d = torch.full((n_select,), -7, dtype=torch.int32, device="cuda")
+    wsp = torch.empty(capi.kernel_lib().tsvm_select_workspace(n), dtype=torch.uint8, device="cuda")
+    capi.call("tsvm_select_working_set", G.ptr(f_d), G.ptr(y_d), G.ptr(a_d), n, C, C, None, 0, G.ptr(out_d), n_select, nu, G.ptr(wsp),
+              G.stream())
+    got = G.host(out_d)
+    assert np.array_equal(got, want), "first mismatch at %s" % np.flatnonzero(got != want)[:5]
+
+
+@pytest.mark.parametrize("nu", [0, 1])
 @pytest.mark.parametrize("tie_mode", [0, 1, 2])
 def test_longer_selection_starts_with_the_shorter_one(tie_mode, nu):
     """Asking for more ids appends runners-up: the first n_select ids do not change."""

