@@ -143,6 +143,33 @@ def test_long_chunks_and_many_support_vectors(monkeypatch):
     assert gm.total_sv > 8000
 
 
+@pytest.mark.parametrize("kt,long_row", [(2, False), (2, True), (0, False), (1, False)])
+@pytest.mark.parametrize("m", [255, 256, 257, 300])
+def test_sparse_rows_on_both_routes(kt, long_row, m):
+    """Sparse support vectors: from 256 rows on a batch is multiplied with their sliced copy, smaller ones (and those with a
+    row too long for it) are staged as a dense matrix.  The two agree in every bit and with the oracle; an empty row and
+    columns that no support vector has are among the rows."""
+    rng = np.random.default_rng(m + kt)
+    n, d = 700, 2400
+
+    def rows(count, width):
+        lens = rng.integers(1, 20, count)
+        lens[3] = 0
+        if width > d and long_row:
+            lens[5] = 1900
+        ptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+        col = np.concatenate([np.sort(rng.choice(width, size=k, replace=False)) for k in lens]).astype(np.int32) + 1
+        val = rng.standard_normal(len(col)).astype(np.float32).astype(np.float64)
+        return D.CsrData(ptr, col, val, np.where(rng.random(count) < 0.5, 1.0, -1.0))
+    tr, te = rows(n, d), rows(m, d + 50)
+    prm = make_param(svm_type=0, kernel_type=kt, C=2.0, gamma=0.05, degree=2, coef0=0.5)
+    gm = Model(0).train(tr, prm)
+    om = O.Model(tr.ptr, tr.col, tr.val, tr.y, _oparam(prm))
+    whole, parts = gm.predict(te)[1], gm.predict(te, 40)[1]
+    assert np.array_equal(whole, parts)
+    assert np.abs(whole - om.predict(te.ptr, te.col, te.val, 100)[1]).max() < 1e-6
+
+
 def test_sparse_class_pair_whose_rows_are_all_empty():
     """A wide, sparse three-class problem in which two classes' rows hold no feature at all: their class pair is a CSR
     sub-problem without a single stored entry (every kernel value is kappa(0, 0)), so there is nothing to slice for the

@@ -412,14 +412,16 @@ std::shared_ptr<DeviceRows> DeviceRows::from_host(const RowStore &rows) {
     const int64_t first = rows.ptr()[0];
     const int *const col = rows.col() + first;
     const kernel_type *const val = rows.val() + first;
-    int max_index = 0, all_float = 1;
-#pragma omp parallel for schedule(static) reduction(max : max_index) reduction(min : all_float) num_threads(threads_for(r.nnz))
+    int max_index = 0, all_float = 1, all_finite = 1;
+#pragma omp parallel for schedule(static) reduction(max : max_index) reduction(min : all_float, all_finite) num_threads(threads_for(r.nnz))
     for (size_t e = 0; e < r.nnz; ++e) {
         max_index = std::max(max_index, col[e]);
         all_float = (double) (float) val[e] != (double) val[e] ? 0 : all_float;
+        all_finite = val[e] - val[e] == 0 ? all_finite : 0;
     }
     r.n_features = (size_t) max_index + 1;
     r.values_fit_float = all_float != 0;
+    r.values_finite = all_finite != 0;
     r.dense = KernelMatrix::choose_dense(r.n, r.n_features, r.nnz);
     r.val.resize(r.nnz);
     r.col.resize(r.nnz);
@@ -786,12 +788,28 @@ void KernelMatrix::get_rows(const RowStore &batch, size_t first, size_t n_rows, 
         abi_check(tsvm_get_rows_dense(R.x.data(), R.ld, nullptr, n, (int) R.n_features, R.self_dot.data(), b.a, b.lda, nullptr, m,
                                       b.sd, (int) param.kernel_type, param.gamma, param.coef0, param.degree,
                                       d_out, row_type(), nullptr, ld, tsvm::work_stream()));
-    } else {
-        if (stage_.size() < (size_t) m * R.n_features) stage_.resize((size_t) m * R.n_features);
-        abi_check(tsvm_csr_stage_rows(b_val_.data(), b_col_.data(), b_ptr_.data(), nullptr, m, (int) R.n_features,
-                                      stage_.data(), tsvm::work_stream()));
-        abi_check(tsvm_get_rows_csr(R.val.data(), R.col.data(), R.row_ptr.data(), nullptr, n, R.self_dot.data(), stage_.data(), m,
-                                    b.sd, (int) param.kernel_type, param.gamma, param.coef0, param.degree,
-                                    d_out, row_type(), nullptr, ld, tsvm::work_stream()));
+        return;
     }
+    // The batch's rows wait in LDS, sixteen at a time, and the support vectors' sliced copy streams by, as in training; a batch
+    // with a row too long for that is staged as a dense matrix, and so is any batch when a support vector holds an infinity
+    // or NaN, whose product with an absent (zero) feature is not zero.  Kernel values of text rows, staged / sliced, us: 6,000
+    // support vectors 65 / 23 for one row, 87 / 38 for 64, 217 / 79 for 1,000, 1,148 / 263 for 4,099; 800 support vectors 24 / 22,
+    // 27 / 33, 65 / 35, 313 / 64; 3,000 31 / 23, 37 / 38, 128 / 42, 674 / 148: few of them fill few workgroups, so few rows go
+    // the staged way there.
+    const int wt = R.values_fit_float ? TSVM_ROW_F32 : TSVM_ROW_F64;
+    int longest = 0;
+    for (int r = 0; r < m; ++r) longest = std::max(longest, (int) (h_ptr_.data()[r + 1] - h_ptr_.data()[r]));
+    if (R.sliced_lds && R.values_finite && (n >= 3072 || m >= 256) && tsvm_get_rows_csr_sliced_lds((int) R.n_features, longest, wt) > 0) {
+        abi_check(tsvm_get_rows_csr_sliced(R.ell_col.data(), R.ell_val.data(), wt, R.slice_ptr.data(), n, R.self_dot.data(),
+                                           b_val_.data(), b_col_.data(), b_ptr_.data(), nullptr, m, b.sd, (int) R.n_features, longest,
+                                           (int) param.kernel_type, param.gamma, param.coef0, param.degree, d_out, row_type(), nullptr, ld,
+                                           tsvm::work_stream()));
+        return;
+    }
+    if (stage_.size() < (size_t) m * R.n_features) stage_.resize((size_t) m * R.n_features);
+    abi_check(tsvm_csr_stage_rows(b_val_.data(), b_col_.data(), b_ptr_.data(), nullptr, m, (int) R.n_features,
+                                  stage_.data(), tsvm::work_stream()));
+    abi_check(tsvm_get_rows_csr(R.val.data(), R.col.data(), R.row_ptr.data(), nullptr, n, R.self_dot.data(), stage_.data(), m,
+                                b.sd, (int) param.kernel_type, param.gamma, param.coef0, param.degree,
+                                d_out, row_type(), nullptr, ld, tsvm::work_stream()));
 }

@@ -26,6 +26,7 @@ struct DeviceRows {
     size_t n = 0, n_features = 0, nnz = 0;
     bool dense = false;
     bool values_fit_float = false;               // every stored value is exactly a float (CSR layout: staging type)
+    bool values_finite = false;                  // no stored value is infinite or NaN (rows taken from host memory)
     int64_t ld = 0;                              // dense row stride (n_features rounded up to 8)
     tsvm::DeviceBuffer<kernel_type> x;           // dense layout [n][ld]
     tsvm::DeviceBuffer<kernel_type> val;         // CSR layout
