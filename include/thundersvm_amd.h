@@ -202,6 +202,12 @@ int tsvm_gather_f64(const double *in, const int *idx, int m, double *out, tsvm_s
 int tsvm_update_f(double *f, const double *alpha_diff, int ws_size, const void *k_rows, int row_type, const int *slots,
                   int64_t ld, int64_t n_cols, int repeat, tsvm_stream stream);
 
+/* The same update for n_rows kernel rows in batches of `batch` (the last one may be shorter), one after the other: what
+ * ceil(n_rows / batch) calls of tsvm_update_f with slots == NULL do, in one launch (csmosolver.cpp:189-214).  coef[t], the
+ * role of alpha_diff, is taken as it is, zeros included. */
+int tsvm_update_f_batches(double *f, const double *coef, int n_rows, int batch, const void *k_rows, int row_type, int64_t ld,
+                          int64_t n_cols, int repeat, tsvm_stream stream);
+
 /* Bytes of device workspace tsvm_c_smo_solve / tsvm_nu_smo_solve need for a working set of ws_size. */
 size_t tsvm_smo_solve_workspace(int ws_size);
 

@@ -66,6 +66,23 @@ def test_update_f_wide_and_repeated(n, ws, ld_pad, row_type):
     assert np.array_equal(G.host(f_d), want)
 
 
+@pytest.mark.parametrize("n,n_rows,batch,repeat", [(1, 1, 101, 1), (63, 31, 101, 2), (64, 32, 16, 1), (65, 33, 101, 1), (5001, 101, 101, 1),
+                                                   (257, 102, 101, 2), (300, 640, 101, 1), (1000, 1010, 101, 2)])
+@pytest.mark.parametrize("row_type", [capi.ROW_F64, capi.ROW_F32])
+def test_update_f_in_batches(n, n_rows, batch, repeat, row_type):
+    """One launch gives what one update_f per batch gives, bit for bit, on both sides of the rows it keeps on their way."""
+    rng = np.random.default_rng(n + n_rows)
+    ld = n + 3
+    k = rng.standard_normal((n_rows, ld)).astype(np.float32 if row_type == capi.ROW_F32 else np.float64)
+    coef, f = rng.standard_normal(n_rows), rng.standard_normal(n * repeat)
+    want, rows = f, np.ascontiguousarray(np.tile(k[:, :n].astype(np.float64), (1, repeat)))
+    for at in range(0, n_rows, batch):
+        want = O.update_f(want, coef[at:at + batch], rows[at:at + batch], n * repeat)
+    f_d, c_d, k_d = G.dev(f), G.dev(coef), G.dev(k)
+    capi.call("tsvm_update_f_batches", G.ptr(f_d), G.ptr(c_d), n_rows, batch, G.ptr(k_d), row_type, ld, n, repeat, G.stream())
+    assert np.array_equal(G.host(f_d), want)
+
+
 def test_fold_ids():
     ids = np.array([0, 5, 9, 10, 19, 7], dtype=np.int32)
     out = torch.zeros(6, dtype=torch.int32, device="cuda")

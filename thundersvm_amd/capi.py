@@ -47,6 +47,7 @@ SIGNATURES = {
     "tsvm_csr_gather_rows": (_int, [_p, _p, _p, _p, _i64, _p, _p, _p, _p]),
     "tsvm_gather_f64": (_int, [_p, _p, _int, _p, _p]),
     "tsvm_update_f": (_int, [_p, _p, _int, _p, _int, _p, _i64, _i64, _int, _p]),
+    "tsvm_update_f_batches": (_int, [_p, _p, _int, _int, _p, _int, _i64, _i64, _int, _p]),
     "tsvm_smo_solve_workspace": (C.c_size_t, [_int]),
     "tsvm_c_smo_solve": (_int, [_p, _p, _p, _p, _p, _int, _dbl, _dbl, _p, _int, _p, _i64, _p, _dbl, _p, _int, _p, _p]),
     "tsvm_c_smo_solve_static_init": (_int, []),

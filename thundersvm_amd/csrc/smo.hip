@@ -434,6 +434,58 @@ __global__ __launch_bounds__(UF_T) void update_f_kernel(double *__restrict__ f, 
     }
 }
 
+// f from a non-zero alpha: batches of rows, each summed and then taken from f (csmosolver.cpp:189-214).  Bound by memory
+// latency: few columns (a few thousand instances), many rows, and the sums of a column one after another.  One column per
+// thread in workgroups of one wavefront (5,001 columns are 79 of them), the rows one stream across the batches, the next UB
+// of them on their way while UB are added: 1,010 rows of 5,001 floats 70 us, ten launches of update_f_kernel 88 and the gaps
+// between them.  nu-SVC on 5,001 x 23 starts from 2,000 such rows: 5.01 -> 4.57 ms.
+#define UB 32
+template <typename TK>
+__global__ __launch_bounds__(64) void update_f_batches_kernel(double *__restrict__ f, const double *__restrict__ coef, int n_rows, int batch,
+                                                              const TK *__restrict__ k_rows, int64_t ld, int64_t n, int repeat) {
+    const int64_t j = (int64_t) blockIdx.x * 64 + threadIdx.x;
+    const TK *const col = k_rows + (j < n ? j : n - 1);
+    double sum = 0.0;
+    int left = batch;   // rows of the batch still to come
+    auto add = [&](int t, double c, TK k) {
+        sum = __builtin_fma(c, (double) k, sum);
+        if (--left == 0 || t == n_rows - 1) {
+            if (j < n)
+                for (int r = 0; r < repeat; ++r) f[r * n + j] -= sum;
+            sum = 0.0;
+            left = batch;
+        }
+    };
+    TK next[UB];
+    double next_c[UB];
+    const int whole = n_rows / UB * UB;
+    auto fetch = [&](int t) {
+#pragma unroll
+        for (int u = 0; u < UB; ++u) next[u] = col[(int64_t) (t + u) * ld];
+#pragma unroll
+        for (int u = 0; u < UB; ++u) next_c[u] = coef[t + u];
+    };
+    if (whole > 0) fetch(0);
+    for (int t = 0; t < whole; t += UB) {
+        TK k[UB];
+        double c[UB];
+#pragma unroll
+        for (int u = 0; u < UB; ++u) { k[u] = next[u]; c[u] = next_c[u]; }
+        fetch(t + UB < whole ? t + UB : t);
+        if (left > UB) {   // no batch ends among these rows, unless they are the last ones
+#pragma unroll
+            for (int u = 0; u < UB; ++u) sum = __builtin_fma(c[u], (double) k[u], sum);
+            left -= UB;
+            if (t + UB == n_rows && j < n)
+                for (int r = 0; r < repeat; ++r) f[r * n + j] -= sum;
+        } else {
+#pragma unroll
+            for (int u = 0; u < UB; ++u) add(t + u, c[u], k[u]);
+        }
+    }
+    for (int t = whole; t < n_rows; ++t) add(t, coef[t], col[(int64_t) t * ld]);
+}
+
 // Pass p: histogram of digit p of the not-yet-decided candidates.  Pass 0 also builds keys and flags; there a
 // workgroup walks one contiguous chunk of the instances and keeps the chunk's marked instances (the half of the
 // previous working set that stays, csmosolver.cpp:65-71: never candidates) as a bit field in LDS.
@@ -879,6 +931,23 @@ int tsvm_update_f(double *f, const double *alpha_diff, int ws_size, const void *
     TSVM_REQUIRE(row_type == TSVM_ROW_F64 || row_type == TSVM_ROW_F32, "tsvm_update_f: unknown row type %d", row_type);
     if (n_cols == 0 || ws_size == 0) return 0;
     dispatch_update_f<0>(f, alpha_diff, ws_size, k_rows, row_type, slots, ld, n_cols, repeat, SelFuse(), tsvm_s(stream));
+    TSVM_LAUNCH_CHECK();
+    return 0;
+}
+
+int tsvm_update_f_batches(double *f, const double *coef, int n_rows, int batch, const void *k_rows, int row_type, int64_t ld,
+                          int64_t n_cols, int repeat, tsvm_stream stream) {
+    TSVM_REQUIRE(f && coef && k_rows, "tsvm_update_f_batches: null pointer");
+    TSVM_REQUIRE(n_rows >= 0 && batch >= 1 && n_cols >= 0 && ld >= n_cols && repeat >= 1, "tsvm_update_f_batches: bad size (rows=%d batch=%d n=%lld ld=%lld)",
+                 n_rows, batch, (long long) n_cols, (long long) ld);
+    TSVM_REQUIRE(row_type == TSVM_ROW_F64 || row_type == TSVM_ROW_F32, "tsvm_update_f_batches: unknown row type %d", row_type);
+    TSVM_REQUIRE((n_cols + 63) / 64 <= 0x7fffffffLL, "tsvm_update_f_batches: %lld columns", (long long) n_cols);
+    if (n_cols == 0 || n_rows == 0) return 0;
+    const dim3 grid((unsigned) ((n_cols + 63) / 64));
+    if (row_type == TSVM_ROW_F32)
+        hipLaunchKernelGGL(update_f_batches_kernel<float>, grid, dim3(64), 0, tsvm_s(stream), f, coef, n_rows, batch, (const float *) k_rows, ld, n_cols, repeat);
+    else
+        hipLaunchKernelGGL(update_f_batches_kernel<double>, grid, dim3(64), 0, tsvm_s(stream), f, coef, n_rows, batch, (const double *) k_rows, ld, n_cols, repeat);
     TSVM_LAUNCH_CHECK();
     return 0;
 }

@@ -876,36 +876,35 @@ void CSMOSolver::solve(const KernelMatrix &k_mat, const std::vector<int> &y, std
     stats = task.stats();
 }
 
-// csmosolver.cpp:189-214: f starts from a non-zero alpha in batches of 101 rows.
+// csmosolver.cpp:189-214: f starts from a non-zero alpha in batches of 101 rows.  Ids and coefficients travel once.  Several
+// batches' rows are computed by one call where they are dense and small (101 rows of a few thousand columns leave most of
+// the chip idle): up to ten batches in INIT_ROWS_BYTES.
 void CSMOSolver::init_f(const std::vector<float_type> &alpha, const std::vector<int> &y, const KernelMatrix &k_mat,
                         float_type *d_f) const {
-    const size_t batch_size = 100;
+    constexpr size_t BATCH = 101, INIT_ROWS_BYTES = (size_t) 64 << 20;
     const int n_u = (int) k_mat.n_columns();
     const int64_t ld = ((int64_t) n_u + 7) / 8 * 8;
-    std::vector<int> idx_vec;
-    std::vector<float_type> alpha_diff_vec;
-    DeviceBuffer<int> d_idx;
-    DeviceBuffer<float_type> d_ad;
-    DeviceBuffer<unsigned char> d_rows;
-    for (size_t i = 0; i < alpha.size(); ++i) {
+    std::vector<int> idx;
+    std::vector<float_type> coef;
+    for (size_t i = 0; i < alpha.size(); ++i)
         if (alpha[i] != 0) {
-            idx_vec.push_back((int) (i % (size_t) n_u));
-            alpha_diff_vec.push_back(-alpha[i] * y[i]);
+            idx.push_back((int) (i % (size_t) n_u));
+            coef.push_back(-alpha[i] * y[i]);
         }
-        if (idx_vec.size() > batch_size || (i == alpha.size() - 1 && !idx_vec.empty())) {
-            const int m = (int) idx_vec.size();
-            if (d_rows.size() == 0) {
-                d_idx.resize(batch_size + 1);
-                d_ad.resize(batch_size + 1);
-                d_rows.resize((batch_size + 1) * (size_t) ld * k_mat.row_elem_size());
-            }
-            d_idx.upload(idx_vec.data(), m);
-            d_ad.upload(alpha_diff_vec.data(), m);
-            k_mat.get_rows(d_idx.data(), m, d_rows.data(), ld, nullptr, tsvm::work_stream());
-            abi_check(tsvm_update_f(d_f, d_ad.data(), m, d_rows.data(), k_mat.row_type(), nullptr, ld, n_u, k_mat.repeat(), tsvm::work_stream()));
-            idx_vec.clear();
-            alpha_diff_vec.clear();
-        }
+    if (idx.empty()) return;
+    const size_t row_bytes = (size_t) ld * k_mat.row_elem_size();
+    const size_t fit = k_mat.dense_layout() ? std::min<size_t>(10, INIT_ROWS_BYTES / row_bytes / BATCH) : 1;
+    const size_t at_once = std::min(std::max<size_t>(fit, 1) * BATCH, idx.size());
+    DeviceBuffer<int> d_idx;
+    DeviceBuffer<float_type> d_coef;
+    DeviceBuffer<unsigned char> d_rows(at_once * row_bytes);
+    d_idx.upload(idx);
+    d_coef.upload(coef);
+    for (size_t at = 0; at < idx.size(); at += at_once) {
+        const int m = (int) std::min(at_once, idx.size() - at);
+        k_mat.get_rows(d_idx.data() + at, m, d_rows.data(), ld, nullptr, tsvm::work_stream());
+        abi_check(tsvm_update_f_batches(d_f, d_coef.data() + at, m, (int) BATCH, d_rows.data(), k_mat.row_type(), ld, n_u, k_mat.repeat(),
+                                        tsvm::work_stream()));
     }
 }
 
