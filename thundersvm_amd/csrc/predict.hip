@@ -51,9 +51,11 @@ __global__ __launch_bounds__(256, 2) void predict_dense_stream_kernel(
     __shared__ __attribute__((aligned(16))) double s_coef[2][NC][GR_BN];
     KernelParam kp = kp_in;
     kp.kernel_type = KT;
-    const unsigned logical = xcd_remap(blockIdx.x, gridDim.x);
-    const int i0 = (int) (logical % m_blocks) * BM;
-    const unsigned chunk = logical / m_blocks;
+    // Workgroups are dealt to the eight XCDs in turn, so every XCD gets an eighth of every chunk's row blocks, and all of them
+    // have the same chunk in their L2 at a time.  A run of chunks per XCD would leave those with the small classes' short chunks
+    // idle: 50,000 rows of 54 columns against 16,076 support vectors in seven classes 3.07 -> 1.76 ms.
+    const int i0 = (int) (blockIdx.x % m_blocks) * BM;
+    const unsigned chunk = blockIdx.x / m_blocks;
     const unsigned jt0 = (unsigned) chunks[2 * chunk], jt1 = (unsigned) chunks[2 * chunk + 1];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -320,9 +322,9 @@ __global__ __launch_bounds__(256, 2) void predict_dense_tile_kernel(
     if (tid < 32) exp_tab[tid] = TSVM_EXP2F_TAB[tid];
     for (int e = tid; e < 2 * BM * nc; e += 256) red[e] = 0.0;
     __syncthreads();
-    const unsigned logical = xcd_remap(blockIdx.x, gridDim.x);
-    const int i0 = (int) (logical % m_blocks) * BM;
-    const unsigned chunk = logical / m_blocks;
+    // (as in predict_dense_stream_kernel)
+    const int i0 = (int) (blockIdx.x % m_blocks) * BM;
+    const unsigned chunk = blockIdx.x / m_blocks;
     const int jt0 = chunks[2 * chunk], jt1 = chunks[2 * chunk + 1];
     for (int jt = jt0; jt < jt1; ++jt) {
         get_rows_tile<KT, 4, double, false, true>(x, ldx, col_map, n_pad, d, sd_x, a, lda, nullptr, m, sd_a, kp, nullptr, nullptr,
