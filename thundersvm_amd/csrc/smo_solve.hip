@@ -15,7 +15,7 @@
 // whatever it does, an LDS access fifty, a block row 250 (from the L2), a value that crosses to the scalar unit and
 // comes back about forty, a branch around a few instructions about forty-five, and a write or a broadcast read by all
 // 256 threads takes the LDS four wavefronts' worth of cycles.  Hence: no branches inside the loop; what one lane knows is written by that
-// lane alone (exec set to one bit around the write); every wavefront keeps its own copy of alpha; each thread reads one
+// lane alone (exec set to one bit around the write); every wavefront keeps its own copy of alpha; each lane reads one
 // wavefront's candidate and two DPP steps compare them; the winner's index by ballot instead of a second reduction; the
 // exit test folded into the loop's branch (the last round computes a step that is not taken); and everything that does
 // not need the row on its way pinned in front of the first instruction that does.
