@@ -69,3 +69,18 @@ def test_folds_side_by_side(svm_type, n, folds):
     got = [Model(svm_type).cross_validation(d, make_param(svm_type=svm_type, gamma=0.2, C=3.0, nu=0.2, p=0.05, cache_bytes=c), folds)
            for c in (-1, 64 << 20)]
     assert np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("svm_type,n", [(0, 60), (0, 120), (0, 250), (0, 300), (0, 700), (3, 30), (3, 61), (3, 200), (3, 400)])
+def test_infinite_C(svm_type, n):
+    """A hard margin: no upper bound on alpha.  Classes that a plane parts with room to spare, and targets that the
+    functions of the kernel take, so that the solution is finite; against the oracle and the path of the larger problems."""
+    x, rng = _rows(n, 77 + n, False)
+    y = (rng.random(n) < 0.4).astype(np.float64)
+    x[:, 0] = x[:, 0] * 0.3 + np.where(y > 0, 2.0, -2.0)
+    d = D.from_dense(x, y if svm_type == 0 else np.sin(x[:, 0]))
+    prm = dict(svm_type=svm_type, gamma=0.05, C=np.inf, p=0.2, max_iter=40)
+    gm, om, _, _ = T._compare(d, d, make_param(**prm), trace=0)
+    assert np.isfinite(gm.coef).all() and gm.total_sv > 0
+    alone = Model(svm_type).train(d, make_param(pair_lanes=1, cache_bytes=0, **prm))   # (asks for the other path)
+    assert np.array_equal(gm.coef, alone.coef) and np.array_equal(gm.rho, alone.rho)

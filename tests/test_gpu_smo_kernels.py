@@ -156,6 +156,23 @@ def test_nu_smo_solve(n, ws):
     assert np.array_equal(G.host(ad_d), ad_want)
 
 
+@pytest.mark.parametrize("ws", [16, 200, 300, 1024])
+def test_nu_smo_solve_infinite_C(ws):
+    """No upper bound on alpha: steps are bounded by alpha >= 0 and the quotient alone, for both labels."""
+    n, eps = ws + 100, 1e-3
+    y, alpha, f, ws_ids, k_rows, diag = _solver_inputs(n, 10, ws, 7 * n, 1.0)
+    a_want, ad_want, diff_want = O.nu_smo_solve(y, f, alpha, ws_ids, np.inf, k_rows, diag, n, eps, 2000)
+    assert np.isfinite(a_want).all() and (a_want >= 0).all() and a_want.max() > 1.0
+    y_d, f_d, a_d, ws_d, k_d, dg_d = G.dev(y), G.dev(f), G.dev(alpha), G.dev(ws_ids), G.dev(k_rows), G.dev(diag)
+    ad_d = torch.zeros(ws, dtype=torch.float64, device="cuda")
+    diff_d = torch.zeros(2, dtype=torch.float64, device="cuda")
+    wsp = torch.empty(capi.kernel_lib().tsvm_smo_solve_workspace(ws), dtype=torch.uint8, device="cuda")
+    capi.call("tsvm_nu_smo_solve", G.ptr(y_d), G.ptr(f_d), G.ptr(a_d), G.ptr(ad_d), G.ptr(ws_d), ws, np.inf, G.ptr(k_d),
+              capi.ROW_F64, None, n, G.ptr(dg_d), eps, G.ptr(diff_d), 2000, G.ptr(wsp), G.stream())
+    assert G.host(diff_d)[0] == diff_want[0]
+    assert np.array_equal(G.host(a_d), a_want) and np.array_equal(G.host(ad_d), ad_want)
+
+
 @pytest.mark.parametrize("ws", [2, 63, 64, 65, 128, 129, 256, 257, 512, 513, 1023, 1024])
 @pytest.mark.parametrize("nu", [False, True])
 @pytest.mark.parametrize("start", ["first iteration", "threshold zero"])

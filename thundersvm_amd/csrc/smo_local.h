@@ -186,12 +186,11 @@ __device__ __forceinline__ unsigned set_member_bits(unsigned m, int tid, int t, 
     return tid == (int) ((unsigned) t / E) ? changed : m;
 }
 
-// How far alpha can move along its label y = +-1 (y > 0 ? Cp - a : a; the element is in I_up while this is positive)
-// and against it (y > 0 ? a : Cn - a; in I_low while positive), smo_kernel.h:13-23 and smo_kernel.cpp:94-99: one fma
-// each on the half bounds, which rounds exactly as the selected subtraction does.
-__device__ __forceinline__ double room_up(double a, double y, double half_Cp) {
-    return __builtin_fma(-y, a, __builtin_fma(y, half_Cp, half_Cp));
-}
-__device__ __forceinline__ double room_low(double a, double y, double half_Cn) {
-    return __builtin_fma(y, a, __builtin_fma(-y, half_Cn, half_Cn));
-}
+// The local solvers hold alpha times its label, z = y * alpha in [lo, hi] with lo = 0, hi = Cp for y > 0 and lo = -Cn,
+// hi = 0 for y < 0: an element is in I_up while z < hi and in I_low while z > lo, a step is bounded by hi - z_i and z_j - lo
+// (smo_kernel.h:13-23, smo_kernel.cpp:94-99), and it moves z_i up and z_j down by the same l.  All of it rounds as the
+// reference's expressions in alpha do (they differ in the sign of both operands), and an infinite C (a hard margin) is a bound like
+// any other.  (The bounds are selected by the label: computed from it, as y * C/2 + C/2, one of them would be inf - inf.)
+struct __align__(16) SvBound {
+    double hi, lo;
+};

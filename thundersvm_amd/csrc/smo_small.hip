@@ -84,7 +84,7 @@ template <int E, int W>
 struct SmallShared {
     static constexpr int N = 64 * E * W;
     double kd[N];
-    double a[W][N];                     // alpha: one copy per wavefront (smo_solve.hip)
+    double z[W][N];                     // alpha times its label (SvBound): one copy per wavefront (smo_solve.hip)
     double f[N], k[N];                  // local solver: f and the row at the candidates; selection: keys and slots on their way between wavefronts; update: coefficients and rows
     unsigned short pos[N];              // position of a slot in the working set, 0xffff outside it
     unsigned short ws[N];
@@ -298,6 +298,7 @@ struct SmallMap {
     __device__ __forceinline__ bool active(int s) const { return s < n0p ? s < n0 : s - n0p < n1; }
     __device__ __forceinline__ int index(int s) const { return s < n0p ? s : n0 + (s - n0p); }
     __device__ __forceinline__ double label(int s) const { return s < n0p ? 1.0 : -1.0; }
+    __device__ __forceinline__ SvBound bound(int s, double Cp, double Cn) const { return s < n0p ? SvBound{Cp, 0.0} : SvBound{0.0, -Cn}; }
 };
 
 template <int E, typename TB>
@@ -313,12 +314,11 @@ __device__ __forceinline__ void ss_load(const TB *row, TB (&out)[E]) {
 }
 
 // The local solver: c_smo_iterate of smo_solve.hip (and nu_smo_solve_kernel) with the instances in place of a gathered
-// working set.  Returns the steps taken; the new alpha is in sh.a.  NONE: the threshold is not positive (see there).
+// working set.  Returns the steps taken; the new alpha is in sh.z.  NONE: the threshold is not positive (see there).
 template <int E, int W, bool NU, bool NONE, typename TB>
 __device__ __forceinline__ int ss_local(SmallShared<E, W> &sh, const SmallMap &map, const TB *K, int64_t ld, int col, const double (&kd)[E], double (&f)[E],
                         unsigned member, double Cp, double Cn, double local_eps, int max_iter) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const double half_Cp = 0.5 * Cp, half_Cn = NU ? half_Cp : 0.5 * Cn;
     constexpr int NP = NU ? 2 : 1;   // pairs of sides
     SvCand *const ci[2] = {sh.ci, sh.ci2}, *const cj[2] = {sh.cj, sh.cj2};
     const int first_slot = sh.ws[0];
@@ -410,19 +410,20 @@ __device__ __forceinline__ int ss_local(SmallShared<E, W> &sh, const SmallMap &m
         ss_load<E, TB>(K + (unsigned) map.row(j2) * (unsigned) ld + col, kJ);
         const TB k_ij = NU ? K[(unsigned) map.row(i) * (unsigned) ld + map.row(j2)] : *(const TB *) (sh.k + j2);
         SV_PIN_MEMORY;
-        const double kd_j = sh.kd[j2], a_j = sh.a[wave][j2], a_i = sh.a[wave][i], f_j = sh.f[j2], y_i = map.label(i), y_j = map.label(j2);
+        const double kd_j = sh.kd[j2], z_j = sh.z[wave][j2], z_i = sh.z[wave][i], f_j = sh.f[j2];
+        const SvBound bound_i = map.bound(i, Cp, Cn), bound_j = map.bound(j2, Cp, Cn);
         SV_PIN;
         go_on = go && !(n_iter > max_iter);
         const double q2 = (-up_value + f_j) / __builtin_fma(-2.0, (double) k_ij, kd_i2 + kd_j);
-        const double l = fmin_f64(room_up(a_i, y_i, half_Cp), fmin_f64(room_low(a_j, y_j, half_Cn), q2));
-        const double na_i = __builtin_fma(l, y_i, a_i), na_j = __builtin_fma(-l, y_j, j2 == i ? na_i : a_j);
-        auto bits = [&](double a, double y) {
-            const unsigned u = room_up(a, y, half_Cp) > 0 ? 1u : 0u, w = room_low(a, y, half_Cn) > 0 ? (1u << NP) : 0u;
-            return (u | w) << (NU && y < 0 ? 1 : 0);
+        const double l = fmin_f64(bound_i.hi - z_i, fmin_f64(z_j - bound_j.lo, q2));
+        const double nz_i = z_i + l, nz_j = (j2 == i ? nz_i : z_j) - l;
+        auto bits = [&](double z, const SvBound &bound, int s) {
+            const unsigned u = z < bound.hi ? 1u : 0u, w = z > bound.lo ? (1u << NP) : 0u;
+            return (u | w) << (NU && s >= map.n0p ? 1 : 0);
         };
-        member = set_member_bits<E, 2 * NP>(member, tid, i, bits(na_i, y_i));
-        member = set_member_bits<E, 2 * NP>(member, tid, j2, bits(na_j, y_j));
-        write_by_lane0(go_on, &sh.a[wave][i], na_i, &sh.a[wave][j2], na_j);
+        member = set_member_bits<E, 2 * NP>(member, tid, i, bits(nz_i, bound_i, i));
+        member = set_member_bits<E, 2 * NP>(member, tid, j2, bits(nz_j, bound_j, j2));
+        write_by_lane0(go_on, &sh.z[wave][i], nz_i, &sh.z[wave][j2], nz_j);
         SV_PIN;
 #pragma unroll
         for (int e = 0; e < E; ++e) f[e] = __builtin_fma(-l, (double) kJ[e] - (double) (second ? kI[NP - 1][e] : kI[0][e]), f[e]);
@@ -520,14 +521,14 @@ __global__ __launch_bounds__(64 * W) void smo_small_kernel(const tsvm_small_prob
     for (int e = 0; e < E; ++e) {
         const int s = tid * E + e;
         act[e] = map.active(s);
-        const double a = act[e] ? alpha[map.index(s)] : 0.0;
+        const double z = act[e] ? alpha[map.index(s)] * map.label(s) : 0.0;
         f[e] = act[e] ? f_out[map.index(s)] : 0.0;
         kd[e] = act[e] ? P.k_diag[map.row(s)] : 1.0;
         sh.kd[s] = kd[e];
 #pragma unroll
-        for (int w = 0; w < W; ++w) sh.a[w][s] = a;
+        for (int w = 0; w < W; ++w) sh.z[w][s] = z;
     }
-    const double y = map.label(tid * E);   // (a thread's four slots are of one group)
+    const SvBound bound = map.bound(tid * E, P.Cp, P.Cn);   // (a thread's four slots are of one group)
     // (a vector that starts at an active slot may end in the columns behind the group's, which nothing uses, or up to
     // three elements behind the matrix)
     const int col = act[0] ? map.row(tid * E) : 0;
@@ -572,7 +573,7 @@ __global__ __launch_bounds__(64 * W) void smo_small_kernel(const tsvm_small_prob
         return filled;
     };
     if (start) {   // f from a non-zero alpha, in batches of 101 rows (csmosolver.cpp:189-214)
-        const int n = make_list(N, [&](int s) { return map.active(s) ? -sh.a[wave][s] * map.label(s) : 0.0; }, [&](int s) { return map.row(s); });
+        const int n = make_list(N, [&](int s) { return map.active(s) ? -sh.z[wave][s] : 0.0; }, [&](int s) { return map.row(s); });
         for (int t = 0; t < n; t += 101) ss_update_f<E, W, TB>(sh, K, ld, col, t, t + 101 < n ? t + 101 : n, f);
         __syncthreads();
     }
@@ -603,11 +604,11 @@ __global__ __launch_bounds__(64 * W) void smo_small_kernel(const tsvm_small_prob
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const int s = tid * E + e;
-            const double a = sh.a[wave][s];
+            const double z = sh.z[wave][s];
             unsigned b = 0;
             if (act[e]) {
-                const unsigned u = is_I_up(a, y, P.Cp, P.Cn) ? 1u : 0u, l = is_I_low(a, y, P.Cp, P.Cn) ? 1u : 0u;
-                b = NU ? (u | l << 2) << (y > 0 ? 0 : 1) : (u | l << 1);
+                const unsigned u = z < bound.hi ? 1u : 0u, l = z > bound.lo ? 1u : 0u;
+                b = NU ? (u | l << 2) << (s < map.n0p ? 0 : 1) : (u | l << 1);
             }
             member_all |= b << ((NU ? 4 : 2) * e);
             sh.flags[s] = (unsigned char) (sh.pos[s] == 0xffff ? b : 0u);
@@ -620,14 +621,14 @@ __global__ __launch_bounds__(64 * W) void smo_small_kernel(const tsvm_small_prob
         for (int t = tid; t < ws; t += 64 * W) sh.pos[sh.ws[t]] = (unsigned short) t;
         __syncthreads();
         unsigned member = 0;
-        double fl[E], a_old[E], mn[2] = {__builtin_inf(), __builtin_inf()}, mx[2] = {-__builtin_inf(), -__builtin_inf()};
+        double fl[E], z_old[E], mn[2] = {__builtin_inf(), __builtin_inf()}, mx[2] = {-__builtin_inf(), -__builtin_inf()};
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const int s = tid * E + e, p = sh.pos[s];
             const unsigned b = p != 0xffff ? (member_all >> ((NU ? 4 : 2) * e)) & (NU ? 15u : 3u) : 0u;
             member |= b << ((NU ? 4 : 2) * e);
             fl[e] = f[e];
-            a_old[e] = sh.a[wave][s];
+            z_old[e] = sh.z[wave][s];
 #pragma unroll
             for (int r = 0; r < (NU ? 2 : 1); ++r) {
                 mn[r] = fmin_f64(mn[r], (b >> r) & 1u ? f[e] : __builtin_inf());
@@ -662,7 +663,7 @@ __global__ __launch_bounds__(64 * W) void smo_small_kernel(const tsvm_small_prob
         __syncthreads();
         double *const old = sh.k;   // (free between the local solver and the list)
 #pragma unroll
-        for (int e = 0; e < E; ++e) old[tid * E + e] = a_old[e];
+        for (int e = 0; e < E; ++e) old[tid * E + e] = z_old[e];
         __syncthreads();
         double ad[E];
         int rr[E], cnt = 0;
@@ -670,7 +671,7 @@ __global__ __launch_bounds__(64 * W) void smo_small_kernel(const tsvm_small_prob
         for (int h = 0; h < E; ++h) {   // thread t owns entries E t .. E t + E - 1
             const int t = tid * E + h;
             const int s = t < ws ? sh.ws[t] : 0;
-            ad[h] = t < ws ? -(sh.a[wave][s] - old[s]) * map.label(s) : 0.0;
+            ad[h] = t < ws ? -(sh.z[wave][s] - old[s]) : 0.0;
             rr[h] = map.row(s);
             cnt += ad[h] != 0.0;
         }
@@ -719,7 +720,7 @@ __global__ __launch_bounds__(64 * W) void smo_small_kernel(const tsvm_small_prob
     for (int e = 0; e < E; ++e) {
         const int s = tid * E + e;
         if (act[e]) {
-            alpha[map.index(s)] = sh.a[wave][s];
+            alpha[map.index(s)] = sh.z[wave][s] * map.label(s) + 0.0;   // (+ 0.0: a zero comes out as +0, as from alpha +- l)
             f_out[map.index(s)] = f[e];
         }
     }

@@ -184,19 +184,16 @@ __device__ __forceinline__ bool solver_elected(int *gate, int epoch, int target_
     return s_elected != 0;
 }
 
-// What the nu solver keeps in LDS, per element of the working set.
+// What the nu solver keeps in LDS, per element of the working set (inactive elements: both bounds zero, so neither in
+// I_up nor in I_low).
 template <int N, int W>
 struct SvShared {
-    double kd[N], y[N];       // diagonal, label (0: inactive element)
-    double a[W][N];           // alpha: every wavefront keeps a copy of its own, which needs no barrier
+    double kd[N];
+    SvBound bound[N];
+    double z[W][N];           // alpha times its label: every wavefront keeps a copy of its own, which needs no barrier
 };
 
-// What c_smo_solve keeps.  alpha is held times its label, z = y * alpha in [lo, hi] with lo = 0, hi = Cp for y > 0 and
-// lo = -Cn, hi = 0 for y < 0: an element is in I_up while z < hi and in I_low while z > lo, and a step moves z_i up and z_j
-// down by the same l.  All of it rounds as the reference's expressions in alpha do (they differ in the sign of both operands).
-struct __align__(16) SvBound {
-    double hi, lo;
-};
+// What c_smo_solve keeps.
 struct __align__(16) SvStep {   // f_t - up and K_ii + K_tt - 2 K_it of a candidate for j2
     double b, a;
 };
@@ -590,9 +587,9 @@ __global__ __launch_bounds__(64 * W) void c_smo_solve_kernel(
 // code's j2n score, which uses kd[ip] and K[ip, .] (smo_kernel.cpp:239), and leaves diff[1] alone.
 // Membership bits per element: 0 = y>0 & a<C (I_up, positive), 1 = y<0 & a>0 (I_up, negative),
 // 2 = y>0 & a>0 (I_low, positive), 3 = y<0 & a<C (I_low, negative).
-__device__ __forceinline__ unsigned nu_member_bits(double a, double y, double half_C) {
-    const unsigned b = (room_up(a, y, half_C) > 0 ? 1u : 0u) | (room_low(a, y, half_C) > 0 ? 4u : 0u);
-    return y > 0 ? b : b << 1;
+__device__ __forceinline__ unsigned nu_member_bits(double z, const SvBound &bound) {
+    const unsigned b = (z < bound.hi ? 1u : 0u) | (z > bound.lo ? 4u : 0u);
+    return bound.hi > 0 ? b : b << 1;
 }
 
 template <int E, int W, int LDK, typename TB>
@@ -612,7 +609,7 @@ __global__ __launch_bounds__(64 * W) void nu_smo_solve_kernel(
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     double f[E], a_old[E], kd[E];
-    unsigned member = 0;
+    unsigned member = 0, plus = 0;   // plus: bit e: element e has a label > 0
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const int t = tid * E + e;
@@ -623,10 +620,12 @@ __global__ __launch_bounds__(64 * W) void nu_smo_solve_kernel(
         const double y = active ? (double) label[w] : 0.0;
         kd[e] = active ? k_diag[w] : 1.0;
         sh.kd[t] = kd[e];
-        sh.y[t] = y;
+        sh.bound[t].hi = y > 0 ? C : 0.0;
+        sh.bound[t].lo = y < 0 ? -C : 0.0;
+        plus |= (y > 0 ? 1u : 0u) << e;
 #pragma unroll
-        for (int w = 0; w < W; ++w) sh.a[w][t] = a_old[e];
-        member |= (active ? nu_member_bits(a_old[e], y, 0.5 * C) : 0u) << (4 * e);
+        for (int w = 0; w < W; ++w) sh.z[w][t] = a_old[e] * y;
+        member |= nu_member_bits(a_old[e] * y, sh.bound[t]) << (4 * e);
     }
     // initial gap -> local stopping threshold (smo_kernel.cpp:176-183); inside the loop the stopping
     // test is evaluated per element, as in the C variant
@@ -658,7 +657,6 @@ __global__ __launch_bounds__(64 * W) void nu_smo_solve_kernel(
     }
     __syncthreads();
     const bool none_possible = __builtin_amdgcn_readfirstlane(local_eps > 0.0 ? 0 : 1) != 0;
-    const double half_C = 0.5 * C;
     int numOfIter = 0;
     while (true) {
         double fup[E], fun[E];
@@ -741,17 +739,18 @@ __global__ __launch_bounds__(64 * W) void nu_smo_solve_kernel(
         TB kJ[E];
         load_row_elems<E, TB>(kws + (unsigned) j2 * (unsigned) LDK, tid, kJ);
         SV_PIN_MEMORY;
-        const double kd_j = sh.kd[j2], y_j = sh.y[j2], a_j = sh.a[wave][j2], y_i = sh.y[i], a_i = sh.a[wave][i], f_j = s_f[side][j2];
+        const double kd_j = sh.kd[j2], z_j = sh.z[wave][j2], z_i = sh.z[wave][i], f_j = s_f[side][j2];
+        const SvBound bound_i = sh.bound[i], bound_j = sh.bound[j2];
         const double kIj = (double) *(const TB *) (s_k[side] + j2);
         SV_PIN;   // the row is on its way while the exit test and the step are computed
         if (numOfIter > max_iter || !go) break;
         const double up_value = take_p ? up_value_p : up_value_n;
         const double q2 = (-up_value + f_j) / __builtin_fma(-2.0, kIj, (take_p ? kd_ip : kd_in) + kd_j);
-        const double l = fmin_f64(room_up(a_i, y_i, half_C), fmin_f64(room_low(a_j, y_j, half_C), q2));
-        const double na_i = __builtin_fma(l, y_i, a_i), na_j = __builtin_fma(-l, y_j, j2 == i ? na_i : a_j);   // (labels are +-1: exact products)
-        member = set_member_bits<E, 4>(member, tid, i, nu_member_bits(na_i, y_i, half_C));
-        member = set_member_bits<E, 4>(member, tid, j2, nu_member_bits(na_j, y_j, half_C));
-        write_by_lane0(1, &sh.a[wave][i], na_i, &sh.a[wave][j2], na_j);
+        const double l = fmin_f64(bound_i.hi - z_i, fmin_f64(z_j - bound_j.lo, q2));
+        const double nz_i = z_i + l, nz_j = (j2 == i ? nz_i : z_j) - l;
+        member = set_member_bits<E, 4>(member, tid, i, nu_member_bits(nz_i, bound_i));
+        member = set_member_bits<E, 4>(member, tid, j2, nu_member_bits(nz_j, bound_j));
+        write_by_lane0(1, &sh.z[wave][i], nz_i, &sh.z[wave][j2], nz_j);
         SV_PIN;   // (nothing above waits for the row)
 #pragma unroll
         for (int e = 0; e < E; ++e) f[e] = __builtin_fma(-l, (double) kJ[e] - (double) (take_p ? kIp[e] : kIn[e]), f[e]);
@@ -761,8 +760,9 @@ __global__ __launch_bounds__(64 * W) void nu_smo_solve_kernel(
     for (int e = 0; e < E; ++e) {
         const int t = tid * E + e;
         if (t < ws) {
-            const double a = sh.a[wave][t];
-            alpha_diff[t] = -(a - a_old[e]) * sh.y[t];
+            const double y = (plus >> e) & 1u ? 1.0 : -1.0;
+            const double a = sh.z[wave][t] * y + 0.0;   // (+ 0.0: a zero comes out as +0, as from alpha +- l)
+            alpha_diff[t] = -(a - a_old[e]) * y;
             alpha[working_set[t]] = a;
         }
     }
