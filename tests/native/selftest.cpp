@@ -1,12 +1,13 @@
 // Self-tests of host-layer pieces that have no other way in from a test: the device buffer type that stands in for
 // the reference's SyncArray (the cases of src/test/test_syncmem.cpp and test_syncarray.cpp that apply), the kernel-row
-// cache's bookkeeping, and the host's bounded wait for the local solver.  Built into a library of its own, next to
+// cache's bookkeeping, the host's bounded wait for the local solver, and the matrices of the scikit entry points.  Built into a library of its own, next to
 // the tests; the product libraries do not contain it.
 #include <chrono>
 #include <stdexcept>
 #include <string>
 #include <vector>
 
+#include "../../thundersvm_amd/host/dataset.h"
 #include "../../thundersvm_amd/host/device.h"
 #include "../../thundersvm_amd/host/row_cache.h"
 #include "../../thundersvm_amd/host/solver.h"
@@ -150,6 +151,25 @@ int tsvm_selftest_solver_wait(int timeout_ms, int never_written) {
     }
     g_selftest_error = "the wait returned although the word never changed";
     return -1;
+}
+
+// No device needed.  DataSet::load_from_sparse (dense == 0) or load_from_dense (row_ptr and col_ptr unused) and the rows it
+// holds afterwards: out_ptr [row_size + 1], out_col / out_val with room for `cap` entries.  Returns the entries, -1 when refused.
+long long tsvm_selftest_load_matrix(int dense, int row_size, int features, float *val, int *row_ptr, int *col_ptr, long long *out_ptr,
+                                    int *out_col, double *out_val, long long cap) {
+    try {
+        DataSet ds;
+        if (dense) ds.load_from_dense(row_size, features, val, nullptr);
+        else ds.load_from_sparse(row_size, val, row_ptr, col_ptr, nullptr);
+        const RowStore &R = ds.rows();
+        const long long nnz = (long long) R.nnz();
+        for (size_t r = 0; r <= R.size(); ++r) out_ptr[r] = R.ptr()[r];
+        for (long long e = 0; e < nnz && e < cap; ++e) { out_col[e] = R.col()[e]; out_val[e] = R.val()[e]; }
+        return nnz;
+    } catch (const std::exception &e) {
+        g_selftest_error = e.what();
+        return -1;
+    }
 }
 
 }  // extern "C"

@@ -214,19 +214,23 @@ void DataSet::load_from_python(float *y, char **x, int len) {
     set_rows(RowStore::from_nodes(nodes));
 }
 
+// (a row whose end lies before its start is an empty one)
 void DataSet::load_from_sparse(int row_size, float *val, int *row_ptr, int *col_ptr, float *label) {
+    if (row_size < 0) throw std::length_error("DataSet: negative number of rows");
     y_.assign(label, label + (label ? row_size : 0));
     n_features_ = 0;
-    const size_t nnz = (size_t) std::max(row_ptr[row_size] - row_ptr[0], 0);
+    size_t nnz = 0;
+    for (int r = 0; r < row_size; ++r) nnz += (size_t) std::max(row_ptr[r + 1] - row_ptr[r], 0);
     auto rows = std::make_shared<RowStore>((size_t) row_size, nnz);
+    int64_t *const to = rows->ptr_mut();
+    for (int r = 0; r < row_size; ++r) to[r + 1] = to[r] + std::max(row_ptr[r + 1] - row_ptr[r], 0);
     int max_index = 0;
 #pragma omp parallel for schedule(static) reduction(max : max_index) num_threads(threads_for(nnz))
     for (int r = 0; r < row_size; ++r) {
-        rows->ptr_mut()[r + 1] = row_ptr[r + 1] - row_ptr[0];
-        for (int e = row_ptr[r]; e < row_ptr[r + 1]; ++e) {
+        for (int64_t at = to[r], e = row_ptr[r]; at < to[r + 1]; ++at, ++e) {
             const int ind = col_ptr[e] + 1;  // to one-based
-            rows->col_mut()[e - row_ptr[0]] = ind;
-            rows->val_mut()[e - row_ptr[0]] = val[e];
+            rows->col_mut()[at] = ind;
+            rows->val_mut()[at] = val[e];
             max_index = std::max(max_index, ind);
         }
     }
@@ -235,6 +239,7 @@ void DataSet::load_from_sparse(int row_size, float *val, int *row_ptr, int *col_
 }
 
 void DataSet::load_from_dense(int row_size, int features, float *data, float *label) {
+    if (row_size < 0 || (row_size > 0 && features < 0)) throw std::length_error("DataSet: negative matrix size");
     y_.assign(label, label + (label ? row_size : 0));
     const size_t nnz = (size_t) row_size * features;
     auto rows = std::make_shared<RowStore>((size_t) row_size, nnz);
@@ -252,11 +257,18 @@ void DataSet::load_from_dense(int row_size, int features, float *data, float *la
 }
 
 void DataSet::load_from_csr(int64_t n, const int64_t *row_ptr, const int *col, const double *val, const double *y, bool keep) {
+    // (the rows are copied in blocks and gathered by these pointers later: what they say has to hold)
+    if (n < 0) throw std::length_error("DataSet: negative number of rows");
+    int decreasing = 0;
+#pragma omp parallel for schedule(static) reduction(| : decreasing) num_threads(threads_for((size_t) n))
+    for (int64_t r = 0; r < n; ++r) decreasing |= row_ptr[r + 1] < row_ptr[r];
+    if (decreasing) throw std::length_error("DataSet: a row ends before it begins (decreasing row pointer)");
     y_.assign(y, y + (y ? n : 0));
-    std::shared_ptr<const RowStore> rows = keep ? RowStore::copy_of((size_t) n, row_ptr, col, val)
-                                                : std::make_shared<RowStore>((size_t) n, row_ptr, col, val);
+    std::shared_ptr<const RowStore> rows = n == 0  ? std::make_shared<RowStore>(0, 0)   // (no pointer is looked at)
+                                           : keep ? RowStore::copy_of((size_t) n, row_ptr, col, val)
+                                                  : std::make_shared<RowStore>((size_t) n, row_ptr, col, val);
     int max_index = 0, zero = 0;
-    const int64_t lo = row_ptr[0], hi = row_ptr[n];
+    const int64_t lo = n ? row_ptr[0] : 0, hi = n ? row_ptr[n] : 0;
 #pragma omp parallel for schedule(static) reduction(max : max_index, zero) num_threads(threads_for((size_t) (hi - lo)))
     for (int64_t e = lo; e < hi; ++e) {
         max_index = std::max(max_index, col[e]);
