@@ -86,3 +86,14 @@ def test_scikit_matrix_of_a_negative_size_is_refused(dense, rows, features):
     buf = np.zeros(64)
     at = buf.ctypes.data
     assert L.tsvm_selftest_load_matrix(dense, rows, features, at, at, at, at, at, at, 0) == -1
+
+
+@pytest.mark.parametrize("entries", [3, 200000])
+def test_feature_id_zero_in_csr_rows_is_noticed(entries):
+    """One feature id 0 anywhere makes a data set zero-based (it moves every feature's place in the linear coefficients)."""
+    rng = np.random.default_rng(entries)
+    csr = D.CsrData(np.array([0, 2, entries], np.int64), rng.integers(1, 9, entries).astype(np.int32), np.ones(entries), np.array([1.0, 0.0]))
+    csr.col[1] = 9
+    assert M.Dataset(csr).csr()[1:] == (9, False)
+    csr.col[entries - 1] = 0
+    assert M.Dataset(csr).csr()[1:] == (9, True)

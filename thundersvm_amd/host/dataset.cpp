@@ -269,7 +269,7 @@ void DataSet::load_from_csr(int64_t n, const int64_t *row_ptr, const int *col, c
                                                   : std::make_shared<RowStore>((size_t) n, row_ptr, col, val);
     int max_index = 0, zero = 0;
     const int64_t lo = n ? row_ptr[0] : 0, hi = n ? row_ptr[n] : 0;
-#pragma omp parallel for schedule(static) reduction(max : max_index, zero) num_threads(threads_for((size_t) (hi - lo)))
+#pragma omp parallel for schedule(static) reduction(max : max_index) reduction(| : zero) num_threads(threads_for((size_t) (hi - lo)))
     for (int64_t e = lo; e < hi; ++e) {
         max_index = std::max(max_index, col[e]);
         zero |= col[e] == 0;
