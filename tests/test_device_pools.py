@@ -1,0 +1,13 @@
+"""The host layer's pools of device blocks and events with two devices: tests/native/two_devices.cpp, a program whose
+stand-ins for the HIP calls know two.  Host only."""
+import os
+import subprocess
+
+import selftest_lib
+
+
+def test_blocks_and_events_go_back_to_their_own_device():
+    selftest_lib.lib()
+    exe = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native", "two_devices")
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout == "ok\n", r.stderr

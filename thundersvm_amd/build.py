@@ -53,13 +53,17 @@ def build_host(extra=()):
 
 
 def build_selftests():
-    """The test-only library (tests/native): self-tests of host-layer pieces, linked against the host library."""
-    src = os.path.join(os.path.dirname(HERE), "tests", "native", "selftest.cpp")
-    if not os.path.exists(src):
+    """The test-only library and program (tests/native): self-tests of host-layer pieces, linked against the host library."""
+    native = os.path.join(os.path.dirname(HERE), "tests", "native")
+    out = os.path.join(native, "libtsvm_selftest.so")
+    links = ["-L", HERE, "-lthundersvm", "-ltsvm_hip", "-Wl,-rpath,$ORIGIN/../../thundersvm_amd", "-L/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib"]
+    if not os.path.exists(os.path.join(native, "selftest.cpp")):
         return None
-    out = os.path.join(os.path.dirname(src), "libtsvm_selftest.so")
-    _run(["g++", "-O2", "-fPIC", "-std=c++17", "-fopenmp", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", src, "-shared", "-o", out,
-          "-L", HERE, "-lthundersvm", "-ltsvm_hip", "-Wl,-rpath,$ORIGIN/../../thundersvm_amd", "-L/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib"])
+    _run(["g++", "-O2", "-fPIC", "-std=c++17", "-fopenmp", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", os.path.join(native, "selftest.cpp"),
+          "-shared", "-o", out, *links])
+    # (-rdynamic: its stand-ins for the HIP calls take the place of the runtime's in the host library)
+    _run(["g++", "-O2", "-std=c++17", "-fopenmp", "-rdynamic", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", os.path.join(native, "two_devices.cpp"),
+          "-o", os.path.join(native, "two_devices"), *links])
     return out
 
 

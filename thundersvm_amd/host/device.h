@@ -40,13 +40,13 @@ hipStream_t work_stream();
 // Blocks are rounded up to quarter powers of two; blocks above 64 MiB and whatever would take the pool over 512 MiB go
 // back to the driver, everything does when the device runs out of memory, on tsvm_release_device_cache() and when the
 // process ends.  A block is handed out again only after the device has been idle since its release (as hipFree would
-// have waited for), unless whoever released it knows that nothing uses it any more (`idle`).  One list per device; any
-// number of threads.
+// have waited for), unless whoever released it knows that nothing uses it any more (`idle`).  One list per device, a
+// block's own, whichever is current when it is released; any number of threads.
 class DevicePool {
 public:
     static DevicePool &instance();
-    void *take(size_t bytes);
-    void give(void *p, size_t bytes, bool idle);
+    void *take(size_t bytes, int *device);   // *device: the current device, whose memory it is
+    void give(void *p, size_t bytes, int device, bool idle);
     void flush();
     // While one exists on a thread, what the thread releases counts as idle.
     struct Idle {
@@ -60,15 +60,20 @@ private:
     Impl &impl();
 };
 
-// Small page-locked, device-mapped host blocks (PINNED_BLOCK bytes each) and events without timing, kept likewise.
+// Small page-locked, device-mapped host blocks (PINNED_BLOCK bytes each; any device's) and events without timing, kept
+// likewise.  An event belongs to the device that was current when it was taken.
 constexpr size_t PINNED_BLOCK = 32768;
 struct PinnedBlock {
     char *host = nullptr, *dev = nullptr;
 };
 PinnedBlock take_pinned_block();
 void give_pinned_block(const PinnedBlock &b);
-hipEvent_t take_event();
-void give_event(hipEvent_t e);
+struct DeviceEvent {
+    hipEvent_t event = nullptr;
+    int device = -1;
+};
+DeviceEvent take_event();
+void give_event(const DeviceEvent &e);
 
 // Copies between pageable host memory and the device through a ring of page-locked chunks: the host fills (or empties)
 // one chunk while the others are on their way.  Asynchronous on `stream` as far as the device side goes; when upload()
@@ -131,9 +136,9 @@ public:
     explicit DeviceBuffer(size_t count) { resize(count); }
     DeviceBuffer(const DeviceBuffer &) = delete;
     DeviceBuffer &operator=(const DeviceBuffer &) = delete;
-    DeviceBuffer(DeviceBuffer &&o) noexcept : ptr_(o.ptr_), count_(o.count_) { o.ptr_ = nullptr; o.count_ = 0; }
+    DeviceBuffer(DeviceBuffer &&o) noexcept : ptr_(o.ptr_), count_(o.count_), device_(o.device_) { o.ptr_ = nullptr; o.count_ = 0; }
     DeviceBuffer &operator=(DeviceBuffer &&o) noexcept {
-        if (this != &o) { release(); ptr_ = o.ptr_; count_ = o.count_; o.ptr_ = nullptr; o.count_ = 0; }
+        if (this != &o) { release(); ptr_ = o.ptr_; count_ = o.count_; device_ = o.device_; o.ptr_ = nullptr; o.count_ = 0; }
         return *this;
     }
     ~DeviceBuffer() { release(); }
@@ -142,7 +147,7 @@ public:
         if (count == count_) return;
         release();
         if (count) {
-            ptr_ = (T *) DevicePool::instance().take(count * sizeof(T));
+            ptr_ = (T *) DevicePool::instance().take(count * sizeof(T), &device_);
             device_bytes_in_use() += count * sizeof(T);
         }
         count_ = count;
@@ -151,7 +156,7 @@ public:
     // device has been idle)
     void release(bool idle = false) {
         if (ptr_) {
-            DevicePool::instance().give(ptr_, count_ * sizeof(T), idle);
+            DevicePool::instance().give(ptr_, count_ * sizeof(T), device_, idle);
             device_bytes_in_use() -= count_ * sizeof(T);
         }
         ptr_ = nullptr;
@@ -180,6 +185,7 @@ public:
 private:
     T *ptr_ = nullptr;
     size_t count_ = 0;
+    int device_ = -1;   // whose memory it is
 };
 
 // Page-locked host staging memory that only grows (hipHostMalloc; copies from it are asynchronous and run at

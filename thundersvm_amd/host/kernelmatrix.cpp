@@ -12,6 +12,12 @@
 using tsvm::abi_check;
 
 namespace tsvm {
+static int current_device() {
+    int dev = 0;
+    TSVM_HIP_CHECK(hipGetDevice(&dev));
+    return dev;
+}
+
 struct DevicePool::Impl {
     static constexpr size_t MAX_BLOCK = (size_t) 64 << 20, MAX_TOTAL = (size_t) 512 << 20;
     std::mutex mu;
@@ -26,11 +32,6 @@ struct DevicePool::Impl {
         const size_t q = p / 8;   // between p/2 and p: p/2 + k * p/8
         return p / 2 + (bytes - p / 2 + q - 1) / q * q;
     }
-    static int device() {
-        int dev = 0;
-        TSVM_HIP_CHECK(hipGetDevice(&dev));
-        return dev;
-    }
     void flush_locked() {
         for (auto *m : {&ready, &waiting}) {
             for (auto &kv : *m)
@@ -44,8 +45,7 @@ struct DevicePool::Impl {
 hipStream_t work_stream() {
     static std::mutex mu;
     static std::map<int, hipStream_t> streams;
-    int dev = 0;
-    TSVM_HIP_CHECK(hipGetDevice(&dev));
+    const int dev = current_device();
     std::lock_guard<std::mutex> lock(mu);
     auto it = streams.find(dev);
     if (it == streams.end()) {
@@ -79,9 +79,9 @@ DevicePool::Impl &DevicePool::impl() {
     return *i;
 }
 
-void *DevicePool::take(size_t bytes) {
+void *DevicePool::take(size_t bytes, int *device) {
     Impl &I = impl();
-    const int dev = Impl::device();
+    const int dev = *device = current_device();
     const size_t size = Impl::block_size(bytes);
     std::lock_guard<std::mutex> lock(I.mu);
     const auto key = std::make_pair(dev, size);
@@ -115,16 +115,15 @@ void *DevicePool::take(size_t bytes) {
     return p;
 }
 
-void DevicePool::give(void *p, size_t bytes, bool idle) {
+void DevicePool::give(void *p, size_t bytes, int device, bool idle) {
     Impl &I = impl();
     const size_t size = Impl::block_size(bytes);
     std::lock_guard<std::mutex> lock(I.mu);
-    int dev = 0;
-    if (size > Impl::MAX_BLOCK || I.total + size > Impl::MAX_TOTAL || hipGetDevice(&dev) != hipSuccess) {
+    if (size > Impl::MAX_BLOCK || I.total + size > Impl::MAX_TOTAL) {
         (void) hipFree(p);
         return;
     }
-    (idle || Idle::depth() > 0 ? I.ready : I.waiting)[std::make_pair(dev, size)].push_back(p);
+    (idle || Idle::depth() > 0 ? I.ready : I.waiting)[std::make_pair(device, size)].push_back(p);
     I.total += size;
 }
 
@@ -183,36 +182,34 @@ void give_pinned_block(const PinnedBlock &b) {
     else (void) hipHostFree(b.host);
 }
 
-hipEvent_t take_event() {
+DeviceEvent take_event() {
     HostPool &h = host_pool();
-    int dev = 0;
-    TSVM_HIP_CHECK(hipGetDevice(&dev));
+    DeviceEvent e;
+    e.device = current_device();
     {
         std::lock_guard<std::mutex> lock(h.mu);
-        std::vector<hipEvent_t> &v = h.events[dev];
+        std::vector<hipEvent_t> &v = h.events[e.device];
         if (!v.empty()) {
-            const hipEvent_t e = v.back();
+            e.event = v.back();
             v.pop_back();
             return e;
         }
     }
-    hipEvent_t e = nullptr;
-    TSVM_HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    TSVM_HIP_CHECK(hipEventCreateWithFlags(&e.event, hipEventDisableTiming));
     return e;
 }
 
-void give_event(hipEvent_t e) {
+void give_event(const DeviceEvent &e) {
     HostPool &h = host_pool();
-    int dev = 0;
-    if (hipGetDevice(&dev) == hipSuccess) {
+    {
         std::lock_guard<std::mutex> lock(h.mu);
-        std::vector<hipEvent_t> &v = h.events[dev];
+        std::vector<hipEvent_t> &v = h.events[e.device];
         if (v.size() < HOST_POOL_MAX) {
-            v.push_back(e);
+            v.push_back(e.event);
             return;
         }
     }
-    (void) hipEventDestroy(e);
+    (void) hipEventDestroy(e.event);
 }
 
 void parallel_memcpy(void *to, const void *from, size_t bytes) {
@@ -231,8 +228,7 @@ struct HostStaging::Impl {
     std::mutex mu;
     struct Chunk {
         char *host = nullptr;
-        hipEvent_t event = nullptr;
-        int device = -1;   // the event's device; -1: nothing pending
+        DeviceEvent pending;   // (no event: nothing is on its way)
     } chunk[CHUNKS];
     int next = 0;
     Chunk &take() {
@@ -243,15 +239,14 @@ struct HostStaging::Impl {
         return c;
     }
     void wait(Chunk &c) {
-        if (c.device < 0) return;
-        TSVM_HIP_CHECK(hipEventSynchronize(c.event));
-        give_event(c.event);
-        c.device = -1;
+        if (!c.pending.event) return;
+        TSVM_HIP_CHECK(hipEventSynchronize(c.pending.event));
+        give_event(c.pending);
+        c.pending = DeviceEvent();
     }
     void record(Chunk &c, hipStream_t stream) {
-        c.event = take_event();
-        TSVM_HIP_CHECK(hipEventRecord(c.event, stream));
-        TSVM_HIP_CHECK(hipGetDevice(&c.device));
+        c.pending = take_event();
+        TSVM_HIP_CHECK(hipEventRecord(c.pending.event, stream));
     }
 };
 

@@ -185,13 +185,13 @@ struct SolveTask::Impl {
     // The chip-wide work of a task is enqueued on stream `sa` (`ids` is the stream the newly selected ids are read
     // back on for the host-side cache bookkeeping: the same one).
     hipStream_t sa = nullptr, ids = nullptr;
-    hipEvent_t selected = nullptr, diff_ready = nullptr;
+    tsvm::DeviceEvent selected, diff_ready;
     // A task that runs alone splits the chip: the local solver (one workgroup, a chain of dependent steps) gets a
     // stream `ss` restricted to one CU of every XCD, everything else runs on `sa`, restricted to the other CUs.
     // The solver then runs next to this iteration's get_rows at nearly its stand-alone speed; sharing CUs with a
     // chip-wide kernel it runs two to three times slower, which is why tasks in lockstep keep the phases apart.
     hipStream_t ss = nullptr;
-    hipEvent_t block_done = nullptr, solved = nullptr;
+    tsvm::DeviceEvent block_done, solved;
     bool split = false;
     // Once the cache holds every row there is no get_rows left to run next to the solver; the iteration then
     // stays on `sa` from start to end and saves the two hand-overs between the streams.
@@ -253,7 +253,7 @@ struct SolveTask::Impl {
     std::chrono::steady_clock::time_point solver_enqueued, next_stream_check;
     bool diff_arrived() {
         if (wait_by_event) {
-            const hipError_t e = hipEventQuery(diff_ready);
+            const hipError_t e = hipEventQuery(diff_ready.event);
             if (e == hipSuccess) return true;
             if (e != hipErrorNotReady) TSVM_HIP_CHECK(e);
             return false;
@@ -428,9 +428,9 @@ struct SolveTask::Impl {
             upload_rotation(cur_slots);
         }
         solver.init_f(alpha, y, k_mat, d_f);
-        TSVM_HIP_CHECK(hipEventRecord(solved, tsvm::work_stream()));   // the rows, the uploads and init_f
-        TSVM_HIP_CHECK(hipStreamWaitEvent(sa, solved, 0));
-        if (ss != sa) TSVM_HIP_CHECK(hipStreamWaitEvent(ss, solved, 0));
+        TSVM_HIP_CHECK(hipEventRecord(solved.event, tsvm::work_stream()));   // the rows, the uploads and init_f
+        TSVM_HIP_CHECK(hipStreamWaitEvent(sa, solved.event, 0));
+        if (ss != sa) TSVM_HIP_CHECK(hipStreamWaitEvent(ss, solved.event, 0));
 
         max_iter = std::max(100000, ws_size > INT_MAX / 100 ? INT_MAX : 100 * ws_size);
         timer.stream = sa;
@@ -474,8 +474,8 @@ struct SolveTask::Impl {
         for (DeviceBuffer<float_type> *b : {&d_alpha_diff, &d_kws}) b->release(true);
         d_start.release(true);
         d_sel_ws.release(true);
-        for (hipEvent_t e : {block_done, solved, selected, diff_ready})
-            if (e) tsvm::give_event(e);
+        for (const tsvm::DeviceEvent &e : {block_done, solved, selected, diff_ready})
+            if (e.event) tsvm::give_event(e);
         if (pinned.host) tsvm::give_pinned_block(pinned);
     }
 
@@ -696,8 +696,8 @@ struct SolveTask::Impl {
                                                   d_slots_a.data(), sa));
             slots = d_slots_a.data();
         } else if (block_on_solver_cus) {
-            TSVM_HIP_CHECK(hipEventRecord(selected, sa));   // the selection is the last thing enqueued on sa
-            TSVM_HIP_CHECK(hipStreamWaitEvent(ss, selected, 0));
+            TSVM_HIP_CHECK(hipEventRecord(selected.event, sa));   // the selection is the last thing enqueued on sa
+            TSVM_HIP_CHECK(hipStreamWaitEvent(ss, selected.event, 0));
             k_mat.get_block(ws_u(), ws_size, d_kws.data(), ldk, ss);
         } else if (block_first) {
             k_mat.get_block(ws_u(), ws_size, d_kws.data(), ldk, sa);
@@ -705,7 +705,7 @@ struct SolveTask::Impl {
             abi_check(tsvm_smo_gather_block(k_rows, row_type, slots, ld, ws_u(), ws_size, d_kws.data(), row_type, sa));
         }
         timer.end(stats.ms_local);
-        if (!on_one_stream && !block_on_solver_cus) TSVM_HIP_CHECK(hipEventRecord(block_done, sa));
+        if (!on_one_stream && !block_on_solver_cus) TSVM_HIP_CHECK(hipEventRecord(block_done.event, sa));
         // (beside the solver when it has a stream of its own, in front of it otherwise)
         if (split && !block_on_solver_cus)
             abi_check(tsvm_smo_warm_block(d_kws.data(), row_type, ws_size, solver_xcd, d_gate.data() + 3, sa));
@@ -721,7 +721,7 @@ struct SolveTask::Impl {
         }
         solver_enqueued = std::chrono::steady_clock::now();
         next_stream_check = solver_enqueued + std::chrono::milliseconds(200);
-        if (!on_one_stream && !block_on_solver_cus) TSVM_HIP_CHECK(hipStreamWaitEvent(ss, block_done, 0));
+        if (!on_one_stream && !block_on_solver_cus) TSVM_HIP_CHECK(hipStreamWaitEvent(ss, block_done.event, 0));
         if (solver_xcd >= 0) {   // elected onto this lane's XCD, where the block has been read (launches are ordered, whichever stream they are on)
             ++solver_epoch;
             if (nu)
@@ -740,11 +740,11 @@ struct SolveTask::Impl {
                                              Cp, Cn, d_kws.data(), row_type, k_mat.diag(), eps, d_diff, max_iter, st));
         }
         timer.end(stats.ms_local);
-        if (!on_one_stream) TSVM_HIP_CHECK(hipEventRecord(solved, ss));
+        if (!on_one_stream) TSVM_HIP_CHECK(hipEventRecord(solved.event, ss));
     }
 
     void enqueue_update() {
-        if (!on_one_stream) TSVM_HIP_CHECK(hipStreamWaitEvent(sa, solved, 0));   // alpha_diff, alpha and diff come from the solver
+        if (!on_one_stream) TSVM_HIP_CHECK(hipStreamWaitEvent(sa, solved.event, 0));   // alpha_diff, alpha and diff come from the solver
         if (select_ahead && fuse_select) {
             // the next selection's first pass over the instances rides on update_f's last one
             advance_window();
@@ -761,7 +761,7 @@ struct SolveTask::Impl {
             std::vector<float_type> ad = d_alpha_diff.to_host();
             for (float_type v : ad) stats.update_rows += v != 0;
         }
-        if (wait_by_event) TSVM_HIP_CHECK(hipEventRecord(diff_ready, sa));
+        if (wait_by_event) TSVM_HIP_CHECK(hipEventRecord(diff_ready.event, sa));
         if (select_ahead) {
             launch_select(iter + 1);
             select_enqueued = true;
@@ -769,7 +769,7 @@ struct SolveTask::Impl {
     }
 
     bool finish_iteration() {
-        if (wait_by_event) TSVM_HIP_CHECK(hipEventSynchronize(diff_ready));
+        if (wait_by_event) TSVM_HIP_CHECK(hipEventSynchronize(diff_ready.event));
         else wait_for_diff();
         const double diff0 = h_diff[0], diff1 = h_diff[1];
         local_iter += (long long) diff1;
