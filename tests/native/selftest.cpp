@@ -153,6 +153,34 @@ int tsvm_selftest_solver_wait(int timeout_ms, int never_written) {
     return -1;
 }
 
+// No device needed: the same wait by asking, for something that is never done, is done at the third look, or fails.
+// 0: as it should be.
+int tsvm_selftest_wait_until_done(int timeout_ms) {
+    static int looks;
+    const auto t0 = std::chrono::steady_clock::now();
+    try {
+        tsvm::wait_until_done([](void *) { return hipErrorNotReady; }, nullptr, timeout_ms);
+        return -1;
+    } catch (const std::runtime_error &e) {
+        g_selftest_error = e.what();
+        const double ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+        if (g_selftest_error.find("TSVM_SOLVER_TIMEOUT_MS") == std::string::npos || ms < timeout_ms || ms >= timeout_ms + 1000.0) return -2;
+    }
+    looks = 0;
+    try {
+        tsvm::wait_until_done([](void *) { return ++looks < 3 ? hipErrorNotReady : hipSuccess; }, nullptr, 10000);
+    } catch (const std::exception &) {
+        return -3;
+    }
+    if (looks != 3) return -4;
+    try {
+        tsvm::wait_until_done([](void *) { return hipErrorInvalidHandle; }, nullptr, 10000);
+        return -5;
+    } catch (const std::runtime_error &) {
+        return 0;
+    }
+}
+
 // No device needed.  DataSet::load_from_sparse (dense == 0) or load_from_dense (row_ptr and col_ptr unused) and the rows it
 // holds afterwards: out_ptr [row_size + 1], out_col / out_val with room for `cap` entries.  Returns the entries, -1 when refused.
 long long tsvm_selftest_load_matrix(int dense, int row_size, int features, float *val, int *row_ptr, int *col_ptr, long long *out_ptr,

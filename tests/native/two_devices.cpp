@@ -1,4 +1,5 @@
-// The pools of the host layer with two devices, which a single-GPU machine does not have: a program of its own whose
+// The pools of the host layer with two devices, which a single-GPU machine does not have, and the wait of a download for a
+// device that does not answer: a program of its own whose
 // definitions of the HIP calls stand in for the runtime's (the host library's calls resolve to them), hand out host memory and
 // remember which device every block, stream and event belongs to.  Exits with 0, or prints what went wrong.
 #include <cstdio>
@@ -10,6 +11,7 @@
 #include "../../thundersvm_amd/host/device.h"
 
 static int g_current = 0, g_failures = 0;
+static bool g_hung = false;                   // events are never reached
 static std::map<const void *, int> g_owner;   // device of every live block, stream and event
 
 static void expect(bool ok, const char *what) {
@@ -42,7 +44,7 @@ hipError_t hipStreamDestroy(hipStream_t s) { return drop(s); }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return make(e, 1); }
 hipError_t hipEventDestroy(hipEvent_t e) { return drop(e); }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
-hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventQuery(hipEvent_t) { return g_hung ? hipErrorNotReady : hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {   // (the runtime refuses this too)
     expect(g_owner.at(e) == g_owner.at(s), "an event is recorded on a stream of the other device");
     return hipSuccess;
@@ -86,6 +88,21 @@ int main() {
         tsvm::DeviceBuffer<int> x(data.size());
         for (int i = 0; i < 5; ++i) x.upload(data.data(), data.size());
         expect(g_owner.at(x.data()) == g_current, "an upload's buffer is on the other device");
+    }
+    // a download that is given a limit gives up on a device that has stopped answering, and the next one is whole
+    tsvm::DeviceBuffer<int> x(data.size());
+    x.upload(data.data(), data.size());
+    std::vector<int> back(data.size(), 0);
+    const auto take = [&](const char *from, size_t off, size_t len) { memcpy((char *) back.data() + off, from, len); };
+    for (int attempt = 0; attempt < 2; ++attempt) {
+        g_hung = attempt == 0;
+        bool gave_up = false;
+        try {
+            tsvm::HostStaging::instance().download(x.data(), data.size() * sizeof(int), take, tsvm::work_stream(), 20);
+        } catch (const std::runtime_error &) {
+            gave_up = true;
+        }
+        expect(gave_up == g_hung && back[0] == (g_hung ? 0 : 7), "a download with a limit");
     }
     if (g_failures == 0) puts("ok");
     return g_failures != 0;

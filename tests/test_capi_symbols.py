@@ -84,6 +84,7 @@ def test_bounded_wait_for_the_local_solver():
     assert b"TSVM_SOLVER_TIMEOUT_MS" in lib.tsvm_selftest_last_error()
     assert lib.tsvm_selftest_solver_wait(60000, 1) == 0, lib.tsvm_selftest_last_error()
     assert b"without reporting" in lib.tsvm_selftest_last_error()
+    assert lib.tsvm_selftest_wait_until_done(200) == 0, lib.tsvm_selftest_last_error()
 
 
 def test_row_cache_bookkeeping():

@@ -1,5 +1,5 @@
-"""The host layer's pools of device blocks and events with two devices: tests/native/two_devices.cpp, a program whose
-stand-ins for the HIP calls know two.  Host only."""
+"""The host layer's pools of device blocks and events with two devices, and the limit of a download's wait:
+tests/native/two_devices.cpp, a program with stand-ins for the HIP calls.  Host only."""
 import os
 import subprocess
 

@@ -90,8 +90,11 @@ public:
         size_t bytes, at;   // at: byte offset in the destination, ascending
     };
     void upload(void *dst, const std::vector<Part> &parts, hipStream_t stream);
-    // take(from, offset, length): bytes [offset, offset + length) have arrived
-    void download(const void *src, size_t bytes, const std::function<void(const char *, size_t, size_t)> &take, hipStream_t stream);
+    // take(from, offset, length): bytes [offset, offset + length) have arrived.  timeout_ms > 0: gives up (std::runtime_error)
+    // when nothing has arrived for that long, for a stream whose kernels may hang; whoever sets it leaves the stream's
+    // memory alone afterwards.
+    void download(const void *src, size_t bytes, const std::function<void(const char *, size_t, size_t)> &take, hipStream_t stream,
+                  long long timeout_ms = 0);
 
     static constexpr size_t CHUNK = (size_t) 4 << 20;
 
@@ -99,6 +102,9 @@ private:
     struct Impl;
     Impl &impl();
 };
+// Asks state_of(thing) until it says hipSuccess; throws any error but hipErrorNotReady, and std::runtime_error after
+// timeout_ms.
+void wait_until_done(hipError_t (*state_of)(void *), void *thing, long long timeout_ms);
 // memcpy on as many threads as pay for a block of this size
 void parallel_memcpy(void *to, const void *from, size_t bytes);
 

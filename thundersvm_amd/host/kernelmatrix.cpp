@@ -3,6 +3,7 @@
 #include <stdexcept>
 
 #include <algorithm>
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -223,6 +224,18 @@ void parallel_memcpy(void *to, const void *from, size_t bytes) {
     for (long i = 0; i < n; ++i) memcpy((char *) to + i * piece, (const char *) from + i * piece, std::min(piece, bytes - i * piece));
 }
 
+void wait_until_done(hipError_t (*state_of)(void *), void *thing, long long timeout_ms) {
+    const auto start = std::chrono::steady_clock::now();
+    for (;;) {
+        const hipError_t e = state_of(thing);
+        if (e == hipSuccess) return;
+        if (e != hipErrorNotReady) TSVM_HIP_CHECK(e);
+        if (std::chrono::steady_clock::now() - start > std::chrono::milliseconds(timeout_ms))
+            throw std::runtime_error("no result from the device after " + std::to_string(timeout_ms) +
+                                     " ms (TSVM_SOLVER_TIMEOUT_MS); the device may be hung");
+    }
+}
+
 struct HostStaging::Impl {
     static constexpr int CHUNKS = 4;
     std::mutex mu;
@@ -231,16 +244,17 @@ struct HostStaging::Impl {
         DeviceEvent pending;   // (no event: nothing is on its way)
     } chunk[CHUNKS];
     int next = 0;
-    Chunk &take() {
+    Chunk &take(long long timeout_ms = 0) {
         Chunk &c = chunk[next];
         next = (next + 1) % CHUNKS;
         if (!c.host) TSVM_HIP_CHECK(hipHostMalloc((void **) &c.host, CHUNK, hipHostMallocPortable));
-        wait(c);
+        wait(c, timeout_ms);
         return c;
     }
-    void wait(Chunk &c) {
+    void wait(Chunk &c, long long timeout_ms) {   // (0: as long as it takes)
         if (!c.pending.event) return;
-        TSVM_HIP_CHECK(hipEventSynchronize(c.pending.event));
+        if (timeout_ms > 0) wait_until_done([](void *e) { return hipEventQuery((hipEvent_t) e); }, c.pending.event, timeout_ms);
+        else TSVM_HIP_CHECK(hipEventSynchronize(c.pending.event));
         give_event(c.pending);
         c.pending = DeviceEvent();
     }
@@ -293,7 +307,8 @@ void HostStaging::upload(void *dst, const std::vector<Part> &parts, hipStream_t 
     }, stream);
 }
 
-void HostStaging::download(const void *src, size_t bytes, const std::function<void(const char *, size_t, size_t)> &take, hipStream_t stream) {
+void HostStaging::download(const void *src, size_t bytes, const std::function<void(const char *, size_t, size_t)> &take, hipStream_t stream,
+                           long long timeout_ms) {
     Impl &I = impl();
     std::lock_guard<std::mutex> lock(I.mu);
     struct Flying { Impl::Chunk *c; size_t off, len; };
@@ -302,14 +317,14 @@ void HostStaging::download(const void *src, size_t bytes, const std::function<vo
     while (head < queue.size() || off < bytes) {
         while (off < bytes && queue.size() - head < Impl::CHUNKS - 1) {
             const size_t len = std::min(CHUNK, bytes - off);
-            Impl::Chunk &c = I.take();
+            Impl::Chunk &c = I.take(timeout_ms);
             TSVM_HIP_CHECK(hipMemcpyAsync(c.host, (const char *) src + off, len, hipMemcpyDeviceToHost, stream));
             I.record(c, stream);
             queue.push_back({&c, off, len});
             off += len;
         }
         const Flying f = queue[head++];
-        I.wait(*f.c);
+        I.wait(*f.c, timeout_ms);
         take(f.c->host, f.off, f.len);
     }
 }

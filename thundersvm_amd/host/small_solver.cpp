@@ -80,14 +80,27 @@ static void run_together(const std::vector<SmallBatch *> &batches, float_type ep
     }
     std::vector<char> got(problems_at);
     const tsvm_small_state *const states = (const tsvm_small_state *) (got.data() + states_at);
-    for (bool first = true, more = true; more; first = false) {
+    // The kernel's own loops are bounded and every launch makes at least one outer iteration of a problem that is not done, so
+    // what is not bounded is what the outer loop of SolveTask is not either: the iterations a problem needs.  Each launch is
+    // waited for no longer than SolveTask waits for a solver, and has to have got further.
+    for (long long done_before = -1, more = true; more;) {
+        const bool first = done_before < 0;
         abi_check(tsvm_smo_solve_small(row_type, (const tsvm_small_problem *) (d.data() + problems_at), n_problems, max_slots,
                                        (tsvm_small_state *) (d.data() + states_at), d_ws.data(), (double *) d.data(), (double *) (d.data() + vec), nu,
                                        eps, out_max_iter, first, stream));
-        tsvm::HostStaging::instance().download(d.data(), problems_at, [&](const char *from, size_t off, size_t len) {
-            tsvm::parallel_memcpy(got.data() + off, from, len);
-        }, stream);
+        try {
+            tsvm::HostStaging::instance().download(d.data(), problems_at, [&](const char *from, size_t off, size_t len) {
+                tsvm::parallel_memcpy(got.data() + off, from, len);
+            }, stream, tsvm::solver_timeout_ms());
+        } catch (...) {   // (the device may still be using them)
+            d.abandon();
+            d_ws.abandon();
+            throw;
+        }
         more = std::any_of(states, states + n_problems, [](const tsvm_small_state &s) { return s.status == 0; });
+        const long long done = std::accumulate(states, states + n_problems, 0ll, [](long long sum, const tsvm_small_state &s) { return sum + s.iter; });
+        if (more && done <= done_before) throw std::runtime_error("SmallBatch: a launch made no progress");
+        done_before = done;
     }
     d.release(true);
     d_ws.release(true);
