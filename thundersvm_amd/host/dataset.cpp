@@ -259,8 +259,7 @@ void DataSet::load_from_dense(int row_size, int features, float *data, float *la
 void DataSet::load_from_csr(int64_t n, const int64_t *row_ptr, const int *col, const double *val, const double *y, bool keep) {
     // (the rows are copied in blocks and gathered by these pointers later: what they say has to hold)
     if (n < 0) throw std::length_error("DataSet: negative number of rows");
-    int decreasing = 0;
-#pragma omp parallel for schedule(static) reduction(| : decreasing) num_threads(threads_for((size_t) n))
+    bool decreasing = false;   // (8 bytes a row, a small part of what is read below: one thread)
     for (int64_t r = 0; r < n; ++r) decreasing |= row_ptr[r + 1] < row_ptr[r];
     if (decreasing) throw std::length_error("DataSet: a row ends before it begins (decreasing row pointer)");
     y_.assign(y, y + (y ? n : 0));
