@@ -258,6 +258,42 @@ def test_c_smo_solve_with_scores_that_a_float_cannot_tell_apart(ws, scores):
     assert np.array_equal(G.host(ad_d), ad_want, equal_nan=True)
 
 
+@pytest.mark.parametrize("ws", [257, 512, 513, 1024])
+@pytest.mark.parametrize("diagonal", ["2^126.5", "2^130", "2^-342", "0"])
+def test_c_smo_solve_with_diagonals_out_of_float_range(ws, diagonal):
+    """A few instances whose K_ii + K_tt - 2 K_it is no normal float, or has no normal float as its reciprocal, and whose f
+    makes them the best second index all the same: the same steps as the oracle's, bit for bit."""
+    rng = np.random.default_rng(ws + len(diagonal))
+    n, Cc, eps, max_iter = ws + 5, 2.0, 1e-30, 60
+    y = np.where(rng.random(n) < 0.5, 1, -1).astype(np.int32)
+    b = rng.random((n, n))
+    k = 0.2 * (b + b.T)
+    f = -y + 0.01 * rng.standard_normal(n)
+    np.fill_diagonal(k, 1.0)
+    ws_ids = rng.permutation(n)[:ws].astype(np.int32)
+    odd = ws_ids[rng.permutation(ws)[:4]]
+    k[odd], k[:, odd] = 0.0, 0.0
+    k[odd, odd] = 0.0 if diagonal == "0" else 2.0 ** float(diagonal[2:])
+    if diagonal in ("2^126.5", "2^130"):           # scores of 8 and less by halves, the others' are below 4
+        y[odd], f[odd] = -1, np.sqrt(np.array([8.0, 6.0, 5.0, 4.5]) * k[odd, odd])
+    else:                                          # up is -1e-60: the odd instances' b is 1e-50, the others' 1e-3, eps 1e-30
+        f = 1e-3 * (1.0 + rng.random(n))
+        y[odd], f[odd] = [1, -1, -1, -1], [-1e-60, 1e-50, 2e-50, 3e-50]
+    k_rows, diag = np.ascontiguousarray(k[ws_ids]), np.ascontiguousarray(np.diag(k))
+    alpha = np.zeros(n)
+    a_want, ad_want, diff_want = O.c_smo_solve(y, f, alpha, ws_ids, Cc, Cc, k_rows, diag, n, eps, max_iter)
+    assert np.count_nonzero(a_want[odd]) >= 2 and diff_want[1] > 1
+    y_d, f_d, ws_d, dg_d, a_d, k_d = G.dev(y), G.dev(f), G.dev(ws_ids), G.dev(diag), G.dev(alpha), G.dev(k_rows)
+    ad_d = torch.zeros(ws, dtype=torch.float64, device="cuda")
+    diff_d = torch.zeros(2, dtype=torch.float64, device="cuda")
+    wsp = torch.empty(capi.kernel_lib().tsvm_smo_solve_workspace(ws), dtype=torch.uint8, device="cuda")
+    capi.call("tsvm_c_smo_solve", G.ptr(y_d), G.ptr(f_d), G.ptr(a_d), G.ptr(ad_d), G.ptr(ws_d), ws, Cc, Cc, G.ptr(k_d), capi.ROW_F64, None,
+              n, G.ptr(dg_d), eps, G.ptr(diff_d), max_iter, G.ptr(wsp), G.stream())
+    assert np.array_equal(G.host(diff_d), diff_want)
+    assert np.array_equal(G.host(a_d), a_want, equal_nan=True)
+    assert np.array_equal(G.host(ad_d), ad_want, equal_nan=True)
+
+
 @pytest.mark.parametrize("nu", [False, True])
 @pytest.mark.parametrize("n,ws", [(300, 16), (2000, 1024), (900, 200)])
 def test_smo_solve_block_on_a_chosen_xcd(n, ws, nu):

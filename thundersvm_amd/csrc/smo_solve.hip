@@ -357,11 +357,16 @@ __device__ __forceinline__ double row_first_min(const double (&x)[E], int base, 
 // 4.2e-7 (b, a, the two products 2^-24 each, b twice; the reciprocal 2^-23), so a lead of 2^-19 = 1.9e-6 is proof, and the
 // winner is then the reference's j2.  Otherwise the function returns false before the step, which c_smo_iterate then takes.
 // (Scores are floored at 2^-80, which makes smaller ones ties; a score without a lead includes every tie, no candidate at
-// all, negative a, and NaN.  One case is not caught: a below 2^-126 with b below 2^-149.)  That replaces E divisions of some
-// fourteen instructions by six each, and the reduction over doubles by one over floats.
+// all, negative a, and NaN.  What falls to the floor although it is larger: an a of 2^126 and more, whose reciprocal is a
+// denormal, that is zero; and a b that is zero or a denormal in float, with an a so small that b^2/a is not, zero times
+// infinity.  Such a b is the difference of an f and an `up` below 2^-73: anything above is a multiple of 2^-126.  A thread that
+// meets either stands for an infinite second-best score, and nothing is decided; four instructions, 740 steps 727 -> 728 us.)
+// That replaces E divisions of some fourteen instructions by six each, and the reduction over doubles by one over floats.
 // Rows of sixteen lanes are reduced by DPP and publish themselves, and after the barrier every lane reads one of the
 // sixteen rows and four more steps compare them: the same eight steps as over a wavefront and then over four of them, without
 // the way through the scalar unit in between.
+#define SV_UP_LEAST_HI 0x3b600000   // 2^-73
+#define SV_A_BITS 0x7e800000         // 2^126
 template <int E, int LDK, typename TB>
 __device__ __forceinline__ bool c_smo_iterate_rounded(SvState<E * 256, 4> &sh, SvCand *s_i, SvScore *s_j, SvStep *s_step, int ws, const TB *kws,
                                                       const double (&kd)[E], double (&f)[E], unsigned &in_up, unsigned &in_low,
@@ -408,13 +413,17 @@ __device__ __forceinline__ bool c_smo_iterate_rounded(SvState<E * 256, 4> &sh, S
         const int violates = __builtin_amdgcn_ballot_w64(!(b_max < local_eps)) != 0;
         double up_i = bound_i.hi - z_i;
         asm("" : "+v"(up_i));
+        int a_max = (__double2hiint(up_value) & 0x7fffffff) < SV_UP_LEAST_HI ? 0x7f800000 : 0;   // (as the bits of a float)
+        asm("" : "+v"(a_max));
         SV_PIN;
         double aIJ[E];
         float q[E];
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             aIJ[e] = __builtin_fma(-2.0, (double) kI[e], a_part[e]);
-            q[e] = __builtin_fmaxf(b32[e] * (b32[e] * __builtin_amdgcn_rcpf((float) aIJ[e])), 0x1p-80f);
+            const float a32 = (float) aIJ[e];
+            a_max = __float_as_int(a32) > a_max ? __float_as_int(a32) : a_max;
+            q[e] = __builtin_fmaxf(b32[e] * (b32[e] * __builtin_amdgcn_rcpf(a32)), 0x1p-80f);
         }
         float best, second;
         if constexpr (E == 4) {
@@ -435,6 +444,7 @@ __device__ __forceinline__ bool c_smo_iterate_rounded(SvState<E * 256, 4> &sh, S
             b_at = is ? b_low[e] : b_at;
             a_at = is ? aIJ[e] : a_at;
         }
+        second = a_max < SV_A_BITS ? second : __builtin_inff();
         const float mine = best;
         row_best_two(best, second);
         const uint64_t who = __builtin_amdgcn_ballot_w64(mine == best);   // (several only if nothing will be decided)
