@@ -476,3 +476,13 @@ def test_device_buffer_accounting_and_round_trip():
     import selftest_lib
     lib = selftest_lib.lib()
     assert lib.tsvm_selftest_device_buffer() == 0, lib.tsvm_selftest_last_error()
+
+
+@pytest.mark.parametrize("kernel_type", [0, 2])
+@pytest.mark.parametrize("n", [49151, 49152])
+def test_f_from_a_non_zero_alpha_on_both_sides_of_the_update(n, kernel_type):
+    """One-class: f starts from nu * n kernel rows in batches of 101; below 49,152 columns the batches are one launch."""
+    rng = np.random.default_rng(n)
+    d = D.from_dense(rng.standard_normal((n, 3)).astype(np.float32), np.ones(n))
+    _compare(d, D.from_dense(rng.standard_normal((50, 3)).astype(np.float32)),
+             make_param(svm_type=2, kernel_type=kernel_type, gamma=0.3, nu=250.5 / n, max_iter=1), trace=0)

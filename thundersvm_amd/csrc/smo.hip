@@ -438,7 +438,8 @@ __global__ __launch_bounds__(UF_T) void update_f_kernel(double *__restrict__ f, 
 // latency: few columns (a few thousand instances), many rows, and the sums of a column one after another.  One column per
 // thread in workgroups of one wavefront (5,001 columns are 79 of them), the rows one stream across the batches, the next UB
 // of them on their way while UB are added: 1,010 rows of 5,001 floats 70 us, ten launches of update_f_kernel 88 and the gaps
-// between them.  nu-SVC on 5,001 x 23 starts from 2,000 such rows: 5.01 -> 4.57 ms.
+// between them.  nu-SVC on 5,001 x 23 starts from 2,000 such rows: 5.01 -> 4.57 ms.  (With many columns update_f_kernel is
+// the better one: whoever has both calls chooses.)
 #define UB 32
 template <typename TK>
 __global__ __launch_bounds__(64) void update_f_batches_kernel(double *__restrict__ f, const double *__restrict__ coef, int n_rows, int batch,

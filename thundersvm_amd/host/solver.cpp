@@ -878,10 +878,15 @@ void CSMOSolver::solve(const KernelMatrix &k_mat, const std::vector<int> &y, std
 
 // csmosolver.cpp:189-214: f starts from a non-zero alpha in batches of 101 rows.  Ids and coefficients travel once.  Several
 // batches' rows are computed by one call where they are dense and small (101 rows of a few thousand columns leave most of
-// the chip idle): up to ten batches in INIT_ROWS_BYTES.
+// the chip idle): up to ten batches in INIT_ROWS_BYTES.  One launch then takes them all from f, while the columns are few; from
+// BATCHES_BELOW columns on, where two batches and then one fit and update_f's wide loads fill the chip by themselves, each
+// batch is a launch of update_f.  Both ways, update_f / in one launch, us, on float rows: 5,000 columns 76 / 59 (ten batches),
+// 30,000 44 / 42 (five), 40,000 36 / 36, 60,000 19 / 21, 160,000 14.4 / 17.4 (one), 600,000 43 / 42; on double rows 20,000
+// 46 / 37, 40,000 25 / 23, 60,000 14.2 / 14.3, 160,000 25.5 / 26.8, 600,000 82 / 92.
 void CSMOSolver::init_f(const std::vector<float_type> &alpha, const std::vector<int> &y, const KernelMatrix &k_mat,
                         float_type *d_f) const {
     constexpr size_t BATCH = 101, INIT_ROWS_BYTES = (size_t) 64 << 20;
+    constexpr int BATCHES_BELOW = 49152;
     const int n_u = (int) k_mat.n_columns();
     const int64_t ld = ((int64_t) n_u + 7) / 8 * 8;
     std::vector<int> idx;
@@ -903,8 +908,14 @@ void CSMOSolver::init_f(const std::vector<float_type> &alpha, const std::vector<
     for (size_t at = 0; at < idx.size(); at += at_once) {
         const int m = (int) std::min(at_once, idx.size() - at);
         k_mat.get_rows(d_idx.data() + at, m, d_rows.data(), ld, nullptr, tsvm::work_stream());
-        abi_check(tsvm_update_f_batches(d_f, d_coef.data() + at, m, (int) BATCH, d_rows.data(), k_mat.row_type(), ld, n_u, k_mat.repeat(),
-                                        tsvm::work_stream()));
+        if (n_u < BATCHES_BELOW) {
+            abi_check(tsvm_update_f_batches(d_f, d_coef.data() + at, m, (int) BATCH, d_rows.data(), k_mat.row_type(), ld, n_u, k_mat.repeat(),
+                                            tsvm::work_stream()));
+            continue;
+        }
+        for (int t = 0; t < m; t += (int) BATCH)
+            abi_check(tsvm_update_f(d_f, d_coef.data() + at + t, std::min((int) BATCH, m - t), d_rows.data() + t * row_bytes, k_mat.row_type(), nullptr,
+                                    ld, n_u, k_mat.repeat(), tsvm::work_stream()));
     }
 }
 
