@@ -9,6 +9,7 @@
 
 #include "../../thundersvm_amd/host/dataset.h"
 #include "../../thundersvm_amd/host/device.h"
+#include "../../thundersvm_amd/host/kernelmatrix.h"
 #include "../../thundersvm_amd/host/row_cache.h"
 #include "../../thundersvm_amd/host/solver.h"
 
@@ -16,9 +17,9 @@ namespace {
 
 thread_local std::string g_selftest_error;
 
-#define SELFTEST_GUARD(body)                       \
+#define SELFTEST_GUARD(...)                        \
     try {                                          \
-        body;                                      \
+        __VA_ARGS__;                               \
         return 0;                                  \
     } catch (const std::exception &e) {            \
         g_selftest_error = e.what();               \
@@ -179,6 +180,29 @@ int tsvm_selftest_wait_until_done(int timeout_ms) {
     } catch (const std::runtime_error &) {
         return 0;
     }
+}
+
+// Needs a device.  What is known about the values of sparse rows and decides how a prediction reads them is known about a
+// subset of them as well.  last: the last row's last value (infinite, or no float, or an ordinary one).
+int tsvm_selftest_subset_of_rows(double last) {
+    SELFTEST_GUARD({
+        const int n = 300, per_row = 5;
+        std::vector<int64_t> ptr(n + 1);
+        std::vector<int> col(n * per_row);
+        std::vector<double> val(n * per_row, 0.5);
+        for (int r = 0; r <= n; ++r) ptr[r] = r * per_row;
+        for (int e = 0; e < n * per_row; ++e) col[e] = 1 + e % per_row * 400 + e / per_row;
+        val.back() = last;
+        const RowStore rows(n, ptr.data(), col.data(), val.data());
+        const std::shared_ptr<DeviceRows> all = DeviceRows::from_host(rows);
+        std::vector<int> ids(100);
+        for (int i = 0; i < 100; ++i) ids[i] = 299 - 2 * i;
+        const std::shared_ptr<DeviceRows> some = DeviceRows::subset(*all, ids.data(), ids.size());
+        auto expect = [](bool ok, const char *what) { if (!ok) throw std::runtime_error(std::string("DeviceRows::subset: ") + what); };
+        expect(!all->dense && !some->dense && all->sliced_lds > 0 && some->sliced_lds > 0, "layout");
+        expect(all->values_finite == (last - last == 0) && some->values_finite == all->values_finite, "finite values");
+        expect(all->values_fit_float == ((double) (float) last == last) && some->values_fit_float == all->values_fit_float, "float values");
+    })
 }
 
 // No device needed.  DataSet::load_from_sparse (dense == 0) or load_from_dense (row_ptr and col_ptr unused) and the rows it

@@ -194,3 +194,12 @@ def test_sparse_class_pair_whose_rows_are_all_empty():
     _, gdec = gm.predict(te)
     _, odec = om.predict(te.ptr, te.col, te.val, 100)
     assert np.abs(gdec - odec).max() < 1e-6
+
+
+@pytest.mark.parametrize("last", [0.5, 0.1, float("inf")])
+def test_what_is_known_of_sparse_values_goes_to_subsets(last):
+    """The models of a sparse cross-validation take their support vectors out of the data set's device rows: finite values
+    let them predict on the sliced copy, as a model of its own does."""
+    import selftest_lib
+    lib = selftest_lib.lib()
+    assert lib.tsvm_selftest_subset_of_rows(last) == 0, lib.tsvm_selftest_last_error()

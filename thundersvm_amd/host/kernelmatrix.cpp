@@ -505,6 +505,7 @@ std::shared_ptr<DeviceRows> DeviceRows::subset(const DeviceRows &base, const int
     r.n_features = base.n_features;
     r.dense = base.dense;
     r.values_fit_float = base.values_fit_float;
+    r.values_finite = base.values_finite;
     r.ld = base.ld;
     tsvm::DeviceBuffer<int> d_rows(n_rows);
     d_rows.upload(rows, n_rows);
