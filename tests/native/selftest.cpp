@@ -205,6 +205,29 @@ int tsvm_selftest_subset_of_rows(double last) {
     })
 }
 
+// Needs a device.  The first of a run of indicator columns that ends with the last one: four ordinary columns and thirty
+// that one entry a row is set in, 20,000 rows; `last` is the very last entry, in the last column (1: the run is there).
+// Returns the first column of the run that get_rows leaves to its epilogue, -1 without one.
+int tsvm_selftest_indicator_run(double last) {
+    const int n = 20000, per_row = 5;
+    std::vector<int64_t> ptr(n + 1);
+    std::vector<int> col(n * per_row);
+    std::vector<double> val(n * per_row, 0.25);
+    for (int r = 0; r <= n; ++r) ptr[r] = r * per_row;
+    for (int r = 0; r < n; ++r) {
+        for (int c = 0; c < 4; ++c) col[r * per_row + c] = 1 + c;
+        col[r * per_row + 4] = r == n - 1 ? 34 : 5 + r % 30;
+        val[r * per_row + 4] = 1.0;
+    }
+    val.back() = last;
+    try {
+        return DeviceRows::from_host(RowStore(n, ptr.data(), col.data(), val.data()))->ind_first;
+    } catch (const std::exception &e) {
+        g_selftest_error = e.what();
+        return -100;
+    }
+}
+
 // No device needed.  DataSet::load_from_sparse (dense == 0) or load_from_dense (row_ptr and col_ptr unused) and the rows it
 // holds afterwards: out_ptr [row_size + 1], out_col / out_val with room for `cap` entries.  Returns the entries, -1 when refused.
 long long tsvm_selftest_load_matrix(int dense, int row_size, int features, float *val, int *row_ptr, int *col_ptr, long long *out_ptr,

@@ -21,6 +21,7 @@ def lib():
         L.tsvm_selftest_row_cache.argtypes = [ctypes.c_int] * 4
         L.tsvm_selftest_solver_wait.argtypes = [ctypes.c_int, ctypes.c_int]
         L.tsvm_selftest_subset_of_rows.argtypes = [ctypes.c_double]
+        L.tsvm_selftest_indicator_run.argtypes = [ctypes.c_double]
         L.tsvm_selftest_load_matrix.restype = ctypes.c_longlong
         L.tsvm_selftest_load_matrix.argtypes = [ctypes.c_int] * 3 + [ctypes.c_void_p] * 6 + [ctypes.c_longlong]
         _LIB = L

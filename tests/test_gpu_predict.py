@@ -203,3 +203,10 @@ def test_what_is_known_of_sparse_values_goes_to_subsets(last):
     import selftest_lib
     lib = selftest_lib.lib()
     assert lib.tsvm_selftest_subset_of_rows(last) == 0, lib.tsvm_selftest_last_error()
+
+
+@pytest.mark.parametrize("last,first", [(1.0, 5), (0.0, 5), (2.0, -1)])
+def test_indicator_columns_are_found_by_all_entries(last, first):
+    """The host looks at the first entries only; what the last of 100,000 holds still decides."""
+    import selftest_lib
+    assert selftest_lib.lib().tsvm_selftest_indicator_run(last) == first

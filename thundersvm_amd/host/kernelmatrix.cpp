@@ -459,9 +459,9 @@ std::shared_ptr<DeviceRows> DeviceRows::from_host(const RowStore &rows) {
         r.col.release();
         r.row_ptr.release();
         // indicator columns are a run that ends with the last column: one other value there, in most data sets the
-        // first, and there are none
+        // first, and there are none (a few of the entries are looked at here, all of them by the device's count)
         bool last_is_indicator = true;
-        for (size_t e = 0; e < r.nnz && last_is_indicator; ++e)
+        for (size_t e = 0; e < std::min<size_t>(r.nnz, 16384) && last_is_indicator; ++e)
             if (col[e] == max_index && val[e] != 0.0 && val[e] != 1.0) last_is_indicator = false;
         if (last_is_indicator) r.find_indicator_columns();
     } else {
