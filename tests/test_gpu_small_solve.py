@@ -84,3 +84,29 @@ def test_infinite_C(svm_type, n):
     assert np.isfinite(gm.coef).all() and gm.total_sv > 0
     alone = Model(svm_type).train(d, make_param(pair_lanes=1, cache_bytes=0, **prm))   # (asks for the other path)
     assert np.array_equal(gm.coef, alone.coef) and np.array_equal(gm.rho, alone.rho)
+
+
+@pytest.mark.parametrize("weight", [0.0, -1.0])
+@pytest.mark.parametrize("sizes,small", [((40, 300, 60), True), ((700, 600, 500), False), ((1500, 1100, 40), False)])
+def test_class_without_room(sizes, small, weight):
+    """A class weight of zero leaves a pair's working set without enough candidates: the small kernel gives such a pair back
+    (beside pairs that it has solved), and the solve ends where it starts.  The third pair is not touched by it."""
+    x, rng = _rows(sum(sizes), 3 * sum(sizes), False)
+    y = np.repeat(np.arange(3), sizes).astype(np.float64)
+    x[:, 0] += y
+    d = D.from_dense(x, y)
+    prm = dict(gamma=0.2, C=3.0)
+    m = Model(0).train(d, make_param(weights={0: weight}, **prm), keep_binary=True)
+    for k in (0, 1):
+        alpha, f = m.binary(k)
+        assert m.stats(k)["n_iter"] == 1 and m.stats(k)["local_iter"] == 0
+        assert not alpha.any() and np.array_equal(f, np.where(np.arange(len(f)) < sizes[0], -1.0, 1.0))
+    rest = Model(0).train(D.from_dense(x[sizes[0]:], y[sizes[0]:]), make_param(**prm), keep_binary=True)
+    assert np.array_equal(m.binary(2)[0], rest.binary(0)[0]) and np.array_equal(m.binary(2)[1], rest.binary(0)[1])
+    assert m.stats(2)["n_iter"] == rest.stats(0)["n_iter"] > 1 and m.rho[2] == rest.rho[0]
+    if small:   # two classes alone: no other pair beside
+        two = Model(0).train(D.from_dense(x[:sizes[0] + 20], y[:sizes[0] + 20]), make_param(weights={1: weight}, **prm), keep_binary=True)
+        assert two.total_sv == 0 and not two.binary(0)[0].any()
+    else:
+        two = Model(0).train(D.from_dense(x[:sizes[0] + sizes[1]], y[:sizes[0] + sizes[1]]), make_param(weights={1: weight}, **prm))
+        assert two.total_sv == 0

@@ -329,6 +329,11 @@ struct SolveTask::Impl {
     bool select_ahead = false, block_first = false, select_enqueued = false;
     bool fuse_select = false;   // update_f also makes the first pass of the selection that follows
     int iter = 0;
+    // A box without room (a class weight of zero; C or the weight negative): with positive ones every instance is in I_up or in
+    // I_low, here one of the two is empty and the other may be too, so that a working set cannot be filled (the selection
+    // then hands out ids of -1, and the reference never returns) while the gap is -infinity from the start.  Nothing is enqueued;
+    // the solve ends in its first iteration with alpha and f as they are.
+    bool inert = false;
 
     Impl(const CSMOSolver &solver, const KernelMatrix &k_mat, const std::vector<int> &y, std::vector<float_type> &alpha,
          float_type &rho, std::vector<float_type> &f_val, float_type eps, float_type Cp, float_type Cn, int ws_size,
@@ -340,6 +345,7 @@ struct SolveTask::Impl {
         if (ws_size < 1 || ws_size > n || ws_size > 1024)
             throw std::invalid_argument("SolveTask: working-set size " + std::to_string(ws_size) + " for " + std::to_string(n) +
                                         " instances (1 .. min(instances, 1024))");
+        inert = !(Cp > 0 && Cn > 0);
         wall0 = std::chrono::steady_clock::now();
         (void) process_epoch();
         stats.ws_size = ws_size;
@@ -769,11 +775,12 @@ struct SolveTask::Impl {
     }
 
     bool finish_iteration() {
-        if (wait_by_event) TSVM_HIP_CHECK(hipEventSynchronize(diff_ready.event));
+        if (inert) h_diff[0] = -INFINITY;
+        else if (wait_by_event) TSVM_HIP_CHECK(hipEventSynchronize(diff_ready.event));
         else wait_for_diff();
         const double diff0 = h_diff[0], diff1 = h_diff[1];
         local_iter += (long long) diff1;
-        if (device_cache && !all_cached) {
+        if (device_cache && !all_cached && !inert) {
             // (the two numbers may still be the previous iteration's: the slots are assigned after the solver was
             // enqueued; they only steer the schedule, and the hit count is made exact at the end)
             stats.cache_lookups += iter == 0 ? ws_size : q;
@@ -781,7 +788,7 @@ struct SolveTask::Impl {
             all_cached = h_cache_info[1] == n_u;
         }
         SolverTrace *trace = solver.trace;
-        if (trace && iter < trace->cap_iters) {
+        if (trace && iter < trace->cap_iters && !inert) {
             trace->diff.push_back(diff0);
             trace->diff.push_back(diff1);
             std::vector<int> w = d_ws.to_host();
@@ -837,11 +844,11 @@ SolveTask::SolveTask(const CSMOSolver &solver, const KernelMatrix &k_mat, const 
                      int out_max_iter, void *pool, size_t pool_bytes, int lane, int n_lanes)
     : impl_(new Impl(solver, k_mat, y, alpha, rho, f_val, eps, Cp, Cn, ws_size, out_max_iter, pool, pool_bytes, lane, n_lanes)) {}
 SolveTask::~SolveTask() { delete impl_; }
-void SolveTask::enqueue_select() { impl_->enqueue_select(); }
-void SolveTask::enqueue_rows() { impl_->enqueue_rows(); }
-void SolveTask::enqueue_block() { impl_->enqueue_block(); }
-void SolveTask::enqueue_solver() { impl_->enqueue_solver(); }
-void SolveTask::enqueue_update() { impl_->enqueue_update(); }
+void SolveTask::enqueue_select() { if (!impl_->inert) impl_->enqueue_select(); }
+void SolveTask::enqueue_rows() { if (!impl_->inert) impl_->enqueue_rows(); }
+void SolveTask::enqueue_block() { if (!impl_->inert) impl_->enqueue_block(); }
+void SolveTask::enqueue_solver() { if (!impl_->inert) impl_->enqueue_solver(); }
+void SolveTask::enqueue_update() { if (!impl_->inert) impl_->enqueue_update(); }
 bool SolveTask::finish_iteration() { return impl_->finish_iteration(); }
 bool SolveTask::rows_ready() const { return impl_->ids_arrived(); }
 bool SolveTask::iteration_done() { return impl_->diff_arrived(); }
