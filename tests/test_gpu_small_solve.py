@@ -110,3 +110,17 @@ def test_class_without_room(sizes, small, weight):
     else:
         two = Model(0).train(D.from_dense(x[:sizes[0] + sizes[1]], y[:sizes[0] + sizes[1]]), make_param(weights={1: weight}, **prm))
         assert two.total_sv == 0
+
+
+@pytest.mark.parametrize("svm_type,n,ws,C,gamma,max_iter,iters,steps", [
+    (0, 300, 4, 3.0, 0.2, 600, 513, 0), (1, 300, 8, 1.0, 0.2, 600, 513, 0), (3, 150, 4, 3.0, 0.2, 600, 257, 0), (0, 900, 8, 3.0, 0.2, 300, 257, 0),
+    (0, 200, 0, 1e6, 0.01, 7, 1, 600000), (3, 300, 0, 1e6, 0.02, 4, 1, 300000)])
+def test_solves_of_several_launches(svm_type, n, ws, C, gamma, max_iter, iters, steps):
+    """A launch ends after 256 outer iterations or 300,000 steps; the next one goes on from what it left: small working sets
+    on overlapping classes, and boxes that are never reached."""
+    x, rng = _rows(n, 900 + n, False)
+    y = (rng.random(n) < 0.5).astype(np.float64)
+    d = D.from_dense(x, y if svm_type < 2 else rng.standard_normal(n))
+    gm, om, _, _ = T._compare(d, d, make_param(svm_type=svm_type, gamma=gamma, C=C, nu=0.3, p=0.05, max_iter=max_iter), ws=ws, trace=0)
+    assert gm.stats(0)["n_iter"] >= iters and gm.stats(0)["local_iter"] >= steps
+    assert np.array_equal(gm.binary(0)[0], om.binary(0)[0]) and np.array_equal(gm.binary(0)[1], om.binary(0)[1])
