@@ -486,3 +486,23 @@ def test_f_from_a_non_zero_alpha_on_both_sides_of_the_update(n, kernel_type):
     d = D.from_dense(rng.standard_normal((n, 3)).astype(np.float32), np.ones(n))
     _compare(d, D.from_dense(rng.standard_normal((50, 3)).astype(np.float32)),
              make_param(svm_type=2, kernel_type=kernel_type, gamma=0.3, nu=250.5 / n, max_iter=1), trace=0)
+
+
+@pytest.mark.parametrize("svm_type", [0, 2, 3])
+def test_linear_coefficients_of_a_fold_with_feature_id_zero(svm_type, tmp_path):
+    """The folds of a cross-validation are as zero-based as the data set: the model of the last one has the linear
+    coefficients that the same rows with every id one larger give."""
+    rng = np.random.default_rng(svm_type)
+    x = rng.standard_normal((90, 4)).astype(np.float32)
+    y = (x[:, 0] > 0).astype(np.float64) if svm_type != 3 else np.round(x[:, 0]).astype(np.float64)   # (folds are cut label by label)
+    one = D.from_dense(x, y)
+    assert one.col.min() == 1 and one.col.max() == 4
+    zero = D.CsrData(one.ptr, one.col - 1, one.val, one.y)
+    lines = []
+    for rows in (one, zero):
+        m = Model(svm_type)
+        m.cross_validation(Dataset(rows), make_param(svm_type=svm_type, kernel_type=0, nu=0.3, C=1.0, p=0.1), 3)
+        m.save(str(tmp_path / "m"))
+        text = open(str(tmp_path / "m")).read().split("\n")
+        lines.append(text[text.index("coef ") + 1].split())
+    assert len(lines[0]) == 4 and lines[0] == lines[1]

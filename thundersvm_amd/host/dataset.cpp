@@ -16,11 +16,18 @@
 #include <memory>
 #include <stdexcept>
 
-DataSet::DataSet(const node2d &instances, int n_features, const std::vector<float_type> &y)
-    : y_(y), rows_(RowStore::from_nodes(instances)), n_features_(n_features) {}
+static bool any_id_zero(const DataSet::node2d &instances) {
+    for (const auto &row : instances)
+        for (const DataSet::node &nd : row)
+            if (nd.index == 0) return true;
+    return false;
+}
 
-DataSet::DataSet(std::shared_ptr<const RowStore> rows, int n_features, const std::vector<float_type> &y)
-    : y_(y), rows_(std::move(rows)), n_features_(n_features) {}
+DataSet::DataSet(const node2d &instances, int n_features, const std::vector<float_type> &y)
+    : y_(y), rows_(RowStore::from_nodes(instances)), n_features_(n_features), zero_based_(any_id_zero(instances)) {}
+
+DataSet::DataSet(std::shared_ptr<const RowStore> rows, int n_features, bool zero_based, const std::vector<float_type> &y)
+    : y_(y), rows_(std::move(rows)), n_features_(n_features), zero_based_(zero_based) {}
 
 void DataSet::set_rows(std::shared_ptr<const RowStore> rows) {
     device_slot_ = std::make_shared<std::shared_ptr<void>>();   // new instances: any device copy is stale
@@ -211,6 +218,7 @@ void DataSet::load_from_python(float *y, char **x, int len) {
             if ((size_t) ind > n_features_) n_features_ = ind;
         }
     }
+    zero_based_ = any_id_zero(nodes);
     set_rows(RowStore::from_nodes(nodes));
 }
 

@@ -14,7 +14,7 @@ public:
 
     DataSet() = default;
     DataSet(const node2d &instances, int n_features, const std::vector<float_type> &y);
-    DataSet(std::shared_ptr<const RowStore> rows, int n_features, const std::vector<float_type> &y);
+    DataSet(std::shared_ptr<const RowStore> rows, int n_features, bool zero_based, const std::vector<float_type> &y);
 
     // n_threads: threads that read and parse (0: as many as OpenMP would start, which the `-o` option sets, as in
     // the reference)

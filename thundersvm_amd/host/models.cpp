@@ -159,7 +159,7 @@ void SvmModel::train_folds(const DataSet &dataset, const std::vector<Fold> &fold
     const std::shared_ptr<DeviceRows> all = dataset.device_cache() ? std::static_pointer_cast<DeviceRows>(dataset.device_cache())
                                                                    : DeviceRows::from_host(dataset.rows());
     const auto rows_of = [&](const std::vector<int> &ids, const std::vector<float_type> &y) {
-        std::unique_ptr<DataSet> d(new DataSet(dataset.rows().gather(ids.data(), ids.size()), (int) dataset.n_features(), y));
+        std::unique_ptr<DataSet> d(new DataSet(dataset.rows().gather(ids.data(), ids.size()), (int) dataset.n_features(), dataset.is_zero_based(), y));
         if (!ids.empty()) d->device_cache() = DeviceRows::subset(*all, ids.data(), ids.size());
         return d;
     };
