@@ -8,6 +8,7 @@ import pytest
 from thundersvm_amd import data as D
 from thundersvm_amd.model import Dataset, Model, make_param
 
+import oracle_lib as O
 import test_gpu_models as T
 
 pytestmark = pytest.mark.gpu
@@ -124,3 +125,21 @@ def test_solves_of_several_launches(svm_type, n, ws, C, gamma, max_iter, iters, 
     gm, om, _, _ = T._compare(d, d, make_param(svm_type=svm_type, gamma=gamma, C=C, nu=0.3, p=0.05, max_iter=max_iter), ws=ws, trace=0)
     assert gm.stats(0)["n_iter"] >= iters and gm.stats(0)["local_iter"] >= steps
     assert np.array_equal(gm.binary(0)[0], om.binary(0)[0]) and np.array_equal(gm.binary(0)[1], om.binary(0)[1])
+
+
+@pytest.mark.parametrize("n,seed,max_iter", [(60, 2, 6), (200, 1, 3), (200, 4, 6), (300, 4, 3), (128, 0, 3), (128, 3, 6)])
+def test_alphas_that_run_away(n, seed, max_iter):
+    """A sigmoid kernel that is not positive definite: steps with a negative a leave the box, alpha grows past 1e154 and the
+    scores b^2/a overflow.  Still the oracle's steps, on this path and on the one of the larger problems."""
+    rng = np.random.default_rng(seed)
+    x = np.stack([rng.standard_normal(n), np.ones(n)], 1).astype(np.float32)
+    d = D.from_dense(x, np.round(x[:, 0]))
+    prm = dict(svm_type=2, kernel_type=3, gamma=0.5, coef0=0.0, nu=0.2, max_iter=max_iter)
+    om = O.Model(d.ptr, d.col, d.val, d.y, T._oparam(make_param(**prm)))
+    want_a, want_f = om.binary(0)
+    assert 1e154 < np.abs(want_a).max() < np.inf
+    for other in ({}, dict(pair_lanes=1, cache_bytes=0)):
+        gm = Model(2).train(d, make_param(**prm, **other), keep_binary=True)
+        a, f = gm.binary(0)
+        assert gm.stats(0)["n_iter"] == om.n_iter[0] and gm.stats(0)["local_iter"] == om.local_iter[0]
+        assert np.array_equal(a, want_a) and np.array_equal(f, want_f)

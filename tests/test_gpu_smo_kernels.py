@@ -295,6 +295,53 @@ def test_c_smo_solve_with_diagonals_out_of_float_range(ws, diagonal):
 
 
 @pytest.mark.parametrize("nu", [False, True])
+@pytest.mark.parametrize("ws", [2, 64, 100, 256, 257, 512, 1024])
+@pytest.mark.parametrize("what", ["scores from 2^1023 on", "infinite scores", "some infinite scores", "NaN rows", "NaN f", "infinite f"])
+def test_local_solvers_beyond_the_finite(ws, nu, what):
+    """Scores that overflow (a kernel that is not positive definite, alphas that have run away) and values that are no
+    numbers: a violating element without a finite score is no candidate, and the second index stays 0 without any, as for
+    the oracle.  Bit for bit, wherever the alphas went."""
+    if what == "infinite f" and ws == 2:
+        pytest.skip("the only element of a side with an infinite f: the gap is inf - inf, which is nobody's threshold")
+    rng = np.random.default_rng(ws + len(what))
+    n, Cc, eps, max_iter = ws + 5, 2.0, 1e-3, 40
+    y = np.where(rng.random(n) < 0.5, 1, -1).astype(np.int32)
+    y[:2] = [1, -1]
+    b = rng.random((n, n))
+    k = 0.2 * (b + b.T)
+    f = -y + 0.01 * rng.standard_normal(n)
+    alpha = np.where(rng.random(n) < 0.3, rng.random(n), 0.0)
+    if "scores" in what:
+        if what.startswith("some"):
+            k[: n // 2], k[:, : n // 2] = 4.0 * k[: n // 2], 4.0 * k[:, : n // 2]   # (positive a, too)
+        else:
+            k = k + 1.1                                                             # (negative a everywhere)
+        f = f * 2.0 ** (510.8 if "2^1023" in what else 520)
+    np.fill_diagonal(k, 1.0)
+    odd = rng.permutation(n)[: max(1, n // 50)]
+    if what == "NaN rows":
+        k[odd], k[:, odd] = np.nan, np.nan
+    elif what == "NaN f":
+        f[odd] = np.nan
+    elif what == "infinite f":
+        f[odd], alpha[odd] = np.where(y[odd] > 0, -np.inf, np.inf), 0.0   # (on one side each: a gap of inf - inf is no number)
+    ws_ids = rng.permutation(n)[:ws].astype(np.int32)
+    k_rows, diag = np.ascontiguousarray(k[ws_ids]), np.ascontiguousarray(np.diag(k))
+    solve, args = (O.nu_smo_solve, (Cc,)) if nu else (O.c_smo_solve, (Cc, Cc))
+    a_want, ad_want, diff_want = solve(y, f, alpha, ws_ids, *args, k_rows, diag, n, eps, max_iter)
+    y_d, f_d, ws_d, dg_d, a_d, k_d = G.dev(y), G.dev(f), G.dev(ws_ids), G.dev(diag), G.dev(alpha), G.dev(k_rows)
+    ad_d = torch.zeros(ws, dtype=torch.float64, device="cuda")
+    diff_d = torch.zeros(2, dtype=torch.float64, device="cuda")
+    wsp = torch.empty(capi.kernel_lib().tsvm_smo_solve_workspace(ws), dtype=torch.uint8, device="cuda")
+    capi.call("tsvm_nu_smo_solve" if nu else "tsvm_c_smo_solve", G.ptr(y_d), G.ptr(f_d), G.ptr(a_d), G.ptr(ad_d), G.ptr(ws_d), ws, *args,
+              G.ptr(k_d), capi.ROW_F64, None, n, G.ptr(dg_d), eps, G.ptr(diff_d), max_iter, G.ptr(wsp), G.stream())
+    got = G.host(diff_d)
+    assert np.array_equal(got if not nu else got[:1], diff_want if not nu else diff_want[:1], equal_nan=True)
+    assert np.array_equal(G.host(a_d), a_want, equal_nan=True)
+    assert np.array_equal(G.host(ad_d), ad_want, equal_nan=True)
+
+
+@pytest.mark.parametrize("nu", [False, True])
 @pytest.mark.parametrize("n,ws", [(300, 16), (2000, 1024), (900, 200)])
 def test_smo_solve_block_on_a_chosen_xcd(n, ws, nu):
     """The block solvers launched as eight workgroups of which one is elected (tsvm_*_smo_solve_block_on_xcd): the same

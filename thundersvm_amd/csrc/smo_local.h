@@ -4,10 +4,12 @@
 #pragma once
 #include "tsvm_device.h"
 
-// What a masked-out element or score is replaced by: larger than any f or score of a problem in range.  Only the
-// high word is replaced (one instruction), so every value from SV_NONE on means "not a candidate".
-#define SV_NONE_HI 0x7fe00000
-#define SV_NONE 0x1p1023
+// What a masked-out element or score is replaced by.  Only the high word is replaced (one instruction), so every value from
+// SV_NONE on means "not a candidate": the last 2^32 finite doubles and infinity, which is no candidate for the reference either.
+// (The high word of infinity itself would make NaNs of the low words.  A lower one is not enough: a solve on a kernel that is
+// not positive definite may run away, and its scores b^2/a pass 2^1023 before they overflow.)
+#define SV_NONE_HI 0x7fefffff
+#define SV_NONE 0x1.fffffp+1023
 
 // x when the sign bit of `bit_at_top` is set, otherwise a value >= SV_NONE (SIGN = 0) or <= -SV_NONE (SIGN = 1).
 template <int SIGN>

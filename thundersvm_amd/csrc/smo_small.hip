@@ -314,17 +314,20 @@ __device__ __forceinline__ void ss_load(const TB *row, TB (&out)[E]) {
 }
 
 // The local solver: c_smo_iterate of smo_solve.hip (and nu_smo_solve_kernel) with the instances in place of a gathered
-// working set.  Returns the steps taken; the new alpha is in sh.z.  NONE: the threshold is not positive (see there).
+// working set.  Returns the steps taken; the new alpha is in sh.z.  NONE and no_score: as there.
 template <int E, int W, bool NU, bool NONE, typename TB>
 __device__ __forceinline__ int ss_local(SmallShared<E, W> &sh, const SmallMap &map, const TB *K, int64_t ld, int col, const double (&kd)[E], double (&f)[E],
-                        unsigned member, double Cp, double Cn, double local_eps, int max_iter) {
+                        unsigned member, double Cp, double Cn, double local_eps, int max_iter, bool &no_score) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     constexpr int NP = NU ? 2 : 1;   // pairs of sides
     SvCand *const ci[2] = {sh.ci, sh.ci2}, *const cj[2] = {sh.cj, sh.cj2};
     const int first_slot = sh.ws[0];
     int n_iter = 0;
     bool go_on;
+    double taken = -__builtin_inf();   // the score of the step
+    int worst = 0;
     do {
+        if (!NONE) worst = imax_sel(worst, __double2hiint(taken));
         double up[NP], m[NP], v;
         int at[NP], is[NP], go;
 #pragma unroll
@@ -394,7 +397,8 @@ __device__ __forceinline__ int ss_local(SmallShared<E, W> &sh, const SmallMap &m
         const double up_value = second ? up[NP - 1] : up[0], kd_i2 = second ? kd_i[NP - 1] : kd_i[0];
         // (two sides' winners may write different rows into one lane's slots when one of them has no candidate, so with
         // two sides K[i, j2] is read from the matrix)
-        if (NONE && is_none(second ? best[NP - 1] : best[0])) {
+        taken = second ? best[NP - 1] : best[0];
+        if (NONE && is_none(taken)) {
             j2 = first_slot;
             __syncthreads();
             if (tid == first_slot / E) {
@@ -429,6 +433,7 @@ __device__ __forceinline__ int ss_local(SmallShared<E, W> &sh, const SmallMap &m
         for (int e = 0; e < E; ++e) f[e] = __builtin_fma(-l, (double) kJ[e] - (double) (second ? kI[NP - 1][e] : kI[0][e]), f[e]);
         n_iter += go_on;
     } while (go_on);
+    if (!NONE) no_score = __builtin_amdgcn_readfirstlane(worst) >= SV_NONE_HI;
     return n_iter;
 }
 
@@ -650,13 +655,26 @@ __global__ __launch_bounds__(64 * W) void smo_small_kernel(const tsvm_small_prob
             for (int w = 1; w < W; ++w) lo = fmin_f64(lo, sh.red[2 * r][w]);
             gap[r] = block_max<W>(sh.red[2 * r + 1]) - lo;
         }
-        diff = NU ? (gap[0] > gap[1] ? gap[0] : gap[1]) : gap[0];
+        diff = NU ? (gap[0] < gap[1] ? gap[1] : gap[0]) : gap[0];
         const double tenth = NU ? 0.1 * diff : 0.1f * diff;   // (a float literal in the C variant, a double in the nu one)
-        const double local_eps = eps > tenth ? eps : tenth;
+        const double local_eps = tenth > eps ? tenth : eps;
         __syncthreads();
-        const int steps = __builtin_amdgcn_readfirstlane(local_eps > 0.0 ? 1 : 0)
-                              ? ss_local<E, W, NU, false, TB>(sh, map, K, ld, col, kd, fl, member, P.Cp, P.Cn, local_eps, P.max_iter)
-                              : ss_local<E, W, NU, true, TB>(sh, map, K, ld, col, kd, fl, member, P.Cp, P.Cn, local_eps, P.max_iter);
+        bool no_score = !__builtin_amdgcn_readfirstlane(local_eps > 0.0 ? 1 : 0);
+        int steps = 0;
+        if (!no_score) {
+            steps = ss_local<E, W, NU, false, TB>(sh, map, K, ld, col, kd, fl, member, P.Cp, P.Cn, local_eps, P.max_iter, no_score);
+            if (no_score) {   // once more from the start
+                __syncthreads();
+#pragma unroll
+                for (int e = 0; e < E; ++e) {
+                    fl[e] = f[e];
+#pragma unroll
+                    for (int w = 0; w < W; ++w) sh.z[w][tid * E + e] = z_old[e];
+                }
+                __syncthreads();
+            }
+        }
+        if (no_score) steps = ss_local<E, W, NU, true, TB>(sh, map, K, ld, col, kd, fl, member, P.Cp, P.Cn, local_eps, P.max_iter, no_score);
         inner_here += steps;
         if (!NU) local_iter += steps;   // (the nu variant reports none, smo_kernel.cpp:283)
         // alpha_diff of the working set, in its order: -(new - old) * y

@@ -205,17 +205,23 @@ struct SvState {
     double f[N], k[N];        // f and row i at the elements of the wavefronts' candidates for j2 (the others are not written)
 };
 
-// The iterations of c_smo_solve.  NONE: the threshold is not positive, so that an element may violate it without being
-// a candidate for j2 (the reference's j2 then stays 0, smo_kernel.cpp:78); otherwise that cannot happen.
+// The iterations of c_smo_solve.  An element that violates may have no score: the threshold is not positive and its f not above
+// `up`, or the score is infinite or NaN (an a that is negative with a b^2 beyond the largest double; kernel values that are no
+// numbers).  The reference's j2 then stays 0 (smo_kernel.cpp:78).  NONE: that is done here.  Without it such a step goes
+// wrong, and `no_score` is set for the caller to start over; one instruction, where a way out of the loop in front of the
+// step costs 5 %.
 // Takes up to `left` steps, counted in n_iter; returns whether the solve has ended (nothing violates, or max_iter).
 template <int E, int W, int LDK, bool NONE, typename TB>
 __device__ __forceinline__ bool c_smo_iterate(SvState<E * 64 * W, W> &sh, SvCand *s_i, SvCand *s_j, int ws, const TB *kws,
                                               const double (&kd)[E], double (&f)[E], unsigned &in_up, unsigned &in_low, double local_eps,
-                                              int max_iter, int &n_iter, int left) {
+                                              int max_iter, int &n_iter, int left, bool &no_score) {
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     bool go_on;
+    double min_t = -TSVM_INF;
+    int worst = 0;   // high word of the largest score that a step was taken on
     do {
+        if (!NONE) worst = imax_sel(worst, __double2hiint(min_t));
         // i = first argmin of f over I_up (smo_kernel.cpp:41-59); with an empty I_up any i does, since nothing violates then
         double fu[E];
 #pragma unroll
@@ -257,7 +263,6 @@ __device__ __forceinline__ bool c_smo_iterate(SvState<E * 64 * W, W> &sh, SvCand
             // (-up > -f in the reference: f > up, which is b > 0; outside I_low b is negative and q of no use)
             qs[e] = __hiloint2double(b_low[e] > 0.0 ? __double2hiint(q) : SV_NONE_HI, __double2loint(q));
         }
-        double min_t;
         const int win_j = wave_first_argmin<E>(qs, tid * E, min_t, m, at);
         publish_row<E, TB>(sh.f + tid * E, sh.k + tid * E, win_j, f, kI);
         if constexpr (W > 1) {
@@ -296,6 +301,7 @@ __device__ __forceinline__ bool c_smo_iterate(SvState<E * 64 * W, W> &sh, SvCand
         for (int e = 0; e < E; ++e) f[e] = __builtin_fma(-l, (double) kJ[e] - (double) kI[e], f[e]);
         n_iter += go_on;
     } while (go_on && --left > 0);
+    if (!NONE) no_score |= __builtin_amdgcn_readfirstlane(go_on ? imax_sel(worst, __double2hiint(min_t)) : worst) >= SV_NONE_HI;
     return !go_on;
 }
 
@@ -513,67 +519,75 @@ __global__ __launch_bounds__(64 * W) void c_smo_solve_kernel(
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     double f[E], a_old[E], kd[E];
-    unsigned in_up = 0, in_low = 0, plus = 0;   // bit e: element e is in I_up, in I_low, has a label > 0
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const int t = tid * E + e;
-        const bool active = t < ws;
-        const int w = active ? working_set[t] : 0;
-        f[e] = active ? f_val[w] : 0.0;
-        a_old[e] = active ? alpha[w] : 0.0;
-        const double y = active ? (double) label[w] : 0.0;
-        kd[e] = active ? k_diag[w] : 1.0;
-        sh.kd[t] = kd[e];
-        sh.bound[t].hi = y > 0 ? Cp : 0.0;
-        sh.bound[t].lo = y < 0 ? -Cn : 0.0;
-        plus |= (y > 0 ? 1u : 0u) << e;
-#pragma unroll
-        for (int w = 0; w < W; ++w) sh.z[w][t] = a_old[e] * y;
-        in_up |= (is_I_up(a_old[e], y, Cp, Cn) ? 1u : 0u) << e;
-        in_low |= (is_I_low(a_old[e], y, Cp, Cn) ? 1u : 0u) << e;
-    }
-    // The initial gap fixes the local stopping threshold (smo_kernel.cpp:61-66).  It is the only place
-    // where the value of low = max of f over I_low is needed: inside the loop the stopping test
-    // low - up < local_eps is evaluated per element, as "no I_low element has f - up >= local_eps"
-    // (the same decision, since rounding the subtraction is monotone), which costs a ballot instead of
-    // a second cross-lane reduction per iteration.
-    double local_eps;
-    {
-        double mn = TSVM_INF, mx = -TSVM_INF;
+    unsigned in_up, in_low, plus;   // bit e: element e is in I_up, in I_low, has a label > 0
+    int n_iter;
+    for (bool with_none = false;;) {
+        in_up = in_low = plus = 0;
+        n_iter = 0;
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            mn = fmin_f64(mn, (in_up >> e) & 1u ? f[e] : TSVM_INF);
-            mx = fmax_f64(mx, (in_low >> e) & 1u ? f[e] : -TSVM_INF);
-        }
-        mn = wave_min_f64(mn);
-        mx = wave_max_f64(mx);
-        if (lane == 0) { s_red[0][wave] = mn; s_red[1][wave] = mx; }
-        __syncthreads();
-        double up0 = s_red[0][0];
+            const int t = tid * E + e;
+            const bool active = t < ws;
+            const int w = active ? working_set[t] : 0;
+            f[e] = active ? f_val[w] : 0.0;
+            a_old[e] = active ? alpha[w] : 0.0;
+            const double y = active ? (double) label[w] : 0.0;
+            kd[e] = active ? k_diag[w] : 1.0;
+            sh.kd[t] = kd[e];
+            sh.bound[t].hi = y > 0 ? Cp : 0.0;
+            sh.bound[t].lo = y < 0 ? -Cn : 0.0;
+            plus |= (y > 0 ? 1u : 0u) << e;
 #pragma unroll
-        for (int w = 1; w < W; ++w) up0 = fmin_f64(up0, s_red[0][w]);
-        const double local_diff = block_max<W>(s_red[1]) - up0;
-        const double t = 0.1f * local_diff;   // float literal, as in the reference (smo_kernel.cpp:64)
-        local_eps = eps > t ? eps : t;
-        if (tid == 0) diff[0] = local_diff;
-    }
-    int n_iter = 0;
-    if (!__builtin_amdgcn_readfirstlane(local_eps > 0.0 ? 1 : 0)) {
-        c_smo_iterate<E, W, LDK, true, TB>(sh, s_i, s_j, ws, kws, kd, f, in_up, in_low, local_eps, max_iter, n_iter, 0x7fffffff);
-    } else if constexpr (W == 4) {
-        // Where rounded scores do not decide they often go on not deciding (far apart points of equal f): the
-        // exact stretch doubles each time the rounded one has been the shorter of the two.
-        bool done;
-        int stretch = 64;
-        do {
-            const int before = n_iter;
-            done = c_smo_iterate_rounded<E, LDK, TB>(sh, s_i, (SvScore *) s_j, s_step, ws, kws, kd, f, in_up, in_low, local_eps, max_iter, n_iter);
-            if (done) break;
-            stretch = n_iter - before > stretch ? 64 : stretch < 1024 ? 2 * stretch : stretch;
-            done = c_smo_iterate<E, W, LDK, false, TB>(sh, s_i, s_j, ws, kws, kd, f, in_up, in_low, local_eps, max_iter, n_iter, stretch);
-        } while (!done);
-    } else {
-        c_smo_iterate<E, W, LDK, false, TB>(sh, s_i, s_j, ws, kws, kd, f, in_up, in_low, local_eps, max_iter, n_iter, 0x7fffffff);
+            for (int w = 0; w < W; ++w) sh.z[w][t] = a_old[e] * y;
+            in_up |= (is_I_up(a_old[e], y, Cp, Cn) ? 1u : 0u) << e;
+            in_low |= (is_I_low(a_old[e], y, Cp, Cn) ? 1u : 0u) << e;
+        }
+        // The initial gap fixes the local stopping threshold (smo_kernel.cpp:61-66).  It is the only place
+        // where the value of low = max of f over I_low is needed: inside the loop the stopping test
+        // low - up < local_eps is evaluated per element, as "no I_low element has f - up >= local_eps"
+        // (the same decision, since rounding the subtraction is monotone), which costs a ballot instead of
+        // a second cross-lane reduction per iteration.
+        double local_eps;
+        {
+            double mn = TSVM_INF, mx = -TSVM_INF;
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                mn = fmin_f64(mn, (in_up >> e) & 1u ? f[e] : TSVM_INF);
+                mx = fmax_f64(mx, (in_low >> e) & 1u ? f[e] : -TSVM_INF);
+            }
+            mn = wave_min_f64(mn);
+            mx = wave_max_f64(mx);
+            if (lane == 0) { s_red[0][wave] = mn; s_red[1][wave] = mx; }
+            __syncthreads();
+            double up0 = s_red[0][0];
+#pragma unroll
+            for (int w = 1; w < W; ++w) up0 = fmin_f64(up0, s_red[0][w]);
+            const double local_diff = block_max<W>(s_red[1]) - up0;
+            const double t = 0.1f * local_diff;   // float literal, as in the reference (smo_kernel.cpp:64)
+            local_eps = t > eps ? t : eps;
+            if (tid == 0) diff[0] = local_diff;
+        }
+        bool no_score = false;
+        if (with_none || !__builtin_amdgcn_readfirstlane(local_eps > 0.0 ? 1 : 0)) {
+            c_smo_iterate<E, W, LDK, true, TB>(sh, s_i, s_j, ws, kws, kd, f, in_up, in_low, local_eps, max_iter, n_iter, 0x7fffffff, no_score);
+        } else if constexpr (W == 4) {
+            // Where rounded scores do not decide they often go on not deciding (far apart points of equal f): the
+            // exact stretch doubles each time the rounded one has been the shorter of the two.
+            bool done;
+            int stretch = 64;
+            do {
+                const int before = n_iter;
+                done = c_smo_iterate_rounded<E, LDK, TB>(sh, s_i, (SvScore *) s_j, s_step, ws, kws, kd, f, in_up, in_low, local_eps, max_iter, n_iter);
+                if (done) break;
+                stretch = n_iter - before > stretch ? 64 : stretch < 1024 ? 2 * stretch : stretch;
+                done = c_smo_iterate<E, W, LDK, false, TB>(sh, s_i, s_j, ws, kws, kd, f, in_up, in_low, local_eps, max_iter, n_iter, stretch, no_score);
+            } while (!done && !no_score);
+        } else {
+            c_smo_iterate<E, W, LDK, false, TB>(sh, s_i, s_j, ws, kws, kd, f, in_up, in_low, local_eps, max_iter, n_iter, 0x7fffffff, no_score);
+        }
+        if (!no_score) break;
+        with_none = true;   // (nothing has been written yet: once more from the start)
+        __syncthreads();
     }
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -660,13 +674,12 @@ __global__ __launch_bounds__(64 * W) void nu_smo_solve_kernel(
 #pragma unroll
         for (int w = 1; w < W; ++w) { up_p0 = fmin_f64(up_p0, s_red[0][w]); up_n0 = fmin_f64(up_n0, s_red[1][w]); }
         const double dp = block_max<W>(s_red[2]) - up_p0, dn = block_max<W>(s_red[3]) - up_n0;
-        const double local_diff = dp > dn ? dp : dn;
+        const double local_diff = dp < dn ? dn : dp;
         const double t = 0.1 * local_diff;
-        local_eps = eps > t ? eps : t;
+        local_eps = t > eps ? t : eps;
         first_diff = local_diff;
     }
     __syncthreads();
-    const bool none_possible = __builtin_amdgcn_readfirstlane(local_eps > 0.0 ? 0 : 1) != 0;
     int numOfIter = 0;
     while (true) {
         double fup[E], fun[E];
@@ -739,7 +752,7 @@ __global__ __launch_bounds__(64 * W) void nu_smo_solve_kernel(
         const int side = take_p ? 0 : 1;
         const int i = take_p ? ip : in;
         int j2 = take_p ? j2p : j2n;
-        if (none_possible && is_none(take_p ? f_val_j2p : f_val_j2n)) {
+        if (is_none(take_p ? f_val_j2p : f_val_j2n)) {   // (as in c_smo_iterate)
             j2 = 0;
             __syncthreads();
             if (tid == 0) { s_f[side][0] = f[0]; *(TB *) s_k[side] = take_p ? kIp[0] : kIn[0]; }

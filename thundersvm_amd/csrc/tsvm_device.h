@@ -379,6 +379,7 @@ __device__ __forceinline__ double fmax_f64(double a, double b) {
     return r;
 }
 __device__ __forceinline__ int imin_sel(int a, int b) { return b < a ? b : a; }
+__device__ __forceinline__ int imax_sel(int a, int b) { return b > a ? b : a; }
 
 __device__ __forceinline__ double wave_min_f64(double v) {
     v = fmin_f64(v, dpp_f64<TSVM_DPP_XOR1>(v));
