@@ -210,3 +210,22 @@ def test_indicator_columns_are_found_by_all_entries(last, first):
     """The host looks at the first entries only; what the last of 100,000 holds still decides."""
     import selftest_lib
     assert selftest_lib.lib().tsvm_selftest_indicator_run(last) == first
+
+
+@pytest.mark.parametrize("m", [1, 255, 256, 300])
+@pytest.mark.parametrize("kt", [0, 2])
+def test_batch_without_any_entry(m, kt):
+    """Rows without entries only, on sparse support vectors: every one is the zero vector."""
+    rng = np.random.default_rng(kt)
+    n, d = 700, 2400
+    col = np.sort(rng.random((n, d)).argsort(1)[:, :12], 1).astype(np.int32).ravel() + 1
+    tr = D.CsrData(np.arange(n + 1, dtype=np.int64) * 12, col, rng.standard_normal(12 * n).astype(np.float32).astype(np.float64),
+                   np.where(rng.random(n) < 0.5, 1.0, -1.0))
+    prm = make_param(kernel_type=kt, C=2.0, gamma=0.05)
+    te = D.CsrData(np.zeros(m + 1, np.int64), np.zeros(0, np.int32), np.zeros(0), None)
+    gm = Model(0).train(tr, prm)
+    want = O.Model(tr.ptr, tr.col, tr.val, tr.y, _oparam(prm)).predict(te.ptr, te.col, te.val, 100)[1]
+    for batch in (-1, 100):
+        got = gm.predict(te, batch)[1]
+        assert got.shape == want.shape and np.abs(got - want).max() < 1e-6 and (got == got[0]).all()
+    assert np.array_equal(gm.predict(Dataset(te).to_device())[1], got)

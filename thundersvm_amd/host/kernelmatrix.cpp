@@ -802,7 +802,7 @@ void KernelMatrix::get_rows(const RowStore &batch, size_t first, size_t n_rows, 
         return;
     }
     // The batch's rows wait in LDS, sixteen at a time, and the support vectors' sliced copy streams by, as in training; a batch
-    // with a row too long for that is staged as a dense matrix, and so is any batch when a support vector holds an infinity
+    // with a row too long for that or without any entry is staged as a dense matrix, and so is any batch when a support vector holds an infinity
     // or NaN, whose product with an absent (zero) feature is not zero.  Kernel values of text rows, staged / sliced, us: 6,000
     // support vectors 65 / 23 for one row, 87 / 38 for 64, 217 / 79 for 1,000, 1,148 / 263 for 4,099; 800 support vectors 24 / 22,
     // 27 / 33, 65 / 35, 313 / 64; 3,000 31 / 23, 37 / 38, 128 / 42, 674 / 148: few of them fill few workgroups, so few rows go
@@ -810,7 +810,7 @@ void KernelMatrix::get_rows(const RowStore &batch, size_t first, size_t n_rows, 
     const int wt = R.values_fit_float ? TSVM_ROW_F32 : TSVM_ROW_F64;
     int longest = 0;
     for (int r = 0; r < m; ++r) longest = std::max(longest, (int) (h_ptr_.data()[r + 1] - h_ptr_.data()[r]));
-    if (R.sliced_lds && R.values_finite && (n >= 3072 || m >= 256) && tsvm_get_rows_csr_sliced_lds((int) R.n_features, longest, wt) > 0) {
+    if (longest > 0 && R.sliced_lds && R.values_finite && (n >= 3072 || m >= 256) && tsvm_get_rows_csr_sliced_lds((int) R.n_features, longest, wt) > 0) {
         abi_check(tsvm_get_rows_csr_sliced(R.ell_col.data(), R.ell_val.data(), wt, R.slice_ptr.data(), n, R.self_dot.data(),
                                            b_val_.data(), b_col_.data(), b_ptr_.data(), nullptr, m, b.sd, (int) R.n_features, longest,
                                            (int) param.kernel_type, param.gamma, param.coef0, param.degree, d_out, row_type(), nullptr, ld,
