@@ -1,5 +1,5 @@
 // What the local SMO solvers share (smo_solve.hip: one call per working set; smo_small.hip: whole solves of small
-// problems): masked extrema over a working set that is spread over the registers of one to eight wavefronts, and LDS writes by
+// problems): masked extrema over a working set that is spread over the registers of one, two or four wavefronts, and LDS writes by
 // single lanes.  See smo_solve.hip for what bounds these kernels and why they are written this way.
 #pragma once
 #include "tsvm_device.h"

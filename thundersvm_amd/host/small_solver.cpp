@@ -12,8 +12,7 @@ using tsvm::DeviceBuffer;
 
 size_t SmallSolve::slots(size_t n_pos, size_t n_neg) { return (n_pos + 3) / 4 * 4 + n_neg; }
 
-// (an odd working set leaves its last place to chance in the shared window, and NaNs are nobody's problem: both stay
-// with SolveTask)
+// (an odd working set leaves its last place to chance in the shared window: that stays with SolveTask)
 bool SmallSolve::takes(size_t n_pos, size_t n_neg, int ws_size) {
     return n_pos + n_neg >= 2 && slots(n_pos, n_neg) <= (size_t) tsvm_smo_small_max() && ws_size >= 2 && ws_size % 2 == 0 &&
            (size_t) ws_size <= n_pos + n_neg;
