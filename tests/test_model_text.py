@@ -71,3 +71,19 @@ def test_malformed_support_vector_line(tmp_path):
         open(path, "w").write("\n".join(lines))
         with pytest.raises(capi.TsvmError):
             Model(0).load(path)
+
+
+def test_rho_that_is_no_number(tmp_path):
+    """What training leaves for a problem without a solution is written as inf, -inf or nan, and read back."""
+    text, coef, *_ = _model_text(20, 3, np.random.default_rng(3))
+    lines = text.split("\n")
+    at = [i for i, l in enumerate(lines) if l.startswith("rho ")][0]
+    lines[at] = "rho nan -inf 0.5 "
+    path, out = str(tmp_path / "in.model"), str(tmp_path / "out.model")
+    open(path, "w").write("\n".join(lines))
+    m = Model(0)
+    m.load(path)
+    assert np.isnan(m.rho[0]) and m.rho[1] == -np.inf and m.rho[2] == 0.5
+    assert m.label.tolist() == [1, 2, 3] and m.total_sv == 20 and np.array_equal(m.coef.reshape(2, 20), coef)
+    m.save(out)
+    assert open(out).read() == "\n".join(lines)

@@ -317,6 +317,21 @@ void SvmModel::load_from_file(std::string path) {
     load_from_string(ss.str());
 }
 
+// The next number of the text; "inf" and "nan", which save_to_string writes for a rho that is none (an infeasible nu, a
+// problem without room) and which the stream's own extraction would end the text at, included.
+static bool next_number(std::istream &in, float_type &v) {
+    std::string t;
+    if (!(in >> t)) return false;
+    char *end;
+    const double d = strtod(t.c_str(), &end);
+    if (end == t.c_str() || *end) {
+        in.setstate(std::ios::failbit);
+        return false;
+    }
+    v = d;
+    return true;
+}
+
 // svmmodel.cpp:280-383
 void SvmModel::load_from_string(std::string data) {
     sv_k_mat.reset();
@@ -346,7 +361,7 @@ void SvmModel::load_from_string(std::string data) {
         } else if (key == "total_sv") {
             iss >> n_total_sv;
         } else if (key == "rho") {
-            for (int i = 0; i < n_binary_models; ++i) iss >> rho[i];
+            for (int i = 0; i < n_binary_models; ++i) next_number(iss, rho[i]);
         } else if (key == "label") {
             label.assign(n_classes, 0);
             for (int i = 0; i < n_classes; ++i) iss >> label[i];
@@ -355,10 +370,10 @@ void SvmModel::load_from_string(std::string data) {
         } else if (key == "probA") {
             param.probability = 1;
             probA.assign(n_binary_models, 0);
-            for (int i = 0; i < n_binary_models; ++i) iss >> probA[i];
+            for (int i = 0; i < n_binary_models; ++i) next_number(iss, probA[i]);
         } else if (key == "probB") {
             probB.assign(n_binary_models, 0);
-            for (int i = 0; i < n_binary_models; ++i) iss >> probB[i];
+            for (int i = 0; i < n_binary_models; ++i) next_number(iss, probB[i]);
         } else if (key == "coef") {
             std::string line;
             std::getline(iss, line);
@@ -366,7 +381,7 @@ void SvmModel::load_from_string(std::string data) {
             std::stringstream ls(line);
             linear_coef.clear();
             float_type v;
-            while (ls >> v) linear_coef.push_back(v);
+            while (next_number(ls, v)) linear_coef.push_back(v);
         } else if (key == "SV") {
             // One line per support vector: `rows` coefficients, then index:value tokens (svmmodel.cpp:356-381).  The
             // lines are most of a large model's text: they are cut into runs of whole lines and parsed side by side,
