@@ -13,6 +13,10 @@ HIP_FLAGS = ["-O3", "--offload-arch=gfx950", "-fPIC", "-std=c++17", "-ffp-contra
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-unused-value",
              "-Wno-unknown-warning-option", "-Wno-unused-command-line-argument"]
 
+# The local solvers' loops are one chain of dependent instructions with little else on the CU: where a loop starts against the
+# instruction cache's lines is worth 1 to 2 % of a step (1,024 elements: 0.986 us unaligned, 0.970 from a multiple of 256).
+FILE_FLAGS = {"smo_solve.hip": ["-falign-loops=256"]}
+
 
 def _run(cmd):
     print(" ".join(cmd), flush=True)
@@ -29,7 +33,8 @@ def build_kernels(extra=(), only=None):
     objs = [os.path.join(objdir, f[:-4] + ".o") for f in srcs]
     todo = [(f, o) for f, o in zip(srcs, objs) if only is None or f in only or not os.path.exists(o)]
     with concurrent.futures.ThreadPoolExecutor(max_workers=min(6, max(1, len(todo)))) as pool:
-        list(pool.map(lambda fo: _run(["hipcc", *HIP_FLAGS, *extra, "-c", "-o", fo[1], os.path.join(CSRC, fo[0])]), todo))
+        list(pool.map(lambda fo: _run(["hipcc", *HIP_FLAGS, *FILE_FLAGS.get(fo[0], []), *extra, "-c", "-o", fo[1],
+                                                     os.path.join(CSRC, fo[0])]), todo))
     _run(["hipcc", *HIP_FLAGS, *extra, "-shared", "-o", KERNEL_LIB, *objs])
     return KERNEL_LIB
 

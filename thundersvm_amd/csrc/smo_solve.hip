@@ -184,6 +184,36 @@ __device__ __forceinline__ bool solver_elected(int *gate, int epoch, int target_
     return s_elected != 0;
 }
 
+// What a thread's elements start from.  Every load is made (for positions beyond ws the last element's: f, alpha and the label are
+// zero and the diagonal 1 there) and none waits for another but for its id; E * 4 loads behind a test each were a chain of sixteen
+// misses.  A whole call of one step 12.0 -> 10.9 us; epsilon-SVR on 40,000 rows (212 launches) 98.8 -> 98.0 ms.
+template <int E>
+__device__ __forceinline__ void gather_elems(const int *__restrict__ working_set, int ws, const double *__restrict__ f_val, const double *alpha_val,
+                                             const int *__restrict__ labels, const double *__restrict__ k_diag, double (&f)[E], double (&alpha)[E],
+                                             double (&kd)[E], int (&label)[E]) {
+    int id[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const int t = (int) threadIdx.x * E + e;
+        id[e] = working_set[t < ws ? t : ws - 1];
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        f[e] = f_val[id[e]];
+        alpha[e] = alpha_val[id[e]];
+        label[e] = labels[id[e]];
+        kd[e] = k_diag[id[e]];
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const bool active = (int) threadIdx.x * E + e < ws;
+        f[e] = active ? f[e] : 0.0;
+        alpha[e] = active ? alpha[e] : 0.0;
+        label[e] = active ? label[e] : 0;
+        kd[e] = active ? kd[e] : 1.0;
+    }
+}
+
 // What the nu solver keeps in LDS, per element of the working set (inactive elements: both bounds zero, so neither in
 // I_up nor in I_low).
 template <int N, int W>
@@ -507,6 +537,9 @@ __global__ __launch_bounds__(64 * W) void c_smo_solve_kernel(
     double *__restrict__ alpha_diff, const int *__restrict__ working_set, int ws, double Cp, double Cn,
     const TB *kws, const double *__restrict__ k_diag, double eps, double *__restrict__ diff,
     int max_iter, int *__restrict__ gate, int epoch, int target_xcd) {
+    double f[E], a_old[E], kd[E];
+    int y_of[E];
+    gather_elems<E>(working_set, ws, f_val, alpha, label, k_diag, f, a_old, kd, y_of);   // (on its way during the election)
     if (gate && !solver_elected(gate, epoch, target_xcd)) return;
     constexpr int N = E * 64 * W;
     __shared__ SvState<N, W> sh;
@@ -519,7 +552,6 @@ __global__ __launch_bounds__(64 * W) void c_smo_solve_kernel(
     __builtin_amdgcn_s_setprio(3);
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    double f[E], a_old[E], kd[E];
     unsigned in_up, in_low, plus;   // bit e: element e is in I_up, in I_low, has a label > 0
     int n_iter;
     for (bool with_none = false;;) {
@@ -528,12 +560,7 @@ __global__ __launch_bounds__(64 * W) void c_smo_solve_kernel(
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const int t = tid * E + e;
-            const bool active = t < ws;
-            const int w = active ? working_set[t] : 0;
-            f[e] = active ? f_val[w] : 0.0;
-            a_old[e] = active ? alpha[w] : 0.0;
-            const double y = active ? (double) label[w] : 0.0;
-            kd[e] = active ? k_diag[w] : 1.0;
+            const double y = (double) y_of[e];
             sh.kd[t] = kd[e];
             sh.bound[t].hi = y > 0 ? Cp : 0.0;
             sh.bound[t].lo = y < 0 ? -Cn : 0.0;
@@ -589,6 +616,7 @@ __global__ __launch_bounds__(64 * W) void c_smo_solve_kernel(
         if (!no_score) break;
         with_none = true;   // (nothing has been written yet: once more from the start)
         __syncthreads();
+        gather_elems<E>(working_set, ws, f_val, alpha, label, k_diag, f, a_old, kd, y_of);
     }
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -623,6 +651,9 @@ __global__ __launch_bounds__(64 * W) void nu_smo_solve_kernel(
     double *__restrict__ alpha_diff, const int *__restrict__ working_set, int ws, double C,
     const TB *kws, const double *__restrict__ k_diag, double eps, double *__restrict__ diff,
     int max_iter, int *__restrict__ gate, int epoch, int target_xcd) {
+    double f[E], a_old[E], kd[E];
+    int y_of[E];
+    gather_elems<E>(working_set, ws, f_val, alpha, label, k_diag, f, a_old, kd, y_of);   // (on its way during the election)
     if (gate && !solver_elected(gate, epoch, target_xcd)) return;
     constexpr int N = E * 64 * W;
     __shared__ SvShared<N, W> sh;
@@ -633,17 +664,11 @@ __global__ __launch_bounds__(64 * W) void nu_smo_solve_kernel(
     __builtin_amdgcn_s_setprio(3);
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    double f[E], a_old[E], kd[E];
     unsigned member = 0, plus = 0;   // plus: bit e: element e has a label > 0
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const int t = tid * E + e;
-        const bool active = t < ws;
-        const int w = active ? working_set[t] : 0;
-        f[e] = active ? f_val[w] : 0.0;
-        a_old[e] = active ? alpha[w] : 0.0;
-        const double y = active ? (double) label[w] : 0.0;
-        kd[e] = active ? k_diag[w] : 1.0;
+        const double y = (double) y_of[e];
         sh.kd[t] = kd[e];
         sh.bound[t].hi = y > 0 ? C : 0.0;
         sh.bound[t].lo = y < 0 ? -C : 0.0;
