@@ -500,6 +500,26 @@ def test_selections_in_a_row_on_one_workspace(n, nu):
 
 
 @pytest.mark.parametrize("nu", [0, 1])
+@pytest.mark.parametrize("group", [2, 63, 64, 255, 300])
+@pytest.mark.parametrize("n,n_select", [(1030, 1000), (6000, 16), (6000, 64), (6000, 512)])
+def test_selection_of_lists_with_equal_values(n, n_select, group, nu):
+    """Every value of f belongs to `group` instances, all free: a list's order within a value, and the place of an instance in the
+    paired side's list, are up to the index, in lists that end inside a group, inside sixteen entries and inside 64."""
+    rng = np.random.default_rng(n + group)
+    f = rng.permutation(np.repeat(rng.normal(size=n // group + 1), group)[:n])
+    y = np.where(rng.random(n) < 0.5, 1, -1).astype(np.int32)
+    alpha = np.full(n, 0.5)
+    want = O.select_working_set(f, y, alpha, 1.0, 1.0, np.zeros(0, dtype=np.int32), n_select, nu=bool(nu))
+    f_d, y_d, a_d = G.dev(f), G.dev(y), G.dev(alpha)
+    wsp = torch.empty(capi.kernel_lib().tsvm_select_workspace(n), dtype=torch.uint8, device="cuda")
+    for entry in ("tsvm_select_working_set", "tsvm_select_working_set_again", "tsvm_select_working_set_again"):
+        out_d = torch.full((n_select,), -7, dtype=torch.int32, device="cuda")
+        capi.call(entry, G.ptr(f_d), G.ptr(y_d), G.ptr(a_d), n, 1.0, 1.0, None, 0, G.ptr(out_d), n_select, nu, G.ptr(wsp), G.stream())
+        got = G.host(out_d)
+        assert np.array_equal(got, want), "first mismatch at %s" % np.flatnonzero(got != want)[:5]
+
+
+@pytest.mark.parametrize("nu", [0, 1])
 @pytest.mark.parametrize("n,tie_mode", [(150, 0), (5000, 2), (200000, 0), (200000, 1)])
 def test_selection_with_folded_ids(n, tie_mode, nu):
     """The 2n-variable problem of SVR (svr.cpp:14-28): the selection also delivers each id modulo n / 2, the stored row

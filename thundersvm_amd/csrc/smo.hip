@@ -47,9 +47,10 @@ struct SelWorkspace {   // device-side layout, carved from the caller's workspac
     uint8_t *flags;     // [n] side membership bits
     uint32_t *hist;     // [SEL_MAX_PASS][SEL_MAX_SIDES][SEL_BINS]
     SelState *state;    // [SEL_MAX_PASS + 1][SEL_MAX_SIDES]
-    uint32_t *count;    // [SEL_MAX_SIDES]
+    uint32_t *count;    // [SEL_MAX_SIDES], then the workgroups of sel_final_kernel that are done
     uint64_t *list_key; // [SEL_MAX_SIDES][MAX_WS]
     uint32_t *list_idx; // [SEL_MAX_SIDES][MAX_WS]
+    int2 *sorted;       // [SEL_MAX_SIDES][MAX_WS] the lists in order: instance, its place in the paired side's list or -1
 };
 
 static size_t sel_align(size_t v) { return (v + 255) & ~(size_t) 255; }
@@ -62,13 +63,14 @@ static size_t sel_carve(void *base, int64_t n, SelWorkspace *w) {
     void *flags = take((size_t) n);
     void *hist = take(sizeof(uint32_t) * SEL_MAX_PASS * SEL_MAX_SIDES * SEL_BINS);
     void *state = take(sizeof(SelState) * (SEL_MAX_PASS + 1) * SEL_MAX_SIDES);
-    void *count = take(sizeof(uint32_t) * SEL_MAX_SIDES);
+    void *count = take(sizeof(uint32_t) * (SEL_MAX_SIDES + 1));
     void *lk = take(sizeof(uint64_t) * SEL_MAX_SIDES * MAX_WS);
     void *li = take(sizeof(uint32_t) * SEL_MAX_SIDES * MAX_WS);
+    void *so = take(sizeof(int2) * SEL_MAX_SIDES * MAX_WS);
     if (w) {
         w->keys = (uint64_t *) keys; w->flags = (uint8_t *) flags;
         w->hist = (uint32_t *) hist; w->state = (SelState *) state; w->count = (uint32_t *) count;
-        w->list_key = (uint64_t *) lk; w->list_idx = (uint32_t *) li;
+        w->list_key = (uint64_t *) lk; w->list_idx = (uint32_t *) li; w->sorted = (int2 *) so;
     }
     return off;
 }
@@ -129,16 +131,17 @@ __device__ __forceinline__ uint64_t f_to_key(double f) {
 __device__ __forceinline__ bool sel_side_descending(int side, int n_sides) { return n_sides == 2 ? side == 1 : side >= 2; }
 
 // What a call needs to find in the workspace: zeroed histograms for the digits that are counted with atomics
-// by the whole grid and zeroed list lengths.  Written by sel_init_kernel, and again
+// by the whole grid and zeroed counters.  Written by sel_init_kernel, and again
 // by sel_final_kernel once it has read what it needs, so that the next call on the same workspace (same n,
 // same sides) can start counting straight away.
-__device__ __forceinline__ void sel_arm(const SelWorkspace &w, const SelGeom &g, int p_full, int64_t gid, int64_t stride) {
+__device__ __forceinline__ void sel_clear_hist(const SelWorkspace &w, int p_full, int64_t gid, int64_t stride) {
     for (int64_t e = gid; e < (int64_t) p_full * SEL_MAX_SIDES * SEL_BINS; e += stride) w.hist[e] = 0;
-    if (gid < SEL_MAX_SIDES) w.count[gid] = 0;
 }
 
-__global__ void sel_init_kernel(SelWorkspace w, SelGeom g, int p_full) {
-    sel_arm(w, g, p_full, (int64_t) blockIdx.x * blockDim.x + threadIdx.x, (int64_t) gridDim.x * blockDim.x);
+__global__ void sel_init_kernel(SelWorkspace w, int p_full) {
+    const int64_t gid = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    sel_clear_hist(w, p_full, gid, (int64_t) gridDim.x * blockDim.x);
+    if (gid <= SEL_MAX_SIDES) w.count[gid] = 0;
 }
 
 // Computes, in LDS, the state after pass p-1's histogram has been consumed (st_out), from the
@@ -601,6 +604,7 @@ __global__ __launch_bounds__(SEL_T) void sel_compact_kernel(SelWorkspace w, int6
     __shared__ SelState st[SEL_MAX_SIDES];
     __shared__ uint32_t scratch[SEL_T + 16];
     sel_advance_state(w, g, p_full, st, scratch);
+    if (blockIdx.x == 0 && (int) threadIdx.x < g.n_sides) w.state[p_full * SEL_MAX_SIDES + threadIdx.x] = st[threadIdx.x];
     if (sel_undecided(g, st)) return;
     sel_collect(w, n, g, st, (int64_t) blockIdx.x * SEL_T + threadIdx.x, (int64_t) gridDim.x * SEL_T);
 }
@@ -633,51 +637,25 @@ __device__ void sel_tail(const SelWorkspace &w, int64_t n, const SelGeom &g, int
     __syncthreads();
 }
 
-// Final step: sort each side's list, replay the alternating scan, write the selection.
+// The lists in order by one workgroup: when it alone has made them (sel_tail).
 __device__ __forceinline__ bool comp_less(uint64_t ka, uint32_t ia, uint64_t kb, uint32_t ib) {
     return ka < kb || (ka == kb && ia < ib);
 }
-
-// (fold_n > 0: the ids are also written modulo fold_n to out_folded, for problems whose instances are stacked
-// copies of fold_n stored rows)
-template <int NS>   // NS = g.n_sides (32 KB of LDS with two sides, 64 KB with four)
-__global__ __launch_bounds__(MAX_WS) void sel_final_kernel(SelWorkspace w, int64_t n, SelGeom g, int p_full,
-                                                           int *__restrict__ out, int fold_n, int *__restrict__ out_folded) {
-    __shared__ uint64_t sk[NS][MAX_WS];
-    __shared__ uint32_t si[NS][MAX_WS];
-    __shared__ int pos_other[NS][MAX_WS];  // position of the same instance in the paired side's list, or -1
-    __shared__ int cnt[SEL_MAX_SIDES];
-    __shared__ int conflict, event[NS / 2], alone_in[NS][MAX_WS / 64];
-    __shared__ SelState st[SEL_MAX_SIDES];
-    __shared__ uint32_t scratch[SEL_T + 16];
+template <int NS>
+__device__ void sel_sort_here(const SelWorkspace &w, const SelGeom &g, const int *cnt, uint64_t (*sk)[MAX_WS], uint32_t (*si)[MAX_WS],
+                              int (&id_out)[NS], int (&pos_other)[NS]) {
     const int tid = threadIdx.x;
-    // the test sel_compact_kernel made: if it left the lists empty, the remaining digits and the lists are made here
-    sel_advance_state(w, g, p_full, st, scratch);
-    if (sel_undecided(g, st)) sel_tail(w, n, g, p_full, st, (uint32_t (*)[SEL_BINS]) &sk[0][0], scratch);
-    if (tid < SEL_MAX_SIDES) {
-        // (an atomic read: the lengths were counted with atomics, by this workgroup itself on the slow path)
-        int c = tid < g.n_sides ? (int) __hip_atomic_load(&w.count[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
-        cnt[tid] = c > MAX_WS ? MAX_WS : c;
-    }
-    if (tid == 0) conflict = 0;
-    __syncthreads();
-    for (int s = 0; s < g.n_sides; ++s) {
-        if (tid < cnt[s]) {
-            sk[s][tid] = w.list_key[s * MAX_WS + tid];
-            si[s][tid] = w.list_idx[s * MAX_WS + tid];
-        } else {
-            sk[s][tid] = ~0ull;
-            si[s][tid] = ~0u;
-        }
+    for (int s = 0; s < NS; ++s) {
+        sk[s][tid] = tid < cnt[s] ? w.list_key[s * MAX_WS + tid] : ~0ull;
+        si[s][tid] = tid < cnt[s] ? w.list_idx[s * MAX_WS + tid] : ~0u;
     }
     __syncthreads();
-    sel_arm(w, g, p_full, tid, MAX_WS);   // everything this call needed from the workspace is in LDS now
     // Bitonic sort, ascending composite, all sides at once.  Thread t owns compare-exchange pair t & 511 of
     // side t >> 9 (and of side 2 + (t >> 9) when there are four), so every thread works in every stage.  With
     // strides up to 64 a wavefront's 64 pairs cover one closed block of 128 entries, stage after stage: such
     // stages only need the wavefront's own LDS accesses kept in order, not a workgroup barrier.
     int m_sort = 2;
-    for (int s = 0; s < g.n_sides; ++s)
+    for (int s = 0; s < NS; ++s)
         while (m_sort < cnt[s]) m_sort <<= 1;   // padding entries are already in place behind the longest list
     const int pr = tid & (MAX_WS / 2 - 1);
     for (int size = 2; size <= m_sort; size <<= 1) {
@@ -686,7 +664,7 @@ __global__ __launch_bounds__(MAX_WS) void sel_final_kernel(SelWorkspace w, int64
             const int hi = lo | strd;
             const bool asc = (lo & size) == 0;
             if (hi < m_sort) {
-                for (int s = tid >> 9; s < g.n_sides; s += 2) {
+                for (int s = tid >> 9; s < NS; s += 2) {
                     const uint64_t ka = sk[s][lo], kb = sk[s][hi];
                     const uint32_t ia = si[s][lo], ib = si[s][hi];
                     const bool sw = asc ? comp_less(kb, ib, ka, ia) : comp_less(ka, ia, kb, ib);
@@ -704,12 +682,13 @@ __global__ __launch_bounds__(MAX_WS) void sel_final_kernel(SelWorkspace w, int64
     }
     __syncthreads();
     // real instance ids; descending sides stored idx_mask - id
-    for (int s = 0; s < g.n_sides; ++s)
-        if (tid < cnt[s] && sel_side_descending(s, g.n_sides)) si[s][tid] = g.idx_mask - si[s][tid];
+    for (int s = 0; s < NS; ++s)
+        if (tid < cnt[s] && sel_side_descending(s, NS)) si[s][tid] = g.idx_mask - si[s][tid];
     __syncthreads();
     // position of each entry in the paired side's list (binary search on the paired side's order)
-    const int half = g.n_sides / 2;
-    for (int s = 0; s < g.n_sides; ++s) {
+    constexpr int half = NS / 2;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
         const int o = s < half ? s + half : s - half;
         int res = -1;
         if (tid < cnt[s]) {
@@ -717,41 +696,151 @@ __global__ __launch_bounds__(MAX_WS) void sel_final_kernel(SelWorkspace w, int64
             const uint64_t k_here = sk[s][tid];
             const uint64_t k_o = ~k_here;
             const uint32_t id = si[s][tid];
-            const uint32_t i_o = sel_side_descending(o, g.n_sides) ? g.idx_mask - id : id;
+            const uint32_t i_o = sel_side_descending(o, NS) ? g.idx_mask - id : id;
             int lo = 0, hi = cnt[o];
             while (lo < hi) {
                 const int mid = (lo + hi) >> 1;
-                const uint32_t im = sel_side_descending(o, g.n_sides) ? g.idx_mask - si[o][mid] : si[o][mid];
+                const uint32_t im = sel_side_descending(o, NS) ? g.idx_mask - si[o][mid] : si[o][mid];
                 if (comp_less(sk[o][mid], im, k_o, i_o)) lo = mid + 1; else hi = mid;
             }
             if (lo < cnt[o] && sk[o][lo] == k_o && si[o][lo] == id) res = lo;
         }
-        pos_other[s][tid] = res;
+        pos_other[s] = res;
+        id_out[s] = (int) si[s][tid];
     }
+}
+
+// Final step: the lists in order, the alternating scan, the selection.
+//
+// The order comes from counting: a wavefront takes an entry, compares it with its side's list, 64 entries at a time, and the
+// entries below it are its place; the same against the paired side's list gives the place of the same instance there.  At
+// most 1,024 entries a side make 32 workgroups, and the one that draws the last ticket makes the scan.  One workgroup
+// that sorted the lists by a bitonic network in LDS and looked the places up by bisection took 26.8 us, 49 with four
+// sides, in which the rest of the chip was idle; this takes 9 (bound by the launch and a chain of three memory latencies).  nu-SVC
+// 5,001 x 23 4.39 -> 4.06 ms, epsilon-SVR 40,000 x 90 96.8 -> 92.9.  Entries per wavefront 1 / 2 / 4 / 8: 92.5 / 92.8 / 93.5 /
+// 95.5 ms there, 848 / 846 / 843 / 840 on seven classes of 300,000 rows, where workgroups wait for room among other pairs'.
+#define SEL_RANK_T 1024
+#define SEL_RANK_EACH 2   // entries a wavefront takes
+#define SEL_RANK_ENTRIES (SEL_RANK_T / 64 * SEL_RANK_EACH)
+
+// The entries of `key` [0, count) that are below (k, i), and whether (k, i) is among them (OWN: it is); one wavefront.
+template <bool OWN>
+__device__ __forceinline__ int sel_place(const uint64_t *key, const uint32_t *idx, int count, uint64_t k, uint32_t i, bool &found) {
+    const int lane = threadIdx.x & 63;
+    int below = 0, equal = 0;
+    for (int t0 = 0; t0 < count; t0 += 256) {   // (t < MAX_WS: what lies behind the list is read but not counted)
+        uint64_t kt[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) kt[u] = key[t0 + u * 64 + lane];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const bool in = t0 + u * 64 + lane < count;
+            below += __popcll(__ballot(in && kt[u] < k));
+            equal += __popcll(__ballot(in && kt[u] == k));
+        }
+    }
+    found = OWN;
+    if (equal > (OWN ? 1 : 0))   // equal values of f: the index decides
+        for (int t = lane; t - lane < count; t += 64) {
+            const uint64_t kt = key[t];
+            const uint32_t it = idx[t];
+            below += __popcll(__ballot(t < count && kt == k && it < i));
+            found |= __ballot(t < count && kt == k && it == i) != 0;
+        }
+    return below;
+}
+
+// (fold_n > 0: the ids are also written modulo fold_n to out_folded, for problems whose instances are stacked
+// copies of fold_n stored rows)
+template <int NS>   // NS = g.n_sides
+__global__ __launch_bounds__(SEL_RANK_T) void sel_final_kernel(SelWorkspace w, int64_t n, SelGeom g, int p_full,
+                                                               int *__restrict__ out, int fold_n, int *__restrict__ out_folded) {
+    // a side's list and its paired side's; on the slow path every side's, and the histograms before that
+    __shared__ union {
+        struct { uint64_t key[NS][MAX_WS]; uint32_t idx[NS][MAX_WS]; } list;
+        uint32_t hist[NS][SEL_BINS];
+    } sh;
+    __shared__ int cnt[SEL_MAX_SIDES];
+    __shared__ int conflict, last, event[NS / 2], alone_in[NS][MAX_WS / 64];
+    __shared__ SelState st[SEL_MAX_SIDES];
+    __shared__ uint32_t scratch[SEL_T + 16];
+    static_assert(SEL_RANK_T == MAX_WS, "one thread per entry in the scan");
+    constexpr int half = NS / 2;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int s_own = (int) blockIdx.x / (MAX_WS / SEL_RANK_ENTRIES), s_paired = s_own < half ? s_own + half : s_own - half;
+    // (the lists are read before it is known how long they are, and whether they are there at all: one latency for everything)
+    uint64_t key[2] = {w.list_key[s_own * MAX_WS + tid], w.list_key[s_paired * MAX_WS + tid]};
+    uint32_t idx[2] = {w.list_idx[s_own * MAX_WS + tid], w.list_idx[s_paired * MAX_WS + tid]};
+    if (tid < NS) {
+        st[tid] = w.state[p_full * SEL_MAX_SIDES + tid];
+        cnt[tid] = (int) w.count[tid];
+    }
+    sel_clear_hist(w, p_full, (int64_t) blockIdx.x * SEL_RANK_T + tid, (int64_t) gridDim.x * SEL_RANK_T);
+    if (tid == 0) conflict = 0;
     __syncthreads();
+    int si[NS], pos_other[NS];   // entry `tid` of every side's list in order: instance, its place in the paired side's list or -1
+    if (sel_undecided(g, st)) {   // (sel_compact_kernel has left the lists empty)
+        if (blockIdx.x != 0) return;
+        sel_tail(w, n, g, p_full, st, sh.hist, scratch);
+        // (counted with atomics by this workgroup itself: an atomic read)
+        if (tid < NS) cnt[tid] = imin_sel((int) __hip_atomic_load(&w.count[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), MAX_WS);
+        __syncthreads();
+        sel_sort_here<NS>(w, g, cnt, sh.list.key, sh.list.idx, si, pos_other);
+    } else {
+        if (tid < NS) cnt[tid] = imin_sel(cnt[tid], MAX_WS);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            sh.list.key[h][tid] = key[h];
+            sh.list.idx[h][tid] = idx[h];
+        }
+        __syncthreads();
+        for (int each = 0; each < SEL_RANK_EACH; ++each) {
+            const int e = (int) blockIdx.x % (MAX_WS / SEL_RANK_ENTRIES) * SEL_RANK_ENTRIES + each * (SEL_RANK_T / 64) + wave;
+            if (e >= cnt[s_own]) break;
+            const uint64_t k = sh.list.key[0][e];
+            const uint32_t i = sh.list.idx[0][e];
+            bool found;
+            const int at = sel_place<true>(sh.list.key[0], sh.list.idx[0], cnt[s_own], k, i, found);
+            // (the paired side reads the order from the other end: it holds the complements of key and index)
+            const int there = sel_place<false>(sh.list.key[1], sh.list.idx[1], cnt[s_paired], ~k, g.idx_mask - i, found);
+            if (lane == 0) w.sorted[s_own * MAX_WS + at] = make_int2((int) (sel_side_descending(s_own, NS) ? g.idx_mask - i : i), found ? there : -1);
+        }
+        // (every wavefront's entry is in the L2 before thread 0 publishes them for the others)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (tid == 0) last = __hip_atomic_fetch_add(&w.count[SEL_MAX_SIDES], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+        __syncthreads();
+        if (!last) return;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            const int2 v = tid < cnt[s] ? w.sorted[s * MAX_WS + tid] : make_int2(-1, -1);
+            si[s] = v.x;
+            pos_other[s] = v.y;
+        }
+    }
+    if (tid <= SEL_MAX_SIDES) w.count[tid] = 0;
     const int k = (int) g.k;
     // fast path: round r takes entry r of every side, provided no entry is already consumed by its pair
-    const int per = k / g.n_sides;
-    bool ok = (k % g.n_sides) == 0;
-    for (int s = 0; s < g.n_sides; ++s) ok = ok && cnt[s] >= per;
+    const int per = k / NS;
+    bool ok = (k % NS) == 0;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) ok = ok && cnt[s] >= per;
     if (ok && tid < per) {
-        for (int s = 0; s < g.n_sides; ++s) {
-            const int po = pos_other[s][tid];
-            if (po < 0) continue;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
             // the paired side has consumed `tid` entries before this pick if it runs later in the round,
             // `tid + 1` if it runs earlier
-            const int o = s < half ? s + half : s - half;
-            const int consumed = o < s ? tid + 1 : tid;
-            if (po < consumed) atomicOr(&conflict, 1);
+            const int consumed = s >= half ? tid + 1 : tid;
+            if (pos_other[s] >= 0 && pos_other[s] < consumed) atomicOr(&conflict, 1);
         }
     }
     __syncthreads();
     if (ok && !conflict) {
         if (tid < per)
-            for (int s = 0; s < g.n_sides; ++s) {
-                const int id = (int) si[s][tid];
-                out[tid * g.n_sides + s] = id;
-                if (fold_n > 0) out_folded[tid * g.n_sides + s] = id % fold_n;
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                out[tid * NS + s] = si[s];
+                if (fold_n > 0) out_folded[tid * NS + s] = si[s] % fold_n;
             }
         return;
     }
@@ -760,14 +849,13 @@ __global__ __launch_bounds__(MAX_WS) void sel_final_kernel(SelWorkspace w, int64
     // the other side has taken, or the end of a list.  By then every instance that is in both lists has been taken
     // (those in front of the event's entry by one side, those behind it by the other), so from there on a side goes
     // on with the entries that are in its list alone.  What remains are prefix counts.  Replayed by one thread the scan took
-    // 0.2 us per pick: 5,001 instances with four sides took 156 us, 49 in this form.
-    const int lane = tid & 63, wave = tid >> 6;
+    // 0.2 us per pick.
     // the turn of side s in round r is number 2 r + (is it a low side?) of its pair
     if (tid < half) event[tid] = 2 * cnt[tid] < 2 * cnt[tid + half] + 1 ? 2 * cnt[tid] : 2 * cnt[tid + half] + 1;
     __syncthreads();
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        const int po = pos_other[s][tid], low = s < half ? 0 : 1;
+        const int po = pos_other[s], low = s < half ? 0 : 1;
         if (po >= 0 && po < tid + low) atomicMin(&event[s - low * half], 2 * tid + low);
     }
     __syncthreads();
@@ -775,7 +863,7 @@ __global__ __launch_bounds__(MAX_WS) void sel_final_kernel(SelWorkspace w, int64
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
         first[s] = s < half ? (event[s] + 1) >> 1 : event[s - half] >> 1;   // picks before the event
-        const bool alone = tid >= first[s] && tid < cnt[s] && pos_other[s][tid] < 0;
+        const bool alone = tid >= first[s] && tid < cnt[s] && pos_other[s] < 0;
         const uint64_t b = __ballot(alone);
         nth[s] = alone ? first[s] + __popcll(b & ((1ull << lane) - 1ull)) : -1;
         if (lane == 0) alone_in[s][wave] = __popcll(b);
@@ -800,7 +888,7 @@ __global__ __launch_bounds__(MAX_WS) void sel_final_kernel(SelWorkspace w, int64
 #pragma unroll
         for (int o = 0; o < NS; ++o) at += (len[o] < nth[s] ? len[o] : nth[s]) + (o < s && len[o] > nth[s] ? 1 : 0);
         if (at < k) {
-            const int id = (int) si[s][tid];
+            const int id = si[s];
             out[at] = id;
             if (fold_n > 0) out_folded[at] = id % fold_n;
         }
@@ -906,7 +994,7 @@ static int select_working_set(const double *f, const int *y, const double *alpha
     unsigned grid = (unsigned) std::min<int64_t>((n + SEL_T - 1) / SEL_T, 496);
     if ((n + grid - 1) / grid > SEL_CHUNK_MAX) grid = (unsigned) ((n + SEL_CHUNK_MAX - 1) / SEL_CHUNK_MAX);
     if (!armed) {
-        hipLaunchKernelGGL(sel_init_kernel, dim3(p_full * SEL_MAX_SIDES * SEL_BINS / 1024), dim3(256), 0, s, w, g, p_full);
+        hipLaunchKernelGGL(sel_init_kernel, dim3(p_full * SEL_MAX_SIDES * SEL_BINS / 1024), dim3(256), 0, s, w, p_full);
         TSVM_LAUNCH_CHECK();
     }
     for (int p = first_pass; p < p_full; ++p) {
@@ -916,8 +1004,8 @@ static int select_working_set(const double *f, const int *y, const double *alpha
     }
     hipLaunchKernelGGL(sel_compact_kernel, dim3(grid), dim3(SEL_T), 0, s, w, n, g, p_full);
     TSVM_LAUNCH_CHECK();
-    if (nu) hipLaunchKernelGGL(sel_final_kernel<4>, dim3(1), dim3(MAX_WS), 0, s, w, n, g, p_full, out, fold_n, out_folded);
-    else hipLaunchKernelGGL(sel_final_kernel<2>, dim3(1), dim3(MAX_WS), 0, s, w, n, g, p_full, out, fold_n, out_folded);
+    if (nu) hipLaunchKernelGGL(sel_final_kernel<4>, dim3(4 * MAX_WS / SEL_RANK_ENTRIES), dim3(SEL_RANK_T), 0, s, w, n, g, p_full, out, fold_n, out_folded);
+    else hipLaunchKernelGGL(sel_final_kernel<2>, dim3(2 * MAX_WS / SEL_RANK_ENTRIES), dim3(SEL_RANK_T), 0, s, w, n, g, p_full, out, fold_n, out_folded);
     TSVM_LAUNCH_CHECK();
     return 0;
 }
