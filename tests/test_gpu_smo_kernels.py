@@ -46,6 +46,34 @@ def test_update_f(n, ws, zero_frac, row_type):
     assert np.array_equal(G.host(f_d), want)
 
 
+@pytest.mark.parametrize("n,ld_pad,shift", [(63, 1, 0), (64, 0, 0), (16384, 0, 0), (16385, 3, 0), (16385, 2, 1), (32768, 0, 0), (32769, 3, 0),
+                                            (32769, 3, 2), (65537, 7, 0), (100003, 0, 0), (262143, 1, 0)])
+@pytest.mark.parametrize("ws,rows,repeat", [(1024, 1024, 1), (1024, 257, 2), (1030, 31, 5), (513, 16, 9), (64, 33, 1), (40, 0, 1)])
+@pytest.mark.parametrize("row_type", [capi.ROW_F64, capi.ROW_F32])
+def test_update_f_below_262144_columns(n, ld_pad, shift, ws, rows, repeat, row_type):
+    """The kernel whose wavefronts take the rows in turn: one, two and four columns per thread (and one where a row's start is not
+    aligned: `shift` elements off), a last group of rows that is full, short or missing, ragged columns, more copies than wavefronts."""
+    if n > 40000 and (rows > 40 or repeat > 2):
+        rows, ws, repeat = min(rows, 40), 64, min(repeat, 2)
+    rng = np.random.default_rng(n + ws + rows)
+    ld = n + ld_pad
+    store = 70
+    dt = np.float32 if row_type == capi.ROW_F32 else np.float64
+    k_all = rng.random(shift + store * ld).astype(dt)
+    k64 = k_all[shift:].reshape(store, ld)[:, :n].astype(np.float64)
+    slots = rng.integers(0, store, size=ws).astype(np.int32)
+    ad = np.zeros(ws)
+    ad[rng.permutation(ws)[:rows]] = rng.standard_normal(rows)
+    f = rng.standard_normal(n * repeat)
+    # (the oracle's update on the distinct non-zero rows, in their order, copy by copy)
+    at = np.flatnonzero(ad)
+    want = np.concatenate([O.update_f(f[r * n:(r + 1) * n], ad[at], np.ascontiguousarray(k64[slots[at]]), n) if rows else f[r * n:(r + 1) * n]
+                           for r in range(repeat)])
+    f_d, ad_d, k_d, s_d = G.dev(f), G.dev(ad), G.dev(k_all), G.dev(slots)
+    capi.call("tsvm_update_f", G.ptr(f_d), G.ptr(ad_d), ws, G.ptr(k_d) + shift * k_all.itemsize, row_type, G.ptr(s_d), ld, n, repeat, G.stream())
+    assert np.array_equal(G.host(f_d), want)
+
+
 @pytest.mark.parametrize("n,ws,ld_pad", [(300001, 64, 7), (262144, 33, 0), (270000, 40, 4)])
 @pytest.mark.parametrize("row_type", [capi.ROW_F64, capi.ROW_F32])
 def test_update_f_wide_and_repeated(n, ws, ld_pad, row_type):
@@ -547,7 +575,7 @@ def test_selection_with_folded_ids(n, tie_mode, nu):
 
 @pytest.mark.parametrize("nu", [0, 1])
 @pytest.mark.parametrize("row_type", [capi.ROW_F64, capi.ROW_F32])
-@pytest.mark.parametrize("n_cols,repeat,ws,ld_pad,tie_mode", [(1, 1, 1, 0, 0), (700, 1, 512, 3, 0), (4099, 2, 64, 1, 2),
+@pytest.mark.parametrize("n_cols,repeat,ws,ld_pad,tie_mode", [(1, 1, 1, 0, 0), (700, 1, 512, 3, 0), (4099, 2, 64, 1, 2), (16385, 1, 300, 1, 0), (32771, 4, 100, 1, 2),
                                                              (300001, 1, 1024, 7, 0), (270000, 2, 200, 0, 0),
                                                              (262144, 1, 1024, 0, 1), (150000, 3, 16, 4, 2)])
 def test_update_f_with_the_next_selection(n_cols, repeat, ws, ld_pad, tie_mode, row_type, nu):

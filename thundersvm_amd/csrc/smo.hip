@@ -264,6 +264,7 @@ struct SelFuse {
 // update_f: f[j] -= sum_t alpha_diff[t] * K_t[j]  (smo_kernel.cpp:300-319)
 // Bandwidth-bound stream over the ws x n kernel rows.  The non-zero alpha_diff entries are
 // compacted (in order) into LDS once per workgroup; rows with alpha_diff == 0 are never read.
+// This kernel is for 262,144 columns and more (update_f_narrow_kernel below for fewer).
 // Each thread owns one to four adjacent columns and keeps 8 to 32 row loads in flight.  On the vector-load
 // path the columns are dealt evenly to a number of workgroups that is a multiple of 248 (every CU, or every
 // CU left to a stream that leaves one CU per XCD to the local solver, gets the same number of workgroups):
@@ -432,6 +433,172 @@ __global__ __launch_bounds__(UF_T) void update_f_kernel(double *__restrict__ f, 
     }
     __syncthreads();
     for (int e = tid; e < NS * SEL_BINS; e += UF_T) {
+        const uint32_t c = (&lhist[0][0])[e];
+        if (c) atomicAdd(&sf.w.hist[e], c);   // hist[0][s][bin], s < NS
+    }
+}
+
+// The same for fewer than 262,144 columns.  One thread per column leaves most of the chip without work then, and a column's some 500
+// rows come in sixteen batches one memory latency apart: 27 us for 3,200 columns and 31 for 40,000.  Here a workgroup has
+// 64 * COLS columns and eight wavefronts; groups of R neighbouring rows are dealt to them in turn, so that all eight have theirs on
+// their way at once, and they add them in turn: the sums of a column stay one chain in the rows' order, handed on through
+// LDS.  Bound by that chain (500 additions and the hand-overs, some 3 us) and the compaction in front of it where columns are few, by
+// HBM where they are many.
+#define UN_WAVES 8
+// (a barrier that waits for LDS only: rows stay on their way across it)
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+template <typename TK, int COLS, int R, int NS>
+__global__ __launch_bounds__(64 * UN_WAVES, 4) void update_f_narrow_kernel(double *__restrict__ f, const double *__restrict__ alpha_diff,
+                                                                        int ws, const TK *__restrict__ k_rows,
+                                                                        const int *__restrict__ slots, int64_t ld, int64_t n, int repeat, SelFuse sf) {
+    typedef TK vec_t __attribute__((ext_vector_type(COLS)));
+    constexpr int T = 64 * UN_WAVES, EACH = UF_CHUNK / T;
+    __shared__ uint32_t lhist[NS > 0 ? NS : 1][NS > 0 ? SEL_BINS : 1];
+    __shared__ uint32_t mark_bits[NS > 0 ? UF_MAX_REPEAT : 1][2 * COLS];
+    __shared__ double s_ad[UF_CHUNK];
+    __shared__ int64_t s_off[UF_CHUNK];
+    __shared__ double s_sum[COLS][64];
+    __shared__ int s_wave_cnt[UN_WAVES];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t col_lo = (int64_t) blockIdx.x * 64 * COLS, j = col_lo + lane * COLS;
+    const int64_t jc = j < n ? j : (n - 1) / COLS * COLS;   // (a lane behind the last column reads that column's vector)
+    // what the epilogue needs of this wavefront's copy of the columns: on its way from here on
+    double fo[COLS], al[COLS];
+    int yv[COLS];
+    auto fetch = [&](int r) {
+#pragma unroll
+        for (int c = 0; c < COLS; ++c) {
+            const int64_t at = (int64_t) r * n + (j + c < n ? j + c : n - 1);
+            fo[c] = f[at];
+            if (NS > 0) {
+                al[c] = sf.alpha[at];
+                yv[c] = sf.y[at];
+            }
+        }
+    };
+    if (wave < repeat) fetch(wave);
+    if (NS > 0) {
+        for (int e = tid; e < NS * SEL_BINS; e += T) (&lhist[0][0])[e] = 0;
+        if (tid < UF_MAX_REPEAT * 2 * COLS) (&mark_bits[0][0])[tid] = 0;
+        if (blockIdx.x == 0 && tid < NS) {
+            SelState s0;
+            s0.pk = 0; s0.pi = 0; s0.k_rem = sf.g.k; s0.done = 0; s0.pad = 0;
+            sf.w.state[tid] = s0;   // the state before digit 0, for the next pass
+        }
+        __syncthreads();
+        for (int i = tid; i < sf.n_marked; i += T) {
+            const int64_t id = sf.marked[i];
+            for (int r = 0; r < repeat; ++r) {
+                const int64_t c = id - r * n;   // column, if the id lies in copy r
+                if (c >= col_lo && c < col_lo + 64 * COLS && c < n) atomicOr(&mark_bits[r][(c - col_lo) >> 5], 1u << ((c - col_lo) & 31));
+            }
+        }
+    }
+    double sum[COLS];
+#pragma unroll
+    for (int c = 0; c < COLS; ++c) sum[c] = 0.0;
+    for (int base = 0; base < ws; base += UF_CHUNK) {
+        // ordered compaction of this chunk's non-zero entries, EACH neighbouring ones per thread
+        double v[EACH];
+        int cnt = 0;
+#pragma unroll
+        for (int e = 0; e < EACH; ++e) {
+            const int t = base + tid * EACH + e;
+            v[e] = t < ws ? alpha_diff[t] : 0.0;
+            cnt += (v[e] != 0.0);
+        }
+        int incl = cnt;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(incl, d, 64);
+            if (lane >= d) incl += o;
+        }
+        if (lane == 63) s_wave_cnt[wave] = incl;
+        __syncthreads();
+        int pos = incl - cnt, total = 0;
+#pragma unroll
+        for (int w = 0; w < UN_WAVES; ++w) {
+            if (w < wave) pos += s_wave_cnt[w];
+            total += s_wave_cnt[w];
+        }
+#pragma unroll
+        for (int e = 0; e < EACH; ++e)
+            if (v[e] != 0.0) {
+                const int t = base + tid * EACH + e;
+                s_ad[pos] = v[e];
+                s_off[pos] = (int64_t) (slots ? slots[t] : t) * ld;
+                ++pos;
+            }
+        __syncthreads();
+        // Groups of R rows are dealt to the wavefronts in turn: group g is wavefront g % UN_WAVES's, which asks for its next one as
+        // soon as it has added the last.
+        const int groups = (total + R - 1) / R;
+        vec_t k[R];
+        auto request = [&](int g) {
+#pragma unroll
+            for (int u = 0; u < R; ++u) k[u] = load_streaming((const vec_t *) (k_rows + s_off[g * R + u < total ? g * R + u : total - 1] + jc));
+        };
+        if (wave < groups) request(wave);
+        for (int g = 0; g < groups; ++g) {
+            if (wave == g % UN_WAVES) {
+                if (g > 0) {   // the sums so far come from the wavefront before
+#pragma unroll
+                    for (int c = 0; c < COLS; ++c) sum[c] = s_sum[c][lane];
+                }
+                const int m = total - g * R;
+                if (m >= R) {
+#pragma unroll
+                    for (int u = 0; u < R; ++u)
+#pragma unroll
+                        for (int c = 0; c < COLS; ++c) sum[c] = __builtin_fma(s_ad[g * R + u], (double) k[u][c], sum[c]);
+                } else {
+#pragma unroll
+                    for (int u = 0; u < R; ++u)
+                        if (u < m)
+#pragma unroll
+                            for (int c = 0; c < COLS; ++c) sum[c] = __builtin_fma(s_ad[g * R + u], (double) k[u][c], sum[c]);
+                }
+#pragma unroll
+                for (int c = 0; c < COLS; ++c) s_sum[c][lane] = sum[c];
+            }
+            lds_barrier();
+            if (wave == g % UN_WAVES && g + UN_WAVES < groups) request(g + UN_WAVES);
+        }
+        if (total > 0) {   // every wavefront goes on from the chunk's sums
+#pragma unroll
+            for (int c = 0; c < COLS; ++c) sum[c] = s_sum[c][lane];
+            __syncthreads();
+        }
+    }
+    if (NS > 0 && ws <= 0) __syncthreads();   // (the marks)
+    for (int r = wave; r < repeat; r += UN_WAVES) {
+        if (r != wave) fetch(r);
+        const int64_t j0 = (int64_t) r * n + j;
+#pragma unroll
+        for (int c = 0; c < COLS; ++c) {
+            const bool in = j + c < n;
+            const double fn = fo[c] - sum[c];
+            if (in) f[j0 + c] = fn;
+            if constexpr (NS > 0) {
+                const uint64_t key = f_to_key(fn);
+                const int bit = lane * COLS + c;
+                uint32_t fl = 0;
+                if (in && !((mark_bits[r][bit >> 5] >> (bit & 31)) & 1u)) fl = sel_flags(al[c], (double) yv[c], sf.Cp, sf.Cn, NS);
+                if (in) {
+                    sf.w.keys[j0 + c] = key;
+                    sf.w.flags[j0 + c] = (uint8_t) fl;
+                }
+#pragma unroll
+                for (int s = 0; s < NS; ++s) {
+                    const uint64_t k2 = sel_side_descending(s, NS) ? ~key : key;
+                    sel_hist_add_wave(lhist[s], (fl >> s) & 1u, (uint32_t) (k2 >> (64 - SEL_DIGIT)));   // digit 0: the key's top bits
+                }
+            }
+        }
+    }
+    if (NS == 0) return;
+    __syncthreads();
+    for (int e = tid; e < NS * SEL_BINS; e += T) {
         const uint32_t c = (&lhist[0][0])[e];
         if (c) atomicAdd(&sf.w.hist[e], c);   // hist[0][s][bin], s < NS
     }
@@ -936,14 +1103,40 @@ static void launch_update_f(double *f, const double *alpha_diff, int ws_size, co
                        (const TK *) k_rows, slots, ld, n, repeat, vec_per_wg, sf);
 }
 
+template <typename TK, int COLS, int R, int NS>
+static void launch_update_f_narrow(double *f, const double *alpha_diff, int ws_size, const void *k_rows, const int *slots,
+                                   int64_t ld, int64_t n, int repeat, const SelFuse &sf, hipStream_t s) {
+    hipLaunchKernelGGL((update_f_narrow_kernel<TK, COLS, R, NS>), dim3((unsigned) ((n + 64 * COLS - 1) / (64 * COLS))), dim3(64 * UN_WAVES), 0, s,
+                       f, alpha_diff, ws_size, (const TK *) k_rows, slots, ld, n, repeat, sf);
+}
+
 // The variant of the kernel for the row type, alignment and size at hand.
 template <int NS>
 static void dispatch_update_f(double *f, const double *alpha_diff, int ws_size, const void *k_rows, int row_type, const int *slots,
                               int64_t ld, int64_t n, int repeat, const SelFuse &sf, hipStream_t s) {
-    // 16-byte loads need every row start 16-byte aligned and the last vector inside the padded row; with few
-    // columns one column per thread and more rows in flight keeps more of the chip busy
+    // vector loads need every row start aligned to the vector and the last vector inside the padded row
     const bool big = n >= (int64_t) UF_T * 1024;
     const bool aligned = (uintptr_t) k_rows % 16 == 0;
+    if (!big) {
+        // As few columns per thread as make do with one workgroup per CU (more workgroups than that leave some CUs two in
+        // turn), beyond 65,536 columns four floats or one double.  500 of 1,024 rows, us a call, one thread per column / here with
+        // 1, 2, 4 floats (1, 2 doubles) per thread:
+        //   floats   3,200: 26.7 / 12.7 15.1 18.6   20,000: 30.7 / 16.9 15.7 19.0   40,000: 31.5 / 26.6 21.5 19.8
+        //           60,000: 34.0 / 32.8 24.3 24.5  120,000: 46.7 / 59.6 45.0 43.2  255,000: 100 / 128 99.6 90.3 (5.6 TB/s)
+        //   doubles  3,200: 32.6 / 14.9 15.3        18,000: 35.7 / 20.0 16.7        40,000: 38.7 / 31.0 34.2
+        //           90,000: 67.0 / 60.5 63.7       200,000: 142 / 127 131 (6.3 TB/s)
+        auto fits = [&](int cols, size_t esz) { return (uintptr_t) k_rows % (cols * esz) == 0 && ld % cols == 0 && n <= (int64_t) 64 * cols * 256; };
+        if (row_type == TSVM_ROW_F32) {
+            if (fits(1, 4)) launch_update_f_narrow<float, 1, 32, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
+            else if (fits(2, 4)) launch_update_f_narrow<float, 2, 16, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
+            else if (aligned && ld % 4 == 0) launch_update_f_narrow<float, 4, 16, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
+            else launch_update_f_narrow<float, 1, 32, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
+        } else {
+            if (!fits(1, 8) && fits(2, 8)) launch_update_f_narrow<double, 2, 16, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
+            else launch_update_f_narrow<double, 1, 16, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
+        }
+        return;
+    }
     if (row_type == TSVM_ROW_F32) {
         if (big && aligned && ld % 4 == 0 && ld >= (n + 3) / 4 * 4) launch_update_f<float, 4, 8, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
         else launch_update_f<float, 1, 32, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
