@@ -365,6 +365,14 @@ int tsvm_select_working_set_folded(const double *f, const int *y, const double *
                                    const int *marked, int n_marked, int *out, int n_select, int nu, void *workspace,
                                    int again, int fold_n, int *out_folded, tsvm_stream stream);
 
+/* The same (fold_n == 0: no folded ids) whose last kernel also writes the ids to host_ids[0..n_select), pinned host memory that
+ * the device can write, and then, behind a system-wide fence, `word` to host_ids[word_at] (word_at >= n_select), which the
+ * host polls: the selection and tsvm_report_ids of its ids in one. */
+int tsvm_select_working_set_report(const double *f, const int *y, const double *alpha, int64_t n, double Cp, double Cn,
+                                   const int *marked, int n_marked, int *out, int n_select, int nu, void *workspace,
+                                   int again, int fold_n, int *out_folded, int *host_ids, int word_at, int word,
+                                   tsvm_stream stream);
+
 /* tsvm_update_f followed by the selection of the next working set on the updated f, in one call: what
  * CSMOSolver::solve does at the end of one outer iteration and the start of the next (csmosolver.cpp:63-77,115-117).
  * The result is that of tsvm_update_f(f, alpha_diff, ws_size, k_rows, row_type, slots, ld, n_cols, repeat) and then
@@ -377,6 +385,12 @@ int tsvm_update_f_select(double *f, const double *alpha_diff, int ws_size, const
                          int64_t ld, int64_t n_cols, int repeat, const int *y, const double *alpha, double Cp, double Cn,
                          const int *marked, int n_marked, int *out, int n_select, int nu, void *workspace, int *out_folded,
                          tsvm_stream stream);
+
+/* The same with the report of tsvm_select_working_set_report. */
+int tsvm_update_f_select_report(double *f, const double *alpha_diff, int ws_size, const void *k_rows, int row_type, const int *slots,
+                                int64_t ld, int64_t n_cols, int repeat, const int *y, const double *alpha, double Cp, double Cn,
+                                const int *marked, int n_marked, int *out, int n_select, int nu, void *workspace, int *out_folded,
+                                int *host_ids, int word_at, int word, tsvm_stream stream);
 
 /* ---------------------------------------------------------------------------------------------
  * predict (kernelmatrix_kernel.cpp:110-147)

@@ -671,3 +671,42 @@ def test_report_ids_to_host_memory():
         assert np.array_equal(got[:n_ids], want) and got[1024] == word
     with pytest.raises(capi.TsvmError):
         capi.call("tsvm_report_ids", G.ptr(ids_d), 600, 0, host.data_ptr(), 512, 1, G.stream())      # the word would lie inside the ids
+
+
+@pytest.mark.parametrize("nu", [0, 1])
+@pytest.mark.parametrize("n,tie_mode,fold", [(150, 0, 0), (5001, 2, 0), (5000, 0, 2500), (70000, 1, 35000)])
+def test_selections_that_report_their_ids(n, tie_mode, fold, nu):
+    """The selection whose last kernel tells the host: the same ids in device memory, folded and in host memory, and the word behind
+    them, on the counting path, the one-workgroup path (ties) and where a side runs dry; alone and behind update_f."""
+    ws = min(1024, 1 << (n.bit_length() - 1))
+    q = ws // 2
+    rng = np.random.default_rng(n)
+    cols = fold if fold else n
+    wsp = torch.empty(capi.kernel_lib().tsvm_select_workspace(n), dtype=torch.uint8, device="cuda")
+    host = torch.full((ws + 16,), -7, dtype=torch.int32).pin_memory()
+    f, y, alpha, C, _ = _select_case(n, q, 0, 11 * n, tie_mode, nu)
+    f_d, y_d, a_d = G.dev(f), G.dev(y), G.dev(alpha)
+    out_d = torch.full((ws,), -7, dtype=torch.int32, device="cuda")
+    fold_d = torch.full((ws,), -7, dtype=torch.int32, device="cuda")
+    capi.call("tsvm_select_working_set_report", G.ptr(f_d), G.ptr(y_d), G.ptr(a_d), n, C, C, None, 0, G.ptr(out_d), ws, nu, G.ptr(wsp), 0, fold,
+              G.ptr(fold_d) if fold else None, host.data_ptr(), ws, 41, G.stream())
+    want = O.select_working_set(f, y, alpha, C, C, np.zeros(0, dtype=np.int32), ws, nu=bool(nu))
+    torch.cuda.synchronize()
+    assert np.array_equal(G.host(out_d), want) and np.array_equal(host.numpy()[:ws], want) and host.numpy()[ws] == 41
+    if fold:
+        assert np.array_equal(G.host(fold_d), np.where(want >= 0, want % fold, -1))
+    marked = np.ascontiguousarray(want[q:][want[q:] >= 0])
+    k = rng.random((32, cols)).astype(np.float32)
+    ad = np.zeros(32) if tie_mode else rng.standard_normal(32)
+    k64 = k.astype(np.float64)
+    f = O.update_f(f, ad, np.ascontiguousarray(np.concatenate([k64, k64], axis=1) if fold else k64), n)
+    want = O.select_working_set(f, y, alpha, C, C, marked, q, nu=bool(nu))
+    ad_d, k_d, m_d = G.dev(ad), G.dev(k), G.dev(marked)
+    capi.call("tsvm_update_f_select_report", G.ptr(f_d), G.ptr(ad_d), 32, G.ptr(k_d), capi.ROW_F32, None, cols, cols, n // cols, G.ptr(y_d), G.ptr(a_d),
+              C, C, G.ptr(m_d), len(marked), G.ptr(out_d), q, nu, G.ptr(wsp), G.ptr(fold_d) if fold else None, host.data_ptr(), ws, 42, G.stream())
+    torch.cuda.synchronize()
+    assert np.array_equal(G.host(f_d), f)
+    assert np.array_equal(G.host(out_d)[:q], want) and np.array_equal(host.numpy()[:q], want) and host.numpy()[ws] == 42
+    with pytest.raises(capi.TsvmError):   # the word would lie inside the ids
+        capi.call("tsvm_select_working_set_report", G.ptr(f_d), G.ptr(y_d), G.ptr(a_d), n, C, C, None, 0, G.ptr(out_d), ws, nu, G.ptr(wsp), 0, 0, None,
+                  host.data_ptr(), ws - 1, 1, G.stream())

@@ -182,9 +182,8 @@ struct SolveTask::Impl {
     // working set as folded ids: a second window, at the same offsets, that the selection fills along with the first
     const int *ws_u() const { return rep > 1 ? d_ws_folded.data() + ws_off : d_ws.data() + ws_off; }
 
-    // The chip-wide work of a task is enqueued on stream `sa` (`ids` is the stream the newly selected ids are read
-    // back on for the host-side cache bookkeeping: the same one).
-    hipStream_t sa = nullptr, ids = nullptr;
+    // The chip-wide work of a task is enqueued on stream `sa`.
+    hipStream_t sa = nullptr;
     tsvm::DeviceEvent selected, diff_ready;
     // A task that runs alone splits the chip: the local solver (one workgroup, a chain of dependent steps) gets a
     // stream `ss` restricted to one CU of every XCD, everything else runs on `sa`, restricted to the other CUs.
@@ -281,11 +280,11 @@ struct SolveTask::Impl {
         }
         return false;
     }
-    // The new ids come to the host from the device itself (tsvm_report_ids, in stream order behind the selection):
+    // The new ids come to the host from the selection's last kernel:
     // h_ids[ws_size] takes the number of the report once its ids are in h_ids.
     int ids_seq = 0;
     bool ids_arrived() const {
-        if (!(caching && !all_cached && !device_cache)) return true;
+        if (!ids_to_host()) return true;
         if (*(volatile int *) (h_ids + ws_size) != ids_seq) return false;
         __atomic_thread_fence(__ATOMIC_ACQUIRE);
         return true;
@@ -299,7 +298,7 @@ struct SolveTask::Impl {
             const auto now = clock::now();
             if (now < next_check) continue;
             next_check = now + std::chrono::milliseconds(200);
-            const hipError_t e = hipStreamQuery(ids);
+            const hipError_t e = hipStreamQuery(sa);
             if (e == hipSuccess) {
                 if (!ids_arrived()) {
                     abandoned = true;
@@ -364,9 +363,6 @@ struct SolveTask::Impl {
             TSVM_HIP_CHECK(hipStreamCreateWithFlags(&sa, hipStreamNonBlocking));
             ss = sa;
         }
-        // The read-back of the newly selected ids follows the selection on the same stream: it is enqueued before
-        // anything else of the iteration, so it waits for nothing but the selection.
-        ids = sa;
         selected = tsvm::take_event();
         diff_ready = tsvm::take_event();
         block_done = tsvm::take_event();
@@ -550,6 +546,9 @@ struct SolveTask::Impl {
         sel_off = next;
     }
 
+    // Whether the host has to hear of the next selection's ids (its row cache needs them): the selection itself tells it.
+    bool ids_to_host() const { return caching && !all_cached && !device_cache; }
+
     void launch_select(int it) {
         const int n_sel = it == 0 ? ws_size : q;
         hipStream_t sel = sa;
@@ -557,10 +556,13 @@ struct SolveTask::Impl {
         else advance_window();
         const int *kept = it == 0 ? nullptr : d_ws.data() + sel_off;            // the half that stays: no candidates
         int *out = d_ws.data() + sel_off + (it == 0 ? 0 : q);
-        if (rep > 1) {
+        int *folded = rep > 1 ? d_ws_folded.data() + sel_off + (it == 0 ? 0 : q) : nullptr;
+        if (ids_to_host()) {
+            abi_check(tsvm_select_working_set_report(d_f, d_y, d_alpha, n, Cp, Cn, kept, it == 0 ? 0 : q, out, n_sel, nu, d_sel_ws.data(),
+                                                     it > 0, rep > 1 ? n_u : 0, folded, d_ids_host, ws_size, ++ids_seq, sel));
+        } else if (rep > 1) {
             abi_check(tsvm_select_working_set_folded(d_f, d_y, d_alpha, n, Cp, Cn, kept, it == 0 ? 0 : q, out,
-                                                     n_sel, nu, d_sel_ws.data(), it > 0, n_u,
-                                                     d_ws_folded.data() + sel_off + (it == 0 ? 0 : q), sel));
+                                                     n_sel, nu, d_sel_ws.data(), it > 0, n_u, folded, sel));
         } else if (it == 0) {
             abi_check(tsvm_select_working_set(d_f, d_y, d_alpha, n, Cp, Cn, kept, 0, out, n_sel, nu,
                                               d_sel_ws.data(), sel));
@@ -571,17 +573,11 @@ struct SolveTask::Impl {
     }
 
     void enqueue_select() {
-        const int n_new = iter == 0 ? ws_size : q;
-        const int first_new = iter == 0 ? 0 : q;
         timer.begin();
         if (!select_enqueued) launch_select(iter);
         select_enqueued = false;
         ws_off = sel_off;
         timer.end(stats.ms_select);
-        if (caching && !all_cached && !device_cache) {
-            // the new ids travel to the host: written there by a small kernel behind the selection
-            abi_check(tsvm_report_ids(ws_ids() + first_new, n_new, 0, d_ids_host, ws_size, ++ids_seq, ids));
-        }
     }
 
     void enqueue_rows() {
@@ -756,9 +752,14 @@ struct SolveTask::Impl {
         if (select_ahead && fuse_select) {
             // the next selection's first pass over the instances rides on update_f's last one
             advance_window();
-            abi_check(tsvm_update_f_select(d_f, d_alpha_diff.data(), ws_size, k_rows, row_type, slots, ld, n_u, rep,
-                                           d_y, d_alpha, Cp, Cn, d_ws.data() + sel_off, q, d_ws.data() + sel_off + q, q,
-                                           nu, d_sel_ws.data(), rep > 1 ? d_ws_folded.data() + sel_off + q : nullptr, sa));
+            int *const kept = d_ws.data() + sel_off, *const folded = rep > 1 ? d_ws_folded.data() + sel_off + q : nullptr;
+            if (ids_to_host())
+                abi_check(tsvm_update_f_select_report(d_f, d_alpha_diff.data(), ws_size, k_rows, row_type, slots, ld, n_u, rep, d_y, d_alpha,
+                                                      Cp, Cn, kept, q, kept + q, q, nu, d_sel_ws.data(), folded, d_ids_host, ws_size,
+                                                      ++ids_seq, sa));
+            else
+                abi_check(tsvm_update_f_select(d_f, d_alpha_diff.data(), ws_size, k_rows, row_type, slots, ld, n_u, rep, d_y, d_alpha, Cp,
+                                               Cn, kept, q, kept + q, q, nu, d_sel_ws.data(), folded, sa));
             select_enqueued = true;
             return;
         }
