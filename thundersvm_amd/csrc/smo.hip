@@ -33,6 +33,7 @@
 #define SEL_MAX_PASS 9
 #define SEL_MAX_SIDES 4
 #define SEL_T 256
+#define SEL_EACH 4   // instances of a thread whose loads are on their way together
 
 struct SelState {
     uint64_t pk;      // resolved high bits of the key part
@@ -152,61 +153,77 @@ __global__ void sel_init_kernel(SelWorkspace w, int p_full) {
 // it fits the side's list (MAX_WS entries), the list is a superset of the k smallest candidates, in which
 // every extra entry is larger than all of them, and sel_final_kernel sorts the list and reads it from the
 // front.  With 11-bit digits that is the normal case after the second or third pass.
-__device__ void sel_advance_state(const SelWorkspace &w, const SelGeom &g, int p, SelState *st_out /* LDS [sides] */,
-                                  uint32_t *scratch /* LDS [SEL_T + 8] */) {
+template <int NS>
+__device__ void sel_advance_state(const SelWorkspace &w, const SelGeom &g, int p, SelState *st_out /* LDS [NS] */,
+                                  uint32_t *scratch /* LDS [NS * SEL_T / 64] */) {
+    constexpr int EACH = SEL_BINS / SEL_T, WAVES = SEL_T / 64;
     const int tid = threadIdx.x;
     const bool worker = tid < SEL_T;
     const int lane = tid & 63, wave = tid >> 6;
-    for (int s = 0; s < g.n_sides; ++s) {
-        SelState st = w.state[(p - 1) * SEL_MAX_SIDES + s];
-        if (!st.done) {
-            const uint32_t *h = w.hist + ((size_t) (p - 1) * SEL_MAX_SIDES + s) * SEL_BINS;
-            uint32_t c[SEL_BINS / SEL_T];
-            uint32_t sum = 0, incl = 0;
-            if (worker) {
+    SelState st[NS];
+    uint32_t c[NS][EACH], sum[NS], incl[NS];
+    if (worker) {   // (every side's state and counts at once: one memory latency)
 #pragma unroll
-                for (int e = 0; e < SEL_BINS / SEL_T; ++e) { c[e] = h[tid * (SEL_BINS / SEL_T) + e]; sum += c[e]; }
-                incl = sum;
+        for (int s = 0; s < NS; ++s) {
+            st[s] = w.state[(p - 1) * SEL_MAX_SIDES + s];
+            const uint4 *h = (const uint4 *) (w.hist + ((size_t) (p - 1) * SEL_MAX_SIDES + s) * SEL_BINS + tid * EACH);
 #pragma unroll
-                for (int d = 1; d < 64; d <<= 1) {
-                    uint32_t o = __shfl_up(incl, d, 64);
-                    if (lane >= d) incl += o;
-                }
-                if (lane == 63) scratch[wave] = incl;
+            for (int e = 0; e < EACH / 4; ++e) {
+                const uint4 v = h[e];
+                c[s][4 * e] = v.x; c[s][4 * e + 1] = v.y; c[s][4 * e + 2] = v.z; c[s][4 * e + 3] = v.w;
             }
-            __syncthreads();
-            if (worker) {
-                uint32_t wave_base = 0, total = 0;
-                for (int wv = 0; wv < SEL_T / 64; ++wv) {
-                    if (wv < wave) wave_base += scratch[wv];
-                    total += scratch[wv];
-                }
-                const uint32_t excl = wave_base + incl - sum;
-                if (total < st.k_rem) {
-                    // fewer candidates than requested (only possible on the first digit): take them all
-                    if (tid == 0) { st.done = 1; st.k_rem = total; st_out[s] = st; }
-                } else if (excl < st.k_rem && st.k_rem <= excl + sum) {
-                    uint32_t below = excl;
-                    int b = 0;
-                    for (int e = 0; e < SEL_BINS / SEL_T; ++e) {
-                        if (below + c[e] >= st.k_rem) { b = tid * (SEL_BINS / SEL_T) + e; break; }
-                        below += c[e];
-                    }
-                    const uint32_t cb = h[b];
-                    const uint32_t taken = g.k - st.k_rem;   // entries of the buckets decided by earlier digits
-                    bool is_key; int shift, width;
-                    sel_digit_geom(p - 1, g.idx_bits, is_key, shift, width);
-                    if (is_key) st.pk |= (uint64_t) b << shift; else st.pi |= (uint32_t) b << shift;
-                    st.k_rem -= below;
-                    st.pad = (uint32_t) p;
-                    if (cb == st.k_rem || p == g.n_pass || taken + below + cb <= (uint32_t) MAX_WS) st.done = 1;
-                    st_out[s] = st;
-                }
+        }
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            sum[s] = 0;
+#pragma unroll
+            for (int e = 0; e < EACH; ++e) sum[s] += c[s][e];
+            incl[s] = sum[s];
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const uint32_t o = __shfl_up(incl[s], d, 64);
+                if (lane >= d) incl[s] += o;
             }
-            __syncthreads();
-        } else {
-            if (tid == 0) st_out[s] = st;
-            __syncthreads();
+            if (lane == 63) scratch[s * WAVES + wave] = incl[s];
+        }
+    }
+    __syncthreads();
+    if (worker) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            if (st[s].done) {
+                if (tid == 0) st_out[s] = st[s];
+                continue;
+            }
+            uint32_t excl = incl[s] - sum[s], total = 0;
+#pragma unroll
+            for (int wv = 0; wv < WAVES; ++wv) {
+                if (wv < wave) excl += scratch[s * WAVES + wv];
+                total += scratch[s * WAVES + wv];
+            }
+            if (total < st[s].k_rem) {
+                // fewer candidates than requested (only possible on the first digit): take them all
+                if (tid == 0) { st[s].done = 1; st[s].k_rem = total; st_out[s] = st[s]; }
+            } else if (excl < st[s].k_rem && st[s].k_rem <= excl + sum[s]) {
+                uint32_t below = excl, cb = 0;
+                int b = 0;
+                bool in_front = true;
+#pragma unroll
+                for (int e = 0; e < EACH; ++e) {
+                    const bool here = in_front && below + c[s][e] >= st[s].k_rem;
+                    if (here) { b = tid * EACH + e; cb = c[s][e]; }
+                    in_front = in_front && !here;
+                    if (in_front) below += c[s][e];
+                }
+                const uint32_t taken = g.k - st[s].k_rem;   // entries of the buckets decided by earlier digits
+                bool is_key; int shift, width;
+                sel_digit_geom(p - 1, g.idx_bits, is_key, shift, width);
+                if (is_key) st[s].pk |= (uint64_t) b << shift; else st[s].pi |= (uint32_t) b << shift;
+                st[s].k_rem -= below;
+                st[s].pad = (uint32_t) p;
+                if (cb == st[s].k_rem || p == g.n_pass || taken + below + cb <= (uint32_t) MAX_WS) st[s].done = 1;
+                st_out[s] = st[s];
+            }
         }
     }
     __syncthreads();
@@ -476,6 +493,20 @@ __global__ __launch_bounds__(64 * UN_WAVES, 4) void update_f_narrow_kernel(doubl
             }
         }
     };
+    // a chunk's coefficients and slots, EACH neighbouring ones per thread
+    double v[EACH];
+    int slot[EACH];
+    auto fetch_chunk = [&](int base) {
+#pragma unroll
+        for (int e = 0; e < EACH; ++e) {
+            const int t = base + tid * EACH + e, tc = t < ws ? t : ws - 1;
+            v[e] = t < ws ? alpha_diff[tc] : 0.0;
+            slot[e] = slots ? slots[tc] : tc;
+        }
+    };
+    // (everything that waits for nothing is asked for first: as four latencies one after another it took 2 us)
+    if (ws > 0) fetch_chunk(0);
+    int mark = NS > 0 && tid < sf.n_marked ? sf.marked[tid] : -1;
     if (wave < repeat) fetch(wave);
     if (NS > 0) {
         for (int e = tid; e < NS * SEL_BINS; e += T) (&lhist[0][0])[e] = 0;
@@ -487,7 +518,7 @@ __global__ __launch_bounds__(64 * UN_WAVES, 4) void update_f_narrow_kernel(doubl
         }
         __syncthreads();
         for (int i = tid; i < sf.n_marked; i += T) {
-            const int64_t id = sf.marked[i];
+            const int64_t id = i == tid ? mark : sf.marked[i];
             for (int r = 0; r < repeat; ++r) {
                 const int64_t c = id - r * n;   // column, if the id lies in copy r
                 if (c >= col_lo && c < col_lo + 64 * COLS && c < n) atomicOr(&mark_bits[r][(c - col_lo) >> 5], 1u << ((c - col_lo) & 31));
@@ -498,15 +529,11 @@ __global__ __launch_bounds__(64 * UN_WAVES, 4) void update_f_narrow_kernel(doubl
 #pragma unroll
     for (int c = 0; c < COLS; ++c) sum[c] = 0.0;
     for (int base = 0; base < ws; base += UF_CHUNK) {
-        // ordered compaction of this chunk's non-zero entries, EACH neighbouring ones per thread
-        double v[EACH];
+        // ordered compaction of this chunk's non-zero entries
+        if (base > 0) fetch_chunk(base);
         int cnt = 0;
 #pragma unroll
-        for (int e = 0; e < EACH; ++e) {
-            const int t = base + tid * EACH + e;
-            v[e] = t < ws ? alpha_diff[t] : 0.0;
-            cnt += (v[e] != 0.0);
-        }
+        for (int e = 0; e < EACH; ++e) cnt += (v[e] != 0.0);
         int incl = cnt;
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
@@ -524,9 +551,8 @@ __global__ __launch_bounds__(64 * UN_WAVES, 4) void update_f_narrow_kernel(doubl
 #pragma unroll
         for (int e = 0; e < EACH; ++e)
             if (v[e] != 0.0) {
-                const int t = base + tid * EACH + e;
                 s_ad[pos] = v[e];
-                s_off[pos] = (int64_t) (slots ? slots[t] : t) * ld;
+                s_off[pos] = (int64_t) slot[e] * ld;
                 ++pos;
             }
         __syncthreads();
@@ -680,7 +706,7 @@ __global__ __launch_bounds__(SEL_T) void sel_pass_kernel(SelWorkspace w, const d
         }
         __syncthreads();
     } else {
-        sel_advance_state(w, g, p, st, scratch);
+        sel_advance_state<NS>(w, g, p, st, scratch);
         if (blockIdx.x == 0 && tid < g.n_sides) w.state[p * SEL_MAX_SIDES + tid] = st[tid];
     }
     bool any = false;
@@ -714,10 +740,18 @@ __global__ __launch_bounds__(SEL_T) void sel_pass_kernel(SelWorkspace w, const d
     } else {
         __syncthreads();
         const int64_t stride = (int64_t) gridDim.x * SEL_T;
-        for (int64_t j = (int64_t) blockIdx.x * SEL_T + tid; j < n; j += stride) {
-            const uint32_t fl = w.flags[j];
-            if (!fl) continue;
-            sel_count(g, st, lhist, p, is_key, shift, dmask, w.keys[j], fl, j);
+        for (int64_t j0 = (int64_t) blockIdx.x * SEL_T + tid; j0 < n; j0 += stride * SEL_EACH) {
+            uint32_t fl[SEL_EACH];
+            uint64_t key[SEL_EACH];
+#pragma unroll
+            for (int e = 0; e < SEL_EACH; ++e) {
+                const int64_t j = j0 + e * stride, jc = j < n ? j : n - 1;
+                fl[e] = j < n ? w.flags[jc] : 0u;
+                key[e] = w.keys[jc];
+            }
+#pragma unroll
+            for (int e = 0; e < SEL_EACH; ++e)
+                if (fl[e]) sel_count(g, st, lhist, p, is_key, shift, dmask, key[e], fl[e], j0 + e * stride);
         }
     }
     __syncthreads();
@@ -728,34 +762,68 @@ __global__ __launch_bounds__(SEL_T) void sel_pass_kernel(SelWorkspace w, const d
     }
 }
 
-// Appends the selected candidates among instances first, first + stride, ... to their sides' lists; st is the
-// final state of every side.
-__device__ __forceinline__ void sel_collect(const SelWorkspace &w, int64_t n, const SelGeom &g, const SelState *st,
-                                            int64_t first, int64_t stride) {
-    for (int64_t j = first; j < n; j += stride) {
-        const uint32_t fl = w.flags[j];
-        if (!fl) continue;
-        const uint64_t key = w.keys[j];
-        for (int s = 0; s < g.n_sides; ++s) {
-            if (!(fl & (1u << s))) continue;
-            const bool desc = sel_side_descending(s, g.n_sides);
-            const uint64_t k2 = desc ? ~key : key;
-            const uint32_t i2 = desc ? g.idx_mask - (uint32_t) j : (uint32_t) j;
-            int cmp;
-            if (st[s].k_rem == 0 && st[s].done) {
-                cmp = 1;  // nothing to take on this side
-            } else {
-                // compare on the digits this side consumed before it was decided
-                cmp = sel_cmp_prefix(k2, i2, st[s], (int) st[s].pad, g.idx_bits);
+// Whether instance j is among those a side takes; st is the side's final state.
+__device__ __forceinline__ bool sel_taken(const SelGeom &g, const SelState &st, uint64_t k2, uint32_t i2) {
+    if (st.k_rem == 0 && st.done) return false;   // nothing to take on this side
+    // compare on the digits this side consumed before it was decided
+    return sel_cmp_prefix(k2, i2, st, (int) st.pad, g.idx_bits) <= 0;
+}
+
+// Appends the selected candidates among instances [lo, hi) to their sides' lists.  A workgroup counts its own first and asks for their
+// places once per side and SEL_EACH instances of each thread: the thousand candidates' own atomics on two addresses took longer than
+// the rest of the kernel (80,000 instances: 13.7 -> 7.4 us, 20,000: 7.2 -> 5.4).
+template <int NS>
+__device__ __forceinline__ void sel_collect(const SelWorkspace &w, const SelGeom &g, const SelState *st, int64_t lo, int64_t hi, uint32_t *scratch) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = (int) blockDim.x >> 6, nt = (int) blockDim.x;
+    for (int64_t j0 = lo; j0 < hi; j0 += (int64_t) nt * SEL_EACH) {
+        uint64_t key[SEL_EACH];
+        uint32_t fl[SEL_EACH];
+#pragma unroll
+        for (int e = 0; e < SEL_EACH; ++e) {
+            const int64_t j = j0 + (int64_t) e * nt + tid;
+            fl[e] = j < hi ? w.flags[j] : 0u;
+            key[e] = w.keys[j < hi ? j : hi - 1];
+        }
+        uint64_t takes[NS][SEL_EACH];   // which lanes' instance e goes to the side's list
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            const bool desc = sel_side_descending(s, NS);
+            int count = 0;
+#pragma unroll
+            for (int e = 0; e < SEL_EACH; ++e) {
+                const uint32_t j = (uint32_t) (j0 + (int64_t) e * nt + tid);
+                takes[s][e] = __ballot(((fl[e] >> s) & 1u) && sel_taken(g, st[s], desc ? ~key[e] : key[e], desc ? g.idx_mask - j : j));
+                count += __popcll(takes[s][e]);
             }
-            if (cmp <= 0) {
-                const uint32_t pos = atomicAdd(&w.count[s], 1u);
-                if (pos < MAX_WS) {
-                    w.list_key[s * MAX_WS + pos] = k2;
-                    w.list_idx[s * MAX_WS + pos] = i2;
+            if (lane == 0) scratch[s * waves + wave] = (uint32_t) count;
+        }
+        __syncthreads();
+        if (tid < NS) {
+            uint32_t total = 0;
+            for (int v = 0; v < waves; ++v) {   // (the counts become the wavefronts' first places)
+                const uint32_t mine = scratch[tid * waves + v];
+                scratch[tid * waves + v] = total;
+                total += mine;
+            }
+            scratch[NS * waves + tid] = total ? atomicAdd(&w.count[tid], total) : 0u;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            const bool desc = sel_side_descending(s, NS);
+            uint32_t at = scratch[NS * waves + s] + scratch[s * waves + wave];
+#pragma unroll
+            for (int e = 0; e < SEL_EACH; ++e) {
+                const uint32_t j = (uint32_t) (j0 + (int64_t) e * nt + tid);
+                const uint32_t pos = at + (uint32_t) __popcll(takes[s][e] & ((1ull << lane) - 1ull));
+                if (((takes[s][e] >> lane) & 1ull) && pos < MAX_WS) {
+                    w.list_key[s * MAX_WS + pos] = desc ? ~key[e] : key[e];
+                    w.list_idx[s * MAX_WS + pos] = desc ? g.idx_mask - j : j;
                 }
+                at += (uint32_t) __popcll(takes[s][e]);
             }
         }
+        __syncthreads();   // (scratch is written again)
     }
 }
 
@@ -767,19 +835,22 @@ __device__ __forceinline__ bool sel_undecided(const SelGeom &g, const SelState *
 
 // After the grid-wide passes every side is normally decided: then this kernel appends every selected candidate
 // to its side's list.  If a boundary bucket is still too large it does nothing, and sel_final_kernel goes on.
+template <int NS>
 __global__ __launch_bounds__(SEL_T) void sel_compact_kernel(SelWorkspace w, int64_t n, SelGeom g, int p_full) {
     __shared__ SelState st[SEL_MAX_SIDES];
     __shared__ uint32_t scratch[SEL_T + 16];
-    sel_advance_state(w, g, p_full, st, scratch);
-    if (blockIdx.x == 0 && (int) threadIdx.x < g.n_sides) w.state[p_full * SEL_MAX_SIDES + threadIdx.x] = st[threadIdx.x];
+    sel_advance_state<NS>(w, g, p_full, st, scratch);
+    if (blockIdx.x == 0 && (int) threadIdx.x < NS) w.state[p_full * SEL_MAX_SIDES + threadIdx.x] = st[threadIdx.x];
     if (sel_undecided(g, st)) return;
-    sel_collect(w, n, g, st, (int64_t) blockIdx.x * SEL_T + threadIdx.x, (int64_t) gridDim.x * SEL_T);
+    const int64_t chunk = (n + gridDim.x - 1) / gridDim.x, lo = (int64_t) blockIdx.x * chunk;
+    sel_collect<NS>(w, g, st, lo, lo + chunk < n ? lo + chunk : n, scratch);
 }
 
 // Digits p_full .. n_pass-1 and the lists, by one workgroup: only when the grid-wide digits left a boundary
 // bucket too large to take whole (many equal f values, e.g. the first iteration of a training run, where the
 // instance index has to break the ties).  The workgroup walks the candidates once per remaining digit: slow but
 // rare, and it keeps a launch per digit out of every call.  st holds the state before digit p_full.
+template <int NS>
 __device__ void sel_tail(const SelWorkspace &w, int64_t n, const SelGeom &g, int p_full, SelState *st,
                          uint32_t (*lhist)[SEL_BINS], uint32_t *scratch) {
     const int tid = threadIdx.x, nt = blockDim.x;
@@ -798,9 +869,9 @@ __device__ void sel_tail(const SelWorkspace &w, int64_t n, const SelGeom &g, int
         uint32_t *gh = w.hist + (size_t) p * SEL_MAX_SIDES * SEL_BINS;
         for (int e = tid; e < g.n_sides * SEL_BINS; e += nt) gh[e] = (&lhist[0][0])[e];
         __syncthreads();   // sel_advance_state reads state[p] and hist[p] back from memory
-        sel_advance_state(w, g, p + 1, st, scratch);
+        sel_advance_state<NS>(w, g, p + 1, st, scratch);
     }
-    sel_collect(w, n, g, st, tid, nt);
+    sel_collect<NS>(w, g, st, 0, n, scratch);
     __syncthreads();
 }
 
@@ -955,7 +1026,7 @@ __global__ __launch_bounds__(SEL_RANK_T) void sel_final_kernel(SelWorkspace w, i
     int si[NS], pos_other[NS];   // entry `tid` of every side's list in order: instance, its place in the paired side's list or -1
     if (sel_undecided(g, st)) {   // (sel_compact_kernel has left the lists empty)
         if (blockIdx.x != 0) return;
-        sel_tail(w, n, g, p_full, st, sh.hist, scratch);
+        sel_tail<NS>(w, n, g, p_full, st, sh.hist, scratch);
         // (counted with atomics by this workgroup itself: an atomic read)
         if (tid < NS) cnt[tid] = imin_sel((int) __hip_atomic_load(&w.count[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), MAX_WS);
         __syncthreads();
@@ -1130,8 +1201,9 @@ static void dispatch_update_f(double *f, const double *alpha_diff, int ws_size, 
     const bool aligned = (uintptr_t) k_rows % 16 == 0;
     if (!big) {
         // As few columns per thread as make do with one workgroup per CU (more workgroups than that leave some CUs two in
-        // turn), beyond 65,536 columns four floats or one double.  500 of 1,024 rows, us a call, one thread per column / here with
+        // turn), floats two up to 65,536 columns and four beyond, doubles one.  500 of 1,024 rows, us a call, one thread per column / here with
         // 1, 2, 4 floats (1, 2 doubles) per thread:
+        // (40,000 columns and the selection's first pass on top, in training: 26.8 us with four, 24.4 with two.)
         //   floats   3,200: 26.7 / 12.7 15.1 18.6   20,000: 30.7 / 16.9 15.7 19.0   40,000: 31.5 / 26.6 21.5 19.8
         //           60,000: 34.0 / 32.8 24.3 24.5  120,000: 46.7 / 59.6 45.0 43.2  255,000: 100 / 128 99.6 90.3 (5.6 TB/s)
         //   doubles  3,200: 32.6 / 14.9 15.3        18,000: 35.7 / 20.0 16.7        40,000: 38.7 / 31.0 34.2
@@ -1139,7 +1211,7 @@ static void dispatch_update_f(double *f, const double *alpha_diff, int ws_size, 
         auto fits = [&](int cols, size_t esz) { return (uintptr_t) k_rows % (cols * esz) == 0 && ld % cols == 0 && n <= (int64_t) 64 * cols * 256; };
         if (row_type == TSVM_ROW_F32) {
             if (fits(1, 4)) launch_update_f_narrow<float, 1, 32, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
-            else if (fits(2, 4)) launch_update_f_narrow<float, 2, 16, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
+            else if (fits(2, 4) || (n <= 65536 && (uintptr_t) k_rows % 8 == 0 && ld % 2 == 0)) launch_update_f_narrow<float, 2, 16, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
             else if (aligned && ld % 4 == 0) launch_update_f_narrow<float, 4, 16, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
             else launch_update_f_narrow<float, 1, 32, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
         } else {
@@ -1193,9 +1265,11 @@ static int select_working_set(const double *f, const int *y, const double *alpha
     // workgroup.  Near convergence the free support vectors crowd within epsilon of the threshold, so the third
     // digit is usually the one that separates them.
     const int p_full = n > ((int64_t) 1 << 26) ? 4 : 3;   // < n_pass, which is at least 7
-    // two workgroups per CU: every workgroup adds its histogram to the global one with atomics, and with more
-    // workgroups those take longer than the counting they spread (n = 800k: 92 us per call with 1024, 80 with 496)
-    unsigned grid = (unsigned) std::min<int64_t>((n + SEL_T - 1) / SEL_T, 496);
+    // Every workgroup adds its histogram to the global one and asks for its candidates' places with atomics, on a few addresses that
+    // most of them share, and with many workgroups those take longer than the counting they spread: four instances a thread, at
+    // least 64 workgroups while there are instances for them, at most two per CU (n = 800k: 92 us per call with 1,024, 80 with 496).
+    unsigned grid = (unsigned) std::min<int64_t>(std::max<int64_t>((n + SEL_T * SEL_EACH - 1) / (SEL_T * SEL_EACH),
+                                                                  std::min<int64_t>((n + SEL_T - 1) / SEL_T, 64)), 496);
     if ((n + grid - 1) / grid > SEL_CHUNK_MAX) grid = (unsigned) ((n + SEL_CHUNK_MAX - 1) / SEL_CHUNK_MAX);
     if (!armed) {
         hipLaunchKernelGGL(sel_init_kernel, dim3(p_full * SEL_MAX_SIDES * SEL_BINS / 1024), dim3(256), 0, s, w, p_full);
@@ -1206,7 +1280,8 @@ static int select_working_set(const double *f, const int *y, const double *alpha
         else hipLaunchKernelGGL(sel_pass_kernel<2>, dim3(grid), dim3(SEL_T), 0, s, w, f, y, alpha, n, Cp, Cn, g, p, marked, n_marked);
         TSVM_LAUNCH_CHECK();
     }
-    hipLaunchKernelGGL(sel_compact_kernel, dim3(grid), dim3(SEL_T), 0, s, w, n, g, p_full);
+    if (nu) hipLaunchKernelGGL(sel_compact_kernel<4>, dim3(grid), dim3(SEL_T), 0, s, w, n, g, p_full);
+    else hipLaunchKernelGGL(sel_compact_kernel<2>, dim3(grid), dim3(SEL_T), 0, s, w, n, g, p_full);
     TSVM_LAUNCH_CHECK();
     if (nu) hipLaunchKernelGGL(sel_final_kernel<4>, dim3(4 * MAX_WS / SEL_RANK_ENTRIES), dim3(SEL_RANK_T), 0, s, w, n, g, p_full, out, fold_n, out_folded, report);
     else hipLaunchKernelGGL(sel_final_kernel<2>, dim3(2 * MAX_WS / SEL_RANK_ENTRIES), dim3(SEL_RANK_T), 0, s, w, n, g, p_full, out, fold_n, out_folded, report);
