@@ -203,11 +203,17 @@ __global__ __launch_bounds__(256, 2) void predict_dense_stream_kernel(
             mj[tj] = IND ? s_mj[gen][wj * 64 + lrow * 4 + tj] : 0;
         }
         // the indicator columns' share of a dot product: 1.0 once per column both rows have set, one addition at a
-        // time (the serial chain over those columns, bit for bit)
+        // time (the serial chain over those columns, bit for bit).  IND = 1..4: that many additions, IND = 5: max_ones of them in a
+        // loop, which as the only form took the RBF kernel of a seven-class model (16,076 support vectors, 50,000 rows) 1.76 ms, not 1.65.
         auto with_indicators = [&](double dot, uint64_t mi, int tj) -> double {
             if (IND) {
                 const int cnt = __popcll(mi & mj[tj]);
-                for (int t = 0; t < max_ones; ++t) dot += cnt > t ? 1.0 : 0.0;
+                if (IND <= 4) {
+#pragma unroll
+                    for (int t = 0; t < IND; ++t) dot += cnt > t ? 1.0 : 0.0;
+                } else {
+                    for (int t = 0; t < max_ones; ++t) dot += cnt > t ? 1.0 : 0.0;
+                }
             }
             return dot;
         };
@@ -414,11 +420,16 @@ int tsvm_predict_dec_values_dense(const double *sv_x, int64_t ldx, int d, const 
         case 6: PD_STREAM(KTYPE, 6, IND_, KT_); break;  \
         default: PD_STREAM(KTYPE, 8, IND_, KT_); break; \
     }
+#define PD_RBF(IND_)                              \
+    do {                                          \
+        if (d <= 16) PD_NC(TSVM_RBF, IND_, 1)     \
+        else PD_NC(TSVM_RBF, IND_, 2)             \
+    } while (0)
 #define PD_KIND(KTYPE)                            \
     do {                                          \
         if (mask_sv) {                            \
-            if (d <= 16) PD_NC(KTYPE, 1, 1)       \
-            else PD_NC(KTYPE, 1, 2)               \
+            if (d <= 16) PD_NC(KTYPE, 5, 1)       \
+            else PD_NC(KTYPE, 5, 2)               \
         } else {                                  \
             if (d <= 16) PD_NC(KTYPE, 0, 1)       \
             else PD_NC(KTYPE, 0, 2)               \
@@ -428,8 +439,15 @@ int tsvm_predict_dec_values_dense(const double *sv_x, int64_t ldx, int d, const 
                 case TSVM_LINEAR: PD_KIND(TSVM_LINEAR); break;
                 case TSVM_POLY: PD_KIND(TSVM_POLY); break;
                 case TSVM_SIGMOID: PD_KIND(TSVM_SIGMOID); break;
-                default: PD_KIND(TSVM_RBF); break;
+                default:
+                    if (mask_sv && max_ones == 1) PD_RBF(1);
+                    else if (mask_sv && max_ones == 2) PD_RBF(2);
+                    else if (mask_sv && max_ones == 3) PD_RBF(3);
+                    else if (mask_sv && max_ones == 4) PD_RBF(4);
+                    else PD_KIND(TSVM_RBF);
+                    break;
             }
+#undef PD_RBF
 #undef PD_KIND
 #undef PD_NC
 #undef PD_STREAM
