@@ -403,6 +403,11 @@ int tsvm_sum_kernel_values(const double *coef, int total_sv, const int *sv_start
                            const double *rho, const void *k_mat, int row_type, int64_t ldk, double *dec_values,
                            int n_classes, int64_t n_instances, tsvm_stream stream);
 
+/* The one-vs-one vote over those decision values (svc.cpp:265-316): winner[r] = the class index with most votes of row r's
+ * pairs, the lowest among equals; 2 <= n_classes <= tsvm_predict_votes_max_classes(). */
+int tsvm_predict_votes_max_classes(void);
+int tsvm_predict_votes(const double *dec_values, int64_t m, int n_classes, int *winner, tsvm_stream stream);
+
 /* SvmModel::predict_dec_values in one pass (src/thundersvm/model/svmmodel.cpp:74-117: KernelMatrix::get_rows of the
  * batch against the support vectors, then sum_kernel_values, kernelmatrix_kernel.cpp:110-147): the same decision
  * values, with the kernel values reduced in registers instead of being written out as a batch x support-vector

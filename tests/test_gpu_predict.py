@@ -229,3 +229,80 @@ def test_batch_without_any_entry(m, kt):
         got = gm.predict(te, batch)[1]
         assert got.shape == want.shape and np.abs(got - want).max() < 1e-6 and (got == got[0]).all()
     assert np.array_equal(gm.predict(Dataset(te).to_device())[1], got)
+
+
+@pytest.mark.parametrize("groups", [1, 2, 3, 4, 5, 7])
+def test_indicator_groups(groups, monkeypatch):
+    """A row sets one column of each one-hot group: so many matches are added one by one, up to four without a loop."""
+    rng = np.random.default_rng(300 + groups)
+    x, y = _blobs(rng, 4, 60, 6)
+    hot = np.zeros((len(y), groups * 9), dtype=np.float32)
+    for g in range(groups):
+        hot[np.arange(len(y)), g * 9 + (y.astype(int) * 2 + rng.integers(0, 3, len(y))) % 9] = 1.0
+    x = np.concatenate([x, hot], axis=1)
+    tr, te = D.CsrData(*_csr(x[:200]), y[:200]), D.CsrData(*_csr(x[200:]), y[200:])
+    _check(tr, te, make_param(svm_type=0, kernel_type=2, gamma=0.1, C=2.0), monkeypatch)
+
+
+def _csr(x):
+    n, d = x.shape
+    return np.arange(n + 1, dtype=np.int64) * d, np.tile(np.arange(1, d + 1, dtype=np.int32), n), x.reshape(-1).astype(np.float64)
+
+
+def _votes(dec, k):
+    m = dec.shape[0]
+    votes = np.zeros((m, k), dtype=int)
+    p = 0
+    for i in range(k):
+        for j in range(i + 1, k):
+            pos = dec[:, p] > 0
+            votes[:, i] += pos
+            votes[:, j] += ~pos
+            p += 1
+    return votes.argmax(axis=1)   # (the first among equals)
+
+
+@pytest.mark.parametrize("k", [2, 3, 7, 33, 64])
+@pytest.mark.parametrize("m", [0, 1, 255, 256, 257, 1000])
+def test_votes(k, m):
+    """The vote kernel against the count in numpy: ties between classes, zeros (a vote for the second class), infinities and NaN."""
+    import torch
+    import gpu_util as G
+    from thundersvm_amd import capi
+    rng = np.random.default_rng(k * 1000 + m)
+    dec = rng.choice([-1.5, -0.0, 0.0, 0.3, 2.0, np.inf, -np.inf, np.nan], size=(m, k * (k - 1) // 2))
+    won = torch.full((m + 1,), -7, dtype=torch.int32, device="cuda")
+    dec_d = G.dev(np.ascontiguousarray(dec if m else np.zeros((1, 1))))
+    capi.call("tsvm_predict_votes", G.ptr(dec_d), m, k, G.ptr(won), G.stream())
+    got = G.host(won)
+    assert np.array_equal(got[:m], _votes(dec, k)) and got[m] == -7
+    with pytest.raises(capi.TsvmError):
+        capi.call("tsvm_predict_votes", G.ptr(dec_d), m, capi.kernel_lib().tsvm_predict_votes_max_classes() + 1, G.ptr(won), G.stream())
+
+
+@pytest.mark.parametrize("k,rows", [(2, 20000), (5, 1638), (5, 1639), (70, 30)])
+@pytest.mark.parametrize("dense", [True, False])
+def test_labels_by_votes_on_the_device_and_on_the_host(k, rows, dense):
+    """Labels are the vote over the decision values that come with them, whichever side takes it (16,384 pair votes on, up to 64
+    classes: the device), in one batch or several, and a prediction leaves nothing to the next one."""
+    rng = np.random.default_rng(k)
+    x, y = _blobs(rng, k, 12 if k > 10 else 40, 6, spread=3.0)
+    if not dense:
+        x[rng.random(x.shape) < 0.3] = 0
+        x = np.concatenate([x, np.zeros((len(y), 3000), dtype=np.float32)], axis=1)
+        x[np.arange(len(y)), rng.integers(6, x.shape[1], len(y))] = 1.0
+    def data(rows_of):
+        if dense:
+            return D.CsrData(*_csr(rows_of), y[:1].repeat(len(rows_of)))
+        ptr = np.concatenate([[0], np.cumsum((rows_of != 0).sum(axis=1))]).astype(np.int64)
+        r, c = np.nonzero(rows_of)
+        return D.CsrData(ptr, c.astype(np.int32) + 1, rows_of[r, c].astype(np.float64), y[:1].repeat(len(rows_of)))
+    tr = data(x)
+    tr = D.CsrData(tr.ptr, tr.col, tr.val, y)
+    prm = make_param(svm_type=0, kernel_type=2, gamma=0.1, C=1.0)
+    m = Model(0).train(tr, prm)
+    many, few = data(x[rng.integers(0, len(y), rows)]), data(x[:3])
+    for d in (many, few, many):
+        for batch in (-1, 700):
+            labels, dec = m.predict(d, batch)
+            assert np.array_equal(labels, m.label[_votes(dec, k)].astype(np.float64))

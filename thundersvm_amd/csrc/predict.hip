@@ -366,9 +366,43 @@ __global__ __launch_bounds__(256) void predict_combine_kernel(const double *__re
     dec[idx] = (s + t) - rho[idx % P];
 }
 
+// The one-vs-one vote (svc.cpp:265-316): per row, one vote per pair, the lowest class index among those with most.  A thread
+// per row, its counts in LDS; bound by the read of the decision values, 8 m P bytes that the kernel before has just written
+// (50,000 rows of 21 pairs: 7 us; one host thread takes some 0.8 ms).
+#define VOTE_T 256
+#define VOTE_MAX_CLASSES 64
+__global__ __launch_bounds__(VOTE_T) void predict_votes_kernel(const double *__restrict__ dec, int64_t m, int n_classes, int *__restrict__ winner) {
+    extern __shared__ unsigned short votes[];   // [n_classes][VOTE_T]
+    const int64_t r = (int64_t) blockIdx.x * VOTE_T + threadIdx.x;
+    if (r >= m) return;
+    for (int c = 0; c < n_classes; ++c) votes[c * VOTE_T + threadIdx.x] = 0;
+    const double *v = dec + r * ((int64_t) n_classes * (n_classes - 1) / 2);
+    for (int i = 0; i < n_classes; ++i)
+        for (int j = i + 1; j < n_classes; ++j) ++votes[(*v++ > 0 ? i : j) * VOTE_T + threadIdx.x];
+    int best = 0, most = votes[threadIdx.x];
+    for (int c = 1; c < n_classes; ++c) {
+        const int n = votes[c * VOTE_T + threadIdx.x];
+        if (n > most) { most = n; best = c; }
+    }
+    winner[r] = best;
+}
+
 static int nc_template(int nc) { return nc <= 4 ? nc : nc <= 6 ? 6 : 8; }
 
 extern "C" {
+
+int tsvm_predict_votes_max_classes(void) { return VOTE_MAX_CLASSES; }
+
+int tsvm_predict_votes(const double *dec_values, int64_t m, int n_classes, int *winner, tsvm_stream stream) {
+    TSVM_REQUIRE(dec_values && winner, "tsvm_predict_votes: null pointer");
+    TSVM_REQUIRE(m >= 0 && m <= 0x7fff0000 && n_classes >= 2 && n_classes <= VOTE_MAX_CLASSES, "tsvm_predict_votes: %lld rows, %d classes (2 .. %d)",
+                 (long long) m, n_classes, VOTE_MAX_CLASSES);
+    if (m == 0) return 0;
+    hipLaunchKernelGGL(predict_votes_kernel, dim3((unsigned) ((m + VOTE_T - 1) / VOTE_T)), dim3(VOTE_T), n_classes * VOTE_T * sizeof(unsigned short),
+                       tsvm_s(stream), dec_values, m, n_classes, winner);
+    TSVM_LAUNCH_CHECK();
+    return 0;
+}
 
 int tsvm_predict_nc_stride(int n_classes, int d, int has_masks) {
     const int nc = n_classes - 1;

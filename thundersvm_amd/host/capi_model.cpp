@@ -188,7 +188,7 @@ int tsvm_model_predict(void *model, void *dataset, int batch_size, double *dec_v
         const DataSet &ds = *(DataSet *) dataset;
         std::vector<float_type> out = m.predict(ds, batch_size);
         if (labels) memcpy(labels, out.data(), sizeof(double) * out.size());
-        if (dec_values) memcpy(dec_values, m.get_dec_value().data(), sizeof(double) * m.get_dec_value().size());
+        if (dec_values) tsvm::parallel_memcpy(dec_values, m.get_dec_value().data(), sizeof(double) * m.get_dec_value().size());
     })
 }
 
@@ -296,7 +296,7 @@ int tsvm_model_predict_csr(void *model, int64_t nrows, const int64_t *row_ptr, c
         ds.load_from_csr(nrows, row_ptr, col, val, nullptr, false);
         std::vector<float_type> out = m.predict(ds, batch_size);
         if (labels) memcpy(labels, out.data(), sizeof(double) * (size_t) nrows);
-        if (dec_values) memcpy(dec_values, m.get_dec_value().data(), sizeof(double) * m.get_dec_value().size());
+        if (dec_values) tsvm::parallel_memcpy(dec_values, m.get_dec_value().data(), sizeof(double) * m.get_dec_value().size());
     })
 }
 

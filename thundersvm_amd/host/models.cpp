@@ -875,6 +875,11 @@ void SVC::train_pairs_in_lockstep(const DataSet &grouped, int lanes, std::vector
     }
 }
 
+// The votes are the device's from 16,384 of them on: below, the launch and its copy cost more than the host's loop.
+bool SVC::votes_on_device(size_t n_rows) const {
+    return param.probability == 0 && n_classes >= 2 && n_classes <= tsvm_predict_votes_max_classes() && n_rows * n_binary_models >= 16384;
+}
+
 std::vector<float_type> SVC::finish_predict(int n_instances) {   // svc.cpp:179-185
     return predict_label(dec_values, n_instances);
 }
@@ -1060,6 +1065,10 @@ void SVC::probability_train(const DataSet &grouped) {
 // probability estimates, the class of highest coupled probability (prob_predict keeps all of them).
 std::vector<float_type> SVC::predict_label(const std::vector<float_type> &dec, int n_instances) {
     std::vector<float_type> out(n_instances);
+    if (param.probability == 0 && n_instances > 0 && vote_winner.size() == (size_t) n_instances) {
+        for (int r = 0; r < n_instances; ++r) out[r] = (float) label[vote_winner[r]];
+        return out;
+    }
     if (param.probability == 0) {
         std::vector<int> votes(n_classes);
         for (int r = 0; r < n_instances; ++r) {

@@ -16,11 +16,12 @@ public:
     virtual ~SvmModel() = default;
     void train(const DataSet &dataset, SvmParam param);
     std::vector<float_type> predict(const DataSet::node2d &instances, int batch_size = -1);
-    void predict_dec_values(const RowStore &rows, std::vector<float_type> &dec_values, int batch_size) const;
+    // winner, when it is asked for: left empty, or every row's class by the one-vs-one vote, taken on the device
+    void predict_dec_values(const RowStore &rows, std::vector<float_type> &dec_values, int batch_size, std::vector<int> *winner = nullptr) const;
     // The same for the instances of a DataSet; when the DataSet has a device-resident copy of its rows in the dense
     // layout (DeviceRows::of), the kernels read the rows where they lie: nothing is assembled on the host or uploaded.
     std::vector<float_type> predict(const DataSet &dataset, int batch_size = -1);
-    void predict_dec_values(const DataSet &dataset, std::vector<float_type> &dec_values, int batch_size) const;
+    void predict_dec_values(const DataSet &dataset, std::vector<float_type> &dec_values, int batch_size, std::vector<int> *winner = nullptr) const;
     virtual std::vector<float_type> cross_validation(DataSet dataset, SvmParam param, int n_fold);
 
     virtual void save_to_file(std::string path);
@@ -92,12 +93,17 @@ protected:
     // what predict returns once dec_values holds the decision values of n_instances rows: the values themselves,
     // class labels (SVC) or the side of the boundary (OneClassSVC)
     virtual std::vector<float_type> finish_predict(int n_instances) { return dec_values; }
+    // whether a prediction of so many rows has its votes taken on the device (vote_winner)
+    virtual bool votes_on_device(size_t) const { return false; }
+    std::vector<int> vote_winner;   // (only while predict runs)
     // the model as the prediction kernels read it (support vectors in HBM, coefficients by padded column)
     struct PredictPlan;
     const PredictPlan &predict_plan() const;
     // one batch, rows already on the device as a dense matrix; false when the kernels do not take this model's shape
     bool predict_batch_fused(const PredictPlan &plan, const kernel_type *a, int64_t lda, const kernel_type *sd_a, size_t m,
-                             bool indicator_values, float_type *dec_out) const;
+                             bool indicator_values, float_type *dec_out, int *winner_out) const;
+    // decision values of m rows and, behind them on the device, room for their winners when those are wanted: to the host
+    void fetch_predictions(float_type *d_dec, size_t m, float_type *dec_out, int *winner_out) const;
     void copy_support_vectors(const RowStore &rows);
     // whether problems may take the path for small ones: the caller has asked for nothing that only the other path does
     bool small_path_allowed() const { return !profile && !(trace_first && solver_stats.empty()) && cache_bytes < 0; }
@@ -135,6 +141,7 @@ protected:
     SvmParam::SVM_TYPE svm_type() const override { return SvmParam::C_SVC; }
     void model_setup(const DataSet &dataset, SvmParam &param) override;
     std::vector<float_type> finish_predict(int n_instances) override;
+    bool votes_on_device(size_t n_rows) const override;
     // One class pair (i, j) of the one-vs-one decomposition: its rows, labels, starting point and solver.
     struct BinaryProblem {
         int i = 0, j = 0, k = 0;

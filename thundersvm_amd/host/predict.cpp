@@ -4,6 +4,7 @@
 // tsvm_sum_kernel_values, as the reference does.
 #include <algorithm>
 #include <cstdlib>
+#include <cstring>
 
 #include "models.h"
 
@@ -99,7 +100,7 @@ static void build_chunks(const std::vector<int> &class_tile, size_t row_blocks, 
 }
 
 bool SvmModel::predict_batch_fused(const PredictPlan &P, const kernel_type *a, int64_t lda, const kernel_type *sd_a, size_t m,
-                                   bool indicator_values, float_type *dec_out) const {
+                                   bool indicator_values, float_type *dec_out, int *winner_out) const {
     const DeviceRows &R = sv_k_mat->rows();
     // (TSVM_PREDICT_UNFUSED: the two-call form for every batch, to compare the two)
     if (P.stride == 0 || getenv("TSVM_PREDICT_UNFUSED")) return false;
@@ -122,9 +123,9 @@ bool SvmModel::predict_batch_fused(const PredictPlan &P, const kernel_type *a, i
                                        P.mask_max.data(), tsvm::work_stream()));
     }
     const int km1 = n_classes - 1;
-    // partial sums and decision values: from the persistent row arena (no allocation per call)
+    // partial sums, decision values and winners: from the persistent row arena (no allocation per call)
     const size_t part_doubles = (size_t) std::max(P.n_chunks, 1) * m * km1, dec_doubles = m * (size_t) n_binary_models;
-    float_type *d_part = (float_type *) tsvm::RowArena::instance().acquire((part_doubles + dec_doubles) * sizeof(float_type), false);
+    float_type *d_part = (float_type *) tsvm::RowArena::instance().acquire((part_doubles + dec_doubles) * sizeof(float_type) + m * sizeof(int), false);
     float_type *d_dec = d_part + part_doubles;
     // (a batch row may set more indicator columns than any support vector does: its matches are bounded by the
     // support vectors' count all the same)
@@ -133,15 +134,27 @@ bool SvmModel::predict_batch_fused(const PredictPlan &P, const kernel_type *a, i
                                             P.class_chunk_start.data(), P.rho.data(), n_classes, a, lda, (int64_t) m, sd_a,
                                             plan_masks ? P.mask_a.data() : nullptr, R.ind_max_ones, (int) param.kernel_type,
                                             param.gamma, param.coef0, param.degree, d_part, d_dec, tsvm::work_stream()));
-    tsvm::HostStaging::instance().download(d_dec, dec_doubles * sizeof(float_type), [dec_out](const char *from, size_t off, size_t len) {
-        tsvm::parallel_memcpy((char *) dec_out + off, from, len);
-    }, tsvm::work_stream());
+    fetch_predictions(d_dec, m, dec_out, winner_out);
     return true;
 }
 
-void SvmModel::predict_dec_values(const RowStore &rows, std::vector<float_type> &dec, int batch_size) const {
+void SvmModel::fetch_predictions(float_type *d_dec, size_t m, float_type *dec_out, int *winner_out) const {
+    const size_t dec_bytes = m * (size_t) n_binary_models * sizeof(float_type);
+    int *const d_winner = (int *) ((char *) d_dec + dec_bytes);
+    if (winner_out) abi_check(tsvm_predict_votes(d_dec, (int64_t) m, n_classes, d_winner, tsvm::work_stream()));
+    tsvm::HostStaging::instance().download(d_dec, dec_bytes + (winner_out ? m * sizeof(int) : 0), [=](const char *from, size_t off, size_t len) {
+        if (off < dec_bytes) tsvm::parallel_memcpy((char *) dec_out + off, from, std::min(len, dec_bytes - off));
+        if (off + len > dec_bytes) {
+            const size_t lo = std::max(off, dec_bytes);
+            memcpy((char *) winner_out + (lo - dec_bytes), from + (lo - off), off + len - lo);
+        }
+    }, tsvm::work_stream());
+}
+
+void SvmModel::predict_dec_values(const RowStore &rows, std::vector<float_type> &dec, int batch_size, std::vector<int> *winner) const {
     const size_t n_rows = rows.size();
-    dec.assign(n_rows * (size_t) n_binary_models, 0);
+    dec.resize(n_rows * (size_t) n_binary_models);   // (every element is written below)
+    if (winner) winner->clear();
     if (n_rows == 0) return;
     const size_t T = sv->size();
     if (T == 0) {
@@ -167,25 +180,28 @@ void SvmModel::predict_dec_values(const RowStore &rows, std::vector<float_type> 
     void *d_k = nullptr;
     const int64_t ldk = ((int64_t) T + 15) / 16 * 16;   // (rows padded to 16 elements: get_rows writes whole aligned vectors)
     DeviceBuffer<float_type> d_dec;
+    if (winner) winner->resize(n_rows);
     for (size_t b0 = 0; b0 < n_rows; b0 += batch_size) {
         const size_t bm = std::min((size_t) batch_size, n_rows - b0);
         if (fused) {
             const KernelMatrix::StagedBatch b = k_mat.stage_batch(rows, b0, bm);
-            if (predict_batch_fused(P, b.a, b.lda, b.sd, bm, b.indicator_values, dec.data() + b0 * n_binary_models)) continue;
+            if (predict_batch_fused(P, b.a, b.lda, b.sd, bm, b.indicator_values, dec.data() + b0 * n_binary_models,
+                                    winner ? winner->data() + b0 : nullptr))
+                continue;
         }
         // kernel values of one batch (taken from the persistent row arena), then the reduction
         if (!d_k) {
             d_k = tsvm::RowArena::instance().acquire(bmax * (size_t) ldk * k_mat.row_elem_size(), false);
-            d_dec.resize(bmax * n_binary_models);
+            d_dec.resize(bmax * n_binary_models + (winner ? (bmax + 1) / 2 : 0));
         }
         k_mat.get_rows(rows, b0, bm, d_k, ldk);
         abi_check(tsvm_sum_kernel_values(P.coef.data(), (int) T, P.sv_start.data(), P.sv_count.data(), P.rho.data(), d_k,
                                          k_mat.row_type(), ldk, d_dec.data(), n_classes, (int64_t) bm, tsvm::work_stream()));
-        d_dec.download(dec.data() + b0 * n_binary_models, bm * n_binary_models);
+        fetch_predictions(d_dec.data(), bm, dec.data() + b0 * n_binary_models, winner ? winner->data() + b0 : nullptr);
     }
 }
 
-void SvmModel::predict_dec_values(const DataSet &dataset, std::vector<float_type> &dec, int batch_size) const {
+void SvmModel::predict_dec_values(const DataSet &dataset, std::vector<float_type> &dec, int batch_size, std::vector<int> *winner) const {
     const std::shared_ptr<void> &slot = dataset.device_cache();
     if (slot && sv->size() > 0 && dataset.n_instances() > 0) {
         const DeviceRows &A = *std::static_pointer_cast<DeviceRows>(slot);
@@ -200,26 +216,36 @@ void SvmModel::predict_dec_values(const DataSet &dataset, std::vector<float_type
                 for (size_t c = (size_t) R.ind_first; c < std::min(R.n_features, A.n_features); ++c)
                     if (st[A.n_features + c] != 0) indicator_values = false;
             }
-            dec.assign(dataset.n_instances() * (size_t) n_binary_models, 0);
+            dec.resize(dataset.n_instances() * (size_t) n_binary_models);   // (every element is written below, or by the call at the end)
+            if (winner) winner->resize(dataset.n_instances());
             const size_t step = batch_size > 0 ? (size_t) batch_size : A.n;
             bool ok = true;
             for (size_t b0 = 0; b0 < A.n && ok; b0 += step) {
                 const size_t bm = std::min(step, A.n - b0);
                 ok = predict_batch_fused(P, A.x.data() + b0 * (size_t) A.ld, A.ld, A.self_dot.data() + b0, bm, indicator_values,
-                                         dec.data() + b0 * n_binary_models);
+                                         dec.data() + b0 * n_binary_models, winner ? winner->data() + b0 : nullptr);
             }
             if (ok) return;
         }
     }
-    predict_dec_values(dataset.rows(), dec, batch_size);
+    predict_dec_values(dataset.rows(), dec, batch_size, winner);
 }
 
+namespace {
+struct ClearAtEnd {   // (a prediction's winners are no other call's)
+    std::vector<int> &v;
+    ~ClearAtEnd() { v.clear(); }
+};
+}  // namespace
+
 std::vector<float_type> SvmModel::predict(const DataSet::node2d &instances, int batch_size) {   // svmmodel.cpp:157-171
-    predict_dec_values(*RowStore::from_nodes(instances), dec_values, batch_size);
+    const ClearAtEnd clear{vote_winner};
+    predict_dec_values(*RowStore::from_nodes(instances), dec_values, batch_size, votes_on_device(instances.size()) ? &vote_winner : nullptr);
     return finish_predict((int) instances.size());
 }
 
 std::vector<float_type> SvmModel::predict(const DataSet &dataset, int batch_size) {
-    predict_dec_values(dataset, dec_values, batch_size);
+    const ClearAtEnd clear{vote_winner};
+    predict_dec_values(dataset, dec_values, batch_size, votes_on_device(dataset.n_instances()) ? &vote_winner : nullptr);
     return finish_predict((int) dataset.n_instances());
 }
