@@ -66,6 +66,11 @@ int tsvm_kernel_diag(const double *self_dot, int64_t n, int kernel_type, double 
 int tsvm_csr_to_dense(const double *val, const int *col, const int64_t *row_ptr, int64_t n, double *x, int64_t ld,
                       tsvm_stream stream);
 
+/* The same, zeros of every column included, with the rows' self dot products (tsvm_csr_self_dot): one launch.  The CSR arrays may
+ * lie in pinned host memory that the device can read. */
+int tsvm_csr_rows_to_dense(const double *val, const int *col, const int64_t *row_ptr, int64_t n, double *x, int64_t ld,
+                           double *self_dot, tsvm_stream stream);
+
 /* Column statistics of the data rows (dense row-major [n][ld], columns 0..d-1; or the nnz stored entries of a CSR
  * matrix with column ids below d): counts[c] = entries of column c (dense: non-zero values; CSR: stored entries),
  * counts[d + c] = how many values of the column are neither 0 nor 1.  counts holds 2*d ints and is cleared by the call.  The per-column entry counts are what the reference's

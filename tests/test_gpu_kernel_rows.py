@@ -599,3 +599,32 @@ def test_indicator_columns(n, n_cont, groups, m, name, kt, prm):
     outb = torch.empty((m, 777), dtype=torch.float64, device="cuda")
     run(capi.ROW_F64, outb, m, x_idx=G.dev(cols), n_cols=777)
     _check(name, G.host(outb), want[:, cols])
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 257])
+@pytest.mark.parametrize("d,ld", [(1, 8), (63, 64), (64, 64), (65, 72), (130, 136), (40, 24)])
+@pytest.mark.parametrize("host", [False, True])
+def test_csr_rows_to_dense(n, d, ld, host):
+    """Rows of no, one, 63, 64, 65 and all entries as a dense matrix over what was there before, entries beyond ld dropped from it and
+    kept in the self dot product, whose bits are the serial chain's; from device memory and from pinned host memory."""
+    rng = np.random.default_rng(n * 1000 + d)
+    lens = np.array([[d, 0, 1, min(d, 63), min(d, 64), min(d, 65)][i % 6] for i in range(n)])
+    ptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    col = np.concatenate([np.sort(rng.permutation(d)[:l]) for l in lens] + [np.zeros(0, dtype=int)]).astype(np.int32)
+    val = rng.standard_normal(len(col))
+    want, dot = np.zeros((n, ld)), np.zeros(n)
+    for i in range(n):
+        for e in range(ptr[i], ptr[i + 1]):
+            if col[e] < ld:
+                want[i, col[e]] = val[e]
+    put = (lambda a: torch.from_numpy(a.copy() if len(a) else np.zeros(1, dtype=a.dtype)).pin_memory()) if host else \
+        (lambda a: G.dev(a if len(a) else np.zeros(1, dtype=a.dtype)))
+    v_d, c_d, p_d = put(val), put(col), put(ptr)
+    x_d = torch.full((n, ld), 7.0, dtype=torch.float64, device="cuda")
+    s_d, t_d = torch.full((n,), 7.0, dtype=torch.float64, device="cuda"), torch.full((n,), 7.0, dtype=torch.float64, device="cuda")
+    capi.call("tsvm_csr_rows_to_dense", v_d.data_ptr(), c_d.data_ptr(), p_d.data_ptr(), n, G.ptr(x_d), ld, G.ptr(s_d), G.stream())
+    assert np.array_equal(G.host(x_d), want)
+    v2, p2 = G.dev(val if len(val) else np.zeros(1)), G.dev(ptr)
+    capi.call("tsvm_csr_self_dot", G.ptr(v2), G.ptr(p2), n, G.ptr(t_d), G.stream())
+    assert np.array_equal(G.host(s_d), G.host(t_d))
+    assert np.allclose(G.host(s_d), [np.dot(val[ptr[i]:ptr[i + 1]], val[ptr[i]:ptr[i + 1]]) for i in range(n)], rtol=1e-13, atol=0)

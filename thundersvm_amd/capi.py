@@ -26,6 +26,7 @@ SIGNATURES = {
     "tsvm_dense_self_dot": (_int, [_p, _i64, _i64, _int, _p, _p]),
     "tsvm_kernel_diag": (_int, [_p, _i64, _int, _dbl, _dbl, _int, _p, _p]),
     "tsvm_csr_to_dense": (_int, [_p, _p, _p, _i64, _p, _i64, _p]),
+    "tsvm_csr_rows_to_dense": (_int, [_p, _p, _p, _i64, _p, _i64, _p, _p]),
     "tsvm_column_stats_dense": (_int, [_p, _i64, _i64, _int, _p, _p]),
     "tsvm_column_stats_csr": (_int, [_p, _p, _i64, _int, _p, _p]),
     "tsvm_indicator_masks": (_int, [_p, _i64, _i64, _int, _int, _p, _p, _p]),

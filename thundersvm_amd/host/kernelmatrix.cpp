@@ -433,14 +433,7 @@ std::shared_ptr<DeviceRows> DeviceRows::from_host(const RowStore &rows) {
     r.values_fit_float = all_float != 0;
     r.values_finite = all_finite != 0;
     r.dense = KernelMatrix::choose_dense(r.n, r.n_features, r.nnz);
-    r.val.resize(r.nnz);
-    r.col.resize(r.nnz);
-    r.row_ptr.resize(r.n + 1);
     tsvm::HostStaging &staging = tsvm::HostStaging::instance();
-    if (r.nnz) {
-        staging.upload(r.val.data(), {{val, r.nnz * sizeof(kernel_type), 0}}, tsvm::work_stream());
-        staging.upload(r.col.data(), {{col, r.nnz * sizeof(int), 0}}, tsvm::work_stream());
-    }
     std::vector<int64_t> ptr;
     const int64_t *host_ptr = rows.ptr();
     if (first != 0 || !r.dense) {
@@ -448,16 +441,22 @@ std::shared_ptr<DeviceRows> DeviceRows::from_host(const RowStore &rows) {
         for (int64_t &p : ptr) p -= first;
         host_ptr = ptr.data();
     }
-    staging.upload(r.row_ptr.data(), {{host_ptr, (r.n + 1) * sizeof(int64_t), 0}}, tsvm::work_stream());
     r.self_dot.resize(r.n);
-    abi_check(tsvm_csr_self_dot(r.val.data(), r.row_ptr.data(), (int64_t) r.n, r.self_dot.data(), tsvm::work_stream()));
     if (r.dense) {
+        // one upload of the three arrays, which are not needed any more once they are a matrix
+        const size_t val_bytes = r.nnz * sizeof(kernel_type), ptr_bytes = (r.n + 1) * sizeof(int64_t), col_bytes = r.nnz * sizeof(int);
+        tsvm::DeviceBuffer<char> csr(ptr_bytes + val_bytes + col_bytes);
+        std::vector<tsvm::HostStaging::Part> parts{{host_ptr, ptr_bytes, 0}};
+        if (r.nnz) {
+            parts.push_back({val, val_bytes, ptr_bytes});
+            parts.push_back({col, col_bytes, ptr_bytes + val_bytes});
+        }
+        staging.upload(csr.data(), parts, tsvm::work_stream());
         r.ld = (int64_t) ((r.n_features + 7) / 8 * 8);
         r.x.resize(r.n * (size_t) r.ld);
-        abi_check(tsvm_csr_to_dense(r.val.data(), r.col.data(), r.row_ptr.data(), (int64_t) r.n, r.x.data(), r.ld, tsvm::work_stream()));
-        r.val.release();
-        r.col.release();
-        r.row_ptr.release();
+        abi_check(tsvm_csr_rows_to_dense((const kernel_type *) (csr.data() + ptr_bytes), (const int *) (csr.data() + ptr_bytes + val_bytes),
+                                         (const int64_t *) csr.data(), (int64_t) r.n, r.x.data(), r.ld, r.self_dot.data(), tsvm::work_stream()));
+        csr.release();
         // indicator columns are a run that ends with the last column: one other value there, in most data sets the
         // first, and there are none (a few of the entries are looked at here, all of them by the device's count)
         bool last_is_indicator = true;
@@ -465,6 +464,15 @@ std::shared_ptr<DeviceRows> DeviceRows::from_host(const RowStore &rows) {
             if (col[e] == max_index && val[e] != 0.0 && val[e] != 1.0) last_is_indicator = false;
         if (last_is_indicator) r.find_indicator_columns();
     } else {
+        r.val.resize(r.nnz);
+        r.col.resize(r.nnz);
+        r.row_ptr.resize(r.n + 1);
+        if (r.nnz) {
+            staging.upload(r.val.data(), {{val, r.nnz * sizeof(kernel_type), 0}}, tsvm::work_stream());
+            staging.upload(r.col.data(), {{col, r.nnz * sizeof(int), 0}}, tsvm::work_stream());
+        }
+        staging.upload(r.row_ptr.data(), {{host_ptr, (r.n + 1) * sizeof(int64_t), 0}}, tsvm::work_stream());
+        abi_check(tsvm_csr_self_dot(r.val.data(), r.row_ptr.data(), (int64_t) r.n, r.self_dot.data(), tsvm::work_stream()));
         r.host_row_ptr = std::move(ptr);
         r.build_sliced();
     }
@@ -740,6 +748,8 @@ void KernelMatrix::get_block(const int *d_idx, int m, void *d_out, int64_t ld, h
                                     stage_blk_.data(), wt, 1, stream));
 }
 
+constexpr size_t READ_FROM_HOST = 4096;   // entries
+
 // The batch goes to the device as CSR (flattened by all cores into pinned memory, copied asynchronously) together
 // with its rows' self dot products; with dense stored rows it is also laid out as a dense matrix of the stored rows'
 // width (columns >= n_features are dropped from the products, kernelmatrix.cpp:392, but stay in the self dot).
@@ -767,23 +777,34 @@ KernelMatrix::StagedBatch KernelMatrix::stage_batch(const RowStore &batch, size_
         col[e] = from_col[e];
         if (col[e] >= ind_lo && col[e] < ind_hi && val[e] != 0.0 && val[e] != 1.0) not_indicator = 1;
     }
-    if (b_val_.size() < total) { b_val_.resize(total); b_col_.resize(total); }
-    if (b_ptr_.size() < (size_t) m + 1) b_ptr_.resize(m + 1);
-    if (total) {
-        TSVM_HIP_CHECK(hipMemcpyAsync(b_val_.data(), val, total * sizeof(kernel_type), hipMemcpyHostToDevice, tsvm::work_stream()));
-        TSVM_HIP_CHECK(hipMemcpyAsync(b_col_.data(), col, total * sizeof(int), hipMemcpyHostToDevice, tsvm::work_stream()));
-    }
-    TSVM_HIP_CHECK(hipMemcpyAsync(b_ptr_.data(), ptr, ((size_t) m + 1) * sizeof(int64_t), hipMemcpyHostToDevice, tsvm::work_stream()));
     if (stage_sd_.size() < (size_t) m) stage_sd_.resize(m);
-    abi_check(tsvm_csr_self_dot(b_val_.data(), b_ptr_.data(), m, stage_sd_.data(), tsvm::work_stream()));
     StagedBatch out;
     out.sd = stage_sd_.data();
     out.indicator_values = R.ind_first >= 0 && !not_indicator;
+    // A request of a few rows is read by the kernel where it is, in page-locked host memory: three copies of a microsecond's work
+    // cost 5 us each.
+    const kernel_type *d_val = val;
+    const int *d_col = col;
+    const int64_t *d_ptr = ptr;
+    if (!R.dense || total > READ_FROM_HOST) {
+        if (b_val_.size() < total) { b_val_.resize(total); b_col_.resize(total); }
+        if (b_ptr_.size() < (size_t) m + 1) b_ptr_.resize(m + 1);
+        if (total) {
+            TSVM_HIP_CHECK(hipMemcpyAsync(b_val_.data(), val, total * sizeof(kernel_type), hipMemcpyHostToDevice, tsvm::work_stream()));
+            TSVM_HIP_CHECK(hipMemcpyAsync(b_col_.data(), col, total * sizeof(int), hipMemcpyHostToDevice, tsvm::work_stream()));
+        }
+        TSVM_HIP_CHECK(hipMemcpyAsync(b_ptr_.data(), ptr, ((size_t) m + 1) * sizeof(int64_t), hipMemcpyHostToDevice, tsvm::work_stream()));
+        d_val = b_val_.data();
+        d_col = b_col_.data();
+        d_ptr = b_ptr_.data();
+    }
     if (R.dense) {
         if (stage_.size() < (size_t) m * R.ld) stage_.resize((size_t) m * R.ld);
-        abi_check(tsvm_csr_to_dense(b_val_.data(), b_col_.data(), b_ptr_.data(), m, stage_.data(), R.ld, tsvm::work_stream()));
+        abi_check(tsvm_csr_rows_to_dense(d_val, d_col, d_ptr, m, stage_.data(), R.ld, stage_sd_.data(), tsvm::work_stream()));
         out.a = stage_.data();
         out.lda = R.ld;
+    } else {
+        abi_check(tsvm_csr_self_dot(d_val, d_ptr, m, stage_sd_.data(), tsvm::work_stream()));
     }
     return out;
 }

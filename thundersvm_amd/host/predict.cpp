@@ -127,6 +127,15 @@ bool SvmModel::predict_batch_fused(const PredictPlan &P, const kernel_type *a, i
     const size_t part_doubles = (size_t) std::max(P.n_chunks, 1) * m * km1, dec_doubles = m * (size_t) n_binary_models;
     float_type *d_part = (float_type *) tsvm::RowArena::instance().acquire((part_doubles + dec_doubles) * sizeof(float_type) + m * sizeof(int), false);
     float_type *d_dec = d_part + part_doubles;
+    // a request of a few rows has its decision values written straight to page-locked host memory: no copy behind the kernels
+    struct HostBlock {
+        tsvm::PinnedBlock block;
+        ~HostBlock() { if (block.host) tsvm::give_pinned_block(block); }
+    } direct;
+    if (!winner_out && dec_doubles * sizeof(float_type) <= tsvm::PINNED_BLOCK) {
+        direct.block = tsvm::take_pinned_block();
+        d_dec = (float_type *) direct.block.dev;
+    }
     // (a batch row may set more indicator columns than any support vector does: its matches are bounded by the
     // support vectors' count all the same)
     abi_check(tsvm_predict_dec_values_dense(R.x.data(), R.ld, d, R.self_dot.data(), plan_masks ? R.ind_mask.data() : nullptr,
@@ -134,7 +143,12 @@ bool SvmModel::predict_batch_fused(const PredictPlan &P, const kernel_type *a, i
                                             P.class_chunk_start.data(), P.rho.data(), n_classes, a, lda, (int64_t) m, sd_a,
                                             plan_masks ? P.mask_a.data() : nullptr, R.ind_max_ones, (int) param.kernel_type,
                                             param.gamma, param.coef0, param.degree, d_part, d_dec, tsvm::work_stream()));
-    fetch_predictions(d_dec, m, dec_out, winner_out);
+    if (direct.block.host) {
+        TSVM_HIP_CHECK(hipStreamSynchronize(tsvm::work_stream()));
+        memcpy(dec_out, direct.block.host, dec_doubles * sizeof(float_type));
+    } else {
+        fetch_predictions(d_dec, m, dec_out, winner_out);
+    }
     return true;
 }
 
