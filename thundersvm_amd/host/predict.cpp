@@ -12,22 +12,23 @@ using tsvm::abi_check;
 using tsvm::DeviceBuffer;
 
 struct SvmModel::PredictPlan {
+    DeviceBuffer<char> arrays;      // all of the following, uploaded together
     // for both paths
-    DeviceBuffer<float_type> rho;
+    const float_type *rho = nullptr;
     // unfused path: the reference's arrays as they are
-    DeviceBuffer<int> sv_start, sv_count;
-    DeviceBuffer<float_type> coef;
+    const int *sv_start = nullptr, *sv_count = nullptr;
+    const float_type *coef = nullptr;
     // fused path: every class's support vectors start on a multiple of 128 columns
     int stride = 0;                 // coefficients stored per padded column (0: the fused kernels do not take this model)
     int64_t n_pad = 0;
     std::vector<int> class_tile;    // [n_classes + 1]: first 128-column tile of every class
-    DeviceBuffer<int> col_map;      // padded column -> support vector
-    DeviceBuffer<float_type> coef_t;   // [n_pad][stride]
+    const int *col_map = nullptr;   // padded column -> support vector
+    const float_type *coef_t = nullptr;   // [n_pad][stride]
     bool many_features = false;     // the 128 x 128 tile kernel (d > 128, no indicator columns)
     // chunk table of the last call, rebuilt when the batch size changes
     mutable size_t chunks_for_m = 0;
     mutable int n_chunks = 0;
-    mutable DeviceBuffer<int> chunks, class_chunk_start;
+    mutable DeviceBuffer<int> chunk_table;   // class_chunk_start, then the chunks
     // the batch rows' indicator masks (grown as needed, kept between calls)
     mutable DeviceBuffer<uint64_t> mask_a;
     mutable DeviceBuffer<int> mask_max;
@@ -44,10 +45,8 @@ const SvmModel::PredictPlan &SvmModel::predict_plan() const {
     const size_t T = sv->size();
     std::vector<int> sv_start(n_classes, 0);
     for (int c = 1; c < n_classes; ++c) sv_start[c] = sv_start[c - 1] + n_sv[c - 1];
-    P.rho.upload(rho);
-    P.sv_start.upload(sv_start);
-    P.sv_count.upload(n_sv);
-    P.coef.upload(coef);
+    std::vector<int> col_map;
+    std::vector<float_type> coef_t;
     const bool masks = R.dense && R.ind_first >= 0;
     const int d = masks ? R.ind_first : (int) R.n_features;
     P.stride = R.dense ? tsvm_predict_nc_stride(n_classes, d, masks) : 0;
@@ -56,8 +55,8 @@ const SvmModel::PredictPlan &SvmModel::predict_plan() const {
         P.class_tile.assign(n_classes + 1, 0);
         for (int c = 0; c < n_classes; ++c) P.class_tile[c + 1] = P.class_tile[c] + (n_sv[c] + 127) / 128;
         P.n_pad = (int64_t) P.class_tile[n_classes] * 128;
-        std::vector<int> col_map((size_t) P.n_pad, 0);
-        std::vector<float_type> coef_t((size_t) P.n_pad * P.stride, 0.0);
+        col_map.assign((size_t) P.n_pad, 0);
+        coef_t.assign((size_t) P.n_pad * P.stride, 0.0);
         const int km1 = n_classes - 1;
         for (int c = 0; c < n_classes; ++c) {
             const int64_t p0 = (int64_t) P.class_tile[c] * 128, p1 = (int64_t) P.class_tile[c + 1] * 128;
@@ -72,9 +71,28 @@ const SvmModel::PredictPlan &SvmModel::predict_plan() const {
                 }
             }
         }
-        P.col_map.upload(col_map);
-        P.coef_t.upload(coef_t);
     }
+    // (eight arrays, most of them some bytes: uploads of 10 us each)
+    std::vector<tsvm::HostStaging::Part> parts;
+    size_t at = 0;
+    auto add = [&](const void *from, size_t bytes) {
+        const size_t here = at;
+        if (bytes) parts.push_back({from, bytes, at});
+        at = (at + bytes + 255) / 256 * 256;
+        return here;
+    };
+    const size_t rho_at = add(rho.data(), rho.size() * sizeof(float_type)), start_at = add(sv_start.data(), sv_start.size() * sizeof(int));
+    const size_t count_at = add(n_sv.data(), n_sv.size() * sizeof(int)), coef_at = add(coef.data(), coef.size() * sizeof(float_type));
+    const size_t map_at = add(col_map.data(), col_map.size() * sizeof(int)), coef_t_at = add(coef_t.data(), coef_t.size() * sizeof(float_type));
+    P.arrays.resize(std::max<size_t>(at, 256));
+    tsvm::HostStaging::instance().upload(P.arrays.data(), parts, tsvm::work_stream());
+    const char *const base = P.arrays.data();
+    P.rho = (const float_type *) (base + rho_at);
+    P.sv_start = (const int *) (base + start_at);
+    P.sv_count = (const int *) (base + count_at);
+    P.coef = (const float_type *) (base + coef_at);
+    P.col_map = (const int *) (base + map_at);
+    P.coef_t = (const float_type *) (base + coef_t_at);
     predict_plan_ = plan;
     return *predict_plan_;
 }
@@ -112,8 +130,8 @@ bool SvmModel::predict_batch_fused(const PredictPlan &P, const kernel_type *a, i
         std::vector<int> chunks, ccs;
         build_chunks(P.class_tile, P.many_features ? (m + 127) / 128 : (m + 63) / 64, P.many_features ? 8 : 32, chunks, ccs);
         P.n_chunks = (int) chunks.size() / 2;
-        P.chunks.upload(chunks);
-        P.class_chunk_start.upload(ccs);
+        ccs.insert(ccs.end(), chunks.begin(), chunks.end());
+        P.chunk_table.upload(ccs);
         P.chunks_for_m = m;
     }
     if (plan_masks) {
@@ -139,8 +157,8 @@ bool SvmModel::predict_batch_fused(const PredictPlan &P, const kernel_type *a, i
     // (a batch row may set more indicator columns than any support vector does: its matches are bounded by the
     // support vectors' count all the same)
     abi_check(tsvm_predict_dec_values_dense(R.x.data(), R.ld, d, R.self_dot.data(), plan_masks ? R.ind_mask.data() : nullptr,
-                                            P.col_map.data(), P.n_pad, P.coef_t.data(), P.chunks.data(), P.n_chunks,
-                                            P.class_chunk_start.data(), P.rho.data(), n_classes, a, lda, (int64_t) m, sd_a,
+                                            P.col_map, P.n_pad, P.coef_t, P.chunk_table.data() + n_classes + 1, P.n_chunks,
+                                            P.chunk_table.data(), P.rho, n_classes, a, lda, (int64_t) m, sd_a,
                                             plan_masks ? P.mask_a.data() : nullptr, R.ind_max_ones, (int) param.kernel_type,
                                             param.gamma, param.coef0, param.degree, d_part, d_dec, tsvm::work_stream()));
     if (direct.block.host) {
@@ -209,7 +227,7 @@ void SvmModel::predict_dec_values(const RowStore &rows, std::vector<float_type> 
             d_dec.resize(bmax * n_binary_models + (winner ? (bmax + 1) / 2 : 0));
         }
         k_mat.get_rows(rows, b0, bm, d_k, ldk);
-        abi_check(tsvm_sum_kernel_values(P.coef.data(), (int) T, P.sv_start.data(), P.sv_count.data(), P.rho.data(), d_k,
+        abi_check(tsvm_sum_kernel_values(P.coef, (int) T, P.sv_start, P.sv_count, P.rho, d_k,
                                          k_mat.row_type(), ldk, d_dec.data(), n_classes, (int64_t) bm, tsvm::work_stream()));
         fetch_predictions(d_dec.data(), bm, dec.data() + b0 * n_binary_models, winner ? winner->data() + b0 : nullptr);
     }
