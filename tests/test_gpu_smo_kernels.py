@@ -287,6 +287,56 @@ def test_c_smo_solve_with_scores_that_a_float_cannot_tell_apart(ws, scores):
 
 
 @pytest.mark.parametrize("ws", [257, 512, 513, 1024])
+@pytest.mark.parametrize("scores", ["apart by 1e-9", "pairs of equals", "sides alike", "negative a", "f times 1e25", "f times 1e-25", "a full side",
+                                    "a = 0 now and then", "row of the other side"])
+def test_nu_smo_solve_with_scores_that_a_float_cannot_tell_apart(ws, scores):
+    """As for the C variant, and over two sides: equal scores of both, a side that has no first index, and a score's a that is
+    row ip's while the step's is row in's.  The same steps as the oracle's, bit for bit."""
+    rng = np.random.default_rng(ws + len(scores))
+    n, Cc, eps, max_iter = ws + 6, 2.0, 1e-3, 60
+    y = np.where(np.arange(n) % 2 == 0, 1, -1).astype(np.int32)
+    b = rng.random((n, n))
+    k = 0.2 * (b + b.T)
+    f = 0.3 * rng.standard_normal(n)
+    alpha = np.where(rng.random(n) < 0.7, Cc * rng.random(n), 0.0)
+    if scores.startswith("apart by"):
+        small = float(scores.split()[-1])
+        k, f = small * k, np.where(rng.random(n) < 0.5, 1.0, -1.0) * (1 + small * rng.random(n))
+    elif scores in ("pairs of equals", "sides alike"):
+        apart = 1 if scores == "sides alike" else 2     # (neighbours have different labels)
+        first = np.flatnonzero(np.arange(n) % (2 * apart) < apart)[: n // (2 * apart)]
+        first = first[first + apart < n]
+        k[first + apart] = k[first]
+        k[:, first + apart] = k[:, first]
+        f[first + apart], alpha[first + apart] = f[first], alpha[first]
+    elif scores == "negative a":
+        k = 4.0 * k
+    elif scores.startswith("f times"):
+        f = f * float(scores.split()[-1])
+        eps = 1e-30 if scores.endswith("-25") else eps
+    elif scores == "a full side":
+        alpha[y > 0] = Cc
+    elif scores == "a = 0 now and then":
+        same = rng.random((n, n)) < 0.05
+        k[same | same.T] = 1.0
+    np.fill_diagonal(k, 1.0)
+    if scores == "row of the other side":
+        k = k * np.where(y > 0, 1.0, 0.01)[:, None] * np.where(y > 0, 1.0, 0.01)[None, :]
+    ws_ids = rng.permutation(n)[:ws].astype(np.int32)
+    k_rows, diag = np.ascontiguousarray(k[ws_ids]), np.ascontiguousarray(np.diag(k))
+    a_want, ad_want, diff_want = O.nu_smo_solve(y, f, alpha, ws_ids, Cc, k_rows, diag, n, eps, max_iter)
+    y_d, f_d, ws_d, dg_d, a_d, k_d = G.dev(y), G.dev(f), G.dev(ws_ids), G.dev(diag), G.dev(alpha), G.dev(k_rows)
+    ad_d = torch.zeros(ws, dtype=torch.float64, device="cuda")
+    diff_d = torch.zeros(2, dtype=torch.float64, device="cuda")
+    wsp = torch.empty(capi.kernel_lib().tsvm_smo_solve_workspace(ws), dtype=torch.uint8, device="cuda")
+    capi.call("tsvm_nu_smo_solve", G.ptr(y_d), G.ptr(f_d), G.ptr(a_d), G.ptr(ad_d), G.ptr(ws_d), ws, Cc, G.ptr(k_d), capi.ROW_F64, None,
+              n, G.ptr(dg_d), eps, G.ptr(diff_d), max_iter, G.ptr(wsp), G.stream())
+    assert G.host(diff_d)[0] == diff_want[0]
+    assert np.array_equal(G.host(a_d), a_want, equal_nan=True)
+    assert np.array_equal(G.host(ad_d), ad_want, equal_nan=True)
+
+
+@pytest.mark.parametrize("ws", [257, 512, 513, 1024])
 @pytest.mark.parametrize("diagonal", ["2^126.5", "2^130", "2^-342", "0"])
 def test_c_smo_solve_with_diagonals_out_of_float_range(ws, diagonal):
     """A few instances whose K_ii + K_tt - 2 K_it is no normal float, or has no normal float as its reciprocal, and whose f
