@@ -46,6 +46,29 @@ def test_one_class_and_regression(n, svm_type, kernel_type, ties):
     T._compare(d, d, make_param(svm_type=svm_type, kernel_type=kernel_type, gamma=0.2, C=3.0, nu=0.3, p=0.05, max_iter=40), trace=0)
 
 
+@pytest.mark.parametrize("n", [257, 300, 512, 513, 900])
+@pytest.mark.parametrize("what", ["almost repeated", "a few repeated", "a near zero", "all scores alike"])
+def test_scores_that_a_float_cannot_tell_apart(n, what):
+    """From 257 slots on the second index is chosen by scores rounded to float: where these are too close to one another, equal,
+    or out of range, or where the first index is a tie, the working set's order and doubles decide as for the oracle."""
+    x, rng = _rows(n, 2000 + n, False)
+    gamma = 0.2
+    if what == "almost repeated":
+        x[n // 2:] = x[:n - n // 2] * (1 + 1e-6 * rng.standard_normal((n - n // 2, 1)))
+    elif what == "a few repeated":
+        twice = rng.permutation(n)[:n // 8 * 2]
+        x[twice[::2]] = x[twice[1::2]]
+    elif what == "a near zero":
+        gamma = 1e-9
+    else:
+        x = (x > 0) * np.float32(1)      # 64 different instances
+    y = (x[:, 0] + 0.5 * x[:, 1] * x[:, 2] > 0.1).astype(np.float64)
+    flip = rng.permutation(n)[:n // 10]
+    y[flip] = 1 - y[flip]
+    d = D.from_dense(x, y)
+    T._compare(d, d, make_param(svm_type=0, kernel_type=2, gamma=gamma, C=3.0, max_iter=40), trace=0)
+
+
 @pytest.mark.parametrize("sizes", [(5, 40, 90), (300, 200, 700, 900), (8, 8, 1100)])
 def test_class_pairs_from_one_matrix(sizes):
     """Small pairs side by side, in the second and third case next to pairs that are too large; the same pairs one at a time."""

@@ -196,3 +196,83 @@ __device__ __forceinline__ unsigned set_member_bits(unsigned m, int tid, int t, 
 struct __align__(16) SvBound {
     double hi, lo;
 };
+
+struct __align__(16) SvStep {   // f_t - up and K_ii + K_tt - 2 K_it of a candidate for j2
+    double b, a;
+};
+
+// One row's (sixteen lanes') best and second-best score, rounded to float.
+struct __align__(16) SvScore {
+    float best, second;
+    int at, go;
+};
+// best and second of a row in all its lanes.  Four instructions per step, ordered so that none of the DPP operands is
+// younger than two instructions: no wait states between the steps, so the second-best costs hardly more than the waits would.
+// LANES: of so many lanes that hold different ones.
+template <int LANES = 16>
+__device__ __forceinline__ void row_best_two(float &best, float &second) {
+    static_assert(LANES == 4 || LANES == 8 || LANES == 16, "a quad, half a row, a row");
+    float t;
+#define SV_BEST_STEP(CTRL)                                          \
+    "v_min_f32_dpp %2, %0, %0 " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_max_f32_dpp %0, %0, %0 " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_max_f32_dpp %1, %1, %1 " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_max_f32 %1, %1, %2\n\t"
+    if constexpr (LANES == 4)
+        asm("s_nop 1\n\t" SV_BEST_STEP("quad_perm:[1,0,3,2]") SV_BEST_STEP("quad_perm:[2,3,0,1]") : "+v"(best), "+v"(second), "=&v"(t));
+    else if constexpr (LANES == 8)
+        asm("s_nop 1\n\t" SV_BEST_STEP("quad_perm:[1,0,3,2]") SV_BEST_STEP("quad_perm:[2,3,0,1]") SV_BEST_STEP("row_half_mirror")
+            : "+v"(best), "+v"(second), "=&v"(t));
+    else
+        asm("s_nop 1\n\t" SV_BEST_STEP("quad_perm:[1,0,3,2]") SV_BEST_STEP("quad_perm:[2,3,0,1]") SV_BEST_STEP("row_half_mirror")
+                SV_BEST_STEP("row_mirror")
+            : "+v"(best), "+v"(second), "=&v"(t));
+#undef SV_BEST_STEP
+}
+// The smallest of a row's x, in all its lanes.
+__device__ __forceinline__ double row_min(double x) {
+    x = fmin_f64(x, dpp_f64<TSVM_DPP_XOR1>(x));
+    x = fmin_f64(x, dpp_f64<TSVM_DPP_XOR2>(x));
+    x = fmin_f64(x, dpp_f64<TSVM_DPP_HALF_MIRROR>(x));
+    return fmin_f64(x, dpp_f64<TSVM_DPP_MIRROR>(x));
+}
+
+// The smallest of a row's E * 16 values; m and at are every lane's own smallest and its first element (as wave_argmin in
+// smo_local.h, whose first four steps these are).
+// TWICE: and `twice` has the lanes whose own smallest occurs more than once.
+template <int E, bool TWICE = false>
+__device__ __forceinline__ double row_first_min(const double (&x)[E], int base, double &m, int &at, uint64_t *twice = nullptr) {
+    m = x[0];
+#pragma unroll
+    for (int e = 1; e < E; ++e) m = fmin_f64(m, x[e]);
+    SV_PIN;
+    uint64_t has[E];
+#pragma unroll
+    for (int e = 0; e < (TWICE ? E : E - 1); ++e) asm volatile("v_cmp_eq_f64_e64 %0, %1, %2" : "=s"(has[e]) : "v"(x[e]), "v"(m));
+    SV_PIN;
+    double r = fmin_f64(m, dpp_f64<TSVM_DPP_XOR1>(m));
+    SV_PIN;
+    at = base + E - 1;
+    if constexpr (E > 2) asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(at) : "v"(at), "v"(base + E - 2), "s"(has[E - 2]));
+    if constexpr (E > 3) asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(at) : "v"(at), "v"(base + E - 3), "s"(has[E - 3]));
+    SV_PIN;
+    r = fmin_f64(r, dpp_f64<TSVM_DPP_XOR2>(r));
+    SV_PIN;
+    if constexpr (E > 1) asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(at) : "v"(at), "v"(base), "s"(has[0]));
+    SV_PIN;
+    if constexpr (TWICE) {
+        uint64_t more = 0, one = has[0];
+#pragma unroll
+        for (int e = 1; e < E; ++e) {
+            more |= one & has[e];
+            one |= has[e];
+        }
+        *twice = more;
+    }
+    r = fmin_f64(r, dpp_f64<TSVM_DPP_HALF_MIRROR>(r));
+    return fmin_f64(r, dpp_f64<TSVM_DPP_MIRROR>(r));
+}
+
+// Bounds of what c_smo_iterate_rounded (smo_solve.hip) decides: the least |up|, and from where on an a is too large (as float bits).
+#define SV_UP_LEAST_HI 0x3b600000   // 2^-73
+#define SV_A_BITS 0x7e800000         // 2^126

@@ -92,7 +92,9 @@ struct SmallShared {
     uint64_t total[2][W];               // per-wavefront counts of a scan
     double red[4][W];
     int event[2], first_x[2], first_y[2], n_list;
-    SvCand ci[W], cj[W], ci2[W], cj2[W];
+    SvCand ci[4 * W], ci2[W], cj[W], cj2[W];
+    SvScore score[4 * W];
+    SvStep step[4 * W];
 };
 
 // sort_f + select_working_set (smo_kernel.cpp:321-332, csmosolver.cpp:123-165, nusmosolver.cpp:48-118): writes k picks to
@@ -319,15 +321,15 @@ __device__ __forceinline__ void ss_load(SS_GLOBAL(TB) *row, TB (&out)[E]) {
 }
 
 // The local solver: c_smo_iterate of smo_solve.hip (and nu_smo_solve_kernel) with the instances in place of a gathered
-// working set.  Returns the steps taken; the new alpha is in sh.z.  NONE and no_score: as there.
-template <int E, int W, bool NU, bool NONE, typename TB>
-__device__ __forceinline__ int ss_local(SmallShared<E, W> &sh, const SmallMap &map, SS_GLOBAL(TB) *K, int64_t ld, int col, const double (&kd)[E], double (&f)[E],
-                        unsigned member, double Cp, double Cn, double local_eps, int max_iter, bool &no_score) {
+// working set.  Takes up to `left` steps (ALL: as many as there are), counted in n_iter; returns whether the solve has ended.  The new alpha is in sh.z.
+// NONE and no_score: as there.
+template <int E, int W, bool NU, bool NONE, bool ALL, typename TB>
+__device__ __forceinline__ bool ss_local(SmallShared<E, W> &sh, const SmallMap &map, SS_GLOBAL(TB) *K, int64_t ld, int col, const double (&kd)[E], double (&f)[E],
+                        unsigned &member, double Cp, double Cn, double local_eps, int max_iter, bool &no_score, int &n_iter, int left) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     constexpr int NP = NU ? 2 : 1;   // pairs of sides
     SvCand *const ci[2] = {sh.ci, sh.ci2}, *const cj[2] = {sh.cj, sh.cj2};
     const int first_slot = sh.ws[0];
-    int n_iter = 0;
     bool go_on;
     double taken = -__builtin_inf();   // the score of the step
     int worst = 0;
@@ -437,9 +439,122 @@ __device__ __forceinline__ int ss_local(SmallShared<E, W> &sh, const SmallMap &m
 #pragma unroll
         for (int e = 0; e < E; ++e) f[e] = __builtin_fma(-l, (double) kJ[e] - (double) (second ? kI[NP - 1][e] : kI[0][e]), f[e]);
         n_iter += go_on;
-    } while (go_on);
-    if (!NONE) no_score = __builtin_amdgcn_readfirstlane(worst) >= SV_NONE_HI;
-    return n_iter;
+    } while (go_on && (ALL || --left > 0));
+    if (!NONE) no_score |= __builtin_amdgcn_readfirstlane(go_on ? imax_sel(worst, __double2hiint(taken)) : worst) >= SV_NONE_HI;
+    return !go_on;
+}
+
+// The C variant's iterations with j2 chosen by b^2/a rounded to float, as long as that decides: c_smo_iterate_rounded of
+// smo_solve.hip, with its proof.  What the working set's order would decide, equal values of f included, is left to ss_local.
+// 963 instances, 1,000 steps: 2.82 -> 2.72 thousand cycles a step; cross-validation of 1203x13 2.31 -> 2.26 ms.
+template <int E, int W, typename TB>
+__device__ __forceinline__ bool ss_rounded(SmallShared<E, W> &sh, const SmallMap &map, SS_GLOBAL(TB) *K, int64_t ld, int col, const double (&kd)[E],
+                                           double (&f)[E], unsigned &member, double Cp, double Cn, double local_eps, int max_iter, int &n_iter) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int R = 4 * W;   // rows of sixteen lanes
+    uint64_t go;
+    for (;;) {
+        double fu[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) fu[e] = keep_or_none<0>(member << (31 - 2 * e), f[e]);
+        double m;
+        int at;
+        uint64_t twice;
+        const double r = row_first_min<E, true>(fu, tid * E, m, at, &twice);
+        const uint64_t mine_is = __builtin_amdgcn_ballot_w64(m == r), has = mine_is | 0x8000800080008000ull;
+        const uint64_t first = has & ~(has - 0x0001000100010001ull);
+        const uint64_t equal = mine_is & (twice | ~first);   // a row that has one has its smallest more than once
+        const int tie = (int) ((unsigned) (equal >> (lane & 48)) & 0xffffu);
+        publish(sh.ci + (tid >> 4), first, m, at, tie);
+        lds_barrier();
+        const SvCand c = sh.ci[lane & (R - 1)];
+        const double up = row_min(c.v);
+        const uint64_t has_up = __builtin_amdgcn_ballot_w64(c.v == up), up_rows = has_up & ((1ull << R) - 1);
+        const uint64_t ties = (up_rows & (up_rows - 1)) | (up_rows & __builtin_amdgcn_ballot_w64(c.flag != 0));
+        const int i = __builtin_amdgcn_readlane(c.at, __builtin_ctzll(has_up)) & (64 * E * W - 1);
+        TB kI[E];
+        ss_load<E, TB>(K + (unsigned) map.row(i) * (unsigned) ld + col, kI);
+        SV_PIN_MEMORY;
+        const double kd_i = sh.kd[i], z_i = sh.z[wave][i];
+        const SvBound bound_i = map.bound(i, Cp, Cn);
+        double part[E], b[E], b_max = -__builtin_inf();
+        float b32[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            part[e] = kd_i + kd[e];
+            b[e] = keep_or_none<1>(member << (30 - 2 * e), -up + f[e]);
+            b_max = fmax_f64(b_max, b[e]);
+            b32[e] = __builtin_fmaxf((float) b[e], 0.0f);
+        }
+        const int violates = __builtin_amdgcn_ballot_w64(!(b_max < local_eps)) != 0;
+        double up_i = bound_i.hi - z_i;
+        asm("" : "+v"(up_i));
+        int a_max = (__double2hiint(up) & 0x7fffffff) < SV_UP_LEAST_HI || ties != 0 ? 0x7f800000 : 0;   // (as the bits of a float)
+        asm("" : "+v"(a_max));
+        SV_PIN;
+        double aIJ[E];
+        float q[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            aIJ[e] = __builtin_fma(-2.0, (double) kI[e], part[e]);
+            const float a32 = (float) aIJ[e];
+            a_max = __float_as_int(a32) > a_max ? __float_as_int(a32) : a_max;
+            q[e] = __builtin_fmaxf(b32[e] * (b32[e] * __builtin_amdgcn_rcpf(a32)), 0x1p-80f);
+        }
+        float best = q[0], second = 0x1p-80f;
+#pragma unroll
+        for (int e = 1; e < E; ++e) {
+            second = __builtin_fmaxf(second, __builtin_fminf(best, q[e]));
+            best = __builtin_fmaxf(best, q[e]);
+        }
+        at = tid * E + E - 1;
+        double b_at = b[E - 1], a_at = aIJ[E - 1];
+#pragma unroll
+        for (int e = E - 2; e >= 0; --e) {
+            const bool is = q[e] == best;
+            at = is ? tid * E + e : at;
+            b_at = is ? b[e] : b_at;
+            a_at = is ? aIJ[e] : a_at;
+        }
+        second = a_max < SV_A_BITS ? second : __builtin_inff();
+        const float mine = best;
+        row_best_two(best, second);
+        const uint64_t who = __builtin_amdgcn_ballot_w64(mine == best);   // (several only if nothing will be decided)
+        publish(sh.score + (tid >> 4), who, best, second, at, violates);
+        publish(sh.step + (tid >> 4), who, b_at, a_at);
+        lds_barrier();
+        const SvScore s = sh.score[lane & (R - 1)];
+        const SvStep step = sh.step[lane & (R - 1)];
+        best = s.best;
+        second = s.second;
+        row_best_two<R>(best, second);
+        const int row = __builtin_ctzll(__builtin_amdgcn_ballot_w64(s.best == best));
+        const int j2 = __builtin_amdgcn_readlane(s.at, row) & (64 * E * W - 1);
+        TB kJ[E];
+        ss_load<E, TB>(K + (unsigned) map.row(j2) * (unsigned) ld + col, kJ);
+        SV_PIN_MEMORY;
+        const double z_j = sh.z[wave][j2];
+        const SvBound bound_j = map.bound(j2, Cp, Cn);
+        SV_PIN;
+        const double steps = step.b / step.a;   // (every row's)
+        const double q2 = readlane_f64(steps, row);
+        SV_PIN;
+        go = __builtin_amdgcn_ballot_w64(s.go != 0);
+        const uint64_t sure = __builtin_amdgcn_ballot_w64(second < best * (1.0f - 0x1p-19f)) & __builtin_amdgcn_ballot_w64(best < 0x1p80f);
+        const uint64_t on = n_iter > max_iter ? 0 : go & sure;
+        if (on == 0) break;
+        const double l = fmin_f64(up_i, fmin_f64(z_j - bound_j.lo, q2));
+        const double nz_i = z_i + l, nz_j = z_j - l;
+        auto bits = [&](double z, const SvBound &bound) { return (z < bound.hi ? 1u : 0u) | (z > bound.lo ? 2u : 0u); };
+        member = set_member_bits<E, 2>(member, tid, i, bits(nz_i, bound_i));
+        member = set_member_bits<E, 2>(member, tid, j2, bits(nz_j, bound_j));
+        write_by_lane0(1, &sh.z[wave][i], nz_i, &sh.z[wave][j2], nz_j);
+        SV_PIN;
+#pragma unroll
+        for (int e = 0; e < E; ++e) f[e] = __builtin_fma(-l, (double) kJ[e] - (double) kI[e], f[e]);
+        ++n_iter;
+    }
+    return go == 0 || n_iter > max_iter;
 }
 
 // f[j] -= sum over the n_list listed rows (coefficients sh.f, rows in sh.k) in order (smo_kernel.cpp:300-319)
@@ -502,6 +617,8 @@ __global__ __launch_bounds__(64 * W) void smo_small_kernel(const tsvm_small_prob
                                                            tsvm_small_state *states, int *ws_all, double *alpha_all, double *f_all, double eps,
                                                            int out_max_iter, int start) {
     constexpr int N = 64 * E * W;
+    // (a lone wavefront's second reduction is six steps in registers; by rows and LDS, rounded: 3 pairs of 100 0.37 -> 0.42 ms)
+    constexpr bool ROUNDED = !NU && W > 1;
     __shared__ SmallShared<E, W> sh;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     if ((int) blockIdx.x >= n_problems) {
@@ -667,7 +784,20 @@ __global__ __launch_bounds__(64 * W) void smo_small_kernel(const tsvm_small_prob
         bool no_score = !__builtin_amdgcn_readfirstlane(local_eps > 0.0 ? 1 : 0);
         int steps = 0;
         if (!no_score) {
-            steps = ss_local<E, W, NU, false, TB>(sh, map, K, ld, col, kd, fl, member, P.Cp, P.Cn, local_eps, P.max_iter, no_score);
+            unsigned now = member;
+            if constexpr (ROUNDED) {
+                bool done;
+                int stretch = 4;   // (as in c_smo_solve_kernel)
+                do {
+                    const int before = steps;
+                    done = ss_rounded<E, W, TB>(sh, map, K, ld, col, kd, fl, now, P.Cp, P.Cn, local_eps, P.max_iter, steps);
+                    if (done) break;
+                    stretch = steps - before > stretch ? 4 : stretch < 1024 ? 8 * stretch : stretch;
+                    done = ss_local<E, W, NU, false, false, TB>(sh, map, K, ld, col, kd, fl, now, P.Cp, P.Cn, local_eps, P.max_iter, no_score, steps, stretch);
+                } while (!done && !no_score);
+            } else {
+                ss_local<E, W, NU, false, true, TB>(sh, map, K, ld, col, kd, fl, now, P.Cp, P.Cn, local_eps, P.max_iter, no_score, steps, 0);
+            }
             if (no_score) {   // once more from the start
                 __syncthreads();
 #pragma unroll
@@ -679,7 +809,10 @@ __global__ __launch_bounds__(64 * W) void smo_small_kernel(const tsvm_small_prob
                 __syncthreads();
             }
         }
-        if (no_score) steps = ss_local<E, W, NU, true, TB>(sh, map, K, ld, col, kd, fl, member, P.Cp, P.Cn, local_eps, P.max_iter, no_score);
+        if (no_score) {
+            steps = 0;
+            ss_local<E, W, NU, true, true, TB>(sh, map, K, ld, col, kd, fl, member, P.Cp, P.Cn, local_eps, P.max_iter, no_score, steps, 0);
+        }
         inner_here += steps;
         if (!NU) local_iter += steps;   // (the nu variant reports none, smo_kernel.cpp:283)
         // alpha_diff of the working set, in its order: -(new - old) * y

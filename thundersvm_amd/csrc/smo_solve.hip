@@ -224,9 +224,6 @@ struct SvShared {
 };
 
 // What c_smo_solve keeps.
-struct __align__(16) SvStep {   // f_t - up and K_ii + K_tt - 2 K_it of a candidate for j2
-    double b, a;
-};
 template <int N, int W>
 struct SvState {
     double kd[N];
@@ -335,59 +332,6 @@ __device__ __forceinline__ bool c_smo_iterate(SvState<E * 64 * W, W> &sh, SvCand
     return !go_on;
 }
 
-// One row's (sixteen lanes') best and second-best score, rounded to float.
-struct __align__(16) SvScore {
-    float best, second;
-    int at, go;
-};
-// best and second of a row in all its lanes.  Four instructions per step, ordered so that none of the DPP operands is
-// younger than two instructions: no wait states between the steps, so the second-best costs hardly more than the waits would.
-__device__ __forceinline__ void row_best_two(float &best, float &second) {
-    float t;
-#define SV_BEST_STEP(CTRL)                                          \
-    "v_min_f32_dpp %2, %0, %0 " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
-    "v_max_f32_dpp %0, %0, %0 " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
-    "v_max_f32_dpp %1, %1, %1 " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
-    "v_max_f32 %1, %1, %2\n\t"
-    asm("s_nop 1\n\t" SV_BEST_STEP("quad_perm:[1,0,3,2]") SV_BEST_STEP("quad_perm:[2,3,0,1]") SV_BEST_STEP("row_half_mirror")
-            SV_BEST_STEP("row_mirror")
-        : "+v"(best), "+v"(second), "=&v"(t));
-#undef SV_BEST_STEP
-}
-// The smallest of a row's x, in all its lanes.
-__device__ __forceinline__ double row_min(double x) {
-    x = fmin_f64(x, dpp_f64<TSVM_DPP_XOR1>(x));
-    x = fmin_f64(x, dpp_f64<TSVM_DPP_XOR2>(x));
-    x = fmin_f64(x, dpp_f64<TSVM_DPP_HALF_MIRROR>(x));
-    return fmin_f64(x, dpp_f64<TSVM_DPP_MIRROR>(x));
-}
-
-// The smallest of a row's E * 16 values; m and at are every lane's own smallest and its first element (as wave_argmin in
-// smo_local.h, whose first four steps these are).
-template <int E>
-__device__ __forceinline__ double row_first_min(const double (&x)[E], int base, double &m, int &at) {
-    m = x[0];
-#pragma unroll
-    for (int e = 1; e < E; ++e) m = fmin_f64(m, x[e]);
-    SV_PIN;
-    uint64_t has[E];
-#pragma unroll
-    for (int e = 0; e < E - 1; ++e) asm volatile("v_cmp_eq_f64_e64 %0, %1, %2" : "=s"(has[e]) : "v"(x[e]), "v"(m));
-    SV_PIN;
-    double r = fmin_f64(m, dpp_f64<TSVM_DPP_XOR1>(m));
-    SV_PIN;
-    at = base + E - 1;
-    if constexpr (E > 2) asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(at) : "v"(at), "v"(base + E - 2), "s"(has[E - 2]));
-    if constexpr (E > 3) asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(at) : "v"(at), "v"(base + E - 3), "s"(has[E - 3]));
-    SV_PIN;
-    r = fmin_f64(r, dpp_f64<TSVM_DPP_XOR2>(r));
-    SV_PIN;
-    asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(at) : "v"(at), "v"(base), "s"(has[0]));
-    SV_PIN;
-    r = fmin_f64(r, dpp_f64<TSVM_DPP_HALF_MIRROR>(r));
-    return fmin_f64(r, dpp_f64<TSVM_DPP_MIRROR>(r));
-}
-
 // The same iterations for four wavefronts with j2 chosen by b^2/a rounded to float, as long as that decides: the largest
 // score has to beat the second by more than both can be off, and to be in float's range.  A score is off by at most
 // 4.2e-7 (b, a, the two products 2^-24 each, b twice; the reciprocal 2^-23), so a lead of 2^-19 = 1.9e-6 is proof, and the
@@ -402,8 +346,6 @@ __device__ __forceinline__ double row_first_min(const double (&x)[E], int base, 
 // Rows of sixteen lanes are reduced by DPP and publish themselves, and after the barrier every lane reads one of the
 // sixteen rows and four more steps compare them: the same eight steps as over a wavefront and then over four of them, without
 // the way through the scalar unit in between.
-#define SV_UP_LEAST_HI 0x3b600000   // 2^-73
-#define SV_A_BITS 0x7e800000         // 2^126
 template <int E, int LDK, typename TB>
 __device__ __forceinline__ bool c_smo_iterate_rounded(SvState<E * 256, 4> &sh, SvCand *s_i, SvScore *s_j, SvStep *s_step, int ws, const TB *kws,
                                                       const double (&kd)[E], double (&f)[E], unsigned &in_up, unsigned &in_low,
