@@ -181,6 +181,11 @@ int tsvm_get_rows_csr_sliced(const int *ell_col, const void *ell_val, int val_ty
  * CSR: rows idx[0..m) of (val, col, row_ptr) written to (out_val, out_col) at the offsets out_ptr[0..m], which the
  * caller has computed from the row lengths. */
 int tsvm_gather_rows_f64(const double *x, int64_t ld, const int *idx, int64_t m, double *out, tsvm_stream stream);
+/* The dense gather together with out_self_dot[r] = self_dot[idx[r]], out_mask[r] = mask[idx[r]] (mask may be NULL) and the
+ * diagonal of tsvm_kernel_diag for the gathered rows (diag may be NULL; then the kernel's parameters are not read). */
+int tsvm_subset_rows_dense(const double *x, int64_t ld, const int *idx, int64_t m, const double *self_dot, const uint64_t *mask,
+                           double *out, double *out_self_dot, uint64_t *out_mask, int kernel_type, double gamma, double coef0, int degree,
+                           double *diag, tsvm_stream stream);
 int tsvm_csr_gather_rows(const double *val, const int *col, const int64_t *row_ptr, const int *idx, int64_t m,
                          const int64_t *out_ptr, double *out_val, int *out_col, tsvm_stream stream);
 

@@ -389,6 +389,27 @@ def test_row_subsets_on_device():
     assert np.array_equal(G.host(oval), sub.val) and np.array_equal(G.host(ocol), sub.col)
 
 
+@pytest.mark.parametrize("n,ld,m", [(1, 8, 1), (40, 8, 64), (300, 24, 255), (300, 784, 257), (70, 8, 33)])
+@pytest.mark.parametrize("kernel", range(5))
+@pytest.mark.parametrize("masks", [False, True])
+def test_subset_rows_dense(n, ld, m, kernel, masks):
+    """Rows, self dot products, masks and the diagonal of a subset (rows named twice included) in one launch."""
+    rng = np.random.default_rng(n + ld + m)
+    x, dot, mask = rng.standard_normal((n, ld)), rng.random(n) * 3, rng.integers(1 << 62, size=n)
+    idx = rng.integers(n, size=m).astype(np.int32)
+    x_d, dot_d, mask_d, idx_d = G.dev(x), G.dev(dot), G.dev(mask), G.dev(idx)
+    out, odot, odiag = (torch.full(s, 7.0, dtype=torch.float64, device="cuda") for s in ((m, ld), (m,), (m + 1,)))
+    omask = torch.full((m,), 7, dtype=torch.int64, device="cuda")
+    capi.call("tsvm_subset_rows_dense", G.ptr(x_d), ld, G.ptr(idx_d), m, G.ptr(dot_d), G.ptr(mask_d) if masks else None, G.ptr(out), G.ptr(odot),
+              G.ptr(omask), kernel, 0.3, 0.5, 3, G.ptr(odiag) if m != 33 else None, G.stream())
+    assert np.array_equal(G.host(out), x[idx]) and np.array_equal(G.host(odot), dot[idx])
+    assert np.array_equal(G.host(omask), mask[idx] if masks else np.full(m, 7))
+    want = torch.full((m + 1,), 7.0, dtype=torch.float64, device="cuda")
+    if m != 33:
+        capi.call("tsvm_kernel_diag", G.ptr(odot), m, kernel, 0.3, 0.5, 3, G.ptr(want), G.stream())
+    assert np.array_equal(G.host(odiag), G.host(want))
+
+
 @pytest.mark.parametrize("n,d,m", [(131072 + 77, 7, 133), (140001, 54, 512), (131072, 90, 200), (135000, 200, 1024), (133333, 16, 65),
                                    (131072 + 5, 24, 100), (131333, 33, 70)])   # one, two, three and more K tiles of 16 columns
 def test_dense_rbf_many_columns_few_features(n, d, m):

@@ -796,18 +796,39 @@ __global__ void dense_self_dot_kernel(const double *__restrict__ x, int64_t ld, 
     self_dot[i] = s;
 }
 
+__device__ __forceinline__ double diag_of(double self_dot, const KernelParam &kp) {
+    switch (kp.kernel_type) {
+        case TSVM_RBF:
+        case TSVM_PRECOMPUTED: return 1.0;
+        case TSVM_LINEAR: return self_dot;
+        default: return tsvm_epilogue(self_dot, 0.0, 0.0, kp, TSVM_EXP2F_TAB);
+    }
+}
+
 __global__ void kernel_diag_kernel(const double *__restrict__ self_dot, int64_t n, KernelParam kp,
                                    double *__restrict__ diag) {
     const int64_t i = blockIdx.x * (int64_t) blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double v;
-    switch (kp.kernel_type) {
-        case TSVM_RBF:
-        case TSVM_PRECOMPUTED: v = 1.0; break;
-        case TSVM_LINEAR: v = self_dot[i]; break;
-        default: v = tsvm_epilogue(self_dot[i], 0.0, 0.0, kp, TSVM_EXP2F_TAB); break;
+    if (i < n) diag[i] = diag_of(self_dot[i], kp);
+}
+
+// gather_rows_f64_kernel together with what else there is one of per row: the self dot product, the indicator mask (if any)
+// and the diagonal (if wanted), by the thread of a row's first vector.  Bound by its launch: as launches of their
+// own the four cost a training of 150x4 0.346 ms (now 0.298) and a cross-validation of 1203x13 in five folds 2.37 (now 2.25).
+__global__ void subset_rows_dense_kernel(const v4d *__restrict__ x, int64_t ld4, const int *__restrict__ idx, int64_t m,
+                                         const double *__restrict__ self_dot, const uint64_t *__restrict__ mask, v4d *__restrict__ out,
+                                         double *__restrict__ out_dot, uint64_t *__restrict__ out_mask, double *__restrict__ diag,
+                                         KernelParam kp) {
+    const int64_t total = m * ld4;
+    for (int64_t e = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (int64_t) gridDim.x * blockDim.x) {
+        const int64_t r = e / ld4, c = e % ld4, from = idx[r];
+        out[e] = x[from * ld4 + c];
+        if (c == 0) {
+            const double dot = self_dot[from];
+            out_dot[r] = dot;
+            if (mask) out_mask[r] = mask[from];
+            if (diag) diag[r] = diag_of(dot, kp);
+        }
     }
-    diag[i] = v;
 }
 
 // Column statistics of the data rows: counts[c] = number of entries in column c (dense layout: non-zero values; CSR:
@@ -1344,6 +1365,23 @@ int tsvm_gather_rows_f64(const double *x, int64_t ld, const int *idx, int64_t m,
     const int64_t total = m * (ld / 4);
     const unsigned grid = (unsigned) std::min<int64_t>((total + 255) / 256, 65536);
     hipLaunchKernelGGL(gather_rows_f64_kernel, dim3(grid), dim3(256), 0, tsvm_s(stream), (const v4d *) x, ld / 4, idx, m, (v4d *) out);
+    TSVM_LAUNCH_CHECK();
+    return 0;
+}
+
+int tsvm_subset_rows_dense(const double *x, int64_t ld, const int *idx, int64_t m, const double *self_dot, const uint64_t *mask,
+                           double *out, double *out_self_dot, uint64_t *out_mask, int kernel_type, double gamma, double coef0, int degree,
+                           double *diag, tsvm_stream stream) {
+    TSVM_REQUIRE(x && idx && out && self_dot && out_self_dot && m >= 0 && ld > 0 && ld % 4 == 0, "tsvm_subset_rows_dense: bad argument");
+    TSVM_REQUIRE(((uintptr_t) x % 32 == 0) && ((uintptr_t) out % 32 == 0), "tsvm_subset_rows_dense: x and out must be 32-byte aligned");
+    TSVM_REQUIRE(!mask || out_mask, "tsvm_subset_rows_dense: masks without an output");
+    TSVM_REQUIRE(!diag || (kernel_type >= 0 && kernel_type <= 4), "tsvm_subset_rows_dense: unknown kernel type %d", kernel_type);
+    if (m == 0) return 0;
+    const int64_t total = m * (ld / 4);
+    const unsigned grid = (unsigned) std::min<int64_t>((total + 255) / 256, 65536);
+    KernelParam kp{kernel_type, degree, gamma, coef0};
+    hipLaunchKernelGGL(subset_rows_dense_kernel, dim3(grid), dim3(256), 0, tsvm_s(stream), (const v4d *) x, ld / 4, idx, m, self_dot, mask,
+                       (v4d *) out, out_self_dot, out_mask, diag, kp);
     TSVM_LAUNCH_CHECK();
     return 0;
 }

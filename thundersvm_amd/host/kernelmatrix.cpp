@@ -506,7 +506,7 @@ void DeviceRows::build_sliced() {
     sliced_lds = need;
 }
 
-std::shared_ptr<DeviceRows> DeviceRows::subset(const DeviceRows &base, const int *rows, size_t n_rows) {
+std::shared_ptr<DeviceRows> DeviceRows::subset(const DeviceRows &base, const int *rows, size_t n_rows, const SvmParam *param, kernel_type *diag) {
     auto out = std::make_shared<DeviceRows>();
     DeviceRows &r = *out;
     r.n = n_rows;
@@ -518,19 +518,23 @@ std::shared_ptr<DeviceRows> DeviceRows::subset(const DeviceRows &base, const int
     tsvm::DeviceBuffer<int> d_rows(n_rows);
     d_rows.upload(rows, n_rows);
     r.self_dot.resize(n_rows);
-    abi_check(tsvm_gather_f64(base.self_dot.data(), d_rows.data(), (int) n_rows, r.self_dot.data(), tsvm::work_stream()));
     if (base.dense) {
         r.x.resize(n_rows * (size_t) r.ld);
-        abi_check(tsvm_gather_rows_f64(base.x.data(), base.ld, d_rows.data(), (int64_t) n_rows, r.x.data(), tsvm::work_stream()));
         r.nnz = n_rows ? base.nnz / std::max<size_t>(base.n, 1) * n_rows : 0;   // estimate, informational only
         if (base.ind_first >= 0) {   // indicator columns of all rows are indicator columns of a subset (masks move as 8-byte words)
             r.ind_first = base.ind_first;
             r.ind_max_ones = base.ind_max_ones;
             r.ind_mask.resize(n_rows);
-            abi_check(tsvm_gather_f64(reinterpret_cast<const double *>(base.ind_mask.data()), d_rows.data(), (int) n_rows,
-                                      reinterpret_cast<double *>(r.ind_mask.data()), tsvm::work_stream()));
         }
+        const SvmParam kernel = param ? *param : SvmParam();
+        abi_check(tsvm_subset_rows_dense(base.x.data(), base.ld, d_rows.data(), (int64_t) n_rows, base.self_dot.data(),
+                                         r.ind_first >= 0 ? base.ind_mask.data() : nullptr, r.x.data(), r.self_dot.data(), r.ind_mask.data(),
+                                         (int) kernel.kernel_type, kernel.gamma, kernel.coef0, kernel.degree, diag, tsvm::work_stream()));
     } else {
+        abi_check(tsvm_gather_f64(base.self_dot.data(), d_rows.data(), (int) n_rows, r.self_dot.data(), tsvm::work_stream()));
+        if (diag)
+            abi_check(tsvm_kernel_diag(r.self_dot.data(), (int64_t) n_rows, (int) param->kernel_type, param->gamma, param->coef0,
+                                       param->degree, diag, tsvm::work_stream()));
         r.host_row_ptr.assign(n_rows + 1, 0);
         for (size_t i = 0; i < n_rows; ++i)
             r.host_row_ptr[i + 1] = r.host_row_ptr[i] + base.host_row_ptr[rows[i] + 1] - base.host_row_ptr[rows[i]];
@@ -600,19 +604,22 @@ KernelMatrix::KernelMatrix(const RowStore &rows, SvmParam param) : param(param) 
 KernelMatrix::KernelMatrix(const DataSet &dataset, const int *rows, size_t n_rows, SvmParam param, int repeat)
     : param(param) {
     std::shared_ptr<DeviceRows> all = DeviceRows::of(dataset);
-    rows_ = rows ? DeviceRows::subset(*all, rows, n_rows) : all;
-    finish(repeat);
+    if (rows) diag_.resize(n_rows * repeat);
+    rows_ = rows ? DeviceRows::subset(*all, rows, n_rows, &this->param, diag_.data()) : all;
+    finish(repeat, rows != nullptr);
 }
 
 // diag from the self dot products (kernelmatrix.cpp:225-247).  With repeat > 1 the reference stacks the
 // same rows several times (the 2n-row problem of SVR, svr.cpp:14-15); here the rows are stored once and
 // only the diagonal, which the solver kernels index by instance id, is replicated.
-void KernelMatrix::finish(int repeat) {
+void KernelMatrix::finish(int repeat, bool have_diag) {
     n_unique_ = rows_->n;
     repeat_ = repeat;
-    diag_.resize(n_unique_ * repeat_);
-    abi_check(tsvm_kernel_diag(rows_->self_dot.data(), (int64_t) n_unique_, (int) param.kernel_type, param.gamma, param.coef0,
-                               param.degree, diag_.data(), tsvm::work_stream()));
+    if (!have_diag) {
+        diag_.resize(n_unique_ * repeat_);
+        abi_check(tsvm_kernel_diag(rows_->self_dot.data(), (int64_t) n_unique_, (int) param.kernel_type, param.gamma, param.coef0,
+                                   param.degree, diag_.data(), tsvm::work_stream()));
+    }
     for (int rep = 1; rep < repeat_; ++rep)
         TSVM_HIP_CHECK(hipMemcpyAsync(diag_.data() + rep * n_unique_, diag_.data(), n_unique_ * sizeof(kernel_type),
                                       hipMemcpyDeviceToDevice, tsvm::work_stream()));

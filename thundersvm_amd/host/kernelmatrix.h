@@ -57,8 +57,10 @@ struct DeviceRows {
 
     // all rows of `rows`, uploaded
     static std::shared_ptr<DeviceRows> from_host(const RowStore &rows);
-    // rows[0..n_rows) of `base`, gathered on the device; keeps base's layout and feature count
-    static std::shared_ptr<DeviceRows> subset(const DeviceRows &base, const int *rows, size_t n_rows);
+    // rows[0..n_rows) of `base`, gathered on the device; keeps base's layout and feature count.  diag: the diagonal of the
+    // kernel `param` comes with them (n_rows entries)
+    static std::shared_ptr<DeviceRows> subset(const DeviceRows &base, const int *rows, size_t n_rows, const SvmParam *param = nullptr,
+                                              kernel_type *diag = nullptr);
     // the device copy of all instances of a DataSet, built on first use and kept with the DataSet
     static std::shared_ptr<DeviceRows> of(const DataSet &dataset);
 };
@@ -120,7 +122,7 @@ public:
     size_t entries_at_most() const;   // stored entries, or more
 
 private:
-    void finish(int repeat);
+    void finish(int repeat, bool have_diag = false);
 
     SvmParam param;
     std::shared_ptr<DeviceRows> rows_;
