@@ -182,10 +182,13 @@ int tsvm_get_rows_csr_sliced(const int *ell_col, const void *ell_val, int val_ty
  * caller has computed from the row lengths. */
 int tsvm_gather_rows_f64(const double *x, int64_t ld, const int *idx, int64_t m, double *out, tsvm_stream stream);
 /* The dense gather together with out_self_dot[r] = self_dot[idx[r]], out_mask[r] = mask[idx[r]] (mask may be NULL) and the
- * diagonal of tsvm_kernel_diag for the gathered rows (diag may be NULL; then the kernel's parameters are not read). */
+ * diagonal of tsvm_kernel_diag for the gathered rows (diag may be NULL; then the kernel's parameters are not read).
+ * ids_on_host != 0: idx lies in host memory and has been read when the call returns; at most
+ * tsvm_subset_rows_dense_max_ids(rows of x) ids. */
+int tsvm_subset_rows_dense_max_ids(int64_t n);
 int tsvm_subset_rows_dense(const double *x, int64_t ld, const int *idx, int64_t m, const double *self_dot, const uint64_t *mask,
                            double *out, double *out_self_dot, uint64_t *out_mask, int kernel_type, double gamma, double coef0, int degree,
-                           double *diag, tsvm_stream stream);
+                           double *diag, int ids_on_host, tsvm_stream stream);
 int tsvm_csr_gather_rows(const double *val, const int *col, const int64_t *row_ptr, const int *idx, int64_t m,
                          const int64_t *out_ptr, double *out_val, int *out_col, tsvm_stream stream);
 

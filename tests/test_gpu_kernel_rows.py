@@ -389,19 +389,23 @@ def test_row_subsets_on_device():
     assert np.array_equal(G.host(oval), sub.val) and np.array_equal(G.host(ocol), sub.col)
 
 
-@pytest.mark.parametrize("n,ld,m", [(1, 8, 1), (40, 8, 64), (300, 24, 255), (300, 784, 257), (70, 8, 33)])
+@pytest.mark.parametrize("n,ld,m", [(1, 8, 1), (40, 8, 64), (300, 24, 255), (300, 784, 257), (70, 8, 33), (65536, 8, 1920)])
 @pytest.mark.parametrize("kernel", range(5))
 @pytest.mark.parametrize("masks", [False, True])
-def test_subset_rows_dense(n, ld, m, kernel, masks):
-    """Rows, self dot products, masks and the diagonal of a subset (rows named twice included) in one launch."""
+@pytest.mark.parametrize("on_host", [False, True])
+def test_subset_rows_dense(n, ld, m, kernel, masks, on_host):
+    """Rows, self dot products, masks and the diagonal of a subset (rows named twice included) in one launch, its ids in
+    device memory or among the kernel's arguments."""
+    assert capi.kernel_lib().tsvm_subset_rows_dense_max_ids(65536) >= 1920 and capi.kernel_lib().tsvm_subset_rows_dense_max_ids(65537) == 0
     rng = np.random.default_rng(n + ld + m)
     x, dot, mask = rng.standard_normal((n, ld)), rng.random(n) * 3, rng.integers(1 << 62, size=n)
     idx = rng.integers(n, size=m).astype(np.int32)
+    idx[-1] = n - 1
     x_d, dot_d, mask_d, idx_d = G.dev(x), G.dev(dot), G.dev(mask), G.dev(idx)
     out, odot, odiag = (torch.full(s, 7.0, dtype=torch.float64, device="cuda") for s in ((m, ld), (m,), (m + 1,)))
     omask = torch.full((m,), 7, dtype=torch.int64, device="cuda")
-    capi.call("tsvm_subset_rows_dense", G.ptr(x_d), ld, G.ptr(idx_d), m, G.ptr(dot_d), G.ptr(mask_d) if masks else None, G.ptr(out), G.ptr(odot),
-              G.ptr(omask), kernel, 0.3, 0.5, 3, G.ptr(odiag) if m != 33 else None, G.stream())
+    capi.call("tsvm_subset_rows_dense", G.ptr(x_d), ld, idx.ctypes.data if on_host else G.ptr(idx_d), m, G.ptr(dot_d), G.ptr(mask_d) if masks else None, G.ptr(out), G.ptr(odot),
+              G.ptr(omask), kernel, 0.3, 0.5, 3, G.ptr(odiag) if m != 33 else None, int(on_host), G.stream())
     assert np.array_equal(G.host(out), x[idx]) and np.array_equal(G.host(odot), dot[idx])
     assert np.array_equal(G.host(omask), mask[idx] if masks else np.full(m, 7))
     want = torch.full((m + 1,), 7.0, dtype=torch.float64, device="cuda")

@@ -44,7 +44,8 @@ SIGNATURES = {
     "tsvm_get_rows_csr_sliced": (_int, [_p, _p, _int, _p, _i64, _p, _p, _p, _p, _p, _int, _p, _int, _int, _int, _dbl, _dbl, _int,
                                         _p, _int, _p, _i64, _p]),
     "tsvm_fold_ids": (_int, [_p, _int, _int, _p, _p]),
-    "tsvm_subset_rows_dense": (_int, [_p, _i64, _p, _i64, _p, _p, _p, _p, _p, _int, _dbl, _dbl, _int, _p, _p]),
+    "tsvm_subset_rows_dense_max_ids": (_int, [_i64]),
+    "tsvm_subset_rows_dense": (_int, [_p, _i64, _p, _i64, _p, _p, _p, _p, _p, _int, _dbl, _dbl, _int, _p, _int, _p]),
     "tsvm_gather_rows_f64": (_int, [_p, _i64, _p, _i64, _p, _p]),
     "tsvm_csr_gather_rows": (_int, [_p, _p, _p, _p, _i64, _p, _p, _p, _p]),
     "tsvm_gather_f64": (_int, [_p, _p, _int, _p, _p]),

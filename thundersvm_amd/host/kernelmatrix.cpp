@@ -515,8 +515,9 @@ std::shared_ptr<DeviceRows> DeviceRows::subset(const DeviceRows &base, const int
     r.values_fit_float = base.values_fit_float;
     r.values_finite = base.values_finite;
     r.ld = base.ld;
-    tsvm::DeviceBuffer<int> d_rows(n_rows);
-    d_rows.upload(rows, n_rows);
+    const bool by_value = base.dense && n_rows <= (size_t) tsvm_subset_rows_dense_max_ids((int64_t) base.n);
+    tsvm::DeviceBuffer<int> d_rows(by_value ? 0 : n_rows);
+    d_rows.upload(rows, d_rows.size());
     r.self_dot.resize(n_rows);
     if (base.dense) {
         r.x.resize(n_rows * (size_t) r.ld);
@@ -527,9 +528,9 @@ std::shared_ptr<DeviceRows> DeviceRows::subset(const DeviceRows &base, const int
             r.ind_mask.resize(n_rows);
         }
         const SvmParam kernel = param ? *param : SvmParam();
-        abi_check(tsvm_subset_rows_dense(base.x.data(), base.ld, d_rows.data(), (int64_t) n_rows, base.self_dot.data(),
+        abi_check(tsvm_subset_rows_dense(base.x.data(), base.ld, by_value ? rows : d_rows.data(), (int64_t) n_rows, base.self_dot.data(),
                                          r.ind_first >= 0 ? base.ind_mask.data() : nullptr, r.x.data(), r.self_dot.data(), r.ind_mask.data(),
-                                         (int) kernel.kernel_type, kernel.gamma, kernel.coef0, kernel.degree, diag, tsvm::work_stream()));
+                                         (int) kernel.kernel_type, kernel.gamma, kernel.coef0, kernel.degree, diag, by_value, tsvm::work_stream()));
     } else {
         abi_check(tsvm_gather_f64(base.self_dot.data(), d_rows.data(), (int) n_rows, r.self_dot.data(), tsvm::work_stream()));
         if (diag)
