@@ -683,6 +683,9 @@ struct SolveTask::Impl {
         timer.end(stats.ms_get_rows);
     }
 
+    double seconds_per_value() const { return 2.0 * ((k_mat.n_features() + 15) / 16 * 16) / 6.6e13; }   // of a dense row, on the whole chip
+    double rows_seconds() const { return seconds_per_value() * (double) last_rows_computed * n_u; }
+
     void enqueue_block() {
         timer.begin();
         on_one_stream = !split || (alone && all_cached);
@@ -690,10 +693,8 @@ struct SolveTask::Impl {
         // same cost per value; the block plus the solver's ~0.4 ms has to fit into the time of the rows.)
         block_on_solver_cus = false;
         if (!on_one_stream && alone && block_first && k_mat.dense_layout() && !all_cached) {
-            const double per_value = 2.0 * ((k_mat.n_features() + 15) / 16 * 16) / 6.6e13;   // seconds on the whole chip
-            const double t_block = per_value * 32.0 * 0.56 * ws_size * (double) ws_size;   // on 8 of 256 CUs; 72 of its 128 tiles
-            const double t_rows = per_value * (double) last_rows_computed * n_u;
-            block_on_solver_cus = t_block + 0.4e-3 <= t_rows;
+            const double t_block = seconds_per_value() * 32.0 * 0.56 * ws_size * (double) ws_size;   // on 8 of 256 CUs; 72 of its 128 tiles
+            block_on_solver_cus = t_block + 0.4e-3 <= rows_seconds();
         }
         if (caching && all_cached) {
             abi_check(tsvm_smo_gather_block_by_id(k_rows, row_type, d_slot_of.data(), ld, ws_u(), ws_size, d_kws.data(), row_type,
@@ -748,6 +749,12 @@ struct SolveTask::Impl {
     }
 
     void enqueue_update() {
+        // The rows that stream through the solver's L2 beside it take the block's place there: it is read once more behind them
+        // (epsilon-SVR 40000x90, rows for 42 us beside a solver of 310: 88.4 -> 81.3 ms), unless they take about as long
+        // as the solver (20000x784, 340 us: 50.2 -> 50.3) or other lanes' rows come through at any time (7 classes
+        // 300000x54: 844 -> 857).
+        if (!on_one_stream && alone && k_mat.dense_layout() && !all_cached && last_rows_computed > 0 && rows_seconds() < 0.1e-3)
+            abi_check(tsvm_smo_warm_block(d_kws.data(), row_type, ws_size, solver_xcd, d_gate.data() + 3, sa));
         if (!on_one_stream) TSVM_HIP_CHECK(hipStreamWaitEvent(sa, solved.event, 0));   // alpha_diff, alpha and diff come from the solver
         if (select_ahead && fuse_select) {
             // the next selection's first pass over the instances rides on update_f's last one
