@@ -389,6 +389,28 @@ def test_row_subsets_on_device():
     assert np.array_equal(G.host(oval), sub.val) and np.array_equal(G.host(ocol), sub.col)
 
 
+@pytest.mark.parametrize("m", [1, 63, 64, 65, 128, 129, 1000, 1024])
+@pytest.mark.parametrize("d", [0, 1, 4, 7, 31, 32, 33, 64, 65, 97])
+@pytest.mark.parametrize("kernel,row_type", [(0, capi.ROW_F64), (1, capi.ROW_F32), (2, capi.ROW_F32), (2, capi.ROW_F64), (3, capi.ROW_F32)])
+def test_symmetric_block(m, d, kernel, row_type):
+    """K(idx, idx) when both sides are the same rows, computed from the tiles on and above the diagonal: the bits of the general
+    call (which takes the same indices from another array), nothing written beside the block, rows named twice included."""
+    rng = np.random.default_rng(m + 100 * d)
+    n, ld, ldo = max(8, m // 2), (d + 7) // 8 * 8 or 8, m + 3
+    x = np.zeros((n, ld))
+    x[:, :d] = rng.standard_normal((n, d))
+    idx = rng.integers(n, size=m).astype(np.int32)
+    x_d, i_d, i2_d, sd = G.dev(x), G.dev(idx), G.dev(idx), G.dev((x * x).sum(axis=1))
+    t = torch.float32 if row_type == capi.ROW_F32 else torch.float64
+    got, want = torch.full((m, ldo), 7.0, dtype=t, device="cuda"), torch.full((m, ldo), 7.0, dtype=t, device="cuda")
+    for ids, out in ((i_d, got), (i2_d, want)):
+        capi.call("tsvm_get_rows_dense", G.ptr(x_d), ld, G.ptr(i_d), m, d, G.ptr(sd), G.ptr(x_d), ld, G.ptr(ids), m, G.ptr(sd), kernel, 0.1, 0.5, 3,
+                  G.ptr(out), row_type, None, ldo, G.stream())
+    got, want = G.host(got), G.host(want)
+    assert np.array_equal(got[:, :m], want[:, :m]) and np.array_equal(got[:, :m], got[:, :m].T)
+    assert (got[:, m:] == 7.0).all()
+
+
 @pytest.mark.parametrize("n,ld,m", [(1, 8, 1), (40, 8, 64), (300, 24, 255), (300, 784, 257), (70, 8, 33), (65536, 8, 1920)])
 @pytest.mark.parametrize("kernel", range(5))
 @pytest.mark.parametrize("masks", [False, True])

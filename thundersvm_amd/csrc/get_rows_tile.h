@@ -42,17 +42,13 @@ template <int TI> struct GrShape {
 };
 
 // One (32*TI) x 128 output tile at rows i0.., columns j0..; As / Bs hold GrShape<TI>::LDS_DOUBLES doubles each.
-// SYM: the output is a symmetric matrix (same rows on both sides, out[i][j] at i*ldo + j): every value is also
-// written to its mirror position, so that tiles below the diagonal need no workgroup.  kappa(a, b) and kappa(b, a)
-// are the same bits: the products of the dot product commute, their order does not change, and the self dot
-// products enter as a commutative sum.
 //
 // FUSE: prediction.  The tile's values are not stored: each is multiplied by its column's fz_nc coefficients
 // (fz_coef[column * fz_nc + c], columns counted before x_idx maps them to rows of x) and the products are summed
 // over the tile's columns into fz_red[(wj * BM + row) * fz_nc + c] in LDS, wj = 0, 1 being the two wavefront
 // columns of the workgroup (each location has exactly one writer, so tiles called one after the other accumulate
 // without atomics).  n must be a multiple of 128 and x_idx given; rows beyond m produce sums nobody reads.
-template <int KT, int TI, typename TO, bool SYM = false, bool FUSE = false>
+template <int KT, int TI, typename TO, bool FUSE = false>
 __device__ __forceinline__ void get_rows_tile(
     const double *__restrict__ x, int64_t ldx, const int *__restrict__ x_idx, int64_t n, int d,
     const double *__restrict__ sd_x, const double *__restrict__ a, int64_t lda, const int *__restrict__ a_idx, int m,
@@ -230,7 +226,7 @@ __device__ __forceinline__ void get_rows_tile(
     // epilogue + store.  Interior tiles take the unguarded path; edge tiles test every element.
     // (Sixteen lanes write 64 or 128 consecutive bytes of an output row: streamed past the L2 when those runs are
     // whole 64-byte pieces of memory, which depends on where the rows start; partial pieces the L2 has to merge.)
-    const bool stream_out = !SYM && ((ldo * (int64_t) sizeof(TO)) % 64 == 0) && ((uintptr_t) out % 64 == 0);
+    const bool stream_out = ((ldo * (int64_t) sizeof(TO)) % 64 == 0) && ((uintptr_t) out % 64 == 0);
     if (full) {
 #pragma unroll
         for (int ti = 0; ti < TI; ++ti) {
@@ -240,14 +236,8 @@ __device__ __forceinline__ void get_rows_tile(
 #pragma unroll
                 for (int tj = 0; tj < 4; ++tj) {
                     const TO val = tsvm_epilogue_as<TO>(acc[ti][tj][v], sdi[ti * 4 + v], sdj[tj], kp, exp_tab);
-                    if (SYM) {   // the solver's block: read again at once
-                        orow[tj * 16] = val;
-                        out[(int64_t) (jb + tj * 16) * ldo + (i0 + wi * (16 * TI) + ti * 16 + 4 * v + lk)] = val;
-                    } else if (stream_out) {
-                        store_streaming(orow + tj * 16, val);
-                    } else {
-                        orow[tj * 16] = val;
-                    }
+                    if (stream_out) store_streaming(orow + tj * 16, val);
+                    else orow[tj * 16] = val;
                 }
             }
         }
@@ -261,15 +251,7 @@ __device__ __forceinline__ void get_rows_tile(
                 TO *orow = out + orow_off[ti * 4 + v] + jb;
 #pragma unroll
                 for (int tj = 0; tj < 4; ++tj)
-                    if (jb + tj * 16 < n) {
-                        const TO val = tsvm_epilogue_as<TO>(acc[ti][tj][v], sdi[ti * 4 + v], sdj[tj], kp, exp_tab);
-                        if (SYM) {
-                            orow[tj * 16] = val;
-                            out[(int64_t) (jb + tj * 16) * ldo + i] = val;
-                        } else {
-                            orow[tj * 16] = val;
-                        }
-                    }
+                    if (jb + tj * 16 < n) orow[tj * 16] = tsvm_epilogue_as<TO>(acc[ti][tj][v], sdi[ti * 4 + v], sdj[tj], kp, exp_tab);
             }
         }
     }

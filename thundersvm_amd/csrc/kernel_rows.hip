@@ -350,27 +350,117 @@ __global__ void indicator_masks_kernel(const double *__restrict__ x, int64_t ld,
     if ((threadIdx.x & 63) == 0 && ones > 0) atomicMax(max_ones, ones);
 }
 
-// The m x m block K(x_idx[r], x_idx[t]) (a == x, a_idx == x_idx, rows written in place): tiles that lie below the
-// diagonal are filled by the mirror writes of the others and get no workgroup.  Column tile j (128 wide) needs the
-// 64-row tiles 0 .. 2j+1, so workgroup c works on column tile j = the largest j with j(j+1) <= c, row tile
-// c - j(j+1); dealt out in this order, every XCD gets the same share of the work.
+// The m x m block K(x_idx[r], x_idx[t]) (a == x, a_idx == x_idx, rows written in place): every value is also written to its
+// mirror position, so that tiles below the diagonal need no workgroup.  kappa(a, b) and kappa(b, a) are the same bits: the
+// products of the dot product commute, their order does not change, and the self dot products enter as a commutative sum.
+//
+// Bound by one workgroup's walk through the features (the solver's block has 1,024 instances, fewer tiles than there are CUs):
+// tiles of 64 x 64, 136 of them on or above the diagonal, by eight wavefronts of 16 x 32, two per SIMD so that one's LDS reads
+// and staging run beside the other's MFMAs.  The values go through LDS, so that the tile and its mirror image are both stored in
+// runs of 64.  1,024 instances of 784 / 90 / 32 features: 40.1 / 11.0 / 9.7 us.  Tiles of 64 x 128 by four wavefronts, 72 of
+// them: 68.4 / 16.0 / 13.3; 64 x 64 by four wavefronts 51.5 / 13.3 / 11.7, with a barrier on either side of the staging instead of two
+// sets of staged columns 43.9 / 11.4 / 9.7.  Column tile j needs the row tiles 0 .. j: workgroup c works on column tile j = the largest j
+// with j(j+1)/2 <= c, row tile c - j(j+1)/2; dealt out in this order, every XCD gets the same share of the work.
+#define SYM_B 64     // rows and columns of a tile
+#define SYM_K 32     // columns of the data staged at a time
+#define SYM_LS 66    // LDS row of a staged column (the staging writes of a wavefront are in all banks)
 template <int KT, typename TO>
-__global__ __launch_bounds__(256, 3) void get_rows_dense_sym_kernel(
+__global__ __launch_bounds__(512) void get_rows_dense_sym_kernel(
     const double *__restrict__ x, int64_t ldx, const int *__restrict__ idx, int m, int d, const double *__restrict__ sd_x,
-    KernelParam kp, TO *__restrict__ out, int64_t ldo, unsigned m_blocks) {
-    __shared__ double As[GrShape<2>::LDS_DOUBLES];
-    __shared__ double Bs[GrShape<2>::LDS_DOUBLES];
+    KernelParam kp_in, TO *__restrict__ out, int64_t ldo) {
+    __shared__ double s_tile[4 * SYM_K * SYM_LS];   // As, Bs twice, and then the values
+    __shared__ double s_sd[2][SYM_B];
     __shared__ uint64_t exp_tab[32];
+    static_assert(SYM_B * (SYM_B + 1) <= 2 * SYM_K * SYM_LS, "the values take the staged columns' place");
+    KernelParam kp = kp_in;
+    kp.kernel_type = KT;
     const int c = (int) blockIdx.x;
-    int jt = (int) ((sqrtf(4.0f * (float) c + 1.0f) - 1.0f) * 0.5f);
-    while (jt > 0 && jt * (jt + 1) > c) --jt;
-    while ((jt + 1) * (jt + 2) <= c) ++jt;
-    const int j0 = jt * GR_BN;
-    const int i0 = (c - jt * (jt + 1)) * GrShape<2>::BM;
-    if (i0 >= m) return;               // (the last column tile has fewer row tiles when m is not a multiple of 128)
-    if (threadIdx.x < 32) exp_tab[threadIdx.x] = TSVM_EXP2F_TAB[threadIdx.x];
+    int jt = (int) ((sqrtf(8.0f * (float) c + 1.0f) - 1.0f) * 0.5f);
+    while (jt > 0 && jt * (jt + 1) / 2 > c) --jt;
+    while ((jt + 1) * (jt + 2) / 2 <= c) ++jt;
+    const int j0 = jt * SYM_B, i0 = (c - jt * (jt + 1) / 2) * SYM_B;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wi = wave >> 1, wj = wave & 1, lrow = lane & 15, lk = lane >> 4;
+    // Sixteen lanes stage the 32 columns of one row, two each.  Rows beyond the last are the last one's copies: what they give is
+    // not stored.
+    typedef double v2d __attribute__((ext_vector_type(2)));
+    const int r_mine = wave * 8 + lk, k_mine = 2 * lrow;
+    const double *pa[2], *pb[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        pa[q] = x + (uint64_t) (uint32_t) idx[min(i0 + r_mine + 4 * q, m - 1)] * (uint32_t) ldx;
+        pb[q] = x + (uint64_t) (uint32_t) idx[min(j0 + r_mine + 4 * q, m - 1)] * (uint32_t) ldx;
+    }
+    v2d ra[2], rb[2];
+    // (rows are padded with zeros to a multiple of eight columns; what would start beyond that re-reads the last two, which are
+    // staged and not multiplied)
+    auto load = [&](int k0) {
+        const int k = min(k0 + k_mine, (int) ldx - 2);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            ra[q] = *(const v2d *) (pa[q] + k);
+            rb[q] = *(const v2d *) (pb[q] + k);
+        }
+    };
+    v4d acc[2];
+#pragma unroll
+    for (int tj = 0; tj < 2; ++tj) acc[tj] = (v4d){0.0, 0.0, 0.0, 0.0};
+    auto mma_step = [&](const double *As, int ks) {
+        const double *const Bs = As + SYM_K * SYM_LS;
+        const int kk = (ks * 4 + lk) * SYM_LS + lrow;
+        const double af = As[kk + wi * 16];
+        double bf[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) bf[t] = Bs[kk + wj * 32 + t * 16];
+#pragma unroll
+        for (int tj = 0; tj < 2; ++tj) acc[tj] = __builtin_amdgcn_mfma_f64_16x16x4f64(af, bf[tj], acc[tj], 0, 0, 0);
+    };
+    if (d > 0) load(0);
+    if (tid < 2 * SYM_B) s_sd[tid >> 6][lane] = sd_x ? sd_x[idx[min((tid >> 6 ? j0 : i0) + lane, m - 1)]] : 0.0;
+    if (tid < 32) exp_tab[tid] = TSVM_EXP2F_TAB[tid];
+    auto stage = [&](double *As) {
+        double *const Bs = As + SYM_K * SYM_LS;
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                As[(k_mine + e) * SYM_LS + r_mine + 4 * q] = ra[q][e];
+                Bs[(k_mine + e) * SYM_LS + r_mine + 4 * q] = rb[q][e];
+            }
+    };
+    // (two sets of staged columns: a wavefront stages the next ones while another still multiplies)
+    double *now = s_tile, *next = s_tile + 2 * SYM_K * SYM_LS;
+    if (d > 0) stage(now);
+    if (d > SYM_K) load(SYM_K);
     __syncthreads();
-    get_rows_tile<KT, 2, TO, true>(x, ldx, idx, m, d, sd_x, x, ldx, idx, m, sd_x, kp, out, nullptr, ldo, i0, j0, As, Bs, exp_tab);
+    int k0 = 0;
+    for (; k0 + SYM_K < d; k0 += SYM_K) {
+#pragma unroll
+        for (int ks = 0; ks < SYM_K / 4; ++ks) mma_step(now, ks);
+        stage(next);
+        if (k0 + 2 * SYM_K < d) load(k0 + 2 * SYM_K);
+        __syncthreads();
+        double *const t = now;
+        now = next;
+        next = t;
+    }
+    for (int ks = 0; ks < (d - k0 + 3) / 4; ++ks) mma_step(now, ks);
+    __syncthreads();
+    TO *const val = (TO *) s_tile;   // [row][column], rows SYM_B + 1 apart
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int r = wi * 16 + 4 * v + lk;
+#pragma unroll
+        for (int tj = 0; tj < 2; ++tj) {
+            const int q = wj * 32 + tj * 16 + lrow;
+            val[r * (SYM_B + 1) + q] = tsvm_epilogue_as<TO>(acc[tj][v], s_sd[0][r], s_sd[1][q], kp, exp_tab);
+        }
+    }
+    __syncthreads();
+    for (int r = wave; r < SYM_B; r += 8) {
+        if (i0 + r < m && j0 + lane < m) out[(int64_t) (i0 + r) * ldo + (j0 + lane)] = val[r * (SYM_B + 1) + lane];
+        if (i0 != j0 && j0 + r < m && i0 + lane < m) out[(int64_t) (j0 + r) * ldo + (i0 + lane)] = val[lane * (SYM_B + 1) + r];
+    }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1076,10 +1166,11 @@ static int get_rows_dense(const double *x, int64_t ldx, const int *x_idx, int64_
     const bool sym = x == a && ldx == lda && x_idx && x_idx == a_idx && n == m && sd_x == sd_a && !out_slots && !m_dev &&
                      ti == 2 && ldo >= n;
     if (sym) {
-        grid = dim3((unsigned) (n_blocks * (n_blocks + 1)));   // column tile j: row tiles 0 .. 2j+1
+        const int64_t tiles = (n + SYM_B - 1) / SYM_B;
+        grid = dim3((unsigned) (tiles * (tiles + 1) / 2));   // column tile j: row tiles 0 .. j
 #define GR_SYM(KTYPE, TO)                                                                                                      \
-    hipLaunchKernelGGL((get_rows_dense_sym_kernel<KTYPE, TO>), grid, block, 0, tsvm_s(stream), x, ldx, x_idx, m, d, sd_x, kp, (TO *) out, \
-                       ldo, m_blocks)
+    hipLaunchKernelGGL((get_rows_dense_sym_kernel<KTYPE, TO>), grid, dim3(512), 0, tsvm_s(stream), x, ldx, x_idx, m, d, sd_x, kp, (TO *) out, \
+                       ldo)
         if (row_type == TSVM_ROW_F32) {
             switch (kernel_type) {
                 case TSVM_POLY: GR_SYM(TSVM_POLY, float); break;

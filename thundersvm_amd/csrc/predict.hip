@@ -333,7 +333,7 @@ __global__ __launch_bounds__(256, 2) void predict_dense_tile_kernel(
     const unsigned chunk = blockIdx.x / m_blocks;
     const int jt0 = chunks[2 * chunk], jt1 = chunks[2 * chunk + 1];
     for (int jt = jt0; jt < jt1; ++jt) {
-        get_rows_tile<KT, 4, double, false, true>(x, ldx, col_map, n_pad, d, sd_x, a, lda, nullptr, m, sd_a, kp, nullptr, nullptr,
+        get_rows_tile<KT, 4, double, true>(x, ldx, col_map, n_pad, d, sd_x, a, lda, nullptr, m, sd_a, kp, nullptr, nullptr,
                                                   0, i0, jt * GR_BN, As, Bs, exp_tab, coef_t, nc, red);
         __syncthreads();   // the tile's staging memory is free for the next tile; the sums are complete at the end
     }

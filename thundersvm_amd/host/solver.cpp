@@ -693,7 +693,7 @@ struct SolveTask::Impl {
         // same cost per value; the block plus the solver's ~0.4 ms has to fit into the time of the rows.)
         block_on_solver_cus = false;
         if (!on_one_stream && alone && block_first && k_mat.dense_layout() && !all_cached) {
-            const double t_block = seconds_per_value() * 32.0 * 0.56 * ws_size * (double) ws_size;   // on 8 of 256 CUs; 72 of its 128 tiles
+            const double t_block = seconds_per_value() * 32.0 * 0.53 * ws_size * (double) ws_size;   // on 8 of 256 CUs; 136 of its 256 tiles
             block_on_solver_cus = t_block + 0.4e-3 <= rows_seconds();
         }
         if (caching && all_cached) {
