@@ -7,7 +7,7 @@
 // problem another 600 us of set-up, and one host thread fed all pairs.  Here an outer iteration's selection is a sort in LDS
 // of some microseconds, the kernel matrix is computed once for all pairs (it holds every pair's rows and columns), the host
 // takes no part between the upload and the result, and the pairs run side by side.  Whole
-// training calls: 45 pairs of 360 instances in 64 columns 31 -> 1.3 ms, 3 pairs of 100 in 4 columns 2.4 -> 0.4 ms.
+// training calls: 45 pairs of 360 instances in 64 columns 31 -> 1.1 ms, 3 pairs of 100 in 4 columns 2.4 -> 0.35 ms.
 //
 // Shape.  At most 1,024 instances (above that a workgroup's share of update_f and of the selection outlasts what the
 // chip-wide kernels take, and their launches no longer matter): W wavefronts of E neighbouring instances per thread.
