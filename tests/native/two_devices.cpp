@@ -12,6 +12,8 @@
 
 static int g_current = 0, g_failures = 0;
 static bool g_hung = false;                   // events are never reached
+static hipError_t g_stream_state = hipSuccess;   // what waiting for a stream says
+static int g_stream_waits = 0;
 static std::map<const void *, int> g_owner;   // device of every live block, stream and event
 
 static void expect(bool ok, const char *what) {
@@ -38,6 +40,8 @@ hipError_t hipMalloc(void **p, size_t bytes) { return make(p, bytes); }
 hipError_t hipFree(void *p) { return drop(p); }
 hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) { return make(p, bytes); }
 hipError_t hipHostFree(void *p) { return drop(p); }
+hipError_t hipHostGetDevicePointer(void **d, void *h, unsigned) { *d = h; return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { ++g_stream_waits; return g_stream_state; }
 hipError_t hipDeviceSynchronize(void) { return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return make(s, 1); }
 hipError_t hipStreamDestroy(hipStream_t s) { return drop(s); }
@@ -73,7 +77,27 @@ static void blocks(bool idle) {
     expect(g_owner.at(d.data()) == 0, "a buffer of device 0 got device 1's memory after a move");
 }
 
+// A block that kernels write a result into: waited for, left by an exception, and left on a stream that reports an error.
+static void result_blocks() {
+    const void *first = nullptr;
+    for (int step = 0; step < 4; ++step) {
+        g_stream_waits = 0;
+        g_stream_state = step == 2 ? hipErrorLaunchFailure : hipSuccess;
+        try {
+            tsvm::ResultBlock b(nullptr);
+            if (step == 0) first = b.dev();
+            expect((b.dev() == first) == (step < 3), "a result's block is not the one that is free");
+            if (step == 0) expect(b.wait() == first, "a result on the host");
+            else throw std::runtime_error("a launch that was refused");
+        } catch (const std::runtime_error &) {
+        }
+        expect(step == 3 || g_stream_waits == 1, "a block went back without anybody having waited for its stream");
+    }
+}
+
 int main() {
+    result_blocks();
+    g_stream_state = hipSuccess;
     blocks(true);
     tsvm::DevicePool::instance().flush();
     blocks(false);

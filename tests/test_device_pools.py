@@ -1,4 +1,4 @@
-"""The host layer's pools of device blocks and events with two devices, and the limit of a download's wait:
+"""The host layer's pools of device blocks, events and result blocks with two devices, and the limit of a download's wait:
 tests/native/two_devices.cpp, a program with stand-ins for the HIP calls.  Host only."""
 import os
 import subprocess

@@ -68,6 +68,27 @@ struct PinnedBlock {
 };
 PinnedBlock take_pinned_block();
 void give_pinned_block(const PinnedBlock &b);
+// Such a block for a result that kernels on `stream` write into it.  Left by an exception before anybody has waited for the
+// stream, it goes back to the pool only behind the kernels, and not at all if the stream cannot be waited for: whoever takes
+// it next may be a solve that reads the solver's words from it.
+class ResultBlock {
+public:
+    explicit ResultBlock(hipStream_t stream) : block_(take_pinned_block()), stream_(stream) {}
+    ResultBlock(const ResultBlock &) = delete;
+    ResultBlock &operator=(const ResultBlock &) = delete;
+    ~ResultBlock() { if (arrived_ || hipStreamSynchronize(stream_) == hipSuccess) give_pinned_block(block_); }
+    char *dev() const { return block_.dev; }
+    const char *wait() {   // the result, on the host
+        TSVM_HIP_CHECK(hipStreamSynchronize(stream_));
+        arrived_ = true;
+        return block_.host;
+    }
+
+private:
+    PinnedBlock block_;
+    hipStream_t stream_;
+    bool arrived_ = false;
+};
 struct DeviceEvent {
     hipEvent_t event = nullptr;
     int device = -1;

@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 
 #include "models.h"
 
@@ -146,13 +147,10 @@ bool SvmModel::predict_batch_fused(const PredictPlan &P, const kernel_type *a, i
     float_type *d_part = (float_type *) tsvm::RowArena::instance().acquire((part_doubles + dec_doubles) * sizeof(float_type) + m * sizeof(int), false);
     float_type *d_dec = d_part + part_doubles;
     // a request of a few rows has its decision values written straight to page-locked host memory: no copy behind the kernels
-    struct HostBlock {
-        tsvm::PinnedBlock block;
-        ~HostBlock() { if (block.host) tsvm::give_pinned_block(block); }
-    } direct;
+    std::unique_ptr<tsvm::ResultBlock> direct;
     if (!winner_out && dec_doubles * sizeof(float_type) <= tsvm::PINNED_BLOCK) {
-        direct.block = tsvm::take_pinned_block();
-        d_dec = (float_type *) direct.block.dev;
+        direct.reset(new tsvm::ResultBlock(tsvm::work_stream()));
+        d_dec = (float_type *) direct->dev();
     }
     // (a batch row may set more indicator columns than any support vector does: its matches are bounded by the
     // support vectors' count all the same)
@@ -161,9 +159,8 @@ bool SvmModel::predict_batch_fused(const PredictPlan &P, const kernel_type *a, i
                                             P.chunk_table.data(), P.rho, n_classes, a, lda, (int64_t) m, sd_a,
                                             plan_masks ? P.mask_a.data() : nullptr, R.ind_max_ones, (int) param.kernel_type,
                                             param.gamma, param.coef0, param.degree, d_part, d_dec, tsvm::work_stream()));
-    if (direct.block.host) {
-        TSVM_HIP_CHECK(hipStreamSynchronize(tsvm::work_stream()));
-        memcpy(dec_out, direct.block.host, dec_doubles * sizeof(float_type));
+    if (direct) {
+        memcpy(dec_out, direct->wait(), dec_doubles * sizeof(float_type));
     } else {
         fetch_predictions(d_dec, m, dec_out, winner_out);
     }
