@@ -357,9 +357,12 @@ __global__ void indicator_masks_kernel(const double *__restrict__ x, int64_t ld,
 // Bound by one workgroup's walk through the features (the solver's block has 1,024 instances, fewer tiles than there are CUs):
 // tiles of 64 x 64, 136 of them on or above the diagonal, by eight wavefronts of 16 x 32, two per SIMD so that one's LDS reads
 // and staging run beside the other's MFMAs.  The values go through LDS, so that the tile and its mirror image are both stored in
-// runs of 64.  1,024 instances of 784 / 90 / 32 features: 40.1 / 11.0 / 9.7 us.  Tiles of 64 x 128 by four wavefronts, 72 of
-// them: 68.4 / 16.0 / 13.3; 64 x 64 by four wavefronts 51.5 / 13.3 / 11.7, with a barrier on either side of the staging instead of two
-// sets of staged columns 43.9 / 11.4 / 9.7.  Column tile j needs the row tiles 0 .. j: workgroup c works on column tile j = the largest j
+// runs of 64.  1,024 instances of 784 / 90 / 32 features: 38.1 / 8.4 / 5.8 us; by four wavefronts 47.9 / 10.5 / 7.5; tiles of
+// 64 x 128 by four wavefronts, 72 of them: 68.5 / 14.5 / 9.9.
+// The columns are staged in one place, with a barrier on either side, 34 KB of LDS: on the solver's CUs these workgroups share
+// the CU with get_rows' (three of 39 KB up to 128 features).  Two sets of staged columns, 69 KB, are no faster alone (39.4 / 8.3
+// / 5.7) and wait there until more of get_rows' workgroups have left: C-SVC on 100,000 x 784 448 ms instead of 396, epsilon-SVR on
+// 400,000 x 90 1,588 instead of 1,420.  Column tile j needs the row tiles 0 .. j: workgroup c works on column tile j = the largest j
 // with j(j+1)/2 <= c, row tile c - j(j+1)/2; dealt out in this order, every XCD gets the same share of the work.
 #define SYM_B 64     // rows and columns of a tile
 #define SYM_K 32     // columns of the data staged at a time
@@ -368,10 +371,11 @@ template <int KT, typename TO>
 __global__ __launch_bounds__(512) void get_rows_dense_sym_kernel(
     const double *__restrict__ x, int64_t ldx, const int *__restrict__ idx, int m, int d, const double *__restrict__ sd_x,
     KernelParam kp_in, TO *__restrict__ out, int64_t ldo) {
-    __shared__ double s_tile[4 * SYM_K * SYM_LS];   // As, Bs twice, and then the values
+    __shared__ double s_tile[2 * SYM_K * SYM_LS];   // As, Bs, and then the values
     __shared__ double s_sd[2][SYM_B];
     __shared__ uint64_t exp_tab[32];
     static_assert(SYM_B * (SYM_B + 1) <= 2 * SYM_K * SYM_LS, "the values take the staged columns' place");
+    static_assert(sizeof(s_tile) + sizeof(s_sd) + sizeof(exp_tab) <= 160 * 1024 - 3 * 38656, "room beside three of get_rows' workgroups");
     KernelParam kp = kp_in;
     kp.kernel_type = KT;
     const int c = (int) blockIdx.x;
@@ -405,8 +409,8 @@ __global__ __launch_bounds__(512) void get_rows_dense_sym_kernel(
     v4d acc[2];
 #pragma unroll
     for (int tj = 0; tj < 2; ++tj) acc[tj] = (v4d){0.0, 0.0, 0.0, 0.0};
-    auto mma_step = [&](const double *As, int ks) {
-        const double *const Bs = As + SYM_K * SYM_LS;
+    double *const As = s_tile, *const Bs = s_tile + SYM_K * SYM_LS;
+    auto mma_step = [&](int ks) {
         const int kk = (ks * 4 + lk) * SYM_LS + lrow;
         const double af = As[kk + wi * 16];
         double bf[2];
@@ -418,8 +422,7 @@ __global__ __launch_bounds__(512) void get_rows_dense_sym_kernel(
     if (d > 0) load(0);
     if (tid < 2 * SYM_B) s_sd[tid >> 6][lane] = sd_x ? sd_x[idx[min((tid >> 6 ? j0 : i0) + lane, m - 1)]] : 0.0;
     if (tid < 32) exp_tab[tid] = TSVM_EXP2F_TAB[tid];
-    auto stage = [&](double *As) {
-        double *const Bs = As + SYM_K * SYM_LS;
+    auto stage = [&] {
 #pragma unroll
         for (int q = 0; q < 2; ++q)
 #pragma unroll
@@ -428,23 +431,19 @@ __global__ __launch_bounds__(512) void get_rows_dense_sym_kernel(
                 Bs[(k_mine + e) * SYM_LS + r_mine + 4 * q] = rb[q][e];
             }
     };
-    // (two sets of staged columns: a wavefront stages the next ones while another still multiplies)
-    double *now = s_tile, *next = s_tile + 2 * SYM_K * SYM_LS;
-    if (d > 0) stage(now);
+    if (d > 0) stage();
     if (d > SYM_K) load(SYM_K);
     __syncthreads();
     int k0 = 0;
     for (; k0 + SYM_K < d; k0 += SYM_K) {
 #pragma unroll
-        for (int ks = 0; ks < SYM_K / 4; ++ks) mma_step(now, ks);
-        stage(next);
+        for (int ks = 0; ks < SYM_K / 4; ++ks) mma_step(ks);
+        __syncthreads();
+        stage();
         if (k0 + 2 * SYM_K < d) load(k0 + 2 * SYM_K);
         __syncthreads();
-        double *const t = now;
-        now = next;
-        next = t;
     }
-    for (int ks = 0; ks < (d - k0 + 3) / 4; ++ks) mma_step(now, ks);
+    for (int ks = 0; ks < (d - k0 + 3) / 4; ++ks) mma_step(ks);
     __syncthreads();
     TO *const val = (TO *) s_tile;   // [row][column], rows SYM_B + 1 apart
 #pragma unroll
