@@ -760,3 +760,18 @@ def test_selections_that_report_their_ids(n, tie_mode, fold, nu):
     with pytest.raises(capi.TsvmError):   # the word would lie inside the ids
         capi.call("tsvm_select_working_set_report", G.ptr(f_d), G.ptr(y_d), G.ptr(a_d), n, C, C, None, 0, G.ptr(out_d), ws, nu, G.ptr(wsp), 0, 0, None,
                   host.data_ptr(), ws - 1, 1, G.stream())
+
+
+@pytest.mark.parametrize("nu", [0, 1])
+def test_a_selection_of_no_ids_still_reports(nu):
+    """n_select == 0: nothing is written but the word that the host polls."""
+    n = 300
+    f, y, alpha, C, _ = _select_case(n, 16, 0, 5, 0, nu)
+    f_d, y_d, a_d = G.dev(f), G.dev(y), G.dev(alpha)
+    wsp = torch.empty(capi.kernel_lib().tsvm_select_workspace(n), dtype=torch.uint8, device="cuda")
+    out_d = torch.full((4,), -7, dtype=torch.int32, device="cuda")
+    host = torch.full((4,), -7, dtype=torch.int32).pin_memory()
+    capi.call("tsvm_select_working_set_report", G.ptr(f_d), G.ptr(y_d), G.ptr(a_d), n, C, C, None, 0, G.ptr(out_d), 0, nu, G.ptr(wsp), 0, 0, None,
+              host.data_ptr(), 1, 43, G.stream())
+    torch.cuda.synchronize()
+    assert host.tolist() == [-7, 43, -7, -7] and out_d.tolist() == [-7] * 4

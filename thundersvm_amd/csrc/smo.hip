@@ -1257,8 +1257,14 @@ static int select_working_set(const double *f, const int *y, const double *alpha
                  MAX_WS);
     TSVM_REQUIRE(n_marked >= 0 && (n_marked == 0 || marked), "tsvm_select_working_set: bad marked list");
     TSVM_REQUIRE(fold_n >= 0 && (fold_n == 0 || out_folded), "tsvm_select_working_set: bad fold arguments");
-    if (n_select == 0) return 0;
     hipStream_t s = tsvm_s(stream);
+    if (n_select == 0) {   // (nothing to select, but whoever polls the word hears of it)
+        if (report.ids) {
+            hipLaunchKernelGGL(report_ids_kernel, dim3(1), dim3(256), 0, s, out, 0, 0, report.word_at, 0, report.word);
+            TSVM_LAUNCH_CHECK();
+        }
+        return 0;
+    }
     const SelWorkspace w = sel_workspace(workspace, n);
     const SelGeom g = sel_geom(n, n_select, nu);
     // The first three digits (33 bits of f) are counted by the whole chip, the rest (rarely needed) by one
