@@ -247,4 +247,12 @@ long long tsvm_selftest_load_matrix(int dense, int row_size, int features, float
     }
 }
 
+// The schedule of a solve that has the chip to itself: bit 0 the block beside the rows, bit 1 a second warming behind them, when the
+// previous iteration computed m_before rows of n values and this one m_now.
+int tsvm_selftest_chip_split(int features, int ws, long long n, long long m_before, long long m_now) {
+    using tsvm::ChipSplit;
+    const bool beside = ChipSplit::block_beside_rows(features, ws, ChipSplit::rows_seconds(features, m_before, n));
+    return (beside ? 1 : 0) | (ChipSplit::warm_behind_rows(beside, ChipSplit::rows_seconds(features, m_now, n)) ? 2 : 0);
+}
+
 }  // extern "C"

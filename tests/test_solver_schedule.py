@@ -1,0 +1,19 @@
+"""Which parts of an iteration run side by side in a solve that has the chip to itself (ChipSplit, host/solver.h).  Host only."""
+import pytest
+
+import selftest_lib
+
+BESIDE, WARM = 1, 2
+
+
+@pytest.mark.parametrize("features,n,before,now,want", [
+    (784, 100000, 512, 512, BESIDE),          # rows for 1.2 ms: the block and the solver fit beside them
+    (784, 20000, 512, 512, 0),                # 0.24 ms: they do not, and the rows outlast a second warming
+    (90, 400000, 512, 512, BESIDE),
+    (90, 40000, 512, 512, WARM),              # 0.06 ms
+    (90, 40000, 0, 0, 0),                     # no rows that would push the block out
+    (784, 100000, 512, 20, BESIDE),           # few misses after many: the block is on the solver's CUs, where it may not be there yet
+    (784, 100000, 20, 512, 0),
+])
+def test_chip_split(features, n, before, now, want):
+    assert selftest_lib.lib().tsvm_selftest_chip_split(features, 1024, n, before, now) == want

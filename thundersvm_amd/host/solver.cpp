@@ -683,19 +683,14 @@ struct SolveTask::Impl {
         timer.end(stats.ms_get_rows);
     }
 
-    double seconds_per_value() const { return 2.0 * ((k_mat.n_features() + 15) / 16 * 16) / 6.6e13; }   // of a dense row, on the whole chip
-    double rows_seconds() const { return seconds_per_value() * (double) last_rows_computed * n_u; }
+    double rows_seconds() const { return tsvm::ChipSplit::rows_seconds(k_mat.n_features(), last_rows_computed, n_u); }
 
     void enqueue_block() {
         timer.begin();
         on_one_stream = !split || (alone && all_cached);
-        // (Dense rows only: the CSR block takes too long on eight CUs.  Both launches are matrix-core work with the
-        // same cost per value; the block plus the solver's ~0.4 ms has to fit into the time of the rows.)
-        block_on_solver_cus = false;
-        if (!on_one_stream && alone && block_first && k_mat.dense_layout() && !all_cached) {
-            const double t_block = seconds_per_value() * 32.0 * 0.53 * ws_size * (double) ws_size;   // on 8 of 256 CUs; 136 of its 256 tiles
-            block_on_solver_cus = t_block + 0.4e-3 <= rows_seconds();
-        }
+        // (dense rows only: the CSR block takes too long on eight CUs)
+        block_on_solver_cus = !on_one_stream && alone && block_first && k_mat.dense_layout() && !all_cached &&
+                              tsvm::ChipSplit::block_beside_rows(k_mat.n_features(), ws_size, rows_seconds());
         if (caching && all_cached) {
             abi_check(tsvm_smo_gather_block_by_id(k_rows, row_type, d_slot_of.data(), ld, ws_u(), ws_size, d_kws.data(), row_type,
                                                   d_slots_a.data(), sa));
@@ -749,11 +744,8 @@ struct SolveTask::Impl {
     }
 
     void enqueue_update() {
-        // The rows that stream through the solver's L2 beside it take the block's place there: it is read once more behind them
-        // (epsilon-SVR 40000x90, rows for 42 us beside a solver of 310: 88.4 -> 81.3 ms), unless they take about as long
-        // as the solver (20000x784, 340 us: 50.2 -> 50.3) or other lanes' rows come through at any time (7 classes
-        // 300000x54: 844 -> 857).
-        if (!on_one_stream && alone && k_mat.dense_layout() && !all_cached && last_rows_computed > 0 && rows_seconds() < 0.1e-3)
+        // (not where other lanes' rows come through at any time: 7 classes 300000x54 844 -> 857)
+        if (!on_one_stream && alone && k_mat.dense_layout() && !all_cached && tsvm::ChipSplit::warm_behind_rows(block_on_solver_cus, rows_seconds()))
             abi_check(tsvm_smo_warm_block(d_kws.data(), row_type, ws_size, solver_xcd, d_gate.data() + 3, sa));
         if (!on_one_stream) TSVM_HIP_CHECK(hipStreamWaitEvent(sa, solved.event, 0));   // alpha_diff, alpha and diff come from the solver
         if (select_ahead && fuse_select) {

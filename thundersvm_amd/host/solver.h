@@ -42,6 +42,23 @@ namespace tsvm {
 void wait_while_pending(const volatile uint64_t *word, uint64_t pending, long long timeout_ms, hipError_t (*stream_state)(void *),
                         void *stream);
 long long solver_timeout_ms();   // TSVM_SOLVER_TIMEOUT_MS, default 300,000
+
+// What a solve that has the chip to itself runs where, by the time that the rows of an iteration take (dense rows).
+struct ChipSplit {
+    // Of m dense rows of n values, on the whole chip.  (Every column counts.  Indicator columns are left to the epilogue, whose
+    // share makes up for it: 512 x 425,000 values of 10 + 44 columns take 1.7 ps each, 1.9 by this.)
+    static double rows_seconds(size_t features, long long m, long long n) { return 2.0 * (double) ((features + 15) / 16 * 16) / 6.6e13 * (double) m * (double) n; }
+    // Whether the block is computed on the solver's eight CUs, beside the previous iteration's number of rows: it and the
+    // solver's ~0.4 ms have to fit into their time (136 of its 256 tiles, on 8 of 256 CUs).
+    static bool block_beside_rows(size_t features, int ws, double rows_seconds) {
+        return 32.0 * 0.53 * ChipSplit::rows_seconds(features, ws, ws) + 0.4e-3 <= rows_seconds;
+    }
+    // Whether the block is read into the solver's L2 a second time, behind the rows that stream through it beside the solver and
+    // take its place there (epsilon-SVR 40000x90, rows for 42 us beside a solver of 310: 88.4 -> 81.3 ms), unless they take
+    // about as long as the solver (20000x784, 340 us: 50.2 -> 50.3).  A block that is itself computed beside the rows may
+    // not be there yet.
+    static bool warm_behind_rows(bool block_beside, double rows_seconds) { return !block_beside && rows_seconds > 0 && rows_seconds < 0.1e-3; }
+};
 }  // namespace tsvm
 
 class CSMOSolver {
