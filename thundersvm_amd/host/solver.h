@@ -49,7 +49,9 @@ struct ChipSplit {
     // share makes up for it: 512 x 425,000 values of 10 + 44 columns take 1.7 ps each, 1.9 by this.)
     static double rows_seconds(size_t features, long long m, long long n) { return 2.0 * (double) ((features + 15) / 16 * 16) / 6.6e13 * (double) m * (double) n; }
     // Whether the block is computed on the solver's eight CUs, beside the previous iteration's number of rows: it and the
-    // solver's ~0.4 ms have to fit into their time (136 of its 256 tiles, on 8 of 256 CUs).
+    // solver's ~0.4 ms have to fit into their time.  (136 of its 256 tiles on 8 of 256 CUs: 422 us for 1,024 instances of 784
+    // columns and 52 of 90 by this, 505 and 116 by measurement, beside get_rows.  With those, 450 rows of 400,000 columns in
+    // place of 390 are what it takes, and epsilon-SVR on 400,000 x 90 takes 1,411 ms in place of 1,408.)
     static bool block_beside_rows(size_t features, int ws, double rows_seconds) {
         return 32.0 * 0.53 * ChipSplit::rows_seconds(features, ws, ws) + 0.4e-3 <= rows_seconds;
     }
