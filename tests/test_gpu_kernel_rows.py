@@ -648,6 +648,24 @@ def test_indicator_columns(n, n_cont, groups, m, name, kt, prm):
     _check(name, G.host(outb), want[:, cols])
 
 
+@pytest.mark.parametrize("m", [1, 64, 65, 200])
+def test_symmetric_block_with_indicator_columns(m):
+    """Both sides the same rows, with masks: the bits of the plain call on all columns."""
+    rng = np.random.default_rng(m)
+    x = np.zeros((300, 24))
+    x[:, :22] = _mixed_rows(rng, 300, 8, (4, 10))
+    x_d, sd = G.dev(x), G.dev((x * x).sum(axis=1))
+    masks, ones = torch.zeros(300, dtype=torch.int64, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+    capi.call("tsvm_indicator_masks", G.ptr(x_d), 24, 300, 8, 14, G.ptr(masks), G.ptr(ones), G.stream())
+    idx = G.dev(rng.permutation(300)[:m].astype(np.int32))
+    got, want = torch.zeros((m, m), dtype=torch.float64, device="cuda"), torch.zeros((m, m), dtype=torch.float64, device="cuda")
+    capi.call("tsvm_get_rows_dense_indicator", G.ptr(x_d), 24, G.ptr(idx), m, 8, G.ptr(sd), G.ptr(masks), G.ptr(x_d), 24, G.ptr(idx), m, None, G.ptr(sd),
+              G.ptr(masks), int(ones[0]), O.RBF, 0.3, 0.0, 3, G.ptr(got), capi.ROW_F64, None, m, G.stream())
+    capi.call("tsvm_get_rows_dense", G.ptr(x_d), 24, G.ptr(idx), m, 22, G.ptr(sd), G.ptr(x_d), 24, G.ptr(idx), m, G.ptr(sd), O.RBF, 0.3, 0.0, 3,
+              G.ptr(want), capi.ROW_F64, None, m, G.stream())
+    assert np.array_equal(G.host(got), G.host(want))
+
+
 @pytest.mark.parametrize("n", [1, 3, 4, 5, 257])
 @pytest.mark.parametrize("d,ld", [(1, 8), (63, 64), (64, 64), (65, 72), (130, 136), (40, 24)])
 @pytest.mark.parametrize("host", [False, True])

@@ -1163,7 +1163,7 @@ static int get_rows_dense(const double *x, int64_t ldx, const int *x_idx, int64_
     dim3 grid((unsigned) (n_blocks * m_blocks)), block(256);
     // the solver's ws x ws block: symmetric, computed from the tiles on and above the diagonal
     const bool sym = x == a && ldx == lda && x_idx && x_idx == a_idx && n == m && sd_x == sd_a && !out_slots && !m_dev &&
-                     ti == 2 && ldo >= n;
+                     !mask_x && ti == 2 && ldo >= n;   // (with masks d does not count the columns that they stand for)
     if (sym) {
         const int64_t tiles = (n + SYM_B - 1) / SYM_B;
         grid = dim3((unsigned) (tiles * (tiles + 1) / 2));   // column tile j: row tiles 0 .. j
