@@ -14,6 +14,7 @@ static int g_current = 0, g_failures = 0;
 static bool g_hung = false;                   // events are never reached
 static hipError_t g_stream_state = hipSuccess;   // what waiting for a stream says
 static int g_stream_waits = 0;
+static unsigned g_host_flags = 0;              // of the last page-locked allocation
 static std::map<const void *, int> g_owner;   // device of every live block, stream and event
 
 static void expect(bool ok, const char *what) {
@@ -38,7 +39,7 @@ hipError_t hipGetDevice(int *d) { *d = g_current; return hipSuccess; }
 hipError_t hipSetDevice(int d) { g_current = d; return hipSuccess; }
 hipError_t hipMalloc(void **p, size_t bytes) { return make(p, bytes); }
 hipError_t hipFree(void *p) { return drop(p); }
-hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) { return make(p, bytes); }
+hipError_t hipHostMalloc(void **p, size_t bytes, unsigned flags) { g_host_flags = flags; return make(p, bytes); }
 hipError_t hipHostFree(void *p) { return drop(p); }
 hipError_t hipHostGetDevicePointer(void **d, void *h, unsigned) { *d = h; return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { ++g_stream_waits; return g_stream_state; }
@@ -98,6 +99,9 @@ static void result_blocks() {
 int main() {
     result_blocks();
     g_stream_state = hipSuccess;
+    tsvm::PinnedBuffer<double> staging;
+    staging.reserve(100);
+    expect(g_host_flags == (hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable), "staging memory that kernels read in place");
     blocks(true);
     tsvm::DevicePool::instance().flush();
     blocks(false);

@@ -216,7 +216,7 @@ private:
 };
 
 // Page-locked host staging memory that only grows (hipHostMalloc; copies from it are asynchronous and run at
-// the link's rate).
+// the link's rate).  Kernels read it in place too: mapped and coherent whatever the environment's default is, on any device.
 template <typename T>
 class PinnedBuffer {
 public:
@@ -229,7 +229,7 @@ public:
         if (ptr_) (void) hipHostFree(ptr_);
         ptr_ = nullptr;
         count_ = 0;
-        TSVM_HIP_CHECK(hipHostMalloc((void **) &ptr_, count * sizeof(T)));
+        TSVM_HIP_CHECK(hipHostMalloc((void **) &ptr_, count * sizeof(T), hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable));
         count_ = count;
     }
     T *data() { return ptr_; }
