@@ -202,7 +202,7 @@ def kernel_figures(train, params):
     ms = event_time(lambda: capi.call("tsvm_update_f", f.data_ptr(), ad.data_ptr(), ws, k_rows.data_ptr(), row_type, None,
                                       ldo, n, 1, None), 20)
     by = float(esz) * ws * n + 16.0 * n + 8.0 * ws   # bytes this kernel has to move with rows of esz-byte values
-    out["update_f"] = dict(kernel="update_f_kernel", ms=ms, ws=ws, n=n, row_bytes_per_value=esz, min_bytes=by, gbs=by / ms / 1e6,
+    out["update_f"] = dict(kernel="update_f_kernel" if n > (65536 if esz == 4 else 32768) else "update_f_narrow_kernel", ms=ms, ws=ws, n=n, row_bytes_per_value=esz, min_bytes=by, gbs=by / ms / 1e6,
                            frac_hbm_peak=by / ms / 1e6 / HBM_PEAK_GBS)
     return out
 
@@ -597,7 +597,7 @@ def main():
                         frac_in_training=it["get_rows_tflops"] / FP64_MFMA_PEAK_TFLOPS,
                         in_training="2*rows*n*d over the get_rows time of a phase-profiled pass")
     roofline["share_of_phase_time"] = share("ms_get_rows")
-    roofline_uf = dict(kernel="update_f_kernel (ws 1024 x n %d, %d-byte kernel values)" % (uf["n"], uf["row_bytes_per_value"]),
+    roofline_uf = dict(kernel="%s (ws 1024 x n %d, %d-byte kernel values)" % (uf["kernel"], uf["n"], uf["row_bytes_per_value"]),
                        bound="hbm", achieved=uf["gbs"], peak=HBM_PEAK_GBS, unit="GB/s", frac=uf["frac_hbm_peak"],
                        traffic=profiled_traffic(args.workload, "update_f"), traffic_unit=traffic_unit, launch_ms=uf["ms"],
                        algorithmic="e*ws*n + 16*n + 8*ws bytes per launch, e=%d ws=1024 n=%d" % (uf["row_bytes_per_value"], uf["n"]),

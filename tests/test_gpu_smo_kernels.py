@@ -678,6 +678,21 @@ def test_update_f_with_the_next_selection(n_cols, repeat, ws, ld_pad, tie_mode, 
         a_d = G.dev(alpha)
 
 
+@pytest.mark.parametrize("row_type,line", [(capi.ROW_F64, 32768), (capi.ROW_F32, 65536)])
+@pytest.mark.parametrize("beyond,ld_pad", [(0, 0), (0, 1), (1, 1), (1, 2)])
+def test_update_f_at_the_line_between_its_kernels(row_type, line, beyond, ld_pad):
+    """The last size of the kernel whose wavefronts take the rows in turn and the first of the one thread per column, rows aligned to two
+    columns and not, with and without the selection's first pass."""
+    n, ws = line + beyond, 48
+    rng = np.random.default_rng(n + ld_pad)
+    k = rng.random((ws, n + ld_pad)).astype(np.float32 if row_type == capi.ROW_F32 else np.float64)
+    f, ad = rng.standard_normal(n), np.where(rng.random(ws) < 0.3, 0.0, rng.standard_normal(ws))
+    f_d, ad_d, k_d = G.dev(f), G.dev(ad), G.dev(k)
+    capi.call("tsvm_update_f", G.ptr(f_d), G.ptr(ad_d), ws, G.ptr(k_d), row_type, None, n + ld_pad, n, 1, G.stream())
+    assert np.array_equal(G.host(f_d), O.update_f(f, ad, np.ascontiguousarray(k[:, :n].astype(np.float64)), n))
+    test_update_f_with_the_next_selection(n, 2, ws, ld_pad, 0, row_type, 0)
+
+
 def test_empty_inputs_are_no_ops():
     """Zero rows, zero columns, an empty working set, nothing to select: every entry point returns success and
     leaves its outputs untouched."""

@@ -281,7 +281,7 @@ struct SelFuse {
 // update_f: f[j] -= sum_t alpha_diff[t] * K_t[j]  (smo_kernel.cpp:300-319)
 // Bandwidth-bound stream over the ws x n kernel rows.  The non-zero alpha_diff entries are
 // compacted (in order) into LDS once per workgroup; rows with alpha_diff == 0 are never read.
-// This kernel is for 262,144 columns and more (update_f_narrow_kernel below for fewer).
+// This kernel is for more than 65,536 columns of floats, 32,768 of doubles (update_f_narrow_kernel below for fewer).
 // Each thread owns one to four adjacent columns and keeps 8 to 32 row loads in flight.  On the vector-load
 // path the columns are dealt evenly to a number of workgroups that is a multiple of 248 (every CU, or every
 // CU left to a stream that leaves one CU per XCD to the local solver, gets the same number of workgroups):
@@ -455,7 +455,7 @@ __global__ __launch_bounds__(UF_T) void update_f_kernel(double *__restrict__ f, 
     }
 }
 
-// The same for fewer than 262,144 columns.  One thread per column leaves most of the chip without work then, and a column's some 500
+// The same for fewer columns.  One thread per column leaves most of the chip without work then, and a column's some 500
 // rows come in sixteen batches one memory latency apart: 27 us for 3,200 columns and 31 for 40,000.  Here a workgroup has
 // 64 * COLS columns and eight wavefronts; groups of R neighbouring rows are dealt to them in turn, so that all eight have theirs on
 // their way at once, and they add them in turn: the sums of a column stay one chain in the rows' order, handed on through
@@ -1196,35 +1196,43 @@ static void launch_update_f_narrow(double *f, const double *alpha_diff, int ws_s
 template <int NS>
 static void dispatch_update_f(double *f, const double *alpha_diff, int ws_size, const void *k_rows, int row_type, const int *slots,
                               int64_t ld, int64_t n, int repeat, const SelFuse &sf, hipStream_t s) {
-    // vector loads need every row start aligned to the vector and the last vector inside the padded row
-    const bool big = n >= (int64_t) UF_T * 1024;
-    const bool aligned = (uintptr_t) k_rows % 16 == 0;
-    if (!big) {
-        // As few columns per thread as make do with one workgroup per CU (more workgroups than that leave some CUs two in
-        // turn), floats two up to 65,536 columns and four beyond, doubles one.  500 of 1,024 rows, us a call, one thread per column / here with
-        // 1, 2, 4 floats (1, 2 doubles) per thread:
-        // (40,000 columns and the selection's first pass on top, in training: 26.8 us with four, 24.4 with two.)
-        //   floats   3,200: 26.7 / 12.7 15.1 18.6   20,000: 30.7 / 16.9 15.7 19.0   40,000: 31.5 / 26.6 21.5 19.8
-        //           60,000: 34.0 / 32.8 24.3 24.5  120,000: 46.7 / 59.6 45.0 43.2  255,000: 100 / 128 99.6 90.3 (5.6 TB/s)
-        //   doubles  3,200: 32.6 / 14.9 15.3        18,000: 35.7 / 20.0 16.7        40,000: 38.7 / 31.0 34.2
-        //           90,000: 67.0 / 60.5 63.7       200,000: 142 / 127 131 (6.3 TB/s)
-        auto fits = [&](int cols, size_t esz) { return (uintptr_t) k_rows % (cols * esz) == 0 && ld % cols == 0 && n <= (int64_t) 64 * cols * 256; };
+    // Vector loads need every row start aligned to the vector and the last vector inside the padded row.
+    const size_t esz = row_type == TSVM_ROW_F32 ? 4 : 8;
+    auto aligned = [&](int cols) { return (uintptr_t) k_rows % (cols * esz) == 0 && ld % cols == 0; };
+    // Few columns: wavefronts that take the rows in turn, one column per thread while that makes do with one workgroup per CU (more
+    // workgroups leave some CUs two in turn), and on to 65,536 columns of floats with two, to 32,768 of doubles.  Of 2,048
+    // rows in slots, us a call, one thread per column and all rows / wavefronts in turn:
+    //   non-zero rows     60          250          500         1,024
+    //   floats  20,000   8.1 /  5.4  21.4 /  9.8  29.3 / 15.2   41.8 /  26.1
+    //           65,536  15.6 /  6.9  24.9 / 15.1  34.1 / 24.6   50.0 /  44.7
+    //          100,000  17.6 /  8.8  28.7 / 22.0  41.2 / 38.5   64.7 /  71.2   (here and below: four columns per thread)
+    //          180,000  20.4 / 13.6  39.7 / 37.3  64.6 / 67.2  112.2 / 131.5
+    //   doubles 20,000  10.2 /  6.2  23.0 / 10.5  35.5 / 16.4   62.5 /  28.4
+    //           40,000  11.8 /  9.2  24.5 / 20.1  37.6 / 33.8   67.9 /  62.1
+    //          100,000  15.3 / 17.2  38.5 / 41.2  67.7 / 72.4  132.1 / 137.9
+    // Beyond the line rows in turn win alone where few rows are non-zero, and lose in training: calls with wavefronts in turn
+    // everywhere / up to the line, ms: C-SVC 100,000 x 784 394.3 / 391.0, 200,000 x 30 483.7 / 468.0, 90,000 x 40 102.2 / 101.1,
+    // epsilon-SVR 100,000 x 90 217.8 / 215.4, linear on 60,000 sparse rows 117.7 / 116.2; seven classes of 240,000 rows 596 / 584, means of
+    // four calls of 574 to 608.
+    const bool narrow = n <= (int64_t) 64 * 256 * (row_type == TSVM_ROW_F32 ? 4 : 2);
+    if (narrow) {
+        const bool one = n <= (int64_t) 64 * 256 || !aligned(2);
         if (row_type == TSVM_ROW_F32) {
-            if (fits(1, 4)) launch_update_f_narrow<float, 1, 32, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
-            else if (fits(2, 4) || (n <= 65536 && (uintptr_t) k_rows % 8 == 0 && ld % 2 == 0)) launch_update_f_narrow<float, 2, 16, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
-            else if (aligned && ld % 4 == 0) launch_update_f_narrow<float, 4, 16, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
-            else launch_update_f_narrow<float, 1, 32, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
+            if (one) launch_update_f_narrow<float, 1, 32, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
+            else launch_update_f_narrow<float, 2, 16, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
         } else {
-            if (!fits(1, 8) && fits(2, 8)) launch_update_f_narrow<double, 2, 16, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
-            else launch_update_f_narrow<double, 1, 16, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
+            if (one) launch_update_f_narrow<double, 1, 16, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
+            else launch_update_f_narrow<double, 2, 16, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
         }
         return;
     }
+    // 16-byte loads from 262,144 columns on; with fewer, one column per thread and more rows in flight keeps more of the chip busy
+    const bool wide = n >= (int64_t) UF_T * 1024;
     if (row_type == TSVM_ROW_F32) {
-        if (big && aligned && ld % 4 == 0 && ld >= (n + 3) / 4 * 4) launch_update_f<float, 4, 8, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
+        if (wide && aligned(4)) launch_update_f<float, 4, 8, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
         else launch_update_f<float, 1, 32, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
     } else {
-        if (big && aligned && ld % 2 == 0 && ld >= (n + 1) / 2 * 2) launch_update_f<double, 2, 8, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
+        if (wide && aligned(2)) launch_update_f<double, 2, 8, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
         else launch_update_f<double, 1, 16, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
     }
 }

@@ -446,9 +446,9 @@ struct SolveTask::Impl {
         // straight from update_f into it; if the diff then says stop, that selection was simply not needed.
         // (Not when tracing, which reads the working set back after each iteration, nor when profiling.)
         select_ahead = !solver.trace && !solver.profile;
-        // With stacked copies (SVR) the first pass rides along where a copy is a wavefront's and the workgroups are few: epsilon-SVR on
-        // 40,000 rows 92.4 -> 91.5 ms, on 120,000 294.3 -> 291.0, but on 3,000 and 12,000 7.55 -> 7.60 and 27.28 -> 27.38; and from
-        // 262,144 columns on a thread has all copies' instances to classify after its rows have streamed by, each behind
+        // With stacked copies (SVR) the first pass rides along from 16,385 columns on (epsilon-SVR on 3,000 and 12,000 rows 7.55 -> 7.60 and
+        // 27.28 -> 27.38 ms with it, on 40,000 92.4 -> 91.5, on 100,000 218.9 -> 216.2, on 120,000 282.0 -> 279.5); from 262,144 columns
+        // on a thread has the instances of all copies of its columns to classify after its rows have streamed by, each behind
         // memory reads that wait on a saturated HBM: slower than the separate pass.
         fuse_select = q > 0 && (rep == 1 || (rep <= 4 && n_u > 16384 && n_u < 262144));
         // The solver reads the ws x ws block of the kernel matrix.  With few features the block is cheap to
