@@ -790,7 +790,8 @@ KernelMatrix::StagedBatch KernelMatrix::stage_batch(const RowStore &batch, size_
     out.sd = stage_sd_.data();
     out.indicator_values = R.ind_first >= 0 && !not_indicator;
     // A request of a few rows is read by the kernel where it is, in page-locked host memory: three copies of a microsecond's work
-    // cost 5 us each.
+    // cost 5 us each.  However many rows the entries are spread over: 4,000 rows of one entry 82 us (as copies 100), 3,900
+    // entries over 16,000 rows 235 (276), over 65,536 rows 283 (296); rows without any entry 203 (196) and 269 (229).
     const kernel_type *d_val = val;
     const int *d_col = col;
     const int64_t *d_ptr = ptr;
