@@ -62,7 +62,8 @@ int tsvm_kernel_diag(const double *self_dot, int64_t n, int kernel_type, double 
 
 /* Scatter CSR rows into a zero-filled dense row-major matrix [n][ld] (column c = feature id c):
  * get_working_set_ins, kernelmatrix_kernel.cpp:9-25, applied to all rows once.  Entries with
- * col >= ld are dropped (the test-row rule of kernelmatrix.cpp:392). */
+ * col >= ld are dropped (the test-row rule of kernelmatrix.cpp:392).  For callers that have a zeroed matrix and want no self
+ * dot products; this library's own rows come from tsvm_csr_rows_to_dense. */
 int tsvm_csr_to_dense(const double *val, const int *col, const int64_t *row_ptr, int64_t n, double *x, int64_t ld,
                       tsvm_stream stream);
 
@@ -177,7 +178,7 @@ int tsvm_get_rows_csr_sliced(const int *ell_col, const void *ell_val, int val_ty
 
 /* Device-side row subsets, so that a sub-problem (one class pair of a one-vs-one run, svc.cpp:147-150) takes its
  * rows from a data set already resident in HBM instead of a host copy:
- * dense: out row r = x row idx[r] (rows of ld doubles, ld % 4 == 0);
+ * dense: out row r = x row idx[r] (rows of ld doubles, ld % 4 == 0; this library's own subsets take tsvm_subset_rows_dense below);
  * CSR: rows idx[0..m) of (val, col, row_ptr) written to (out_val, out_col) at the offsets out_ptr[0..m], which the
  * caller has computed from the row lengths. */
 int tsvm_gather_rows_f64(const double *x, int64_t ld, const int *idx, int64_t m, double *out, tsvm_stream stream);
@@ -346,7 +347,8 @@ int tsvm_nu_smo_solve(const int *y, const double *f_val, double *alpha, double *
  * modulo fold_n when fold_n > 0, and then, behind a system-wide fence, writes `word` to host_ids[word_at]
  * (word_at >= n_ids): a host thread that polls that word sees the ids once it sees the word.  It has no counterpart in
  * the reference, whose select_working_set runs on the host (csmosolver.cpp:123-165); it replaces a device-to-host copy
- * and the event behind it for callers that keep a host-side table of which kernel row lives where. */
+ * and the event behind it for callers that keep a host-side table of which kernel row lives where.  (This library's own
+ * selections report their ids themselves: tsvm_select_working_set_report.) */
 int tsvm_report_ids(const int *ids, int n_ids, int fold_n, int *host_ids, int word_at, int word, tsvm_stream stream);
 
 /* Bytes of device workspace tsvm_select_working_set needs for n instances. */
