@@ -231,6 +231,25 @@ def test_batch_without_any_entry(m, kt):
     assert np.array_equal(gm.predict(Dataset(te).to_device())[1], got)
 
 
+@pytest.mark.parametrize("rows,entries", [(600, 4095), (600, 4096), (600, 4097), (9000, 37), (9000, 4096), (9000, 4097)])
+def test_few_entries_are_read_in_place(rows, entries):
+    """Dense support vectors: a batch of up to 4,096 entries is read by the kernel where it lies in host memory, however many rows
+    they are spread over.  Either way the values are those of the same rows resident on the device, bit for bit, and the oracle's."""
+    rng = np.random.default_rng(rows + entries)
+    x, y = _blobs(rng, 3, 60, 9)
+    tr = D.from_dense(x, y)
+    prm = make_param(svm_type=0, kernel_type=2, gamma=0.3, C=2.0)
+    at = np.sort(rng.choice(rows * 9, size=entries, replace=False))
+    te = D.CsrData(np.searchsorted(at, np.arange(rows + 1, dtype=np.int64) * 9).astype(np.int64), (at % 9).astype(np.int32) + 1,
+                   rng.standard_normal(entries).astype(np.float32).astype(np.float64), np.zeros(rows))
+    gm = Model(0).train(tr, prm)
+    got = gm.predict(te)[1]
+    assert np.array_equal(got, gm.predict(Dataset(te).to_device())[1])
+    assert np.array_equal(got, gm.predict(te)[1])
+    om = O.Model(tr.ptr, tr.col, tr.val, tr.y, _oparam(prm))
+    assert np.abs(got - om.predict(te.ptr, te.col, te.val, 100)[1]).max() < 1e-6
+
+
 @pytest.mark.parametrize("groups", [1, 2, 3, 4, 5, 7])
 def test_indicator_groups(groups, monkeypatch):
     """A row sets one column of each one-hot group: so many matches are added one by one, up to four without a loop."""
