@@ -956,7 +956,7 @@ __device__ void sel_sort_here(const SelWorkspace &w, const SelGeom &g, const int
 // that sorted the lists by a bitonic network in LDS and looked the places up by bisection took 26.8 us, 49 with four
 // sides, in which the rest of the chip was idle; this takes 9 (bound by the launch and a chain of three memory latencies).  nu-SVC
 // 5,001 x 23 4.39 -> 4.06 ms, epsilon-SVR 40,000 x 90 96.8 -> 92.9.  Entries per wavefront 1 / 2 / 4 / 8: 92.5 / 92.8 / 93.5 /
-// 95.5 ms there, 848 / 846 / 843 / 840 on seven classes of 300,000 rows, where workgroups wait for room among other pairs'.
+// 95.5 ms there, 848 / 846 / 843 / 840 on seven classes of 300,000 rows, whose runs differ by more than that.
 #define SEL_RANK_T 1024
 #define SEL_RANK_EACH 2   // entries a wavefront takes
 #define SEL_RANK_ENTRIES (SEL_RANK_T / 64 * SEL_RANK_EACH)
@@ -989,8 +989,8 @@ __device__ __forceinline__ int sel_place(const uint64_t *key, const uint32_t *id
 }
 
 // Where a selection's ids go on the host, when it is to hear of them: pinned memory that the device can write, and a word behind
-// them that the host polls (as report_ids_kernel below, in a launch less: epsilon-SVR on 40,000 rows 91.5 -> 90.9 ms, seven
-// classes of 300,000 rows, where every launch waits its turn among other pairs', 877 -> 853).
+// them that the host polls (as report_ids_kernel below, in a launch less: epsilon-SVR on 40,000 rows 91.5 -> 90.9 ms; seven
+// classes of 300,000 rows level within the 3 % that its runs differ by).
 struct SelReport {
     int *ids = nullptr, *word_at = nullptr, word = 0;
 };
