@@ -956,7 +956,9 @@ __device__ void sel_sort_here(const SelWorkspace &w, const SelGeom &g, const int
 // that sorted the lists by a bitonic network in LDS and looked the places up by bisection took 26.8 us, 49 with four
 // sides, in which the rest of the chip was idle; this takes 9 (bound by the launch and a chain of three memory latencies).  nu-SVC
 // 5,001 x 23 4.39 -> 4.06 ms, epsilon-SVR 40,000 x 90 96.8 -> 92.9.  Entries per wavefront 1 / 2 / 4 / 8: 92.5 / 92.8 / 93.5 /
-// 95.5 ms there, 848 / 846 / 843 / 840 on seven classes of 300,000 rows, whose runs differ by more than that.
+// 95.5 ms there.  Among lanes, whose workgroups wait for room among other pairs', more entries would be better: seven classes of
+// 300,000 rows 848 / 846 / 843 / 840, of 500,000 rows 1,525 with two and 1,505 with eight (means of three and two runs; 1,498 when
+// one workgroup sorted).
 #define SEL_RANK_T 1024
 #define SEL_RANK_EACH 2   // entries a wavefront takes
 #define SEL_RANK_ENTRIES (SEL_RANK_T / 64 * SEL_RANK_EACH)
