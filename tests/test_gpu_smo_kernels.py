@@ -74,6 +74,25 @@ def test_update_f_below_262144_columns(n, ld_pad, shift, ws, rows, repeat, row_t
     assert np.array_equal(G.host(f_d), want)
 
 
+@pytest.mark.parametrize("n,rows", [(65, 255), (65, 256), (130, 257), (130, 1025), (200, 2111), (28672, 300), (28673, 300)])
+@pytest.mark.parametrize("row_type", [capi.ROW_F64, capi.ROW_F32])
+def test_update_f_wavefronts_in_turn(n, rows, row_type):
+    """Every wavefront's second and later groups, a last group of one row, three chunks of the working set (one of them without a
+    non-zero entry), and the line between one and two columns per thread."""
+    rng = np.random.default_rng(n + rows)
+    ws, ld, store = 3 * 1024, (n + 7) // 8 * 8, 50
+    k = rng.random((store, ld)).astype(np.float32 if row_type == capi.ROW_F32 else np.float64)
+    slots = rng.integers(0, store, size=ws).astype(np.int32)
+    ad = np.zeros(ws)
+    at = np.sort(np.concatenate([rng.permutation(1024)[:min(rows, 1024)], 2048 + rng.permutation(1024)[:max(min(rows, 2048) - 1024, 0)]]))
+    ad[at] = rng.standard_normal(len(at))
+    f = rng.standard_normal(n)
+    want = O.update_f(f, ad[at], np.ascontiguousarray(k[slots[at], :n].astype(np.float64)), n)
+    f_d, ad_d, k_d, s_d = G.dev(f), G.dev(ad), G.dev(k), G.dev(slots)
+    capi.call("tsvm_update_f", G.ptr(f_d), G.ptr(ad_d), ws, G.ptr(k_d), row_type, G.ptr(s_d), ld, n, 1, G.stream())
+    assert np.array_equal(G.host(f_d), want)
+
+
 @pytest.mark.parametrize("n,ws,ld_pad", [(300001, 64, 7), (262144, 33, 0), (270000, 40, 4)])
 @pytest.mark.parametrize("row_type", [capi.ROW_F64, capi.ROW_F32])
 def test_update_f_wide_and_repeated(n, ws, ld_pad, row_type):

@@ -459,11 +459,41 @@ __global__ __launch_bounds__(UF_T) void update_f_kernel(double *__restrict__ f, 
 // rows come in sixteen batches one memory latency apart: 27 us for 3,200 columns and 31 for 40,000.  Here a workgroup has
 // 64 * COLS columns and eight wavefronts; groups of R neighbouring rows are dealt to them in turn, so that all eight have theirs on
 // their way at once, and they add them in turn: the sums of a column stay one chain in the rows' order, handed on through
-// LDS.  Bound by that chain (500 additions and the hand-overs, some 3 us) and the compaction in front of it where columns are few, by
-// HBM where they are many.
+// LDS.  Bound by that chain where columns are few, by HBM where they are many.  A row of the chain costs its addition and whatever stands
+// between two of them: the coefficients lie in a register, a lane each, and come by v_readlane four rows ahead (read from LDS one
+// pair after another, each pair behind a wait, a row took 50 cycles; 26 with the hand-overs now), and a wavefront that asks for its
+// next rows (some 1,600 cycles of issue) holds up nobody, since the others wait for the turn's number and not at a barrier.  1,024 and 516
+// of 1,024 float rows, us: 3,200 columns 19.6 / 11.5 -> 15.9 / 9.9, 16,384 20.2 / 12.3 -> 17.1 / 10.8; with the selection behind it,
+// 516 rows: 40.1 -> 32.9 and 46.1 -> 38.5.
 #define UN_WAVES 8
-// (a barrier that waits for LDS only: rows stay on their way across it)
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+// The sums of a wavefront's columns on their way to the next: written, then the number of the turn (the LDS takes a wavefront's
+// accesses in order), and read behind that number until it is the wanted one.  Rows stay on their way meanwhile, across no barrier.
+template <int COLS>
+__device__ __forceinline__ void un_pass_turn(int *turn, int next, double *slot, const double (&sum)[COLS]) {
+    if constexpr (COLS == 1)
+        asm volatile("ds_write_b64 %0, %1\n\tds_write_b32 %2, %3" :: "v"(lds_at(slot)), "v"(sum[0]), "v"(lds_at(turn)), "v"(next) : "memory");
+    else
+        asm volatile("ds_write2_b64 %0, %1, %2 offset1:1\n\tds_write_b32 %3, %4"
+                     :: "v"(lds_at(slot)), "v"(sum[0]), "v"(sum[1]), "v"(lds_at(turn)), "v"(next) : "memory");
+}
+template <int COLS>
+__device__ __forceinline__ void un_take_turn(int *turn, int mine, double *slot, double (&sum)[COLS]) {
+    static_assert(COLS == 1 || COLS == 2, "columns per thread");
+    typedef double v2d __attribute__((ext_vector_type(2)));
+    int at;
+    do {
+        if constexpr (COLS == 1) {
+            asm volatile("ds_read_b32 %0, %2\n\tds_read_b64 %1, %3\n\ts_waitcnt lgkmcnt(0)"
+                         : "=&v"(at), "=&v"(sum[0]) : "v"(lds_at(turn)), "v"(lds_at(slot)) : "memory");
+        } else {
+            v2d both;
+            asm volatile("ds_read_b32 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)"
+                         : "=&v"(at), "=&v"(both) : "v"(lds_at(turn)), "v"(lds_at(slot)) : "memory");
+            sum[0] = both[0];
+            sum[1] = both[1];
+        }
+    } while (__builtin_amdgcn_readfirstlane(at) != mine);
+}
 template <typename TK, int COLS, int R, int NS>
 __global__ __launch_bounds__(64 * UN_WAVES, 4) void update_f_narrow_kernel(double *__restrict__ f, const double *__restrict__ alpha_diff,
                                                                         int ws, const TK *__restrict__ k_rows,
@@ -474,8 +504,8 @@ __global__ __launch_bounds__(64 * UN_WAVES, 4) void update_f_narrow_kernel(doubl
     __shared__ uint32_t mark_bits[NS > 0 ? UF_MAX_REPEAT : 1][2 * COLS];
     __shared__ double s_ad[UF_CHUNK];
     __shared__ int64_t s_off[UF_CHUNK];
-    __shared__ double s_sum[COLS][64];
-    __shared__ int s_wave_cnt[UN_WAVES];
+    __shared__ __align__(16) double s_sum[64 * COLS];
+    __shared__ int s_wave_cnt[UN_WAVES], s_turn;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t col_lo = (int64_t) blockIdx.x * 64 * COLS, j = col_lo + lane * COLS;
     const int64_t jc = j < n ? j : (n - 1) / COLS * COLS;   // (a lane behind the last column reads that column's vector)
@@ -508,6 +538,7 @@ __global__ __launch_bounds__(64 * UN_WAVES, 4) void update_f_narrow_kernel(doubl
     if (ws > 0) fetch_chunk(0);
     int mark = NS > 0 && tid < sf.n_marked ? sf.marked[tid] : -1;
     if (wave < repeat) fetch(wave);
+    if (tid == 0) s_turn = 0;
     if (NS > 0) {
         for (int e = tid; e < NS * SEL_BINS; e += T) (&lhist[0][0])[e] = 0;
         if (tid < UF_MAX_REPEAT * 2 * COLS) (&mark_bits[0][0])[tid] = 0;
@@ -528,6 +559,7 @@ __global__ __launch_bounds__(64 * UN_WAVES, 4) void update_f_narrow_kernel(doubl
     double sum[COLS];
 #pragma unroll
     for (int c = 0; c < COLS; ++c) sum[c] = 0.0;
+    int turns = 0;   // groups of the chunks before
     for (int base = 0; base < ws; base += UF_CHUNK) {
         // ordered compaction of this chunk's non-zero entries
         if (base > 0) fetch_chunk(base);
@@ -557,42 +589,62 @@ __global__ __launch_bounds__(64 * UN_WAVES, 4) void update_f_narrow_kernel(doubl
             }
         __syncthreads();
         // Groups of R rows are dealt to the wavefronts in turn: group g is wavefront g % UN_WAVES's, which asks for its next one as
-        // soon as it has added the last.
+        // soon as it has added the last.  s_turn is the group whose turn it is; a wavefront waits for its own and nothing else, so
+        // that another's requests hold nobody up.
         const int groups = (total + R - 1) / R;
         vec_t k[R];
+        double ad = 0.0;   // lane u's is the coefficient of the group's row u
         auto request = [&](int g) {
+            ad = s_ad[g * R + (lane & (R - 1)) < total ? g * R + (lane & (R - 1)) : total - 1];
 #pragma unroll
             for (int u = 0; u < R; ++u) k[u] = load_streaming((const vec_t *) (k_rows + s_off[g * R + u < total ? g * R + u : total - 1] + jc));
         };
         if (wave < groups) request(wave);
-        for (int g = 0; g < groups; ++g) {
-            if (wave == g % UN_WAVES) {
-                if (g > 0) {   // the sums so far come from the wavefront before
+#pragma unroll 1
+        for (int g = wave; g < groups; g += UN_WAVES) {
+            if (turns + g > 0) un_take_turn<COLS>(&s_turn, turns + g, s_sum + lane * COLS, sum);   // the sums so far come from the wavefront before
+            __builtin_amdgcn_s_setprio(2);   // (in front of the wavefronts that wait)
+            const int m = total - g * R;
+            if (m >= R) {
+                constexpr int AHEAD = 4;   // rows whose coefficient and values are made ready while one is added
+                double a[AHEAD], wide[AHEAD][COLS];
+                auto ready = [&](int u) {
+                    a[u % AHEAD] = readlane_f64(ad, u);
 #pragma unroll
-                    for (int c = 0; c < COLS; ++c) sum[c] = s_sum[c][lane];
+                    for (int c = 0; c < COLS; ++c) wide[u % AHEAD][c] = (double) k[u][c];
+                };
+#pragma unroll
+                for (int u = 0; u < AHEAD; ++u) ready(u);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < R; ++u) {
+#pragma unroll
+                    for (int c = 0; c < COLS; ++c) sum[c] = __builtin_fma(a[u % AHEAD], wide[u % AHEAD][c], sum[c]);
+                    if (u + AHEAD < R) ready(u + AHEAD);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-                const int m = total - g * R;
-                if (m >= R) {
+            } else {
 #pragma unroll
-                    for (int u = 0; u < R; ++u)
+                for (int u = 0; u < R; ++u)
+                    if (u < m) {
+                        const double a = readlane_f64(ad, u);
 #pragma unroll
-                        for (int c = 0; c < COLS; ++c) sum[c] = __builtin_fma(s_ad[g * R + u], (double) k[u][c], sum[c]);
-                } else {
-#pragma unroll
-                    for (int u = 0; u < R; ++u)
-                        if (u < m)
-#pragma unroll
-                            for (int c = 0; c < COLS; ++c) sum[c] = __builtin_fma(s_ad[g * R + u], (double) k[u][c], sum[c]);
-                }
-#pragma unroll
-                for (int c = 0; c < COLS; ++c) s_sum[c][lane] = sum[c];
+                        for (int c = 0; c < COLS; ++c) {
+                            TK v = k[u][c];
+                            asm("" : "+v"(v));   // (or the conversions of both branches would be made in front of them, and all be held)
+                            sum[c] = __builtin_fma(a, (double) v, sum[c]);
+                        }
+                    }
             }
-            lds_barrier();
-            if (wave == g % UN_WAVES && g + UN_WAVES < groups) request(g + UN_WAVES);
+            un_pass_turn<COLS>(&s_turn, turns + g + 1, s_sum + lane * COLS, sum);
+            __builtin_amdgcn_s_setprio(0);
+            if (g + UN_WAVES < groups) request(g + UN_WAVES);
         }
+        turns += groups;
+        __syncthreads();
         if (total > 0) {   // every wavefront goes on from the chunk's sums
 #pragma unroll
-            for (int c = 0; c < COLS; ++c) sum[c] = s_sum[c][lane];
+            for (int c = 0; c < COLS; ++c) sum[c] = s_sum[lane * COLS + c];
             __syncthreads();
         }
     }
@@ -1201,11 +1253,13 @@ static void dispatch_update_f(double *f, const double *alpha_diff, int ws_size, 
     // Vector loads need every row start aligned to the vector and the last vector inside the padded row.
     const size_t esz = row_type == TSVM_ROW_F32 ? 4 : 8;
     auto aligned = [&](int cols) { return (uintptr_t) k_rows % (cols * esz) == 0 && ld % cols == 0; };
-    // Few columns: wavefronts that take the rows in turn, one column per thread while that makes do with one workgroup per CU (more
-    // workgroups leave some CUs two in turn), and on to 65,536 columns of floats with two, to 32,768 of doubles.  Of 2,048
-    // rows in slots, us a call, one thread per column and all rows / wavefronts in turn:
+    // Few columns: wavefronts that take the rows in turn, and on to 65,536 columns of floats with two columns per thread, to 32,768 of
+    // doubles.  One column per thread up to 28,672 columns of floats, twice as many workgroups whose first pass of the selection then ends in
+    // more atomics on the same addresses (with the selection, 516 rows, two columns / one: 20,000 43.2 / 39.5 us, 28,000
+    // 44.5 / 41.8, 40,000 46.1 / 50.9), and up to 16,384 of doubles (20,000 44.4 / 45.7).  Of 2,048
+    // rows in slots, us a call, one thread per column and all rows / wavefronts in turn (two columns per thread):
     //   non-zero rows     60          250          500         1,024
-    //   floats  20,000   8.1 /  5.4  21.4 /  9.8  29.3 / 15.2   41.8 /  26.1
+    //   floats  20,000   8.1 /  5.2  21.4 /  9.2  29.3 / 14.6   41.8 /  24.7   (one column per thread: 5.1, 8.6, 12.3, 18.5)
     //           65,536  15.6 /  6.9  24.9 / 15.1  34.1 / 24.6   50.0 /  44.7
     //          100,000  17.6 /  8.8  28.7 / 22.0  41.2 / 38.5   64.7 /  71.2   (here and below: four columns per thread)
     //          180,000  20.4 / 13.6  39.7 / 37.3  64.6 / 67.2  112.2 / 131.5
@@ -1218,7 +1272,7 @@ static void dispatch_update_f(double *f, const double *alpha_diff, int ws_size, 
     // four calls of 574 to 608.
     const bool narrow = n <= (int64_t) 64 * 256 * (row_type == TSVM_ROW_F32 ? 4 : 2);
     if (narrow) {
-        const bool one = n <= (int64_t) 64 * 256 || !aligned(2);
+        const bool one = n <= (row_type == TSVM_ROW_F32 ? 28672 : 16384) || !aligned(2);
         if (row_type == TSVM_ROW_F32) {
             if (one) launch_update_f_narrow<float, 1, 32, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);
             else launch_update_f_narrow<float, 2, 16, NS>(f, alpha_diff, ws_size, k_rows, slots, ld, n, repeat, sf, s);

@@ -88,12 +88,6 @@ __device__ __forceinline__ int wave_first_argmin(const double (&x)[E], int base,
     return wave_argmin<E, false>(x, base, value, m, at, twice);
 }
 
-// The LDS address of a __shared__ object as the ds instructions take it.
-template <typename T>
-__device__ __forceinline__ unsigned lds_at(const T *p) {
-    return (unsigned) (uintptr_t) (const __attribute__((address_space(3))) T *) p;
-}
-
 // One wavefront's best candidate for the others: the workgroup's minimum is taken over W of these.
 struct __align__(16) SvCand {
     double v;

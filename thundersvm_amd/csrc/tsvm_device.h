@@ -344,6 +344,11 @@ __device__ __forceinline__ double dpp_f64(double v) {
     int lo = dpp_i32<CTRL, ROW_MASK>(__double2loint(v)), hi = dpp_i32<CTRL, ROW_MASK>(__double2hiint(v));
     return __hiloint2double(hi, lo);
 }
+// The LDS address of a __shared__ object as the ds instructions take it.
+template <typename T>
+__device__ __forceinline__ unsigned lds_at(const T *p) {
+    return (unsigned) (uintptr_t) (const __attribute__((address_space(3))) T *) p;
+}
 __device__ __forceinline__ double readlane_f64(double v, int lane) {
     int lo = __builtin_amdgcn_readlane(__double2loint(v), lane), hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
     return __hiloint2double(hi, lo);
