@@ -450,6 +450,22 @@ int tsvm_predict_dec_values_dense(const double *sv_x, int64_t ldx, int d, const 
                                   int max_ones, int kernel_type, double gamma, double coef0, int degree, double *partial,
                                   double *dec_values, tsvm_stream stream);
 
+/* The same for several groups of rows in one launch, each with a model of its own whose support vectors are rows of the same dense matrix
+ * x as the rows themselves (the folds of a cross-validation: the reference predicts them one after another,
+ * src/thundersvm/model/svmmodel.cpp:50-66).  All models have n_classes classes; d <= 128, all columns through the matrix cores.
+ * Their padded columns follow one another in col_map (rows of x) and coef_t, their chunks in `chunks`.  rows[0..m): the rows of x to
+ * predict, group by group, row_group[r] the group of entry r; group g has class_chunk_start[g * (n_classes + 1) ..] (first chunk of
+ * every class, counted from the group's first) and rho[g * P ..].  tasks: one for every chunk of a group and 64 of its entries:
+ * entries row_begin .. row_end - 1 (the group's end; the workgroup takes the first 64), chunk `chunk`, which is the group's number `part`.
+ * partial: workspace of (most chunks of a group) * m * (n_classes - 1) doubles. */
+typedef struct tsvm_predict_task {
+    int row_begin, row_end, chunk, part;
+} tsvm_predict_task;
+int tsvm_predict_groups_dense(const double *x, int64_t ldx, int d, const double *sd, const int *col_map, int64_t n_pad, const double *coef_t,
+                              const int *chunks, const tsvm_predict_task *tasks, int n_tasks, const int *rows, int64_t m,
+                              const int *row_group, const int *class_chunk_start, const double *rho, int n_classes, int kernel_type, double gamma,
+                              double coef0, int degree, double *partial, double *dec_values, tsvm_stream stream);
+
 #ifdef __cplusplus
 }
 #endif

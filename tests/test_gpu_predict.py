@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import oracle_lib as O
+from thundersvm_amd import capi
 from thundersvm_amd import data as D
 from thundersvm_amd.model import Dataset, Model, make_param
 
@@ -325,3 +326,28 @@ def test_labels_by_votes_on_the_device_and_on_the_host(k, rows, dense):
         for batch in (-1, 700):
             labels, dec = m.predict(d, batch)
             assert np.array_equal(labels, m.label[_votes(dec, k)].astype(np.float64))
+
+
+@pytest.mark.parametrize("svm_type,classes", [(capi.EPSILON_SVR, 2), (capi.NU_SVR, 2), (capi.C_SVC, 3), (capi.ONE_CLASS, 2)])
+@pytest.mark.parametrize("n,d,kernel,folds", [(40, 3, capi.RBF, 5), (129, 16, capi.POLY, 2), (645, 17, capi.RBF, 10), (1003, 127, capi.LINEAR, 3),
+                                              (1003, 128, capi.RBF, 3), (3300, 5, capi.RBF, 3)])
+def test_folds_predicted_together(svm_type, classes, n, d, kernel, folds, monkeypatch):
+    """A cross-validation whose folds are predicted by one launch gives what one call per fold gives: ragged blocks of rows, a fold
+    of more than one batch (3,300 rows of three classes), one column too many for the kernel (128 features make 129 columns)."""
+    rng = np.random.default_rng(n + d)
+    x = rng.standard_normal((n, d)).astype(np.float32)
+    c = rng.permutation(np.arange(n) % classes)
+    # (folds are cut label by label, whatever the model: svmmodel.cpp:31-71)
+    y = np.sign(x[:, 0]) if svm_type in (capi.EPSILON_SVR, capi.NU_SVR) else np.ones(n) if svm_type == capi.ONE_CLASS else c + 1.0
+    if svm_type == capi.C_SVC:
+        x[:, :2] += 1.5 * np.stack([c, c * c], axis=1)
+    data = D.from_dense(x, y)
+    prm = make_param(svm_type=svm_type, kernel_type=kernel, C=1.0, gamma=0.1 / d, nu=0.3, p=0.05, degree=2)
+    together = Model(svm_type).cross_validation(Dataset(data), prm, folds)
+    monkeypatch.setenv("TSVM_PREDICT_UNFUSED", "1")
+    one_by_one = Model(svm_type).cross_validation(Dataset(data), prm, folds)
+    if svm_type in (capi.EPSILON_SVR, capi.NU_SVR):
+        # (the same kernel values and coefficients, their sums in another order: 1,000 terms of 2^-53 each, coefficients of at most 1)
+        np.testing.assert_allclose(together, one_by_one, rtol=0, atol=1e-9 * (1 + np.abs(one_by_one).max()))
+    else:
+        assert np.mean(together != one_by_one) <= 0.002   # (a decision value of about zero may fall on either side)

@@ -31,7 +31,8 @@ __global__ __launch_bounds__(256, 2) void predict_dense_stream_kernel(
     const double *__restrict__ x, int64_t ldx, const int *__restrict__ col_map, int d, const double *__restrict__ sd_x,
     const uint64_t *__restrict__ mask_x, const double *__restrict__ a, int64_t lda, int m, const double *__restrict__ sd_a,
     const uint64_t *__restrict__ mask_a, int max_ones, KernelParam kp_in, const double *__restrict__ coef_t,
-    const int *__restrict__ chunks, unsigned m_blocks, double *__restrict__ partial, int nc_out) {
+    const int *__restrict__ chunks, unsigned m_blocks, double *__restrict__ partial, int nc_out, const tsvm_predict_task *__restrict__ tasks,
+    const int *__restrict__ a_idx) {
     constexpr int TI = 2;
     constexpr int BM = GrShape<TI>::BM;
     constexpr int KTILE = GrShape<TI>::KTILE;
@@ -54,14 +55,23 @@ __global__ __launch_bounds__(256, 2) void predict_dense_stream_kernel(
     // Workgroups are dealt to the eight XCDs in turn, so every XCD gets an eighth of every chunk's row blocks, and all of them
     // have the same chunk in their L2 at a time.  A run of chunks per XCD would leave those with the small classes' short chunks
     // idle: 50,000 rows of 54 columns against 16,076 support vectors in seven classes 3.07 -> 1.76 ms.
-    const int i0 = (int) (blockIdx.x % m_blocks) * BM;
-    const unsigned chunk = blockIdx.x / m_blocks;
-    const unsigned jt0 = (unsigned) chunks[2 * chunk], jt1 = (unsigned) chunks[2 * chunk + 1];
+    // (Groups of rows that have their own support vectors come with a table of who does what, and their rows by number.)
+    tsvm_predict_task t;
+    if (tasks) {
+        t = tasks[blockIdx.x];
+    } else {
+        t.row_begin = (int) (blockIdx.x % m_blocks) * BM;
+        t.row_end = m;
+        t.chunk = t.part = (int) (blockIdx.x / m_blocks);
+    }
+    const int i0 = t.row_begin;
+    const unsigned jt0 = (unsigned) chunks[2 * t.chunk], jt1 = (unsigned) chunks[2 * t.chunk + 1];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
     const int wi = wave >> 1, wj = wave & 1;
-    const int m_last = m - 1;
+    const int m_last = t.row_end - 1;
+    const auto batch_row = [&](int r) { return a_idx ? a_idx[min(r, m_last)] : min(r, m_last); };
     const int a_row = tid / A_TPR, a_k = (tid % A_TPR) * (4 * A_VEC);
     const int b_row = tid >> 1, b_k = (tid & 1) * (4 * B_VEC);
     const int lrow = lane & 15;
@@ -72,11 +82,11 @@ __global__ __launch_bounds__(256, 2) void predict_dense_stream_kernel(
 
     if (tid < 32) exp_tab[tid] = TSVM_EXP2F_TAB[tid];
     if (tid < BM) {
-        const int r = min(i0 + tid, m_last);
+        const int r = batch_row(i0 + tid);
         s_sdi[tid] = sd_a ? sd_a[r] : 0.0;
         s_mi[tid] = IND ? mask_a[r] : 0;
     }
-    const double *a_ptr = a + (uint64_t) (uint32_t) min(i0 + a_row, m_last) * (uint32_t) lda;
+    const double *a_ptr = a + (uint64_t) (uint32_t) batch_row(i0 + a_row) * (uint32_t) lda;
 
     const int n_kt = K_TILES == 1 ? (d > 0 ? 1 : 0) : (d + KTILE - 1) / KTILE;
     const int n_ks_last = (d - (n_kt - 1) * KTILE + 3) / 4;
@@ -302,7 +312,7 @@ __global__ __launch_bounds__(256, 2) void predict_dense_stream_kernel(
     __syncthreads();
     for (int e = tid; e < BM * nc_out; e += 256) {
         const int r = e / nc_out, c = e % nc_out;
-        if (i0 + r < m) partial[((int64_t) chunk * m + i0 + r) * nc_out + c] = red[r * NC + c] + red[(BM + r) * NC + c];
+        if (i0 + r <= m_last) partial[((int64_t) t.part * m + i0 + r) * nc_out + c] = red[r * NC + c] + red[(BM + r) * NC + c];
     }
 }
 
@@ -344,11 +354,12 @@ __global__ __launch_bounds__(256, 2) void predict_dense_tile_kernel(
 }
 
 // dec[r * P + p] for pair p = (i < j): the chunks of class i under coefficient row j - 1, then the chunks of class j
-// under coefficient row i, each in chunk order, minus rho[p] (the order of kernelmatrix_kernel.cpp:129-143).
+// under coefficient row i, each in chunk order, minus rho[p] (the order of kernelmatrix_kernel.cpp:129-143).  row_group: groups of
+// rows have class_chunk_start and rho of their own.
 __global__ __launch_bounds__(256) void predict_combine_kernel(const double *__restrict__ partial, int64_t m, int nc,
                                                               const int *__restrict__ class_chunk_start,
                                                               const double *__restrict__ rho, int n_classes,
-                                                              double *__restrict__ dec) {
+                                                              const int *__restrict__ row_group, double *__restrict__ dec) {
     const int64_t P = (int64_t) n_classes * (n_classes - 1) / 2;
     const int64_t idx = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= m * P) return;
@@ -359,6 +370,10 @@ __global__ __launch_bounds__(256) void predict_combine_kernel(const double *__re
         ++i;
     }
     const int j = i + 1 + p;
+    if (row_group) {
+        class_chunk_start += (int64_t) row_group[r] * (n_classes + 1);
+        rho += row_group[r] * P;
+    }
     double s = 0.0;
     for (int ch = class_chunk_start[i]; ch < class_chunk_start[i + 1]; ++ch) s += partial[((int64_t) ch * m + r) * nc + (j - 1)];
     double t = 0.0;
@@ -388,6 +403,56 @@ __global__ __launch_bounds__(VOTE_T) void predict_votes_kernel(const double *__r
 }
 
 static int nc_template(int nc) { return nc <= 4 ? nc : nc <= 6 ? 6 : 8; }
+
+// The variant of the kernel for the model's shape: its kernel, coefficient rows (`stride`), indicator columns and K tiles.
+static void launch_stream(dim3 grid, const double *sv_x, int64_t ldx, const int *col_map, int d, const double *sd_sv, const uint64_t *mask_sv,
+                          const double *a, int64_t lda, int m, const double *sd_a, const uint64_t *mask_a, int max_ones, const KernelParam &kp,
+                          const double *coef_t, int stride, const int *chunks, unsigned m_blocks, double *partial, int nc,
+                          const tsvm_predict_task *tasks, const int *a_idx, hipStream_t s) {
+#define PD_STREAM(KTYPE, NC_, IND_, KT_)                                                                                        \
+    hipLaunchKernelGGL((predict_dense_stream_kernel<KTYPE, NC_, IND_, KT_>), grid, dim3(256), 0, s, sv_x, ldx, col_map, d, sd_sv,    \
+               mask_sv, a, lda, m, sd_a, mask_a, max_ones, kp, coef_t, chunks, m_blocks, partial, nc, tasks, a_idx)
+#define PD_NC(KTYPE, IND_, KT_)                         \
+    switch (stride) {                                   \
+        case 1: PD_STREAM(KTYPE, 1, IND_, KT_); break;  \
+        case 2: PD_STREAM(KTYPE, 2, IND_, KT_); break;  \
+        case 3: PD_STREAM(KTYPE, 3, IND_, KT_); break;  \
+        case 4: PD_STREAM(KTYPE, 4, IND_, KT_); break;  \
+        case 6: PD_STREAM(KTYPE, 6, IND_, KT_); break;  \
+        default: PD_STREAM(KTYPE, 8, IND_, KT_); break; \
+    }
+#define PD_RBF(IND_)                              \
+    do {                                          \
+        if (d <= 16) PD_NC(TSVM_RBF, IND_, 1)     \
+        else PD_NC(TSVM_RBF, IND_, 2)             \
+    } while (0)
+#define PD_KIND(KTYPE)                            \
+    do {                                          \
+        if (mask_sv) {                            \
+            if (d <= 16) PD_NC(KTYPE, 5, 1)       \
+            else PD_NC(KTYPE, 5, 2)               \
+        } else {                                  \
+            if (d <= 16) PD_NC(KTYPE, 0, 1)       \
+            else PD_NC(KTYPE, 0, 2)               \
+        }                                         \
+    } while (0)
+    switch (kp.kernel_type) {
+        case TSVM_LINEAR: PD_KIND(TSVM_LINEAR); break;
+        case TSVM_POLY: PD_KIND(TSVM_POLY); break;
+        case TSVM_SIGMOID: PD_KIND(TSVM_SIGMOID); break;
+        default:
+            if (mask_sv && max_ones == 1) PD_RBF(1);
+            else if (mask_sv && max_ones == 2) PD_RBF(2);
+            else if (mask_sv && max_ones == 3) PD_RBF(3);
+            else if (mask_sv && max_ones == 4) PD_RBF(4);
+            else PD_KIND(TSVM_RBF);
+            break;
+    }
+#undef PD_RBF
+#undef PD_KIND
+#undef PD_NC
+#undef PD_STREAM
+}
 
 extern "C" {
 
@@ -442,49 +507,8 @@ int tsvm_predict_dec_values_dense(const double *sv_x, int64_t ldx, int d, const 
             const unsigned m_blocks = (unsigned) ((m + 63) / 64);
             TSVM_REQUIRE((int64_t) m_blocks * n_chunks < (int64_t) 0x7fffffff, "tsvm_predict_dec_values_dense: grid too large");
             const dim3 grid(m_blocks * (unsigned) n_chunks);
-#define PD_STREAM(KTYPE, NC_, IND_, KT_)                                                                                        \
-    hipLaunchKernelGGL((predict_dense_stream_kernel<KTYPE, NC_, IND_, KT_>), grid, block, 0, tsvm_s(stream), sv_x, ldx, col_map, d, \
-                       sd_sv, mask_sv, a, lda, (int) m, sd_a, mask_a, max_ones, kp, coef_t, chunks, m_blocks, partial, nc)
-#define PD_NC(KTYPE, IND_, KT_)                         \
-    switch (stride) {                                   \
-        case 1: PD_STREAM(KTYPE, 1, IND_, KT_); break;  \
-        case 2: PD_STREAM(KTYPE, 2, IND_, KT_); break;  \
-        case 3: PD_STREAM(KTYPE, 3, IND_, KT_); break;  \
-        case 4: PD_STREAM(KTYPE, 4, IND_, KT_); break;  \
-        case 6: PD_STREAM(KTYPE, 6, IND_, KT_); break;  \
-        default: PD_STREAM(KTYPE, 8, IND_, KT_); break; \
-    }
-#define PD_RBF(IND_)                              \
-    do {                                          \
-        if (d <= 16) PD_NC(TSVM_RBF, IND_, 1)     \
-        else PD_NC(TSVM_RBF, IND_, 2)             \
-    } while (0)
-#define PD_KIND(KTYPE)                            \
-    do {                                          \
-        if (mask_sv) {                            \
-            if (d <= 16) PD_NC(KTYPE, 5, 1)       \
-            else PD_NC(KTYPE, 5, 2)               \
-        } else {                                  \
-            if (d <= 16) PD_NC(KTYPE, 0, 1)       \
-            else PD_NC(KTYPE, 0, 2)               \
-        }                                         \
-    } while (0)
-            switch (kernel_type) {
-                case TSVM_LINEAR: PD_KIND(TSVM_LINEAR); break;
-                case TSVM_POLY: PD_KIND(TSVM_POLY); break;
-                case TSVM_SIGMOID: PD_KIND(TSVM_SIGMOID); break;
-                default:
-                    if (mask_sv && max_ones == 1) PD_RBF(1);
-                    else if (mask_sv && max_ones == 2) PD_RBF(2);
-                    else if (mask_sv && max_ones == 3) PD_RBF(3);
-                    else if (mask_sv && max_ones == 4) PD_RBF(4);
-                    else PD_KIND(TSVM_RBF);
-                    break;
-            }
-#undef PD_RBF
-#undef PD_KIND
-#undef PD_NC
-#undef PD_STREAM
+            launch_stream(grid, sv_x, ldx, col_map, d, sd_sv, mask_sv, a, lda, (int) m, sd_a, mask_a, max_ones, kp, coef_t, stride, chunks, m_blocks,
+                          partial, nc, nullptr, nullptr, tsvm_s(stream));
         } else {
             const unsigned m_blocks = (unsigned) ((m + 127) / 128);
             TSVM_REQUIRE((int64_t) m_blocks * n_chunks < (int64_t) 0x7fffffff, "tsvm_predict_dec_values_dense: grid too large");
@@ -505,7 +529,34 @@ int tsvm_predict_dec_values_dense(const double *sv_x, int64_t ldx, int d, const 
     }
     const int64_t P = (int64_t) n_classes * nc / 2;
     hipLaunchKernelGGL(predict_combine_kernel, dim3((unsigned) ((m * P + 255) / 256)), block, 0, tsvm_s(stream), partial, m, nc,
-                       class_chunk_start, rho, n_classes, dec_values);
+                       class_chunk_start, rho, n_classes, nullptr, dec_values);
+    TSVM_LAUNCH_CHECK();
+    return 0;
+}
+
+int tsvm_predict_groups_dense(const double *x, int64_t ldx, int d, const double *sd, const int *col_map, int64_t n_pad, const double *coef_t,
+                              const int *chunks, const tsvm_predict_task *tasks, int n_tasks, const int *rows, int64_t m,
+                              const int *row_group, const int *class_chunk_start, const double *rho, int n_classes, int kernel_type, double gamma,
+                              double coef0, int degree, double *partial, double *dec_values, tsvm_stream stream) {
+    TSVM_REQUIRE(x && col_map && coef_t && chunks && tasks && rows && row_group && class_chunk_start && rho && partial && dec_values,
+                 "tsvm_predict_groups_dense: null pointer");
+    TSVM_REQUIRE(n_classes >= 2 && m >= 0 && m <= 0x7fff0000 && n_tasks >= 0 && n_pad >= 0 && n_pad % GR_BN == 0 && n_pad <= 0x7fff0000,
+                 "tsvm_predict_groups_dense: bad size");
+    TSVM_REQUIRE(ldx % 8 == 0 && d >= 0 && d <= ldx && d <= 128 && ldx <= 0x7fffffff && (uintptr_t) x % 32 == 0,
+                 "tsvm_predict_groups_dense: d %d (at most 128 and ldx), ldx %lld (a multiple of 8), x 32-byte aligned", d, (long long) ldx);
+    TSVM_REQUIRE(kernel_type >= 0 && kernel_type < TSVM_PRECOMPUTED, "tsvm_predict_groups_dense: kernel type %d", kernel_type);
+    TSVM_REQUIRE(kernel_type != TSVM_RBF || sd, "tsvm_predict_groups_dense: RBF needs self dot products");
+    const int nc = n_classes - 1, stride = tsvm_predict_nc_stride(n_classes, d, 0);
+    TSVM_REQUIRE(stride > 0, "tsvm_predict_groups_dense: %d classes are too many", n_classes);
+    if (m == 0) return 0;
+    if (n_tasks > 0) {
+        launch_stream(dim3((unsigned) n_tasks), x, ldx, col_map, d, sd, nullptr, x, ldx, (int) m, sd, nullptr, 0, KernelParam{kernel_type, degree, gamma, coef0},
+                      coef_t, stride, chunks, 1, partial, nc, tasks, rows, tsvm_s(stream));
+        TSVM_LAUNCH_CHECK();
+    }
+    const int64_t P = (int64_t) n_classes * nc / 2;
+    hipLaunchKernelGGL(predict_combine_kernel, dim3((unsigned) ((m * P + 255) / 256)), dim3(256), 0, tsvm_s(stream), partial, m, nc, class_chunk_start,
+                       rho, n_classes, row_group, dec_values);
     TSVM_LAUNCH_CHECK();
     return 0;
 }

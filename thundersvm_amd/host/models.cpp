@@ -182,14 +182,23 @@ void SvmModel::train_folds(const DataSet &dataset, const std::vector<Fold> &fold
         std::vector<SmallBatch *> batches;
         for (Begun &b : begun) batches.push_back(&b.training.small);
         SmallBatch::run(batches, begun[0].model->param.epsilon, begun[0].model->max_iter);
+        std::vector<FoldRows> with;
         for (Begun &b : begun) {
-            SvmModel &m = *b.model;
             b.training.finish(b.training.small);
-            if (!m.sv_indices.empty()) m.sv_k_mat.reset(new KernelMatrix(*b.rows, m.sv_indices.data(), m.sv_indices.size(), m.param));
-            const std::unique_ptr<DataSet> test = rows_of(folds[b.k].test_idx, {});
-            std::vector<float_type> dec;
-            m.predict_dec_values(*test, dec, 1000);
-            take(b.k, m, dec);
+            with.push_back({b.model, &folds[b.k].train_idx, &folds[b.k].test_idx});
+        }
+        std::vector<std::vector<float_type>> dec;
+        const bool together = begun.size() > 1 && predict_folds(*all, with, dec);
+        for (size_t i = 0; i < begun.size(); ++i) {
+            Begun &b = begun[i];
+            SvmModel &m = *b.model;
+            if (!together) {
+                dec.resize(begun.size());
+                if (!m.sv_indices.empty()) m.sv_k_mat.reset(new KernelMatrix(*b.rows, m.sv_indices.data(), m.sv_indices.size(), m.param));
+                const std::unique_ptr<DataSet> test = rows_of(folds[b.k].test_idx, {});
+                m.predict_dec_values(*test, dec[i], FOLD_BATCH);
+            }
+            take(b.k, m, dec[i]);
             b.training = Training();
             b.rows.reset();
         }

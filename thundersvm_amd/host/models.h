@@ -80,6 +80,14 @@ protected:
     // trains model_of(k) on fold k of the dataset's instances and hands it over with the decision values of the others
     static void train_folds(const DataSet &dataset, const std::vector<Fold> &folds, const SvmParam &param, const std::function<SvmModel &(size_t)> &model_of,
                             const std::function<void(size_t, SvmModel &, std::vector<float_type> &)> &take);
+    // Decision values of several folds at once, each fold's rows by its own model, whose support vectors are rows of the same dense
+    // matrix: dec[k] as model k's predict_dec_values would have them.  False when the kernels do not take the models' shape.
+    static constexpr int FOLD_BATCH = 1000;   // rows of a fold that are predicted at a time
+    struct FoldRows {
+        const SvmModel *model;
+        const std::vector<int> *train_idx, *test_idx;
+    };
+    static bool predict_folds(const DeviceRows &all, const std::vector<FoldRows> &folds, std::vector<std::vector<float_type>> &dec);
     void copy_settings(const SvmModel &other);
     // the two halves for a model of one binary problem
     struct SingleProblem {
@@ -99,6 +107,7 @@ protected:
     // the model as the prediction kernels read it (support vectors in HBM, coefficients by padded column)
     struct PredictPlan;
     const PredictPlan &predict_plan() const;
+    void pad_classes(int stride, std::vector<int> &class_tile, std::vector<int> &col_map, std::vector<float_type> &coef_t) const;
     // one batch, rows already on the device as a dense matrix; false when the kernels do not take this model's shape
     bool predict_batch_fused(const PredictPlan &plan, const kernel_type *a, int64_t lda, const kernel_type *sd_a, size_t m,
                              bool indicator_values, float_type *dec_out, int *winner_out) const;

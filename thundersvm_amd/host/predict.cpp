@@ -12,6 +12,26 @@
 using tsvm::abi_check;
 using tsvm::DeviceBuffer;
 
+namespace {
+struct OneUpload {   // several arrays that go to the device in one copy, each at a multiple of 256 bytes
+    std::vector<tsvm::HostStaging::Part> parts;
+    size_t at = 0;
+    size_t add(const void *from, size_t bytes) {
+        const size_t here = at;
+        if (bytes) parts.push_back({from, bytes, at});
+        at = (at + bytes + 255) / 256 * 256;
+        return here;
+    }
+    template <typename T>
+    size_t add(const std::vector<T> &v) { return add(v.data(), v.size() * sizeof(T)); }
+    const char *send(DeviceBuffer<char> &to) const {
+        to.resize(std::max<size_t>(at, 256));
+        tsvm::HostStaging::instance().upload(to.data(), parts, tsvm::work_stream());
+        return to.data();
+    }
+};
+}  // namespace
+
 struct SvmModel::PredictPlan {
     DeviceBuffer<char> arrays;      // all of the following, uploaded together
     // for both paths
@@ -35,6 +55,32 @@ struct SvmModel::PredictPlan {
     mutable DeviceBuffer<int> mask_max;
 };
 
+// The padded columns of the support vectors (class_tile: first 128-column tile of every class, n_classes + 1) appended to
+// col_map and coef_t.
+void SvmModel::pad_classes(int stride, std::vector<int> &class_tile, std::vector<int> &col_map, std::vector<float_type> &coef_t) const {
+    const size_t T = sv->size(), first = col_map.size();
+    class_tile.assign(n_classes + 1, 0);
+    for (int c = 0; c < n_classes; ++c) class_tile[c + 1] = class_tile[c] + (n_sv[c] + 127) / 128;
+    const size_t n_pad = (size_t) class_tile[n_classes] * 128;
+    col_map.resize(first + n_pad, 0);
+    coef_t.resize((first + n_pad) * stride, 0.0);
+    int sv_start = 0;
+    for (int c = 0; c < n_classes; ++c) {
+        const size_t p0 = first + (size_t) class_tile[c] * 128, p1 = first + (size_t) class_tile[c + 1] * 128;
+        for (size_t p = p0; p < p1; ++p) {
+            const int t = (int) (p - p0);
+            if (t < n_sv[c]) {
+                const int l = sv_start + t;
+                col_map[p] = l;
+                for (int r = 0; r < n_classes - 1; ++r) coef_t[p * stride + r] = coef[(size_t) r * T + l];
+            } else {
+                col_map[p] = sv_start;   // a valid row; its coefficients stay zero
+            }
+        }
+        sv_start += n_sv[c];
+    }
+}
+
 const SvmModel::PredictPlan &SvmModel::predict_plan() const {
     if (predict_plan_) return *predict_plan_;
     // the support vectors' device copy is built by the first predict call and kept for the next ones (the
@@ -43,7 +89,6 @@ const SvmModel::PredictPlan &SvmModel::predict_plan() const {
     auto plan = std::make_shared<PredictPlan>();
     PredictPlan &P = *plan;
     const DeviceRows &R = sv_k_mat->rows();
-    const size_t T = sv->size();
     std::vector<int> sv_start(n_classes, 0);
     for (int c = 1; c < n_classes; ++c) sv_start[c] = sv_start[c - 1] + n_sv[c - 1];
     std::vector<int> col_map;
@@ -53,41 +98,16 @@ const SvmModel::PredictPlan &SvmModel::predict_plan() const {
     P.stride = R.dense ? tsvm_predict_nc_stride(n_classes, d, masks) : 0;
     if (P.stride > 0) {
         P.many_features = d > 128 && !masks;
-        P.class_tile.assign(n_classes + 1, 0);
-        for (int c = 0; c < n_classes; ++c) P.class_tile[c + 1] = P.class_tile[c] + (n_sv[c] + 127) / 128;
+        pad_classes(P.stride, P.class_tile, col_map, coef_t);
         P.n_pad = (int64_t) P.class_tile[n_classes] * 128;
-        col_map.assign((size_t) P.n_pad, 0);
-        coef_t.assign((size_t) P.n_pad * P.stride, 0.0);
-        const int km1 = n_classes - 1;
-        for (int c = 0; c < n_classes; ++c) {
-            const int64_t p0 = (int64_t) P.class_tile[c] * 128, p1 = (int64_t) P.class_tile[c + 1] * 128;
-            for (int64_t p = p0; p < p1; ++p) {
-                const int t = (int) (p - p0);
-                if (t < n_sv[c]) {
-                    const int l = sv_start[c] + t;
-                    col_map[p] = l;
-                    for (int r = 0; r < km1; ++r) coef_t[(size_t) p * P.stride + r] = coef[(size_t) r * T + l];
-                } else {
-                    col_map[p] = sv_start[c];   // a valid row; its coefficients stay zero
-                }
-            }
-        }
     }
     // (eight arrays, most of them some bytes: uploads of 10 us each)
-    std::vector<tsvm::HostStaging::Part> parts;
-    size_t at = 0;
-    auto add = [&](const void *from, size_t bytes) {
-        const size_t here = at;
-        if (bytes) parts.push_back({from, bytes, at});
-        at = (at + bytes + 255) / 256 * 256;
-        return here;
-    };
+    OneUpload up;
+    const auto add = [&](const void *from, size_t bytes) { return up.add(from, bytes); };
     const size_t rho_at = add(rho.data(), rho.size() * sizeof(float_type)), start_at = add(sv_start.data(), sv_start.size() * sizeof(int));
     const size_t count_at = add(n_sv.data(), n_sv.size() * sizeof(int)), coef_at = add(coef.data(), coef.size() * sizeof(float_type));
     const size_t map_at = add(col_map.data(), col_map.size() * sizeof(int)), coef_t_at = add(coef_t.data(), coef_t.size() * sizeof(float_type));
-    P.arrays.resize(std::max<size_t>(at, 256));
-    tsvm::HostStaging::instance().upload(P.arrays.data(), parts, tsvm::work_stream());
-    const char *const base = P.arrays.data();
+    const char *const base = up.send(P.arrays);
     P.rho = (const float_type *) (base + rho_at);
     P.sv_start = (const int *) (base + start_at);
     P.sv_count = (const int *) (base + count_at);
@@ -258,6 +278,76 @@ void SvmModel::predict_dec_values(const DataSet &dataset, std::vector<float_type
         }
     }
     predict_dec_values(dataset.rows(), dec, batch_size, winner);
+}
+
+bool SvmModel::predict_folds(const DeviceRows &all, const std::vector<FoldRows> &folds, std::vector<std::vector<float_type>> &dec) {
+    const SvmModel &first = *folds[0].model;
+    const int k = first.n_classes, P = first.n_binary_models, d = (int) all.n_features;
+    const int stride = all.dense && d <= 128 && !getenv("TSVM_PREDICT_UNFUSED") ? tsvm_predict_nc_stride(k, d, 0) : 0;
+    if (stride == 0 || P != k * (k - 1) / 2 || first.param.kernel_type == SvmParam::PRECOMPUTED) return false;
+    for (const FoldRows &f : folds)
+        if (f.model->n_classes != k || f.model->n_binary_models != P || f.model->sv->size() == 0) return false;
+    // A group is a fold's batch of rows, as its own call would take them; the chunks of columns are cut for it as there.
+    std::vector<int> col_map, rows, row_group, chunks, chunk_start;
+    std::vector<float_type> coef_t, rho;
+    std::vector<tsvm_predict_task> tasks;
+    int most_parts = 0, group = 0;
+    for (const FoldRows &f : folds) {
+        const SvmModel &m = *f.model;
+        const size_t col0 = col_map.size();
+        std::vector<int> class_tile;
+        m.pad_classes(stride, class_tile, col_map, coef_t);
+        for (size_t p = col0; p < col_map.size(); ++p) col_map[p] = (*f.train_idx)[m.sv_indices[col_map[p]]];
+        for (size_t b0 = 0; b0 < f.test_idx->size(); b0 += FOLD_BATCH, ++group) {
+            const int row0 = (int) rows.size(), bm = (int) std::min<size_t>(FOLD_BATCH, f.test_idx->size() - b0), chunk0 = (int) chunks.size() / 2;
+            rows.insert(rows.end(), f.test_idx->begin() + b0, f.test_idx->begin() + b0 + bm);
+            row_group.insert(row_group.end(), bm, group);
+            std::vector<int> mine, starts;
+            build_chunks(class_tile, (bm + 63) / 64, 32, mine, starts);
+            const int parts = (int) mine.size() / 2;
+            for (int part = 0; part < parts; ++part)
+                for (int r = 0; r < bm; r += 64) tasks.push_back({row0 + r, row0 + bm, chunk0 + part, part});
+            for (int tile : mine) chunks.push_back((int) (col0 / 128) + tile);
+            chunk_start.insert(chunk_start.end(), starts.begin(), starts.end());
+            rho.insert(rho.end(), m.rho.begin(), m.rho.begin() + P);
+            most_parts = std::max(most_parts, parts);
+        }
+    }
+    const size_t m_all = rows.size(), part_doubles = (size_t) std::max(most_parts, 1) * m_all * (k - 1), dec_bytes = m_all * P * sizeof(float_type);
+    dec.resize(folds.size());
+    for (size_t i = 0; i < folds.size(); ++i) dec[i].resize(folds[i].test_idx->size() * P);
+    if (m_all == 0) return true;
+    OneUpload up;
+    const size_t tasks_at = up.add(tasks), rows_at = up.add(rows), group_at = up.add(row_group), map_at = up.add(col_map), coef_at = up.add(coef_t);
+    const size_t chunks_at = up.add(chunks), start_at = up.add(chunk_start), rho_at = up.add(rho);
+    DeviceBuffer<char> arrays;
+    const char *const at = up.send(arrays);
+    float_type *const d_part = (float_type *) tsvm::RowArena::instance().acquire(part_doubles * sizeof(float_type) + dec_bytes, false);
+    float_type *d_dec = d_part + part_doubles;
+    std::unique_ptr<tsvm::ResultBlock> direct;
+    if (dec_bytes <= tsvm::PINNED_BLOCK) {   // (straight to page-locked host memory, as a request of a few rows)
+        direct.reset(new tsvm::ResultBlock(tsvm::work_stream()));
+        d_dec = (float_type *) direct->dev();
+    }
+    const SvmParam &p = first.param;
+    abi_check(tsvm_predict_groups_dense(all.x.data(), all.ld, d, all.self_dot.data(), (const int *) (at + map_at), (int64_t) col_map.size(),
+                                        (const float_type *) (at + coef_at), (const int *) (at + chunks_at), (const tsvm_predict_task *) (at + tasks_at),
+                                        (int) tasks.size(), (const int *) (at + rows_at), (int64_t) m_all, (const int *) (at + group_at),
+                                        (const int *) (at + start_at), (const float_type *) (at + rho_at), k, (int) p.kernel_type, p.gamma, p.coef0,
+                                        p.degree, d_part, d_dec, tsvm::work_stream()));
+    std::vector<float_type> all_dec(m_all * P);
+    if (direct)
+        memcpy(all_dec.data(), direct->wait(), dec_bytes);
+    else
+        tsvm::HostStaging::instance().download(d_dec, dec_bytes, [&](const char *from, size_t off, size_t len) {
+            tsvm::parallel_memcpy((char *) all_dec.data() + off, from, len);
+        }, tsvm::work_stream());
+    size_t from = 0;
+    for (std::vector<float_type> &v : dec) {
+        std::copy(all_dec.begin() + from, all_dec.begin() + from + v.size(), v.begin());
+        from += v.size();
+    }
+    return true;
 }
 
 namespace {
