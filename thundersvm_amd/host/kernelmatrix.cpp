@@ -2,6 +2,8 @@
 #include "kernelmatrix.h"
 #include <stdexcept>
 
+#include <omp.h>
+
 #include <algorithm>
 #include <chrono>
 #include <cstdio>
@@ -220,7 +222,7 @@ void parallel_memcpy(void *to, const void *from, size_t bytes) {
         return;
     }
     const long n = (long) ((bytes + piece - 1) / piece);
-#pragma omp parallel for schedule(static)
+#pragma omp parallel for schedule(static) num_threads((int) std::min<long>(n, omp_get_max_threads()))
     for (long i = 0; i < n; ++i) memcpy((char *) to + i * piece, (const char *) from + i * piece, std::min(piece, bytes - i * piece));
 }
 

@@ -935,9 +935,13 @@ float_type CSMOSolver::calculate_rho(const std::vector<float_type> &f_val, const
     double sum_free = 0;
     float_type up_value = INFINITY, low_value = -INFINITY;
     for (size_t i = 0; i < alpha.size(); ++i) {
-        if (free_sv(alpha[i], y[i], Cp, Cn)) { n_free++; sum_free += f_val[i]; }
-        if (up_set(alpha[i], y[i], Cp, Cn)) up_value = std::min(up_value, f_val[i]);
-        if (low_set(alpha[i], y[i], Cp, Cn)) low_value = std::max(low_value, f_val[i]);
+        const float_type a = alpha[i], f = f_val[i], C = y[i] > 0 ? Cp : Cn;
+        const bool above = a > 0, below = a < C, up = y[i] > 0 ? below : above, low = y[i] > 0 ? above : below;
+        // (selects, not branches: which instance is free is anybody's guess)
+        n_free += above & below;
+        sum_free = above & below ? sum_free + f : sum_free;
+        up_value = up && f < up_value ? f : up_value;
+        low_value = low && low_value < f ? f : low_value;
     }
     return n_free != 0 ? sum_free / n_free : -(up_value + low_value) / 2;
 }
