@@ -299,6 +299,19 @@ int tsvm_nu_smo_solve_block_on_xcd(const int *y, const double *f_val, double *al
                                    int ws_size, double C, const void *kws, int block_type, const double *k_diag, double eps,
                                    double *diff, int max_iter, int *gate, int epoch, int xcd, tsvm_stream stream);
 
+/* The same on one CU, for a stream that has them all: the launch puts a workgroup on every CU of the chip (256), the one on CU `cu` of die
+ * `xcd` (as tsvm_where numbers them) solves, the others of that die read the block into its L2.  If no workgroup lands there another
+ * one solves.  Launches that share a gate are all of this kind.  diff has a third entry: the int at diff + 2 becomes `epoch` when the
+ * solver has its CU. */
+int tsvm_c_smo_solve_block_on_cu(const int *y, const double *f_val, double *alpha, double *alpha_diff, const int *working_set,
+                                 int ws_size, double Cp, double Cn, const void *kws, int block_type, const double *k_diag, double eps,
+                                 double *diff, int max_iter, int *gate, int epoch, int xcd, int cu, tsvm_stream stream);
+int tsvm_nu_smo_solve_block_on_cu(const int *y, const double *f_val, double *alpha, double *alpha_diff, const int *working_set,
+                                  int ws_size, double C, const void *kws, int block_type, const double *k_diag, double eps,
+                                  double *diff, int max_iter, int *gate, int epoch, int xcd, int cu, tsvm_stream stream);
+/* out[b] = die << 16 | CU of workgroup b of a launch of n (at most 1,024) on `stream`. */
+int tsvm_where(int *out, int n, tsvm_stream stream);
+
 /* What a solve's device state starts from (CSMOSolver::solve's array constructions, csmosolver.cpp:26-56), in one launch: n_diff
  * entries of alpha_diff zeroed, the block's columns beyond ws_size zeroed (for ws_size below the block's row stride), slot_of_id[0..n_ids) = -1, two ints of state and
  * four of gate zeroed (either may be NULL). */

@@ -487,6 +487,45 @@ def test_smo_solve_block_on_a_chosen_xcd(n, ws, nu):
                                              7, G.ptr(dg_d), eps, G.ptr(diff_d), 10, G.ptr(gate), 1, 0, G.stream()) != 0
 
 
+@pytest.mark.parametrize("nu", [False, True])
+@pytest.mark.parametrize("n,ws", [(300, 16), (300, 130), (900, 200), (900, 300), (2000, 1024)])
+def test_smo_solve_block_on_a_chosen_cu(n, ws, nu):
+    """The block solvers launched on every CU of which one solves (tsvm_*_smo_solve_block_on_cu): the same result as ever for CUs
+    that the launch visits and for one that does not exist, where the last workgroup to arrive solves; exactly one does."""
+    Cc, eps = 1.0, 1e-3
+    y, alpha, f, ws_ids, k_rows, diag = _solver_inputs(n, 10, ws, 9 * n + ws, Cc, nu)
+    if nu:
+        a_want, ad_want, diff_want = O.nu_smo_solve(y, f, alpha, ws_ids, Cc, k_rows, diag, n, eps, 100000)
+    else:
+        a_want, ad_want, diff_want = O.c_smo_solve(y, f, alpha, ws_ids, Cc, Cc, k_rows, diag, n, eps, 100000)
+    block = np.zeros((ws, capi.kernel_lib().tsvm_smo_solve_block_ld(ws)))
+    block[:, :ws] = k_rows[:, ws_ids]
+    y_d, f_d, ws_d, dg_d = G.dev(y), G.dev(f), G.dev(ws_ids), G.dev(diag)
+    blocks = [(G.dev(block), capi.ROW_F64), (G.dev(block.astype(np.float32)), capi.ROW_F32)]
+    where_d = torch.zeros(256, dtype=torch.int32, device="cuda")
+    capi.call("tsvm_where", G.ptr(where_d), 256, G.stream())
+    where = G.host(where_d)
+    assert set(where >> 16) == set(range(8))
+    gate = torch.zeros(4, dtype=torch.int32, device="cuda")
+    targets = [(int(where[b]) >> 16, int(where[b]) & 0xffff) for b in (0, 9, 130, 255)] + [(0, 0x7fff), (7, 0x7fff), (0, int(where[8]) & 0xffff)]
+    for epoch, (xcd, cu) in enumerate(targets, start=1):
+        a_d = G.dev(alpha)
+        ad_d = torch.zeros(ws, dtype=torch.float64, device="cuda")
+        diff_d = torch.zeros(3, dtype=torch.float64, device="cuda")
+        blk, bt = blocks[epoch % 2]
+        args = (G.ptr(y_d), G.ptr(f_d), G.ptr(a_d), G.ptr(ad_d), G.ptr(ws_d), ws) + ((Cc,) if nu else (Cc, Cc))
+        capi.call("tsvm_nu_smo_solve_block_on_cu" if nu else "tsvm_c_smo_solve_block_on_cu", *args, G.ptr(blk), bt, G.ptr(dg_d), eps, G.ptr(diff_d),
+                  100000, G.ptr(gate), epoch, xcd, cu, G.stream())
+        g = G.host(gate)
+        assert g[0] == epoch and g[1] == 256 * epoch and 0 <= g[2] < 8
+        assert G.host(diff_d)[0] == diff_want[0] and G.host(diff_d).view(np.int32)[4] == epoch
+        assert np.array_equal(G.host(a_d), a_want)
+        assert np.array_equal(G.host(ad_d), ad_want)
+    with pytest.raises(capi.TsvmError):
+        capi.call("tsvm_nu_smo_solve_block_on_cu" if nu else "tsvm_c_smo_solve_block_on_cu", *args, G.ptr(blk), bt, G.ptr(dg_d), eps, G.ptr(diff_d),
+                  100000, G.ptr(gate), 1, 0, -1, G.stream())
+
+
 def _select_case(n, n_select, n_marked, seed, tie_mode, nu):
     rng = np.random.default_rng(seed)
     y = np.where(rng.random(n) < 0.5, 1, -1).astype(np.int32)

@@ -64,6 +64,9 @@ SIGNATURES = {
     "tsvm_nu_smo_solve_block": (_int, [_p, _p, _p, _p, _p, _int, _dbl, _p, _int, _p, _dbl, _p, _int, _p]),
     "tsvm_c_smo_solve_block_on_xcd": (_int, [_p, _p, _p, _p, _p, _int, _dbl, _dbl, _p, _int, _p, _dbl, _p, _int, _p, _int, _int, _p]),
     "tsvm_nu_smo_solve_block_on_xcd": (_int, [_p, _p, _p, _p, _p, _int, _dbl, _p, _int, _p, _dbl, _p, _int, _p, _int, _int, _p]),
+    "tsvm_c_smo_solve_block_on_cu": (_int, [_p, _p, _p, _p, _p, _int, _dbl, _dbl, _p, _int, _p, _dbl, _p, _int, _p, _int, _int, _int, _p]),
+    "tsvm_nu_smo_solve_block_on_cu": (_int, [_p, _p, _p, _p, _p, _int, _dbl, _p, _int, _p, _dbl, _p, _int, _p, _int, _int, _int, _p]),
+    "tsvm_where": (_int, [_p, _int, _p]),
     "tsvm_smo_start": (_int, [_p, _int, _p, _int, _int, _p, _int, _p, _p, _p]),
     "tsvm_smo_warm_block": (_int, [_p, _int, _int, _int, _p, _p]),
     "tsvm_smo_small_max": (_int, []),

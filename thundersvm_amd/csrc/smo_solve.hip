@@ -165,10 +165,12 @@ __device__ __forceinline__ void load_row_elems(const TB *__restrict__ row, int t
 // eight per launch) claims it if nobody has.  gate[2] tells the host where the solver ran.  Launches that share a gate
 // must be ordered (one stream); gate starts as zeros, epoch at 1.
 #define TSVM_SOLVER_GRID_ON_XCD 8
+__device__ __forceinline__ int own_xcd() { return (int) __builtin_amdgcn_s_getreg(20 | (0 << 6) | (3 << 11)); }   // XCC_ID
+__device__ __forceinline__ int own_cu() { return (int) __builtin_amdgcn_s_getreg(4 | (8 << 6) | (7 << 11)); }     // HW_ID: CU, SH and SE
 __device__ __forceinline__ bool solver_elected(int *gate, int epoch, int target_xcd) {
     __shared__ int s_elected;
     if (threadIdx.x == 0) {
-        const int xcd = (int) __builtin_amdgcn_s_getreg(20 | (0 << 6) | (3 << 11));   // XCC_ID
+        const int xcd = own_xcd();
         bool won = false;
         if (xcd == target_xcd) won = atomicCAS(&gate[0], epoch - 1, epoch) == epoch - 1;
         __threadfence();
@@ -182,6 +184,54 @@ __device__ __forceinline__ bool solver_elected(int *gate, int epoch, int target_
     }
     __syncthreads();
     return s_elected != 0;
+}
+
+// One solver on a chosen CU, for a launch on a stream that has every CU.  As many workgroups as the chip has CUs, each asking for a whole CU's
+// LDS: one lands on every CU (256 different ones of 256 in every launch looked at), and the one on the CU that the row kernels'
+// stream leaves out does the work.  The kernels before and behind it are then on its own stream, without the two markers
+// that a solver on a stream of its own needs (some 11 us each).  Election as above (the last to arrive claims a launch that nobody has
+// claimed, wherever it is); every atomic has come back before the next is made.  The others on that XCD read the block
+// into its L2 before they leave (in place of warm_block_kernel, 10 us in front of the solver).  `started` tells the host that
+// the solver has its CU: rows that take the other CUs before that keep those workgroups, and with them the block, out
+// (20000 x 784, solver beside 340 us of rows 337 us, 427 when they came first).
+#define TSVM_SOLVER_GRID_ON_CU 256
+__device__ __forceinline__ bool solver_elected_on_cu(int *gate, int epoch, bool on_target, int *started) {
+    __shared__ int s_elected;
+    if (threadIdx.x == 0) {
+        int won = 0, seen = epoch - 1;
+        if (on_target) won = __hip_atomic_compare_exchange_strong(&gate[0], &seen, epoch, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(won) :: "memory");
+        int arrived = __hip_atomic_fetch_add(&gate[1], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(arrived) :: "memory");
+        if (!won && arrived % TSVM_SOLVER_GRID_ON_CU == TSVM_SOLVER_GRID_ON_CU - 1) {
+            seen = epoch - 1;
+            won = __hip_atomic_compare_exchange_strong(&gate[0], &seen, epoch, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (won) {
+            gate[2] = own_xcd();
+            __hip_atomic_store(started, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        s_elected = won;
+    }
+    __syncthreads();
+    return s_elected != 0;
+}
+// Workgroup b is number b / 8 of its XCD's thirty-two, as a rule.
+__device__ __forceinline__ void warm_share(const void *block, unsigned bytes, int *gate) {
+    if (bytes > SV_L2_BYTES) return;
+    const uint4 *const p = (const uint4 *) block;
+    const unsigned n16 = bytes / 16, per = (n16 + SV_WARM_SLICES - 1) / SV_WARM_SLICES, lo = (blockIdx.x >> 3) * per, hi = lo + per < n16 ? lo + per : n16;
+    unsigned any = 0;
+    for (unsigned i = lo + threadIdx.x; i < hi; i += blockDim.x) {
+        const uint4 v = p[i];
+        any |= v.x & v.y & v.z & v.w;
+    }
+    if (any == 0xfff5a5a5u) gate[3] = 0;   // (keeps the loads; no kernel value has these bits)
+}
+
+// The CU every workgroup runs on: XCD in the upper half, CU in the lower.
+__global__ __launch_bounds__(64) void where_kernel(int *out) {
+    if (threadIdx.x == 0) out[blockIdx.x] = own_xcd() << 16 | own_cu();
 }
 
 // What a thread's elements start from.  Every load is made (for positions beyond ws the last element's: f, alpha and the label are
@@ -212,6 +262,25 @@ __device__ __forceinline__ void gather_elems(const int *__restrict__ working_set
         label[e] = active ? label[e] : 0;
         kd[e] = active ? kd[e] : 1.0;
     }
+}
+
+// Whether this workgroup of a launch is the one that solves, with what its elements start from.  (What is gathered is on its way during
+// the election; those that can only be elected last gather behind it.)
+template <int E>
+__device__ __forceinline__ bool solver_begins(int *gate, int epoch, int target_xcd, int target_cu, int *started, const void *block, unsigned bytes,
+                                              const int *__restrict__ working_set, int ws, const double *__restrict__ f_val, const double *alpha_val,
+                                              const int *__restrict__ labels, const double *__restrict__ k_diag, double (&f)[E], double (&alpha)[E],
+                                              double (&kd)[E], int (&label)[E]) {
+    const bool on_xcd = target_cu < 0 || own_xcd() == target_xcd, likely = on_xcd && (target_cu < 0 || own_cu() == target_cu);
+    if (likely) gather_elems<E>(working_set, ws, f_val, alpha_val, labels, k_diag, f, alpha, kd, label);
+    if (!gate) return true;
+    if (target_cu < 0) return solver_elected(gate, epoch, target_xcd);
+    if (!solver_elected_on_cu(gate, epoch, likely, started)) {
+        if (on_xcd) warm_share(block, bytes, gate);
+        return false;
+    }
+    if (!likely) gather_elems<E>(working_set, ws, f_val, alpha_val, labels, k_diag, f, alpha, kd, label);
+    return true;
 }
 
 // What the nu solver keeps in LDS, per element of the working set (inactive elements: both bounds zero, so neither in
@@ -478,11 +547,12 @@ __global__ __launch_bounds__(64 * W) void c_smo_solve_kernel(
     const int *__restrict__ label, const double *__restrict__ f_val, double *__restrict__ alpha,
     double *__restrict__ alpha_diff, const int *__restrict__ working_set, int ws, double Cp, double Cn,
     const TB *kws, const double *__restrict__ k_diag, double eps, double *__restrict__ diff,
-    int max_iter, int *__restrict__ gate, int epoch, int target_xcd) {
+    int max_iter, int *__restrict__ gate, int epoch, int target_xcd, int target_cu) {
     double f[E], a_old[E], kd[E];
     int y_of[E];
-    gather_elems<E>(working_set, ws, f_val, alpha, label, k_diag, f, a_old, kd, y_of);   // (on its way during the election)
-    if (gate && !solver_elected(gate, epoch, target_xcd)) return;
+    if (!solver_begins<E>(gate, epoch, target_xcd, target_cu, (int *) (diff + 2), kws, (unsigned) (ws * LDK * sizeof(TB)), working_set, ws, f_val, alpha, label, k_diag, f, a_old, kd,
+                          y_of))
+        return;
     constexpr int N = E * 64 * W;
     __shared__ SvState<N, W> sh;
     __shared__ double s_red[2][W];
@@ -843,11 +913,12 @@ __global__ __launch_bounds__(64 * W) void nu_smo_solve_kernel(
     const int *__restrict__ label, const double *__restrict__ f_val, double *__restrict__ alpha,
     double *__restrict__ alpha_diff, const int *__restrict__ working_set, int ws, double C,
     const TB *kws, const double *__restrict__ k_diag, double eps, double *__restrict__ diff,
-    int max_iter, int *__restrict__ gate, int epoch, int target_xcd) {
+    int max_iter, int *__restrict__ gate, int epoch, int target_xcd, int target_cu) {
     double f[E], a_old[E], kd[E];
     int y_of[E];
-    gather_elems<E>(working_set, ws, f_val, alpha, label, k_diag, f, a_old, kd, y_of);   // (on its way during the election)
-    if (gate && !solver_elected(gate, epoch, target_xcd)) return;
+    if (!solver_begins<E>(gate, epoch, target_xcd, target_cu, (int *) (diff + 2), kws, (unsigned) (ws * LDK * sizeof(TB)), working_set, ws, f_val, alpha, label, k_diag, f, a_old, kd,
+                          y_of))
+        return;
     constexpr int N = E * 64 * W;
     __shared__ SvShared<N, W> sh;
     __shared__ double s_f[2][N], s_k[2][N];   // f and the rows ip / in at the elements of the wavefronts' candidates for j2
@@ -999,7 +1070,7 @@ static int launch_gather(const void *k_rows, int row_type, const int *slots, int
 #define TSVM_LAUNCH_SOLVER(KERNEL, TB, EVAL, WVAL, LDKVAL, ...)                                                \
     do {                                                                                                       \
         size_t dyn_ = 0;                                                                                       \
-        if (solver_grid_ == 1) {                                                                               \
+        if (solver_grid_ != TSVM_SOLVER_GRID_ON_XCD) {                                                         \
             const int rc_ = solver_dyn_lds(reinterpret_cast<const void *>(KERNEL<EVAL, WVAL, LDKVAL, TB>), &dyn_); \
             if (rc_) return rc_;                                                                               \
         }                                                                                                      \
@@ -1040,13 +1111,13 @@ int tsvm_c_smo_solve(const int *y, const double *f_val, double *alpha, double *a
     TSVM_REQUIRE(ws_size >= 1 && ws_size <= MAX_WS, "tsvm_c_smo_solve: ws_size %d outside [1, %d]", ws_size, MAX_WS);
     hipStream_t s = tsvm_s(stream);
     int *gate_ = nullptr;
-    const int epoch_ = 0, target_xcd_ = 0, solver_grid_ = 1;
+    const int epoch_ = 0, target_xcd_ = 0, target_cu_ = -1, solver_grid_ = 1;
     const int block_type_ = row_type;   // the block keeps the rows' element type
     int rc = launch_gather(k_rows, row_type, slots, ld, working_set, ws_size, workspace, block_type_, s);
     if (rc) return rc;
     const void *kws_ = workspace;
     TSVM_DISPATCH_E(c_smo_solve_kernel, (y, f_val, alpha, alpha_diff, working_set, ws_size, Cp, Cn),
-                    (k_diag, eps, diff, max_iter, gate_, epoch_, target_xcd_));
+                    (k_diag, eps, diff, max_iter, gate_, epoch_, target_xcd_, target_cu_));
     TSVM_LAUNCH_CHECK();
     return 0;
 }
@@ -1105,7 +1176,7 @@ int tsvm_c_smo_solve_static(const int *y, const double *f_val, double *alpha, do
     if (rc) return rc;
     hipStream_t s = tsvm_s(stream);
     int *gate_ = nullptr;
-    const int epoch_ = 0, target_xcd_ = 0, solver_grid_ = 1;
+    const int epoch_ = 0, target_xcd_ = 0, target_cu_ = -1, solver_grid_ = 1;
     // the gather writes every element of the ws x ldk block the solver reads (columns beyond ws as zeros), so
     // nothing of the previous call's content is read
     const int block_type_ = row_type;
@@ -1113,7 +1184,7 @@ int tsvm_c_smo_solve_static(const int *y, const double *f_val, double *alpha, do
     if (rc) return rc;
     const void *kws_ = block;
     TSVM_DISPATCH_E(c_smo_solve_kernel, (y, f_val, alpha, alpha_diff, working_set, ws_size, Cp, Cn),
-                    (k_diag, eps, diff, max_iter, gate_, epoch_, target_xcd_));
+                    (k_diag, eps, diff, max_iter, gate_, epoch_, target_xcd_, target_cu_));
     TSVM_LAUNCH_CHECK();
     return 0;
 }
@@ -1190,28 +1261,28 @@ int tsvm_smo_warm_block(const void *kws, int block_type, int ws_size, int xcd, i
 
 static int c_block(const int *y, const double *f_val, double *alpha, double *alpha_diff, const int *working_set, int ws_size,
                    double Cp, double Cn, const void *kws_, int block_type_, const double *k_diag, double eps, double *diff,
-                   int max_iter, int *gate_, int epoch_, int target_xcd_, tsvm_stream stream) {
+                   int max_iter, int *gate_, int epoch_, int target_xcd_, int target_cu_, tsvm_stream stream) {
     TSVM_REQUIRE(y && f_val && alpha && alpha_diff && working_set && kws_ && k_diag && diff, "tsvm_c_smo_solve_block: null pointer");
     TSVM_REQUIRE(ws_size >= 1 && ws_size <= MAX_WS, "tsvm_c_smo_solve_block: ws_size %d outside [1, %d]", ws_size, MAX_WS);
     TSVM_REQUIRE(block_type_ == TSVM_ROW_F64 || block_type_ == TSVM_ROW_F32, "tsvm_c_smo_solve_block: unknown block type %d", block_type_);
     hipStream_t s = tsvm_s(stream);
-    const int solver_grid_ = gate_ ? TSVM_SOLVER_GRID_ON_XCD : 1;
+    const int solver_grid_ = !gate_ ? 1 : target_cu_ < 0 ? TSVM_SOLVER_GRID_ON_XCD : TSVM_SOLVER_GRID_ON_CU;
     TSVM_DISPATCH_E(c_smo_solve_kernel, (y, f_val, alpha, alpha_diff, working_set, ws_size, Cp, Cn),
-                    (k_diag, eps, diff, max_iter, gate_, epoch_, target_xcd_));
+                    (k_diag, eps, diff, max_iter, gate_, epoch_, target_xcd_, target_cu_));
     TSVM_LAUNCH_CHECK();
     return 0;
 }
 
 static int nu_block(const int *y, const double *f_val, double *alpha, double *alpha_diff, const int *working_set, int ws_size,
                     double C, const void *kws_, int block_type_, const double *k_diag, double eps, double *diff, int max_iter,
-                    int *gate_, int epoch_, int target_xcd_, tsvm_stream stream) {
+                    int *gate_, int epoch_, int target_xcd_, int target_cu_, tsvm_stream stream) {
     TSVM_REQUIRE(y && f_val && alpha && alpha_diff && working_set && kws_ && k_diag && diff, "tsvm_nu_smo_solve_block: null pointer");
     TSVM_REQUIRE(ws_size >= 1 && ws_size <= MAX_WS, "tsvm_nu_smo_solve_block: ws_size %d outside [1, %d]", ws_size, MAX_WS);
     TSVM_REQUIRE(block_type_ == TSVM_ROW_F64 || block_type_ == TSVM_ROW_F32, "tsvm_nu_smo_solve_block: unknown block type %d", block_type_);
     hipStream_t s = tsvm_s(stream);
-    const int solver_grid_ = gate_ ? TSVM_SOLVER_GRID_ON_XCD : 1;
+    const int solver_grid_ = !gate_ ? 1 : target_cu_ < 0 ? TSVM_SOLVER_GRID_ON_XCD : TSVM_SOLVER_GRID_ON_CU;
     TSVM_DISPATCH_E(nu_smo_solve_kernel, (y, f_val, alpha, alpha_diff, working_set, ws_size, C),
-                    (k_diag, eps, diff, max_iter, gate_, epoch_, target_xcd_));
+                    (k_diag, eps, diff, max_iter, gate_, epoch_, target_xcd_, target_cu_));
     TSVM_LAUNCH_CHECK();
     return 0;
 }
@@ -1220,14 +1291,14 @@ int tsvm_c_smo_solve_block(const int *y, const double *f_val, double *alpha, dou
                            int ws_size, double Cp, double Cn, const void *kws, int block_type, const double *k_diag, double eps,
                            double *diff, int max_iter, tsvm_stream stream) {
     return c_block(y, f_val, alpha, alpha_diff, working_set, ws_size, Cp, Cn, kws, block_type, k_diag, eps, diff, max_iter, nullptr, 0,
-                   0, stream);
+                   0, -1, stream);
 }
 
 int tsvm_nu_smo_solve_block(const int *y, const double *f_val, double *alpha, double *alpha_diff, const int *working_set,
                             int ws_size, double C, const void *kws, int block_type, const double *k_diag, double eps, double *diff,
                             int max_iter, tsvm_stream stream) {
     return nu_block(y, f_val, alpha, alpha_diff, working_set, ws_size, C, kws, block_type, k_diag, eps, diff, max_iter, nullptr, 0, 0,
-                    stream);
+                    -1, stream);
 }
 
 int tsvm_c_smo_solve_block_on_xcd(const int *y, const double *f_val, double *alpha, double *alpha_diff, const int *working_set,
@@ -1235,7 +1306,7 @@ int tsvm_c_smo_solve_block_on_xcd(const int *y, const double *f_val, double *alp
                                   double *diff, int max_iter, int *gate, int epoch, int xcd, tsvm_stream stream) {
     TSVM_REQUIRE(gate && epoch >= 1 && xcd >= 0 && xcd < TSVM_SOLVER_GRID_ON_XCD, "tsvm_c_smo_solve_block_on_xcd: bad gate, epoch or xcd");
     return c_block(y, f_val, alpha, alpha_diff, working_set, ws_size, Cp, Cn, kws, block_type, k_diag, eps, diff, max_iter, gate, epoch,
-                   xcd, stream);
+                   xcd, -1, stream);
 }
 
 int tsvm_nu_smo_solve_block_on_xcd(const int *y, const double *f_val, double *alpha, double *alpha_diff, const int *working_set,
@@ -1243,7 +1314,31 @@ int tsvm_nu_smo_solve_block_on_xcd(const int *y, const double *f_val, double *al
                                    double *diff, int max_iter, int *gate, int epoch, int xcd, tsvm_stream stream) {
     TSVM_REQUIRE(gate && epoch >= 1 && xcd >= 0 && xcd < TSVM_SOLVER_GRID_ON_XCD, "tsvm_nu_smo_solve_block_on_xcd: bad gate, epoch or xcd");
     return nu_block(y, f_val, alpha, alpha_diff, working_set, ws_size, C, kws, block_type, k_diag, eps, diff, max_iter, gate, epoch, xcd,
-                    stream);
+                    -1, stream);
+}
+
+int tsvm_c_smo_solve_block_on_cu(const int *y, const double *f_val, double *alpha, double *alpha_diff, const int *working_set,
+                                 int ws_size, double Cp, double Cn, const void *kws, int block_type, const double *k_diag, double eps,
+                                 double *diff, int max_iter, int *gate, int epoch, int xcd, int cu, tsvm_stream stream) {
+    TSVM_REQUIRE(gate && epoch >= 1 && xcd >= 0 && xcd < TSVM_SOLVER_GRID_ON_XCD && cu >= 0, "tsvm_c_smo_solve_block_on_cu: bad gate, epoch, xcd or cu");
+    return c_block(y, f_val, alpha, alpha_diff, working_set, ws_size, Cp, Cn, kws, block_type, k_diag, eps, diff, max_iter, gate, epoch,
+                   xcd, cu, stream);
+}
+
+int tsvm_nu_smo_solve_block_on_cu(const int *y, const double *f_val, double *alpha, double *alpha_diff, const int *working_set,
+                                  int ws_size, double C, const void *kws, int block_type, const double *k_diag, double eps,
+                                  double *diff, int max_iter, int *gate, int epoch, int xcd, int cu, tsvm_stream stream) {
+    TSVM_REQUIRE(gate && epoch >= 1 && xcd >= 0 && xcd < TSVM_SOLVER_GRID_ON_XCD && cu >= 0, "tsvm_nu_smo_solve_block_on_cu: bad gate, epoch, xcd or cu");
+    return nu_block(y, f_val, alpha, alpha_diff, working_set, ws_size, C, kws, block_type, k_diag, eps, diff, max_iter, gate, epoch, xcd,
+                    cu, stream);
+}
+
+int tsvm_where(int *out, int n, tsvm_stream stream) {
+    TSVM_REQUIRE(out && n >= 0 && n <= 1024, "tsvm_where: bad arguments");
+    if (n == 0) return 0;
+    hipLaunchKernelGGL(where_kernel, dim3(n), dim3(64), 0, tsvm_s(stream), out);
+    TSVM_LAUNCH_CHECK();
+    return 0;
 }
 
 int tsvm_nu_smo_solve(const int *y, const double *f_val, double *alpha, double *alpha_diff, const int *working_set,
@@ -1255,13 +1350,13 @@ int tsvm_nu_smo_solve(const int *y, const double *f_val, double *alpha, double *
     TSVM_REQUIRE(ws_size >= 1 && ws_size <= MAX_WS, "tsvm_nu_smo_solve: ws_size %d outside [1, %d]", ws_size, MAX_WS);
     hipStream_t s = tsvm_s(stream);
     int *gate_ = nullptr;
-    const int epoch_ = 0, target_xcd_ = 0, solver_grid_ = 1;
+    const int epoch_ = 0, target_xcd_ = 0, target_cu_ = -1, solver_grid_ = 1;
     const int block_type_ = row_type;
     int rc = launch_gather(k_rows, row_type, slots, ld, working_set, ws_size, workspace, block_type_, s);
     if (rc) return rc;
     const void *kws_ = workspace;
     TSVM_DISPATCH_E(nu_smo_solve_kernel, (y, f_val, alpha, alpha_diff, working_set, ws_size, C),
-                    (k_diag, eps, diff, max_iter, gate_, epoch_, target_xcd_));
+                    (k_diag, eps, diff, max_iter, gate_, epoch_, target_xcd_, target_cu_));
     TSVM_LAUNCH_CHECK();
     return 0;
 }

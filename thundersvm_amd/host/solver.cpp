@@ -49,6 +49,9 @@ struct LaneStreams {
 // exactly the CUs on which the lanes' solvers land
 struct LaneGroup {
     std::vector<LaneStreams> lanes;
+    // A group of one lane: a stream with every CU, and the CU that the lane's chip-wide stream leaves out (tsvm_where's number).
+    hipStream_t chain = nullptr;
+    int solver_cu = -1;
 };
 std::mutex g_masked_mutex;
 std::map<long long, std::vector<LaneGroup>> g_masked;   // keyed by device and lane count
@@ -69,7 +72,28 @@ void destroy_masked_streams() {
                 if (m.solver) (void) hipStreamDestroy(m.solver);
                 if (m.chip) (void) hipStreamDestroy(m.chip);
             }
+    for (auto &kv : g_masked)
+        for (LaneGroup &g : kv.second)
+            if (g.chain) (void) hipStreamDestroy(g.chain);
     g_masked.clear();
+}
+
+// What a group of one lane has besides.
+bool find_solver_cu(LaneGroup &g) {
+    const uint32_t all[8] = {~0u, ~0u, ~0u, ~0u, ~0u, ~0u, ~0u, ~0u};
+    if (hipExtStreamCreateWithCUMask(&g.chain, 8, all) != hipSuccess) {
+        (void) hipGetLastError();
+        g.chain = nullptr;
+        return false;
+    }
+    DeviceBuffer<int> d_where(8);
+    int where[8];
+    abi_check(tsvm_where(d_where.data(), 8, g.lanes[0].solver));   // (one workgroup on every XCD's only CU)
+    TSVM_HIP_CHECK(hipMemcpyAsync(where, d_where.data(), sizeof(where), hipMemcpyDeviceToHost, g.lanes[0].solver));
+    TSVM_HIP_CHECK(hipStreamSynchronize(g.lanes[0].solver));
+    for (int w : where)
+        if (w >> 16 == 0) g.solver_cu = w & 0xffff;
+    return g.solver_cu >= 0;
 }
 
 // Makes the 2 * n_lanes streams of a group.  Bit i of a CU mask names CU i/8 of XCD i%8 on the 8-XCD, 256-CU part (a
@@ -99,6 +123,7 @@ bool make_lane_group(int n_lanes, LaneGroup &g) {
         }
         g.lanes.clear();
     }
+    if (ok && n_lanes == 1) ok = find_solver_cu(g);
     return ok;
 }
 
@@ -184,24 +209,32 @@ struct SolveTask::Impl {
 
     // The chip-wide work of a task is enqueued on stream `sa`.
     hipStream_t sa = nullptr;
-    tsvm::DeviceEvent selected, diff_ready;
-    // A task that runs alone splits the chip: the local solver (one workgroup, a chain of dependent steps) gets a
+    tsvm::DeviceEvent diff_ready;
+    // Tasks beside others split the chip: the local solver (one workgroup, a chain of dependent steps) gets a
     // stream `ss` restricted to one CU of every XCD, everything else runs on `sa`, restricted to the other CUs.
     // The solver then runs next to this iteration's get_rows at nearly its stand-alone speed; sharing CUs with a
     // chip-wide kernel it runs two to three times slower, which is why tasks in lockstep keep the phases apart.
     hipStream_t ss = nullptr;
     tsvm::DeviceEvent block_done, solved;
     bool split = false;
-    // Once the cache holds every row there is no get_rows left to run next to the solver; the iteration then
-    // stays on `sa` from start to end and saves the two hand-overs between the streams.
-    bool on_one_stream = false, alone = true;   // alone: no other task's kernels on the chip
-    // When the previous iteration computed many rows this one probably will too, and its get_rows will outlast the
-    // solver by far.  The block is then computed on the solver's few CUs (several times slower, still well inside
-    // the time get_rows takes), so that get_rows need not wait for it on the chip-wide stream.
-    int last_rows_computed = 0;
-    bool block_on_solver_cus = false;
+    // A task that is the only one goes further (`chain`): selection, block, solver and update_f follow one another on `sa`, which has
+    // every CU, and no marker stands between them; the solver finds its CU by itself (tsvm_c_smo_solve_block_on_cu).  The rows,
+    // which are not part of that chain, are computed beside it on `sr`, which leaves that CU out.  What orders the two
+    // streams is the host: it enqueues the rows once the selection has reported, and update_f once the rows have
+    // (h_rows_done), both while the solver still runs as a rule.  epsilon-SVR on 40,000 x 90: the solver starts 1 us behind its block
+    // and update_f 1 us behind the solver, in place of 12 and 11.
+    bool chain = false;
+    hipStream_t sr = nullptr;
+    int solver_cu = -1;
+    hipStream_t rows_stream() const { return chain ? sr : sa; }
+    volatile int *h_rows_done = nullptr;
+    int *d_rows_done = nullptr;
+    int rows_seq = 0;   // the number that h_rows_done takes with the rows enqueued last
+    bool on_one_stream = false;   // block and solver are on `sa`
+    int last_rows_computed = 0;   // (this iteration's will probably be as many)
     long long masked_key = 0;
     int masked_lane = 0;
+    hipStream_t masked_chip = nullptr;   // the chip-wide stream of the pool that this task holds
     int solver_xcd = -1, solver_epoch = 0;   // masked streams: the XCD this lane's solver is launched onto, launches so far
     tsvm::DeviceBuffer<int> d_gate;
 
@@ -289,20 +322,21 @@ struct SolveTask::Impl {
         __atomic_thread_fence(__ATOMIC_ACQUIRE);
         return true;
     }
-    void wait_for_ids() {
+    // Waits until *word is `want`, which work on `stream` writes.
+    void wait_for_word(const volatile int *word, int want, hipStream_t stream, const char *what) {
         using clock = std::chrono::steady_clock;
         const auto start = clock::now();
         auto next_check = start + std::chrono::milliseconds(200);
-        for (unsigned long long spins = 1; !ids_arrived(); ++spins) {
+        for (unsigned long long spins = 1; *word != want; ++spins) {
             if (spins % 4096 != 0) continue;
             const auto now = clock::now();
             if (now < next_check) continue;
             next_check = now + std::chrono::milliseconds(200);
-            const hipError_t e = hipStreamQuery(sa);
+            const hipError_t e = hipStreamQuery(stream);
             if (e == hipSuccess) {
-                if (!ids_arrived()) {
+                if (*word != want) {
                     abandoned = true;
-                    throw std::runtime_error("SolveTask: the selection finished without reporting its ids");
+                    throw std::runtime_error(std::string("SolveTask: ") + what + " finished without reporting");
                 }
             } else if (e != hipErrorNotReady) {
                 abandoned = true;
@@ -310,9 +344,13 @@ struct SolveTask::Impl {
             }
             if (now - start > std::chrono::milliseconds(tsvm::solver_timeout_ms())) {
                 abandoned = true;
-                throw std::runtime_error("SolveTask: no ids from the selection (TSVM_SOLVER_TIMEOUT_MS); the device may be hung");
+                throw std::runtime_error(std::string("SolveTask: no word from ") + what + " (TSVM_SOLVER_TIMEOUT_MS); the device may be hung");
             }
         }
+        __atomic_thread_fence(__ATOMIC_ACQUIRE);
+    }
+    void wait_for_ids() {
+        if (ids_to_host()) wait_for_word(h_ids + ws_size, ids_seq, sa, "the selection");
     }
     int rotation_base = 0;   // iteration at which d_slots_a was valid
     long long window_lookups = 0, window_hits = 0, window_first = 0, first_touches = 0;
@@ -353,7 +391,6 @@ struct SolveTask::Impl {
         d_alpha_diff.resize(ws_size);
         d_sel_ws.resize(tsvm_select_workspace(n));
         d_kws.resize((size_t) ws_size * ldk);
-        alone = n_lanes == 1;
         split = !solver.profile && create_split_streams(lane, n_lanes);
         if (split) {
             solver_xcd = lane;
@@ -363,7 +400,6 @@ struct SolveTask::Impl {
             TSVM_HIP_CHECK(hipStreamCreateWithFlags(&sa, hipStreamNonBlocking));
             ss = sa;
         }
-        selected = tsvm::take_event();
         diff_ready = tsvm::take_event();
         block_done = tsvm::take_event();
         solved = tsvm::take_event();
@@ -411,8 +447,11 @@ struct SolveTask::Impl {
         d_ids_host = (int *) (pinned.dev + 64);
         h_slots = h_ids + ws_size + 16;
         h_cache_info[0] = h_cache_info[1] = 0;
+        h_rows_done = h_cache_info + 2;
+        d_rows_done = d_cache_info + 2;
+        *h_rows_done = 0;
         h_ids[ws_size] = 0;
-        h_diff[0] = h_diff[1] = 0;
+        h_diff[0] = h_diff[1] = h_diff[2] = 0;
         // what the device starts from: the three vectors in one copy, the rest by one kernel
         const size_t f_at = ((size_t) n * sizeof(float_type) + 255) / 256 * 256;
         d_start.resize(2 * f_at + (size_t) n * sizeof(int));
@@ -433,6 +472,7 @@ struct SolveTask::Impl {
         TSVM_HIP_CHECK(hipEventRecord(solved.event, tsvm::work_stream()));   // the rows, the uploads and init_f
         TSVM_HIP_CHECK(hipStreamWaitEvent(sa, solved.event, 0));
         if (ss != sa) TSVM_HIP_CHECK(hipStreamWaitEvent(ss, solved.event, 0));
+        if (chain) TSVM_HIP_CHECK(hipStreamWaitEvent(sr, solved.event, 0));
 
         max_iter = std::max(100000, ws_size > INT_MAX / 100 ? INT_MAX : 100 * ws_size);
         timer.stream = sa;
@@ -471,6 +511,7 @@ struct SolveTask::Impl {
         }
         if (sa) (void) hipStreamSynchronize(sa);   // a selection enqueued ahead may still be running
         if (ss && ss != sa) (void) hipStreamSynchronize(ss);
+        if (chain) (void) hipStreamSynchronize(sr);
         if (split) release_split_streams();         // masked streams go back to the pool
         else if (sa) (void) hipStreamDestroy(sa);
         // (both streams are empty: nothing uses the buffers any more)
@@ -478,7 +519,7 @@ struct SolveTask::Impl {
         for (DeviceBuffer<float_type> *b : {&d_alpha_diff, &d_kws}) b->release(true);
         d_start.release(true);
         d_sel_ws.release(true);
-        for (const tsvm::DeviceEvent &e : {block_done, solved, selected, diff_ready})
+        for (const tsvm::DeviceEvent &e : {block_done, solved, diff_ready})
             if (e.event) tsvm::give_event(e);
         if (pinned.host) tsvm::give_pinned_block(pinned);
     }
@@ -493,10 +534,10 @@ struct SolveTask::Impl {
         masked_lane = lane;
         std::lock_guard<std::mutex> lock(g_masked_mutex);
         std::vector<LaneGroup> &groups = g_masked[masked_key];
-        LaneStreams *mine = nullptr;
+        LaneGroup *group = nullptr;
         for (LaneGroup &g : groups)
-            if (!g.lanes[lane].in_use) { mine = &g.lanes[lane]; break; }
-        if (!mine) {
+            if (!g.lanes[lane].in_use) { group = &g; break; }
+        if (!group) {
             LaneGroup g;
             if (!make_lane_group(n_lanes, g)) return false;
             static bool registered = false;
@@ -505,18 +546,27 @@ struct SolveTask::Impl {
                 atexit(destroy_masked_streams);
             }
             groups.push_back(std::move(g));
-            mine = &groups.back().lanes[lane];
+            group = &groups.back();
         }
-        mine->in_use = true;
-        sa = mine->chip;
-        ss = mine->solver;
+        LaneStreams &mine = group->lanes[lane];
+        mine.in_use = true;
+        masked_chip = mine.chip;
+        if (n_lanes == 1) {
+            chain = true;
+            solver_cu = group->solver_cu;
+            sa = ss = group->chain;
+            sr = mine.chip;
+        } else {
+            sa = mine.chip;
+            ss = mine.solver;
+        }
         return true;
     }
 
     void release_split_streams() {
         std::lock_guard<std::mutex> lock(g_masked_mutex);
         for (LaneGroup &g : g_masked[masked_key])
-            if (g.lanes[masked_lane].chip == sa) g.lanes[masked_lane].in_use = false;
+            if (g.lanes[masked_lane].chip == masked_chip) g.lanes[masked_lane].in_use = false;
     }
 
     // without a cache the slot tables just alternate: the two halves of the working set swap places
@@ -547,7 +597,8 @@ struct SolveTask::Impl {
     }
 
     // Whether the host has to hear of the next selection's ids (its row cache needs them): the selection itself tells it.
-    bool ids_to_host() const { return caching && !all_cached && !device_cache; }
+    // (In a chain the host has to know that the selection is done before it enqueues the rows on their own stream.)
+    bool ids_to_host() const { return chain ? !all_cached : caching && !all_cached && !device_cache; }
 
     void launch_select(int it) {
         const int n_sel = it == 0 ? ws_size : q;
@@ -590,11 +641,20 @@ struct SolveTask::Impl {
             return;
         }
         timer.begin();
+        hipStream_t st = rows_stream();
+        // Rows that take about as long as the solver, or less, come when it has its CU; where they take longer than block and solver
+        // together they go ahead of both.
+        if (chain) wait_for_ids();
+        const auto solver_first = [&] {
+            if (chain && !rows_ahead())
+                wait_for_word((const volatile int *) (h_diff + 2), solver_epoch, sa, "the solver's start");
+        };
         if (device_cache) {
             int *miss_ids = d_slots_a.data() + ws_size, *miss_slots = d_slots_a.data() + 2 * ws_size;
+            solver_first();
             abi_check(tsvm_row_slots_assign(ws_u() + first_new, n_new, d_slot_of.data(), d_cache_state.data(), miss_ids, miss_slots,
-                                            ws_u(), ws_size, d_slots_a.data(), d_cache_info, sa));
-            k_mat.get_rows_counted(miss_ids, n_new, d_cache_state.data() + 1, k_rows, ld, miss_slots, sa);
+                                            ws_u(), ws_size, d_slots_a.data(), d_cache_info, st));
+            k_mat.get_rows_counted(miss_ids, n_new, d_cache_state.data() + 1, k_rows, ld, miss_slots, st);
             slots = d_slots_a.data();
         } else if (caching) {
             // look the new ids up and compute only the rows that are not cached
@@ -633,15 +693,16 @@ struct SolveTask::Impl {
             const int n_miss = (int) miss_ids.size();
             last_rows_computed = n_miss;
             stats.rows_computed += n_miss;
+            solver_first();
             TSVM_HIP_CHECK(hipMemcpyAsync(d_slots_a.data(), h_slots, sizeof(int) * (n_miss ? 3 * (size_t) ws_size : (size_t) ws_size),
-                                          hipMemcpyHostToDevice, sa));
+                                          hipMemcpyHostToDevice, st));
             if (n_miss) {
-                k_mat.get_rows(d_slots_a.data() + ws_size, n_miss, k_rows, ld, d_slots_a.data() + 2 * ws_size, sa);
+                k_mat.get_rows(d_slots_a.data() + ws_size, n_miss, k_rows, ld, d_slots_a.data() + 2 * ws_size, st);
             }
             slots = d_slots_a.data();
             if (cache.used == n_u && d_slot_of.size() == (size_t) n_u) {
                 TSVM_HIP_CHECK(hipMemcpyAsync(d_slot_of.data(), cache.slot_of.data(), sizeof(int) * (size_t) n_u,
-                                              hipMemcpyHostToDevice, sa));
+                                              hipMemcpyHostToDevice, st));
                 all_cached = true;
             }
             // A cache that has started evicting and still does not hit only costs the id read-back:
@@ -654,6 +715,7 @@ struct SolveTask::Impl {
                 const long long again = dl - (first_touches - window_first);
                 if (again * 4 >= dl && dh * 100 < again * off_below_percent) {
                     TSVM_HIP_CHECK(hipStreamSynchronize(sa));
+                    if (chain) TSVM_HIP_CHECK(hipStreamSynchronize(sr));
                     caching = false;
                     stats.cache_disabled = true;
                     if (rep > 1) {
@@ -663,7 +725,7 @@ struct SolveTask::Impl {
                         // path without a cache does at its first iteration.
                         for (int t = 0; t < ws_size; ++t) cur_slots[t] = t;
                         upload_rotation(cur_slots);
-                        k_mat.get_rows(ws_u(), ws_size, k_rows, ld, d_slots_a.data(), sa);
+                        k_mat.get_rows(ws_u(), ws_size, k_rows, ld, d_slots_a.data(), st);
                         last_rows_computed = ws_size;
                     } else {
                         upload_rotation(cur_slots);
@@ -678,36 +740,32 @@ struct SolveTask::Impl {
             // new rows go to the slots the dropped rows occupied
             last_rows_computed = n_new;
             stats.rows_computed += n_new;
-            k_mat.get_rows(ws_u() + first_new, n_new, k_rows, ld, slots + first_new, sa);
+            solver_first();
+            k_mat.get_rows(ws_u() + first_new, n_new, k_rows, ld, slots + first_new, st);
         }
+        if (chain) abi_check(tsvm_report_ids(ws_ids(), 0, 0, d_rows_done, 0, ++rows_seq, sr));
         timer.end(stats.ms_get_rows);
     }
 
+    bool rows_ahead() const { return tsvm::ChipSplit::block_beside_rows(k_mat.n_features(), ws_size, rows_seconds()); }
     double rows_seconds() const { return tsvm::ChipSplit::rows_seconds(k_mat.n_features(), last_rows_computed, n_u); }
 
     void enqueue_block() {
         timer.begin();
-        on_one_stream = !split || (alone && all_cached);
-        // (dense rows only: the CSR block takes too long on eight CUs)
-        block_on_solver_cus = !on_one_stream && alone && block_first && k_mat.dense_layout() && !all_cached &&
-                              tsvm::ChipSplit::block_beside_rows(k_mat.n_features(), ws_size, rows_seconds());
+        on_one_stream = !split || chain;
         if (caching && all_cached) {
             abi_check(tsvm_smo_gather_block_by_id(k_rows, row_type, d_slot_of.data(), ld, ws_u(), ws_size, d_kws.data(), row_type,
                                                   d_slots_a.data(), sa));
             slots = d_slots_a.data();
-        } else if (block_on_solver_cus) {
-            TSVM_HIP_CHECK(hipEventRecord(selected.event, sa));   // the selection is the last thing enqueued on sa
-            TSVM_HIP_CHECK(hipStreamWaitEvent(ss, selected.event, 0));
-            k_mat.get_block(ws_u(), ws_size, d_kws.data(), ldk, ss);
         } else if (block_first) {
             k_mat.get_block(ws_u(), ws_size, d_kws.data(), ldk, sa);
         } else {
             abi_check(tsvm_smo_gather_block(k_rows, row_type, slots, ld, ws_u(), ws_size, d_kws.data(), row_type, sa));
         }
         timer.end(stats.ms_local);
-        if (!on_one_stream && !block_on_solver_cus) TSVM_HIP_CHECK(hipEventRecord(block_done.event, sa));
-        // (beside the solver when it has a stream of its own, in front of it otherwise)
-        if (split && !block_on_solver_cus)
+        if (!on_one_stream) TSVM_HIP_CHECK(hipEventRecord(block_done.event, sa));
+        // (beside the solver; in a chain the solver's own launch does it)
+        if (split && !chain)
             abi_check(tsvm_smo_warm_block(d_kws.data(), row_type, ws_size, solver_xcd, d_gate.data() + 3, sa));
     }
 
@@ -721,8 +779,16 @@ struct SolveTask::Impl {
         }
         solver_enqueued = std::chrono::steady_clock::now();
         next_stream_check = solver_enqueued + std::chrono::milliseconds(200);
-        if (!on_one_stream && !block_on_solver_cus) TSVM_HIP_CHECK(hipStreamWaitEvent(ss, block_done.event, 0));
-        if (solver_xcd >= 0) {   // elected onto this lane's XCD, where the block has been read (launches are ordered, whichever stream they are on)
+        if (!on_one_stream) TSVM_HIP_CHECK(hipStreamWaitEvent(ss, block_done.event, 0));
+        if (chain) {
+            ++solver_epoch;
+            if (nu)
+                abi_check(tsvm_nu_smo_solve_block_on_cu(d_y, d_f, d_alpha, d_alpha_diff.data(), ws_ids(), ws_size, Cp, d_kws.data(), row_type, k_mat.diag(),
+                                                        eps, d_diff, max_iter, d_gate.data(), solver_epoch, 0, solver_cu, st));
+            else
+                abi_check(tsvm_c_smo_solve_block_on_cu(d_y, d_f, d_alpha, d_alpha_diff.data(), ws_ids(), ws_size, Cp, Cn, d_kws.data(), row_type,
+                                                       k_mat.diag(), eps, d_diff, max_iter, d_gate.data(), solver_epoch, 0, solver_cu, st));
+        } else if (solver_xcd >= 0) {   // elected onto this lane's XCD, where the block has been read (launches are ordered, whichever stream they are on)
             ++solver_epoch;
             if (nu)
                 abi_check(tsvm_nu_smo_solve_block_on_xcd(d_y, d_f, d_alpha, d_alpha_diff.data(), ws_ids(), ws_size, Cp,
@@ -745,8 +811,9 @@ struct SolveTask::Impl {
 
     void enqueue_update() {
         // (not where other lanes' rows come through at any time: 7 classes 300000x54 844 -> 857)
-        if (!on_one_stream && alone && k_mat.dense_layout() && !all_cached && tsvm::ChipSplit::warm_behind_rows(block_on_solver_cus, rows_seconds()))
-            abi_check(tsvm_smo_warm_block(d_kws.data(), row_type, ws_size, solver_xcd, d_gate.data() + 3, sa));
+        if (chain && k_mat.dense_layout() && !all_cached && tsvm::ChipSplit::warm_behind_rows(rows_ahead(), rows_seconds()))
+            abi_check(tsvm_smo_warm_block(d_kws.data(), row_type, ws_size, solver_xcd, d_gate.data() + 3, rows_stream()));
+        if (chain && rows_seq != *h_rows_done) wait_for_word(h_rows_done, rows_seq, sr, "the rows");
         if (!on_one_stream) TSVM_HIP_CHECK(hipStreamWaitEvent(sa, solved.event, 0));   // alpha_diff, alpha and diff come from the solver
         if (select_ahead && fuse_select) {
             // the next selection's first pass over the instances rides on update_f's last one

@@ -48,17 +48,17 @@ struct ChipSplit {
     // Of m dense rows of n values, on the whole chip.  (Every column counts.  Indicator columns are left to the epilogue, whose
     // share makes up for it: 512 x 425,000 values of 10 + 44 columns take 1.7 ps each, 1.9 by this.)
     static double rows_seconds(size_t features, long long m, long long n) { return 2.0 * (double) ((features + 15) / 16 * 16) / 6.6e13 * (double) m * (double) n; }
-    // Whether the block is computed on the solver's eight CUs, beside the previous iteration's number of rows: it and the
-    // solver's ~0.4 ms have to fit into their time.  (136 of its 256 tiles on 8 of 256 CUs: 422 us for 1,024 instances of 784
-    // columns and 52 of 90 by this, 505 and 116 by measurement, beside get_rows.  With those, 450 rows of 400,000 columns in
-    // place of 390 are what it takes, and epsilon-SVR on 400,000 x 90 takes 1,411 ms in place of 1,408.)
+    // Whether the rows go ahead of the block and the solver (they are enqueued when the selection has reported, and not when the solver
+    // has its CU): when they, by the previous iteration's number of them, outlast the solver's ~0.4 ms and a block that has to find
+    // its CUs among them (136 of its 256 tiles, as if on 8 of the 256).  Until then they wait for the solver, whose launch
+    // reads the block into its L2 from the CUs that the rows would hold: 20,000 x 784 (340 us of rows an iteration) 39.3 ms a call,
+    // 40.9 with the rows always ahead.
     static bool block_beside_rows(size_t features, int ws, double rows_seconds) {
         return 32.0 * 0.53 * ChipSplit::rows_seconds(features, ws, ws) + 0.4e-3 <= rows_seconds;
     }
     // Whether the block is read into the solver's L2 a second time, behind the rows that stream through it beside the solver and
     // take its place there (epsilon-SVR 40000x90, rows for 42 us beside a solver of 310: 88.4 -> 81.3 ms), unless they take
-    // about as long as the solver (20000x784, 340 us: 50.2 -> 50.3).  A block that is itself computed beside the rows may
-    // not be there yet.
+    // about as long as the solver (20000x784, 340 us: 50.2 -> 50.3).  Behind rows that go ahead the block may not be there yet.
     static bool warm_behind_rows(bool block_beside, double rows_seconds) { return !block_beside && rows_seconds > 0 && rows_seconds < 0.1e-3; }
 };
 }  // namespace tsvm
@@ -103,8 +103,8 @@ private:
 
 // One SMO solve as a resumable sequence of enqueue steps.  CSMOSolver::solve runs one task to completion; a
 // one-vs-one run keeps several tasks (class pairs) in flight and enqueues their steps in turn.  The local
-// solver is a single workgroup bound by latency; it runs on a stream restricted to compute units of its own
-// (one per XCD and lane), everything else of the task on a stream restricted to the remaining ones, so the
+// solver is a single workgroup bound by latency; it runs on compute units of its own (one per XCD and lane), by a stream that is restricted to
+// them or, in a task that runs alone, by finding its unit itself; what runs beside it is on a stream restricted to the remaining ones, so the
 // solver of an iteration runs next to that iteration's get_rows.  Where such streams cannot be had the task
 // uses one ordinary stream, and the driver of several tasks keeps their solver phases apart from their
 // chip-wide phases with events.  The steps of one outer iteration:
