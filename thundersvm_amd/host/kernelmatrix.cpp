@@ -2,8 +2,6 @@
 #include "kernelmatrix.h"
 #include <stdexcept>
 
-#include <omp.h>
-
 #include <algorithm>
 #include <chrono>
 #include <cstdio>
@@ -222,7 +220,8 @@ void parallel_memcpy(void *to, const void *from, size_t bytes) {
         return;
     }
     const long n = (long) ((bytes + piece - 1) / piece);
-#pragma omp parallel for schedule(static) num_threads((int) std::min<long>(n, omp_get_max_threads()))
+    // (the whole team, also for fewer pieces: a team of another size than the last one's ends and starts threads)
+#pragma omp parallel for schedule(static) num_threads(thread_limit())
     for (long i = 0; i < n; ++i) memcpy((char *) to + i * piece, (const char *) from + i * piece, std::min(piece, bytes - i * piece));
 }
 

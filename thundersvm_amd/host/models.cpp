@@ -551,7 +551,7 @@ void SVC::finish_training(const DataSet &grouped, std::vector<BinaryProblem> &sm
     const std::vector<int> &count = grouped.count(), &start = grouped.start();
     std::vector<unsigned char> is_sv(n, 0);   // by place in the grouped order
     const int threads = threads_for((size_t) n * (n_classes - 1));
-#pragma omp parallel for schedule(dynamic, 1) num_threads(std::min(threads, n_classes))
+#pragma omp parallel for schedule(dynamic, 1) num_threads(threads)
     for (int c = 0; c < n_classes; ++c)
         for (int kk = 0; kk < n_binary_models; ++kk) {
             if (pair_of[kk].first != c && pair_of[kk].second != c) continue;

@@ -5,7 +5,8 @@
 #include <algorithm>
 #include <cstring>
 
-int threads_for(size_t entries) { return (int) std::max<size_t>(1, std::min<size_t>((size_t) omp_get_max_threads(), entries / 32768)); }
+int thread_limit() { return (3 * omp_get_max_threads() + 3) / 4; }
+int threads_for(size_t entries) { return (int) std::max<size_t>(1, std::min<size_t>((size_t) thread_limit(), entries / 32768)); }
 
 // (none of the arrays is value-initialised: whoever fills them does so on many threads, which also take the page faults)
 RowStore::RowStore(size_t n, size_t nnz)
