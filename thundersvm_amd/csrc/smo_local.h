@@ -145,11 +145,27 @@ __device__ __forceinline__ void publish_row(double *f_slot, double *k_slot, int 
                      "ds_write2_b64 %2, %7, %8 offset1:1\n\tds_write2_b64 %2, %9, %10 offset0:2 offset1:3\n\t" SV_EXEC_OFF
                      :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "v"(k[0]), "v"(k[1]), "v"(k[2]), "v"(k[3]) : "memory");
 }
+// The same for a record that is already a run of four registers, and for a score with its step.
+typedef int SvWords __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void publish_words(unsigned slot, uint64_t lanes, const SvWords &v) {
+    asm volatile(SV_EXEC_ON "ds_write_b128 %1, %2\n\t" SV_EXEC_OFF :: "s"(lanes), "v"(slot), "v"(v) : "memory");
+}
+__device__ __forceinline__ void publish_score(unsigned slot, uint64_t lanes, float best, float second, int at, int go, double b, double a) {
+    const SvWords v = {__float_as_int(best), __float_as_int(second), at, go};
+    asm volatile(SV_EXEC_ON "ds_write_b128 %1, %2\n\tds_write2_b64 %1, %3, %4 offset0:2 offset1:3\n\t" SV_EXEC_OFF
+                 :: "s"(lanes), "v"(slot), "v"(v), "v"(b), "v"(a) : "memory");
+}
+__device__ __forceinline__ double lds_f64(unsigned at) { return *(const __attribute__((address_space(3))) double *) (uintptr_t) at; }
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 // (p, then q: if both name one element the second value is the final one; `on` = 0: nothing is written)
 __device__ __forceinline__ void write_by_lane0(int on, double *p, double v, double *q, double w) {
     asm volatile(SV_EXEC_ON "ds_write_b64 %1, %2\n\tds_write_b64 %3, %4\n\t" SV_EXEC_OFF
                  :: "s"((uint64_t) (uint32_t) __builtin_amdgcn_readfirstlane(on)), "v"(lds_at(p)), "v"(v), "v"(lds_at(q)), "v"(w) : "memory");
+}
+
+// (the same by LDS addresses)
+__device__ __forceinline__ void write_by_lane0(int on, unsigned p, double v, unsigned q, double w) {
+    asm volatile(SV_EXEC_ON "ds_write_b64 %1, %2\n\tds_write_b64 %3, %4\n\t" SV_EXEC_OFF :: "s"((uint64_t) (uint32_t) on), "v"(p), "v"(v), "v"(q), "v"(w) : "memory");
 }
 
 // The workgroup's best candidate: every lane reads one of the W, two DPP steps compare them.  The elements of a
@@ -181,6 +197,17 @@ __device__ __forceinline__ unsigned set_member_bits(unsigned m, int tid, int t, 
     const unsigned changed = (m & ~field) | (bits << sh);
     return tid == (int) ((unsigned) t / E) ? changed : m;
 }
+
+// Membership bits of the c variant, one per element, in three instructions a change.  own_bit: element t's bit in the thread that owns
+// it; in another one it is a bit from E on, which nobody reads.  A decision that all lanes have come to alike is a mask of
+// ones or zeros in a scalar register.
+template <int E>
+__device__ __forceinline__ unsigned own_bit(int tid, int t) {
+    const unsigned at = (unsigned) (t - tid * E);
+    return 1u << (at < 31u ? at : 31u);
+}
+__device__ __forceinline__ unsigned same_in_all_lanes(bool x) { return (unsigned) __builtin_amdgcn_ballot_w64(x); }
+__device__ __forceinline__ unsigned put_bits(unsigned m, unsigned bits, unsigned on) { return (m & ~bits) | (bits & on); }
 
 // The local solvers hold alpha times its label, z = y * alpha in [lo, hi] with lo = 0, hi = Cp for y > 0 and lo = -Cn,
 // hi = 0 for y < 0: an element is in I_up while z < hi and in I_low while z > lo, a step is bounded by hi - z_i and z_j - lo
@@ -221,6 +248,82 @@ __device__ __forceinline__ void row_best_two(float &best, float &second) {
         asm("s_nop 1\n\t" SV_BEST_STEP("quad_perm:[1,0,3,2]") SV_BEST_STEP("quad_perm:[2,3,0,1]") SV_BEST_STEP("row_half_mirror")
                 SV_BEST_STEP("row_mirror")
             : "+v"(best), "+v"(second), "=&v"(t));
+#undef SV_BEST_STEP
+}
+struct SvScoreStep {
+    SvScore score;
+    SvStep step;
+};
+
+// What follows are whole chains in one asm block each, with registers of their own from v144 on (the halves of a register pair
+// cannot be named otherwise): between the builtins and one-instruction blocks that they replace the compiler puts
+// wait states, as it does not know what such a block holds.  A DPP operand is two wait states old everywhere, a mask
+// that a comparison wrote is read three instructions later.
+#define SV_DPP_MOV(TO, FROM, CTRL) "v_mov_b32_dpp " TO ", " FROM " " CTRL " row_mask:0xf bank_mask:0xf\n\t"
+#define SV_MIN_STEP(CTRL) SV_DPP_MOV("v148", "v150", CTRL) SV_DPP_MOV("v149", "v151", CTRL) "v_min_f64 v[150:151], v[150:151], v[148:149]\n\t"
+// row_first_min with the candidate as the record that is published (its last word is anything); `has`: the lanes that have the row's smallest.
+template <int E>
+__device__ __forceinline__ void row_first_candidate(const double (&x)[E], const int (&at)[E], SvWords &rec, uint64_t &has) {
+    uint64_t h0, h1, h2;
+    if constexpr (E == 4) {
+        asm("v_min_f64 v[144:145], %5, %6\n\t"
+            "v_min_f64 v[148:149], %7, %8\n\t"
+            "v_min_f64 v[144:145], v[144:145], v[148:149]\n\t"
+            "v_cmp_eq_f64_e64 %2, %5, v[144:145]\n\t"
+            "v_cmp_eq_f64_e64 %3, %6, v[144:145]\n\t"
+            "v_cmp_eq_f64_e64 %4, %7, v[144:145]\n\t"
+            SV_DPP_MOV("v148", "v144", "quad_perm:[1,0,3,2]") SV_DPP_MOV("v149", "v145", "quad_perm:[1,0,3,2]")
+            "v_min_f64 v[150:151], v[144:145], v[148:149]\n\t"
+            "v_cndmask_b32_e64 v146, %12, %11, %4\n\t"
+            "v_cndmask_b32_e64 v146, v146, %10, %3\n\t"
+            SV_MIN_STEP("quad_perm:[2,3,0,1]")
+            "v_cndmask_b32_e64 v146, v146, %9, %2\n\t"
+            "s_nop 0\n\t" SV_MIN_STEP("row_half_mirror")
+            "s_nop 1\n\t" SV_MIN_STEP("row_mirror")
+            "v_cmp_eq_f64_e64 %1, v[144:145], v[150:151]"
+            : "=&{v[144:147]}"(rec), "=&s"(has), "=&s"(h0), "=&s"(h1), "=&s"(h2)
+            : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3])
+            : "v148", "v149", "v150", "v151");
+    } else {
+        static_assert(E == 2, "elements per thread");
+        asm("v_min_f64 v[144:145], %3, %4\n\t"
+            "v_cmp_eq_f64_e64 %2, %3, v[144:145]\n\t"
+            "s_nop 0\n\t"
+            SV_DPP_MOV("v148", "v144", "quad_perm:[1,0,3,2]") SV_DPP_MOV("v149", "v145", "quad_perm:[1,0,3,2]")
+            "v_min_f64 v[150:151], v[144:145], v[148:149]\n\t"
+            "v_cndmask_b32_e64 v146, %6, %5, %2\n\t"
+            "s_nop 0\n\t" SV_MIN_STEP("quad_perm:[2,3,0,1]")
+            "s_nop 1\n\t" SV_MIN_STEP("row_half_mirror")
+            "s_nop 1\n\t" SV_MIN_STEP("row_mirror")
+            "v_cmp_eq_f64_e64 %1, v[144:145], v[150:151]"
+            : "=&{v[144:147]}"(rec), "=&s"(has), "=&s"(h0)
+            : "v"(x[0]), "v"(x[1]), "v"(at[0]), "v"(at[1])
+            : "v148", "v149", "v150", "v151");
+    }
+}
+// row_min, with the lanes that have it.
+__device__ __forceinline__ void row_min_and_who(double x, double &value, uint64_t &who) {
+    const double t = dpp_f64<TSVM_DPP_XOR1>(x);
+    asm("v_min_f64 v[150:151], %2, %3\n\t"
+        "s_nop 1\n\t" SV_MIN_STEP("quad_perm:[2,3,0,1]")
+        "s_nop 1\n\t" SV_MIN_STEP("row_half_mirror")
+        "s_nop 1\n\t" SV_DPP_MOV("v148", "v150", "row_mirror") SV_DPP_MOV("v149", "v151", "row_mirror")
+        "v_min_f64 %0, v[150:151], v[148:149]\n\t"
+        "v_cmp_eq_f64_e64 %1, %2, %0"
+        : "=&v"(value), "=s"(who) : "v"(x), "v"(t) : "v148", "v149", "v150", "v151");
+}
+// row_best_two over sixteen lanes, with the lanes that have the best.
+__device__ __forceinline__ void row_best_two_and_who(float mine, float second_in, float &best, float &second, uint64_t &who) {
+    float t;
+#define SV_BEST_STEP(CTRL, B, S)                                          \
+    "v_min_f32_dpp %2, " B ", " B " " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_max_f32_dpp %0, " B ", " B " " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_max_f32_dpp %1, " S ", " S " " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_max_f32 %1, %1, %2\n\t"
+    asm("s_nop 1\n\t" SV_BEST_STEP("quad_perm:[1,0,3,2]", "%4", "%5") SV_BEST_STEP("quad_perm:[2,3,0,1]", "%0", "%1")
+            SV_BEST_STEP("row_half_mirror", "%0", "%1") SV_BEST_STEP("row_mirror", "%0", "%1")
+        "v_cmp_eq_f32_e64 %3, %4, %0"
+        : "=&v"(best), "=&v"(second), "=&v"(t), "=s"(who) : "v"(mine), "v"(second_in));
 #undef SV_BEST_STEP
 }
 // The smallest of a row's x, in all its lanes.
@@ -269,4 +372,5 @@ __device__ __forceinline__ double row_first_min(const double (&x)[E], int base, 
 
 // Bounds of what c_smo_iterate_rounded (smo_solve.hip) decides: the least |up|, and from where on an a is too large (as float bits).
 #define SV_UP_LEAST_HI 0x3b600000   // 2^-73
+#define SV_UP_LEAST 0x1p-73
 #define SV_A_BITS 0x7e800000         // 2^126

@@ -20,7 +20,7 @@
 // exit test folded into the loop's branch (the last round computes a step that is not taken); and everything that does
 // not need the row on its way pinned in front of the first instruction that does.
 // Measured on a call of 483 iterations with ws = 1024: 1.37 us per iteration before that, 1.08 with it (2,590 cycles);
-// 0.97 with the scores ranked in float where that decides (c_smo_iterate_rounded).
+// 0.97 with the scores ranked in float where that decides (c_smo_iterate_rounded), 0.87 since its chains are single blocks.
 //
 // Reductions are lexicographic (value, element index) minima, so ties go to the lowest
 // index exactly as the reference's serial loops resolve them, and all arithmetic is the reference's
@@ -157,6 +157,31 @@ __device__ __forceinline__ void load_row_elems(const TB *__restrict__ row, int t
     }
 }
 
+// The same by buffer loads: the row's offset in bytes is a scalar operand of the load, without an addition of addresses in front of it.
+template <int E, typename TB>
+struct BlockRows {
+    __amdgpu_buffer_rsrc_t block;
+    int at;
+    __device__ __forceinline__ BlockRows(const TB *kws, unsigned n, int tid)
+        : block(__builtin_amdgcn_make_buffer_rsrc((void *) kws, 0, (int) (n * sizeof(TB)), 0x00027000)), at(tid * E * (int) sizeof(TB)) {}
+    __device__ __forceinline__ void load(int row, TB (&out)[E]) const {
+        constexpr int BYTES = E * (int) sizeof(TB);
+        static_assert(BYTES == 8 || BYTES % 16 == 0, "two or four elements");
+        typedef unsigned v2u __attribute__((ext_vector_type(2)));
+        typedef unsigned v4u __attribute__((ext_vector_type(4)));
+        if constexpr (BYTES == 8) {
+            const v2u v = __builtin_amdgcn_raw_buffer_load_b64(block, at, row, 0);
+            __builtin_memcpy(out, &v, 8);
+        } else {
+#pragma unroll
+            for (int b = 0; b < BYTES / 16; ++b) {
+                const v4u v = __builtin_amdgcn_raw_buffer_load_b128(block, at + 16 * b, row, 0);
+                __builtin_memcpy((char *) out + 16 * b, &v, 16);
+            }
+        }
+    }
+};
+
 // One solver on a chosen XCD.  A kernel of one workgroup runs on whichever XCD its stream's hardware queue starts
 // dealing at; launched as eight workgroups under a CU mask with one CU per XCD, one workgroup lands on every XCD, and
 // the one that finds itself on target_xcd does the work while the others leave at once.  Exactly one workgroup is
@@ -292,11 +317,14 @@ struct SvShared {
     double z[W][N];           // alpha times its label: every wavefront keeps a copy of its own, which needs no barrier
 };
 
-// What c_smo_solve keeps.
+// What c_smo_solve keeps.  (An element's bounds and diagonal are read by one address.)
+struct __align__(32) SvElem {
+    SvBound bound;
+    double kd, unused;
+};
 template <int N, int W>
 struct SvState {
-    double kd[N];
-    SvBound bound[N];
+    SvElem elem[N];
     double z[W][N];           // every wavefront keeps a copy of its own, which needs no barrier
     double f[N], k[N];        // f and row i at the elements of the wavefronts' candidates for j2 (the others are not written)
 };
@@ -336,8 +364,8 @@ __device__ __forceinline__ bool c_smo_iterate(SvState<E * 64 * W, W> &sh, SvCand
         TB kI[E];
         load_row_elems<E, TB>(kws + (unsigned) i * (unsigned) LDK, tid, kI);
         SV_PIN_MEMORY;
-        const double kd_i = sh.kd[i], z_i = sh.z[wave][i];
-        const SvBound bound_i = sh.bound[i];
+        const double kd_i = sh.elem[i].kd, z_i = sh.z[wave][i];
+        const SvBound bound_i = sh.elem[i].bound;
         double a_part[E], b_low[E], b_max = -TSVM_INF;
 #pragma unroll
         for (int e = 0; e < E; ++e) {
@@ -378,8 +406,8 @@ __device__ __forceinline__ bool c_smo_iterate(SvState<E * 64 * W, W> &sh, SvCand
         TB kJ[E];
         load_row_elems<E, TB>(kws + (unsigned) j2 * (unsigned) LDK, tid, kJ);
         SV_PIN_MEMORY;
-        const SvBound bound_j = sh.bound[j2];
-        const double kd_j = sh.kd[j2], z_j = sh.z[wave][j2], f_j = sh.f[j2];
+        const SvBound bound_j = sh.elem[j2].bound;
+        const double kd_j = sh.elem[j2].kd, z_j = sh.z[wave][j2], f_j = sh.f[j2];
         const double kIj = (double) *(const TB *) (sh.k + j2);
         SV_PIN;   // the row is on its way while the step is computed
         // two-variable step (smo_kernel.cpp:92-103; the last round computes one that is not taken)
@@ -387,10 +415,11 @@ __device__ __forceinline__ bool c_smo_iterate(SvState<E * 64 * W, W> &sh, SvCand
         const double q2 = (-up_value + f_j) / __builtin_fma(-2.0, kIj, kd_i + kd_j);
         const double l = fmin_f64(up_i, fmin_f64(z_j - bound_j.lo, q2));
         const double nz_i = z_i + l, nz_j = (NONE && j2 == i ? nz_i : z_j) - l;
-        in_up = set_member_bits<E, 1>(in_up, tid, i, nz_i < bound_i.hi ? 1u : 0u);
-        in_low = set_member_bits<E, 1>(in_low, tid, i, nz_i > bound_i.lo ? 1u : 0u);
-        in_up = set_member_bits<E, 1>(in_up, tid, j2, nz_j < bound_j.hi ? 1u : 0u);
-        in_low = set_member_bits<E, 1>(in_low, tid, j2, nz_j > bound_j.lo ? 1u : 0u);
+        const unsigned bit_i = own_bit<E>(tid, i), bit_j = own_bit<E>(tid, j2);
+        const unsigned up_i_on = same_in_all_lanes(nz_i < bound_i.hi), low_i_on = same_in_all_lanes(nz_i > bound_i.lo);
+        const unsigned up_j_on = same_in_all_lanes(nz_j < bound_j.hi), low_j_on = same_in_all_lanes(nz_j > bound_j.lo);
+        in_up = put_bits(put_bits(in_up, bit_i, up_i_on), bit_j, up_j_on);
+        in_low = put_bits(put_bits(in_low, bit_i, low_i_on), bit_j, low_j_on);
         write_by_lane0(go_on, &sh.z[wave][i], nz_i, &sh.z[wave][j2], nz_j);
         SV_PIN;   // (nothing above waits for the row)
 #pragma unroll
@@ -415,40 +444,55 @@ __device__ __forceinline__ bool c_smo_iterate(SvState<E * 64 * W, W> &sh, SvCand
 // Rows of sixteen lanes are reduced by DPP and publish themselves, and after the barrier every lane reads one of the
 // sixteen rows and four more steps compare them: the same eight steps as over a wavefront and then over four of them, without
 // the way through the scalar unit in between.
+// A step is bound by the issue of its instructions, so it is counted in them: 351 and 35 wait states -> 300 and 15 with the chains of
+// DPP steps in one block each, membership bits changed by masks (put_bits), rows read at a scalar offset (BlockRows), one
+// address for an element's bounds and diagonal, a limit of steps that shares the way out with the stopping test, and z and in_low
+// written while the next step waits for its candidates.  A whole call: epsilon-SVR 40000x90 (54,594 steps) 74.8 -> 69.1 ms, sparse text
+// 18000 (24,020) 34.0 -> 32.0, 20,000 x 784 (32,880) 39.2 -> 37.8.
 template <int E, int LDK, typename TB>
-__device__ __forceinline__ bool c_smo_iterate_rounded(SvState<E * 256, 4> &sh, SvCand *s_i, SvScore *s_j, SvStep *s_step, int ws, const TB *kws,
+__device__ __forceinline__ bool c_smo_iterate_rounded(SvState<E * 256, 4> &sh, SvCand *s_i, SvScoreStep *s_j, int ws, const TB *kws,
                                                       const double (&kd)[E], double (&f)[E], unsigned &in_up, unsigned &in_low,
                                                       double local_eps, int max_iter, int &n_iter) {
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    SvCand *const my_i = s_i + (tid >> 4);
-    SvScore *const my_j = s_j + (tid >> 4);
+    const unsigned my_i = lds_at(s_i + (tid >> 4)), my_j = lds_at(s_j + (tid >> 4));
+    unsigned my_z = lds_at(&sh.z[wave][0]);
+    asm("" : "+v"(my_z));
+    const BlockRows<E, TB> rows(kws, (unsigned) ws * (unsigned) LDK, tid);
+    int at_of[E];   // (whoever is chosen without being a candidate is one that exists)
+#pragma unroll
+    for (int e = 0; e < E; ++e) at_of[e] = tid * E + e < ws ? tid * E + e : ws - 1;
     uint64_t go;
-    // the last step's changes to in_low, which are made while the next row is on its way
-    unsigned bit_i = 0, bit_j = 0, low_i = 0, low_j = 0;
-    int owner_i = -1, owner_j = -1;
+    // what a step leaves to the waits of the next: its changes to in_low, and the two elements' new z
+    unsigned bit_i = 0, bit_j = 0, low_i = 0, low_j = 0, z_at_i = my_z, z_at_j = my_z;
+    double nz_i = 0, nz_j = 0;
+    int pending = 0;
     for (;;) {
         double fu[E];
 #pragma unroll
         for (int e = 0; e < E; ++e) fu[e] = keep_or_none<0>(in_up << (31 - e), f[e]);
-        double m;
-        int at;
-        const double r = row_first_min<E>(fu, tid * E, m, at);
+        SvWords cand;
+        uint64_t has;
+        row_first_candidate<E>(fu, at_of, cand, has);
         // the lowest lane of every row that has it (every field of sixteen bits has one set, whatever is NaN)
-        const uint64_t has = __builtin_amdgcn_ballot_w64(m == r) | 0x8000800080008000ull;
-        publish(my_i, has & ~(has - 0x0001000100010001ull), m, at, 0);
+        has |= 0x8000800080008000ull;
+        publish_words(my_i, has & ~(has - 0x0001000100010001ull), cand);
         lds_barrier();
         const SvCand ci = s_i[lane & 15];
-        const double up_value = row_min(ci.v);
-        int i = __builtin_amdgcn_readlane(ci.at, __builtin_ctzll(__builtin_amdgcn_ballot_w64(ci.v == up_value)));
-        i = i < ws ? i : ws - 1;
+        write_by_lane0(pending, z_at_i, nz_i, z_at_j, nz_j);
+        in_low = put_bits(put_bits(in_low, bit_i, low_i), bit_j, low_j);
+        double up_value;
+        uint64_t first;
+        row_min_and_who(ci.v, up_value, first);
+        const int i = __builtin_amdgcn_readlane(ci.at, __builtin_ctzll(first));
         TB kI[E];
-        load_row_elems<E, TB>(kws + (unsigned) i * (unsigned) LDK, tid, kI);
+        rows.load(i * (LDK * (int) sizeof(TB)), kI);
         SV_PIN_MEMORY;
-        const double kd_i = sh.kd[i], z_i = sh.z[wave][i];
-        const SvBound bound_i = sh.bound[i];
-        in_low = tid == owner_i ? (in_low & ~bit_i) | low_i : in_low;
-        in_low = tid == owner_j ? (in_low & ~bit_j) | low_j : in_low;
+        z_at_i = my_z + 8u * (unsigned) i;
+        const SvBound bound_i = sh.elem[i].bound;
+        const double kd_i = sh.elem[i].kd, z_i = lds_f64(z_at_i);
+        bit_i = own_bit<E>(tid, i);
+        asm("" : "+v"(bit_i));
         double a_part[E], b_low[E], b_max = -TSVM_INF;
         float b32[E];
 #pragma unroll
@@ -458,10 +502,10 @@ __device__ __forceinline__ bool c_smo_iterate_rounded(SvState<E * 256, 4> &sh, S
             b32[e] = __builtin_fmaxf((float) b_low[e], 0.0f);
             a_part[e] = kd_i + kd[e];
         }
-        const int violates = __builtin_amdgcn_ballot_w64(!(b_max < local_eps)) != 0;
+        const int violates = (__builtin_amdgcn_ballot_w64(!(b_max < local_eps)) != 0) & (n_iter <= max_iter);   // (the way out is one test)
         double up_i = bound_i.hi - z_i;
         asm("" : "+v"(up_i));
-        int a_max = (__double2hiint(up_value) & 0x7fffffff) < SV_UP_LEAST_HI ? 0x7f800000 : 0;   // (as the bits of a float)
+        int a_max = __builtin_fabs(up_value) < SV_UP_LEAST ? 0x7f800000 : 0;   // (as the bits of a float)
         asm("" : "+v"(a_max));
         SV_PIN;
         double aIJ[E];
@@ -473,71 +517,65 @@ __device__ __forceinline__ bool c_smo_iterate_rounded(SvState<E * 256, 4> &sh, S
             a_max = __float_as_int(a32) > a_max ? __float_as_int(a32) : a_max;
             q[e] = __builtin_fmaxf(b32[e] * (b32[e] * __builtin_amdgcn_rcpf(a32)), 0x1p-80f);
         }
-        float best, second;
+        float mine, second;
         if constexpr (E == 4) {
             const float h0 = __builtin_fmaxf(q[0], q[1]), h1 = __builtin_fmaxf(q[2], q[3]);
-            best = __builtin_fmaxf(h0, h1);
+            mine = __builtin_fmaxf(h0, h1);
             second = __builtin_fmaxf(__builtin_fmaxf(__builtin_fminf(h0, h1), __builtin_fminf(q[0], q[1])), __builtin_fminf(q[2], q[3]));
         } else {
             static_assert(E == 2, "elements per thread");
-            best = __builtin_fmaxf(q[0], q[1]);
+            mine = __builtin_fmaxf(q[0], q[1]);
             second = __builtin_fminf(q[0], q[1]);
         }
-        at = tid * E + E - 1;
+        int at = at_of[E - 1];
         double b_at = b_low[E - 1], a_at = aIJ[E - 1];
 #pragma unroll
         for (int e = E - 2; e >= 0; --e) {
-            const bool is = q[e] == best;
-            at = is ? tid * E + e : at;
+            const bool is = q[e] == mine;
+            at = is ? at_of[e] : at;
             b_at = is ? b_low[e] : b_at;
             a_at = is ? aIJ[e] : a_at;
         }
         second = a_max < SV_A_BITS ? second : __builtin_inff();
-        const float mine = best;
-        row_best_two(best, second);
-        const uint64_t who = __builtin_amdgcn_ballot_w64(mine == best);   // (several only if nothing will be decided)
-        publish(my_j, who, best, second, at, violates);
-        publish(s_step + (tid >> 4), who, b_at, a_at);
+        float best, next;
+        uint64_t who;   // (several only if nothing will be decided)
+        row_best_two_and_who(mine, second, best, next, who);
+        publish_score(my_j, who, best, next, at, violates, b_at, a_at);
         lds_barrier();
-        const SvScore cj = s_j[lane & 15];
-        const SvStep step = s_step[lane & 15];
-        best = cj.best;
-        second = cj.second;
-        row_best_two(best, second);
-        const int row = __builtin_ctzll(__builtin_amdgcn_ballot_w64(cj.best == best));
-        int j2 = __builtin_amdgcn_readlane(cj.at, row);
-        j2 = j2 < ws ? j2 : ws - 1;
+        const SvScoreStep cj = s_j[lane & 15];
+        uint64_t won;
+        row_best_two_and_who(cj.score.best, cj.score.second, best, next, won);
+        const int row = __builtin_ctzll(won);
+        const int j2 = __builtin_amdgcn_readlane(cj.score.at, row);
         TB kJ[E];
-        load_row_elems<E, TB>(kws + (unsigned) j2 * (unsigned) LDK, tid, kJ);
+        rows.load(j2 * (LDK * (int) sizeof(TB)), kJ);
         SV_PIN_MEMORY;
-        const SvBound bound_j = sh.bound[j2];
-        const double z_j = sh.z[wave][j2];
+        z_at_j = my_z + 8u * (unsigned) j2;
+        const SvBound bound_j = sh.elem[j2].bound;
+        const double z_j = lds_f64(z_at_j);
         SV_PIN;
-        const double steps = step.b / step.a;   // (every row's, while the bounds are read)
+        const double steps = cj.step.b / cj.step.a;   // (every row's, while the bounds are read)
         const double q2 = readlane_f64(steps, row);
-        SV_PIN;
+        bit_j = own_bit<E>(tid, j2);
         // (the two comparisons come out the same in every lane)
-        go = __builtin_amdgcn_ballot_w64(cj.go != 0);
-        const uint64_t sure = __builtin_amdgcn_ballot_w64(second < best * (1.0f - 0x1p-19f)) & __builtin_amdgcn_ballot_w64(best < 0x1p80f);
-        const uint64_t on = n_iter > max_iter ? 0 : go & sure;
-        if (on == 0) break;
-        const double l = fmin_f64(up_i, fmin_f64(z_j - bound_j.lo, q2));
-        const double nz_i = z_i + l, nz_j = z_j - l;
-        owner_i = i / E;
-        owner_j = j2 / E;
-        bit_i = 1u << (i & (E - 1));
-        bit_j = 1u << (j2 & (E - 1));
-        low_i = nz_i > bound_i.lo ? bit_i : 0;
-        low_j = nz_j > bound_j.lo ? bit_j : 0;
-        in_up = tid == owner_i ? (in_up & ~bit_i) | (nz_i < bound_i.hi ? bit_i : 0) : in_up;
-        in_up = tid == owner_j ? (in_up & ~bit_j) | (nz_j < bound_j.hi ? bit_j : 0) : in_up;
-        write_by_lane0(1, &sh.z[wave][i], nz_i, &sh.z[wave][j2], nz_j);
+        go = __builtin_amdgcn_ballot_w64(cj.score.go != 0);
+        const uint64_t sure = __builtin_amdgcn_ballot_w64(next < best * (1.0f - 0x1p-19f)) & __builtin_amdgcn_ballot_w64(best < 0x1p80f);
+        if ((go & sure) == 0) break;
+        SV_PIN;
+        const double l = fmin_f64(fmin_f64(up_i, z_j - bound_j.lo), q2);
+        nz_i = z_i + l;
+        nz_j = z_j - l;
+        const unsigned up_i_on = same_in_all_lanes(nz_i < bound_i.hi), up_j_on = same_in_all_lanes(nz_j < bound_j.hi);
+        low_i = same_in_all_lanes(nz_i > bound_i.lo);
+        low_j = same_in_all_lanes(nz_j > bound_j.lo);
+        in_up = put_bits(put_bits(in_up, bit_i, up_i_on), bit_j, up_j_on);
+        pending = 1;
         SV_PIN;
 #pragma unroll
         for (int e = 0; e < E; ++e) f[e] = __builtin_fma(-l, (double) kJ[e] - (double) kI[e], f[e]);
         ++n_iter;
     }
-    return go == 0 || n_iter > max_iter;
+    return go == 0;
 }
 
 // Elements beyond ws are given y = 0, which puts them in neither I_up nor I_low.
@@ -556,8 +594,8 @@ __global__ __launch_bounds__(64 * W) void c_smo_solve_kernel(
     constexpr int N = E * 64 * W;
     __shared__ SvState<N, W> sh;
     __shared__ double s_red[2][W];
-    __shared__ SvCand s_i[4 * W], s_j[4 * W];   // (SvScore has SvCand's size)
-    __shared__ SvStep s_step[4 * W];
+    __shared__ SvCand s_i[4 * W], s_j[4 * W];
+    __shared__ SvScoreStep s_score[4 * W];
 
     // This workgroup is a chain of dependent operations; when a chip-wide kernel runs next to it on
     // another stream its wavefronts must not wait behind that kernel's for issue slots.
@@ -573,9 +611,9 @@ __global__ __launch_bounds__(64 * W) void c_smo_solve_kernel(
         for (int e = 0; e < E; ++e) {
             const int t = tid * E + e;
             const double y = (double) y_of[e];
-            sh.kd[t] = kd[e];
-            sh.bound[t].hi = y > 0 ? Cp : 0.0;
-            sh.bound[t].lo = y < 0 ? -Cn : 0.0;
+            sh.elem[t].kd = kd[e];
+            sh.elem[t].bound.hi = y > 0 ? Cp : 0.0;
+            sh.elem[t].bound.lo = y < 0 ? -Cn : 0.0;
             plus |= (y > 0 ? 1u : 0u) << e;
 #pragma unroll
             for (int w = 0; w < W; ++w) sh.z[w][t] = a_old[e] * y;
@@ -620,7 +658,7 @@ __global__ __launch_bounds__(64 * W) void c_smo_solve_kernel(
             int stretch = 4;
             do {
                 const int before = n_iter;
-                done = c_smo_iterate_rounded<E, LDK, TB>(sh, s_i, (SvScore *) s_j, s_step, ws, kws, kd, f, in_up, in_low, local_eps, max_iter, n_iter);
+                done = c_smo_iterate_rounded<E, LDK, TB>(sh, s_i, s_score, ws, kws, kd, f, in_up, in_low, local_eps, max_iter, n_iter);
                 if (done) break;
                 stretch = n_iter - before > stretch ? 4 : stretch < 1024 ? 8 * stretch : stretch;
                 done = c_smo_iterate<E, W, LDK, false, TB>(sh, s_i, s_j, ws, kws, kd, f, in_up, in_low, local_eps, max_iter, n_iter, stretch, no_score);
