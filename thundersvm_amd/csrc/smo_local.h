@@ -119,10 +119,10 @@ __device__ __forceinline__ void publish(S *slot, uint64_t lanes, double x, doubl
 }
 // The same with the lane's E values of f and of the block row for the step (the row's values in slots of eight bytes).
 // (One asm statement each: nothing else may come between the two writes of exec.)
+// `only`: the lanes that write, each to slots of its own.
 template <int E, typename TB>
-__device__ __forceinline__ void publish_row(double *f_slot, double *k_slot, int lane, const double (&f)[E], const TB (&k)[E]) {
+__device__ __forceinline__ void publish_row(double *f_slot, double *k_slot, uint64_t only, const double (&f)[E], const TB (&k)[E]) {
     const unsigned fa = lds_at(f_slot), ka = lds_at(k_slot);
-    const uint64_t only = 1ull << lane;
     static_assert(E == 1 || E == 2 || E == 4, "elements per thread");
     if constexpr (E == 1 && sizeof(TB) == 4)
         asm volatile(SV_EXEC_ON "ds_write_b64 %1, %3\n\tds_write_b32 %2, %4\n\t" SV_EXEC_OFF
@@ -168,19 +168,6 @@ __device__ __forceinline__ void write_by_lane0(int on, unsigned p, double v, uns
     asm volatile(SV_EXEC_ON "ds_write_b64 %1, %2\n\tds_write_b64 %3, %4\n\t" SV_EXEC_OFF :: "s"((uint64_t) (uint32_t) on), "v"(p), "v"(v), "v"(q), "v"(w) : "memory");
 }
 
-// The workgroup's best candidate: every lane reads one of the W, two DPP steps compare them.  The elements of a
-// wavefront are neighbours and the wavefronts follow one another: among equal values the first wavefront has the
-// lowest element.  `at` and `flags` come back as scalars.
-template <int W>
-__device__ __forceinline__ void block_argmin(const SvCand *slots, int lane, double &v, int &at, int &flags) {
-    static_assert(W == 2 || W == 4, "quad_perm steps");
-    const SvCand c = slots[lane & (W - 1)];
-    double m = fmin_f64(c.v, dpp_f64<TSVM_DPP_XOR1>(c.v));
-    if (W == 4) m = fmin_f64(m, dpp_f64<TSVM_DPP_XOR2>(m));
-    v = m;
-    at = __builtin_amdgcn_readlane(c.at, __builtin_ctzll(__builtin_amdgcn_ballot_w64(c.v == m)));
-    flags = __builtin_amdgcn_ballot_w64(c.flag != 0) != 0;
-}
 template <int W>
 __device__ __forceinline__ double block_max(const double *s_v) {
     double v = s_v[0];
@@ -198,12 +185,12 @@ __device__ __forceinline__ unsigned set_member_bits(unsigned m, int tid, int t, 
     return tid == (int) ((unsigned) t / E) ? changed : m;
 }
 
-// Membership bits of the c variant, one per element, in three instructions a change.  own_bit: element t's bit in the thread that owns
-// it; in another one it is a bit from E on, which nobody reads.  A decision that all lanes have come to alike is a mask of
+// Membership bits in three instructions a change.  own_bit: element t's first bit (of EACH) in the thread that owns it; in another
+// one it is a bit beyond the elements', which nobody reads.  A decision that all lanes have come to alike is a mask of
 // ones or zeros in a scalar register.
-template <int E>
+template <int E, int EACH = 1>
 __device__ __forceinline__ unsigned own_bit(int tid, int t) {
-    const unsigned at = (unsigned) (t - tid * E);
+    const unsigned at = (unsigned) (t - tid * E) * EACH;
     return 1u << (at < 31u ? at : 31u);
 }
 __device__ __forceinline__ unsigned same_in_all_lanes(bool x) { return (unsigned) __builtin_amdgcn_ballot_w64(x); }
@@ -301,6 +288,76 @@ __device__ __forceinline__ void row_first_candidate(const double (&x)[E], const 
             : "v148", "v149", "v150", "v151");
     }
 }
+// Two of them, for the nu variant's sides: each chain fills the other's wait states.
+#define SV_MOVS(CTRL) SV_DPP_MOV("v148", "v150", CTRL) SV_DPP_MOV("v149", "v151", CTRL) SV_DPP_MOV("v156", "v158", CTRL) SV_DPP_MOV("v157", "v159", CTRL)
+#define SV_MINS "v_min_f64 v[150:151], v[150:151], v[148:149]\n\tv_min_f64 v[158:159], v[158:159], v[156:157]\n\t"
+#define SV_FIRST_MOVS(CTRL) SV_DPP_MOV("v148", "v144", CTRL) SV_DPP_MOV("v149", "v145", CTRL) SV_DPP_MOV("v156", "v152", CTRL) SV_DPP_MOV("v157", "v153", CTRL) \
+    "v_min_f64 v[150:151], v[144:145], v[148:149]\n\tv_min_f64 v[158:159], v[152:153], v[156:157]\n\t"
+template <int E>
+__device__ __forceinline__ void row_first_candidates(const double (&x)[E], const double (&y)[E], const int (&at)[E], SvWords &rec_x, SvWords &rec_y,
+                                                     uint64_t &has_x, uint64_t &has_y) {
+    uint64_t x0, x1, x2, y0, y1, y2;
+    if constexpr (E == 4) {
+        asm("v_min_f64 v[144:145], %10, %11\n\t"
+            "v_min_f64 v[152:153], %14, %15\n\t"
+            "v_min_f64 v[148:149], %12, %13\n\t"
+            "v_min_f64 v[156:157], %16, %17\n\t"
+            "v_min_f64 v[144:145], v[144:145], v[148:149]\n\t"
+            "v_min_f64 v[152:153], v[152:153], v[156:157]\n\t"
+            "v_cmp_eq_f64_e64 %4, %10, v[144:145]\n\t"
+            "v_cmp_eq_f64_e64 %5, %11, v[144:145]\n\t"
+            "v_cmp_eq_f64_e64 %6, %12, v[144:145]\n\t"
+            "v_cmp_eq_f64_e64 %7, %14, v[152:153]\n\t"
+            "v_cmp_eq_f64_e64 %8, %15, v[152:153]\n\t"
+            "v_cmp_eq_f64_e64 %9, %16, v[152:153]\n\t"
+            SV_FIRST_MOVS("quad_perm:[1,0,3,2]")
+            "v_cndmask_b32_e64 v146, %21, %20, %6\n\t"
+            "v_cndmask_b32_e64 v154, %21, %20, %9\n\t"
+            SV_MOVS("quad_perm:[2,3,0,1]") SV_MINS
+            "v_cndmask_b32_e64 v146, v146, %19, %5\n\t"
+            "v_cndmask_b32_e64 v154, v154, %19, %8\n\t"
+            SV_MOVS("row_half_mirror") SV_MINS
+            "v_cndmask_b32_e64 v146, v146, %18, %4\n\t"
+            "v_cndmask_b32_e64 v154, v154, %18, %7\n\t"
+            SV_MOVS("row_mirror") SV_MINS
+            "v_cmp_eq_f64_e64 %2, v[144:145], v[150:151]\n\t"
+            "v_cmp_eq_f64_e64 %3, v[152:153], v[158:159]"
+            : "=&{v[144:147]}"(rec_x), "=&{v[152:155]}"(rec_y), "=&s"(has_x), "=&s"(has_y), "=&s"(x0), "=&s"(x1), "=&s"(x2), "=&s"(y0), "=&s"(y1), "=&s"(y2)
+            : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(y[0]), "v"(y[1]), "v"(y[2]), "v"(y[3]), "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3])
+            : "v148", "v149", "v150", "v151", "v156", "v157", "v158", "v159");
+    } else {
+        static_assert(E == 2, "elements per thread");
+        asm("v_min_f64 v[144:145], %6, %7\n\t"
+            "v_min_f64 v[152:153], %8, %9\n\t"
+            "v_cmp_eq_f64_e64 %4, %6, v[144:145]\n\t"
+            "v_cmp_eq_f64_e64 %5, %8, v[152:153]\n\t"
+            SV_FIRST_MOVS("quad_perm:[1,0,3,2]")
+            "v_cndmask_b32_e64 v146, %11, %10, %4\n\t"
+            SV_MOVS("quad_perm:[2,3,0,1]") SV_MINS
+            "v_cndmask_b32_e64 v154, %11, %10, %5\n\t"
+            SV_MOVS("row_half_mirror") SV_MINS
+            "s_nop 0\n\t" SV_MOVS("row_mirror") SV_MINS
+            "v_cmp_eq_f64_e64 %2, v[144:145], v[150:151]\n\t"
+            "v_cmp_eq_f64_e64 %3, v[152:153], v[158:159]"
+            : "=&{v[144:147]}"(rec_x), "=&{v[152:155]}"(rec_y), "=&s"(has_x), "=&s"(has_y), "=&s"(x0), "=&s"(y0)
+            : "v"(x[0]), "v"(x[1]), "v"(y[0]), "v"(y[1]), "v"(at[0]), "v"(at[1])
+            : "v148", "v149", "v150", "v151", "v156", "v157", "v158", "v159");
+    }
+}
+__device__ __forceinline__ void row_mins_and_who(double x, double y, double &min_x, double &min_y, uint64_t &who_x, uint64_t &who_y) {
+    const double s = dpp_f64<TSVM_DPP_XOR1>(x), t = dpp_f64<TSVM_DPP_XOR1>(y);
+    asm("v_min_f64 v[150:151], %4, %5\n\t"
+        "v_min_f64 v[158:159], %6, %7\n\t"
+        "s_nop 0\n\t" SV_MOVS("quad_perm:[2,3,0,1]") SV_MINS
+        "s_nop 0\n\t" SV_MOVS("row_half_mirror") SV_MINS
+        "s_nop 0\n\t" SV_MOVS("row_mirror")
+        "v_min_f64 %0, v[150:151], v[148:149]\n\t"
+        "v_min_f64 %1, v[158:159], v[156:157]\n\t"
+        "v_cmp_eq_f64_e64 %2, %4, %0\n\t"
+        "v_cmp_eq_f64_e64 %3, %6, %1"
+        : "=&v"(min_x), "=&v"(min_y), "=&s"(who_x), "=&s"(who_y) : "v"(x), "v"(s), "v"(y), "v"(t)
+        : "v148", "v149", "v150", "v151", "v156", "v157", "v158", "v159");
+}
 // row_min, with the lanes that have it.
 __device__ __forceinline__ void row_min_and_who(double x, double &value, uint64_t &who) {
     const double t = dpp_f64<TSVM_DPP_XOR1>(x);
@@ -311,6 +368,46 @@ __device__ __forceinline__ void row_min_and_who(double x, double &value, uint64_
         "v_min_f64 %0, v[150:151], v[148:149]\n\t"
         "v_cmp_eq_f64_e64 %1, %2, %0"
         : "=&v"(value), "=s"(who) : "v"(x), "v"(t) : "v148", "v149", "v150", "v151");
+}
+// The lowest lane of every row among those that are set; the last one where none is (whatever is NaN).
+__device__ __forceinline__ uint64_t lowest_of_rows(uint64_t lanes) {
+    lanes |= 0x8000800080008000ull;
+    return lanes & ~(lanes - 0x0001000100010001ull);
+}
+// The smallest of four wavefronts' E * 256 values and the number of the first element that has it, over sixteen rows of lanes; `flag`
+// comes back as whether any row's was set.  also: writes by the rows' candidates, by their lanes, in front of the barrier.
+template <int E, typename F>
+__device__ __forceinline__ void block_first_min(SvCand *slots, const double (&x)[E], const int (&at)[E], int flag, F also, double &value, int &first, int &any) {
+    SvWords rec;
+    uint64_t has, who;
+    row_first_candidate<E>(x, at, rec, has);
+    const uint64_t lanes = lowest_of_rows(has);
+    also(lanes);
+    rec[3] = flag;
+    publish_words(lds_at(slots + (threadIdx.x >> 4)), lanes, rec);
+    lds_barrier();
+    const SvCand c = slots[threadIdx.x & 15];
+    row_min_and_who(c.v, value, who);
+    first = __builtin_amdgcn_readlane(c.at, __builtin_ctzll(who));
+    any = __builtin_amdgcn_ballot_w64(c.flag != 0) != 0;
+}
+template <int E, typename F>
+__device__ __forceinline__ void block_first_mins(SvCand *slots_x, SvCand *slots_y, const double (&x)[E], const double (&y)[E], const int (&at)[E], int flag, F also,
+                                                 double &min_x, double &min_y, int &first_x, int &first_y, int &any) {
+    SvWords rec_x, rec_y;
+    uint64_t has_x, has_y, who_x, who_y;
+    row_first_candidates<E>(x, y, at, rec_x, rec_y, has_x, has_y);
+    const uint64_t lanes_x = lowest_of_rows(has_x), lanes_y = lowest_of_rows(has_y);
+    also(lanes_x, lanes_y);
+    rec_x[3] = flag;
+    publish_words(lds_at(slots_x + (threadIdx.x >> 4)), lanes_x, rec_x);
+    publish_words(lds_at(slots_y + (threadIdx.x >> 4)), lanes_y, rec_y);
+    lds_barrier();
+    const SvCand cx = slots_x[threadIdx.x & 15], cy = slots_y[threadIdx.x & 15];
+    row_mins_and_who(cx.v, cy.v, min_x, min_y, who_x, who_y);
+    first_x = __builtin_amdgcn_readlane(cx.at, __builtin_ctzll(who_x));
+    first_y = __builtin_amdgcn_readlane(cy.at, __builtin_ctzll(who_y));
+    any = __builtin_amdgcn_ballot_w64(cx.flag != 0) != 0;
 }
 // row_best_two over sixteen lanes, with the lanes that have the best.
 __device__ __forceinline__ void row_best_two_and_who(float mine, float second_in, float &best, float &second, uint64_t &who) {

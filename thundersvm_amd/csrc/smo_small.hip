@@ -385,7 +385,7 @@ __device__ __forceinline__ bool ss_local(SmallShared<E, W> &sh, const SmallMap &
                 qs[e] = __hiloint2double(b[q][e] > 0.0 ? __double2hiint(s) : SV_NONE_HI, __double2loint(s));
             }
             const int win = wave_argmin_by_pos<E>(qs, sh.pos, tid, best[q], v, at[q]);
-            publish_row<E, TB>(sh.f + tid * E, sh.k + tid * E, win, f, kI[q]);
+            publish_row<E, TB>(sh.f + tid * E, sh.k + tid * E, 1ull << win, f, kI[q]);
             if constexpr (W > 1) publish(cj[q] + wave, 1ull << win, v, at[q], go);
             else js[q] = __builtin_amdgcn_readlane(at[q], win);
         }

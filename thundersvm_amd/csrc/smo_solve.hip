@@ -308,20 +308,19 @@ __device__ __forceinline__ bool solver_begins(int *gate, int epoch, int target_x
     return true;
 }
 
-// What the nu solver keeps in LDS, per element of the working set (inactive elements: both bounds zero, so neither in
-// I_up nor in I_low).
-template <int N, int W>
-struct SvShared {
-    double kd[N];
-    SvBound bound[N];
-    double z[W][N];           // alpha times its label: every wavefront keeps a copy of its own, which needs no barrier
-};
-
-// What c_smo_solve keeps.  (An element's bounds and diagonal are read by one address.)
+// What the solvers keep in LDS per element of the working set (inactive elements: both bounds zero, so neither in I_up nor in
+// I_low).  Bounds and diagonal are read by one address.
 struct __align__(32) SvElem {
     SvBound bound;
     double kd, unused;
 };
+template <int N, int W>
+struct SvShared {
+    SvElem elem[N];
+    double z[W][N];           // alpha times its label: every wavefront keeps a copy of its own, which needs no barrier
+};
+
+// What c_smo_solve keeps.
 template <int N, int W>
 struct SvState {
     SvElem elem[N];
@@ -329,7 +328,11 @@ struct SvState {
     double f[N], k[N];        // f and row i at the elements of the wavefronts' candidates for j2 (the others are not written)
 };
 
-// The iterations of c_smo_solve.  An element that violates may have no score: the threshold is not positive and its f not above
+// The iterations of c_smo_solve.  Four wavefronts compare by rows of sixteen lanes (block_first_min), as c_smo_iterate_rounded does: the same
+// eight steps as over a wavefront and then over four, without the way through the scalar unit in between, worth its sixteen records
+// since the chains are single blocks (3200x32, where nothing is decided by rounded scores: 2.58 -> 2.53 ms a call; z and in_low
+// left to the next step's waits, as there: 2.55).
+// An element that violates may have no score: the threshold is not positive and its f not above
 // `up`, or the score is infinite or NaN (an a that is negative with a b^2 beyond the largest double; kernel values that are no
 // numbers).  The reference's j2 then stays 0 (smo_kernel.cpp:78).  NONE: that is done here.  Without it such a step goes
 // wrong, and `no_score` is set for the caller to start over; one instruction, where a way out of the loop in front of the
@@ -340,7 +343,15 @@ __device__ __forceinline__ bool c_smo_iterate(SvState<E * 64 * W, W> &sh, SvCand
                                               const double (&kd)[E], double (&f)[E], unsigned &in_up, unsigned &in_low, double local_eps,
                                               int max_iter, int &n_iter, int left, bool &no_score) {
     const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const BlockRows<E, TB> rows(kws, (unsigned) ws * (unsigned) LDK, tid);
+    auto load_row = [&](int r, TB (&out)[E]) {
+        if constexpr (W == 4) rows.load(r * (LDK * (int) sizeof(TB)), out);
+        else load_row_elems<E, TB>(kws + (unsigned) r * (unsigned) LDK, tid, out);
+    };
+    int own[E];   // (whoever is chosen without being a candidate is one that exists)
+#pragma unroll
+    for (int e = 0; e < E; ++e) own[e] = tid * E + e < ws ? tid * E + e : ws - 1;
     bool go_on;
     double min_t = -TSVM_INF;
     int worst = 0;   // high word of the largest score that a step was taken on
@@ -352,17 +363,15 @@ __device__ __forceinline__ bool c_smo_iterate(SvState<E * 64 * W, W> &sh, SvCand
         for (int e = 0; e < E; ++e) fu[e] = keep_or_none<0>(in_up << (31 - e), f[e]);
         double up_value, m;
         int at, i, j2, go;
-        const int win_i = wave_first_argmin<E>(fu, tid * E, up_value, m, at);
-        if constexpr (W > 1) {
-            publish(s_i + wave, 1ull << win_i, m, at, 0);
-            lds_barrier();
-            block_argmin<W>(s_i, lane, up_value, i, go);
+        if constexpr (W == 4) {
+            block_first_min<E>(s_i, fu, own, 0, [](uint64_t) {}, up_value, i, go);
         } else {
+            const int win_i = wave_first_argmin<E>(fu, tid * E, up_value, m, at);
             i = __builtin_amdgcn_readlane(at, win_i);
+            i = i < ws ? i : ws - 1;   // (without a candidate the index may be an inactive element's)
         }
-        i = i < ws ? i : ws - 1;   // (without a candidate the index may be an inactive element's)
         TB kI[E];
-        load_row_elems<E, TB>(kws + (unsigned) i * (unsigned) LDK, tid, kI);
+        load_row(i, kI);
         SV_PIN_MEMORY;
         const double kd_i = sh.elem[i].kd, z_i = sh.z[wave][i];
         const SvBound bound_i = sh.elem[i].bound;
@@ -387,13 +396,11 @@ __device__ __forceinline__ bool c_smo_iterate(SvState<E * 64 * W, W> &sh, SvCand
             // (-up > -f in the reference: f > up, which is b > 0; outside I_low b is negative and q of no use)
             qs[e] = __hiloint2double(b_low[e] > 0.0 ? __double2hiint(q) : SV_NONE_HI, __double2loint(q));
         }
-        const int win_j = wave_first_argmin<E>(qs, tid * E, min_t, m, at);
-        publish_row<E, TB>(sh.f + tid * E, sh.k + tid * E, win_j, f, kI);
-        if constexpr (W > 1) {
-            publish(s_j + wave, 1ull << win_j, m, at, go);
-            lds_barrier();
-            block_argmin<W>(s_j, lane, min_t, j2, go);
+        if constexpr (W == 4) {
+            block_first_min<E>(s_j, qs, own, go, [&](uint64_t lanes) { publish_row<E, TB>(sh.f + tid * E, sh.k + tid * E, lanes, f, kI); }, min_t, j2, go);
         } else {
+            const int win_j = wave_first_argmin<E>(qs, tid * E, min_t, m, at);
+            publish_row<E, TB>(sh.f + tid * E, sh.k + tid * E, 1ull << win_j, f, kI);
             j2 = __builtin_amdgcn_readlane(at, win_j);
         }
         if (NONE && is_none(min_t)) {
@@ -402,9 +409,9 @@ __device__ __forceinline__ bool c_smo_iterate(SvState<E * 64 * W, W> &sh, SvCand
             if (tid == 0) { sh.f[0] = f[0]; *(TB *) sh.k = kI[0]; }
             __syncthreads();
         }
-        j2 = j2 < ws ? j2 : ws - 1;
+        if constexpr (W != 4) j2 = j2 < ws ? j2 : ws - 1;
         TB kJ[E];
-        load_row_elems<E, TB>(kws + (unsigned) j2 * (unsigned) LDK, tid, kJ);
+        load_row(j2, kJ);
         SV_PIN_MEMORY;
         const SvBound bound_j = sh.elem[j2].bound;
         const double kd_j = sh.elem[j2].kd, z_j = sh.z[wave][j2], f_j = sh.f[j2];
@@ -474,9 +481,7 @@ __device__ __forceinline__ bool c_smo_iterate_rounded(SvState<E * 256, 4> &sh, S
         SvWords cand;
         uint64_t has;
         row_first_candidate<E>(fu, at_of, cand, has);
-        // the lowest lane of every row that has it (every field of sixteen bits has one set, whatever is NaN)
-        has |= 0x8000800080008000ull;
-        publish_words(my_i, has & ~(has - 0x0001000100010001ull), cand);
+        publish_words(my_i, lowest_of_rows(has), cand);
         lds_barrier();
         const SvCand ci = s_i[lane & 15];
         write_by_lane0(pending, z_at_i, nz_i, z_at_j, nz_j);
@@ -704,7 +709,15 @@ __device__ __forceinline__ bool nu_iterate(SvShared<E * 64 * W, W> &sh, double (
                                            SvCand *s_jp, SvCand *s_jn, int ws, const TB *kws, const double (&kd)[E], double (&f)[E], unsigned &member,
                                            double local_eps, int max_iter, int &n_iter, int left) {
     const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const BlockRows<E, TB> rows(kws, (unsigned) ws * (unsigned) LDK, tid);
+    auto load_row = [&](int r, TB (&out)[E]) {
+        if constexpr (W == 4) rows.load(r * (LDK * (int) sizeof(TB)), out);
+        else load_row_elems<E, TB>(kws + (unsigned) r * (unsigned) LDK, tid, out);
+    };
+    int own[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) own[e] = tid * E + e < ws ? tid * E + e : ws - 1;
     for (; left > 0; --left) {
         double fup[E], fun[E];
 #pragma unroll
@@ -714,15 +727,11 @@ __device__ __forceinline__ bool nu_iterate(SvShared<E * 64 * W, W> &sh, double (
         }
         double up_value_p, up_value_n, m_p, m_n;
         int ip, in, at_p, at_n, go;
-        const int win_ip = wave_first_argmin<E>(fup, tid * E, up_value_p, m_p, at_p);
-        const int win_in = wave_first_argmin<E>(fun, tid * E, up_value_n, m_n, at_n);
-        if constexpr (W > 1) {
-            publish(s_ip + wave, 1ull << win_ip, m_p, at_p, 0);
-            publish(s_in + wave, 1ull << win_in, m_n, at_n, 0);
-            lds_barrier();
-            block_argmin<W>(s_ip, lane, up_value_p, ip, go);
-            block_argmin<W>(s_in, lane, up_value_n, in, go);
+        if constexpr (W == 4) {
+            block_first_mins<E>(s_ip, s_in, fup, fun, own, 0, [](uint64_t, uint64_t) {}, up_value_p, up_value_n, ip, in, go);
         } else {
+            const int win_ip = wave_first_argmin<E>(fup, tid * E, up_value_p, m_p, at_p);
+            const int win_in = wave_first_argmin<E>(fun, tid * E, up_value_n, m_n, at_n);
             ip = __builtin_amdgcn_readlane(at_p, win_ip);
             in = __builtin_amdgcn_readlane(at_n, win_in);
         }
@@ -730,10 +739,10 @@ __device__ __forceinline__ bool nu_iterate(SvShared<E * 64 * W, W> &sh, double (
         ip = is_none(up_value_p) ? 0 : ip;
         in = is_none(up_value_n) ? 0 : in;
         TB kIp[E], kIn[E];
-        load_row_elems<E, TB>(kws + (unsigned) ip * (unsigned) LDK, tid, kIp);
-        load_row_elems<E, TB>(kws + (unsigned) in * (unsigned) LDK, tid, kIn);
+        load_row(ip, kIp);
+        load_row(in, kIn);
         SV_PIN_MEMORY;
-        const double kd_ip = sh.kd[ip], kd_in = sh.kd[in];
+        const double kd_ip = sh.elem[ip].kd, kd_in = sh.elem[in].kd;
         double a_part[E], lp[E], ln[E], b_max = -TSVM_INF;
 #pragma unroll
         for (int e = 0; e < E; ++e) {
@@ -756,18 +765,16 @@ __device__ __forceinline__ bool nu_iterate(SvShared<E * 64 * W, W> &sh, double (
         }
         double f_val_j2p, f_val_j2n;
         int j2p, j2n;
-        const int win_jp = wave_first_argmin<E>(qp, tid * E, f_val_j2p, m_p, at_p);
-        const int win_jn = wave_first_argmin<E>(qn, tid * E, f_val_j2n, m_n, at_n);
-        publish_row<E, TB>(s_f[0] + tid * E, s_k[0] + tid * E, win_jp, f, kIp);
-        publish_row<E, TB>(s_f[1] + tid * E, s_k[1] + tid * E, win_jn, f, kIn);
-        if constexpr (W > 1) {
-            publish(s_jp + wave, 1ull << win_jp, m_p, at_p, go);
-            publish(s_jn + wave, 1ull << win_jn, m_n, at_n, go);
-            lds_barrier();
-            block_argmin<W>(s_jp, lane, f_val_j2p, j2p, go);
-            int go_n;
-            block_argmin<W>(s_jn, lane, f_val_j2n, j2n, go_n);
+        if constexpr (W == 4) {
+            block_first_mins<E>(s_jp, s_jn, qp, qn, own, go, [&](uint64_t lanes_p, uint64_t lanes_n) {
+                publish_row<E, TB>(s_f[0] + tid * E, s_k[0] + tid * E, lanes_p, f, kIp);
+                publish_row<E, TB>(s_f[1] + tid * E, s_k[1] + tid * E, lanes_n, f, kIn);
+            }, f_val_j2p, f_val_j2n, j2p, j2n, go);
         } else {
+            const int win_jp = wave_first_argmin<E>(qp, tid * E, f_val_j2p, m_p, at_p);
+            const int win_jn = wave_first_argmin<E>(qn, tid * E, f_val_j2n, m_n, at_n);
+            publish_row<E, TB>(s_f[0] + tid * E, s_k[0] + tid * E, 1ull << win_jp, f, kIp);
+            publish_row<E, TB>(s_f[1] + tid * E, s_k[1] + tid * E, 1ull << win_jn, f, kIn);
             j2p = __builtin_amdgcn_readlane(at_p, win_jp);
             j2n = __builtin_amdgcn_readlane(at_n, win_jn);
         }
@@ -782,12 +789,12 @@ __device__ __forceinline__ bool nu_iterate(SvShared<E * 64 * W, W> &sh, double (
             if (tid == 0) { s_f[side][0] = f[0]; *(TB *) s_k[side] = take_p ? kIp[0] : kIn[0]; }
             __syncthreads();
         }
-        j2 = j2 < ws ? j2 : ws - 1;
+        if constexpr (W != 4) j2 = j2 < ws ? j2 : ws - 1;
         TB kJ[E];
-        load_row_elems<E, TB>(kws + (unsigned) j2 * (unsigned) LDK, tid, kJ);
+        load_row(j2, kJ);
         SV_PIN_MEMORY;
-        const double kd_j = sh.kd[j2], z_j = sh.z[wave][j2], z_i = sh.z[wave][i], f_j = s_f[side][j2];
-        const SvBound bound_i = sh.bound[i], bound_j = sh.bound[j2];
+        const double kd_j = sh.elem[j2].kd, z_j = sh.z[wave][j2], z_i = sh.z[wave][i], f_j = s_f[side][j2];
+        const SvBound bound_i = sh.elem[i].bound, bound_j = sh.elem[j2].bound;
         const double kIj = (double) *(const TB *) (s_k[side] + j2);
         SV_PIN;   // the row is on its way while the exit test and the step are computed
         if (n_iter > max_iter || !go) return true;
@@ -795,8 +802,11 @@ __device__ __forceinline__ bool nu_iterate(SvShared<E * 64 * W, W> &sh, double (
         const double q2 = (-up_value + f_j) / __builtin_fma(-2.0, kIj, (take_p ? kd_ip : kd_in) + kd_j);
         const double l = fmin_f64(bound_i.hi - z_i, fmin_f64(z_j - bound_j.lo, q2));
         const double nz_i = z_i + l, nz_j = (j2 == i ? nz_i : z_j) - l;
-        member = set_member_bits<E, 4>(member, tid, i, nu_member_bits(nz_i, bound_i));
-        member = set_member_bits<E, 4>(member, tid, j2, nu_member_bits(nz_j, bound_j));
+        const unsigned bit_i = own_bit<E, 4>(tid, i) << (bound_i.hi > 0 ? 0 : 1), bit_j = own_bit<E, 4>(tid, j2) << (bound_j.hi > 0 ? 0 : 1);
+        const unsigned up_i_on = same_in_all_lanes(nz_i < bound_i.hi), low_i_on = same_in_all_lanes(nz_i > bound_i.lo);
+        const unsigned up_j_on = same_in_all_lanes(nz_j < bound_j.hi), low_j_on = same_in_all_lanes(nz_j > bound_j.lo);
+        member = put_bits(put_bits(member, bit_i, up_i_on), bit_i << 2, low_i_on);
+        member = put_bits(put_bits(member, bit_j, up_j_on), bit_j << 2, low_j_on);
         write_by_lane0(1, &sh.z[wave][i], nz_i, &sh.z[wave][j2], nz_j);
         SV_PIN;   // (nothing above waits for the row)
 #pragma unroll
@@ -810,15 +820,27 @@ __device__ __forceinline__ bool nu_iterate(SvShared<E * 64 * W, W> &sh, double (
 // (c_smo_iterate_rounded: the same bounds, over the scores of both sides, whose largest has to beat every other; a side without
 // a candidate for i leaves it undecided).  Both sides' scores have row ip's a (smo_kernel.cpp:239), the step the chosen
 // side's own.  Bound by the issue of its instructions: eight divisions of doubles and two reductions over them become four
-// reciprocals and one over floats.  1024 elements, 401 steps: 672 -> 539 us; a nu-SVC training of 5001x23: 4.00 -> 3.56 ms.
+// reciprocals and one over floats.  1024 elements, 401 steps: 672 -> 539 us; a nu-SVC training of 5001x23: 4.00 -> 3.56 ms.  With the two
+// sides' chains of DPP steps interleaved (each fills the other's wait states) and the rest as in c_smo_iterate_rounded 3.14 -> 3.02.
 template <int E, int LDK, typename TB>
-__device__ __forceinline__ bool nu_iterate_rounded(SvShared<E * 256, 4> &sh, SvCand *s_ip, SvCand *s_in, SvScore *s_j, SvStep *s_step, int ws, const TB *kws,
+__device__ __forceinline__ bool nu_iterate_rounded(SvShared<E * 256, 4> &sh, SvCand *s_ip, SvCand *s_in, SvScoreStep *s_j, int ws, const TB *kws,
                                                    const double (&kd)[E], double (&f)[E], unsigned &member, double local_eps, int max_iter,
                                                    int &n_iter) {
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     constexpr int SIDE_N = 1 << 16;   // in an element's number: the score is the negative side's
+    const unsigned my_ip = lds_at(s_ip + (tid >> 4)), my_in = lds_at(s_in + (tid >> 4)), my_j = lds_at(s_j + (tid >> 4));
+    unsigned my_z = lds_at(&sh.z[wave][0]);
+    asm("" : "+v"(my_z));
+    const BlockRows<E, TB> rows(kws, (unsigned) ws * (unsigned) LDK, tid);
+    int own[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) own[e] = tid * E + e < ws ? tid * E + e : ws - 1;
     uint64_t go;
+    // (as in c_smo_iterate_rounded)
+    unsigned bit_i = 0, bit_j = 0, low_i = 0, low_j = 0, z_at_i = my_z, z_at_j = my_z;
+    double nz_i = 0, nz_j = 0;
+    int pending = 0;
     for (;;) {
         double fup[E], fun[E];
 #pragma unroll
@@ -826,25 +848,24 @@ __device__ __forceinline__ bool nu_iterate_rounded(SvShared<E * 256, 4> &sh, SvC
             fup[e] = keep_or_none<0>(member << (31 - 4 * e), f[e]);
             fun[e] = keep_or_none<0>(member << (30 - 4 * e), f[e]);
         }
-        double m_p, m_n;
-        int at_p, at_n;
-        const double r_p = row_first_min<E>(fup, tid * E, m_p, at_p), r_n = row_first_min<E>(fun, tid * E, m_n, at_n);
-        const uint64_t has_p = __builtin_amdgcn_ballot_w64(m_p == r_p) | 0x8000800080008000ull;
-        const uint64_t has_n = __builtin_amdgcn_ballot_w64(m_n == r_n) | 0x8000800080008000ull;
-        publish(s_ip + (tid >> 4), has_p & ~(has_p - 0x0001000100010001ull), m_p, at_p, 0);
-        publish(s_in + (tid >> 4), has_n & ~(has_n - 0x0001000100010001ull), m_n, at_n, 0);
+        SvWords cand_p, cand_n;
+        uint64_t has_p, has_n;
+        row_first_candidates<E>(fup, fun, own, cand_p, cand_n, has_p, has_n);
+        publish_words(my_ip, lowest_of_rows(has_p), cand_p);
+        publish_words(my_in, lowest_of_rows(has_n), cand_n);
         lds_barrier();
         const SvCand cp = s_ip[lane & 15], cn = s_in[lane & 15];
-        const double up_p = row_min(cp.v), up_n = row_min(cn.v);
-        int ip = __builtin_amdgcn_readlane(cp.at, __builtin_ctzll(__builtin_amdgcn_ballot_w64(cp.v == up_p)));
-        int in = __builtin_amdgcn_readlane(cn.at, __builtin_ctzll(__builtin_amdgcn_ballot_w64(cn.v == up_n)));
-        ip = ip < ws ? ip : ws - 1;
-        in = in < ws ? in : ws - 1;
+        write_by_lane0(pending, z_at_i, nz_i, z_at_j, nz_j);
+        member = put_bits(put_bits(member, bit_i, low_i), bit_j, low_j);
+        double up_p, up_n;
+        uint64_t who_p, who_n;
+        row_mins_and_who(cp.v, cn.v, up_p, up_n, who_p, who_n);
+        const int ip = __builtin_amdgcn_readlane(cp.at, __builtin_ctzll(who_p)), in = __builtin_amdgcn_readlane(cn.at, __builtin_ctzll(who_n));
         TB kIp[E], kIn[E];
-        load_row_elems<E, TB>(kws + (unsigned) ip * (unsigned) LDK, tid, kIp);
-        load_row_elems<E, TB>(kws + (unsigned) in * (unsigned) LDK, tid, kIn);
+        rows.load(ip * (LDK * (int) sizeof(TB)), kIp);
+        rows.load(in * (LDK * (int) sizeof(TB)), kIn);
         SV_PIN_MEMORY;
-        const double kd_ip = sh.kd[ip], kd_in = sh.kd[in];
+        const double kd_ip = sh.elem[ip].kd, kd_in = sh.elem[in].kd;
         double a_part[E], lp[E], ln[E], b_max = -TSVM_INF;
         float p32[E], n32[E];
 #pragma unroll
@@ -856,7 +877,7 @@ __device__ __forceinline__ bool nu_iterate_rounded(SvShared<E * 256, 4> &sh, SvC
             p32[e] = __builtin_fmaxf((float) lp[e], 0.0f);
             n32[e] = __builtin_fmaxf((float) ln[e], 0.0f);
         }
-        const int violates = __builtin_amdgcn_ballot_w64(!(b_max < local_eps)) != 0;
+        const int violates = (__builtin_amdgcn_ballot_w64(!(b_max < local_eps)) != 0) & (n_iter <= max_iter);
         // (as the bits of a float: nothing is decided with an `up` of no candidate or too close to zero)
         const int hp = __double2hiint(up_p) & 0x7fffffff, hn = __double2hiint(up_n) & 0x7fffffff;
         int a_max = hp < SV_UP_LEAST_HI || hp >= SV_NONE_HI || hn < SV_UP_LEAST_HI || hn >= SV_NONE_HI ? 0x7f800000 : 0;
@@ -877,16 +898,16 @@ __device__ __forceinline__ bool nu_iterate_rounded(SvShared<E * 256, 4> &sh, SvC
             const bool n_side = qn > qp;
             b_of[e] = n_side ? ln[e] : lp[e];
             k_of[e] = n_side ? kIn[e] : kIp[e];
-            at_of[e] = n_side ? (tid * E + e) | SIDE_N : tid * E + e;
+            at_of[e] = n_side ? own[e] | SIDE_N : own[e];
         }
-        float best, second;
+        float mine, second;
         if constexpr (E == 4) {
             const float h0 = __builtin_fmaxf(q[0], q[1]), h1 = __builtin_fmaxf(q[2], q[3]);
-            best = __builtin_fmaxf(h0, h1);
+            mine = __builtin_fmaxf(h0, h1);
             second = __builtin_fmaxf(__builtin_fmaxf(__builtin_fminf(h0, h1), __builtin_fminf(q[0], q[1])), __builtin_fminf(q[2], q[3]));
         } else {
             static_assert(E == 2, "elements per thread");
-            best = __builtin_fmaxf(q[0], q[1]);
+            mine = __builtin_fmaxf(q[0], q[1]);
             second = __builtin_fminf(q[0], q[1]);
         }
         second = __builtin_fmaxf(second, low);
@@ -895,7 +916,7 @@ __device__ __forceinline__ bool nu_iterate_rounded(SvShared<E * 256, 4> &sh, SvC
         TB k_at = k_of[E - 1];
 #pragma unroll
         for (int e = E - 2; e >= 0; --e) {
-            const bool is = q[e] == best;
+            const bool is = q[e] == mine;
             at = is ? at_of[e] : at;
             b_at = is ? b_of[e] : b_at;
             k_at = is ? k_of[e] : k_at;
@@ -903,47 +924,50 @@ __device__ __forceinline__ bool nu_iterate_rounded(SvShared<E * 256, 4> &sh, SvC
         }
         const double a_at = __builtin_fma(-2.0, (double) k_at, (at & SIDE_N ? kd_in : kd_ip) + kd_at);
         second = a_max < SV_A_BITS ? second : __builtin_inff();
-        const float mine = best;
-        row_best_two(best, second);
-        const uint64_t who = __builtin_amdgcn_ballot_w64(mine == best);   // (several only if nothing will be decided)
-        publish(s_j + (tid >> 4), who, best, second, at, violates);
-        publish(s_step + (tid >> 4), who, b_at, a_at);
+        float best, next;
+        uint64_t who;   // (several only if nothing will be decided)
+        row_best_two_and_who(mine, second, best, next, who);
+        publish_score(my_j, who, best, next, at, violates, b_at, a_at);
         lds_barrier();
-        const SvScore cj = s_j[lane & 15];
-        const SvStep step = s_step[lane & 15];
-        best = cj.best;
-        second = cj.second;
-        row_best_two(best, second);
-        const int row = __builtin_ctzll(__builtin_amdgcn_ballot_w64(cj.best == best));
-        const int won = __builtin_amdgcn_readlane(cj.at, row);
+        const SvScoreStep cj = s_j[lane & 15];
+        uint64_t first;
+        row_best_two_and_who(cj.score.best, cj.score.second, best, next, first);
+        const int row = __builtin_ctzll(first);
+        const int won = __builtin_amdgcn_readlane(cj.score.at, row);
         const bool n_side = (won & SIDE_N) != 0;
-        int j2 = won & (SIDE_N - 1);
-        j2 = j2 < ws ? j2 : ws - 1;
-        const int i = n_side ? in : ip;
+        const int j2 = won & (SIDE_N - 1), i = n_side ? in : ip;
         TB kJ[E];
-        load_row_elems<E, TB>(kws + (unsigned) j2 * (unsigned) LDK, tid, kJ);
+        rows.load(j2 * (LDK * (int) sizeof(TB)), kJ);
         SV_PIN_MEMORY;
-        const SvBound bound_i = sh.bound[i], bound_j = sh.bound[j2];
-        const double z_i = sh.z[wave][i], z_j = sh.z[wave][j2];
+        z_at_i = my_z + 8u * (unsigned) i;
+        z_at_j = my_z + 8u * (unsigned) j2;
+        const SvBound bound_i = sh.elem[i].bound, bound_j = sh.elem[j2].bound;
+        const double z_i = lds_f64(z_at_i), z_j = lds_f64(z_at_j);
         SV_PIN;
-        const double steps = step.b / step.a;   // (every row's, while the bounds are read)
+        const double steps = cj.step.b / cj.step.a;   // (every row's, while the bounds are read)
         const double q2 = readlane_f64(steps, row);
+        // (an element that a step is taken on is of the side it was chosen for)
+        const unsigned up_bit_i = own_bit<E, 4>(tid, i) << (n_side ? 1 : 0), up_bit_j = own_bit<E, 4>(tid, j2) << (n_side ? 1 : 0);
+        go = __builtin_amdgcn_ballot_w64(cj.score.go != 0);
+        const uint64_t sure = __builtin_amdgcn_ballot_w64(next < best * (1.0f - 0x1p-19f)) & __builtin_amdgcn_ballot_w64(best < 0x1p80f);
+        if ((go & sure) == 0) break;
         SV_PIN;
-        go = __builtin_amdgcn_ballot_w64(cj.go != 0);
-        const uint64_t sure = __builtin_amdgcn_ballot_w64(second < best * (1.0f - 0x1p-19f)) & __builtin_amdgcn_ballot_w64(best < 0x1p80f);
-        const uint64_t on = n_iter > max_iter ? 0 : go & sure;
-        if (on == 0) break;
-        const double l = fmin_f64(bound_i.hi - z_i, fmin_f64(z_j - bound_j.lo, q2));
-        const double nz_i = z_i + l, nz_j = z_j - l;
-        member = set_member_bits<E, 4>(member, tid, i, nu_member_bits(nz_i, bound_i));
-        member = set_member_bits<E, 4>(member, tid, j2, nu_member_bits(nz_j, bound_j));
-        write_by_lane0(1, &sh.z[wave][i], nz_i, &sh.z[wave][j2], nz_j);
+        const double l = fmin_f64(fmin_f64(bound_i.hi - z_i, z_j - bound_j.lo), q2);
+        nz_i = z_i + l;
+        nz_j = z_j - l;
+        const unsigned up_i_on = same_in_all_lanes(nz_i < bound_i.hi), up_j_on = same_in_all_lanes(nz_j < bound_j.hi);
+        low_i = same_in_all_lanes(nz_i > bound_i.lo);
+        low_j = same_in_all_lanes(nz_j > bound_j.lo);
+        bit_i = up_bit_i << 2;
+        bit_j = up_bit_j << 2;
+        member = put_bits(put_bits(member, up_bit_i, up_i_on), up_bit_j, up_j_on);
+        pending = 1;
         SV_PIN;
 #pragma unroll
         for (int e = 0; e < E; ++e) f[e] = __builtin_fma(-l, (double) kJ[e] - (double) (n_side ? kIn[e] : kIp[e]), f[e]);
         ++n_iter;
     }
-    return go == 0 || n_iter > max_iter;
+    return go == 0;
 }
 
 template <int E, int W, int LDK, typename TB>
@@ -961,8 +985,8 @@ __global__ __launch_bounds__(64 * W) void nu_smo_solve_kernel(
     __shared__ SvShared<N, W> sh;
     __shared__ double s_f[2][N], s_k[2][N];   // f and the rows ip / in at the elements of the wavefronts' candidates for j2
     __shared__ double s_red[4][W];
-    __shared__ SvCand s_ip[4 * W], s_in[4 * W], s_jp[4 * W], s_jn[W];   // (SvScore has SvCand's size)
-    __shared__ SvStep s_step[4 * W];
+    __shared__ SvCand s_ip[4 * W], s_in[4 * W], s_jp[4 * W], s_jn[4 * W];
+    __shared__ SvScoreStep s_score[4 * W];
 
     __builtin_amdgcn_s_setprio(3);
     const int tid = threadIdx.x;
@@ -972,13 +996,13 @@ __global__ __launch_bounds__(64 * W) void nu_smo_solve_kernel(
     for (int e = 0; e < E; ++e) {
         const int t = tid * E + e;
         const double y = (double) y_of[e];
-        sh.kd[t] = kd[e];
-        sh.bound[t].hi = y > 0 ? C : 0.0;
-        sh.bound[t].lo = y < 0 ? -C : 0.0;
+        sh.elem[t].kd = kd[e];
+        sh.elem[t].bound.hi = y > 0 ? C : 0.0;
+        sh.elem[t].bound.lo = y < 0 ? -C : 0.0;
         plus |= (y > 0 ? 1u : 0u) << e;
 #pragma unroll
         for (int w = 0; w < W; ++w) sh.z[w][t] = a_old[e] * y;
-        member |= nu_member_bits(a_old[e] * y, sh.bound[t]) << (4 * e);
+        member |= nu_member_bits(a_old[e] * y, sh.elem[t].bound) << (4 * e);
     }
     // initial gap -> local stopping threshold (smo_kernel.cpp:176-183); inside the loop the stopping
     // test is evaluated per element, as in the C variant
@@ -1016,7 +1040,7 @@ __global__ __launch_bounds__(64 * W) void nu_smo_solve_kernel(
             int stretch = 4;   // (as in c_smo_solve_kernel)
             do {
                 const int before = n_iter;
-                done = nu_iterate_rounded<E, LDK, TB>(sh, s_ip, s_in, (SvScore *) s_jp, s_step, ws, kws, kd, f, member, local_eps, max_iter, n_iter);
+                done = nu_iterate_rounded<E, LDK, TB>(sh, s_ip, s_in, s_score, ws, kws, kd, f, member, local_eps, max_iter, n_iter);
                 if (done) break;
                 stretch = n_iter - before > stretch ? 4 : stretch < 1024 ? 8 * stretch : stretch;
                 done = nu_iterate<E, W, LDK, TB>(sh, s_f, s_k, s_ip, s_in, s_jp, s_jn, ws, kws, kd, f, member, local_eps, max_iter, n_iter, stretch);
