@@ -108,15 +108,6 @@ __device__ __forceinline__ void publish_words(unsigned slot, uint64_t lanes, int
 __device__ __forceinline__ void publish(SvCand *slot, uint64_t lanes, double m, int at, int flag) {
     publish_words(lds_at(slot), lanes, __double2loint(m), __double2hiint(m), at, flag);
 }
-template <typename S>
-__device__ __forceinline__ void publish(S *slot, uint64_t lanes, float best, float second, int at, int go) {
-    publish_words(lds_at(slot), lanes, __float_as_int(best), __float_as_int(second), at, go);
-}
-template <typename S>
-__device__ __forceinline__ void publish(S *slot, uint64_t lanes, double x, double y) {
-    static_assert(sizeof(S) == 16, "two doubles");
-    asm volatile(SV_EXEC_ON "ds_write2_b64 %1, %2, %3 offset1:1\n\t" SV_EXEC_OFF :: "s"(lanes), "v"(lds_at(slot)), "v"(x), "v"(y) : "memory");
-}
 // The same with the lane's E values of f and of the block row for the step (the row's values in slots of eight bytes).
 // (One asm statement each: nothing else may come between the two writes of exec.)
 // `only`: the lanes that write, each to slots of its own.
@@ -214,29 +205,6 @@ struct __align__(16) SvScore {
     float best, second;
     int at, go;
 };
-// best and second of a row in all its lanes.  Four instructions per step, ordered so that none of the DPP operands is
-// younger than two instructions: no wait states between the steps, so the second-best costs hardly more than the waits would.
-// LANES: of so many lanes that hold different ones.
-template <int LANES = 16>
-__device__ __forceinline__ void row_best_two(float &best, float &second) {
-    static_assert(LANES == 4 || LANES == 8 || LANES == 16, "a quad, half a row, a row");
-    float t;
-#define SV_BEST_STEP(CTRL)                                          \
-    "v_min_f32_dpp %2, %0, %0 " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
-    "v_max_f32_dpp %0, %0, %0 " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
-    "v_max_f32_dpp %1, %1, %1 " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
-    "v_max_f32 %1, %1, %2\n\t"
-    if constexpr (LANES == 4)
-        asm("s_nop 1\n\t" SV_BEST_STEP("quad_perm:[1,0,3,2]") SV_BEST_STEP("quad_perm:[2,3,0,1]") : "+v"(best), "+v"(second), "=&v"(t));
-    else if constexpr (LANES == 8)
-        asm("s_nop 1\n\t" SV_BEST_STEP("quad_perm:[1,0,3,2]") SV_BEST_STEP("quad_perm:[2,3,0,1]") SV_BEST_STEP("row_half_mirror")
-            : "+v"(best), "+v"(second), "=&v"(t));
-    else
-        asm("s_nop 1\n\t" SV_BEST_STEP("quad_perm:[1,0,3,2]") SV_BEST_STEP("quad_perm:[2,3,0,1]") SV_BEST_STEP("row_half_mirror")
-                SV_BEST_STEP("row_mirror")
-            : "+v"(best), "+v"(second), "=&v"(t));
-#undef SV_BEST_STEP
-}
 struct SvScoreStep {
     SvScore score;
     SvStep step;
@@ -248,7 +216,8 @@ struct SvScoreStep {
 // that a comparison wrote is read three instructions later.
 #define SV_DPP_MOV(TO, FROM, CTRL) "v_mov_b32_dpp " TO ", " FROM " " CTRL " row_mask:0xf bank_mask:0xf\n\t"
 #define SV_MIN_STEP(CTRL) SV_DPP_MOV("v148", "v150", CTRL) SV_DPP_MOV("v149", "v151", CTRL) "v_min_f64 v[150:151], v[150:151], v[148:149]\n\t"
-// row_first_min with the candidate as the record that is published (its last word is anything); `has`: the lanes that have the row's smallest.
+// The smallest of a row's E * 16 values: every lane's own smallest and its first element as the record that the lane publishes (its last word is
+// anything); `has`: the lanes whose own is the row's.  (The first four steps of wave_argmin.)
 template <int E>
 __device__ __forceinline__ void row_first_candidate(const double (&x)[E], const int (&at)[E], SvWords &rec, uint64_t &has) {
     uint64_t h0, h1, h2;
@@ -287,6 +256,30 @@ __device__ __forceinline__ void row_first_candidate(const double (&x)[E], const 
             : "v"(x[0]), "v"(x[1]), "v"(at[0]), "v"(at[1])
             : "v148", "v149", "v150", "v151");
     }
+}
+// The same for four elements per thread with `twice`, the lanes whose own smallest occurs more than once.
+__device__ __forceinline__ void row_first_candidate(const double (&x)[4], const int (&at)[4], SvWords &rec, uint64_t &has, uint64_t &twice) {
+    uint64_t h0, h1, h2, h3;
+    asm("v_min_f64 v[144:145], %6, %7\n\t"
+        "v_min_f64 v[148:149], %8, %9\n\t"
+        "v_min_f64 v[144:145], v[144:145], v[148:149]\n\t"
+        "v_cmp_eq_f64_e64 %2, %6, v[144:145]\n\t"
+        "v_cmp_eq_f64_e64 %3, %7, v[144:145]\n\t"
+        "v_cmp_eq_f64_e64 %4, %8, v[144:145]\n\t"
+        SV_DPP_MOV("v148", "v144", "quad_perm:[1,0,3,2]") SV_DPP_MOV("v149", "v145", "quad_perm:[1,0,3,2]")
+        "v_min_f64 v[150:151], v[144:145], v[148:149]\n\t"
+        "v_cndmask_b32_e64 v146, %13, %12, %4\n\t"
+        "v_cndmask_b32_e64 v146, v146, %11, %3\n\t"
+        SV_MIN_STEP("quad_perm:[2,3,0,1]")
+        "v_cndmask_b32_e64 v146, v146, %10, %2\n\t"
+        "v_cmp_eq_f64_e64 %5, %9, v[144:145]\n\t"
+        SV_MIN_STEP("row_half_mirror")
+        "s_nop 1\n\t" SV_MIN_STEP("row_mirror")
+        "v_cmp_eq_f64_e64 %1, v[144:145], v[150:151]"
+        : "=&{v[144:147]}"(rec), "=&s"(has), "=&s"(h0), "=&s"(h1), "=&s"(h2), "=&s"(h3)
+        : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3])
+        : "v148", "v149", "v150", "v151");
+    twice = (h0 & h1) | ((h0 | h1) & h2) | ((h0 | h1 | h2) & h3);
 }
 // Two of them, for the nu variant's sides: each chain fills the other's wait states.
 #define SV_MOVS(CTRL) SV_DPP_MOV("v148", "v150", CTRL) SV_DPP_MOV("v149", "v151", CTRL) SV_DPP_MOV("v156", "v158", CTRL) SV_DPP_MOV("v157", "v159", CTRL)
@@ -358,10 +351,19 @@ __device__ __forceinline__ void row_mins_and_who(double x, double y, double &min
         : "=&v"(min_x), "=&v"(min_y), "=&s"(who_x), "=&s"(who_y) : "v"(x), "v"(s), "v"(y), "v"(t)
         : "v148", "v149", "v150", "v151", "v156", "v157", "v158", "v159");
 }
-// row_min, with the lanes that have it.
+// The smallest of a row's x in all its lanes, and the lanes that have it.  LANES: of so many lanes that hold different ones.
+template <int LANES = 16>
 __device__ __forceinline__ void row_min_and_who(double x, double &value, uint64_t &who) {
     const double t = dpp_f64<TSVM_DPP_XOR1>(x);
-    asm("v_min_f64 v[150:151], %2, %3\n\t"
+    static_assert(LANES == 8 || LANES == 16, "half a row, a row");
+    if constexpr (LANES == 8)
+        asm("v_min_f64 v[150:151], %2, %3\n\t"
+            "s_nop 1\n\t" SV_MIN_STEP("quad_perm:[2,3,0,1]")
+            "s_nop 1\n\t" SV_DPP_MOV("v148", "v150", "row_half_mirror") SV_DPP_MOV("v149", "v151", "row_half_mirror")
+            "v_min_f64 %0, v[150:151], v[148:149]\n\t"
+            "v_cmp_eq_f64_e64 %1, %2, %0"
+            : "=&v"(value), "=s"(who) : "v"(x), "v"(t) : "v148", "v149", "v150", "v151");
+    else asm("v_min_f64 v[150:151], %2, %3\n\t"
         "s_nop 1\n\t" SV_MIN_STEP("quad_perm:[2,3,0,1]")
         "s_nop 1\n\t" SV_MIN_STEP("row_half_mirror")
         "s_nop 1\n\t" SV_DPP_MOV("v148", "v150", "row_mirror") SV_DPP_MOV("v149", "v151", "row_mirror")
@@ -409,7 +411,10 @@ __device__ __forceinline__ void block_first_mins(SvCand *slots_x, SvCand *slots_
     first_y = __builtin_amdgcn_readlane(cy.at, __builtin_ctzll(who_y));
     any = __builtin_amdgcn_ballot_w64(cx.flag != 0) != 0;
 }
-// row_best_two over sixteen lanes, with the lanes that have the best.
+// Best and second of a row in all its lanes, and the lanes that have the best.  Four instructions per step, ordered so that none of the
+// DPP operands is younger than two instructions: no wait states between the steps, so the second-best costs hardly more than the
+// waits would.
+template <int LANES = 16>
 __device__ __forceinline__ void row_best_two_and_who(float mine, float second_in, float &best, float &second, uint64_t &who) {
     float t;
 #define SV_BEST_STEP(CTRL, B, S)                                          \
@@ -417,56 +422,18 @@ __device__ __forceinline__ void row_best_two_and_who(float mine, float second_in
     "v_max_f32_dpp %0, " B ", " B " " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
     "v_max_f32_dpp %1, " S ", " S " " CTRL " row_mask:0xf bank_mask:0xf\n\t" \
     "v_max_f32 %1, %1, %2\n\t"
-    asm("s_nop 1\n\t" SV_BEST_STEP("quad_perm:[1,0,3,2]", "%4", "%5") SV_BEST_STEP("quad_perm:[2,3,0,1]", "%0", "%1")
+    static_assert(LANES == 8 || LANES == 16, "half a row, a row");
+    if constexpr (LANES == 8)
+        asm("s_nop 1\n\t" SV_BEST_STEP("quad_perm:[1,0,3,2]", "%4", "%5") SV_BEST_STEP("quad_perm:[2,3,0,1]", "%0", "%1")
+                SV_BEST_STEP("row_half_mirror", "%0", "%1")
+            "v_cmp_eq_f32_e64 %3, %4, %0"
+            : "=&v"(best), "=&v"(second), "=&v"(t), "=s"(who) : "v"(mine), "v"(second_in));
+    else asm("s_nop 1\n\t" SV_BEST_STEP("quad_perm:[1,0,3,2]", "%4", "%5") SV_BEST_STEP("quad_perm:[2,3,0,1]", "%0", "%1")
             SV_BEST_STEP("row_half_mirror", "%0", "%1") SV_BEST_STEP("row_mirror", "%0", "%1")
         "v_cmp_eq_f32_e64 %3, %4, %0"
         : "=&v"(best), "=&v"(second), "=&v"(t), "=s"(who) : "v"(mine), "v"(second_in));
 #undef SV_BEST_STEP
 }
-// The smallest of a row's x, in all its lanes.
-__device__ __forceinline__ double row_min(double x) {
-    x = fmin_f64(x, dpp_f64<TSVM_DPP_XOR1>(x));
-    x = fmin_f64(x, dpp_f64<TSVM_DPP_XOR2>(x));
-    x = fmin_f64(x, dpp_f64<TSVM_DPP_HALF_MIRROR>(x));
-    return fmin_f64(x, dpp_f64<TSVM_DPP_MIRROR>(x));
-}
-
-// The smallest of a row's E * 16 values; m and at are every lane's own smallest and its first element (as wave_argmin in
-// smo_local.h, whose first four steps these are).
-// TWICE: and `twice` has the lanes whose own smallest occurs more than once.
-template <int E, bool TWICE = false>
-__device__ __forceinline__ double row_first_min(const double (&x)[E], int base, double &m, int &at, uint64_t *twice = nullptr) {
-    m = x[0];
-#pragma unroll
-    for (int e = 1; e < E; ++e) m = fmin_f64(m, x[e]);
-    SV_PIN;
-    uint64_t has[E];
-#pragma unroll
-    for (int e = 0; e < (TWICE ? E : E - 1); ++e) asm volatile("v_cmp_eq_f64_e64 %0, %1, %2" : "=s"(has[e]) : "v"(x[e]), "v"(m));
-    SV_PIN;
-    double r = fmin_f64(m, dpp_f64<TSVM_DPP_XOR1>(m));
-    SV_PIN;
-    at = base + E - 1;
-    if constexpr (E > 2) asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(at) : "v"(at), "v"(base + E - 2), "s"(has[E - 2]));
-    if constexpr (E > 3) asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(at) : "v"(at), "v"(base + E - 3), "s"(has[E - 3]));
-    SV_PIN;
-    r = fmin_f64(r, dpp_f64<TSVM_DPP_XOR2>(r));
-    SV_PIN;
-    if constexpr (E > 1) asm volatile("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(at) : "v"(at), "v"(base), "s"(has[0]));
-    SV_PIN;
-    if constexpr (TWICE) {
-        uint64_t more = 0, one = has[0];
-#pragma unroll
-        for (int e = 1; e < E; ++e) {
-            more |= one & has[e];
-            one |= has[e];
-        }
-        *twice = more;
-    }
-    r = fmin_f64(r, dpp_f64<TSVM_DPP_HALF_MIRROR>(r));
-    return fmin_f64(r, dpp_f64<TSVM_DPP_MIRROR>(r));
-}
-
 // Bounds of what c_smo_iterate_rounded (smo_solve.hip) decides: the least |up|, and from where on an a is too large (as float bits).
 #define SV_UP_LEAST_HI 0x3b600000   // 2^-73
 #define SV_UP_LEAST 0x1p-73

@@ -93,8 +93,7 @@ struct SmallShared {
     double red[4][W];
     int event[2], first_x[2], first_y[2], n_list;
     SvCand ci[4 * W], ci2[W], cj[W], cj2[W];
-    SvScore score[4 * W];
-    SvStep step[4 * W];
+    SvScoreStep score[4 * W];
 };
 
 // sort_f + select_working_set (smo_kernel.cpp:321-332, csmosolver.cpp:123-165, nusmosolver.cpp:48-118): writes k picks to
@@ -446,36 +445,51 @@ __device__ __forceinline__ bool ss_local(SmallShared<E, W> &sh, const SmallMap &
 
 // The C variant's iterations with j2 chosen by b^2/a rounded to float, as long as that decides: c_smo_iterate_rounded of
 // smo_solve.hip, with its proof.  What the working set's order would decide, equal values of f included, is left to ss_local.
-// 963 instances, 1,000 steps: 2.82 -> 2.72 thousand cycles a step; cross-validation of 1203x13 2.31 -> 2.26 ms.
+// 963 instances, 1,000 steps: 2.82 -> 2.72 thousand cycles a step; cross-validation of 1203x13 2.31 -> 2.26 ms.  With that function's
+// chains in single blocks, bits by masks and writes in the next step's waits 1.67 -> 1.61.
 template <int E, int W, typename TB>
 __device__ __forceinline__ bool ss_rounded(SmallShared<E, W> &sh, const SmallMap &map, SS_GLOBAL(TB) *K, int64_t ld, int col, const double (&kd)[E],
                                            double (&f)[E], unsigned &member, double Cp, double Cn, double local_eps, int max_iter, int &n_iter) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     constexpr int R = 4 * W;   // rows of sixteen lanes
+    const unsigned my_i = lds_at(sh.ci + (tid >> 4)), my_j = lds_at(sh.score + (tid >> 4));
+    unsigned my_z = lds_at(&sh.z[wave][0]);
+    asm("" : "+v"(my_z));
+    int own[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) own[e] = tid * E + e;
     uint64_t go;
+    // what a step leaves to the waits of the next: I_low's bits, and the two elements' new z
+    unsigned bit_i = 0, bit_j = 0, low_i = 0, low_j = 0, z_at_i = my_z, z_at_j = my_z;
+    double nz_i = 0, nz_j = 0;
+    int pending = 0;
     for (;;) {
         double fu[E];
 #pragma unroll
         for (int e = 0; e < E; ++e) fu[e] = keep_or_none<0>(member << (31 - 2 * e), f[e]);
-        double m;
-        int at;
-        uint64_t twice;
-        const double r = row_first_min<E, true>(fu, tid * E, m, at, &twice);
-        const uint64_t mine_is = __builtin_amdgcn_ballot_w64(m == r), has = mine_is | 0x8000800080008000ull;
-        const uint64_t first = has & ~(has - 0x0001000100010001ull);
-        const uint64_t equal = mine_is & (twice | ~first);   // a row that has one has its smallest more than once
-        const int tie = (int) ((unsigned) (equal >> (lane & 48)) & 0xffffu);
-        publish(sh.ci + (tid >> 4), first, m, at, tie);
+        SvWords cand;
+        uint64_t mine_is, twice;
+        row_first_candidate(fu, own, cand, mine_is, twice);
+        const uint64_t first = lowest_of_rows(mine_is), equal = mine_is & (twice | ~first);   // a row that has one has its smallest more than once
+        cand[3] = (int) ((unsigned) (equal >> (lane & 48)) & 0xffffu);
+        publish_words(my_i, first, cand);
         lds_barrier();
         const SvCand c = sh.ci[lane & (R - 1)];
-        const double up = row_min(c.v);
-        const uint64_t has_up = __builtin_amdgcn_ballot_w64(c.v == up), up_rows = has_up & ((1ull << R) - 1);
+        write_by_lane0(pending, z_at_i, nz_i, z_at_j, nz_j);
+        member = put_bits(put_bits(member, bit_i, low_i), bit_j, low_j);
+        double up;
+        uint64_t has_up;
+        row_min_and_who<R>(c.v, up, has_up);
+        const uint64_t up_rows = has_up & ((1ull << R) - 1);
         const uint64_t ties = (up_rows & (up_rows - 1)) | (up_rows & __builtin_amdgcn_ballot_w64(c.flag != 0));
-        const int i = __builtin_amdgcn_readlane(c.at, __builtin_ctzll(has_up)) & (64 * E * W - 1);
+        const int i = __builtin_amdgcn_readlane(c.at, __builtin_ctzll(has_up));
         TB kI[E];
         ss_load<E, TB>(K + (unsigned) map.row(i) * (unsigned) ld + col, kI);
         SV_PIN_MEMORY;
-        const double kd_i = sh.kd[i], z_i = sh.z[wave][i];
+        z_at_i = my_z + 8u * (unsigned) i;
+        const double kd_i = sh.kd[i], z_i = lds_f64(z_at_i);
+        unsigned up_bit_i = own_bit<E, 2>(tid, i);
+        asm("" : "+v"(up_bit_i));
         const SvBound bound_i = map.bound(i, Cp, Cn);
         double part[E], b[E], b_max = -__builtin_inf();
         float b32[E];
@@ -486,10 +500,10 @@ __device__ __forceinline__ bool ss_rounded(SmallShared<E, W> &sh, const SmallMap
             b_max = fmax_f64(b_max, b[e]);
             b32[e] = __builtin_fmaxf((float) b[e], 0.0f);
         }
-        const int violates = __builtin_amdgcn_ballot_w64(!(b_max < local_eps)) != 0;
+        const int violates = (__builtin_amdgcn_ballot_w64(!(b_max < local_eps)) != 0) & (n_iter <= max_iter);   // (the way out is one test)
         double up_i = bound_i.hi - z_i;
         asm("" : "+v"(up_i));
-        int a_max = (__double2hiint(up) & 0x7fffffff) < SV_UP_LEAST_HI || ties != 0 ? 0x7f800000 : 0;   // (as the bits of a float)
+        int a_max = __builtin_fabs(up) < SV_UP_LEAST || ties != 0 ? 0x7f800000 : 0;   // (as the bits of a float)
         asm("" : "+v"(a_max));
         SV_PIN;
         double aIJ[E];
@@ -501,60 +515,62 @@ __device__ __forceinline__ bool ss_rounded(SmallShared<E, W> &sh, const SmallMap
             a_max = __float_as_int(a32) > a_max ? __float_as_int(a32) : a_max;
             q[e] = __builtin_fmaxf(b32[e] * (b32[e] * __builtin_amdgcn_rcpf(a32)), 0x1p-80f);
         }
-        float best = q[0], second = 0x1p-80f;
+        float mine = q[0], second = 0x1p-80f;
 #pragma unroll
         for (int e = 1; e < E; ++e) {
-            second = __builtin_fmaxf(second, __builtin_fminf(best, q[e]));
-            best = __builtin_fmaxf(best, q[e]);
+            second = __builtin_fmaxf(second, __builtin_fminf(mine, q[e]));
+            mine = __builtin_fmaxf(mine, q[e]);
         }
-        at = tid * E + E - 1;
+        int at = own[E - 1];
         double b_at = b[E - 1], a_at = aIJ[E - 1];
 #pragma unroll
         for (int e = E - 2; e >= 0; --e) {
-            const bool is = q[e] == best;
-            at = is ? tid * E + e : at;
+            const bool is = q[e] == mine;
+            at = is ? own[e] : at;
             b_at = is ? b[e] : b_at;
             a_at = is ? aIJ[e] : a_at;
         }
         second = a_max < SV_A_BITS ? second : __builtin_inff();
-        const float mine = best;
-        row_best_two(best, second);
-        const uint64_t who = __builtin_amdgcn_ballot_w64(mine == best);   // (several only if nothing will be decided)
-        publish(sh.score + (tid >> 4), who, best, second, at, violates);
-        publish(sh.step + (tid >> 4), who, b_at, a_at);
+        float best, next;
+        uint64_t who;   // (several only if nothing will be decided)
+        row_best_two_and_who(mine, second, best, next, who);
+        publish_score(my_j, who, best, next, at, violates, b_at, a_at);
         lds_barrier();
-        const SvScore s = sh.score[lane & (R - 1)];
-        const SvStep step = sh.step[lane & (R - 1)];
-        best = s.best;
-        second = s.second;
-        row_best_two<R>(best, second);
-        const int row = __builtin_ctzll(__builtin_amdgcn_ballot_w64(s.best == best));
-        const int j2 = __builtin_amdgcn_readlane(s.at, row) & (64 * E * W - 1);
+        const SvScoreStep s = sh.score[lane & (R - 1)];
+        uint64_t won;
+        row_best_two_and_who<R>(s.score.best, s.score.second, best, next, won);
+        const int row = __builtin_ctzll(won);
+        const int j2 = __builtin_amdgcn_readlane(s.score.at, row);
         TB kJ[E];
         ss_load<E, TB>(K + (unsigned) map.row(j2) * (unsigned) ld + col, kJ);
         SV_PIN_MEMORY;
-        const double z_j = sh.z[wave][j2];
+        z_at_j = my_z + 8u * (unsigned) j2;
+        const double z_j = lds_f64(z_at_j);
         const SvBound bound_j = map.bound(j2, Cp, Cn);
         SV_PIN;
-        const double steps = step.b / step.a;   // (every row's)
+        const double steps = s.step.b / s.step.a;   // (every row's)
         const double q2 = readlane_f64(steps, row);
+        const unsigned up_bit_j = own_bit<E, 2>(tid, j2);
+        go = __builtin_amdgcn_ballot_w64(s.score.go != 0);
+        const uint64_t sure = __builtin_amdgcn_ballot_w64(next < best * (1.0f - 0x1p-19f)) & __builtin_amdgcn_ballot_w64(best < 0x1p80f);
+        if ((go & sure) == 0) break;
         SV_PIN;
-        go = __builtin_amdgcn_ballot_w64(s.go != 0);
-        const uint64_t sure = __builtin_amdgcn_ballot_w64(second < best * (1.0f - 0x1p-19f)) & __builtin_amdgcn_ballot_w64(best < 0x1p80f);
-        const uint64_t on = n_iter > max_iter ? 0 : go & sure;
-        if (on == 0) break;
-        const double l = fmin_f64(up_i, fmin_f64(z_j - bound_j.lo, q2));
-        const double nz_i = z_i + l, nz_j = z_j - l;
-        auto bits = [&](double z, const SvBound &bound) { return (z < bound.hi ? 1u : 0u) | (z > bound.lo ? 2u : 0u); };
-        member = set_member_bits<E, 2>(member, tid, i, bits(nz_i, bound_i));
-        member = set_member_bits<E, 2>(member, tid, j2, bits(nz_j, bound_j));
-        write_by_lane0(1, &sh.z[wave][i], nz_i, &sh.z[wave][j2], nz_j);
+        const double l = fmin_f64(fmin_f64(up_i, z_j - bound_j.lo), q2);
+        nz_i = z_i + l;
+        nz_j = z_j - l;
+        const unsigned up_i_on = same_in_all_lanes(nz_i < bound_i.hi), up_j_on = same_in_all_lanes(nz_j < bound_j.hi);
+        low_i = same_in_all_lanes(nz_i > bound_i.lo);
+        low_j = same_in_all_lanes(nz_j > bound_j.lo);
+        bit_i = up_bit_i << 1;
+        bit_j = up_bit_j << 1;
+        member = put_bits(put_bits(member, up_bit_i, up_i_on), up_bit_j, up_j_on);
+        pending = 1;
         SV_PIN;
 #pragma unroll
         for (int e = 0; e < E; ++e) f[e] = __builtin_fma(-l, (double) kJ[e] - (double) kI[e], f[e]);
         ++n_iter;
     }
-    return go == 0 || n_iter > max_iter;
+    return go == 0;
 }
 
 // f[j] -= sum over the n_list listed rows (coefficients sh.f, rows in sh.k) in order (smo_kernel.cpp:300-319)
