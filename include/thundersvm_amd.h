@@ -420,6 +420,15 @@ int tsvm_update_f_select_report(double *f, const double *alpha_diff, int ws_size
                                 const int *marked, int n_marked, int *out, int n_select, int nu, void *workspace, int *out_folded,
                                 int *host_ids, int word_at, int word, tsvm_stream stream);
 
+/* The same with one pass over the instances in all, where the last selection on this workspace is a guide to where the candidates end (its
+ * result is the same whatever the guide is worth).  host_ids may be NULL: no report.  *missed, memory that the device can write
+ * and the host can read, becomes 1 when the guide has not decided the selection, which has then taken several times as long:
+ * f has moved too far, or too many instances share a value; the caller is better off with the calls above for a while. */
+int tsvm_update_f_select_guided(double *f, const double *alpha_diff, int ws_size, const void *k_rows, int row_type, const int *slots,
+                                int64_t ld, int64_t n_cols, int repeat, const int *y, const double *alpha, double Cp, double Cn,
+                                const int *marked, int n_marked, int *out, int n_select, int nu, void *workspace, int *out_folded,
+                                int *host_ids, int word_at, int word, int *missed, tsvm_stream stream);
+
 /* ---------------------------------------------------------------------------------------------
  * predict (kernelmatrix_kernel.cpp:110-147)
  * ------------------------------------------------------------------------------------------- */

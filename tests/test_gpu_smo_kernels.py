@@ -736,6 +736,65 @@ def test_update_f_with_the_next_selection(n_cols, repeat, ws, ld_pad, tie_mode, 
         a_d = G.dev(alpha)
 
 
+@pytest.mark.parametrize("nu", [0, 1])
+@pytest.mark.parametrize("n_cols,repeat,row_type", [(2, 1, capi.ROW_F32), (700, 1, capi.ROW_F64), (3200, 1, capi.ROW_F32), (30000, 2, capi.ROW_F32),
+                                                    (70001, 1, capi.ROW_F64), (262144, 1, capi.ROW_F32)])
+def test_guided_selections(n_cols, repeat, row_type, nu):
+    """Selections that follow one another with the last one as a guide: f that moves a little, by far more than the guide reaches (either
+    way, and in scale), ends in ties, has infinite values, and sides with fewer candidates than are asked for; and selections by
+    digits in between, which find the workspace as they want it.  The ids are the oracle's whatever the guide was worth."""
+    n = n_cols * repeat
+    rng = np.random.default_rng(n + nu)
+    sel = min(1024, 1 << (n.bit_length() - 1))
+    q = max(sel // 2, 1)
+    ld = n_cols
+    k_d = G.dev(np.zeros((1, ld), dtype=np.float32 if row_type == capi.ROW_F32 else np.float64))
+    ad_d = G.dev(np.zeros(1))
+    y = np.where(rng.random(n) < 0.5, 1, -1).astype(np.int32)
+    y[0] = 1
+    C, f = 1.0, rng.standard_normal(n)
+    wsp = torch.empty(capi.kernel_lib().tsvm_select_workspace(n), dtype=torch.uint8, device="cuda")
+    wsp.random_(0, 256)
+    y_d = G.dev(y)
+    prev = None
+    missed_d = torch.zeros(1, dtype=torch.int32, device="cuda")
+    near = rng.standard_normal(n)
+    steps = [("digits", f), ("guided", f), ("guided", f + 0.01 * near), ("guided", f + 1e4), ("digits", f), ("guided", 1e-6 * f), ("guided", 1e6 * f),
+             ("guided", np.round(f)), ("guided", f), ("guided", np.full(n, -1.0)), ("guided", f), ("guided", np.where(near > 1.5, np.inf, f)),
+             ("guided", np.where(near > 1.5, -np.inf, f)), ("digits", np.zeros(n)), ("guided", f), ("few", f), ("guided", f - 0.02 * near)]
+    for at, (how, fn) in enumerate(steps):
+        alpha = rng.choice([0.0, 0.5 * C, C], size=n)
+        if how == "few":   # (I_up has some seven instances)
+            alpha = np.where(y > 0, C, 0.0)
+            alpha[rng.integers(0, n, size=7)] = 0.5 * C
+        fn = np.ascontiguousarray(fn, dtype=np.float64)
+        marked = np.zeros(0, dtype=np.int32) if prev is None else np.ascontiguousarray(prev[prev >= 0][-q:])
+        n_select = sel if prev is None else q
+        want = O.select_working_set(fn, y, alpha, C, C, marked, n_select, nu=bool(nu))
+        f_d, a_d, m_d = G.dev(fn), G.dev(alpha), G.dev(marked if len(marked) else np.zeros(1, dtype=np.int32))
+        out_d = torch.full((n_select,), -7, dtype=torch.int32, device="cuda")
+        fold_d = torch.full((n_select,), -7, dtype=torch.int32, device="cuda")
+        missed_d.zero_()
+        m_ptr = G.ptr(m_d) if len(marked) else None
+        args = (G.ptr(f_d), G.ptr(ad_d), 1, G.ptr(k_d), row_type, None, ld, n_cols, repeat, G.ptr(y_d), G.ptr(a_d), C, C, m_ptr, len(marked),
+                G.ptr(out_d), n_select, nu, G.ptr(wsp), G.ptr(fold_d) if repeat > 1 else None)
+        if prev is None:
+            capi.call("tsvm_select_working_set", G.ptr(f_d), G.ptr(y_d), G.ptr(a_d), n, C, C, None, 0, G.ptr(out_d), n_select, nu, G.ptr(wsp), G.stream())
+        elif how == "digits":
+            capi.call("tsvm_update_f_select", *args, G.stream())
+        else:
+            capi.call("tsvm_update_f_select_guided", *args, None, 0, 0, G.ptr(missed_d), G.stream())
+        got = G.host(out_d)
+        assert np.array_equal(got, want), "step %d (%s): first mismatch at %s" % (at, how, np.flatnonzero(got != want)[:5])
+        if repeat > 1 and prev is not None:
+            assert np.array_equal(G.host(fold_d), np.where(want >= 0, want % n_cols, -1))
+        if at == 2 or n <= 1024:
+            assert G.host(missed_d)[0] == 0
+        if at == 9 and n > 8192:   # (thousands of equal values)
+            assert G.host(missed_d)[0] == 1
+        prev = got
+
+
 @pytest.mark.parametrize("row_type,line", [(capi.ROW_F64, 32768), (capi.ROW_F32, 65536)])
 @pytest.mark.parametrize("beyond,ld_pad", [(0, 0), (0, 1), (1, 1), (1, 2)])
 def test_update_f_at_the_line_between_its_kernels(row_type, line, beyond, ld_pad):

@@ -79,6 +79,7 @@ SIGNATURES = {
     "tsvm_select_working_set_report": (_int, [_p, _p, _p, _i64, _dbl, _dbl, _p, _int, _p, _int, _int, _p, _int, _int, _p, _p, _int, _int, _p]),
     "tsvm_update_f_select": (_int, [_p, _p, _int, _p, _int, _p, _i64, _i64, _int, _p, _p, _dbl, _dbl, _p, _int, _p, _int, _int, _p, _p, _p]),
     "tsvm_update_f_select_report": (_int, [_p, _p, _int, _p, _int, _p, _i64, _i64, _int, _p, _p, _dbl, _dbl, _p, _int, _p, _int, _int, _p, _p, _p, _int, _int, _p]),
+    "tsvm_update_f_select_guided": (_int, [_p, _p, _int, _p, _int, _p, _i64, _i64, _int, _p, _p, _dbl, _dbl, _p, _int, _p, _int, _int, _p, _p, _p, _int, _int, _p, _p]),
     "tsvm_sum_kernel_values": (_int, [_p, _int, _p, _p, _p, _p, _int, _i64, _p, _int, _i64, _p]),
     "tsvm_predict_votes_max_classes": (_int, []),
     "tsvm_predict_votes": (_int, [_p, _i64, _int, _p, _p]),

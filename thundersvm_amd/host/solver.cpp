@@ -230,6 +230,26 @@ struct SolveTask::Impl {
     volatile int *h_rows_done = nullptr;
     int *d_rows_done = nullptr;
     int rows_seq = 0;   // the number that h_rows_done takes with the rows enqueued last
+    // Selections are guided by the one before (tsvm_update_f_select_guided), but for the first (the first solve moves f by more than a
+    // guide reaches, from values that are mostly equal); when one has not been decided that way, which costs as much as ten others save, the
+    // next few go by digits, twice as many each time until 32 in a row have been decided.
+    volatile int *h_missed = nullptr;
+    int *d_missed = nullptr;
+    int unguided = 1, unguided_next = 2, decided_in_row = 0;
+    bool next_is_guided() {
+        if (*h_missed) {
+            *h_missed = 0;
+            unguided = unguided_next;
+            unguided_next = std::min(2 * unguided_next, 32);
+            decided_in_row = 0;
+        }
+        if (unguided > 0) {
+            --unguided;
+            return false;
+        }
+        if (++decided_in_row == 32) unguided_next = 2;
+        return true;
+    }
     bool on_one_stream = false;   // block and solver are on `sa`
     int last_rows_computed = 0;   // (this iteration's will probably be as many)
     long long masked_key = 0;
@@ -450,6 +470,9 @@ struct SolveTask::Impl {
         h_rows_done = h_cache_info + 2;
         d_rows_done = d_cache_info + 2;
         *h_rows_done = 0;
+        h_missed = h_cache_info + 3;
+        d_missed = d_cache_info + 3;
+        *h_missed = 0;
         h_ids[ws_size] = 0;
         h_diff[0] = h_diff[1] = h_diff[2] = 0;
         // what the device starts from: the three vectors in one copy, the rest by one kernel
@@ -486,11 +509,11 @@ struct SolveTask::Impl {
         // straight from update_f into it; if the diff then says stop, that selection was simply not needed.
         // (Not when tracing, which reads the working set back after each iteration, nor when profiling.)
         select_ahead = !solver.trace && !solver.profile;
-        // With stacked copies (SVR) the first pass rides along from 16,385 columns on (epsilon-SVR on 3,000 and 12,000 rows 7.55 -> 7.60 and
-        // 27.28 -> 27.38 ms with it, on 40,000 92.4 -> 91.5, on 100,000 218.9 -> 216.2, on 120,000 282.0 -> 279.5); from 262,144 columns
+        // With stacked copies (SVR) too: a guided selection has no other pass (epsilon-SVR on 3,000 and 12,000 rows 6.70 -> 6.51 and 20.6 -> 19.9 ms
+        // with it; by digits, which make a second and a third all the same, 7.55 -> 7.60 and 27.28 -> 27.38).  From 262,144 columns
         // on a thread has the instances of all copies of its columns to classify after its rows have streamed by, each behind
         // memory reads that wait on a saturated HBM: slower than the separate pass.
-        fuse_select = q > 0 && (rep == 1 || (rep <= 4 && n_u > 16384 && n_u < 262144));
+        fuse_select = q > 0 && (rep == 1 || (rep <= 4 && n_u < 262144));
         // The solver reads the ws x ws block of the kernel matrix.  With few features the block is cheap to
         // compute on its own, without the stored rows, so it and the solver can be enqueued before the host
         // does the cache bookkeeping.  With many features that small launch (64 workgroups walking the whole
@@ -819,6 +842,14 @@ struct SolveTask::Impl {
             // the next selection's first pass over the instances rides on update_f's last one
             advance_window();
             int *const kept = d_ws.data() + sel_off, *const folded = rep > 1 ? d_ws_folded.data() + sel_off + q : nullptr;
+            if (next_is_guided()) {
+                const bool report = ids_to_host();
+                abi_check(tsvm_update_f_select_guided(d_f, d_alpha_diff.data(), ws_size, k_rows, row_type, slots, ld, n_u, rep, d_y, d_alpha, Cp, Cn, kept, q,
+                                                      kept + q, q, nu, d_sel_ws.data(), folded, report ? d_ids_host : nullptr, ws_size,
+                                                      report ? ++ids_seq : 0, d_missed, sa));
+                select_enqueued = true;
+                return;
+            }
             if (ids_to_host())
                 abi_check(tsvm_update_f_select_report(d_f, d_alpha_diff.data(), ws_size, k_rows, row_type, slots, ld, n_u, rep, d_y, d_alpha,
                                                       Cp, Cn, kept, q, kept + q, q, nu, d_sel_ws.data(), folded, d_ids_host, ws_size,
