@@ -110,8 +110,8 @@ __device__ __forceinline__ void publish(SvCand *slot, uint64_t lanes, double m, 
 }
 // The same with the lane's E values of f and of the block row for the step (the row's values in slots of eight bytes).
 // (One asm statement each: nothing else may come between the two writes of exec.)
-// `only`: the lanes that write, each to slots of its own.
-template <int E, typename TB>
+// `only`: the lanes that write, each to slots of its own.  S: doubles from one slot for f to the next.
+template <int E, typename TB, int S = 1>
 __device__ __forceinline__ void publish_row(double *f_slot, double *k_slot, uint64_t only, const double (&f)[E], const TB (&k)[E]) {
     const unsigned fa = lds_at(f_slot), ka = lds_at(k_slot);
     static_assert(E == 1 || E == 2 || E == 4, "elements per thread");
@@ -122,19 +122,19 @@ __device__ __forceinline__ void publish_row(double *f_slot, double *k_slot, uint
         asm volatile(SV_EXEC_ON "ds_write_b64 %1, %3\n\tds_write_b64 %2, %4\n\t" SV_EXEC_OFF
                      :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(k[0]) : "memory");
     else if constexpr (E == 2 && sizeof(TB) == 4)
-        asm volatile(SV_EXEC_ON "ds_write2_b64 %1, %3, %4 offset1:1\n\tds_write2_b32 %2, %5, %6 offset1:2\n\t" SV_EXEC_OFF
-                     :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(f[1]), "v"(k[0]), "v"(k[1]) : "memory");
+        asm volatile(SV_EXEC_ON "ds_write2_b64 %1, %3, %4 offset1:%7\n\tds_write2_b32 %2, %5, %6 offset1:2\n\t" SV_EXEC_OFF
+                     :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(f[1]), "v"(k[0]), "v"(k[1]), "n"(S) : "memory");
     else if constexpr (E == 2)
-        asm volatile(SV_EXEC_ON "ds_write2_b64 %1, %3, %4 offset1:1\n\tds_write2_b64 %2, %5, %6 offset1:1\n\t" SV_EXEC_OFF
-                     :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(f[1]), "v"(k[0]), "v"(k[1]) : "memory");
+        asm volatile(SV_EXEC_ON "ds_write2_b64 %1, %3, %4 offset1:%7\n\tds_write2_b64 %2, %5, %6 offset1:1\n\t" SV_EXEC_OFF
+                     :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(f[1]), "v"(k[0]), "v"(k[1]), "n"(S) : "memory");
     else if constexpr (sizeof(TB) == 4)
-        asm volatile(SV_EXEC_ON "ds_write2_b64 %1, %3, %4 offset1:1\n\tds_write2_b64 %1, %5, %6 offset0:2 offset1:3\n\t"
+        asm volatile(SV_EXEC_ON "ds_write2_b64 %1, %3, %4 offset1:%11\n\tds_write2_b64 %1, %5, %6 offset0:%12 offset1:%13\n\t"
                      "ds_write2_b32 %2, %7, %8 offset1:2\n\tds_write2_b32 %2, %9, %10 offset0:4 offset1:6\n\t" SV_EXEC_OFF
-                     :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "v"(k[0]), "v"(k[1]), "v"(k[2]), "v"(k[3]) : "memory");
+                     :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "v"(k[0]), "v"(k[1]), "v"(k[2]), "v"(k[3]), "n"(S), "n"(2 * S), "n"(3 * S) : "memory");
     else
-        asm volatile(SV_EXEC_ON "ds_write2_b64 %1, %3, %4 offset1:1\n\tds_write2_b64 %1, %5, %6 offset0:2 offset1:3\n\t"
+        asm volatile(SV_EXEC_ON "ds_write2_b64 %1, %3, %4 offset1:%11\n\tds_write2_b64 %1, %5, %6 offset0:%12 offset1:%13\n\t"
                      "ds_write2_b64 %2, %7, %8 offset1:1\n\tds_write2_b64 %2, %9, %10 offset0:2 offset1:3\n\t" SV_EXEC_OFF
-                     :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "v"(k[0]), "v"(k[1]), "v"(k[2]), "v"(k[3]) : "memory");
+                     :: "s"(only), "v"(fa), "v"(ka), "v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "v"(k[0]), "v"(k[1]), "v"(k[2]), "v"(k[3]), "n"(S), "n"(2 * S), "n"(3 * S) : "memory");
 }
 // The same for a record that is already a run of four registers, and for a score with its step.
 typedef int SvWords __attribute__((ext_vector_type(4)));

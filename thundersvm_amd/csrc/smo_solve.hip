@@ -310,9 +310,11 @@ __device__ __forceinline__ bool solver_begins(int *gate, int epoch, int target_x
 
 // What the solvers keep in LDS per element of the working set (inactive elements: both bounds zero, so neither in I_up nor in
 // I_low).  Bounds and diagonal are read by one address.
+// (A workgroup that only passes by, of another lane's launch, has to find room beside a solver: at most half of the CU's 160 KB.  With
+// 82 KB in place of 73 every launch waited for the others' solvers, and seven classes of 92,000 rows took 20 % longer.)
 struct __align__(32) SvElem {
     SvBound bound;
-    double kd, unused;
+    double kd, f;             // f: c_smo_iterate's, at the wavefronts' candidates for j2 (the others are not written)
 };
 template <int N, int W>
 struct SvShared {
@@ -325,7 +327,7 @@ template <int N, int W>
 struct SvState {
     SvElem elem[N];
     double z[W][N];           // every wavefront keeps a copy of its own, which needs no barrier
-    double f[N], k[N];        // f and row i at the elements of the wavefronts' candidates for j2 (the others are not written)
+    double k[N];              // row i at the elements of the wavefronts' candidates for j2 (as f)
 };
 
 // The iterations of c_smo_solve.  Four wavefronts compare by rows of sixteen lanes (block_first_min), as c_smo_iterate_rounded does: the same
@@ -397,16 +399,16 @@ __device__ __forceinline__ bool c_smo_iterate(SvState<E * 64 * W, W> &sh, SvCand
             qs[e] = __hiloint2double(b_low[e] > 0.0 ? __double2hiint(q) : SV_NONE_HI, __double2loint(q));
         }
         if constexpr (W == 4) {
-            block_first_min<E>(s_j, qs, own, go, [&](uint64_t lanes) { publish_row<E, TB>(sh.f + tid * E, sh.k + tid * E, lanes, f, kI); }, min_t, j2, go);
+            block_first_min<E>(s_j, qs, own, go, [&](uint64_t lanes) { publish_row<E, TB, 4>(&sh.elem[tid * E].f, sh.k + tid * E, lanes, f, kI); }, min_t, j2, go);
         } else {
             const int win_j = wave_first_argmin<E>(qs, tid * E, min_t, m, at);
-            publish_row<E, TB>(sh.f + tid * E, sh.k + tid * E, 1ull << win_j, f, kI);
+            publish_row<E, TB, 4>(&sh.elem[tid * E].f, sh.k + tid * E, 1ull << win_j, f, kI);
             j2 = __builtin_amdgcn_readlane(at, win_j);
         }
         if (NONE && is_none(min_t)) {
             j2 = 0;
             __syncthreads();
-            if (tid == 0) { sh.f[0] = f[0]; *(TB *) sh.k = kI[0]; }
+            if (tid == 0) { sh.elem[0].f = f[0]; *(TB *) sh.k = kI[0]; }
             __syncthreads();
         }
         if constexpr (W != 4) j2 = j2 < ws ? j2 : ws - 1;
@@ -414,7 +416,7 @@ __device__ __forceinline__ bool c_smo_iterate(SvState<E * 64 * W, W> &sh, SvCand
         load_row(j2, kJ);
         SV_PIN_MEMORY;
         const SvBound bound_j = sh.elem[j2].bound;
-        const double kd_j = sh.elem[j2].kd, z_j = sh.z[wave][j2], f_j = sh.f[j2];
+        const double kd_j = sh.elem[j2].kd, z_j = sh.z[wave][j2], f_j = sh.elem[j2].f;
         const double kIj = (double) *(const TB *) (sh.k + j2);
         SV_PIN;   // the row is on its way while the step is computed
         // two-variable step (smo_kernel.cpp:92-103; the last round computes one that is not taken)
@@ -601,6 +603,7 @@ __global__ __launch_bounds__(64 * W) void c_smo_solve_kernel(
     __shared__ double s_red[2][W];
     __shared__ SvCand s_i[4 * W], s_j[4 * W];
     __shared__ SvScoreStep s_score[4 * W];
+    static_assert(sizeof(sh) + sizeof(s_red) + sizeof(s_i) + sizeof(s_j) + sizeof(s_score) <= 80 * 1024, "two workgroups on a CU");
 
     // This workgroup is a chain of dependent operations; when a chip-wide kernel runs next to it on
     // another stream its wavefronts must not wait behind that kernel's for issue slots.
