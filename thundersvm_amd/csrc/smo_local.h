@@ -167,15 +167,6 @@ __device__ __forceinline__ double block_max(const double *s_v) {
     return v;
 }
 
-// Replaces the WIDTH membership bits of element t (the same in all threads) in the bit field of the thread that owns it.
-template <int E, int WIDTH>
-__device__ __forceinline__ unsigned set_member_bits(unsigned m, int tid, int t, unsigned bits) {
-    const int sh = (t & (E - 1)) * WIDTH;
-    const unsigned field = ((1u << WIDTH) - 1u) << sh;
-    const unsigned changed = (m & ~field) | (bits << sh);
-    return tid == (int) ((unsigned) t / E) ? changed : m;
-}
-
 // Membership bits in three instructions a change.  own_bit: element t's first bit (of EACH) in the thread that owns it; in another
 // one it is a bit beyond the elements', which nobody reads.  A decision that all lanes have come to alike is a mask of
 // ones or zeros in a scalar register.

@@ -427,12 +427,12 @@ __device__ __forceinline__ bool ss_local(SmallShared<E, W> &sh, const SmallMap &
         const double q2 = (-up_value + f_j) / __builtin_fma(-2.0, (double) k_ij, kd_i2 + kd_j);
         const double l = fmin_f64(bound_i.hi - z_i, fmin_f64(z_j - bound_j.lo, q2));
         const double nz_i = z_i + l, nz_j = (j2 == i ? nz_i : z_j) - l;
-        auto bits = [&](double z, const SvBound &bound, int s) {
-            const unsigned u = z < bound.hi ? 1u : 0u, w = z > bound.lo ? (1u << NP) : 0u;
-            return (u | w) << (NU && s >= map.n0p ? 1 : 0);
-        };
-        member = set_member_bits<E, 2 * NP>(member, tid, i, bits(nz_i, bound_i, i));
-        member = set_member_bits<E, 2 * NP>(member, tid, j2, bits(nz_j, bound_j, j2));
+        // (150x4 0.437 -> 0.417 ms a call, nu-SVC of 600 rows 1.41 -> 1.37, against a shifted field, a comparison and a selection for each)
+        const unsigned up_bit_i = own_bit<E, 2 * NP>(tid, i) << (NU && i >= map.n0p ? 1 : 0), up_bit_j = own_bit<E, 2 * NP>(tid, j2) << (NU && j2 >= map.n0p ? 1 : 0);
+        const unsigned up_i_on = same_in_all_lanes(nz_i < bound_i.hi), low_i_on = same_in_all_lanes(nz_i > bound_i.lo);
+        const unsigned up_j_on = same_in_all_lanes(nz_j < bound_j.hi), low_j_on = same_in_all_lanes(nz_j > bound_j.lo);
+        member = put_bits(put_bits(member, up_bit_i, up_i_on), up_bit_i << NP, low_i_on);
+        member = put_bits(put_bits(member, up_bit_j, up_j_on), up_bit_j << NP, low_j_on);
         write_by_lane0(go_on, &sh.z[wave][i], nz_i, &sh.z[wave][j2], nz_j);
         SV_PIN;
 #pragma unroll
