@@ -20,7 +20,8 @@
 // exit test folded into the loop's branch (the last round computes a step that is not taken); and everything that does
 // not need the row on its way pinned in front of the first instruction that does.
 // Measured on a call of 483 iterations with ws = 1024: 1.37 us per iteration before that, 1.08 with it (2,590 cycles);
-// 0.97 with the scores ranked in float where that decides (c_smo_iterate_rounded), 0.87 since its chains are single blocks.
+// 0.97 with the scores ranked in float where that decides (c_smo_iterate_rounded); a tenth less since its chains are single blocks
+// (epsilon-SVR 40000x90, launches' starts and ends included: 1.08 -> 0.98 a step).
 //
 // Reductions are lexicographic (value, element index) minima, so ties go to the lowest
 // index exactly as the reference's serial loops resolve them, and all arithmetic is the reference's
