@@ -255,4 +255,10 @@ int tsvm_selftest_chip_split(int features, int ws, long long n, long long m_befo
     return (beside ? 1 : 0) | (ChipSplit::warm_behind_rows(beside, ChipSplit::rows_seconds(features, m_now, n)) ? 2 : 0);
 }
 
+// Whether an iteration's rows go ahead of the block and the solver, when the previous one computed m_before rows of n values.
+int tsvm_selftest_rows_ahead(int dense, int features, int ws, long long n, long long m_before) {
+    using tsvm::ChipSplit;
+    return ChipSplit::rows_ahead(dense != 0, features, ws, ChipSplit::rows_seconds(features, m_before, n));
+}
+
 }  // extern "C"

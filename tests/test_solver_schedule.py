@@ -17,3 +17,14 @@ BESIDE, WARM = 1, 2
 ])
 def test_chip_split(features, n, before, now, want):
     assert selftest_lib.lib().tsvm_selftest_chip_split(features, 1024, n, before, now) == want
+
+
+@pytest.mark.parametrize("dense,features,n,before,want", [
+    (1, 784, 100000, 512, True),
+    (1, 784, 20000, 512, False),
+    (0, 20958, 18000, 512, False),
+    (0, 20958, 60000, 512, False),            # sparse rows take microseconds where the dense price says milliseconds
+    (0, 784, 100000, 512, False),
+])
+def test_rows_ahead(dense, features, n, before, want):
+    assert selftest_lib.lib().tsvm_selftest_rows_ahead(dense, features, 1024, n, before) == want

@@ -770,7 +770,7 @@ struct SolveTask::Impl {
         timer.end(stats.ms_get_rows);
     }
 
-    bool rows_ahead() const { return tsvm::ChipSplit::block_beside_rows(k_mat.n_features(), ws_size, rows_seconds()); }
+    bool rows_ahead() const { return tsvm::ChipSplit::rows_ahead(k_mat.dense_layout(), k_mat.n_features(), ws_size, rows_seconds()); }
     double rows_seconds() const { return tsvm::ChipSplit::rows_seconds(k_mat.n_features(), last_rows_computed, n_u); }
 
     void enqueue_block() {

@@ -56,6 +56,8 @@ struct ChipSplit {
     static bool block_beside_rows(size_t features, int ws, double rows_seconds) {
         return 32.0 * 0.53 * ChipSplit::rows_seconds(features, ws, ws) + 0.4e-3 <= rows_seconds;
     }
+    // (dense data only: rows_seconds prices every column, of sparse rows of 50 entries among 20,958 columns 400 times too high)
+    static bool rows_ahead(bool dense, size_t features, int ws, double rows_seconds) { return dense && block_beside_rows(features, ws, rows_seconds); }
     // Whether the block is read into the solver's L2 a second time, behind the rows that stream through it beside the solver and
     // take its place there (epsilon-SVR 40000x90, rows for 42 us beside a solver of 310: 88.4 -> 81.3 ms), unless they take
     // about as long as the solver (20000x784, 340 us: 50.2 -> 50.3).  Behind rows that go ahead the block may not be there yet.
