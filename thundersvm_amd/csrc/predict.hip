@@ -26,13 +26,23 @@ typedef double v2d __attribute__((ext_vector_type(2)));
 // kernel (64 batch rows x 128 columns, the next tile's first loads requested ahead of the epilogue), with NC
 // running sums per batch row and lane in registers for the whole chunk.
 // ------------------------------------------------------------------------------------------------
-template <int KT, int NC, int IND, int K_TILES>   // K_TILES: 1 = a single K tile (d <= 16), 2 = any number
+// Groups of rows that have their own support vectors come with a table of who does what and their rows by number.  A variant of its
+// own: as two pointers that are mostly null, every workgroup waited for the loads behind them to be ruled out before it
+// asked for its rows (a request of three rows 35.9 -> 36.2 us).
+template <bool GROUPS>
+struct StreamGroups {
+    const tsvm_predict_task *tasks;
+    const int *rows;
+};
+template <>
+struct StreamGroups<false> {};
+
+template <int KT, int NC, int IND, int K_TILES, bool GROUPS>   // K_TILES: 1 = a single K tile (d <= 16), 2 = any number
 __global__ __launch_bounds__(256, 2) void predict_dense_stream_kernel(
     const double *__restrict__ x, int64_t ldx, const int *__restrict__ col_map, int d, const double *__restrict__ sd_x,
     const uint64_t *__restrict__ mask_x, const double *__restrict__ a, int64_t lda, int m, const double *__restrict__ sd_a,
     const uint64_t *__restrict__ mask_a, int max_ones, KernelParam kp_in, const double *__restrict__ coef_t,
-    const int *__restrict__ chunks, unsigned m_blocks, double *__restrict__ partial, int nc_out, const tsvm_predict_task *__restrict__ tasks,
-    const int *__restrict__ a_idx) {
+    const int *__restrict__ chunks, unsigned m_blocks, double *__restrict__ partial, int nc_out, StreamGroups<GROUPS> groups) {
     constexpr int TI = 2;
     constexpr int BM = GrShape<TI>::BM;
     constexpr int KTILE = GrShape<TI>::KTILE;
@@ -55,10 +65,9 @@ __global__ __launch_bounds__(256, 2) void predict_dense_stream_kernel(
     // Workgroups are dealt to the eight XCDs in turn, so every XCD gets an eighth of every chunk's row blocks, and all of them
     // have the same chunk in their L2 at a time.  A run of chunks per XCD would leave those with the small classes' short chunks
     // idle: 50,000 rows of 54 columns against 16,076 support vectors in seven classes 3.07 -> 1.76 ms.
-    // (Groups of rows that have their own support vectors come with a table of who does what, and their rows by number.)
     tsvm_predict_task t;
-    if (tasks) {
-        t = tasks[blockIdx.x];
+    if constexpr (GROUPS) {
+        t = groups.tasks[blockIdx.x];
     } else {
         t.row_begin = (int) (blockIdx.x % m_blocks) * BM;
         t.row_end = m;
@@ -71,7 +80,10 @@ __global__ __launch_bounds__(256, 2) void predict_dense_stream_kernel(
     const int wave = tid >> 6;
     const int wi = wave >> 1, wj = wave & 1;
     const int m_last = t.row_end - 1;
-    const auto batch_row = [&](int r) { return a_idx ? a_idx[min(r, m_last)] : min(r, m_last); };
+    const auto batch_row = [&](int r) {
+        if constexpr (GROUPS) return groups.rows[min(r, m_last)];
+        else return min(r, m_last);
+    };
     const int a_row = tid / A_TPR, a_k = (tid % A_TPR) * (4 * A_VEC);
     const int b_row = tid >> 1, b_k = (tid & 1) * (4 * B_VEC);
     const int lrow = lane & 15;
@@ -354,8 +366,9 @@ __global__ __launch_bounds__(256, 2) void predict_dense_tile_kernel(
 }
 
 // dec[r * P + p] for pair p = (i < j): the chunks of class i under coefficient row j - 1, then the chunks of class j
-// under coefficient row i, each in chunk order, minus rho[p] (the order of kernelmatrix_kernel.cpp:129-143).  row_group: groups of
+// under coefficient row i, each in chunk order, minus rho[p] (the order of kernelmatrix_kernel.cpp:129-143).  GROUPS: groups of
 // rows have class_chunk_start and rho of their own.
+template <bool GROUPS>
 __global__ __launch_bounds__(256) void predict_combine_kernel(const double *__restrict__ partial, int64_t m, int nc,
                                                               const int *__restrict__ class_chunk_start,
                                                               const double *__restrict__ rho, int n_classes,
@@ -370,7 +383,7 @@ __global__ __launch_bounds__(256) void predict_combine_kernel(const double *__re
         ++i;
     }
     const int j = i + 1 + p;
-    if (row_group) {
+    if constexpr (GROUPS) {
         class_chunk_start += (int64_t) row_group[r] * (n_classes + 1);
         rho += row_group[r] * P;
     }
@@ -404,14 +417,16 @@ __global__ __launch_bounds__(VOTE_T) void predict_votes_kernel(const double *__r
 
 static int nc_template(int nc) { return nc <= 4 ? nc : nc <= 6 ? 6 : 8; }
 
-// The variant of the kernel for the model's shape: its kernel, coefficient rows (`stride`), indicator columns and K tiles.
+// The variant of the kernel for the model's shape: its kernel, coefficient rows (`stride`), indicator columns (not with groups) and
+// K tiles.
+template <bool GROUPS>
 static void launch_stream(dim3 grid, const double *sv_x, int64_t ldx, const int *col_map, int d, const double *sd_sv, const uint64_t *mask_sv,
                           const double *a, int64_t lda, int m, const double *sd_a, const uint64_t *mask_a, int max_ones, const KernelParam &kp,
                           const double *coef_t, int stride, const int *chunks, unsigned m_blocks, double *partial, int nc,
-                          const tsvm_predict_task *tasks, const int *a_idx, hipStream_t s) {
+                          const StreamGroups<GROUPS> &groups, hipStream_t s) {
 #define PD_STREAM(KTYPE, NC_, IND_, KT_)                                                                                        \
-    hipLaunchKernelGGL((predict_dense_stream_kernel<KTYPE, NC_, IND_, KT_>), grid, dim3(256), 0, s, sv_x, ldx, col_map, d, sd_sv,    \
-               mask_sv, a, lda, m, sd_a, mask_a, max_ones, kp, coef_t, chunks, m_blocks, partial, nc, tasks, a_idx)
+    hipLaunchKernelGGL((predict_dense_stream_kernel<KTYPE, NC_, IND_, KT_, GROUPS>), grid, dim3(256), 0, s, sv_x, ldx, col_map, d, sd_sv,    \
+               mask_sv, a, lda, m, sd_a, mask_a, max_ones, kp, coef_t, chunks, m_blocks, partial, nc, groups)
 #define PD_NC(KTYPE, IND_, KT_)                         \
     switch (stride) {                                   \
         case 1: PD_STREAM(KTYPE, 1, IND_, KT_); break;  \
@@ -421,34 +436,34 @@ static void launch_stream(dim3 grid, const double *sv_x, int64_t ldx, const int 
         case 6: PD_STREAM(KTYPE, 6, IND_, KT_); break;  \
         default: PD_STREAM(KTYPE, 8, IND_, KT_); break; \
     }
-#define PD_RBF(IND_)                              \
+#define PD_KIND(KTYPE, IND_)                      \
     do {                                          \
-        if (d <= 16) PD_NC(TSVM_RBF, IND_, 1)     \
-        else PD_NC(TSVM_RBF, IND_, 2)             \
+        if (d <= 16) PD_NC(KTYPE, IND_, 1)        \
+        else PD_NC(KTYPE, IND_, 2)                \
     } while (0)
-#define PD_KIND(KTYPE)                            \
-    do {                                          \
-        if (mask_sv) {                            \
-            if (d <= 16) PD_NC(KTYPE, 5, 1)       \
-            else PD_NC(KTYPE, 5, 2)               \
-        } else {                                  \
-            if (d <= 16) PD_NC(KTYPE, 0, 1)       \
-            else PD_NC(KTYPE, 0, 2)               \
-        }                                         \
-    } while (0)
-    switch (kp.kernel_type) {
-        case TSVM_LINEAR: PD_KIND(TSVM_LINEAR); break;
-        case TSVM_POLY: PD_KIND(TSVM_POLY); break;
-        case TSVM_SIGMOID: PD_KIND(TSVM_SIGMOID); break;
-        default:
-            if (mask_sv && max_ones == 1) PD_RBF(1);
-            else if (mask_sv && max_ones == 2) PD_RBF(2);
-            else if (mask_sv && max_ones == 3) PD_RBF(3);
-            else if (mask_sv && max_ones == 4) PD_RBF(4);
-            else PD_KIND(TSVM_RBF);
-            break;
+    if constexpr (!GROUPS) {
+        if (mask_sv) {
+            switch (kp.kernel_type) {
+                case TSVM_LINEAR: PD_KIND(TSVM_LINEAR, 5); break;
+                case TSVM_POLY: PD_KIND(TSVM_POLY, 5); break;
+                case TSVM_SIGMOID: PD_KIND(TSVM_SIGMOID, 5); break;
+                default:
+                    if (max_ones == 1) PD_KIND(TSVM_RBF, 1);
+                    else if (max_ones == 2) PD_KIND(TSVM_RBF, 2);
+                    else if (max_ones == 3) PD_KIND(TSVM_RBF, 3);
+                    else if (max_ones == 4) PD_KIND(TSVM_RBF, 4);
+                    else PD_KIND(TSVM_RBF, 5);
+                    break;
+            }
+            return;
+        }
     }
-#undef PD_RBF
+    switch (kp.kernel_type) {
+        case TSVM_LINEAR: PD_KIND(TSVM_LINEAR, 0); break;
+        case TSVM_POLY: PD_KIND(TSVM_POLY, 0); break;
+        case TSVM_SIGMOID: PD_KIND(TSVM_SIGMOID, 0); break;
+        default: PD_KIND(TSVM_RBF, 0); break;
+    }
 #undef PD_KIND
 #undef PD_NC
 #undef PD_STREAM
@@ -507,8 +522,8 @@ int tsvm_predict_dec_values_dense(const double *sv_x, int64_t ldx, int d, const 
             const unsigned m_blocks = (unsigned) ((m + 63) / 64);
             TSVM_REQUIRE((int64_t) m_blocks * n_chunks < (int64_t) 0x7fffffff, "tsvm_predict_dec_values_dense: grid too large");
             const dim3 grid(m_blocks * (unsigned) n_chunks);
-            launch_stream(grid, sv_x, ldx, col_map, d, sd_sv, mask_sv, a, lda, (int) m, sd_a, mask_a, max_ones, kp, coef_t, stride, chunks, m_blocks,
-                          partial, nc, nullptr, nullptr, tsvm_s(stream));
+            launch_stream<false>(grid, sv_x, ldx, col_map, d, sd_sv, mask_sv, a, lda, (int) m, sd_a, mask_a, max_ones, kp, coef_t, stride, chunks, m_blocks,
+                                 partial, nc, {}, tsvm_s(stream));
         } else {
             const unsigned m_blocks = (unsigned) ((m + 127) / 128);
             TSVM_REQUIRE((int64_t) m_blocks * n_chunks < (int64_t) 0x7fffffff, "tsvm_predict_dec_values_dense: grid too large");
@@ -528,7 +543,7 @@ int tsvm_predict_dec_values_dense(const double *sv_x, int64_t ldx, int d, const 
         TSVM_LAUNCH_CHECK();
     }
     const int64_t P = (int64_t) n_classes * nc / 2;
-    hipLaunchKernelGGL(predict_combine_kernel, dim3((unsigned) ((m * P + 255) / 256)), block, 0, tsvm_s(stream), partial, m, nc,
+    hipLaunchKernelGGL(predict_combine_kernel<false>, dim3((unsigned) ((m * P + 255) / 256)), block, 0, tsvm_s(stream), partial, m, nc,
                        class_chunk_start, rho, n_classes, nullptr, dec_values);
     TSVM_LAUNCH_CHECK();
     return 0;
@@ -550,12 +565,12 @@ int tsvm_predict_groups_dense(const double *x, int64_t ldx, int d, const double 
     TSVM_REQUIRE(stride > 0, "tsvm_predict_groups_dense: %d classes are too many", n_classes);
     if (m == 0) return 0;
     if (n_tasks > 0) {
-        launch_stream(dim3((unsigned) n_tasks), x, ldx, col_map, d, sd, nullptr, x, ldx, (int) m, sd, nullptr, 0, KernelParam{kernel_type, degree, gamma, coef0},
-                      coef_t, stride, chunks, 1, partial, nc, tasks, rows, tsvm_s(stream));
+        launch_stream<true>(dim3((unsigned) n_tasks), x, ldx, col_map, d, sd, nullptr, x, ldx, (int) m, sd, nullptr, 0, KernelParam{kernel_type, degree, gamma, coef0},
+                            coef_t, stride, chunks, 1, partial, nc, {tasks, rows}, tsvm_s(stream));
         TSVM_LAUNCH_CHECK();
     }
     const int64_t P = (int64_t) n_classes * nc / 2;
-    hipLaunchKernelGGL(predict_combine_kernel, dim3((unsigned) ((m * P + 255) / 256)), dim3(256), 0, tsvm_s(stream), partial, m, nc, class_chunk_start,
+    hipLaunchKernelGGL(predict_combine_kernel<true>, dim3((unsigned) ((m * P + 255) / 256)), dim3(256), 0, tsvm_s(stream), partial, m, nc, class_chunk_start,
                        rho, n_classes, row_group, dec_values);
     TSVM_LAUNCH_CHECK();
     return 0;
