@@ -2,6 +2,8 @@
 // the reference's SyncArray (the cases of src/test/test_syncmem.cpp and test_syncarray.cpp that apply), the kernel-row
 // cache's bookkeeping, the host's bounded wait for the local solver, and the matrices of the scikit entry points.  Built into a library of its own, next to
 // the tests; the product libraries do not contain it.
+#include <omp.h>
+
 #include <chrono>
 #include <stdexcept>
 #include <string>
@@ -11,6 +13,7 @@
 #include "../../thundersvm_amd/host/device.h"
 #include "../../thundersvm_amd/host/kernelmatrix.h"
 #include "../../thundersvm_amd/host/row_cache.h"
+#include "../../thundersvm_amd/host/rows.h"
 #include "../../thundersvm_amd/host/solver.h"
 
 namespace {
@@ -259,6 +262,16 @@ int tsvm_selftest_chip_split(int features, int ws, long long n, long long m_befo
 int tsvm_selftest_rows_ahead(int dense, int features, int ws, long long n, long long m_before) {
     using tsvm::ChipSplit;
     return ChipSplit::rows_ahead(dense != 0, features, ws, ChipSplit::rows_seconds(features, m_before, n));
+}
+
+// The team of a parallel region when nobody has asked for a number of threads (how 0), n has been asked for as -o and n_jobs do (1), or a
+// program has set n for itself (2).
+int tsvm_selftest_thread_limit(int how, int n) {
+    if (how == 1) set_threads(n);
+    if (how == 2) omp_set_num_threads(n);
+    const int limit = thread_limit();
+    set_threads(0);
+    return limit;
 }
 
 }  // extern "C"

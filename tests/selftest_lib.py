@@ -26,5 +26,6 @@ def lib():
         L.tsvm_selftest_load_matrix.argtypes = [ctypes.c_int] * 3 + [ctypes.c_void_p] * 6 + [ctypes.c_longlong]
         L.tsvm_selftest_chip_split.argtypes = [ctypes.c_int] * 2 + [ctypes.c_longlong] * 3
         L.tsvm_selftest_rows_ahead.argtypes = [ctypes.c_int] * 3 + [ctypes.c_longlong] * 2
+        L.tsvm_selftest_thread_limit.argtypes = [ctypes.c_int] * 2
         _LIB = L
     return _LIB

@@ -6,6 +6,7 @@ import subprocess
 
 import pytest
 
+import selftest_lib
 from thundersvm_amd import model
 from thundersvm_amd.model import TsvmParam
 
@@ -78,3 +79,17 @@ def test_train_predict_cli(tmp_path):
     assert "Accuracy = 0.98" in r.stderr                       # README.md:95-98 of the reference
     labels = [float(v) for v in open(out).read().split()]
     assert len(labels) == 150
+
+
+def test_threads_that_are_asked_for_are_used():
+    """-o n and n_jobs = n, and a program's own omp_set_num_threads, give a team of n; a quarter is left free only of what nobody asked for."""
+    L = selftest_lib.lib()
+    for asked in (1, 2, 3, 5, 8, 16, os.cpu_count()):
+        assert L.tsvm_selftest_thread_limit(1, asked) == asked
+    free = L.tsvm_selftest_thread_limit(0, 0)
+    for own in (1, 2, 3, 5, 8, 16):
+        if (3 * own + 3) // 4 != free:   # (not the number there is)
+            assert L.tsvm_selftest_thread_limit(2, own) == own
+    rc = parse("-o", "4", "dataset/test_dataset.txt")[0]
+    assert rc == 0 and L.tsvm_selftest_thread_limit(0, 0) == 4
+    assert L.tsvm_selftest_thread_limit(0, 0) == free

@@ -1,6 +1,5 @@
 #include "cmdparser.h"
-
-#include <omp.h>
+#include "rows.h"
 
 #include <cstdlib>
 #include <cstring>
@@ -73,7 +72,7 @@ void CMDParser::parse_train(int argc, char **argv, int first) {
     param_cmd.nr_weight = (int) weights_.size();
     param_cmd.weight_label = weight_labels_.empty() ? nullptr : weight_labels_.data();
     param_cmd.weight = weights_.empty() ? nullptr : weights_.data();
-    if (n_cores > 0) omp_set_num_threads(n_cores);
+    if (n_cores > 0) set_threads(n_cores);
     else if (n_cores != -1) throw std::invalid_argument("the number of cpu cores must be positive or -1");
     if (i >= argc) throw std::invalid_argument("no training file given");
     if (!check_parameter()) throw std::invalid_argument("invalid parameter");
@@ -100,7 +99,7 @@ void CMDParser::parse_predict(int argc, char **argv, int first) {
             default: throw std::invalid_argument(std::string("Unknown option: -") + opt);
         }
     }
-    if (n_cores > 0) omp_set_num_threads(n_cores);
+    if (n_cores > 0) set_threads(n_cores);
     if (i + 2 >= argc) throw std::invalid_argument("expected: test_file model_file output_file");
     svmpredict_input_file = argv[i];
     svmpredict_model_file_name = argv[i + 1];

@@ -3,9 +3,22 @@
 #include <omp.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 
-int thread_limit() { return (3 * omp_get_max_threads() + 3) / 4; }
+namespace {
+const int g_threads_at_start = omp_get_max_threads();
+std::atomic<int> g_threads_asked{0};
+}  // namespace
+
+void set_threads(int n) {
+    g_threads_asked = n;
+    omp_set_num_threads(n > 0 ? n : g_threads_at_start);
+}
+int thread_limit() {
+    const int n = omp_get_max_threads();
+    return n == g_threads_asked || n != g_threads_at_start ? n : (3 * n + 3) / 4;
+}
 int threads_for(size_t entries) { return (int) std::max<size_t>(1, std::min<size_t>((size_t) thread_limit(), entries / 32768)); }
 
 // (none of the arrays is value-initialised: whoever fills them does so on many threads, which also take the page faults)

@@ -53,11 +53,13 @@ private:
     mutable node2d nodes_;
 };
 
-// The most threads of a training or prediction call's parallel regions: three quarters of what there is.  The team goes on spinning
+// The most threads of a training or prediction call's parallel regions: as many as the caller has asked for (set_threads, or
+// omp_set_num_threads in a program of its own), else three quarters of what there is.  The team goes on spinning
 // for some 75 ms behind a region, so calls that follow one another faster keep all of it busy, the thread that waits for the
 // device and the runtime's own among it; with a thread for every CPU that a container has been given its scheduler then
 // stops the process for tens of milliseconds (epsilon-SVR 40000x90 with 16 threads on 16 CPUs: one call in
 // three takes 78 to 190 ms in place of 75).
 int thread_limit();
+void set_threads(int n);   // -o, n_jobs; 0: nobody has asked
 // Threads that pay for a loop over `entries` row entries: a parallel region costs some ten microseconds to enter.
 int threads_for(size_t entries);

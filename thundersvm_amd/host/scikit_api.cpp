@@ -1,8 +1,6 @@
 // The functions the reference's Python package calls (include/thundersvm_scikit.h; reference:
 // src/thundersvm/thundersvm-scikit.cpp).  Marshalling only: float32 arrays in and out, the models themselves are
 // the classes of models.h.  No exception leaves this file.
-#include <omp.h>
-
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -44,7 +42,7 @@ void train_on(DataSet &train, int svm_type, int kernel_type, int degree, float g
               int *succeed, SvmModel *model) {
     succeed[0] = 1;
     tsvm::Log::enabled() = verbose != 0;
-    if (n_cores > 0) omp_set_num_threads(n_cores);
+    if (n_cores > 0) set_threads(n_cores);
     else if (n_cores != -1) std::fprintf(stderr, "thundersvm: n_jobs must be positive or -1\n");
     std::vector<int> w_label(weight_label, weight_label + (weight_size > 0 ? weight_size : 0));
     std::vector<float_type> w(weight, weight + (weight_size > 0 ? weight_size : 0));
