@@ -315,7 +315,7 @@ __device__ __forceinline__ bool solver_begins(int *gate, int epoch, int target_x
 // 82 KB in place of 73 every launch waited for the others' solvers, and seven classes of 92,000 rows took 20 % longer.)
 struct __align__(32) SvElem {
     SvBound bound;
-    double kd, f;             // f: c_smo_iterate's, at the wavefronts' candidates for j2 (the others are not written)
+    double kd, f;             // f: c_smo_iterate's alone, at the wavefronts' candidates for j2 (the others are not written)
 };
 template <int N, int W>
 struct SvShared {
@@ -709,7 +709,7 @@ __device__ __forceinline__ unsigned nu_member_bits(double z, const SvBound &boun
 
 // The iterations of nu_smo_solve.  Takes up to `left` steps, counted in n_iter; returns whether the solve has ended.
 template <int E, int W, int LDK, typename TB>
-__device__ __forceinline__ bool nu_iterate(SvShared<E * 64 * W, W> &sh, double (&s_f)[2][E * 64 * W], double (&s_k)[2][E * 64 * W], SvCand *s_ip, SvCand *s_in,
+__device__ __forceinline__ bool nu_iterate(SvShared<E * 64 * W, W> &sh, double (&s_f)[2][E * 4 * W], double (&s_k)[2][E * 4 * W], SvCand *s_ip, SvCand *s_in,
                                            SvCand *s_jp, SvCand *s_jn, int ws, const TB *kws, const double (&kd)[E], double (&f)[E], unsigned &member,
                                            double local_eps, int max_iter, int &n_iter, int left) {
     const int tid = threadIdx.x;
@@ -722,6 +722,7 @@ __device__ __forceinline__ bool nu_iterate(SvShared<E * 64 * W, W> &sh, double (
     int own[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) own[e] = tid * E + e < ws ? tid * E + e : ws - 1;
+    const int row_at = (tid >> 4) * E;   // where this lane publishes its elements when it is its row's candidate
     for (; left > 0; --left) {
         double fup[E], fun[E];
 #pragma unroll
@@ -771,14 +772,14 @@ __device__ __forceinline__ bool nu_iterate(SvShared<E * 64 * W, W> &sh, double (
         int j2p, j2n;
         if constexpr (W == 4) {
             block_first_mins<E>(s_jp, s_jn, qp, qn, own, go, [&](uint64_t lanes_p, uint64_t lanes_n) {
-                publish_row<E, TB>(s_f[0] + tid * E, s_k[0] + tid * E, lanes_p, f, kIp);
-                publish_row<E, TB>(s_f[1] + tid * E, s_k[1] + tid * E, lanes_n, f, kIn);
+                publish_row<E, TB>(s_f[0] + row_at, s_k[0] + row_at, lanes_p, f, kIp);
+                publish_row<E, TB>(s_f[1] + row_at, s_k[1] + row_at, lanes_n, f, kIn);
             }, f_val_j2p, f_val_j2n, j2p, j2n, go);
         } else {
             const int win_jp = wave_first_argmin<E>(qp, tid * E, f_val_j2p, m_p, at_p);
             const int win_jn = wave_first_argmin<E>(qn, tid * E, f_val_j2n, m_n, at_n);
-            publish_row<E, TB>(s_f[0] + tid * E, s_k[0] + tid * E, 1ull << win_jp, f, kIp);
-            publish_row<E, TB>(s_f[1] + tid * E, s_k[1] + tid * E, 1ull << win_jn, f, kIn);
+            publish_row<E, TB>(s_f[0] + row_at, s_k[0] + row_at, 1ull << win_jp, f, kIp);
+            publish_row<E, TB>(s_f[1] + row_at, s_k[1] + row_at, 1ull << win_jn, f, kIn);
             j2p = __builtin_amdgcn_readlane(at_p, win_jp);
             j2n = __builtin_amdgcn_readlane(at_n, win_jn);
         }
@@ -797,9 +798,10 @@ __device__ __forceinline__ bool nu_iterate(SvShared<E * 64 * W, W> &sh, double (
         TB kJ[E];
         load_row(j2, kJ);
         SV_PIN_MEMORY;
-        const double kd_j = sh.elem[j2].kd, z_j = sh.z[wave][j2], z_i = sh.z[wave][i], f_j = s_f[side][j2];
+        const int j2_at = j2 / (16 * E) * E + j2 % E;   // (the lane that has published it is the only one of its row)
+        const double kd_j = sh.elem[j2].kd, z_j = sh.z[wave][j2], z_i = sh.z[wave][i], f_j = s_f[side][j2_at];
         const SvBound bound_i = sh.elem[i].bound, bound_j = sh.elem[j2].bound;
-        const double kIj = (double) *(const TB *) (s_k[side] + j2);
+        const double kIj = (double) *(const TB *) (s_k[side] + j2_at);
         SV_PIN;   // the row is on its way while the exit test and the step are computed
         if (n_iter > max_iter || !go) return true;
         const double up_value = take_p ? up_value_p : up_value_n;
@@ -987,10 +989,13 @@ __global__ __launch_bounds__(64 * W) void nu_smo_solve_kernel(
         return;
     constexpr int N = E * 64 * W;
     __shared__ SvShared<N, W> sh;
-    __shared__ double s_f[2][N], s_k[2][N];   // f and the rows ip / in at the elements of the wavefronts' candidates for j2
+    // f and the rows ip / in at the elements of the lanes that publish a candidate for j2, one of every sixteen.  (Slots for all elements
+    // made it 98 KB, with which two lanes' launches do not fit a CU: a nu-SVC of four classes, 40,000 rows of 23 columns, 24.9 -> 21.9 ms.)
+    __shared__ double s_f[2][4 * W * E], s_k[2][4 * W * E];
     __shared__ double s_red[4][W];
     __shared__ SvCand s_ip[4 * W], s_in[4 * W], s_jp[4 * W], s_jn[4 * W];
     __shared__ SvScoreStep s_score[4 * W];
+    static_assert(sizeof(sh) + sizeof(s_f) + sizeof(s_k) + sizeof(s_red) + 4 * sizeof(s_ip) + sizeof(s_score) <= 80 * 1024, "two workgroups on a CU");
 
     __builtin_amdgcn_s_setprio(3);
     const int tid = threadIdx.x;
