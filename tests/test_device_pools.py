@@ -11,3 +11,11 @@ def test_blocks_and_events_go_back_to_their_own_device():
     exe = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native", "two_devices")
     r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout == "ok\n", r.stderr
+
+
+def test_masked_streams_that_cannot_be_made():
+    """tests/native/lane_streams.cpp: every call that makes a group of streams fails in turn; nothing is left behind, and nothing is tried again."""
+    selftest_lib.lib()
+    exe = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native", "lane_streams")
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout == "ok\n", r.stderr

@@ -59,7 +59,7 @@ def build_host(extra=()):
 
 
 def build_selftests():
-    """The test-only library and program (tests/native): self-tests of host-layer pieces, linked against the host library."""
+    """The test-only library and programs (tests/native): self-tests of host-layer pieces, linked against the host library."""
     native = os.path.join(os.path.dirname(HERE), "tests", "native")
     out = os.path.join(native, "libtsvm_selftest.so")
     links = ["-L", HERE, "-lthundersvm", "-ltsvm_hip", "-Wl,-rpath,$ORIGIN/../../thundersvm_amd", "-L/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib"]
@@ -67,9 +67,10 @@ def build_selftests():
         return None
     _run(["g++", "-O2", "-fPIC", "-std=c++17", "-fopenmp", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", os.path.join(native, "selftest.cpp"),
           "-shared", "-o", out, *links])
-    # (-rdynamic: its stand-ins for the HIP calls take the place of the runtime's in the host library)
-    _run(["g++", "-O2", "-std=c++17", "-fopenmp", "-rdynamic", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", os.path.join(native, "two_devices.cpp"),
-          "-o", os.path.join(native, "two_devices"), *links])
+    # (-rdynamic: their stand-ins for the HIP calls take the place of the runtime's in the host library)
+    for program in ("two_devices", "lane_streams"):
+        _run(["g++", "-O2", "-std=c++17", "-fopenmp", "-rdynamic", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", os.path.join(native, program + ".cpp"),
+              "-o", os.path.join(native, program), *links])
     return out
 
 

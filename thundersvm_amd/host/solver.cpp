@@ -1,4 +1,5 @@
 #include "solver.h"
+#include "lane_streams.h"
 #include "row_cache.h"
 
 #include <chrono>
@@ -38,93 +39,10 @@ struct PhaseTimer {
     }
 };
 
-// CU-masked streams are kept for the life of the process and handed from one solve to the next: creating one
-// makes a hardware queue, which costs far more than a solve's other set-up (and every few creations the runtime
-// spends tens of milliseconds on queue housekeeping).  Keyed by device, lane and lane count (which fix the masks).
-struct LaneStreams {
-    hipStream_t chip = nullptr, solver = nullptr;
-    bool in_use = false;
-};
-// the streams of all lanes of one lane count on one device: made together, because the chip-wide mask leaves out
-// exactly the CUs on which the lanes' solvers land
-struct LaneGroup {
-    std::vector<LaneStreams> lanes;
-    // A group of one lane: a stream with every CU, and the CU that the lane's chip-wide stream leaves out (tsvm_where's number).
-    hipStream_t chain = nullptr;
-    int solver_cu = -1;
-};
-std::mutex g_masked_mutex;
-std::map<long long, std::vector<LaneGroup>> g_masked;   // keyed by device and lane count
-
 // the clock reading of the process's first solve: solves report their start and end relative to it
 std::chrono::steady_clock::time_point process_epoch() {
     static const std::chrono::steady_clock::time_point t0 = std::chrono::steady_clock::now();
     return t0;
-}
-
-// The pooled streams are destroyed by an atexit handler, registered when the first one is made and therefore run
-// before the HIP runtime's own tear-down (which, under a profiler, crashed on queues still alive at that point).
-void destroy_masked_streams() {
-    std::lock_guard<std::mutex> lock(g_masked_mutex);
-    for (auto &kv : g_masked)
-        for (LaneGroup &g : kv.second)
-            for (LaneStreams &m : g.lanes) {
-                if (m.solver) (void) hipStreamDestroy(m.solver);
-                if (m.chip) (void) hipStreamDestroy(m.chip);
-            }
-    for (auto &kv : g_masked)
-        for (LaneGroup &g : kv.second)
-            if (g.chain) (void) hipStreamDestroy(g.chain);
-    g_masked.clear();
-}
-
-// What a group of one lane has besides.
-bool find_solver_cu(LaneGroup &g) {
-    const uint32_t all[8] = {~0u, ~0u, ~0u, ~0u, ~0u, ~0u, ~0u, ~0u};
-    if (hipExtStreamCreateWithCUMask(&g.chain, 8, all) != hipSuccess) {
-        (void) hipGetLastError();
-        g.chain = nullptr;
-        return false;
-    }
-    DeviceBuffer<int> d_where(8);
-    int where[8];
-    abi_check(tsvm_where(d_where.data(), 8, g.lanes[0].solver));   // (one workgroup on every XCD's only CU)
-    TSVM_HIP_CHECK(hipMemcpyAsync(where, d_where.data(), sizeof(where), hipMemcpyDeviceToHost, g.lanes[0].solver));
-    TSVM_HIP_CHECK(hipStreamSynchronize(g.lanes[0].solver));
-    for (int w : where)
-        if (w >> 16 == 0) g.solver_cu = w & 0xffff;
-    return g.solver_cu >= 0;
-}
-
-// Makes the 2 * n_lanes streams of a group.  Bit i of a CU mask names CU i/8 of XCD i%8 on the 8-XCD, 256-CU part (a
-// mask has to leave every XCD at least one CU: workgroups are dealt to the XCDs in turn).  Every solver stream gets
-// CU 0 of every XCD, and lane l's solver is launched so that it runs on XCD l (tsvm_c_smo_solve_block_on_xcd: eight
-// workgroups, one per XCD, the one on XCD l solves, the others leave at once).  The lanes thus share the eight CUs
-// without sharing a CU, each solver behind another L2.  The chip-wide streams get every CU but those the solvers
-// really run on, CU 0 of XCDs 0 .. n_lanes-1: 255 CUs for one lane, 248 for eight.  (On the CUs the two masks share,
-// a solver launch's seven idle workgroups wait for room like any workgroup; the solver's result is behind them only in
-// stream order, and they are gone long before it is done.)
-bool make_lane_group(int n_lanes, LaneGroup &g) {
-    g.lanes.assign(n_lanes, LaneStreams());
-    uint32_t small[8] = {0xffu, 0, 0, 0, 0, 0, 0, 0};
-    uint32_t big[8] = {~((1u << n_lanes) - 1u), ~0u, ~0u, ~0u, ~0u, ~0u, ~0u, ~0u};   // all but CU 0 of XCDs 0 .. n_lanes-1
-    bool ok = true;
-    for (int l = 0; l < n_lanes && ok; ++l) {
-        ok = hipExtStreamCreateWithCUMask(&g.lanes[l].solver, 8, small) == hipSuccess;
-        if (!ok) { g.lanes[l].solver = nullptr; break; }
-        ok = hipExtStreamCreateWithCUMask(&g.lanes[l].chip, 8, big) == hipSuccess;
-        if (!ok) g.lanes[l].chip = nullptr;
-    }
-    if (!ok) {
-        (void) hipGetLastError();
-        for (LaneStreams &m : g.lanes) {
-            if (m.solver) (void) hipStreamDestroy(m.solver);
-            if (m.chip) (void) hipStreamDestroy(m.chip);
-        }
-        g.lanes.clear();
-    }
-    if (ok && n_lanes == 1) ok = find_solver_cu(g);
-    return ok;
 }
 
 }  // namespace
@@ -252,9 +170,7 @@ struct SolveTask::Impl {
     }
     bool on_one_stream = false;   // block and solver are on `sa`
     int last_rows_computed = 0;   // (this iteration's will probably be as many)
-    long long masked_key = 0;
-    int masked_lane = 0;
-    hipStream_t masked_chip = nullptr;   // the chip-wide stream of the pool that this task holds
+    tsvm::LaneLease lease;   // the streams of the pool that this task holds
     int solver_xcd = -1, solver_epoch = 0;   // masked streams: the XCD this lane's solver is launched onto, launches so far
     tsvm::DeviceBuffer<int> d_gate;
 
@@ -535,7 +451,7 @@ struct SolveTask::Impl {
         if (sa) (void) hipStreamSynchronize(sa);   // a selection enqueued ahead may still be running
         if (ss && ss != sa) (void) hipStreamSynchronize(ss);
         if (chain) (void) hipStreamSynchronize(sr);
-        if (split) release_split_streams();         // masked streams go back to the pool
+        if (split) tsvm::give_lane_streams(lease);  // masked streams go back to the pool
         else if (sa) (void) hipStreamDestroy(sa);
         // (both streams are empty: nothing uses the buffers any more)
         for (DeviceBuffer<int> *b : {&d_ws, &d_slots_a, &d_slots_b, &d_ws_folded, &d_gate, &d_slot_of, &d_cache_state}) b->release(true);
@@ -547,49 +463,17 @@ struct SolveTask::Impl {
         if (pinned.host) tsvm::give_pinned_block(pinned);
     }
 
-    // Two streams with disjoint CU masks from the pool (make_lane_group above).  Anything unexpected (another CU
-    // count, a call failing, TSVM_NO_CU_SPLIT set) leaves the task on one plain stream.
+    // Streams from the pool (lane_streams.h).  Anything unexpected (another CU count, a call failing, TSVM_NO_CU_SPLIT set) leaves
+    // the task on one plain stream.
     bool create_split_streams(int lane, int n_lanes) {
         if (!SolveTask::cu_split_available() || n_lanes < 1 || n_lanes > 8 || lane < 0 || lane >= n_lanes) return false;
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess) return false;
-        masked_key = (long long) dev * 16 + n_lanes;
-        masked_lane = lane;
-        std::lock_guard<std::mutex> lock(g_masked_mutex);
-        std::vector<LaneGroup> &groups = g_masked[masked_key];
-        LaneGroup *group = nullptr;
-        for (LaneGroup &g : groups)
-            if (!g.lanes[lane].in_use) { group = &g; break; }
-        if (!group) {
-            LaneGroup g;
-            if (!make_lane_group(n_lanes, g)) return false;
-            static bool registered = false;
-            if (!registered) {
-                registered = true;
-                atexit(destroy_masked_streams);
-            }
-            groups.push_back(std::move(g));
-            group = &groups.back();
-        }
-        LaneStreams &mine = group->lanes[lane];
-        mine.in_use = true;
-        masked_chip = mine.chip;
-        if (n_lanes == 1) {
-            chain = true;
-            solver_cu = group->solver_cu;
-            sa = ss = group->chain;
-            sr = mine.chip;
-        } else {
-            sa = mine.chip;
-            ss = mine.solver;
-        }
+        if (!tsvm::take_lane_streams(lane, n_lanes, lease)) return false;
+        chain = lease.chain != nullptr;
+        solver_cu = lease.solver_cu;
+        sa = chain ? lease.chain : lease.chip;
+        ss = chain ? sa : lease.solver;
+        sr = chain ? lease.chip : nullptr;
         return true;
-    }
-
-    void release_split_streams() {
-        std::lock_guard<std::mutex> lock(g_masked_mutex);
-        for (LaneGroup &g : g_masked[masked_key])
-            if (g.lanes[masked_lane].chip == masked_chip) g.lanes[masked_lane].in_use = false;
     }
 
     // without a cache the slot tables just alternate: the two halves of the working set swap places
