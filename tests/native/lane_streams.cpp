@@ -68,14 +68,13 @@ static void attempt(int n_lanes, int fail_at) {
         return;
     }
     expect(tsvm::take_lane_streams(0, n_lanes, lease), "no streams");
-    const size_t each = n_lanes == 1 ? 3 : 2 * n_lanes;
-    expect(g_live.size() == before + each, "two streams a lane, three for the only one");
-    expect(n_lanes == 1 ? lease.chain && lease.solver_cu == 100 : lease.solver && !lease.chain, "a lane's streams");
+    expect(g_live.size() == before + 2 * n_lanes, "two streams a lane");
+    expect(n_lanes == 1 ? lease.chain && !lease.solver && lease.solver_cu == 100 : lease.solver && !lease.chain, "a lane's streams");
     tsvm::LaneLease second, again;
     expect(tsvm::take_lane_streams(0, n_lanes, second) && second.chip != lease.chip, "streams that are in use");
-    expect(g_live.size() == before + 2 * each && second.solver_cu == lease.solver_cu, "as many streams of a second group");
+    expect(g_live.size() == before + 4 * n_lanes && second.solver_cu == lease.solver_cu, "two streams a lane of a second group");
     tsvm::give_lane_streams(lease);
-    expect(tsvm::take_lane_streams(0, n_lanes, again) && again.chip == lease.chip && g_live.size() == before + 2 * each, "streams that were given back");
+    expect(tsvm::take_lane_streams(0, n_lanes, again) && again.chip == lease.chip && g_live.size() == before + 4 * n_lanes, "streams that were given back");
 }
 
 int main() {

@@ -24,7 +24,7 @@ struct LaneStreams {
 // exactly the CUs on which the lanes' solvers land
 struct LaneGroup {
     std::vector<LaneStreams> lanes;
-    hipStream_t chain = nullptr;   // of one lane, besides
+    hipStream_t chain = nullptr;   // of one lane, in place of the solver's
 };
 std::mutex g_mutex;
 std::map<long long, std::vector<LaneGroup>> g_groups;
@@ -77,19 +77,22 @@ int find_solver_cu(hipStream_t stream) {
 // without sharing a CU, each solver behind another L2.  The chip-wide streams get every CU but those the solvers
 // really run on, CU 0 of XCDs 0 .. n_lanes-1: 255 CUs for one lane, 248 for eight.  (On the CUs the two masks share,
 // a solver launch's seven idle workgroups wait for room like any workgroup; the solver's result is behind them only in
-// stream order, and they are gone long before it is done.)  A lane that is the only one has a stream with every CU besides, on which
-// its solver finds that CU by itself; the solver stream only shows which one it is.
+// stream order, and they are gone long before it is done.)  A lane that is the only one has a stream with every CU instead, on which
+// its solver finds that CU by itself; a solver stream only shows, the first time, which one it is, and is given back: a
+// process that also has the streams of other lane counts has more queues than the hardware runs at a time, and each costs (after
+// solves in one, three and six lanes a nu-SVC of 21 pairs takes 250 ms, 360 with that queue kept, 88 in a process of its own).
 void make_lane_group(int device, int n_lanes, LaneGroup &g) {
     const uint32_t small[8] = {0xffu, 0, 0, 0, 0, 0, 0, 0}, all[8] = {~0u, ~0u, ~0u, ~0u, ~0u, ~0u, ~0u, ~0u};
     const uint32_t big[8] = {~((1u << n_lanes) - 1u), ~0u, ~0u, ~0u, ~0u, ~0u, ~0u, ~0u};   // all but CU 0 of XCDs 0 .. n_lanes-1
     g.lanes.assign(n_lanes, LaneStreams());
     for (LaneStreams &m : g.lanes) {
-        m.solver = masked_stream(small);
+        if (n_lanes > 1 || !g_solver_cu.count(device)) m.solver = masked_stream(small);
         m.chip = masked_stream(big);
     }
     if (n_lanes > 1) return;
     g.chain = masked_stream(all);
     if (!g_solver_cu.count(device)) g_solver_cu[device] = find_solver_cu(g.lanes[0].solver);
+    destroy(g.lanes[0].solver);
 }
 
 }  // namespace
