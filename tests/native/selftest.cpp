@@ -264,6 +264,19 @@ int tsvm_selftest_rows_ahead(int dense, int features, int ws, long long n, long 
     return ChipSplit::rows_ahead(dense != 0, features, ws, ChipSplit::rows_seconds(features, m_before, n));
 }
 
+// Of `selections` selections of n instances in a row, how many are guided when every miss_every-th guided one fails (0: none does).
+int tsvm_selftest_guided(long long n, int selections, int miss_every) {
+    tsvm::GuideSchedule guides(n);
+    int guided = 0;
+    bool missed = false;
+    for (int i = 0; i < selections; ++i) {
+        const bool is = guides.next(missed);
+        missed = is && miss_every > 0 && ++guided % miss_every == 0;
+        if (is && miss_every == 0) ++guided;
+    }
+    return guided;
+}
+
 // The team of a parallel region when nobody has asked for a number of threads (how 0), n has been asked for as -o and n_jobs do (1), or a
 // program has set n for itself (2).
 int tsvm_selftest_thread_limit(int how, int n) {

@@ -27,5 +27,6 @@ def lib():
         L.tsvm_selftest_chip_split.argtypes = [ctypes.c_int] * 2 + [ctypes.c_longlong] * 3
         L.tsvm_selftest_rows_ahead.argtypes = [ctypes.c_int] * 3 + [ctypes.c_longlong] * 2
         L.tsvm_selftest_thread_limit.argtypes = [ctypes.c_int] * 2
+        L.tsvm_selftest_guided.argtypes = [ctypes.c_longlong, ctypes.c_int, ctypes.c_int]
         _LIB = L
     return _LIB

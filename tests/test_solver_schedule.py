@@ -28,3 +28,19 @@ def test_chip_split(features, n, before, now, want):
 ])
 def test_rows_ahead(dense, features, n, before, want):
     assert selftest_lib.lib().tsvm_selftest_rows_ahead(dense, features, 1024, n, before) == want
+
+
+@pytest.mark.parametrize("n", [2, 1000, 40000, 300000, 1 << 20])
+def test_guides_that_fail_cost_little(n):
+    """The first selection goes by digits and guides that decide are used ever after.  A guide that fails costs 3.6 ns an instance: however
+    often they do, 10 us a selection at most, over 20,000 of them."""
+    L = selftest_lib.lib()
+    assert L.tsvm_selftest_guided(n, 1000, 0) == 999
+    for every in (1, 2, 32, 33, 100):
+        guided = L.tsvm_selftest_guided(n, 20000, every)
+        assert guided // every * 3.6e-3 * n <= 10.0 * 20000
+        assert guided > 0
+
+
+def test_no_guides_for_many_instances():
+    assert selftest_lib.lib().tsvm_selftest_guided((1 << 20) + 1, 1000, 0) == 0

@@ -148,25 +148,14 @@ struct SolveTask::Impl {
     volatile int *h_rows_done = nullptr;
     int *d_rows_done = nullptr;
     int rows_seq = 0;   // the number that h_rows_done takes with the rows enqueued last
-    // Selections are guided by the one before (tsvm_update_f_select_guided), but for the first (the first solve moves f by more than a
-    // guide reaches, from values that are mostly equal); when one has not been decided that way, which costs as much as ten others save, the
-    // next few go by digits, twice as many each time until 32 in a row have been decided.
+    // Selections are guided by the one before (tsvm_update_f_select_guided) as GuideSchedule has it.
     volatile int *h_missed = nullptr;
     int *d_missed = nullptr;
-    int unguided = 1, unguided_next = 2, decided_in_row = 0;
+    tsvm::GuideSchedule guides;
     bool next_is_guided() {
-        if (*h_missed) {
-            *h_missed = 0;
-            unguided = unguided_next;
-            unguided_next = std::min(2 * unguided_next, 32);
-            decided_in_row = 0;
-        }
-        if (unguided > 0) {
-            --unguided;
-            return false;
-        }
-        if (++decided_in_row == 32) unguided_next = 2;
-        return true;
+        const bool missed = *h_missed != 0;
+        if (missed) *h_missed = 0;
+        return guides.next(missed);
     }
     bool on_one_stream = false;   // block and solver are on `sa`
     int last_rows_computed = 0;   // (this iteration's will probably be as many)
@@ -314,7 +303,7 @@ struct SolveTask::Impl {
         : solver(solver), k_mat(k_mat), y(y), alpha(alpha), rho(rho), f_val(f_val), eps(eps), Cp(Cp), Cn(Cn), ws_size(ws_size),
           out_max_iter(out_max_iter), n((int) k_mat.n_instances()), n_u((int) k_mat.n_columns()), rep(k_mat.repeat()),
           row_type(k_mat.row_type()), row_esz(k_mat.row_elem_size()), q(ws_size / 2), ld(((int64_t) n_u + 7) / 8 * 8),
-          nu(solver.is_nu()), ldk(tsvm_smo_solve_block_ld(ws_size)), timer(solver.profile) {
+          nu(solver.is_nu()), ldk(tsvm_smo_solve_block_ld(ws_size)), guides(n), timer(solver.profile) {
         if (ws_size < 1 || ws_size > n || ws_size > 1024)
             throw std::invalid_argument("SolveTask: working-set size " + std::to_string(ws_size) + " for " + std::to_string(n) +
                                         " instances (1 .. min(instances, 1024))");

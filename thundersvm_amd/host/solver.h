@@ -63,6 +63,41 @@ struct ChipSplit {
     // about as long as the solver (20000x784, 340 us: 50.2 -> 50.3).  Behind rows that go ahead the block may not be there yet.
     static bool warm_behind_rows(bool block_beside, double rows_seconds) { return !block_beside && rows_seconds > 0 && rows_seconds < 0.1e-3; }
 };
+
+// Which selections of n instances are guided by the one before (tsvm_update_f_select_guided).  The first is not: the first solve moves f
+// by more than a guide reaches, from values that are mostly equal.  Where the guide does not decide, one workgroup resolves
+// the digits of all instances, which takes time with their number, while what a guide that decides saves hardly grows:
+//   instances              20,000   40,000  100,000  300,000  1,000,000  16,000,000
+//   by digits, us            33.7     32.6     39.8     52.3       71.2         471   (with update_f of one row in front)
+//   guided and decided       25.4     25.2     27.7     34.3       48.9         327
+//   guided and not            104      157      362    1,009      3,609      58,000
+// So behind one that was not, the next go by digits, twice as many each time up to n / 1,250 (32 at least): if every guide failed they would cost
+// some 4 us a selection whatever n is.  As many decided in a row, which have saved more than that failure cost, and it starts with two again.
+// Above 2^20 instances, where an iteration takes a millisecond or more and a guide saves 2 % of it or less, there are none.
+class GuideSchedule {
+public:
+    explicit GuideSchedule(long long n) : none_(n > (1 << 20)), most_(none_ ? 0 : (int) (n / 1250 > 32 ? n / 1250 : 32)) {}
+    // Whether the next selection is guided; missed: a guide has failed since this was last asked.
+    bool next(bool missed) {
+        if (none_) return false;
+        if (missed) {
+            unguided_ = stretch_;
+            stretch_ = 2 * stretch_ < most_ ? 2 * stretch_ : most_;
+            decided_ = 0;
+        }
+        if (unguided_ > 0) {
+            --unguided_;
+            return false;
+        }
+        if (++decided_ == most_) stretch_ = 2;
+        return true;
+    }
+
+private:
+    const bool none_;
+    const int most_;
+    int unguided_ = 1, stretch_ = 2, decided_ = 0;
+};
 }  // namespace tsvm
 
 class CSMOSolver {
