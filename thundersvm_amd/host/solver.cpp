@@ -540,9 +540,10 @@ struct SolveTask::Impl {
         hipStream_t st = rows_stream();
         // Rows that take about as long as the solver, or less, come when it has its CU; where they take longer than block and solver
         // together they go ahead of both.
+        const bool ahead = rows_ahead();   // (by the last iteration's rows)
         if (chain) wait_for_ids();
         const auto solver_first = [&] {
-            if (chain && !rows_ahead())
+            if (chain && !ahead)
                 wait_for_word((const volatile int *) (h_diff + 2), solver_epoch, sa, "the solver's start");
         };
         if (device_cache) {
@@ -639,7 +640,13 @@ struct SolveTask::Impl {
             solver_first();
             k_mat.get_rows(ws_u() + first_new, n_new, k_rows, ld, slots + first_new, st);
         }
-        if (chain) abi_check(tsvm_report_ids(ws_ids(), 0, 0, d_rows_done, 0, ++rows_seq, sr));
+        if (chain) {
+            // (not where other lanes' rows come through at any time: 7 classes 300000x54 844 -> 857; in front of the word that update_f waits
+            // for, so that the next block is not computed while this one is read)
+            if (k_mat.dense_layout() && !all_cached && tsvm::ChipSplit::warm_behind_rows(ahead, rows_seconds()))
+                abi_check(tsvm_smo_warm_block(d_kws.data(), row_type, ws_size, solver_xcd, d_gate.data() + 3, sr));
+            abi_check(tsvm_report_ids(ws_ids(), 0, 0, d_rows_done, 0, ++rows_seq, sr));
+        }
         timer.end(stats.ms_get_rows);
     }
 
@@ -706,9 +713,6 @@ struct SolveTask::Impl {
     }
 
     void enqueue_update() {
-        // (not where other lanes' rows come through at any time: 7 classes 300000x54 844 -> 857)
-        if (chain && k_mat.dense_layout() && !all_cached && tsvm::ChipSplit::warm_behind_rows(rows_ahead(), rows_seconds()))
-            abi_check(tsvm_smo_warm_block(d_kws.data(), row_type, ws_size, solver_xcd, d_gate.data() + 3, rows_stream()));
         if (chain && rows_seq != *h_rows_done) wait_for_word(h_rows_done, rows_seq, sr, "the rows");
         if (!on_one_stream) TSVM_HIP_CHECK(hipStreamWaitEvent(sa, solved.event, 0));   // alpha_diff, alpha and diff come from the solver
         if (select_ahead && fuse_select) {
