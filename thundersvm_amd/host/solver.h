@@ -50,9 +50,14 @@ struct ChipSplit {
     static double rows_seconds(size_t features, long long m, long long n) { return 2.0 * (double) ((features + 15) / 16 * 16) / 6.6e13 * (double) m * (double) n; }
     // Whether the rows go ahead of the block and the solver (they are enqueued when the selection has reported, and not when the solver
     // has its CU): when they, by the previous iteration's number of them, outlast the solver's ~0.4 ms and a block that has to find
-    // its CUs among them (136 of its 256 tiles, as if on 8 of the 256).  Until then they wait for the solver, whose launch
-    // reads the block into its L2 from the CUs that the rows would hold: 20,000 x 784 (340 us of rows an iteration) 39.3 ms a call,
-    // 40.9 with the rows always ahead.
+    // its CUs among them (priced as 136 of its 256 tiles on 8 CUs, some 35 times what it takes alone).  Until then they wait for the
+    // solver, whose launch reads the block into its L2 from the CUs that the rows would hold.  With 512 rows computed an iteration
+    // the line lies at 67,000 instances of 784 columns, 120,000 of 300 and 300,000 of 90.  A call in ms, by the rule / always ahead /
+    // always behind the solver:
+    //   784 columns    20,000   50.1 /  51.9 /  50.1      40,000   92.8 /  90.5 /  92.9      60,000   176 /   170 /   176      90,000   309 /   308 /   315
+    //   300 columns    60,000    183 /   219 /   183     120,000    461 /   557 /   461
+    //    90 columns    40,000   66.1 /  77.3 /  66.0     150,000    296 /   322 /   296     300,000   796 /   833 /   795     500,000 2,715 / 2,665 / 2,719
+    // (It leaves 3 % at 784 columns below its line, and 2 % far above it at 90, where fewer rows are computed in most iterations.)
     static bool block_beside_rows(size_t features, int ws, double rows_seconds) {
         return 32.0 * 0.53 * ChipSplit::rows_seconds(features, ws, ws) + 0.4e-3 <= rows_seconds;
     }
