@@ -526,6 +526,27 @@ def test_smo_solve_block_on_a_chosen_cu(n, ws, nu):
                   100000, G.ptr(gate), 1, 0, -1, G.stream())
 
 
+@pytest.mark.parametrize("on", ["xcd", "cu"])
+def test_arrivals_beyond_the_largest_int(on):
+    """Somebody solves when the gate's count of workgroups has passed 2^31: here the last to arrive, as nobody is on the CU that is asked for
+    (a die that is asked for has a workgroup: there only the count goes on)."""
+    n, ws, Cc, eps = 300, 130, 1.0, 1e-3
+    y, alpha, f, ws_ids, k_rows, diag = _solver_inputs(n, 10, ws, 7, Cc, False)
+    a_want, ad_want, diff_want = O.c_smo_solve(y, f, alpha, ws_ids, Cc, Cc, k_rows, diag, n, eps, 100000)
+    block = np.zeros((ws, capi.kernel_lib().tsvm_smo_solve_block_ld(ws)))
+    block[:, :ws] = k_rows[:, ws_ids]
+    y_d, f_d, ws_d, dg_d, blk_d = G.dev(y), G.dev(f), G.dev(ws_ids), G.dev(diag), G.dev(block)
+    gate = G.dev(np.array([0, -2 ** 31, 0, 0], dtype=np.int32))
+    for epoch in (1, 2):
+        a_d = G.dev(alpha)
+        ad_d, diff_d = torch.zeros(ws, dtype=torch.float64, device="cuda"), torch.zeros(3, dtype=torch.float64, device="cuda")
+        where = (0,) if on == "xcd" else (0, 0x7fff)
+        capi.call("tsvm_c_smo_solve_block_on_" + on, G.ptr(y_d), G.ptr(f_d), G.ptr(a_d), G.ptr(ad_d), G.ptr(ws_d), ws, Cc, Cc, G.ptr(blk_d), capi.ROW_F64,
+                  G.ptr(dg_d), eps, G.ptr(diff_d), 100000, G.ptr(gate), epoch, *where, G.stream())
+        assert G.host(gate)[0] == epoch and G.host(diff_d)[0] == diff_want[0]
+        assert np.array_equal(G.host(a_d), a_want) and np.array_equal(G.host(ad_d), ad_want)
+
+
 def _select_case(n, n_select, n_marked, seed, tie_mode, nu):
     rng = np.random.default_rng(seed)
     y = np.where(rng.random(n) < 0.5, 1, -1).astype(np.int32)

@@ -200,7 +200,7 @@ __device__ __forceinline__ bool solver_elected(int *gate, int epoch, int target_
         bool won = false;
         if (xcd == target_xcd) won = atomicCAS(&gate[0], epoch - 1, epoch) == epoch - 1;
         __threadfence();
-        const int arrived = atomicAdd(&gate[1], 1);
+        const unsigned arrived = atomicAdd((unsigned *) &gate[1], 1u);
         if (!won && (arrived % TSVM_SOLVER_GRID_ON_XCD) == TSVM_SOLVER_GRID_ON_XCD - 1) {
             __threadfence();
             won = atomicCAS(&gate[0], epoch - 1, epoch) == epoch - 1;
@@ -227,7 +227,8 @@ __device__ __forceinline__ bool solver_elected_on_cu(int *gate, int epoch, bool 
         int won = 0, seen = epoch - 1;
         if (on_target) won = __hip_atomic_compare_exchange_strong(&gate[0], &seen, epoch, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         asm volatile("s_waitcnt vmcnt(0)" : "+v"(won) :: "memory");
-        int arrived = __hip_atomic_fetch_add(&gate[1], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // (unsigned: 8.4 million launches take the count beyond the largest int)
+        unsigned arrived = __hip_atomic_fetch_add((unsigned *) &gate[1], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         asm volatile("s_waitcnt vmcnt(0)" : "+v"(arrived) :: "memory");
         if (!won && arrived % TSVM_SOLVER_GRID_ON_CU == TSVM_SOLVER_GRID_ON_CU - 1) {
             seen = epoch - 1;
