@@ -90,6 +90,8 @@ int tsvm_model_predict(void *model, void *dataset, int batch_size, double *dec_v
  * n_fold folds in class order, predictions[i] = the prediction for instance i by the model trained without its
  * fold (a label for the classifiers, a value for the regressors). */
 int tsvm_model_cross_validation(void *model, void *dataset, const tsvm_param *param, int n_fold, double *predictions);
+/* Folds of the model's last cross-validation that were predicted by a launch for several of them (0 before the first). */
+int64_t tsvm_model_folds_together(void *model);
 
 /* SvmModel::train on a LibSVM text file (DataSet::load_from_file). */
 int tsvm_model_train_file(void *model, const char *path, const tsvm_param *param);

@@ -5,7 +5,9 @@ distinguish: one to eleven coefficient rows, few / many features, indicator colu
 that do and do not fill a tile, rows already resident on the device."""
 import numpy as np
 import pytest
+import torch
 
+import gpu_util as G
 import oracle_lib as O
 from thundersvm_amd import capi
 from thundersvm_amd import data as D
@@ -351,3 +353,97 @@ def test_folds_predicted_together(svm_type, classes, n, d, kernel, folds, monkey
         np.testing.assert_allclose(together, one_by_one, rtol=0, atol=1e-9 * (1 + np.abs(one_by_one).max()))
     else:
         assert np.mean(together != one_by_one) <= 0.002   # (a decision value of about zero may fall on either side)
+
+
+@pytest.mark.parametrize("svm_type,classes", [(capi.EPSILON_SVR, 2), (capi.NU_SVR, 2), (capi.C_SVC, 3), (capi.ONE_CLASS, 1)])
+@pytest.mark.parametrize("n,d,hot,kernel,folds", [(40, 3, 0, capi.RBF, 5), (129, 16, 0, capi.POLY, 2), (545, 17, 0, capi.RBF, 10), (603, 127, 0, capi.LINEAR, 3),
+                                                  (603, 128, 0, capi.RBF, 3), (610, 6, 50, capi.LINEAR, 5), (610, 6, 50, capi.RBF, 5), (9000, 5, 0, capi.RBF, 3)])
+def test_folds_are_predicted_as_one_by_one(svm_type, classes, n, d, hot, kernel, folds):
+    """Every value of a cross-validation is, to the last bit, what a model that is trained on the fold's rows by themselves predicts in batches of
+    1,000 rows.  Folds of small problems with up to 128 columns are predicted by one launch (128 features make 129)."""
+    rng = np.random.default_rng(n + d + hot)
+    x = rng.standard_normal((n, d + hot)).astype(np.float32)
+    x[:, :d] *= (10.0 ** rng.uniform(-2, 0, d)).astype(np.float32)
+    x[:, d:] = 0
+    if hot:
+        x[np.arange(n), d + rng.integers(0, hot - 2, n)] = 1
+        x[np.arange(n), d + hot - 2 + rng.integers(0, 2, n)] = 1
+    c = rng.permutation(np.arange(n) % classes)
+    y = np.sign(x[:, 0]) if svm_type in (capi.EPSILON_SVR, capi.NU_SVR) else c + 1.0
+    data = D.from_dense(x, y)
+    prm = make_param(svm_type=svm_type, kernel_type=kernel, C=1.0, gamma=0.1 / d, nu=0.3, p=0.05, degree=2, max_iter=30)
+    m = Model(svm_type)
+    got = m.cross_validation(Dataset(data), prm, folds)
+    # the folds (svmmodel.cpp:31-71): label by label in the order of the first instances, the last one takes what is left
+    train, test = [[] for _ in range(folds)], [[] for _ in range(folds)]
+    for label in y[np.sort(np.unique(y, return_index=True)[1])]:
+        ids = np.flatnonzero(y == label)
+        each = len(ids) // folds
+        for k in range(folds):
+            lo, hi = each * k, len(ids) if k == folds - 1 else each * (k + 1)
+            test[k].append(ids[lo:hi])
+            train[k].append(np.concatenate([ids[:lo], ids[hi:]]))
+    want = np.zeros(n)
+    for k in range(folds):
+        tr, te = np.concatenate(train[k]), np.concatenate(test[k])
+        want[te] = Model(svm_type).train(D.from_dense(x[tr], y[tr]), prm).predict(D.from_dense(x[te], y[te]), 1000)[0]
+    assert np.array_equal(got, want)
+    small = n < 9000 and d < 128
+    assert m.folds_together() == (folds if small else 0)
+
+
+@pytest.mark.parametrize("k,d,kernel", [(2, 3, capi.RBF), (2, 16, capi.SIGMOID), (3, 17, capi.POLY), (4, 40, capi.RBF), (7, 54, capi.RBF), (9, 128, capi.LINEAR)])
+def test_groups_of_rows_in_one_launch(k, d, kernel):
+    """tsvm_predict_groups_dense gives, to the last bit, what a call of tsvm_predict_dec_values_dense gives for every group: groups of 1, 63, 64, 65
+    and 200 rows, classes of no support vectors, of one tile of 128 columns and of several, chunks of one tile and of two."""
+    rng = np.random.default_rng(10 * k + d)
+    n, ldx, nc, P = 500, (d + 7) // 8 * 8, k - 1, k * (k - 1) // 2
+    x = np.zeros((n, ldx))
+    x[:, :d] = rng.standard_normal((n, d))
+    sd = (x * x).sum(axis=1)
+    stride = capi.kernel_lib().tsvm_predict_nc_stride(k, d, 0)
+    assert stride >= nc
+    x_d, sd_d = G.dev(x), G.dev(sd)
+    args = (kernel, 0.5 / d, 0.25, 2)
+    col_map, coef, chunks, tasks, rows, row_group, starts, rhos, want = [], [], [], [], [], [], [], [], []
+    most = 0
+    for g, m in enumerate([1, 63, 64, 65, 200]):
+        n_sv = [130 if c % 3 == 0 else 0 if (c + g) % 4 == 1 else 1 + 40 * c for c in range(k)]
+        col0, row0, chunk0, per = sum(map(len, col_map)), len(rows), len(chunks), 1 + g % 2
+        mine, start, tile = [], [0], 0
+        for c in range(k):
+            tiles = (n_sv[c] + 127) // 128
+            ids, w = np.zeros(128 * tiles, dtype=np.int32), np.zeros((128 * tiles, stride))
+            ids[:n_sv[c]] = rng.integers(0, n, n_sv[c])
+            w[:n_sv[c], :nc] = rng.standard_normal((n_sv[c], nc))
+            col_map.append(ids)
+            coef.append(w)
+            mine += [(t, min(t + per, tile + tiles)) for t in range(tile, tile + tiles, per)]
+            tile += tiles
+            start.append(len(mine))
+        ids = rng.integers(0, n, m).astype(np.int32)
+        rho = rng.standard_normal(P)
+        group_cols, group_coef = np.concatenate(col_map[-k:]), np.concatenate(coef[-k:])
+        part_d = torch.full((len(mine) * m * nc,), np.nan, dtype=torch.float64, device="cuda")
+        dec_d = torch.full((m, P), np.nan, dtype=torch.float64, device="cuda")
+        held = [G.dev(group_cols), G.dev(group_coef), G.dev(np.array(mine, dtype=np.int32)), G.dev(np.array(start, dtype=np.int32)), G.dev(rho), G.dev(x[ids]), G.dev(sd[ids])]
+        capi.call("tsvm_predict_dec_values_dense", G.ptr(x_d), ldx, d, G.ptr(sd_d), None, G.ptr(held[0]), len(group_cols), G.ptr(held[1]), G.ptr(held[2]), len(mine),
+                  G.ptr(held[3]), G.ptr(held[4]), k, G.ptr(held[5]), ldx, m, G.ptr(held[6]), None, 0, *args, G.ptr(part_d), G.ptr(dec_d), G.stream())
+        want.append(G.host(dec_d))
+        tasks += [(row0 + r, row0 + m, chunk0 + part, part) for part in range(len(mine)) for r in range(0, m, 64)]
+        chunks += [(col0 // 128 + a, col0 // 128 + b) for a, b in mine]
+        rows += list(ids)
+        row_group += [g] * m
+        starts += start
+        rhos.append(rho)
+        most = max(most, len(mine))
+    want = np.concatenate(want)
+    assert np.isfinite(want).all() and np.abs(want).max() > 0
+    cols = np.concatenate(col_map)
+    held = [G.dev(cols), G.dev(np.concatenate(coef)), G.dev(np.array(chunks, dtype=np.int32)), G.dev(np.array(tasks, dtype=np.int32)), G.dev(np.array(rows, dtype=np.int32)),
+            G.dev(np.array(row_group, dtype=np.int32)), G.dev(np.array(starts, dtype=np.int32)), G.dev(np.concatenate(rhos))]
+    part_d = torch.full((most * len(rows) * nc,), np.nan, dtype=torch.float64, device="cuda")
+    dec_d = torch.full((len(rows), P), np.nan, dtype=torch.float64, device="cuda")
+    capi.call("tsvm_predict_groups_dense", G.ptr(x_d), ldx, d, G.ptr(sd_d), G.ptr(held[0]), len(cols), G.ptr(held[1]), G.ptr(held[2]), G.ptr(held[3]), len(tasks),
+              G.ptr(held[4]), len(rows), G.ptr(held[5]), G.ptr(held[6]), G.ptr(held[7]), k, *args, G.ptr(part_d), G.ptr(dec_d), G.stream())
+    assert np.array_equal(G.host(dec_d), want)

@@ -759,7 +759,7 @@ def test_update_f_with_the_next_selection(n_cols, repeat, ws, ld_pad, tie_mode, 
 
 @pytest.mark.parametrize("nu", [0, 1])
 @pytest.mark.parametrize("n_cols,repeat,row_type", [(2, 1, capi.ROW_F32), (700, 1, capi.ROW_F64), (3200, 1, capi.ROW_F32), (30000, 2, capi.ROW_F32),
-                                                    (70001, 1, capi.ROW_F64), (262144, 1, capi.ROW_F32)])
+                                                    (70001, 1, capi.ROW_F64), (262144, 1, capi.ROW_F32), (1 << 20, 1, capi.ROW_F32)])
 def test_guided_selections(n_cols, repeat, row_type, nu):
     """Selections that follow one another with the last one as a guide: f that moves a little, by far more than the guide reaches (either
     way, and in scale), ends in ties, has infinite values, and sides with fewer candidates than are asked for; and selections by

@@ -202,6 +202,8 @@ int tsvm_model_cross_validation(void *model, void *dataset, const tsvm_param *pa
     })
 }
 
+int64_t tsvm_model_folds_together(void *model) { return (int64_t) ((Handle *) model)->model->folds_together; }
+
 int tsvm_model_train_file(void *model, const char *path, const tsvm_param *param) {
     TSVM_GUARD({
         Handle *h = (Handle *) model;

@@ -154,7 +154,7 @@ void SvmModel::copy_settings(const SvmModel &other) {
 
 // The dataset's rows go to the device once; every fold takes its rows, its support vectors and the rows it is applied to
 // from there.  Folds whose problems are small (SmallBatch) are set up first and solved together.
-void SvmModel::train_folds(const DataSet &dataset, const std::vector<Fold> &folds, const SvmParam &p, const std::function<SvmModel &(size_t)> &model_of,
+size_t SvmModel::train_folds(const DataSet &dataset, const std::vector<Fold> &folds, const SvmParam &p, const std::function<SvmModel &(size_t)> &model_of,
                            const std::function<void(size_t, SvmModel &, std::vector<float_type> &)> &take) {
     const std::shared_ptr<DeviceRows> all = dataset.device_cache() ? std::static_pointer_cast<DeviceRows>(dataset.device_cache())
                                                                    : DeviceRows::from_host(dataset.rows());
@@ -169,6 +169,7 @@ void SvmModel::train_folds(const DataSet &dataset, const std::vector<Fold> &fold
         std::unique_ptr<DataSet> rows;
         Training training;
     };
+    size_t n_together = 0;
     constexpr size_t ROWS_AT_ONCE = 65536;   // (what the folds in flight hold on the host and the device grows with their rows)
     for (size_t k = 0; k < folds.size();) {
         std::vector<Begun> begun;
@@ -189,6 +190,7 @@ void SvmModel::train_folds(const DataSet &dataset, const std::vector<Fold> &fold
         }
         std::vector<std::vector<float_type>> dec;
         const bool together = begun.size() > 1 && predict_folds(*all, with, dec);
+        if (together) n_together += begun.size();
         for (size_t i = 0; i < begun.size(); ++i) {
             Begun &b = begun[i];
             SvmModel &m = *b.model;
@@ -203,6 +205,7 @@ void SvmModel::train_folds(const DataSet &dataset, const std::vector<Fold> &fold
             b.rows.reset();
         }
     }
+    return n_together;
 }
 
 // Stratified folds in class order (svmmodel.cpp:31-71).
@@ -235,7 +238,7 @@ std::vector<float_type> SvmModel::cross_validation(DataSet dataset, SvmParam p, 
         others[k]->copy_settings(*this);
         return *others[k];
     };
-    train_folds(dataset, folds, p, model_of, [&](size_t k, SvmModel &m, std::vector<float_type> &dec) {
+    folds_together = train_folds(dataset, folds, p, model_of, [&](size_t k, SvmModel &m, std::vector<float_type> &dec) {
         m.dec_values.swap(dec);
         const std::vector<float_type> y_predict = m.finish_predict((int) folds[k].test_idx.size());
         for (size_t i = 0; i < y_predict.size(); ++i) y_predict_all[folds[k].test_idx[i]] = y_predict[i];

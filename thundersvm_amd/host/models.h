@@ -59,6 +59,7 @@ public:
     bool profile = false;
     bool keep_binary = false;             // keep binary_alpha / binary_f (tests)
     long long cache_bytes = -1;           // kernel-row cache budget handed to the solver (-1 auto, 0 off)
+    size_t folds_together = 0;            // of the last cross-validation: folds that were predicted by a launch for several (tests)
     int pair_lanes = 0;                   // class pairs of a one-vs-one run in flight (0: automatic, 1: one at a time)
 
 protected:
@@ -77,8 +78,9 @@ protected:
         std::vector<int> train_idx, test_idx;
         std::vector<float_type> y_train;
     };
-    // trains model_of(k) on fold k of the dataset's instances and hands it over with the decision values of the others
-    static void train_folds(const DataSet &dataset, const std::vector<Fold> &folds, const SvmParam &param, const std::function<SvmModel &(size_t)> &model_of,
+    // trains model_of(k) on fold k of the dataset's instances and hands it over with the decision values of the others; returns how many
+    // folds were predicted by a launch for several
+    static size_t train_folds(const DataSet &dataset, const std::vector<Fold> &folds, const SvmParam &param, const std::function<SvmModel &(size_t)> &model_of,
                             const std::function<void(size_t, SvmModel &, std::vector<float_type> &)> &take);
     // Decision values of several folds at once, each fold's rows by its own model, whose support vectors are rows of the same dense
     // matrix: dec[k] as model k's predict_dec_values would have them.  False when the kernels do not take the models' shape.

@@ -84,6 +84,8 @@ def host_lib():
         L.tsvm_model_binary.argtypes = [C.c_void_p, C.c_int, _dp, _dp]
         L.tsvm_model_trace.argtypes = [C.c_void_p, _ip, C.POINTER(_dp), C.POINTER(_ip)]
         L.tsvm_model_predict_csr.argtypes = [C.c_void_p, C.c_int64, _i64p, _ip, _dp, C.c_int, _dp, _dp]
+        L.tsvm_model_folds_together.restype = C.c_int64
+        L.tsvm_model_folds_together.argtypes = [C.c_void_p]
         L.tsvm_model_save.argtypes = [C.c_void_p, C.c_char_p]
         L.tsvm_model_load.argtypes = [C.c_void_p, C.c_char_p]
         _HOST = L
@@ -268,6 +270,10 @@ class Model:
         out = np.zeros(dataset.n)
         _check(L.tsvm_model_cross_validation(self.h, dataset.h, C.byref(prm), n_fold, _p(out, _dp)))
         return out
+
+    def folds_together(self):
+        """Folds of the last cross-validation that were predicted by a launch for several of them."""
+        return host_lib().tsvm_model_folds_together(self.h)
 
     def save(self, path):
         _check(host_lib().tsvm_model_save(self.h, path.encode()))
