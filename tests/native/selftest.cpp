@@ -7,6 +7,7 @@
 #include <chrono>
 #include <stdexcept>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../thundersvm_amd/host/dataset.h"
@@ -277,12 +278,18 @@ int tsvm_selftest_guided(long long n, int selections, int miss_every) {
     return guided;
 }
 
-// The team of a parallel region when nobody has asked for a number of threads (how 0), n has been asked for as -o and n_jobs do (1), or a
-// program has set n for itself (2).
+// The team of a parallel region when nobody has asked for a number of threads (how 0), n has been asked for as -o and n_jobs do (1), a
+// program has set n for itself (2), or another of its threads has asked for n (3).
 int tsvm_selftest_thread_limit(int how, int n) {
     if (how == 1) set_threads(n);
     if (how == 2) omp_set_num_threads(n);
-    const int limit = thread_limit();
+    int limit = 0;
+    if (how == 3) {
+        set_threads(n);
+        std::thread([&] { limit = thread_limit(); }).join();
+    } else {
+        limit = thread_limit();
+    }
     set_threads(0);
     return limit;
 }

@@ -90,6 +90,8 @@ def test_threads_that_are_asked_for_are_used():
     for own in (1, 2, 3, 5, 8, 16):
         if (3 * own + 3) // 4 != free:   # (not the number there is)
             assert L.tsvm_selftest_thread_limit(2, own) == own
+    for asked in range(1, 2 * free + 2):   # (the number there is among them)
+        assert L.tsvm_selftest_thread_limit(3, asked) == free
     rc = parse("-o", "4", "dataset/test_dataset.txt")[0]
     assert rc == 0 and L.tsvm_selftest_thread_limit(0, 0) == 4
     assert L.tsvm_selftest_thread_limit(0, 0) == free

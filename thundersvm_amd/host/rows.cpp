@@ -3,21 +3,20 @@
 #include <omp.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cstring>
 
 namespace {
 const int g_threads_at_start = omp_get_max_threads();
-std::atomic<int> g_threads_asked{0};
+thread_local int t_threads_asked = 0;   // (omp_set_num_threads is the calling thread's, too)
 }  // namespace
 
 void set_threads(int n) {
-    g_threads_asked = n;
+    t_threads_asked = n;
     omp_set_num_threads(n > 0 ? n : g_threads_at_start);
 }
 int thread_limit() {
     const int n = omp_get_max_threads();
-    return n == g_threads_asked || n != g_threads_at_start ? n : (3 * n + 3) / 4;
+    return n == t_threads_asked || n != g_threads_at_start ? n : (3 * n + 3) / 4;
 }
 int threads_for(size_t entries) { return (int) std::max<size_t>(1, std::min<size_t>((size_t) thread_limit(), entries / 32768)); }
 

@@ -60,6 +60,6 @@ private:
 // stops the process for tens of milliseconds (epsilon-SVR 40000x90 with 16 threads on 16 CPUs: one call in
 // three takes 78 to 190 ms in place of 75).
 int thread_limit();
-void set_threads(int n);   // -o, n_jobs; 0: nobody has asked
+void set_threads(int n);   // -o, n_jobs, for the calling thread's regions; 0: nobody has asked
 // Threads that pay for a loop over `entries` row entries: a parallel region costs some ten microseconds to enter.
 int threads_for(size_t entries);
