@@ -149,8 +149,7 @@ __device__ __forceinline__ bool sel_side_descending(int side, int n_sides) { ret
 // guide was; if it does not fit the list, the digits are resolved from the first by sel_final_kernel's tail, which says so
 // (`missed`; none of the 5,000 selections of seven classes of 300,000 rows but one, two of 98 of 20,000 x 784), and the caller asks
 // for a selection by digits for a while.  Two launches less per outer iteration: epsilon-SVR 40000x90 69.4 -> 66.8 ms a call,
-// 30,000 blobs of which thousands share a value 25.0 -> 21.4, seven classes of 300,000 rows, where every launch waits among other
-// lanes', 913 -> 852.  Bins from the first entry on instead, in units of the k-th's distance, missed where the candidates
+// 30,000 blobs of which thousands share a value 25.0 -> 21.4; seven classes of 300,000 rows within what their runs differ by.  Bins from the first entry on instead, in units of the k-th's distance, missed where the candidates
 // crowd around the k-th (five of 42 of 20,000 x 784, 43.2 -> 44.1 ms).
 struct SelGuide {
     double at, scale;

@@ -427,7 +427,7 @@ __device__ __forceinline__ bool ss_local(SmallShared<E, W> &sh, const SmallMap &
         const double q2 = (-up_value + f_j) / __builtin_fma(-2.0, (double) k_ij, kd_i2 + kd_j);
         const double l = fmin_f64(bound_i.hi - z_i, fmin_f64(z_j - bound_j.lo, q2));
         const double nz_i = z_i + l, nz_j = (j2 == i ? nz_i : z_j) - l;
-        // (150x4 0.437 -> 0.417 ms a call, nu-SVC of 600 rows 1.41 -> 1.37, against a shifted field, a comparison and a selection for each)
+        // (nu-SVC of 600 rows 1.41 -> 1.37 ms a call, against a shifted field, a comparison and a selection for each)
         const unsigned up_bit_i = own_bit<E, 2 * NP>(tid, i) << (NU && i >= map.n0p ? 1 : 0), up_bit_j = own_bit<E, 2 * NP>(tid, j2) << (NU && j2 >= map.n0p ? 1 : 0);
         const unsigned up_i_on = same_in_all_lanes(nz_i < bound_i.hi), low_i_on = same_in_all_lanes(nz_i > bound_i.lo);
         const unsigned up_j_on = same_in_all_lanes(nz_j < bound_j.hi), low_j_on = same_in_all_lanes(nz_j > bound_j.lo);

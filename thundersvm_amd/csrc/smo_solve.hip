@@ -220,6 +220,13 @@ __device__ __forceinline__ bool solver_elected(int *gate, int epoch, int target_
 // into its L2 before they leave (in place of warm_block_kernel, 10 us in front of the solver).  `started` tells the host that
 // the solver has its CU: rows that take the other CUs before that keep those workgroups, and with them the block, out
 // (20000 x 784, solver beside 340 us of rows 337 us, 427 when they came first).
+// The launch has ended when every workgroup has found a CU with all of its LDS free: beside kernels of other streams, the caller's own
+// or another solve's, it waits for more than eight workgroups on CUs of their own did, each of which waited at two markers, though.  A
+// call in ms, when the solver had a stream of its own / now (the steps themselves are 10 % shorter now):
+//   beside                          nothing      products of 2,048    of 6,144 (bf16)   copies of 256 MB   another call
+//   epsilon-SVR 40000x90          78.6 / 65.9       203 /   84          249 /  121         266 / 139         159 / 134
+//   nu-SVC 5001x23                3.50 / 3.08      4.46 / 3.89         11.0 / 10.4        7.98 / 7.14       7.00 / 6.03
+//   C-SVC 20000x784               34.1 / 31.6      44.4 / 38.0         76.0 / 72.4        70.8 / 62.9       69.8 / 65.0
 #define TSVM_SOLVER_GRID_ON_CU 256
 __device__ __forceinline__ bool solver_elected_on_cu(int *gate, int epoch, bool on_target, int *started) {
     __shared__ int s_elected;
