@@ -13,6 +13,7 @@
 #include "../../thundersvm_amd/host/dataset.h"
 #include "../../thundersvm_amd/host/device.h"
 #include "../../thundersvm_amd/host/kernelmatrix.h"
+#include "../../thundersvm_amd/host/models.h"
 #include "../../thundersvm_amd/host/row_cache.h"
 #include "../../thundersvm_amd/host/rows.h"
 #include "../../thundersvm_amd/host/solver.h"
@@ -257,6 +258,33 @@ int tsvm_selftest_chip_split(int features, int ws, long long n, long long m_befo
     using tsvm::ChipSplit;
     const bool beside = ChipSplit::block_beside_rows(features, ws, ChipSplit::rows_seconds(features, m_before, n));
     return (beside ? 1 : 0) | (ChipSplit::warm_behind_rows(beside, ChipSplit::rows_seconds(features, m_now, n)) ? 2 : 0);
+}
+
+// The marks of n_classes classes with `each` instances and c % 3 more in class c, whose instance l of pair (i, j) is a support vector where
+// (l + 3 i + 7 j) % 11 is 0: the time that takes on one thread in us, or -1 if one is wrong.
+double tsvm_selftest_mark_support_vectors(int n_classes, int each) {
+    std::vector<int> count(n_classes), start(n_classes);
+    int n = 0;
+    for (int c = 0; c < n_classes; ++c) {
+        start[c] = n;
+        count[c] = each + c % 3;
+        n += count[c];
+    }
+    std::vector<std::vector<double>> alpha;
+    std::vector<unsigned char> want(n, 0);
+    for (int i = 0; i < n_classes; ++i)
+        for (int j = i + 1; j < n_classes; ++j) {
+            alpha.emplace_back(count[i] + count[j], 0.0);
+            for (int l = 0; l < count[i] + count[j]; ++l)
+                if ((l + 3 * i + 7 * j) % 11 == 0) {
+                    alpha.back()[l] = l % 2 ? 0.5 : -0.5;
+                    want[l < count[i] ? start[i] + l : start[j] + l - count[i]] = 1;
+                }
+        }
+    const auto t0 = std::chrono::steady_clock::now();
+    const std::vector<unsigned char> got = tsvm::mark_support_vectors(count, start, alpha, 1);
+    const double us = std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count();
+    return got == want ? us : -1;
 }
 
 // Whether an iteration's rows go ahead of the block and the solver, when the previous one computed m_before rows of n values.

@@ -28,5 +28,7 @@ def lib():
         L.tsvm_selftest_rows_ahead.argtypes = [ctypes.c_int] * 3 + [ctypes.c_longlong] * 2
         L.tsvm_selftest_thread_limit.argtypes = [ctypes.c_int] * 2
         L.tsvm_selftest_guided.argtypes = [ctypes.c_longlong, ctypes.c_int, ctypes.c_int]
+        L.tsvm_selftest_mark_support_vectors.restype = ctypes.c_double
+        L.tsvm_selftest_mark_support_vectors.argtypes = [ctypes.c_int] * 2
         _LIB = L
     return _LIB

@@ -44,3 +44,13 @@ def test_guides_that_fail_cost_little(n):
 
 def test_no_guides_for_many_instances():
     assert selftest_lib.lib().tsvm_selftest_guided((1 << 20) + 1, 1000, 0) == 0
+
+
+@pytest.mark.parametrize("classes,each", [(1, 3), (2, 1), (3, 5), (7, 40), (150, 2)])
+def test_marks_of_support_vectors(classes, each):
+    assert selftest_lib.lib().tsvm_selftest_mark_support_vectors(classes, each) >= 0
+
+
+def test_marks_take_time_with_the_pairs():
+    """Two million pairs are gone through twice, once for each class (0.1 s), and not once for every class (3.6 s)."""
+    assert 0 <= selftest_lib.lib().tsvm_selftest_mark_support_vectors(2000, 1) < 1e6

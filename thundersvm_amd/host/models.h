@@ -11,6 +11,13 @@
 #include "solver.h"
 #include "svmparam.h"
 
+namespace tsvm {
+// Whether an instance is a support vector of any class pair, by place in the grouped order: `count` and `start` of the classes, alpha of
+// the pairs (0, 1), (0, 2) ... each its two classes' instances one after the other.
+std::vector<unsigned char> mark_support_vectors(const std::vector<int> &count, const std::vector<int> &start, const std::vector<std::vector<float_type>> &alpha,
+                                                int threads);
+}  // namespace tsvm
+
 class SvmModel {
 public:
     virtual ~SvmModel() = default;
