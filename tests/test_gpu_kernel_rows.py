@@ -648,6 +648,35 @@ def test_indicator_columns(n, n_cont, groups, m, name, kt, prm):
     _check(name, G.host(outb), want[:, cols])
 
 
+@pytest.mark.parametrize("most", [2, 3, 5, 64])
+@pytest.mark.parametrize("n,n_cont,n_ind,m", [(517, 5, 64, 67), (130, 17, 31, 64)])
+def test_indicator_columns_with_any_number_of_ones(n, n_cont, n_ind, m, most):
+    """Rows that set 0 .. `most` of the 0/1 columns, the first and the last among them: every count up to the largest, more additions
+    than are unrolled, tiles with fewer rows and columns than a whole one; the bits of the oracle's serial chain."""
+    rng = np.random.default_rng(most * 100 + n)
+    most = min(most, n_ind)
+    x = np.zeros((n, n_cont + n_ind), dtype=np.float32)
+    x[:, :n_cont] = rng.standard_normal((n, n_cont))
+    for r in range(n):
+        x[r, n_cont + rng.permutation(n_ind)[:rng.integers(0, most + 1)]] = 1
+    x[:3, n_cont:] = 0
+    x[:2, [n_cont, n_cont + n_ind - 1]] = 1                 # two rows that share the ends
+    x[3, n_cont + rng.permutation(n_ind)[:most]] = 1
+    data = from_dense(x)
+    p = O.make_param(kernel_type=O.RBF, expf_mode=1, gamma=0.3)
+    x_d, nf, ld, sd, diag = _device_km(data, O.RBF, dict(gamma=0.3))
+    first = 1 + n_cont
+    masks = torch.zeros(n, dtype=torch.int64, device="cuda")
+    max_ones = torch.zeros(1, dtype=torch.int32, device="cuda")
+    capi.call("tsvm_indicator_masks", G.ptr(x_d), ld, n, first, nf - first, G.ptr(masks), G.ptr(max_ones), G.stream())
+    idx = rng.integers(0, n, size=m).astype(np.int32)
+    idx[:4] = [0, 1, 2, 3]
+    out = torch.full((m, n), -3.0, dtype=torch.float64, device="cuda")
+    capi.call("tsvm_get_rows_dense_indicator", G.ptr(x_d), ld, None, n, first, G.ptr(sd), G.ptr(masks), G.ptr(x_d), ld, G.ptr(G.dev(idx)), m, None,
+              G.ptr(sd), G.ptr(masks), int(G.host(max_ones)[0]), O.RBF, 0.3, 0.0, 3, G.ptr(out), capi.ROW_F64, None, n, G.stream())
+    _check("rbf", G.host(out), O.KernelMatrix(data.ptr, data.col, data.val, p).get_rows(idx))
+
+
 @pytest.mark.parametrize("m", [1, 64, 65, 200])
 def test_symmetric_block_with_indicator_columns(m):
     """Both sides the same rows, with masks: the bits of the plain call on all columns."""

@@ -73,9 +73,10 @@ __global__ __launch_bounds__(256, 3) void get_rows_dense_stream_kernel(
     // wavefront may stage the next tile's while another still reads this tile's in its epilogue)
     __shared__ double s_sdi[BM];
     __shared__ uint64_t s_mi[BM];
-    __shared__ int s_slot[BM];
+    __shared__ uint64_t s_row[BM];   // where the row is in `out`, in elements
     __shared__ double s_sdj[2][GR_BN];
     __shared__ uint64_t s_mj[2][GR_BN];
+    __shared__ uint64_t ind_tab[IND >= 2 ? IND_TAB : 1];
     KernelParam kp = kp_in;
     kp.kernel_type = KT;
     const unsigned logical = xcd_remap(blockIdx.x, gridDim.x);
@@ -102,10 +103,11 @@ __global__ __launch_bounds__(256, 3) void get_rows_dense_stream_kernel(
     const int b_col = (b_row & 64) + ((b_row & 15) << 2) + ((b_row >> 4) & 3);   // column (in the tile) staged by this thread
 
     if (tid < 32) exp_tab[tid] = TSVM_EXP2F_TAB[tid];
+    if constexpr (IND >= 2) ind_tab[tid] = indicator_tab_entry((unsigned) tid);
     if (tid < BM) {
         const int r = min(i0 + tid, m_last);
         const int id = a_idx ? a_idx[r] : r;
-        s_slot[tid] = out_slots ? out_slots[r] : r;
+        s_row[tid] = (uint64_t) (uint32_t) (out_slots ? out_slots[r] : r) * (uint32_t) ldo;
         s_sdi[tid] = sd_a ? sd_a[id] : 0.0;
         s_mi[tid] = IND ? mask_a[id] : 0;
     }
@@ -259,25 +261,12 @@ __global__ __launch_bounds__(256, 3) void get_rows_dense_stream_kernel(
 #pragma unroll
         for (int tj = 0; tj < 4; ++tj) {
             sdj[tj] = s_sdj[gen][wj * 64 + lrow * 4 + tj];
-            mj[tj] = IND ? s_mj[gen][wj * 64 + lrow * 4 + tj] : 0;
+            mj[tj] = IND == 1 ? s_mj[gen][wj * 64 + lrow * 4 + tj] : 0;
         }
-        // one value: the indicator columns' share, then the kernel function.  IND = 1..4: that many additions,
-        // unrolled (the addend is 1.0 or 0.0: no branch); IND = 5: max_ones of them in a loop
-        auto with_indicators = [&](double dot, uint64_t mi, int tj) -> double {
-            if (IND) {
-                const int cnt = __popcll(mi & mj[tj]);
-                if (IND <= 4) {
-#pragma unroll
-                    for (int t = 0; t < IND; ++t) dot += cnt > t ? 1.0 : 0.0;
-                } else {
-                    for (int t = 0; t < max_ones; ++t) dot += cnt > t ? 1.0 : 0.0;
-                }
-            }
-            return dot;
-        };
-        auto finish = [&](double dot, double sdi, uint64_t mi, int tj) -> TO {
-            return tsvm_epilogue_as<TO>(with_indicators(dot, mi, tj), sdi, sdj[tj], kp, exp_tab);
-        };
+        // the indicator columns' share, then one value at a time the kernel function
+        if constexpr (IND >= 2) add_indicators<IND, TI>(acc, s_mi + wi * (16 * TI), s_mj[gen] + wj * 64, lrow, lk, max_ones, ind_tab);
+        auto dot_of = [&](int ti, int v, uint64_t mi, int tj) { return IND == 1 ? one_indicator(acc[ti][tj][v], mi, mj[tj]) : acc[ti][tj][v]; };
+        auto finish = [&](double dot, double sdi, int tj) -> TO { return tsvm_epilogue_as<TO>(dot, sdi, sdj[tj], kp, exp_tab); };
         // interior tiles store without a test, four columns at a time; edge tiles (and outputs whose rows are not
         // 16-byte aligned) test and store every element
         typedef TO vec4_t __attribute__((ext_vector_type(4)));
@@ -288,8 +277,8 @@ __global__ __launch_bounds__(256, 3) void get_rows_dense_stream_kernel(
                 for (int v = 0; v < 4; ++v) {
                     const int r = wi * (16 * TI) + ti * 16 + 4 * v + lk;   // row of the tile
                     const double sdi = s_sdi[r];
-                    const uint64_t mi = IND ? s_mi[r] : 0;
-                    TO *orow = out + (int64_t) ((uint64_t) (uint32_t) s_slot[r] * (uint32_t) ldo) + jb;
+                    const uint64_t mi = IND == 1 ? s_mi[r] : 0;
+                    TO *orow = out + s_row[r] + jb;
                     vec4_t res;
                     if constexpr (KT == TSVM_RBF && sizeof(TO) == 4) {
                         // expf's two out-of-range cases cost four instructions per value; one look at the largest
@@ -297,7 +286,7 @@ __global__ __launch_bounds__(256, 3) void get_rows_dense_stream_kernel(
                         // any value of this store needs them.  Every instruction saved is an issue slot for the MFMAs.
                         float xs[4];
 #pragma unroll
-                        for (int tj = 0; tj < 4; ++tj) xs[tj] = tsvm_rbf_arg(with_indicators(acc[ti][tj][v], mi, tj), sdi, sdj[tj], kp);
+                        for (int tj = 0; tj < 4; ++tj) xs[tj] = tsvm_rbf_arg(dot_of(ti, v, mi, tj), sdi, sdj[tj], kp);
                         const float mx = fmaxf(fmaxf(fabsf(xs[0]), fabsf(xs[1])), fmaxf(fabsf(xs[2]), fabsf(xs[3])));
                         if (__builtin_amdgcn_ballot_w64(mx > 88.0f) == 0) {
 #pragma unroll
@@ -308,7 +297,7 @@ __global__ __launch_bounds__(256, 3) void get_rows_dense_stream_kernel(
                         }
                     } else {
 #pragma unroll
-                        for (int tj = 0; tj < 4; ++tj) res[tj] = finish(acc[ti][tj][v], sdi, mi, tj);
+                        for (int tj = 0; tj < 4; ++tj) res[tj] = finish(dot_of(ti, v, mi, tj), sdi, tj);
                     }
                     store_streaming((vec4_t *) orow, res);
                 }
@@ -321,11 +310,11 @@ __global__ __launch_bounds__(256, 3) void get_rows_dense_stream_kernel(
                     const int r = wi * (16 * TI) + ti * 16 + 4 * v + lk;
                     if (i0 + r >= m) continue;
                     const double sdi = s_sdi[r];
-                    const uint64_t mi = IND ? s_mi[r] : 0;
-                    TO *orow = out + (int64_t) ((uint64_t) (uint32_t) s_slot[r] * (uint32_t) ldo) + jb;
+                    const uint64_t mi = IND == 1 ? s_mi[r] : 0;
+                    TO *orow = out + s_row[r] + jb;
 #pragma unroll
                     for (int tj = 0; tj < 4; ++tj)
-                        if (jb + tj < n) orow[tj] = finish(acc[ti][tj][v], sdi, mi, tj);   // (single values: left to the L2 to merge)
+                        if (jb + tj < n) orow[tj] = finish(dot_of(ti, v, mi, tj), sdi, tj);   // (single values: left to the L2 to merge)
                 }
             }
         }
@@ -375,7 +364,7 @@ __global__ __launch_bounds__(512) void get_rows_dense_sym_kernel(
     __shared__ double s_sd[2][SYM_B];
     __shared__ uint64_t exp_tab[32];
     static_assert(SYM_B * (SYM_B + 1) <= 2 * SYM_K * SYM_LS, "the values take the staged columns' place");
-    static_assert(sizeof(s_tile) + sizeof(s_sd) + sizeof(exp_tab) <= 160 * 1024 - 3 * 38656, "room beside three of get_rows' workgroups");
+    static_assert(sizeof(s_tile) + sizeof(s_sd) + sizeof(exp_tab) <= 160 * 1024 - 3 * 40960, "room beside three of get_rows' workgroups");
     KernelParam kp = kp_in;
     kp.kernel_type = KT;
     const int c = (int) blockIdx.x;

@@ -59,6 +59,7 @@ __global__ __launch_bounds__(256, 2) void predict_dense_stream_kernel(
     // reads this tile's)
     __shared__ double s_sdj[2][GR_BN];
     __shared__ uint64_t s_mj[2][GR_BN];
+    __shared__ uint64_t ind_tab[IND >= 2 ? IND_TAB : 1];
     __shared__ __attribute__((aligned(16))) double s_coef[2][NC][GR_BN];
     KernelParam kp = kp_in;
     kp.kernel_type = KT;
@@ -93,6 +94,7 @@ __global__ __launch_bounds__(256, 2) void predict_dense_stream_kernel(
     const int b_col = (b_row & 64) + ((b_row & 15) << 2) + ((b_row >> 4) & 3);
 
     if (tid < 32) exp_tab[tid] = TSVM_EXP2F_TAB[tid];
+    if constexpr (IND >= 2) ind_tab[tid] = indicator_tab_entry((unsigned) tid);
     if (tid < BM) {
         const int r = batch_row(i0 + tid);
         s_sdi[tid] = sd_a ? sd_a[r] : 0.0;
@@ -222,33 +224,20 @@ __global__ __launch_bounds__(256, 2) void predict_dense_stream_kernel(
 #pragma unroll
         for (int tj = 0; tj < 4; ++tj) {
             sdj[tj] = s_sdj[gen][wj * 64 + lrow * 4 + tj];
-            mj[tj] = IND ? s_mj[gen][wj * 64 + lrow * 4 + tj] : 0;
+            mj[tj] = IND == 1 ? s_mj[gen][wj * 64 + lrow * 4 + tj] : 0;
         }
-        // the indicator columns' share of a dot product: 1.0 once per column both rows have set, one addition at a
-        // time (the serial chain over those columns, bit for bit).  IND = 1..4: that many additions, IND = 5: max_ones of them in a
-        // loop, which as the only form took the RBF kernel of a seven-class model (16,076 support vectors, 50,000 rows) 1.76 ms, not 1.65.
-        auto with_indicators = [&](double dot, uint64_t mi, int tj) -> double {
-            if (IND) {
-                const int cnt = __popcll(mi & mj[tj]);
-                if (IND <= 4) {
-#pragma unroll
-                    for (int t = 0; t < IND; ++t) dot += cnt > t ? 1.0 : 0.0;
-                } else {
-                    for (int t = 0; t < max_ones; ++t) dot += cnt > t ? 1.0 : 0.0;
-                }
-            }
-            return dot;
-        };
+        auto dot_of = [&](int ti, int v, uint64_t mi, int tj) { return IND == 1 ? one_indicator(acc[ti][tj][v], mi, mj[tj]) : acc[ti][tj][v]; };
+        if constexpr (IND >= 2) add_indicators<IND, TI>(acc, s_mi + wi * (16 * TI), s_mj[gen] + wj * 64, lrow, lk, max_ones, ind_tab);
         // one batch row's four kernel values, widened to double as the reference widens them before its sums
         auto row_values = [&](int ti, int v, double *kv) {
             const int r = wi * (16 * TI) + ti * 16 + 4 * v + lk;
             const double sdi = s_sdi[r];
-            const uint64_t mi = IND ? s_mi[r] : 0;
+            const uint64_t mi = IND == 1 ? s_mi[r] : 0;
             if constexpr (KT == TSVM_RBF) {
                 // expf's two out-of-range cases only where some argument of the wavefront needs them
                 float xs[4];
 #pragma unroll
-                for (int tj = 0; tj < 4; ++tj) xs[tj] = tsvm_rbf_arg(with_indicators(acc[ti][tj][v], mi, tj), sdi, sdj[tj], kp);
+                for (int tj = 0; tj < 4; ++tj) xs[tj] = tsvm_rbf_arg(dot_of(ti, v, mi, tj), sdi, sdj[tj], kp);
                 const float mx = fmaxf(fmaxf(fabsf(xs[0]), fabsf(xs[1])), fmaxf(fabsf(xs[2]), fabsf(xs[3])));
                 if (__builtin_amdgcn_ballot_w64(mx > 88.0f) == 0) {
 #pragma unroll
@@ -259,7 +248,7 @@ __global__ __launch_bounds__(256, 2) void predict_dense_stream_kernel(
                 }
             } else {
 #pragma unroll
-                for (int tj = 0; tj < 4; ++tj) kv[tj] = tsvm_epilogue(with_indicators(acc[ti][tj][v], mi, tj), sdi, sdj[tj], kp, exp_tab);
+                for (int tj = 0; tj < 4; ++tj) kv[tj] = tsvm_epilogue(dot_of(ti, v, mi, tj), sdi, sdj[tj], kp, exp_tab);
             }
         };
         auto coef_of = [&](int c, double *cj) {   // coefficient row c of this lane's four columns
