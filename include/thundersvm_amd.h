@@ -472,6 +472,17 @@ int tsvm_predict_dec_values_dense(const double *sv_x, int64_t ldx, int d, const 
                                   int max_ones, int kernel_type, double gamma, double coef0, int degree, double *partial,
                                   double *dec_values, tsvm_stream stream);
 
+/* The sums per 128 columns for a request of a few rows in one launch.  rows (8-byte aligned host memory): rows[m][d] with sv_x's columns, indicator columns
+ * among them, then from the next multiple of eight bytes the rows' self dot products as m doubles, tsvm_predict_few_rows_bytes(m, d) in
+ * all (0: more columns than the kernel takes).  What fits travels with the launch and has been read when the call returns; what
+ * does not is read by the kernel at rows_device, the same memory as the device sees it (may be NULL otherwise).  coef_t as above, nc <= 8
+ * coefficient rows at a stride of coef_stride.  partial[(tile * m + r) * nc + c]: what tsvm_predict_dec_values_dense leaves there with
+ * one tile per chunk, bit for bit, each written once; adding the tiles is the caller's (partial may be device-mapped host memory). */
+size_t tsvm_predict_few_rows_bytes(int m, int d);
+int tsvm_predict_few_rows(const double *sv_x, int64_t ldx, int d, const double *sd_sv, const int *col_map, int64_t n_pad, const double *coef_t,
+                          int coef_stride, int nc, const float *rows, const float *rows_device, int m, int kernel_type, double gamma, double coef0,
+                          int degree, double *partial, tsvm_stream stream);
+
 /* The same for several groups of rows in one launch, each with a model of its own whose support vectors are rows of the same dense matrix
  * x as the rows themselves (the folds of a cross-validation: the reference predicts them one after another,
  * src/thundersvm/model/svmmodel.cpp:50-66).  All models have n_classes classes; d <= 128, all columns through the matrix cores.

@@ -447,3 +447,35 @@ def test_groups_of_rows_in_one_launch(k, d, kernel):
     capi.call("tsvm_predict_groups_dense", G.ptr(x_d), ldx, d, G.ptr(sd_d), G.ptr(held[0]), len(cols), G.ptr(held[1]), G.ptr(held[2]), G.ptr(held[3]), len(tasks),
               G.ptr(held[4]), len(rows), G.ptr(held[5]), G.ptr(held[6]), G.ptr(held[7]), k, *args, G.ptr(part_d), G.ptr(dec_d), G.stream())
     assert np.array_equal(G.host(dec_d), want)
+
+
+@pytest.mark.parametrize("k,d,hot,kernel", [(2, 1, 0, capi.RBF), (2, 32, 0, capi.RBF), (3, 33, 0, capi.POLY), (4, 60, 0, capi.SIGMOID), (9, 127, 0, capi.LINEAR),
+                                            (7, 5, 40, capi.RBF), (2, 12, 64, capi.LINEAR), (10, 4, 0, capi.RBF), (2, 150, 0, capi.RBF)])
+def test_requests_of_a_few_rows(k, d, hot, kernel):
+    """A few rows in one launch against the same rows as part of a batch that takes the kernels for many: the same bits, whatever of
+    the batch's rows a request asks for; ten classes and 150 columns take the other route."""
+    rng = np.random.default_rng(1000 * k + d)
+    x, y = _blobs(rng, k, 260 // k + 20, d, one_hot=hot)
+    xt, _ = _blobs(np.random.default_rng(2000 * k + d), k, 100 // k, d, one_hot=hot)
+    xt[3] = 0.0
+    gm = Model(0).train(D.from_dense(x, y), make_param(svm_type=0, kernel_type=kernel, gamma=0.5 / d, coef0=0.1, degree=2, C=3.0))
+    lab, dec = gm.predict(D.from_dense(xt, np.zeros(len(xt))))
+    for first, m in [(0, 1), (3, 1), (0, 2), (5, 3), (1, 4), (2, 5), (0, 7), (1, 8), (0, 9), (7, 15), (4, 16), (0, 17)]:
+        l, v = gm.predict(D.from_dense(xt[first:first + m], np.zeros(m)))
+        assert np.array_equal(v, dec[first:first + m]) and np.array_equal(l, lab[first:first + m]), (first, m)
+
+
+def test_requests_of_a_few_rows_that_are_not_plain_floats():
+    """Values that are no floats, infinite ones, and columns that no support vector has: what the kernels for many rows give."""
+    rng = np.random.default_rng(5)
+    x, y = _blobs(rng, 2, 150, 6)
+    gm = Model(0).train(D.from_dense(x, y), make_param(svm_type=0, kernel_type=2, gamma=0.1, C=3.0))
+    rows = np.concatenate([x[:40].astype(np.float64), 3.0 * rng.standard_normal((40, 6))])
+    rows[1, 2], rows[2, 0] = 0.1, np.inf
+    xt = np.zeros((80, 9))
+    xt[:, :6], xt[5, 8], xt[7, 7] = rows, 2.5, 1e-3
+    ptr, col = np.arange(81, dtype=np.int64) * 9, np.tile(np.arange(1, 10, dtype=np.int32), 80)
+    _, dec = gm.predict(D.CsrData(ptr, col, xt.reshape(-1), np.zeros(80)))
+    for first, m in [(0, 1), (1, 1), (2, 1), (0, 8), (3, 5), (41, 3), (70, 10)]:
+        _, v = gm.predict(D.CsrData(ptr[:m + 1], col[:9 * m], xt[first:first + m].reshape(-1).copy(), np.zeros(m)))
+        assert np.array_equal(v, dec[first:first + m], equal_nan=True), (first, m)

@@ -86,6 +86,8 @@ SIGNATURES = {
     "tsvm_predict_nc_stride": (_int, [_int, _int, _int]),
     "tsvm_predict_dec_values_dense": (_int, [_p, _i64, _int, _p, _p, _p, _i64, _p, _p, _int, _p, _p, _int, _p, _i64, _i64, _p, _p,
                                              _int, _int, _dbl, _dbl, _int, _p, _p, _p]),
+    "tsvm_predict_few_rows_bytes": (C.c_size_t, [_int, _int]),
+    "tsvm_predict_few_rows": (_int, [_p, _i64, _int, _p, _p, _i64, _p, _int, _int, _p, _p, _int, _int, _dbl, _dbl, _int, _p, _p]),
     "tsvm_predict_groups_dense": (_int, [_p, _i64, _int, _p, _p, _i64, _p, _p, _p, _int, _p, _i64, _p, _p, _p, _int, _int, _dbl, _dbl, _int, _p, _p, _p]),
 }
 

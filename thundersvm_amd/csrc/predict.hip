@@ -16,6 +16,7 @@
 #include "tsvm_internal.h"
 
 #include <algorithm>
+#include <cstring>
 
 #include "get_rows_tile.h"
 
@@ -28,7 +29,7 @@ typedef double v2d __attribute__((ext_vector_type(2)));
 // ------------------------------------------------------------------------------------------------
 // Groups of rows that have their own support vectors come with a table of who does what and their rows by number.  A variant of its
 // own: as two pointers that are mostly null, every workgroup waited for the loads behind them to be ruled out before it
-// asked for its rows (a request of three rows 35.9 -> 36.2 us).
+// asked for its rows (a request of three rows, when those came this way, 35.9 -> 36.2 us).
 template <bool GROUPS>
 struct StreamGroups {
     const tsvm_predict_task *tasks;
@@ -354,6 +355,120 @@ __global__ __launch_bounds__(256, 2) void predict_dense_tile_kernel(
     }
 }
 
+// ------------------------------------------------------------------------------------------------
+// A request of a few rows: one launch in place of three (rows laid out dense, kernel values, classes' sums).
+//
+// Nothing in it is long, so what counts is the launches and the dependent reads in front of the arithmetic.  The rows come among the
+// kernel's own arguments, or as many as do not fit there from page-locked host memory in one read; a workgroup takes four of them
+// and 128 support vectors, a lane per support vector, which asks for 32 of its columns at a time; and the sums per tile of
+// 128 columns go straight to page-locked memory, where the host adds them (a workgroup that waited for the others would cost more
+// than those few additions).  No matrix cores: so few rows give them a fraction of their work, and a lane's chain of fmas over the
+// columns is the same serial sum.
+//
+// The sums have the order of predict_dense_stream_kernel with one tile per chunk: a quad of lanes is one of its lanes (four
+// consecutive columns, one fma after another), sixteen quads are its row of sixteen lanes, a wavefront one of its two wavefront
+// columns.  The same bits.  Three rows, 2,000 support vectors of 32 columns: 36 us a call by three launches, 24 by one, 19 without
+// the runtime's wait behind it (ResultBlock::wait_for).
+// ------------------------------------------------------------------------------------------------
+#define FEW_R 4              // rows of a workgroup
+#define FEW_ARGS 896         // values of a launch's 4 KB of arguments
+#define FEW_ARGS_SMALL 224   // (the runtime copies what a launch has: 1 KB)
+#define FEW_K 32             // columns of its support vector that a lane asks for at a time
+#define FEW_D 192            // columns at most
+
+// [m][d] values as floats, then m self dot products as doubles, at a multiple of eight bytes
+template <int N>
+struct __attribute__((aligned(8))) FewRows {
+    float v[N];
+    __device__ __forceinline__ const float *values() const { return v; }
+};
+template <>
+struct FewRows<0> {
+    const float *p;
+    __device__ __forceinline__ const float *values() const { return p; }
+};
+
+// lane `from` of a quad's value in all four of its lanes
+template <int FROM>
+__device__ __forceinline__ double quad_lane(double v) { return dpp_f64<FROM * 0x55>(v); }
+
+template <int KT, int N>
+__global__ __launch_bounds__(128) void predict_few_kernel(const double *__restrict__ x, int64_t ldx, const int *__restrict__ col_map, int d,
+                                                          const double *__restrict__ sd_x, const FewRows<N> rows, int m, KernelParam kp_in,
+                                                          const double *__restrict__ coef_t, int stride, int nc, double *__restrict__ partial) {
+    constexpr int R = FEW_R;
+    __shared__ __attribute__((aligned(16))) double s_a[FEW_D * R];   // [column][row]
+    __shared__ double s_sd[R];
+    __shared__ uint64_t exp_tab[32];
+    __shared__ double s_sum[2][R * 8];
+    KernelParam kp = kp_in;
+    kp.kernel_type = KT;
+    const int tid = threadIdx.x, lane = tid & 63, wj = tid >> 6;
+    const int p = (int) blockIdx.x * GR_BN + tid, r0 = (int) blockIdx.y * R;
+    const int d4 = (d + 3) & ~3;
+    const int col = col_map[p];
+    double cj[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) cj[c] = c < nc ? coef_t[(int64_t) p * stride + c] : 0.0;
+    const double *xr = x + (uint64_t) (uint32_t) col * (uint32_t) ldx;
+    const int k_last = (int) ldx - 4;   // (rows are padded to a multiple of eight columns)
+    v4d xv[FEW_K / 4];
+    auto request = [&](int k0) {
+#pragma unroll
+        for (int q = 0; q < FEW_K / 4; ++q) xv[q] = *(const v4d *) (xr + min(k0 + 4 * q, k_last));
+    };
+    request(0);
+    const double sdj = sd_x ? sd_x[col] : 0.0;
+    if (tid < 32) exp_tab[tid] = TSVM_EXP2F_TAB[tid];
+    const float *const v = rows.values();
+    if (tid < R) s_sd[tid] = r0 + tid < m ? ((const double *) (v + ((m * d + 1) & ~1)))[r0 + tid] : 0.0;
+    for (int e = tid; e < R * d4; e += 128) {
+        const int k = e / R, r = r0 + e % R;
+        s_a[e] = r < m && k < d ? (double) v[r * d + k] : 0.0;
+    }
+    __syncthreads();
+    double acc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = 0.0;
+    for (int k0 = 0; k0 < d4; k0 += FEW_K) {
+        if (k0 > 0) request(k0);
+#pragma unroll
+        for (int q = 0; q < FEW_K / 4; ++q) {
+            if (k0 + 4 * q < d4) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int r = 0; r < R; ++r) acc[r] = __builtin_fma(s_a[(k0 + 4 * q + e) * R + r], xv[q][e], acc[r]);
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = tsvm_epilogue(acc[r], s_sd[r], sdj, kp, exp_tab);
+    for (int c = 0; c < nc; ++c) {
+        double w = cj[0];
+#pragma unroll
+        for (int u = 1; u < 8; ++u) w = c == u ? cj[u] : w;
+        const double w0 = quad_lane<0>(w), w1 = quad_lane<1>(w), w2 = quad_lane<2>(w), w3 = quad_lane<3>(w);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            double t = w0 * quad_lane<0>(acc[r]);
+            t = __builtin_fma(w1, quad_lane<1>(acc[r]), t);
+            t = __builtin_fma(w2, quad_lane<2>(acc[r]), t);
+            t = __builtin_fma(w3, quad_lane<3>(acc[r]), t);
+            t += dpp_f64<TSVM_DPP_HALF_MIRROR>(t);   // quads 0 and 1, 2 and 3 of sixteen lanes
+            t += dpp_f64<TSVM_DPP_MIRROR>(t);        // and those two pairs
+            t += shfl_xor_f64(t, 16);
+            t += shfl_xor_f64(t, 32);
+            if (lane == 0) s_sum[wj][r * 8 + c] = t;
+        }
+    }
+    __syncthreads();
+    if (tid < R * nc) {
+        const int r = tid / nc, c = tid % nc;
+        if (r0 + r < m) partial[((int64_t) blockIdx.x * m + r0 + r) * nc + c] = s_sum[0][r * 8 + c] + s_sum[1][r * 8 + c];
+    }
+}
+
 // dec[r * P + p] for pair p = (i < j): the chunks of class i under coefficient row j - 1, then the chunks of class j
 // under coefficient row i, each in chunk order, minus rho[p] (the order of kernelmatrix_kernel.cpp:129-143).  GROUPS: groups of
 // rows have class_chunk_start and rho of their own.
@@ -534,6 +649,58 @@ int tsvm_predict_dec_values_dense(const double *sv_x, int64_t ldx, int d, const 
     const int64_t P = (int64_t) n_classes * nc / 2;
     hipLaunchKernelGGL(predict_combine_kernel<false>, dim3((unsigned) ((m * P + 255) / 256)), block, 0, tsvm_s(stream), partial, m, nc,
                        class_chunk_start, rho, n_classes, nullptr, dec_values);
+    TSVM_LAUNCH_CHECK();
+    return 0;
+}
+
+size_t tsvm_predict_few_rows_bytes(int m, int d) {
+    if (m < 1 || d < 1 || d > FEW_D || (int64_t) m * d > (1 << 20)) return 0;
+    return (size_t) (((int64_t) m * d + 1) / 2 * 2 + 2 * m) * sizeof(float);
+}
+
+int tsvm_predict_few_rows(const double *sv_x, int64_t ldx, int d, const double *sd_sv, const int *col_map, int64_t n_pad, const double *coef_t,
+                          int coef_stride, int nc, const float *rows, const float *rows_device, int m, int kernel_type, double gamma, double coef0,
+                          int degree, double *partial, tsvm_stream stream) {
+    TSVM_REQUIRE(sv_x && col_map && coef_t && rows && partial, "tsvm_predict_few_rows: null pointer");
+    if (m == 0) return 0;
+    const size_t bytes = tsvm_predict_few_rows_bytes(m, d);
+    TSVM_REQUIRE(bytes > 0, "tsvm_predict_few_rows: %d rows of %d columns (1 .. %d)", m, d, FEW_D);
+    TSVM_REQUIRE(bytes <= FEW_ARGS * sizeof(float) || (rows_device && (uintptr_t) rows_device % 8 == 0),
+                 "tsvm_predict_few_rows: %d rows of %d columns do not fit a launch's arguments and are not in memory that the device reads", m, d);
+    TSVM_REQUIRE(nc >= 1 && nc <= 8 && coef_stride >= nc && n_pad >= 0 && n_pad % GR_BN == 0 && n_pad <= 0x7fff0000,
+                 "tsvm_predict_few_rows: %d coefficient rows (1 .. 8) at a stride of %d, %lld columns", nc, coef_stride, (long long) n_pad);
+    TSVM_REQUIRE(ldx % 8 == 0 && d <= ldx && ldx <= 0x7fffffff && (uintptr_t) sv_x % 32 == 0,
+                 "tsvm_predict_few_rows: ldx %lld (a multiple of 8, at least %d), sv_x 32-byte aligned", (long long) ldx, d);
+    TSVM_REQUIRE(kernel_type >= 0 && kernel_type <= 4, "tsvm_predict_few_rows: unknown kernel type %d", kernel_type);
+    TSVM_REQUIRE((kernel_type != TSVM_RBF && kernel_type != TSVM_PRECOMPUTED) || sd_sv, "tsvm_predict_few_rows: RBF needs self dot products");
+    const unsigned groups = (unsigned) (m + FEW_R - 1) / FEW_R;
+    TSVM_REQUIRE(groups <= 65535, "tsvm_predict_few_rows: %d rows", m);
+    if (n_pad == 0) return 0;
+    const KernelParam kp{kernel_type, degree, gamma, coef0};
+    const dim3 grid((unsigned) (n_pad / GR_BN), groups), block(128);
+#define PD_FEW(KTYPE, N)                                                                                                                       \
+    hipLaunchKernelGGL((predict_few_kernel<KTYPE, N>), grid, block, 0, tsvm_s(stream), sv_x, ldx, col_map, d, sd_sv, args, m, kp, coef_t, coef_stride, nc, partial)
+#define PD_FEW_KIND(N)                                      \
+    switch (kernel_type) {                                  \
+        case TSVM_LINEAR: PD_FEW(TSVM_LINEAR, N); break;    \
+        case TSVM_POLY: PD_FEW(TSVM_POLY, N); break;        \
+        case TSVM_SIGMOID: PD_FEW(TSVM_SIGMOID, N); break;  \
+        default: PD_FEW(TSVM_RBF, N); break;                \
+    }
+    if (bytes <= FEW_ARGS_SMALL * sizeof(float)) {
+        FewRows<FEW_ARGS_SMALL> args;
+        memcpy(args.v, rows, bytes);
+        PD_FEW_KIND(FEW_ARGS_SMALL)
+    } else if (bytes <= FEW_ARGS * sizeof(float)) {
+        FewRows<FEW_ARGS> args;
+        memcpy(args.v, rows, bytes);
+        PD_FEW_KIND(FEW_ARGS)
+    } else {
+        const FewRows<0> args{rows_device};
+        PD_FEW_KIND(0)
+    }
+#undef PD_FEW_KIND
+#undef PD_FEW
     TSVM_LAUNCH_CHECK();
     return 0;
 }

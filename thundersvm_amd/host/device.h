@@ -78,11 +78,20 @@ public:
     ResultBlock &operator=(const ResultBlock &) = delete;
     ~ResultBlock() { if (arrived_ || hipStreamSynchronize(stream_) == hipSuccess) give_pinned_block(block_); }
     char *dev() const { return block_.dev; }
+    char *host() const { return block_.host; }
+    void unused() { arrived_ = true; }   // nothing that is enqueued uses it (any more)
     const char *wait() {   // the result, on the host
         TSVM_HIP_CHECK(hipStreamSynchronize(stream_));
         arrived_ = true;
         return block_.host;
     }
+    // The same for `count` numbers that the kernels write one by one, each once, by looking at them: the runtime's own wait is some
+    // microseconds behind the last write.  expect() comes before the kernels; nothing that they compute is NOT_YET, a signalling NaN.
+    static constexpr uint64_t NOT_YET = 0x7ff4a5c3961e87d2ull;
+    void expect(size_t count) {
+        for (size_t i = 0; i < count; ++i) ((volatile uint64_t *) block_.host)[i] = NOT_YET;
+    }
+    const double *wait_for(size_t count);
 
 private:
     PinnedBlock block_;

@@ -183,6 +183,24 @@ void give_pinned_block(const PinnedBlock &b) {
     else (void) hipHostFree(b.host);
 }
 
+const double *ResultBlock::wait_for(size_t count) {
+    const volatile uint64_t *const word = (const volatile uint64_t *) block_.host;
+    const auto start = std::chrono::steady_clock::now();
+    size_t at = 0;
+    for (unsigned spins = 1; at < count; ++spins) {
+        if (word[at] != NOT_YET) {
+            ++at;
+        } else if (spins % 256 == 0 && std::chrono::steady_clock::now() - start > std::chrono::milliseconds(2)) {
+            wait();   // (behind other work, or the kernels have failed)
+            for (; at < count; ++at)
+                if (word[at] == NOT_YET) throw std::runtime_error("ResultBlock: the kernels finished without a result");
+        }
+    }
+    __atomic_thread_fence(__ATOMIC_ACQUIRE);
+    arrived_ = true;
+    return (const double *) block_.host;
+}
+
 DeviceEvent take_event() {
     HostPool &h = host_pool();
     DeviceEvent e;

@@ -120,6 +120,8 @@ protected:
     // one batch, rows already on the device as a dense matrix; false when the kernels do not take this model's shape
     bool predict_batch_fused(const PredictPlan &plan, const kernel_type *a, int64_t lda, const kernel_type *sd_a, size_t m,
                              bool indicator_values, float_type *dec_out, int *winner_out) const;
+    // a request of a few rows, taken from host memory by one launch; false when its shape or its values are not for it
+    bool predict_few(const PredictPlan &plan, const RowStore &rows, size_t first, size_t m, float_type *dec_out) const;
     // decision values of m rows and, behind them on the device, room for their winners when those are wanted: to the host
     void fetch_predictions(float_type *d_dec, size_t m, float_type *dec_out, int *winner_out) const;
     void copy_support_vectors(const RowStore &rows);

@@ -3,6 +3,7 @@
 // (tsvm_predict_dec_values_dense) and never written out; otherwise kernel rows per batch, then
 // tsvm_sum_kernel_values, as the reference does.
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <memory>
@@ -31,6 +32,12 @@ struct OneUpload {   // several arrays that go to the device in one copy, each a
     }
 };
 }  // namespace
+
+// A request of a few rows goes by one launch as long as its sums and its rows fit a page-locked block each and what the workgroups
+// read over the link, every row once per 128 support vectors, is no more than this.  Calls by one launch / by the kernels for many,
+// us: 770 support vectors of 32 columns, one row 19 / 34, 64 rows 24 / 37, 200 rows (0.2 MB) 35 / 61; 2,050, 64 rows 26 / 39;
+// 5,740 of 60 columns in six classes, 16 rows (0.2 MB) 29 / 45; 3,550 of 120, one row 25 / 46, 32 rows (0.48 MB) 35 / 53.
+constexpr size_t FEW_LINK_BYTES = (size_t) 512 << 10;
 
 struct SvmModel::PredictPlan {
     DeviceBuffer<char> arrays;      // all of the following, uploaded together
@@ -187,6 +194,54 @@ bool SvmModel::predict_batch_fused(const PredictPlan &P, const kernel_type *a, i
     return true;
 }
 
+bool SvmModel::predict_few(const PredictPlan &P, const RowStore &rows, size_t first, size_t m, float_type *dec_out) const {
+    const DeviceRows &R = sv_k_mat->rows();
+    const int d = (int) R.n_features, nc = n_classes - 1;
+    const size_t tiles = (size_t) P.n_pad / 128, sums = tiles * m * nc, in_bytes = m <= 4096 ? tsvm_predict_few_rows_bytes((int) m, d) : 0;
+    if (P.stride == 0 || P.many_features || tiles == 0 || in_bytes == 0 || in_bytes > tsvm::PINNED_BLOCK || sums * sizeof(float_type) > tsvm::PINNED_BLOCK)
+        return false;
+    if (tiles * in_bytes > FEW_LINK_BYTES) return false;
+    tsvm::ResultBlock in(tsvm::work_stream()), out(tsvm::work_stream());
+    float *const dense = (float *) in.host();
+    double *const sd = (double *) (dense + (m * d + 1) / 2 * 2);
+    std::fill(dense, dense + (m * d + 1) / 2 * 2, 0.0f);
+    const int64_t *const ptr = rows.ptr() + first;
+    for (size_t r = 0; r < m; ++r) {
+        double s = 0.0;
+        for (int64_t e = ptr[r]; e < ptr[r + 1]; ++e) {
+            const double v = rows.val()[e];
+            const int c = rows.col()[e];
+            // (other values than finite floats: the square below would not be exact, or a product with an absent column not zero)
+            if (!((double) (float) v == v) || std::isinf(v) || c < 0) {
+                in.unused();
+                out.unused();
+                return false;
+            }
+            if (c < d) dense[r * d + c] = (float) v;
+            s += v * v;   // (the square of a float is exact: what fma(v, v, s) gives)
+        }
+        sd[r] = s;
+    }
+    out.expect(sums);
+    abi_check(tsvm_predict_few_rows(R.x.data(), R.ld, d, R.self_dot.data(), P.col_map, P.n_pad, P.coef_t, P.stride, nc, dense, (const float *) in.dev(),
+                                    (int) m, (int) param.kernel_type, param.gamma, param.coef0, param.degree, (float_type *) out.dev(),
+                                    tsvm::work_stream()));
+    const float_type *const part = out.wait_for(sums);
+    in.unused();   // (whoever wrote the sums has read the rows)
+    // every pair's two classes, tile after tile, as predict_combine_kernel adds them
+    for (size_t r = 0; r < m; ++r) {
+        float_type *to = dec_out + r * n_binary_models;
+        for (int i = 0, p = 0; i < n_classes; ++i)
+            for (int j = i + 1; j < n_classes; ++j, ++p) {
+                double s = 0.0, t = 0.0;
+                for (int tile = P.class_tile[i]; tile < P.class_tile[i + 1]; ++tile) s += part[((size_t) tile * m + r) * nc + (j - 1)];
+                for (int tile = P.class_tile[j]; tile < P.class_tile[j + 1]; ++tile) t += part[((size_t) tile * m + r) * nc + i];
+                to[p] = (s + t) - rho[p];
+            }
+    }
+    return true;
+}
+
 void SvmModel::fetch_predictions(float_type *d_dec, size_t m, float_type *dec_out, int *winner_out) const {
     const size_t dec_bytes = m * (size_t) n_binary_models * sizeof(float_type);
     int *const d_winner = (int *) ((char *) d_dec + dec_bytes);
@@ -233,6 +288,7 @@ void SvmModel::predict_dec_values(const RowStore &rows, std::vector<float_type> 
     for (size_t b0 = 0; b0 < n_rows; b0 += batch_size) {
         const size_t bm = std::min((size_t) batch_size, n_rows - b0);
         if (fused) {
+            if (!winner && predict_few(P, rows, b0, bm, dec.data() + b0 * n_binary_models)) continue;
             const KernelMatrix::StagedBatch b = k_mat.stage_batch(rows, b0, bm);
             if (predict_batch_fused(P, b.a, b.lda, b.sd, bm, b.indicator_values, dec.data() + b0 * n_binary_models,
                                     winner ? winner->data() + b0 : nullptr))
