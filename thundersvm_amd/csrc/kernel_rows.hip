@@ -136,7 +136,7 @@ __global__ __launch_bounds__(256, 3) void get_rows_dense_stream_kernel(
     };
     // Rows are zero-padded up to ldx / lda (multiples of 8); the last 16-column tile may reach past that: vectors
     // that would start beyond the row re-read its last four columns instead (staged, never multiplied).
-    auto load_tile = [&](int kt, bool last) {
+    auto load_tile = [&](int kt, bool last, bool with_a = true) {
         const int k0 = kt * KTILE;
         if (!last) {
 #pragma unroll
@@ -144,8 +144,10 @@ __global__ __launch_bounds__(256, 3) void get_rows_dense_stream_kernel(
 #pragma unroll
             for (int q = 0; q < B_VEC; ++q) rb[q] = *(const v4d *) (x_ptr + (k0 + b_k + 4 * q));
         } else {
+            if (K_TILES != 1 || with_a) {
 #pragma unroll
-            for (int q = 0; q < A_VEC; ++q) ra[q] = *(const v4d *) (a_ptr + min(k0 + a_k + 4 * q, (int) lda - 4));
+                for (int q = 0; q < A_VEC; ++q) ra[q] = *(const v4d *) (a_ptr + min(k0 + a_k + 4 * q, (int) lda - 4));
+            }
 #pragma unroll
             for (int q = 0; q < B_VEC; ++q) rb[q] = *(const v4d *) (x_ptr + min(k0 + b_k + 4 * q, (int) ldx - 4));
         }
@@ -153,12 +155,14 @@ __global__ __launch_bounds__(256, 3) void get_rows_dense_stream_kernel(
     // (IND: the columns from d on are live data, not padding, and the last group of four columns may reach into
     // them: the working rows' values there are staged as zeros, which makes every such product an exact zero)
     const int k_live = d - (n_kt - 1) * KTILE;   // columns of the last K tile that belong to the product
-    auto stage_tile = [&](bool last) {
+    auto stage_tile = [&](bool last, bool with_a = true) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
+            if (K_TILES != 1 || with_a) {
 #pragma unroll
-            for (int q = 0; q < A_VEC; ++q)
-                As[(a_k + 4 * q + e) * LS + a_row] = (IND && last && a_k + 4 * q + e >= k_live) ? 0.0 : ra[q][e];
+                for (int q = 0; q < A_VEC; ++q)
+                    As[(a_k + 4 * q + e) * LS + a_row] = (IND && last && a_k + 4 * q + e >= k_live) ? 0.0 : ra[q][e];
+            }
 #pragma unroll
             for (int q = 0; q < B_VEC; ++q) Bs[(b_k + 4 * q + e) * LS + b_row] = rb[q][e];
         }
@@ -243,12 +247,12 @@ __global__ __launch_bounds__(256, 3) void get_rows_dense_stream_kernel(
                     __syncthreads();
                 }
             }
-            stage_tile(true);
+            stage_tile(true, jt == jt0);   // (a single K tile: the rows stay where they are for all of the column tiles)
         }
         __syncthreads();   // the staged tile, this tile's column data and (first tile) the row data are in LDS
         if (jt + 1 < jt1) {   // the next column tile's requests go out now, ahead of this tile's epilogue
             request_tile(jt + 1);
-            if (n_kt > 0) load_tile(0, n_kt == 1);
+            if (n_kt > 0) load_tile(0, n_kt == 1, false);
         }
         if (n_kt > 0) {
 #pragma unroll
@@ -283,17 +287,18 @@ __global__ __launch_bounds__(256, 3) void get_rows_dense_stream_kernel(
                     if constexpr (KT == TSVM_RBF && sizeof(TO) == 4) {
                         // expf's two out-of-range cases cost four instructions per value; one look at the largest
                         // magnitude among the wavefront's arguments (a NaN passes: it needs neither case) tells whether
-                        // any value of this store needs them.  Every instruction saved is an issue slot for the MFMAs.
+                        // any value of this store needs them.  Every instruction saved is an issue slot for the MFMAs (and the
+                        // limits are put in afterwards: as two versions of the exp behind a branch the four results were
+                        // moved together again, one and a half instructions per value).
                         float xs[4];
 #pragma unroll
                         for (int tj = 0; tj < 4; ++tj) xs[tj] = tsvm_rbf_arg(dot_of(ti, v, mi, tj), sdi, sdj[tj], kp);
                         const float mx = fmaxf(fmaxf(fabsf(xs[0]), fabsf(xs[1])), fmaxf(fabsf(xs[2]), fabsf(xs[3])));
-                        if (__builtin_amdgcn_ballot_w64(mx > 88.0f) == 0) {
 #pragma unroll
-                            for (int tj = 0; tj < 4; ++tj) res[tj] = tsvm_expf_in_range(xs[tj], exp_tab);
-                        } else {
+                        for (int tj = 0; tj < 4; ++tj) res[tj] = tsvm_expf_in_range(xs[tj], exp_tab);
+                        if (__builtin_amdgcn_ballot_w64(mx > 88.0f) != 0) {
 #pragma unroll
-                            for (int tj = 0; tj < 4; ++tj) res[tj] = tsvm_expf(xs[tj], exp_tab);
+                            for (int tj = 0; tj < 4; ++tj) res[tj] = tsvm_expf_limits(xs[tj], res[tj]);
                         }
                     } else {
 #pragma unroll

@@ -125,7 +125,7 @@ __global__ __launch_bounds__(256, 2) void predict_dense_stream_kernel(
             pre_c[q] = c < NC ? coef_t[(int64_t) p * NC + c] : 0.0;
         }
     };
-    auto load_tile = [&](int kt, bool last) {
+    auto load_tile = [&](int kt, bool last, bool with_a = true) {
         const int k0 = kt * KTILE;
         if (!last) {
 #pragma unroll
@@ -133,20 +133,24 @@ __global__ __launch_bounds__(256, 2) void predict_dense_stream_kernel(
 #pragma unroll
             for (int q = 0; q < B_VEC; ++q) rb[q] = *(const v4d *) (x_ptr + (k0 + b_k + 4 * q));
         } else {
+            if (K_TILES != 1 || with_a) {
 #pragma unroll
-            for (int q = 0; q < A_VEC; ++q) ra[q] = *(const v4d *) (a_ptr + min(k0 + a_k + 4 * q, (int) lda - 4));
+                for (int q = 0; q < A_VEC; ++q) ra[q] = *(const v4d *) (a_ptr + min(k0 + a_k + 4 * q, (int) lda - 4));
+            }
 #pragma unroll
             for (int q = 0; q < B_VEC; ++q) rb[q] = *(const v4d *) (x_ptr + min(k0 + b_k + 4 * q, (int) ldx - 4));
         }
     };
     // (IND: the columns from d on are live data, not padding: the batch rows' values there are staged as zeros)
     const int k_live = d - (n_kt - 1) * KTILE;
-    auto stage_tile = [&](bool last) {
+    auto stage_tile = [&](bool last, bool with_a = true) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
+            if (K_TILES != 1 || with_a) {
 #pragma unroll
-            for (int q = 0; q < A_VEC; ++q)
-                As[(a_k + 4 * q + e) * LS + a_row] = (IND && last && a_k + 4 * q + e >= k_live) ? 0.0 : ra[q][e];
+                for (int q = 0; q < A_VEC; ++q)
+                    As[(a_k + 4 * q + e) * LS + a_row] = (IND && last && a_k + 4 * q + e >= k_live) ? 0.0 : ra[q][e];
+            }
 #pragma unroll
             for (int q = 0; q < B_VEC; ++q) Bs[(b_k + 4 * q + e) * LS + b_row] = rb[q][e];
         }
@@ -207,12 +211,12 @@ __global__ __launch_bounds__(256, 2) void predict_dense_stream_kernel(
                     __syncthreads();
                 }
             }
-            stage_tile(true);
+            stage_tile(true, jt == jt0);   // (a single K tile: the rows stay where they are for all of the column tiles)
         }
         __syncthreads();   // the staged tile, this tile's column data and (first tile) the row data are in LDS
         if (jt + 1 < jt1) {   // the next column tile's requests go out now, ahead of this tile's epilogue
             request_tile(jt + 1);
-            if (n_kt > 0) load_tile(0, n_kt == 1);
+            if (n_kt > 0) load_tile(0, n_kt == 1, false);
         }
         if (n_kt > 0) {
 #pragma unroll
@@ -240,13 +244,15 @@ __global__ __launch_bounds__(256, 2) void predict_dense_stream_kernel(
 #pragma unroll
                 for (int tj = 0; tj < 4; ++tj) xs[tj] = tsvm_rbf_arg(dot_of(ti, v, mi, tj), sdi, sdj[tj], kp);
                 const float mx = fmaxf(fmaxf(fabsf(xs[0]), fabsf(xs[1])), fmaxf(fabsf(xs[2]), fabsf(xs[3])));
-                if (__builtin_amdgcn_ballot_w64(mx > 88.0f) == 0) {
+                float ks[4];
 #pragma unroll
-                    for (int tj = 0; tj < 4; ++tj) kv[tj] = (double) tsvm_expf_in_range(xs[tj], exp_tab);
-                } else {
+                for (int tj = 0; tj < 4; ++tj) ks[tj] = tsvm_expf_in_range(xs[tj], exp_tab);
+                if (__builtin_amdgcn_ballot_w64(mx > 88.0f) != 0) {
 #pragma unroll
-                    for (int tj = 0; tj < 4; ++tj) kv[tj] = (double) tsvm_expf(xs[tj], exp_tab);
+                    for (int tj = 0; tj < 4; ++tj) ks[tj] = tsvm_expf_limits(xs[tj], ks[tj]);
                 }
+#pragma unroll
+                for (int tj = 0; tj < 4; ++tj) kv[tj] = (double) ks[tj];
             } else {
 #pragma unroll
                 for (int tj = 0; tj < 4; ++tj) kv[tj] = tsvm_epilogue(dot_of(ti, v, mi, tj), sdi, sdj[tj], kp, exp_tab);

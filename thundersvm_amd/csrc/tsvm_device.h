@@ -58,12 +58,12 @@ __device__ __forceinline__ float tsvm_expf_in_range(float x, const uint64_t *tab
     y = y * s;
     return (float) y;
 }
-__device__ __forceinline__ float tsvm_expf(float x, const uint64_t *tab) {
-    float res = tsvm_expf_in_range(x, tab);
+// `res`, what that gave for x, or x's own result where it is out of range
+__device__ __forceinline__ float tsvm_expf_limits(float x, float res) {
     res = x > 0x1.62e42ep6f ? __builtin_inff() : res;   // > log(2^128)
-    res = x < -0x1.9fe368p6f ? 0.0f : res;              // < log(2^-150)
-    return res;
+    return x < -0x1.9fe368p6f ? 0.0f : res;             // < log(2^-150)
 }
+__device__ __forceinline__ float tsvm_expf(float x, const uint64_t *tab) { return tsvm_expf_limits(x, tsvm_expf_in_range(x, tab)); }
 
 // powf, the routine glibc (>= 2.28) uses: log2(x) from a 16-entry table and a quartic, in double, times y, then
 // 2^that through the expf table and cubic; every a*b+c is one fma (the form the library's FMA build takes on the
