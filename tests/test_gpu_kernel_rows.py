@@ -234,6 +234,14 @@ def test_csr_sliced_path(name, kt, prm, n, d, m, max_k):
     assert capi.kernel_lib().tsvm_get_rows_csr_sliced_lds(200000, 10, capi.ROW_F32) == 0
 
 
+@pytest.mark.parametrize("kt,n,d,m,max_k", [(O.RBF, 1300, 3000, 4130, 40),        # runs of slices that go over from one block of rows to the next
+                                            (O.RBF, 3000, 20958, 2100, 90),       # blocks in two halves among them
+                                            (O.LINEAR, 11700, 3000, 5555, 90)])  # two panels
+def test_csr_sliced_runs_across_blocks(kt, n, d, m, max_k):
+    name, _, prm = next(k for k in KERNELS if k[1] == kt)
+    test_csr_sliced_path(name, kt, prm, n, d, m, max_k)
+
+
 @pytest.mark.parametrize("n", [700, 5000])   # four / sixteen stored rows per workgroup
 @pytest.mark.parametrize("name,kt,prm", KERNELS)
 def test_csr_path(name, kt, prm, n):
