@@ -134,6 +134,14 @@ int tsvm_csr_stage_rows(const double *val, const int *col, const int64_t *row_pt
 int tsvm_csr_scatter_rows(const double *val, const int *col, const int64_t *row_ptr, const int *idx, int m,
                           int n_features, void *w, int w_type, int clear, tsvm_stream stream);
 
+/* out[r * ldo + t] = kernel value of rows idx[r] and idx[t], r, t < m <= 16384.  For rows whose values are finite and whose columns ascend, at least
+ * one entry among all of them; the entries are those of tsvm_get_rows_csr, bit for bit.  w [n_features][m], elements of w_type as for
+ * tsvm_get_rows_csr_staged, all-zero before; it is left with the rows in it and their numbers in ids [m].  To be used again it has to be
+ * another call's w_old, with its ids as ids_old and its m as m_old: that call takes them out. */
+int tsvm_csr_block(const double *val, const int *col, const int64_t *row_ptr, const int *idx, int m, const double *sd, void *w, int *ids, void *w_old,
+                   const int *ids_old, int m_old, int w_type, int kernel_type, double gamma, double coef0, int degree, void *out, int row_type, int64_t ldo,
+                   tsvm_stream stream);
+
 /* tsvm_get_rows_csr with the staged working rows held as w_type elements (TSVM_ROW_F64 or TSVM_ROW_F32).  Float
  * staging is exact when every value of the working rows is a float (values read from a LibSVM file or handed over
  * as float arrays are): products and sums are formed in double either way, and the kernel's time goes into

@@ -242,6 +242,47 @@ def test_csr_sliced_runs_across_blocks(kt, n, d, m, max_k):
     test_csr_sliced_path(name, kt, prm, n, d, m, max_k)
 
 
+@pytest.mark.parametrize("sizes", [(1, 2, 1), (63, 64, 65), (130, 1, 130), (512, 1023, 512)])   # calls one after another, their staging matrices in turn
+@pytest.mark.parametrize("name,kt,prm", KERNELS)
+def test_csr_block(name, kt, prm, sizes):
+    """tsvm_csr_block (the solver's block: entries above the diagonal computed, the others mirrored) against the oracle's rows, bit for bit:
+    empty rows, rows that occur twice, what the call before has left in the other staging matrix, both staging types, rows of odd length."""
+    rng = np.random.default_rng(sum(sizes))
+    n, d = 1100, 2500
+    ptr, col, val = [0], [], []
+    for i in range(n):
+        c = np.sort(rng.choice(d, size=int(rng.integers(0, 70)) if i % 5 else i % 3, replace=False, p=None)) + 1
+        c[:len(c) // 2] = np.arange(1, len(c) // 2 + 1)   # (features that many rows have)
+        c = np.unique(c)
+        col.extend(c)
+        val.extend(rng.standard_normal(len(c)).astype(np.float32))
+        ptr.append(len(col))
+    data = CsrData(ptr, col, np.asarray(val, dtype=np.float64))
+    okm = O.KernelMatrix(data.ptr, data.col, data.val, O.make_param(kernel_type=kt, expf_mode=1, **prm))
+    nf = okm.n_features
+    val_d, col_d, ptr_d = G.dev(data.val), G.dev(data.col), G.dev(data.ptr)
+    sd = torch.empty(n, dtype=torch.float64, device="cuda")
+    capi.call("tsvm_csr_self_dot", G.ptr(val_d), G.ptr(ptr_d), n, G.ptr(sd), G.stream())
+    for wt, rt, pad in ((capi.ROW_F32, capi.ROW_F64 if kt == O.LINEAR else capi.ROW_F32, 0), (capi.ROW_F64, capi.ROW_F64, 3)):
+        w = [torch.zeros(nf * max(sizes), dtype=torch.float32 if wt == capi.ROW_F32 else torch.float64, device="cuda") for _ in range(2)]
+        ids = [torch.zeros(max(sizes), dtype=torch.int32, device="cuda") for _ in range(2)]
+        before = 0
+        for turn, m in enumerate(sizes):
+            idx = rng.integers(0, n, size=m).astype(np.int32)
+            if m > 2: idx[-1] = idx[0]
+            idx_d = G.dev(idx)
+            now, last = turn % 2, 1 - turn % 2
+            ldo = (m + 7) // 8 * 8 + pad
+            out = torch.full((m, ldo), -3.0, dtype=torch.float32 if rt == capi.ROW_F32 else torch.float64, device="cuda")
+            capi.call("tsvm_csr_block", G.ptr(val_d), G.ptr(col_d), G.ptr(ptr_d), G.ptr(idx_d), m, G.ptr(sd), G.ptr(w[now]), G.ptr(ids[now]),
+                      G.ptr(w[last]), G.ptr(ids[last]), before, wt, kt, prm.get("gamma", 0.0), prm.get("coef0", 0.0), prm.get("degree", 3),
+                      G.ptr(out), rt, ldo, G.stream())
+            got = G.host(out).astype(np.float64)
+            _check(name, got[:, :m], okm.get_rows(idx)[:, idx])
+            assert (got[:, m:] == -3.0).all() and not w[last].any() and np.array_equal(G.host(ids[now])[:m], idx)
+            before = m
+
+
 @pytest.mark.parametrize("n", [700, 5000])   # four / sixteen stored rows per workgroup
 @pytest.mark.parametrize("name,kt,prm", KERNELS)
 def test_csr_path(name, kt, prm, n):

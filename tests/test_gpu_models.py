@@ -151,6 +151,19 @@ def test_sparse_multiclass(kernel):
     assert gm.n_binary == 6
 
 
+def test_sparse_rows_in_any_order():
+    """Rows whose entries do not ascend: the solver's block is not the mirror of its upper half to the last bit there, and every value is the
+    stored row's own sum, as in the oracle."""
+    w = D.workload_c3(scale=0.05, kernel="linear")
+    tr = w["train"]
+    col, val = tr.col.copy(), tr.val.copy()
+    for r in range(0, tr.n, 3):
+        lo, hi = tr.ptr[r], tr.ptr[r + 1]
+        col[lo:hi], val[lo:hi] = tr.col[lo:hi][::-1], tr.val[lo:hi][::-1]
+    from thundersvm_amd.data import CsrData
+    _compare(CsrData(tr.ptr, col, val, tr.y), None, make_param(**w["params"]), trace=16)
+
+
 def test_workload_c5_small():
     w = D.workload_c5(scale=0.01)
     _compare(w["train"], w["test"], make_param(**w["params"]), trace=64)

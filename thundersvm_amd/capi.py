@@ -37,6 +37,7 @@ SIGNATURES = {
     "tsvm_csr_stage_rows": (_int, [_p, _p, _p, _p, _int, _int, _p, _p]),
     "tsvm_csr_scatter_rows": (_int, [_p, _p, _p, _p, _int, _int, _p, _int, _int, _p]),
     "tsvm_get_rows_csr": (_int, [_p, _p, _p, _p, _i64, _p, _p, _int, _p, _int, _dbl, _dbl, _int, _p, _int, _p, _i64, _p]),
+    "tsvm_csr_block": (_int, [_p, _p, _p, _p, _int, _p, _p, _p, _p, _p, _int, _int, _int, _dbl, _dbl, _int, _p, _int, _i64, _p]),
     "tsvm_get_rows_csr_staged": (_int, [_p, _p, _p, _p, _i64, _p, _p, _int, _int, _p, _int, _dbl, _dbl, _int, _p, _int, _p, _i64, _p]),
     "tsvm_csr_slice_widths": (_int, [_p, _i64, _p, _p]),
     "tsvm_csr_to_sliced": (_int, [_p, _p, _p, _i64, _p, _int, _p, _p, _int, _p]),

@@ -442,8 +442,10 @@ std::shared_ptr<DeviceRows> DeviceRows::from_host(const RowStore &rows) {
     const int *const col = rows.col() + first;
     const kernel_type *const val = rows.val() + first;
     int max_index = 0, all_float = 1, all_finite = 1;
-#pragma omp parallel for schedule(static) reduction(max : max_index) reduction(min : all_float, all_finite) num_threads(threads_for(r.nnz))
+    size_t descents = 0;   // entries whose column is not larger than the one's before
+#pragma omp parallel for schedule(static) reduction(max : max_index) reduction(min : all_float, all_finite) reduction(+ : descents) num_threads(threads_for(r.nnz))
     for (size_t e = 0; e < r.nnz; ++e) {
+        descents += col[e] <= col[e > 0 ? e - 1 : 0];
         max_index = std::max(max_index, col[e]);
         all_float = (double) (float) val[e] != (double) val[e] ? 0 : all_float;
         all_finite = val[e] - val[e] == 0 ? all_finite : 0;
@@ -452,6 +454,17 @@ std::shared_ptr<DeviceRows> DeviceRows::from_host(const RowStore &rows) {
     r.values_fit_float = all_float != 0;
     r.values_finite = all_finite != 0;
     r.dense = KernelMatrix::choose_dense(r.n, r.n_features, r.nnz);
+    if (!r.dense) {
+        // (the first entry counts as one, and any other may only be one where a row begins)
+        const int64_t *const at = rows.ptr();
+        size_t at_starts = 0;
+#pragma omp parallel for schedule(static) reduction(+ : at_starts) num_threads(threads_for(r.nnz))
+        for (size_t i = 0; i < r.n; ++i) {
+            const int64_t e = at[i] - first;
+            at_starts += at[i + 1] > at[i] && col[e] <= col[e > 0 ? e - 1 : 0];
+        }
+        r.columns_ascend = descents == at_starts;
+    }
     tsvm::HostStaging &staging = tsvm::HostStaging::instance();
     std::vector<int64_t> ptr;
     const int64_t *host_ptr = rows.ptr();
@@ -533,6 +546,7 @@ std::shared_ptr<DeviceRows> DeviceRows::subset(const DeviceRows &base, const int
     r.dense = base.dense;
     r.values_fit_float = base.values_fit_float;
     r.values_finite = base.values_finite;
+    r.columns_ascend = base.columns_ascend;
     r.ld = base.ld;
     const bool by_value = base.dense && n_rows <= (size_t) tsvm_subset_rows_dense_max_ids((int64_t) base.n);
     tsvm::DeviceBuffer<int> d_rows(by_value ? 0 : n_rows);
@@ -762,8 +776,25 @@ void KernelMatrix::get_block(const int *d_idx, int m, void *d_out, int64_t ld, h
         return;
     }
     const int wt = R.values_fit_float ? TSVM_ROW_F32 : TSVM_ROW_F64;
+    const size_t bytes = (size_t) m * R.n_features * (R.values_fit_float ? sizeof(float) : sizeof(double));
+    // K(r, t) is K(t, r) to the last bit unless a value times an absent (zero) one is not zero, or the two rows' common features come in two orders
+    if (R.values_finite && R.columns_ascend && R.nnz > 0) {
+        BlockStage &now = turn_[turn_now_], &last = turn_[turn_now_ ^ 1];
+        if (now.w.size() < bytes) {
+            grow_zeroed(now.w, bytes, stream);
+            now.m = 0;
+        }
+        if (now.m != 0) throw std::logic_error("KernelMatrix::get_block: rows in the staging matrix");
+        if (now.ids.size() < (size_t) m) now.ids.resize(m);
+        abi_check(tsvm_csr_block(R.val.data(), R.col.data(), R.row_ptr.data(), d_idx, m, R.self_dot.data(), now.w.data(), now.ids.data(), last.w.data(),
+                                 last.ids.data(), last.m, wt, (int) param.kernel_type, param.gamma, param.coef0, param.degree, d_out, row_type(), ld, stream));
+        now.m = m;
+        last.m = 0;
+        turn_now_ ^= 1;
+        return;
+    }
     // kept all-zero between uses, as in get_rows
-    grow_zeroed(stage_blk_, (size_t) m * R.n_features * (R.values_fit_float ? sizeof(float) : sizeof(double)), stream);
+    grow_zeroed(stage_blk_, bytes, stream);
     if (stage_blk_sd_.size() < (size_t) m) stage_blk_sd_.resize(m);
     abi_check(tsvm_csr_scatter_rows(R.val.data(), R.col.data(), R.row_ptr.data(), d_idx, m, (int) R.n_features,
                                     stage_blk_.data(), wt, 0, stream));

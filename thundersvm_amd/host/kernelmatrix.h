@@ -27,6 +27,7 @@ struct DeviceRows {
     bool dense = false;
     bool values_fit_float = false;               // every stored value is exactly a float (CSR layout: staging type)
     bool values_finite = false;                  // no stored value is infinite or NaN (rows taken from host memory)
+    bool columns_ascend = false;                 // within every row, none of them twice
     int64_t ld = 0;                              // dense row stride (n_features rounded up to 8)
     tsvm::DeviceBuffer<kernel_type> x;           // dense layout [n][ld]
     tsvm::DeviceBuffer<kernel_type> val;         // CSR layout
@@ -134,6 +135,14 @@ private:
     // transposed staging of CSR working rows (get_rows / get_block), all-zero between uses; float elements when
     // the rows' values are floats
     mutable tsvm::DeviceBuffer<unsigned char> stage_w_, stage_blk_;
+    // get_block's two that take turns (tsvm_csr_block): the rows that are in them are taken out by the next call
+    struct BlockStage {
+        tsvm::DeviceBuffer<unsigned char> w;
+        tsvm::DeviceBuffer<int> ids;
+        int m = 0;
+    };
+    mutable BlockStage turn_[2];
+    mutable int turn_now_ = 0;
     mutable tsvm::DeviceBuffer<kernel_type> stage_blk_sd_;
     mutable tsvm::DeviceBuffer<kernel_type> stage_sd_;
     mutable tsvm::DeviceBuffer<kernel_type> b_val_;
