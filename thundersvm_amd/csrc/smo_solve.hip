@@ -132,7 +132,7 @@ __global__ void smo_start_kernel(double *alpha_diff, int n_diff, TB *kws, int ws
 // XCDs, they are in none: a row then takes some 700 cycles instead of 250).  Workgroup b runs on XCD b % 8 as a rule;
 // those on another one leave.  One call of 455 iterations at ws = 1024: 1.22 us per iteration on a block that has just
 // been written, 1.09 after this kernel, which takes about 6 us.
-#define SV_L2_BYTES (4u << 20)   // blocks larger than an XCD's L2 are left alone
+#define SV_L2_BYTES (4u << 20)   // (warm_block_kernel leaves larger blocks alone; warm_share)
 #define SV_WARM_SLICES 32
 __global__ __launch_bounds__(256) void warm_block_kernel(const uint4 *__restrict__ p, unsigned n16, int xcd, int *__restrict__ sink) {
     if ((int) __builtin_amdgcn_s_getreg(20 | (0 << 6) | (3 << 11)) != xcd) return;   // XCC_ID
@@ -251,9 +251,15 @@ __device__ __forceinline__ bool solver_elected_on_cu(int *gate, int epoch, bool 
     return s_elected != 0;
 }
 // Workgroup b is number b / 8 of its XCD's thirty-two, as a rule.
+// Of a block that is larger than the L2 (1,024 rows of doubles, 8 MB), what has been selected last, the most violating first: the rows behind
+// the half that the working set keeps, three quarters of an L2 of them.  Linear text, 18,000 rows, a call: none 32.4 ms, 384 of those rows
+// 31.5 (448 as much, all 512 a little less), 448 of the kept ones 32.3.
 __device__ __forceinline__ void warm_share(const void *block, unsigned bytes, int *gate) {
-    if (bytes > SV_L2_BYTES) return;
-    const uint4 *const p = (const uint4 *) block;
+    const uint4 *p = (const uint4 *) block;
+    if (bytes > SV_L2_BYTES) {
+        p += bytes / 2 / 16;
+        bytes = bytes / 2 < SV_L2_BYTES / 4 * 3 ? bytes / 2 : SV_L2_BYTES / 4 * 3;
+    }
     const unsigned n16 = bytes / 16, per = (n16 + SV_WARM_SLICES - 1) / SV_WARM_SLICES, lo = (blockIdx.x >> 3) * per, hi = lo + per < n16 ? lo + per : n16;
     unsigned any = 0;
     for (unsigned i = lo + threadIdx.x; i < hi; i += blockDim.x) {
