@@ -254,9 +254,12 @@ __device__ __forceinline__ bool solver_elected_on_cu(int *gate, int epoch, bool 
 // Of a block that is larger than the L2 (1,024 rows of doubles, 8 MB), what has been selected last, the most violating first: the rows behind
 // the half that the working set keeps, three quarters of an L2 of them.  Linear text, 18,000 rows, a call: none 32.4 ms, 384 of those rows
 // 31.5 (448 as much, all 512 a little less), 448 of the kept ones 32.3.
+// (LARGE: a variant of its own, as the test in the others moved their loops: the nu variant's steps took 3 % longer.)
+template <bool LARGE>
 __device__ __forceinline__ void warm_share(const void *block, unsigned bytes, int *gate) {
     const uint4 *p = (const uint4 *) block;
     if (bytes > SV_L2_BYTES) {
+        if (!LARGE) return;
         p += bytes / 2 / 16;
         bytes = bytes / 2 < SV_L2_BYTES / 4 * 3 ? bytes / 2 : SV_L2_BYTES / 4 * 3;
     }
@@ -306,7 +309,7 @@ __device__ __forceinline__ void gather_elems(const int *__restrict__ working_set
 
 // Whether this workgroup of a launch is the one that solves, with what its elements start from.  (What is gathered is on its way during
 // the election; those that can only be elected last gather behind it.)
-template <int E>
+template <int E, bool LARGE>
 __device__ __forceinline__ bool solver_begins(int *gate, int epoch, int target_xcd, int target_cu, int *started, const void *block, unsigned bytes,
                                               const int *__restrict__ working_set, int ws, const double *__restrict__ f_val, const double *alpha_val,
                                               const int *__restrict__ labels, const double *__restrict__ k_diag, double (&f)[E], double (&alpha)[E],
@@ -316,7 +319,7 @@ __device__ __forceinline__ bool solver_begins(int *gate, int epoch, int target_x
     if (!gate) return true;
     if (target_cu < 0) return solver_elected(gate, epoch, target_xcd);
     if (!solver_elected_on_cu(gate, epoch, likely, started)) {
-        if (on_xcd) warm_share(block, bytes, gate);
+        if (on_xcd) warm_share<LARGE>(block, bytes, gate);
         return false;
     }
     if (!likely) gather_elems<E>(working_set, ws, f_val, alpha_val, labels, k_diag, f, alpha, kd, label);
@@ -610,7 +613,7 @@ __global__ __launch_bounds__(64 * W) void c_smo_solve_kernel(
     int max_iter, int *__restrict__ gate, int epoch, int target_xcd, int target_cu) {
     double f[E], a_old[E], kd[E];
     int y_of[E];
-    if (!solver_begins<E>(gate, epoch, target_xcd, target_cu, (int *) (diff + 2), kws, (unsigned) (ws * LDK * sizeof(TB)), working_set, ws, f_val, alpha, label, k_diag, f, a_old, kd,
+    if (!solver_begins<E, (sizeof(TB) * LDK * LDK > SV_L2_BYTES)>(gate, epoch, target_xcd, target_cu, (int *) (diff + 2), kws, (unsigned) (ws * LDK * sizeof(TB)), working_set, ws, f_val, alpha, label, k_diag, f, a_old, kd,
                           y_of))
         return;
     constexpr int N = E * 64 * W;
@@ -998,7 +1001,7 @@ __global__ __launch_bounds__(64 * W) void nu_smo_solve_kernel(
     int max_iter, int *__restrict__ gate, int epoch, int target_xcd, int target_cu) {
     double f[E], a_old[E], kd[E];
     int y_of[E];
-    if (!solver_begins<E>(gate, epoch, target_xcd, target_cu, (int *) (diff + 2), kws, (unsigned) (ws * LDK * sizeof(TB)), working_set, ws, f_val, alpha, label, k_diag, f, a_old, kd,
+    if (!solver_begins<E, (sizeof(TB) * LDK * LDK > SV_L2_BYTES)>(gate, epoch, target_xcd, target_cu, (int *) (diff + 2), kws, (unsigned) (ws * LDK * sizeof(TB)), working_set, ws, f_val, alpha, label, k_diag, f, a_old, kd,
                           y_of))
         return;
     constexpr int N = E * 64 * W;
