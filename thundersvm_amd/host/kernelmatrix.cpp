@@ -445,10 +445,8 @@ std::shared_ptr<DeviceRows> DeviceRows::from_host(const RowStore &rows) {
     const int *const col = rows.col() + first;
     const kernel_type *const val = rows.val() + first;
     int max_index = 0, all_float = 1, all_finite = 1;
-    size_t descents = 0;   // entries whose column is not larger than the one's before
-#pragma omp parallel for schedule(static) reduction(max : max_index) reduction(min : all_float, all_finite) reduction(+ : descents) num_threads(threads_for(r.nnz))
+#pragma omp parallel for schedule(static) reduction(max : max_index) reduction(min : all_float, all_finite) num_threads(threads_for(r.nnz))
     for (size_t e = 0; e < r.nnz; ++e) {
-        descents += col[e] <= col[e > 0 ? e - 1 : 0];
         max_index = std::max(max_index, col[e]);
         all_float = (double) (float) val[e] != (double) val[e] ? 0 : all_float;
         all_finite = val[e] - val[e] == 0 ? all_finite : 0;
@@ -458,13 +456,18 @@ std::shared_ptr<DeviceRows> DeviceRows::from_host(const RowStore &rows) {
     r.values_finite = all_finite != 0;
     r.dense = KernelMatrix::choose_dense(r.n, r.n_features, r.nnz);
     if (!r.dense) {
-        // (the first entry counts as one, and any other may only be one where a row begins)
+        // (an entry whose column is not larger than the one's before may only be one where a row begins)
         const int64_t *const at = rows.ptr();
-        size_t at_starts = 0;
-#pragma omp parallel for schedule(static) reduction(+ : at_starts) num_threads(threads_for(r.nnz))
-        for (size_t i = 0; i < r.n; ++i) {
-            const int64_t e = at[i] - first;
-            at_starts += at[i + 1] > at[i] && col[e] <= col[e > 0 ? e - 1 : 0];
+        int64_t descents = 0, at_starts = 0;
+#pragma omp parallel num_threads(threads_for(r.nnz))
+        {
+#pragma omp for schedule(static) reduction(+ : descents) nowait
+            for (size_t e = 1; e < r.nnz; ++e) descents += col[e] <= col[e - 1];
+#pragma omp for schedule(static) reduction(+ : at_starts)
+            for (size_t i = 0; i < r.n; ++i) {
+                const int64_t e = at[i] - first;
+                at_starts += e > 0 && at[i + 1] > at[i] && col[e] <= col[e - 1];
+            }
         }
         r.columns_ascend = descents == at_starts;
     }
