@@ -12,34 +12,33 @@
 #include "get_rows_tile.h"
 
 
-// Workgroups walk their XCD's share of the tiles in steps of as many as it has: with a grid of all tiles that is one tile each; a grid of
-// GR_WGS gives every CU two workgroups and the tiles of the last, partial round to the first ones, which are on CUs of their own.  Left to the
-// dispatcher, some of those went to one CU in pairs while others had nothing: 512 rows of 20,000 columns, 784 features (628 tiles)
-// beside a solver 340 -> 316 us in the middle (best 285 -> 313), and a training call of 20,000 rows 1.5 % less.  The last round in tiles of 64
-// rows, two for one, took 346: a workgroup that is alone on its CU is bound by latency.  Only for a few rounds: in longer launches the dispatcher evens out more than that.
-#define GR_WGS 496u          // two on each of 248 CUs
+// Tiles from `tile0` on, one for each workgroup.
+// Workgroups are dealt to a die's four groups of eight CUs in turn, whether or not a group has a CU that its stream leaves to a solver, so
+// that a launch of 496, two for each of 248 CUs, lasts as long as three of them on one CU (287 us).  On such a stream a launch of a few
+// rounds is made in rounds of GR_WGS tiles, which all have their place, and the rest, most of which then have a CU each, as a launch
+// of their own: 512 rows of 20,000 columns, 784 features (628 tiles) beside a solver 340 us in the middle -> 197 + 113.  (A loop over
+// the tiles in a grid of 496 workgroups 316: its registers cost the K loop instructions, and on a stream that has the chip 310 for 288.)
+// Longer launches even out.
+#define GR_WGS 448u
 #define GR_WGS_ROUNDS 4u
 template <int KT, int TI, typename TO>
 __global__ __launch_bounds__(256, (TI == 2 ? 3 : 2)) void get_rows_dense_kernel(
     const double *__restrict__ x, int64_t ldx, const int *__restrict__ x_idx, int64_t n, int d,
     const double *__restrict__ sd_x, const double *__restrict__ a, int64_t lda, const int *__restrict__ a_idx, int m,
     const double *__restrict__ sd_a, KernelParam kp, TO *__restrict__ out, const int *__restrict__ out_slots,
-    int64_t ldo, const int *__restrict__ m_dev) {
+    int64_t ldo, const int *__restrict__ m_dev, unsigned tile0) {
     __shared__ double As[GrShape<TI>::LDS_DOUBLES];
     __shared__ double Bs[GrShape<TI>::LDS_DOUBLES];
     __shared__ uint64_t exp_tab[32];
     if (threadIdx.x < 32) exp_tab[threadIdx.x] = TSVM_EXP2F_TAB[threadIdx.x];
     __syncthreads();
-    if (m_dev) m = *m_dev;   // the number of working rows is only known on the device (m sized the grid)
+    if (m_dev) m = *m_dev;   // the number of working rows is only known on the device (m sized the grid): workgroups beyond it leave
     const unsigned m_blocks = (unsigned) (m + GrShape<TI>::BM - 1) / GrShape<TI>::BM, tiles = (unsigned) ((n + GR_BN - 1) / GR_BN) * m_blocks;
-    const unsigned xcd = blockIdx.x % 8, step = (gridDim.x + 7 - xcd) / 8;
-    const unsigned per = tiles / 8, rem = tiles % 8, first = xcd * per + (xcd < rem ? xcd : rem), mine = per + (xcd < rem ? 1 : 0);
-    for (unsigned u = blockIdx.x / 8; u < mine; u += step) {
-        if (u >= step) __syncthreads();   // every wavefront is done with the staged columns of the tile before
-        const int j0 = (int) ((first + u) / m_blocks) * GR_BN;   // n fits 31 bits (checked by the host)
-        const int i0 = (int) ((first + u) % m_blocks) * GrShape<TI>::BM;
-        get_rows_tile<KT, TI, TO>(x, ldx, x_idx, n, d, sd_x, a, lda, a_idx, m, sd_a, kp, out, out_slots, ldo, i0, j0, As, Bs, exp_tab);
-    }
+    if (tile0 + blockIdx.x >= tiles) return;
+    const unsigned tile = tile0 + xcd_remap(blockIdx.x, tiles - tile0 < gridDim.x ? tiles - tile0 : gridDim.x);
+    const int j0 = (int) (tile / m_blocks) * GR_BN;   // n fits 31 bits (checked by the host)
+    const int i0 = (int) (tile % m_blocks) * GrShape<TI>::BM;
+    get_rows_tile<KT, TI, TO>(x, ldx, x_idx, n, d, sd_x, a, lda, a_idx, m, sd_a, kp, out, out_slots, ldo, i0, j0, As, Bs, exp_tab);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1252,6 +1251,18 @@ static int stream_tiles_per_wg() {
     return v;
 }
 
+// Whether a stream has been made with a mask that is not all of the chip's 256 CUs.
+static bool leaves_cus_out(hipStream_t stream) {
+    uint32_t mask[8] = {};
+    if (!stream || hipExtStreamGetCUMask(stream, 8, mask) != hipSuccess) {
+        (void) hipGetLastError();
+        return false;
+    }
+    int cus = 0;
+    for (uint32_t word : mask) cus += __builtin_popcount(word);
+    return cus > 0 && cus < 256;
+}
+
 static int get_rows_dense(const double *x, int64_t ldx, const int *x_idx, int64_t n, int d, const double *sd_x, const double *a,
                           int64_t lda, const int *a_idx, int m, const int *m_dev, const double *sd_a, int kernel_type, double gamma,
                           double coef0, int degree, void *out, int row_type, const int *out_slots, int64_t ldo,
@@ -1282,7 +1293,11 @@ static int get_rows_dense(const double *x, int64_t ldx, const int *x_idx, int64_
     const int64_t n_blocks = (n + GR_BN - 1) / GR_BN;
     TSVM_REQUIRE(n_blocks * m_blocks < (int64_t) 0x7fffffff, "tsvm_get_rows_dense: grid too large");
     dim3 grid((unsigned) (n_blocks * m_blocks)), block(256);
-    if (ti == 4 && grid.x > GR_WGS && grid.x <= GR_WGS_ROUNDS * GR_WGS) grid.x = GR_WGS;
+    unsigned last = 0;   // tiles of a launch of their own
+    if (ti == 4 && grid.x > GR_WGS && grid.x <= GR_WGS_ROUNDS * GR_WGS && leaves_cus_out(tsvm_s(stream))) {
+        last = grid.x % GR_WGS;
+        grid.x -= last;
+    }
     // the solver's ws x ws block: symmetric, computed from the tiles on and above the diagonal
     const bool sym = x == a && ldx == lda && x_idx && x_idx == a_idx && n == m && sd_x == sd_a && !out_slots && !m_dev &&
                      !mask_x && ti == 2 && ldo >= n;   // (with masks d does not count the columns that they stand for)
@@ -1344,9 +1359,13 @@ static int get_rows_dense(const double *x, int64_t ldx, const int *x_idx, int64_
                 case 4: GR_STREAM(KTYPE, TO, 4); break;                                                               \
                 default: GR_STREAM(KTYPE, TO, 5); break;                                                              \
             }                                                                                                         \
-        } else                                                                                                        \
+        } else {                                                                                                      \
             hipLaunchKernelGGL((get_rows_dense_kernel<KTYPE, 4, TO>), grid, block, 0, tsvm_s(stream), x, ldx, x_idx, n, d, sd_x, \
-                               a, lda, a_idx, m, sd_a, kp, (TO *) out, out_slots, ldo, m_dev);                        \
+                               a, lda, a_idx, m, sd_a, kp, (TO *) out, out_slots, ldo, m_dev, 0u);                    \
+            if (last)                                                                                                 \
+                hipLaunchKernelGGL((get_rows_dense_kernel<KTYPE, 4, TO>), dim3(last), block, 0, tsvm_s(stream), x, ldx, x_idx, n, d, sd_x, \
+                                   a, lda, a_idx, m, sd_a, kp, (TO *) out, out_slots, ldo, m_dev, grid.x);            \
+        }                                                                                                             \
     } while (0)
 #define GR_LAUNCH(KTYPE)                                        \
     do {                                                        \
