@@ -1,4 +1,7 @@
 """Helpers for the GPU parity tests: device buffers through torch, calls through the C ABI."""
+import contextlib
+import ctypes
+
 import numpy as np
 import torch
 
@@ -51,3 +54,19 @@ def float_ulp_diff(a, b):
     ia = np.where(ia < 0, -(ia & 0x7fffffff), ia)
     ib = np.where(ib < 0, -(ib & 0x7fffffff), ib)
     return np.abs(ia - ib)
+
+
+@contextlib.contextmanager
+def stream_without_cus(lanes):
+    """torch's current stream is one that leaves out the first CU of dies 0 .. lanes-1, as the rows' streams beside that many solvers do."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    torch.cuda.synchronize()
+    handle = ctypes.c_void_p()
+    mask = (ctypes.c_uint32 * 8)(0xffffffff & ~((1 << lanes) - 1), *[0xffffffff] * 7)
+    assert hip.hipExtStreamCreateWithCUMask(ctypes.byref(handle), 8, mask) == 0
+    try:
+        with torch.cuda.stream(torch.cuda.ExternalStream(handle.value)):
+            yield
+            torch.cuda.synchronize()
+    finally:
+        assert hip.hipStreamDestroy(handle) == 0

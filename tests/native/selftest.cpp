@@ -4,12 +4,14 @@
 // the tests; the product libraries do not contain it.
 #include <omp.h>
 
+#include <algorithm>
 #include <chrono>
 #include <stdexcept>
 #include <string>
 #include <thread>
 #include <vector>
 
+#include "../../thundersvm_amd/csrc/sliced_deal.h"
 #include "../../thundersvm_amd/host/dataset.h"
 #include "../../thundersvm_amd/host/device.h"
 #include "../../thundersvm_amd/host/kernelmatrix.h"
@@ -320,6 +322,29 @@ int tsvm_selftest_thread_limit(int how, int n) {
     }
     set_threads(0);
     return limit;
+}
+
+// The sliced CSR kernel's work, n stored rows and n_blocks blocks of working rows: 0 if its workgroups take every slice of every block exactly
+// once.  out: workgroups, the most slices that one takes, the most tiles that one builds.
+int tsvm_selftest_sliced_deal(long long n, long long n_blocks, int places, long long *out) {
+    const SlicedDeal deal = sliced_deal(n, n_blocks, (unsigned) places);
+    const long long n_slices = (n + 63) / 64;
+    std::vector<unsigned char> taken(n_slices * n_blocks, 0);
+    out[0] = deal.workgroups;
+    out[1] = out[2] = 0;
+    for (unsigned w = 0; w < deal.workgroups; ++w) {
+        SlicedWalk walk(deal, w);
+        long long slices = 0, tiles = 0;
+        for (unsigned block, slice0, slice1; walk.next(deal, block, slice0, slice1); ++tiles) {
+            if (block >= n_blocks || slice1 <= slice0 || slice1 > n_slices) return -1;
+            for (unsigned s = slice0; s < slice1; ++s)
+                if (taken[block * n_slices + s]++) return -1;
+            slices += slice1 - slice0;
+        }
+        out[1] = std::max(out[1], slices);
+        out[2] = std::max(out[2], tiles);
+    }
+    return std::count(taken.begin(), taken.end(), 1) == (long long) taken.size() ? 0 : -1;
 }
 
 }  // extern "C"

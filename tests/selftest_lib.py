@@ -27,6 +27,7 @@ def lib():
         L.tsvm_selftest_chip_split.argtypes = [ctypes.c_int] * 2 + [ctypes.c_longlong] * 3
         L.tsvm_selftest_rows_ahead.argtypes = [ctypes.c_int] * 3 + [ctypes.c_longlong] * 2
         L.tsvm_selftest_thread_limit.argtypes = [ctypes.c_int] * 2
+        L.tsvm_selftest_sliced_deal.argtypes = [ctypes.c_longlong] * 2 + [ctypes.c_int, ctypes.c_void_p]
         L.tsvm_selftest_guided.argtypes = [ctypes.c_longlong, ctypes.c_int, ctypes.c_int]
         L.tsvm_selftest_mark_support_vectors.restype = ctypes.c_double
         L.tsvm_selftest_mark_support_vectors.argtypes = [ctypes.c_int] * 2

@@ -5,6 +5,8 @@ ragged shapes.  Bars: all four kernels bit-exact (the oracle runs its restated e
 tests/test_oracle_expf.py pins to libm; test_poly_and_sigmoid_rows_match_libm checks the GPU against libm itself);
 decision values 1e-9.
 """
+import contextlib
+
 import numpy as np
 import pytest
 import torch
@@ -236,10 +238,46 @@ def test_csr_sliced_path(name, kt, prm, n, d, m, max_k):
 
 @pytest.mark.parametrize("kt,n,d,m,max_k", [(O.RBF, 1300, 3000, 4130, 40),        # runs of slices that go over from one block of rows to the next
                                             (O.RBF, 3000, 20958, 2100, 90),       # blocks in two halves among them
-                                            (O.LINEAR, 11700, 3000, 5555, 90)])  # two panels
+                                            (O.LINEAR, 11700, 3000, 5555, 90)])  # 184 slices a block
 def test_csr_sliced_runs_across_blocks(kt, n, d, m, max_k):
     name, _, prm = next(k for k in KERNELS if k[1] == kt)
     test_csr_sliced_path(name, kt, prm, n, d, m, max_k)
+
+
+@pytest.mark.parametrize("lanes", [0, 1, 8])
+@pytest.mark.parametrize("kt,n,d,m,max_k", [(O.RBF, 70, 3000, 4099, 40),          # whole blocks of two slices, two of them for some workgroups
+                                            (O.POLY, 300, 3000, 4500, 40),
+                                            (O.LINEAR, 2500, 3000, 777, 40),      # parts of a block
+                                            (O.SIGMOID, 4200, 3000, 3700, 20)])   # more blocks than places beside a solver, fewer on the whole chip
+def test_csr_sliced_deals(kt, n, d, m, max_k, lanes):
+    name, _, prm = next(k for k in KERNELS if k[1] == kt)
+    with G.stream_without_cus(lanes) if lanes else contextlib.nullcontext():
+        test_csr_sliced_path(name, kt, prm, n, d, m, max_k)
+
+
+def test_csr_sliced_few_stored_rows_fill_the_chip():
+    """70 stored rows against 4,099: 257 blocks of sixteen, a workgroup of a CU each and two for one of them.  Sixteen workgroups for all of
+    them took 12 times as long as 2,048 rows (416 and 34 us with 64 stored rows); now less than twice."""
+    n, d, max_k = 70, 3000, 40
+    rng = np.random.default_rng(1)
+    rows = [np.sort(rng.choice(d, size=max_k, replace=False)) + 1 for _ in range(4099)]
+    data = CsrData(np.arange(4100) * max_k, np.concatenate(rows), rng.standard_normal(4099 * max_k).astype(np.float32).astype(np.float64))
+    (val_d, col_d, ptr_d), sp_d, ell_col, ell_val = _sliced_copy(CsrData(data.ptr[:n + 1], data.col[:n * max_k], data.val[:n * max_k]), n, d + 1, capi.ROW_F32)
+    val_d, col_d, ptr_d = G.dev(data.val), G.dev(data.col), G.dev(data.ptr)
+    sd = torch.empty(4099, dtype=torch.float64, device="cuda")
+    capi.call("tsvm_csr_self_dot", G.ptr(val_d), G.ptr(ptr_d), 4099, G.ptr(sd), G.stream())
+    out = torch.empty((4099, n), dtype=torch.float32, device="cuda")
+    best = {}
+    for m in [2048, 4099] * 6:
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        torch.cuda.synchronize()
+        a.record()
+        capi.call("tsvm_get_rows_csr_sliced", G.ptr(ell_col), G.ptr(ell_val), capi.ROW_F32, G.ptr(sp_d), n, G.ptr(sd), G.ptr(val_d), G.ptr(col_d),
+                  G.ptr(ptr_d), None, m, G.ptr(sd), d + 1, max_k, O.RBF, 0.1, 0.0, 3, G.ptr(out), capi.ROW_F32, None, n, G.stream())
+        b.record()
+        torch.cuda.synchronize()
+        best[m] = min(best.get(m, 1e9), a.elapsed_time(b))
+    assert best[4099] < 4 * best[2048], best
 
 
 @pytest.mark.parametrize("sizes", [(1, 2, 1), (63, 64, 65), (130, 1, 130), (512, 1023, 512)])   # calls one after another, their staging matrices in turn

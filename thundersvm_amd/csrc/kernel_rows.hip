@@ -10,6 +10,7 @@
 #include <cstdlib>
 
 #include "get_rows_tile.h"
+#include "sliced_deal.h"
 
 
 // Tiles from `tile0` on, one for each workgroup.
@@ -617,8 +618,8 @@ __global__ __launch_bounds__(SL_T) void get_rows_csr_sliced_kernel(
     const int *__restrict__ ell_col, const TV *__restrict__ ell_val, const int64_t *__restrict__ slice_ptr, int64_t n,
     const double *__restrict__ sd_x, const double *__restrict__ a_val, const int *__restrict__ a_col,
     const int64_t *__restrict__ a_ptr, const int *__restrict__ a_idx, int m, const double *__restrict__ sd_a, int d,
-    int slot_cap, KernelParam kp_in, TO *__restrict__ out, const int *__restrict__ out_slots, int64_t ldo, unsigned n_ib,
-    unsigned panels, unsigned per_panel, size_t off_remap, size_t off_bits, size_t off_base) {
+    int slot_cap, KernelParam kp_in, TO *__restrict__ out, const int *__restrict__ out_slots, int64_t ldo, SlicedDeal deal,
+    size_t off_remap, size_t off_bits, size_t off_base) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     __shared__ uint64_t exp_tab[32];
     __shared__ double s_sdi[SL_IB];
@@ -632,21 +633,13 @@ __global__ __launch_bounds__(SL_T) void get_rows_csr_sliced_kernel(
     unsigned *bits = (unsigned *) (lds + off_bits);
     unsigned *wbase = (unsigned *) (lds + off_base);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const unsigned logical = xcd_remap(blockIdx.x, gridDim.x);
     const int n_words = (d + 1 + 31) / 32;
     const int wpt = (n_words + SL_T - 1) / SL_T;
     typedef double tile4 __attribute__((ext_vector_type(4)));
     if (tid < 32) exp_tab[tid] = TSVM_EXP2F_TAB[tid];
-    // This workgroup's share of its panel: the panel's slices once for every block of sixteen working rows, cut into equal runs.
-    const int64_t n_slices = (n + 63) / 64;
-    const unsigned panel = logical / per_panel, part = logical % per_panel;
-    const int64_t first_slice = n_slices * panel / panels, width_p = n_slices * (panel + 1) / panels - first_slice;
-    const int64_t units = width_p * n_ib, t1 = units * (part + 1) / per_panel;
-    for (int64_t t = units * part / per_panel, t_next; t < t1; t = t_next) {
-    const int i0 = (int) (t / width_p) * SL_IB;
-    const int64_t slice0 = first_slice + t % width_p;
-    t_next = t - t % width_p + width_p < t1 ? t - t % width_p + width_p : t1;
-    const int64_t slice1 = slice0 + (t_next - t);
+    SlicedWalk walk(deal, xcd_remap(blockIdx.x, gridDim.x));
+    for (unsigned block, slice0, slice1; walk.next(deal, block, slice0, slice1);) {
+    const int i0 = (int) block * SL_IB;
     if (tid < SL_IB) {
         const int i = i0 + tid < m ? i0 + tid : m - 1;
         const int64_t row = a_idx ? (int64_t) a_idx[i] : (int64_t) i;
@@ -717,10 +710,10 @@ __global__ __launch_bounds__(SL_T) void get_rows_csr_sliced_kernel(
         }
         __syncthreads();
 
-        for (int64_t slice = slice0 + wave; slice < slice1; slice += SL_T / 64) {   // (wavefront-uniform; no barrier inside this loop)
+        for (unsigned slice = slice0 + wave; slice < slice1; slice += SL_T / 64) {   // (wavefront-uniform; no barrier inside this loop)
             const int64_t base = slice_ptr[slice];
             const int width = (int) ((slice_ptr[slice + 1] - base) >> 6);
-            const int64_t j = slice * 64 + lane;
+            const int64_t j = (int64_t) slice * 64 + lane;
             double acc[SL_IB];
 #pragma unroll
             for (int r = 0; r < SL_IB; ++r) acc[r] = 0.0;
@@ -1578,26 +1571,6 @@ size_t tsvm_get_rows_csr_sliced_lds(int n_features, int max_row_nnz, int val_typ
     return l.total;
 }
 
-// How the slices of n stored rows, once for each of n_ib blocks of working rows, are dealt to workgroups, of which a CU holds one: in panels
-// of neighbouring slices, each cut into per_panel equal runs.
-// One run is a block of working rows where panels x n_ib fills the chip, or what of it the solver's streams leave (248 CUs); otherwise a
-// run goes over from one block to the next, which costs it a second tile, and there are as many as CUs: with a workgroup for each
-// block and panel 4,099 rows (257 blocks) against 7,000 took five rounds of the chip for four and a hundredth of work (under the
-// profiler 341 -> 273 us; the prediction call 568 -> 504).
-// A panel is no larger than what an XCD's L2 holds, as its workgroups are at different places of it, if the runs stay a few tiles' work long.
-struct SlicedGrid {
-    unsigned panels, per_panel;
-};
-static SlicedGrid sliced_grid(int64_t n, unsigned n_ib, int max_row_nnz, int entry_bytes) {
-    constexpr int64_t CUS = 248, WAVES = SL_T / 64;
-    const int64_t slices = (n + 63) / 64, steps = (slices + WAVES - 1) / WAVES;
-    const int64_t whole = std::min<int64_t>(CUS / n_ib, steps);
-    if (whole >= 1 && (whole == steps || whole * n_ib * 10 >= CUS * 9)) return {(unsigned) whole, n_ib};
-    const int64_t units = slices * n_ib, by_l2 = n * max_row_nnz * entry_bytes / (4 << 20);
-    const int64_t panels = std::max<int64_t>(1, std::min({by_l2, units / (CUS * 8 * WAVES), slices}));
-    return {(unsigned) panels, (unsigned) std::max<int64_t>(1, std::min<int64_t>(CUS, units / panels / WAVES))};
-}
-
 int tsvm_get_rows_csr_sliced(const int *ell_col, const void *ell_val, int val_type, const int64_t *slice_ptr, int64_t n,
                              const double *sd_x, const double *a_val, const int *a_col, const int64_t *a_ptr, const int *a_idx,
                              int m, const double *sd_a, int n_features, int max_row_nnz, int kernel_type, double gamma,
@@ -1617,10 +1590,8 @@ int tsvm_get_rows_csr_sliced(const int *ell_col, const void *ell_val, int val_ty
     if (n == 0 || m == 0) return 0;
     KernelParam kp{kernel_type, degree, gamma, coef0};
     const SlicedLds l = sliced_lds(n_features);
-    const unsigned n_ib = (unsigned) ((m + SL_IB - 1) / SL_IB);
-    const SlicedGrid g = sliced_grid(n, n_ib, max_row_nnz, val_type == TSVM_ROW_F32 ? 8 : 12);
-    TSVM_REQUIRE((int64_t) g.panels * g.per_panel < (int64_t) 0x7fffffff, "tsvm_get_rows_csr_sliced: grid too large");
-    const dim3 grid(g.panels * g.per_panel), block(SL_T);
+    const SlicedDeal deal = sliced_deal(n, ((int64_t) m + SL_IB - 1) / SL_IB, leaves_cus_out(tsvm_s(stream)) ? 224 : 256);
+    const dim3 grid(deal.workgroups), block(SL_T);
 #define SL_LAUNCH_K(KTYPE, TO, TV)                                                                                           \
     do {                                                                                                                     \
         static bool opted_ = false;                                                                                          \
@@ -1631,7 +1602,7 @@ int tsvm_get_rows_csr_sliced(const int *ell_col, const void *ell_val, int val_ty
         }                                                                                                                    \
         hipLaunchKernelGGL((get_rows_csr_sliced_kernel<KTYPE, TO, TV>), grid, block, l.total, tsvm_s(stream), ell_col,       \
                            (const TV *) ell_val, slice_ptr, n, sd_x, a_val, a_col, a_ptr, a_idx, m, sd_a, n_features, l.slot_cap, kp, \
-                           (TO *) out, out_slots, ldo, n_ib, g.panels, g.per_panel, l.remap, l.bits, l.base);                                \
+                           (TO *) out, out_slots, ldo, deal, l.remap, l.bits, l.base); \
     } while (0)
 #define SL_LAUNCH(TO, TV)                                              \
     do {                                                               \

@@ -890,8 +890,8 @@ void KernelMatrix::get_rows(const RowStore &batch, size_t first, size_t n_rows, 
     // The batch's rows wait in LDS, sixteen at a time, and the support vectors' sliced copy streams by, as in training; a batch
     // with a row too long for that or without any entry is staged as a dense matrix, and so is any batch when a support vector holds an infinity
     // or NaN, whose product with an absent (zero) feature is not zero.  Kernel values of text rows, staged / sliced, us: 6,000
-    // support vectors 65 / 23 for one row, 87 / 38 for 64, 217 / 79 for 1,000, 1,148 / 263 for 4,099; 800 support vectors 24 / 22,
-    // 27 / 33, 65 / 35, 313 / 64; 3,000 31 / 23, 37 / 38, 128 / 42, 674 / 148 (4,099 rows before their blocks were dealt out evenly, a fifth less since): few of them fill few workgroups, so few rows go
+    // support vectors 71 / 25 for one row, 98 / 32 for 64, 228 / 73 for 1,000, 1,159 / 221 for 4,099; 800 support vectors 25 / 25,
+    // 28 / 31, 68 / 33, 322 / 64; 3,000 33 / 25, 40 / 34, 137 / 44, 680 / 146: few of them fill few workgroups, so few rows go
     // the staged way there.
     const int wt = R.values_fit_float ? TSVM_ROW_F32 : TSVM_ROW_F64;
     int longest = 0;
