@@ -637,6 +637,66 @@ def test_row_store_managed_on_the_device(n, d, ws):
     assert np.array_equal(st[h_slot_of][:, :n], all_rows)  # each row computed into its slot, nothing else touched
 
 
+@pytest.mark.parametrize("row_type", [capi.ROW_F32, capi.ROW_F64])
+@pytest.mark.parametrize("n,d", [(18433, 200), (20001, 200), (21504, 136), (21505, 200), (26625, 512), (28672, 520), (28673, 520), (28672, 200)])
+def test_rows_of_many_features_beside_a_solver(n, d, row_type):
+    """580, 628, 672, 836 and 896 tiles, which beside a solver are two launches, 676, 900 and 896 of fewer features, which are one.  On a stream
+    that leaves out one CU, and one that leaves out eight: the bits of the call on the whole chip, whose rows
+    test_get_rows_* hold to the oracle; all rows, and as many of them as the device says, from none to all, into scattered slots."""
+    rng = np.random.default_rng(n)
+    m = 512
+    x = torch.from_numpy(rng.standard_normal((n, d)).astype(np.float32)).cuda().double()
+    sd = (x * x).sum(1)
+    dt = torch.float32 if row_type == capi.ROW_F32 else torch.float64
+    idx = rng.integers(0, n, m).astype(np.int32)
+    want = G.host(G.get_rows_dense(x, d, n, d, sd, x, d, G.dev(idx), m, sd, O.RBF, gamma=0.01, row_type=row_type))
+    slots = rng.permutation(m + 9)[:m].astype(np.int32)
+    idx_d, slots_d = G.dev(idx), G.dev(slots)
+    for lanes in (1, 8):
+        for count in (m, 0, 1, 129, 300, 385, 511, None):
+            out = torch.full((m + 9, n), -3.0, dtype=dt, device="cuda")
+            rows = m if count is None else count
+            m_d = G.dev(np.array([rows], dtype=np.int32))
+            with G.stream_without_cus(lanes):
+                if count is None:
+                    capi.call("tsvm_get_rows_dense", G.ptr(x), d, None, n, d, G.ptr(sd), G.ptr(x), d, G.ptr(idx_d), m, G.ptr(sd), O.RBF, 0.01, 0.0, 3,
+                              G.ptr(out), row_type, G.ptr(slots_d), n, G.stream())
+                else:
+                    capi.call("tsvm_get_rows_dense_counted", G.ptr(x), d, None, n, d, G.ptr(sd), G.ptr(x), d, G.ptr(idx_d), m, G.ptr(m_d), G.ptr(sd), O.RBF,
+                              0.01, 0.0, 3, G.ptr(out), row_type, G.ptr(slots_d), n, G.stream())
+            assert torch.equal(out[torch.from_numpy(slots[:rows]).long().cuda()], torch.from_numpy(want[:rows]).cuda()), (lanes, count)
+            rest = np.setdiff1d(np.arange(m + 9), slots[:rows])
+            assert (out[torch.from_numpy(rest).cuda()] == -3.0).all(), (lanes, count)
+
+
+def test_rows_beside_a_solver_in_one_launch_where_two_are_slower():
+    """900 tiles of 784 features on 255 CUs: 397 us in one launch, 505 as 896 and 4; at most a tenth more than on the whole chip."""
+    n, d, m = 28800, 784, 512
+    x = torch.rand((n, d), dtype=torch.float64, device="cuda")
+    sd = (x * x).sum(1)
+    idx = torch.randint(0, n, (m,), dtype=torch.int32, device="cuda")
+    out = torch.empty((m, n), dtype=torch.float32, device="cuda")
+
+    def best():
+        times = []
+        for _ in range(8):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            torch.cuda.synchronize()
+            a.record()
+            capi.call("tsvm_get_rows_dense", G.ptr(x), d, None, n, d, G.ptr(sd), G.ptr(x), d, G.ptr(idx), m, G.ptr(sd), O.RBF, 0.01, 0.0, 3, G.ptr(out),
+                      capi.ROW_F32, None, n, G.stream())
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    whole = best()
+    with G.stream_without_cus(1):
+        beside = best()
+    print("900 tiles: %.0f us, on 255 CUs %.0f" % (1e3 * whole, 1e3 * beside))
+    assert beside < 1.15 * whole
+
+
 @pytest.mark.parametrize("name,kt,prm", KERNELS)
 @pytest.mark.parametrize("n,d,ws", [(300, 20, 64), (3000, 54, 1000), (2600, 200, 1024), (1500, 784, 200)])
 def test_working_set_block(name, kt, prm, n, d, ws):

@@ -13,30 +13,37 @@
 #include "sliced_deal.h"
 
 
-// Tiles from `tile0` on, one for each workgroup.
-// Workgroups are dealt to a die's four groups of eight CUs in turn, whether or not a group has a CU that its stream leaves to a solver, so
-// that a launch of 496, two for each of 248 CUs, lasts as long as three of them on one CU (287 us).  On such a stream a launch of a few
-// rounds is made in rounds of GR_WGS tiles, which all have their place, and the rest, most of which then have a CU each, as a launch
-// of their own: 512 rows of 20,000 columns, 784 features (628 tiles) beside a solver 340 us in the middle -> 197 + 113.  (A loop over
-// the tiles in a grid of 496 workgroups 316: its registers cost the K loop instructions, and on a stream that has the chip 310 for 288.)
-// Longer launches even out.
-#define GR_WGS 448u
-#define GR_WGS_ROUNDS 4u
+// One tile for each workgroup, two workgroups a CU.
+// Beside a solver (a stream that leaves its CU out) some counts of tiles are made in two launches: GR_FIRST tiles, which all have their
+// place (workgroups are dealt to a die's four groups of eight CUs in turn, whether or not a group lacks one: fourteen for each), and the
+// rest.  In one launch the rest take the places that become free first, mostly two of a CU that has just ended its two, while other
+// CUs have nothing.  us in one launch / two, 784 features, 255 CUs:
+//   tiles  508      512      560      580      628      660      700      800      832      864      892      900      1,000    1,252    1,792
+//          238/238  286/304  292/304  335/305  336/305  336/306  373/381  380/381  378/381  396/382  396/382  397/505  465/507  553/586  736/734
+// (some of them one launch's luck with places: 580 295 to 335).  So from 18 tiles for a group of CUs on to where the rest are more than one
+// a CU, and, with tiles long enough, from 26 to where they are more than two; 200 features at 628 tiles 108/95, at 864 112/116, 3,000
+// 1,200/1,110 and at 896 1,440/1,402.  (Where several solves share the chip nobody knows which places are free.)
+// The number of rows may only be known on the device (m_dev, of m at most): of two launches, the first is then of all tiles and the
+// second's workgroups leave unless the count asks for two (512 rows of 20,000 columns, 300 of them wanted: 201 us; as two launches 310).
+#define GR_FIRST 448u
+__host__ __device__ inline bool two_launches(unsigned tiles, int d) { return (tiles > 576 && tiles <= 672) || (tiles > 832 && tiles <= 896 && d >= 512); }
 template <int KT, int TI, typename TO>
 __global__ __launch_bounds__(256, (TI == 2 ? 3 : 2)) void get_rows_dense_kernel(
     const double *__restrict__ x, int64_t ldx, const int *__restrict__ x_idx, int64_t n, int d,
     const double *__restrict__ sd_x, const double *__restrict__ a, int64_t lda, const int *__restrict__ a_idx, int m,
     const double *__restrict__ sd_a, KernelParam kp, TO *__restrict__ out, const int *__restrict__ out_slots,
-    int64_t ldo, const int *__restrict__ m_dev, unsigned tile0) {
+    int64_t ldo, const int *__restrict__ m_dev, int part) {   // part: 0 all tiles, 1 and 2 the first and the second of two launches
     __shared__ double As[GrShape<TI>::LDS_DOUBLES];
     __shared__ double Bs[GrShape<TI>::LDS_DOUBLES];
     __shared__ uint64_t exp_tab[32];
     if (threadIdx.x < 32) exp_tab[threadIdx.x] = TSVM_EXP2F_TAB[threadIdx.x];
     __syncthreads();
-    if (m_dev) m = *m_dev;   // the number of working rows is only known on the device (m sized the grid): workgroups beyond it leave
+    if (m_dev) m = *m_dev;
     const unsigned m_blocks = (unsigned) (m + GrShape<TI>::BM - 1) / GrShape<TI>::BM, tiles = (unsigned) ((n + GR_BN - 1) / GR_BN) * m_blocks;
-    if (tile0 + blockIdx.x >= tiles) return;
-    const unsigned tile = tile0 + xcd_remap(blockIdx.x, tiles - tile0 < gridDim.x ? tiles - tile0 : gridDim.x);
+    const bool two = part != 0 && two_launches(tiles, d);
+    const unsigned first = part == 2 ? (two ? GR_FIRST : tiles) : 0, here = (two && part == 1 ? GR_FIRST : tiles) - first;
+    if (blockIdx.x >= here) return;
+    const unsigned tile = first + xcd_remap(blockIdx.x, here < gridDim.x ? here : gridDim.x);
     const int j0 = (int) (tile / m_blocks) * GR_BN;   // n fits 31 bits (checked by the host)
     const int i0 = (int) (tile % m_blocks) * GrShape<TI>::BM;
     get_rows_tile<KT, TI, TO>(x, ldx, x_idx, n, d, sd_x, a, lda, a_idx, m, sd_a, kp, out, out_slots, ldo, i0, j0, As, Bs, exp_tab);
@@ -1244,16 +1251,16 @@ static int stream_tiles_per_wg() {
     return v;
 }
 
-// Whether a stream has been made with a mask that is not all of the chip's 256 CUs.
-static bool leaves_cus_out(hipStream_t stream) {
+// How many of the chip's 256 CUs a stream's mask has.
+static int cus_of(hipStream_t stream) {
     uint32_t mask[8] = {};
     if (!stream || hipExtStreamGetCUMask(stream, 8, mask) != hipSuccess) {
         (void) hipGetLastError();
-        return false;
+        return 256;
     }
     int cus = 0;
     for (uint32_t word : mask) cus += __builtin_popcount(word);
-    return cus > 0 && cus < 256;
+    return cus > 0 ? cus : 256;
 }
 
 static int get_rows_dense(const double *x, int64_t ldx, const int *x_idx, int64_t n, int d, const double *sd_x, const double *a,
@@ -1286,11 +1293,8 @@ static int get_rows_dense(const double *x, int64_t ldx, const int *x_idx, int64_
     const int64_t n_blocks = (n + GR_BN - 1) / GR_BN;
     TSVM_REQUIRE(n_blocks * m_blocks < (int64_t) 0x7fffffff, "tsvm_get_rows_dense: grid too large");
     dim3 grid((unsigned) (n_blocks * m_blocks)), block(256);
-    unsigned last = 0;   // tiles of a launch of their own
-    if (ti == 4 && grid.x > GR_WGS && grid.x <= GR_WGS_ROUNDS * GR_WGS && leaves_cus_out(tsvm_s(stream))) {
-        last = grid.x % GR_WGS;
-        grid.x -= last;
-    }
+    const bool two = ti == 4 && two_launches(grid.x, d) && cus_of(tsvm_s(stream)) == 255;
+    const dim3 first(two && !m_dev ? GR_FIRST : grid.x), second(grid.x - GR_FIRST);
     // the solver's ws x ws block: symmetric, computed from the tiles on and above the diagonal
     const bool sym = x == a && ldx == lda && x_idx && x_idx == a_idx && n == m && sd_x == sd_a && !out_slots && !m_dev &&
                      !mask_x && ti == 2 && ldo >= n;   // (with masks d does not count the columns that they stand for)
@@ -1353,11 +1357,11 @@ static int get_rows_dense(const double *x, int64_t ldx, const int *x_idx, int64_
                 default: GR_STREAM(KTYPE, TO, 5); break;                                                              \
             }                                                                                                         \
         } else {                                                                                                      \
-            hipLaunchKernelGGL((get_rows_dense_kernel<KTYPE, 4, TO>), grid, block, 0, tsvm_s(stream), x, ldx, x_idx, n, d, sd_x, \
-                               a, lda, a_idx, m, sd_a, kp, (TO *) out, out_slots, ldo, m_dev, 0u);                    \
-            if (last)                                                                                                 \
-                hipLaunchKernelGGL((get_rows_dense_kernel<KTYPE, 4, TO>), dim3(last), block, 0, tsvm_s(stream), x, ldx, x_idx, n, d, sd_x, \
-                                   a, lda, a_idx, m, sd_a, kp, (TO *) out, out_slots, ldo, m_dev, grid.x);            \
+            hipLaunchKernelGGL((get_rows_dense_kernel<KTYPE, 4, TO>), first, block, 0, tsvm_s(stream), x, ldx, x_idx, n, d, sd_x, \
+                               a, lda, a_idx, m, sd_a, kp, (TO *) out, out_slots, ldo, m_dev, two ? 1 : 0);           \
+            if (two)                                                                                                  \
+                hipLaunchKernelGGL((get_rows_dense_kernel<KTYPE, 4, TO>), second, block, 0, tsvm_s(stream), x, ldx, x_idx, n, d, sd_x, \
+                                   a, lda, a_idx, m, sd_a, kp, (TO *) out, out_slots, ldo, m_dev, 2);                 \
         }                                                                                                             \
     } while (0)
 #define GR_LAUNCH(KTYPE)                                        \
@@ -1590,7 +1594,7 @@ int tsvm_get_rows_csr_sliced(const int *ell_col, const void *ell_val, int val_ty
     if (n == 0 || m == 0) return 0;
     KernelParam kp{kernel_type, degree, gamma, coef0};
     const SlicedLds l = sliced_lds(n_features);
-    const SlicedDeal deal = sliced_deal(n, ((int64_t) m + SL_IB - 1) / SL_IB, leaves_cus_out(tsvm_s(stream)) ? 224 : 256);
+    const SlicedDeal deal = sliced_deal(n, ((int64_t) m + SL_IB - 1) / SL_IB, cus_of(tsvm_s(stream)) < 256 ? 224 : 256);
     const dim3 grid(deal.workgroups), block(SL_T);
 #define SL_LAUNCH_K(KTYPE, TO, TV)                                                                                           \
     do {                                                                                                                     \
