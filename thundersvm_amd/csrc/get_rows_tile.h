@@ -66,6 +66,7 @@ __device__ __forceinline__ v4i indicator_bytes(unsigned bits, const uint64_t *ta
     const uint64_t t0 = tab[bits & 0xff], t1 = tab[bits >> 8];
     return (v4i){(int) (uint32_t) t0, (int) (t0 >> 32), (int) (uint32_t) t1, (int) (t1 >> 32)};
 }
+typedef uint16_t __attribute__((may_alias)) mask_part_t;   // (the masks are written as 64-bit words)
 // A single addition is left to the epilogue (IND = 1, `one_indicator`): and, compare, select and add cost what the bytes, the product,
 // its conversion and the add do (512 rows of 100,003 columns, 30 of 41 features indicators: 93.6 us that way, 95.1 this way).
 __device__ __forceinline__ double one_indicator(double dot, uint64_t mi, uint64_t mj) { return dot + ((mi & mj) != 0 ? 1.0 : 0.0); }
@@ -74,7 +75,7 @@ __device__ __forceinline__ double one_indicator(double dot, uint64_t mi, uint64_
 template <int IND, int TI>
 __device__ __forceinline__ void add_indicators(v4d (&acc)[TI][4], const uint64_t *m_rows, const uint64_t *m_cols, int lrow, int lk, int max_ones,
                                                const uint64_t *tab) {
-    const uint16_t *const rows = (const uint16_t *) m_rows + lk, *const cols = (const uint16_t *) m_cols + lk;   // bits 16 lk ..
+    const mask_part_t *const rows = (const mask_part_t *) m_rows + lk, *const cols = (const mask_part_t *) m_cols + lk;   // bits 16 lk ..
     unsigned rbits[TI], cbits[4];
 #pragma unroll
     for (int ti = 0; ti < TI; ++ti) rbits[ti] = rows[4 * (ti * 16 + 4 * (lrow & 3) + (lrow >> 2))];
