@@ -68,7 +68,7 @@ def build_selftests():
     _run(["g++", "-O2", "-fPIC", "-std=c++17", "-fopenmp", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", os.path.join(native, "selftest.cpp"),
           "-shared", "-o", out, *links])
     # (-rdynamic: their stand-ins for the HIP calls take the place of the runtime's in the host library)
-    for program in ("two_devices", "lane_streams"):
+    for program in ("two_devices", "lane_streams", "sparse_block"):
         _run(["g++", "-O2", "-std=c++17", "-fopenmp", "-rdynamic", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", os.path.join(native, program + ".cpp"),
               "-o", os.path.join(native, program), *links])
     return out

@@ -771,6 +771,13 @@ void KernelMatrix::get_rows_counted(const int *d_idx, int m_max, const int *d_m,
                                           param.gamma, param.coef0, param.degree, d_out, row_type(), d_out_slots, ld, stream));
 }
 
+// Staging matrices of up to this size come in pairs, so that one's rows are taken out by the launch that puts the next block's into the
+// other.  It is a launch of 1 to 3 us that this saves, and nothing once the matrix is larger than the caches, where the two cost
+// more than the launch: the block of 1,024 rows of 3,000 features (floats, 12 MB) 26.4 us with two, 27.7 with one, of 21,000 (86 MB)
+// 32.2 / 33.4, doubles (172 MB) 49.1 / 48.0, of 200,000 (819 MB) 38.5 / 35.3.  A row cache takes nine tenths of what memory is free before
+// the first block is asked for: of 3.2 million features one matrix is 13 GB, and a second need not fit.
+constexpr size_t STAGE_TURNS_MAX = (size_t) 128 << 20;
+
 // K(x_idx[r], x_idx[t]) for r, t < m: the same kernels with the column set restricted to the m rows,
 // so every value is bit-identical to the corresponding entry of a full kernel row.  Elements are row_type() wide.
 void KernelMatrix::get_block(const int *d_idx, int m, void *d_out, int64_t ld, hipStream_t stream) const {
@@ -785,18 +792,32 @@ void KernelMatrix::get_block(const int *d_idx, int m, void *d_out, int64_t ld, h
     const size_t bytes = (size_t) m * R.n_features * (R.values_fit_float ? sizeof(float) : sizeof(double));
     // K(r, t) is K(t, r) to the last bit unless a value times an absent (zero) one is not zero, or the two rows' common features come in two orders
     if (R.values_finite && R.columns_ascend && R.nnz > 0) {
-        BlockStage &now = turn_[turn_now_], &last = turn_[turn_now_ ^ 1];
-        if (now.w.size() < bytes) {
-            grow_zeroed(now.w, bytes, stream);
-            now.m = 0;
+        if (turn_[turn_now_].m != 0) throw std::logic_error("KernelMatrix::get_block: rows in the staging matrix");
+        bool turns = std::max(bytes, turn_[turn_now_].w.size()) <= STAGE_TURNS_MAX && !one_stage_;
+        try {
+            grow_zeroed(turn_[turn_now_].w, bytes, stream);
+        } catch (const std::bad_alloc &) {
+            BlockStage &first = turn_[turn_now_ ^ 1];
+            if (first.w.size() < bytes) throw;
+            (void) hipGetLastError();   // no room for a second one: the first has to do from now on
+            if (first.m) abi_check(tsvm_csr_scatter_rows(R.val.data(), R.col.data(), R.row_ptr.data(), first.ids.data(), first.m, (int) R.n_features,
+                                                         first.w.data(), wt, 1, stream));
+            first.m = 0;
+            turn_now_ ^= 1;
+            one_stage_ = true;
+            turns = false;
         }
-        if (now.m != 0) throw std::logic_error("KernelMatrix::get_block: rows in the staging matrix");
+        BlockStage &now = turn_[turn_now_], &last = turn_[turn_now_ ^ 1];
         if (now.ids.size() < (size_t) m) now.ids.resize(m);
         abi_check(tsvm_csr_block(R.val.data(), R.col.data(), R.row_ptr.data(), d_idx, m, R.self_dot.data(), now.w.data(), now.ids.data(), last.w.data(),
                                  last.ids.data(), last.m, wt, (int) param.kernel_type, param.gamma, param.coef0, param.degree, d_out, row_type(), ld, stream));
-        now.m = m;
         last.m = 0;
-        turn_now_ ^= 1;
+        if (turns) {
+            now.m = m;
+            turn_now_ ^= 1;
+        } else {
+            abi_check(tsvm_csr_scatter_rows(R.val.data(), R.col.data(), R.row_ptr.data(), d_idx, m, (int) R.n_features, now.w.data(), wt, 1, stream));
+        }
         return;
     }
     // kept all-zero between uses, as in get_rows

@@ -135,7 +135,8 @@ private:
     // transposed staging of CSR working rows (get_rows / get_block), all-zero between uses; float elements when
     // the rows' values are floats
     mutable tsvm::DeviceBuffer<unsigned char> stage_w_, stage_blk_;
-    // get_block's two that take turns (tsvm_csr_block): the rows that are in them are taken out by the next call
+    // get_block's two that take turns (tsvm_csr_block): the rows that are in them are taken out by the next call.  Large ones, and one that
+    // the device has no second beside (one_stage_), are used alone.
     struct BlockStage {
         tsvm::DeviceBuffer<unsigned char> w;
         tsvm::DeviceBuffer<int> ids;
@@ -143,6 +144,7 @@ private:
     };
     mutable BlockStage turn_[2];
     mutable int turn_now_ = 0;
+    mutable bool one_stage_ = false;
     mutable tsvm::DeviceBuffer<kernel_type> stage_blk_sd_;
     mutable tsvm::DeviceBuffer<kernel_type> stage_sd_;
     mutable tsvm::DeviceBuffer<kernel_type> b_val_;
