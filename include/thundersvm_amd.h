@@ -137,7 +137,7 @@ int tsvm_csr_scatter_rows(const double *val, const int *col, const int64_t *row_
 /* out[r * ldo + t] = kernel value of rows idx[r] and idx[t], r, t < m <= 16384.  For rows whose values are finite and whose columns ascend, at least
  * one entry among all of them; the entries are those of tsvm_get_rows_csr, bit for bit.  w [n_features][m], elements of w_type as for
  * tsvm_get_rows_csr_staged, all-zero before; it is left with the rows in it and their numbers in ids [m].  To be used again it has to be
- * another call's w_old, with its ids as ids_old and its m as m_old: that call takes them out. */
+ * another call's w_old, with its ids as ids_old and its m as m_old: that call takes them out, one of no rows, too. */
 int tsvm_csr_block(const double *val, const int *col, const int64_t *row_ptr, const int *idx, int m, const double *sd, void *w, int *ids, void *w_old,
                    const int *ids_old, int m_old, int w_type, int kernel_type, double gamma, double coef0, int degree, void *out, int row_type, int64_t ldo,
                    tsvm_stream stream);

@@ -280,7 +280,7 @@ def test_csr_sliced_few_stored_rows_fill_the_chip():
     assert best[4099] < 4 * best[2048], best
 
 
-@pytest.mark.parametrize("sizes", [(1, 2, 1), (63, 64, 65), (130, 1, 130), (512, 1023, 512)])   # calls one after another, their staging matrices in turn
+@pytest.mark.parametrize("sizes", [(1, 2, 1), (63, 64, 65), (130, 1, 130), (512, 1023, 512), (65, 0, 64)])   # calls one after another, their staging matrices in turn
 @pytest.mark.parametrize("name,kt,prm", KERNELS)
 def test_csr_block(name, kt, prm, sizes):
     """tsvm_csr_block (the solver's block: entries above the diagonal computed, the others mirrored) against the oracle's rows, bit for bit:

@@ -1456,14 +1456,14 @@ int tsvm_csr_scatter_rows(const double *val, const int *col, const int64_t *row_
 int tsvm_csr_block(const double *val, const int *col, const int64_t *row_ptr, const int *idx, int m, const double *sd, void *w, int *ids, void *w_old,
                    const int *ids_old, int m_old, int w_type, int kernel_type, double gamma, double coef0, int degree, void *out, int row_type, int64_t ldo,
                    tsvm_stream stream) {
-    TSVM_REQUIRE(val && col && row_ptr && idx && w && ids && out, "tsvm_csr_block: null pointer");
+    TSVM_REQUIRE(val && col && row_ptr && (m == 0 || (idx && w && ids && out)), "tsvm_csr_block: null pointer");
     TSVM_REQUIRE(w_type == TSVM_ROW_F64 || w_type == TSVM_ROW_F32, "tsvm_csr_block: unknown staging type %d", w_type);
     TSVM_REQUIRE(m >= 0 && m <= 16384 && m_old >= 0 && m_old <= 16384 && ldo >= m, "tsvm_csr_block: %d rows (at most 16384), %d before", m, m_old);
     TSVM_REQUIRE(m_old == 0 || (w_old && ids_old && w_old != w && ids_old != ids), "tsvm_csr_block: no rows of the last time");
     TSVM_REQUIRE(kernel_type >= 0 && kernel_type <= 4, "tsvm_csr_block: unknown kernel type %d", kernel_type);
     TSVM_REQUIRE(row_type_ok(row_type, kernel_type), "tsvm_csr_block: row type %d not valid for kernel type %d", row_type, kernel_type);
     TSVM_REQUIRE((kernel_type != TSVM_RBF && kernel_type != TSVM_PRECOMPUTED) || sd, "tsvm_csr_block: RBF needs self dot products");
-    if (m == 0) return 0;
+    if (m == 0 && m_old == 0) return 0;
     const KernelParam kp{kernel_type, degree, gamma, coef0};
     const int tiles = (m + 63) / 64, esz = row_type == TSVM_ROW_F32 ? 4 : 8;
     const dim3 grid((unsigned) (tiles * (tiles + 1) / 2 * (64 / (4 * CSB_J))));
@@ -1477,6 +1477,7 @@ int tsvm_csr_block(const double *val, const int *col, const int64_t *row_ptr, co
         hipLaunchKernelGGL(csr_restage_rows_kernel<TW>, dim3((unsigned) ((m + m_old + 3) / 4)), dim3(256), 0, tsvm_s(stream), val, col, row_ptr, idx, \
                            m, (TW *) w, ids, ids_old, m_old, (TW *) w_old);                                                                    \
         TSVM_LAUNCH_CHECK();                                                                                                                   \
+        if (m == 0) return 0;   /* (the last call's rows are out) */                                                                           \
         if (row_type == TSVM_ROW_F32) CSB_LAUNCH(float, TW);                                                                                   \
         else CSB_LAUNCH(double, TW);                                                                                                           \
     } while (0)
