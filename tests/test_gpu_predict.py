@@ -452,17 +452,84 @@ def test_groups_of_rows_in_one_launch(k, d, kernel):
 @pytest.mark.parametrize("k,d,hot,kernel", [(2, 1, 0, capi.RBF), (2, 32, 0, capi.RBF), (3, 33, 0, capi.POLY), (4, 60, 0, capi.SIGMOID), (9, 127, 0, capi.LINEAR),
                                             (7, 5, 40, capi.RBF), (2, 12, 64, capi.LINEAR), (10, 4, 0, capi.RBF), (2, 150, 0, capi.RBF)])
 def test_requests_of_a_few_rows(k, d, hot, kernel):
-    """A few rows in one launch against the same rows as part of a batch that takes the kernels for many: the same bits, whatever of
-    the batch's rows a request asks for; ten classes and 150 columns take the other route."""
+    """A few rows in one launch against the same rows as part of a batch on the device, which takes the kernels for many whatever its size: the
+    same bits, whatever of the batch's rows a request asks for; ten classes and 150 columns take the other route."""
     rng = np.random.default_rng(1000 * k + d)
     x, y = _blobs(rng, k, 260 // k + 20, d, one_hot=hot)
     xt, _ = _blobs(np.random.default_rng(2000 * k + d), k, 100 // k, d, one_hot=hot)
     xt[3] = 0.0
     gm = Model(0).train(D.from_dense(x, y), make_param(svm_type=0, kernel_type=kernel, gamma=0.5 / d, coef0=0.1, degree=2, C=3.0))
-    lab, dec = gm.predict(D.from_dense(xt, np.zeros(len(xt))))
+    lab, dec = gm.predict(Dataset(D.from_dense(xt, np.zeros(len(xt)))).to_device())
     for first, m in [(0, 1), (3, 1), (0, 2), (5, 3), (1, 4), (2, 5), (0, 7), (1, 8), (0, 9), (7, 15), (4, 16), (0, 17)]:
         l, v = gm.predict(D.from_dense(xt[first:first + m], np.zeros(m)))
         assert np.array_equal(v, dec[first:first + m]) and np.array_equal(l, lab[first:first + m]), (first, m)
+
+
+@pytest.mark.parametrize("kernel", [capi.RBF, capi.POLY, capi.SIGMOID, capi.LINEAR])
+@pytest.mark.parametrize("k,d,hot", [(2, 1, 0), (2, 33, 0), (3, 16, 0), (4, 128, 0), (5, 100, 64), (7, 128, 64), (9, 60, 0), (8, 31, 33)])
+def test_few_rows_kernel(k, d, hot, kernel):
+    """tsvm_predict_few_rows' sums per 128 support vectors are those that tsvm_predict_dec_values_dense leaves, to the last bit: rows among
+    the launch's arguments, in both sizes of these, and read from page-locked memory; up to 192 columns, the last `hot` of them indicators;
+    classes of no support vectors, of one tile and of several."""
+    rng = np.random.default_rng(100 * k + d + kernel)
+    n, all_d, nc = 600, d + hot, k - 1
+    ldx = (all_d + 7) // 8 * 8
+
+    def rows_of(count):
+        x = np.zeros((count, ldx))
+        x[:, :d] = rng.standard_normal((count, d)).astype(np.float32)
+        if hot:
+            for _ in range(3):
+                x[np.arange(count), d + rng.integers(0, hot, count)] = 1
+        return x
+
+    sv = rows_of(n)
+    n_sv = [0 if k > 2 and c == 1 else 1 + (97 * c) % 250 for c in range(k)]
+    stride = capi.kernel_lib().tsvm_predict_nc_stride(k, d, 1 if hot else 0)
+    assert stride >= nc
+    cols, coefs, tiles = [], [], 0
+    chunks, starts = [], [0]
+    for c in range(k):
+        t = (n_sv[c] + 127) // 128
+        ids, w = np.zeros(128 * t, dtype=np.int32), np.zeros((128 * t, stride))
+        ids[:n_sv[c]] = rng.integers(0, n, n_sv[c])
+        w[:n_sv[c], :nc] = rng.standard_normal((n_sv[c], nc))
+        cols.append(ids)
+        coefs.append(w)
+        chunks += [(i, i + 1) for i in range(tiles, tiles + t)]
+        tiles += t
+        starts.append(tiles)
+    sv_d, sd_d, map_d, coef_d = G.dev(sv), G.dev((sv * sv).sum(axis=1)), G.dev(np.concatenate(cols)), G.dev(np.concatenate(coefs))
+    chunk_d, start_d, rho_d = G.dev(np.array(chunks, dtype=np.int32)), G.dev(np.array(starts, dtype=np.int32)), torch.zeros(k * nc // 2, dtype=torch.float64, device="cuda")
+
+    def masks_of(x_d, count):
+        masks, most = torch.zeros(count, dtype=torch.int64, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+        capi.call("tsvm_indicator_masks", G.ptr(x_d), ldx, count, d, hot, G.ptr(masks), G.ptr(most), G.stream())
+        return masks, int(G.host(most)[0])
+
+    mask_sv, ones = masks_of(sv_d, n) if hot else (None, 0)
+    args = (kernel, 0.5 / d, 0.1, 3)
+    for m in (1, 2, 3, 4, 5, 9, 16, 61):
+        a = rows_of(m)
+        if m > 2: a[2] = 0.0
+        a_d, asd = G.dev(a), (a * a).sum(axis=1)
+        asd_d = G.dev(asd)
+        mask_a = masks_of(a_d, m)[0] if hot else None
+        part = torch.full((tiles * m * nc,), np.nan, dtype=torch.float64, device="cuda")
+        dec = torch.empty(m * k * nc // 2, dtype=torch.float64, device="cuda")
+        capi.call("tsvm_predict_dec_values_dense", G.ptr(sv_d), ldx, d, G.ptr(sd_d), G.ptr(mask_sv), G.ptr(map_d), 128 * tiles, G.ptr(coef_d), G.ptr(chunk_d), tiles,
+                  G.ptr(start_d), G.ptr(rho_d), k, G.ptr(a_d), ldx, m, G.ptr(asd_d), G.ptr(mask_a), ones, *args, G.ptr(part), G.ptr(dec), G.stream())
+        size = capi.kernel_lib().tsvm_predict_few_rows_bytes(m, all_d)
+        values = (m * all_d + 1) // 2 * 2
+        assert size == 4 * values + 8 * m
+        request = torch.zeros(size, dtype=torch.uint8).pin_memory()
+        request.numpy()[:4 * m * all_d] = np.ascontiguousarray(a[:, :all_d].astype(np.float32)).view(np.uint8).ravel()
+        request.numpy()[4 * values:] = asd.view(np.uint8)
+        few = torch.full((tiles * m * nc,), -7.0, dtype=torch.float64, device="cuda")
+        capi.call("tsvm_predict_few_rows", G.ptr(sv_d), ldx, all_d, G.ptr(sd_d), G.ptr(map_d), 128 * tiles, G.ptr(coef_d), stride, nc, request.data_ptr(),
+                  request.data_ptr(), m, *args, G.ptr(few), G.stream())
+        assert np.array_equal(G.host(few), G.host(part)), m
+        assert np.isfinite(G.host(part)).all() and np.abs(G.host(part)).max() > 0
 
 
 def test_requests_of_a_few_rows_that_are_not_plain_floats():
@@ -475,7 +542,7 @@ def test_requests_of_a_few_rows_that_are_not_plain_floats():
     xt = np.zeros((80, 9))
     xt[:, :6], xt[5, 8], xt[7, 7] = rows, 2.5, 1e-3
     ptr, col = np.arange(81, dtype=np.int64) * 9, np.tile(np.arange(1, 10, dtype=np.int32), 80)
-    _, dec = gm.predict(D.CsrData(ptr, col, xt.reshape(-1), np.zeros(80)))
+    _, dec = gm.predict(D.CsrData(ptr, col, xt.reshape(-1), np.zeros(80)))   # (a value that is no float: the kernels for many rows)
     for first, m in [(0, 1), (1, 1), (2, 1), (0, 8), (3, 5), (41, 3), (70, 10)]:
         _, v = gm.predict(D.CsrData(ptr[:m + 1], col[:9 * m], xt[first:first + m].reshape(-1).copy(), np.zeros(m)))
         assert np.array_equal(v, dec[first:first + m], equal_nan=True), (first, m)
