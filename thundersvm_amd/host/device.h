@@ -37,7 +37,7 @@ hipStream_t work_stream();
 
 // Device blocks that buffers have released, kept for the next buffer of about the same size: hipMalloc and hipFree cost
 // microseconds to milliseconds each (hipFree waits for the device), and a small training run makes some forty of them.
-// Blocks are rounded up to quarter powers of two; blocks above 64 MiB and whatever would take the pool over 512 MiB go
+// Blocks are rounded up to quarter powers of two; blocks above 256 MiB and whatever would take the pool over 2 GiB go
 // back to the driver, everything does when the device runs out of memory, on tsvm_release_device_cache() and when the
 // process ends.  A block is handed out again only after the device has been idle since its release (as hipFree would
 // have waited for), unless whoever released it knows that nothing uses it any more (`idle`).  One list per device, a
