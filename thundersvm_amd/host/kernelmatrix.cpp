@@ -22,7 +22,8 @@ static int current_device() {
 struct DevicePool::Impl {
     // A block beyond that is allocated and freed by every training call, and a free waits for all that the device has in flight, other class
     // pairs' kernels among it.  With 64 MB / 512 MB the staging matrices of 21,000 features (86 MB each) and the rows of the larger pairs of
-    // 300,000 instances (115 MB) were: linear text, 18,000 rows, 31.8 -> 31.2 ms a call, seven classes of 300,000 579.7 -> 572.8 and 664.8 -> 656.6.
+    // 300,000 instances (115 MB) were: linear text, 18,000 rows, 31.8 -> 31.2 ms a call; seven classes of 300,000 rows 579.7 -> 572.8 and 664.8 ->
+    // 656.6 on two cards, within what runs differ by on a third.
     static constexpr size_t MAX_BLOCK = (size_t) 256 << 20, MAX_TOTAL = (size_t) 2 << 30;
     std::mutex mu;
     // [device, block size] -> blocks; `waiting`: released since the device was last known to be idle
